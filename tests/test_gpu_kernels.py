@@ -37,6 +37,34 @@ def test_gemm_f32(gpu, M, N, K):
         assert torch.equal(one[0], out[M - 1])
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 8, 32), (16, 2048, 96), (17, 2049, 128), (33, 70, 320), (64, 2052, 2080), (65, 64, 2048),
+                                   (300, 2050, 2048), (130, 66, 4160), (1030, 4100, 160), (500, 2048, 64)])
+def test_gemm_f32_matrix_cores(gpu, M, N, K):
+    """The kernel for inner sizes that are multiples of 32, in blocks of 16, 32 and 64: the bits of the general kernel's
+    ascending chain of fused multiply-adds, which operands off a 16-byte border take."""
+    from tuff_amd.csrc import ops
+    x, w, y0 = _r(M, K, seed=1).to(gpu), _r(N, K, seed=2).to(gpu), _r(M, N, seed=3).to(gpu)
+    x[0] *= 1e-20                                     # products of denormal size
+    w[N // 2] *= 1e-20
+    out = torch.full((M, N), float("nan"), device=gpu)
+    ops.gemm(x, w, out)
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + K * 2.0 ** -149    # any order of K additions
+    assert ((out.double() - x.double() @ w.double().T).abs() <= bound).all()
+    off = torch.empty(M * K + 1, device=gpu)[1:].view(M, K)
+    off.copy_(x)
+    general = torch.empty(M, N, device=gpu)
+    ops.gemm(off, w, general)
+    assert torch.equal(out, general)
+    acc = y0.clone()
+    ops.gemm(x, w, acc, accumulate=True)
+    assert torch.equal(acc, y0 + out)
+    for m in (1, 16, 17, 64, 65):                     # a row does not depend on the other rows of the call
+        if m < M:
+            some = torch.empty(m, N, device=gpu)
+            ops.gemm(x[M - m:], w, some)
+            assert torch.equal(some, out[M - m:]), m
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 8), (5, 1000, 96), (17, 33, 40), (64, 777, 240), (65, 130, 136),
                                    (200, 300, 328), (300, 64, 2048), (128, 128, 64), (2, 2048, 8192),
                                    (72, 2048, 8192), (512, 2050, 2048), (130, 1026, 1000),

@@ -62,6 +62,27 @@ __device__ __forceinline__ void static_for(F&& f) {
     }
 }
 
+// Memory straight into LDS through a buffer: lane l's 16 bytes at `offset` bytes (a lane's) + `scalar` bytes (the wave's)
+// of the buffer go to lds + 16 l.  Bytes beyond the buffer read as zero and are not fetched.  A buffer load and not a global
+// one: behind a global load into LDS the compiler no longer knows which counter stands for what, and waits for every read
+// of LDS under way whenever it needs one of them.
+typedef __amdgpu_buffer_rsrc_t buffer_t;
+__device__ __forceinline__ buffer_t make_buffer(const void* base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)base, 0, bytes, 0x00027000);
+}
+__device__ __forceinline__ void load_to_lds(buffer_t buf, void* lds, int offset, int scalar) {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(buf, (__attribute__((address_space(3))) void*)lds, 16, offset, scalar, 0, 0);
+#endif
+}
+
+// s_waitcnt vmcnt(VM) lgkmcnt(0)
+template <int VM>
+__device__ __forceinline__ void wait_loads_and_lds() {
+    static_assert(VM >= 0 && VM < 64, "vmcnt has six bits");
+    __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | 0x0070);
+}
+
 static inline int launch_status() { return (int)hipGetLastError(); }
 
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }

@@ -292,12 +292,6 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_tiled_kernel
 // 35.1 -> 27.4, 2048 x 8192 102.7 -> 81.3, 16384 x 2048 157.6 -> 148.6, 6144 x 2048 69.0 -> 61.2.
 // With all CUs busy and random operands the clock, not the instruction stream, sets the pace: the
 // same loop over constant data runs a quarter faster.
-template <int VM>
-__device__ __forceinline__ void wait_loads_and_lds() {               // s_waitcnt vmcnt(VM) lgkmcnt(0)
-    static_assert(VM >= 0 && VM < 64, "vmcnt has six bits");
-    __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | 0x0070);
-}
-
 template <int TM, int TN, int WAVES_M, int WAVES_N, int STAGES, int MODE, int AROUND>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* __restrict__ Y, int M, int N, int K,
