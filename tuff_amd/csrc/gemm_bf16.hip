@@ -281,7 +281,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_tiled_kernel
             store_quad<MODE>(Y, m0 + wm + i * 16 + r16, n0 + wn + j * 16 + g * 4, M, N, acc[i][j]);
 }
 
-// The same product with the operands going from memory straight into LDS (global_load_lds_dwordx4),
+// The same product with the operands going from memory straight into LDS (load_to_lds),
 // without a stop in registers; used where K is a multiple of 64.  A wave's load instruction fills
 // 1 KB of LDS, lane l the 16 bytes at 16 l.  X keeps the swizzled row-major layout above: an
 // instruction covers eight rows of 128 bytes, and the lane that fills chunk position p of row r
@@ -304,7 +304,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     extern __shared__ __attribute__((aligned(16))) bf16_t tiles[];       // [STAGES][BM * TBK] of X then [STAGES][BN * TBK] of W
     bf16_t* As = tiles;
     bf16_t* Bs = tiles + STAGES * BM * TBK;
-    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int wm = (wave / WAVES_N) * 16 * TM, wn = (wave % WAVES_N) * 16 * TN;
     const int r16 = lane % 16, g = lane / 16;
     const long long m0 = (long long)blockIdx.y * BM, n0 = (long long)blockIdx.x * BN;
@@ -316,34 +316,29 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int kb = K / 32;
-    const bf16_t* Xb = X + m0 * K;
-    const bf16_t* Wb = W + (n0 / 16) * (long long)kb * 512;
     const int last_a = (int)min((long long)BM - 1, (long long)M - 1 - m0);
     const int last_tile = (int)min((long long)BN / 16 - 1, (N - 1 - n0) / 16);
-    // instruction q of X (q = wave + NW i) fills rows 8 q .. 8 q + 7; instruction q of W fills block q % 2 of row tile q / 2
-    unsigned offa[IA], offb[IB];
+    // instruction q of X (q = wave + NW i) fills rows 8 q .. 8 q + 7; instruction q of W fills block q % 2 of row tile q / 2;
+    // offsets in bytes from the block's first row (tile), rows beyond the matrix read its last one
+    int offa[IA], offb[IB];
 #pragma unroll
     for (int i = 0; i < IA; ++i)
-        offa[i] = (unsigned)min((wave + NW * i) * 8 + lane / 8, last_a) * (unsigned)K + (((lane % 8) ^ (lane / 8)) * 8);
+        offa[i] = (min((wave + NW * i) * 8 + lane / 8, last_a) * K + (((lane % 8) ^ (lane / 8)) * 8)) * 2;
 #pragma unroll
     for (int i = 0; i < IB; ++i) {
         const int q = wave + NW * i;
-        offb[i] = ((unsigned)min(q / 2, last_tile) * (unsigned)kb + q % 2) * 512u + lane * 8;
+        offb[i] = (min(q / 2, last_tile) * kb + q % 2) * 1024 + lane * 16;
     }
+    const buffer_t xbuf = make_buffer(X + m0 * K, (last_a + 1) * K * 2);
+    const buffer_t wbuf = make_buffer(W + (n0 / 16) * (long long)kb * 512, (last_tile + 1) * kb * 1024);
     const int nk = K / TBK;
     const int kt_begin = blockIdx.z * steps_per_slice, kt_end = min(nk, kt_begin + steps_per_slice);
 
     auto issue = [&](int buf, int kt) {
-        const bf16_t* xs = Xb + kt * TBK;
-        const bf16_t* wsrc = Wb + (unsigned)(kt * 2) * 512u;
 #pragma unroll
-        for (int i = 0; i < IA; ++i)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xs + offa[i]),
-                                             (__attribute__((address_space(3))) void*)(As + buf * BM * TBK + (wave + NW * i) * 512), 16, 0, 0);
+        for (int i = 0; i < IA; ++i) load_to_lds(xbuf, As + buf * BM * TBK + (wave + NW * i) * 512, offa[i], kt * (TBK * 2));
 #pragma unroll
-        for (int i = 0; i < IB; ++i)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wsrc + offb[i]),
-                                             (__attribute__((address_space(3))) void*)(Bs + buf * BN * TBK + (wave + NW * i) * 512), 16, 0, 0);
+        for (int i = 0; i < IB; ++i) load_to_lds(wbuf, Bs + buf * BN * TBK + (wave + NW * i) * 512, offb[i], kt * 2048);
     };
     const int fa0 = swz(wm + r16, g), fa1 = swz(wm + r16, 4 + g);
     const int fb = (wn / 16) * 1024 + lane * 8;                        // block h of MFMA tile j: + (2 j + h) * 512
@@ -387,14 +382,17 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     // Step kt lives in buffer (kt - kt_begin) % STAGES.  Before step kt is multiplied the loads of
     // steps kt .. kt + STAGES - 2 are under way; a wave waits until all but those of the later steps
     // have landed, the barrier then says the same of everybody's and that nobody reads the buffer
-    // of step kt - 1 any more, which the loads of step kt + STAGES - 1 go into.
+    // of step kt - 1 any more, which the loads of step kt + STAGES - 1 go into.  Two loops, of the steps with loads to issue
+    // and of the last ones, with no branch inside: with the loads through buffers (load_to_lds) the compiler then counts the
+    // fragment reads under way and waits for the ones it needs, where it waited for all of them, those just issued among
+    // them, before every group of MFMAs.
     static_for<STAGES - 1>([&](auto s) {
         constexpr int st = decltype(s)::value;
         if (kt_begin + st < kt_end) issue(st, kt_begin + st);
     });
     // TILED_SCALED: the sum of squares of each of the block's rows, in SS_PARTS parts: thread (part, row) adds the groups
     // part, part + SS_PARTS, ... in that order, sixteen loads at a time (one after the other would be as many trips to
-    // memory: a product of few rows leaves 256 groups for 2,048 columns); behind the first barrier of the loop the parts
+    // memory: a product of few rows leaves 256 groups for 2,048 columns); behind the loop the parts
     // of a row are added in their order and the row's scale is left for the epilogue.  (Up to sixteen groups, as the
     // tiled products of a prompt leave them: one thread a row, the scale at once.)
     constexpr int SS_PARTS = (64 * NW) / BM >= 4 ? 4 : (64 * NW) / BM >= 2 ? 2 : 1;
@@ -434,36 +432,32 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         }
         // read in the epilogue, behind the barriers of the loop (every wave waits for its LDS writes before each)
     }
-    for (int kt0 = kt_begin; kt0 < kt_end; kt0 += STAGES) {
-        static_for<STAGES>([&](auto u) {
-            constexpr int buf = decltype(u)::value;
-            const int kt = kt0 + buf;
-            if (kt < kt_end) {
-                const int later = min(STAGES - 2, kt_end - 1 - kt);      // steps after kt whose loads are under way
-                bool waited = false;
-                static_for<STAGES - 1>([&](auto l) {
-                    constexpr int n = decltype(l)::value;
-                    if (!waited && later == n) { wait_loads_and_lds<n * (IA + IB)>(); waited = true; }
-                });
-                __builtin_amdgcn_s_barrier();
-                if (kt + STAGES - 1 < kt_end) issue((buf + STAGES - 1) % STAGES, kt + STAGES - 1);
-                if constexpr (AROUND == TILED_SCALED) {
-                    if (kt == kt_begin && ex.n_ss > 16 && tid < BM && gridDim.z == 1) {
-                        float t = row_ss[0][tid];
-#pragma unroll
-                        for (int q = 1; q < SS_PARTS; ++q) t += row_ss[q][tid];
-                        row_scale[tid] = 1.0f / sqrtf(t / (float)K + ex.eps);
-                    }
-                }
-                read_half(S0(), buf, S0());
-                mult(S1());                                            // the second half of the step before (zeros at first)
-                spread();
-                read_half(S1(), buf, S1());
-                mult(S0());
-                spread();
-            }
-        });
+    auto products = [&](int buf) {
+        read_half(S0(), buf, S0());
+        mult(S1());                                            // the second half of the step before (zeros at first)
+        spread();
+        read_half(S1(), buf, S1());
+        mult(S0());
+        spread();
+    };
+    int buf = 0, kt = kt_begin;
+    for (; kt + STAGES - 1 < kt_end; ++kt) {
+        wait_loads_and_lds<(STAGES - 2) * (IA + IB)>();
+        __builtin_amdgcn_s_barrier();
+        issue(buf == 0 ? STAGES - 1 : buf - 1, kt + STAGES - 1);
+        products(buf);
+        buf = buf + 1 == STAGES ? 0 : buf + 1;
     }
+    static_for<STAGES - 1>([&](auto i) {                       // the last STAGES - 1 steps, fewer if there are fewer
+        constexpr int later = STAGES - 2 - decltype(i)::value;
+        if (kt < kt_end - later) {
+            wait_loads_and_lds<later * (IA + IB)>();
+            __builtin_amdgcn_s_barrier();
+            products(buf);
+            buf = buf + 1 == STAGES ? 0 : buf + 1;
+            ++kt;
+        }
+    });
     if (kt_begin < kt_end) mult(S1());
 
     if (gridDim.z > 1) {
@@ -476,7 +470,15 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         return;
     }
     if constexpr (AROUND == TILED_SCALED) {
-        if (kt_end - kt_begin < 2) __syncthreads();        // a single step: no barrier has followed the scales yet
+        if (ex.n_ss > 16) {                                    // (the parts were written before the loop's first barrier)
+            if (tid < BM) {
+                float t = row_ss[0][tid];
+#pragma unroll
+                for (int q = 1; q < SS_PARTS; ++q) t += row_ss[q][tid];
+                row_scale[tid] = 1.0f / sqrtf(t / (float)K + ex.eps);
+            }
+            __syncthreads();
+        }
     }
     if constexpr (AROUND == TILED_EMIT) {
         // whole blocks of columns only (the host sees to it): Y += acc, the next norm's operand, the row's sum of squares

@@ -183,12 +183,16 @@ __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(co
         products(buf);
         buf = buf + 1 == STAGES ? 0 : buf + 1;
     }
-    for (; s < steps; ++s) {
-        wait_loads_and_lds<0>();
-        if (WAVES > 1) __builtin_amdgcn_s_barrier();
-        products(buf);
-        buf = buf + 1 == STAGES ? 0 : buf + 1;
-    }
+    static_for<STAGES - 1>([&](auto i) {                  // the last STAGES - 1 steps, fewer if there are fewer
+        constexpr int later = STAGES - 2 - decltype(i)::value;
+        if (s < steps - later) {
+            wait_loads_and_lds<2 * IN * later>();
+            if (WAVES > 1) __builtin_amdgcn_s_barrier();
+            products(buf);
+            buf = buf + 1 == STAGES ? 0 : buf + 1;
+            ++s;
+        }
+    });
     multiply(H1());
 #pragma unroll
     for (int i = 0; i < T; ++i) {
