@@ -76,6 +76,17 @@ __device__ __forceinline__ void load_to_lds(buffer_t buf, void* lds, int offset,
 #endif
 }
 
+// An offset that lies beyond every buffer, also with a wave's scalar offset added: the lane reads zero.
+constexpr int NOWHERE = (int)0x80000000;
+// 16 bytes, or one float, at `offset` (a lane's) + `scalar` (the wave's) bytes of the buffer.  STREAMING: read once and never again.
+template <bool STREAMING>
+__device__ __forceinline__ bf16x8 load_buffer(buffer_t buf, int offset, int scalar) {
+    return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(buf, offset, scalar, STREAMING ? 2 : 0));
+}
+__device__ __forceinline__ float load_buffer_float(buffer_t buf, int offset, int scalar) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buf, offset, scalar, 0));
+}
+
 // s_waitcnt vmcnt(VM) lgkmcnt(0)
 template <int VM>
 __device__ __forceinline__ void wait_loads_and_lds() {

@@ -578,8 +578,12 @@ struct ConvTail {
 // in memory (SS_ROWS), as for every product of 17 to 64 rows.
 constexpr int SS_ROWS_WIDE = 64;
 
+// Waves a SIMD has to hold.  Eight waves over 32 columns: two workgroups a CU (at most 128 registers a lane), so that the 512
+// workgroups of 16,384 columns run side by side and not in two rounds.
+constexpr int skinny16_waves_a_simd(int NW, int COLS, int MT) { return NW == 8 && COLS == 32 && MT == 1 ? 4 : 1; }
+
 template <int NW, int MODE, int NORM, bool EMIT, int COLS, int MT>
-__global__ __launch_bounds__(NW * WAVE) void gemm_bf16_skinny16_kernel(const void* __restrict__ Xv, const bf16_t* __restrict__ W,
+__global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) void gemm_bf16_skinny16_kernel(const void* __restrict__ Xv, const bf16_t* __restrict__ W,
                                                                        void* __restrict__ Y, int M, int N, int K,
                                                                        const float* __restrict__ norm_w, float eps,
                                                                        const int* __restrict__ rows, long long ldx,
@@ -599,20 +603,21 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_skinny16_kernel(const voi
     __shared__ float red[MT][TN][NW][WAVE][4];
     __shared__ float ssq[16][ROWS];                                      // [wave or part][row]
     extern __shared__ __attribute__((aligned(16))) float nw_lds[];       // NORM_INSIDE: the norm weight, K floats
-    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int r16 = lane % 16, g = lane / 16;
     // OUT_CONV: workgroup b takes the channels 8 b .. 8 b + 7: half (b % 2) of the three row tiles of group b / 2
     const long long n0 = CONV ? (long long)(blockIdx.x / 2) * 48 + (blockIdx.x % 2) * 8 : (long long)blockIdx.x * COLS;
     const int nchunks = (K + SK_CHUNK - 1) / SK_CHUNK;
-    const bf16_t* X = (const bf16_t*)Xv;
     const long long w_rows = min((long long)N, n0 + COLS);               // this tile's rows of W end here
     // tile-major W: this lane's piece of a block; a workgroup of 8 columns owns half a row tile
     const int kb = (K + 31) / 32, n_tiles16 = (N + 15) / 16;
     const long long tile0 = n0 / 16;
     const int wpiece = COLS == 8 ? g * 16 + (int)(n0 % 16) + r16 : lane;
     const bool wlane = COLS == 8 ? r16 < 8 : true;
-    const float* xrow = nullptr;
-    if (NORM == NORM_INSIDE && r16 < M) xrow = (const float*)Xv + (long long)(rows ? rows[r16] : r16) * ldx;
+    // NORM_INSIDE: this lane's row of x; a lane without one reads row 0 and its values count as zero
+    const bool xlane = r16 < M;
+    const int xr = NORM == NORM_INSIDE && xlane ? (rows ? rows[r16] : r16) : 0;
+    const float* xrow = (const float*)Xv + (NORM == NORM_INSIDE ? (long long)xr * ldx : 0);
 
     // What the epilogue adds to is read now, not after the last product: a load at the end would
     // cost one more trip to memory.  (Thread t of every 256 -> element (row (t / 64) * 4 + t % 4,
@@ -637,11 +642,12 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_skinny16_kernel(const voi
         }
     }
 
-    // OUT_CONV: likewise the rows of the state and the taps that the convolution reads (slot -> state: two trips to
-    // memory one after the other, which now run beside the product instead of behind it); the first CONV_AHEAD rows of the
-    // state, which is all of them up to a kernel length of CONV_AHEAD + 1, and the last tap.
+    // OUT_CONV: likewise the taps and the rows of the state that the convolution reads: the first CONV_AHEAD rows, which is
+    // all of them up to a kernel length of CONV_AHEAD + 1, and the last tap.  Slot -> state are two trips to memory one after
+    // the other: the slot is asked for before the first operands of the product and the state's rows behind them.
     constexpr int CONV_AHEAD = 4;
     float st_ahead[CONV ? EPI_TILES : 1][CONV_AHEAD], tap_ahead[CONV ? EPI_TILES : 1][CONV_AHEAD + 1];
+    int slot_ahead[CONV ? EPI_TILES : 1];
     if constexpr (CONV) {
 #pragma unroll
         for (int i = 0; i < EPI_TILES; ++i) {
@@ -649,13 +655,11 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_skinny16_kernel(const voi
             const int row = mt * 16 + (l / 16) * 4 + t % 4, ch = (int)blockIdx.x * 8 + (l % 16), d = N / 3, Kc = cv.taps;
 #pragma unroll
             for (int k = 0; k <= CONV_AHEAD; ++k) tap_ahead[i][k] = 0.f;
-#pragma unroll
-            for (int k = 0; k < CONV_AHEAD; ++k) st_ahead[i][k] = 0.f;
+            slot_ahead[i] = cv.state_slot[min(row, M - 1)];
             if (mt < MT && (l % 16) < 8 && row < M && ch < d) {
-                const float* st = cv.state + (long long)cv.state_slot[row] * (Kc - 1) * d;
 #pragma unroll
                 for (int k = 0; k < CONV_AHEAD; ++k)
-                    if (k < Kc - 1) { st_ahead[i][k] = st[(long long)k * d + ch]; tap_ahead[i][k] = cv.tap(ch, k); }
+                    if (k < Kc - 1) tap_ahead[i][k] = cv.tap(ch, k);
                 tap_ahead[i][CONV_AHEAD] = cv.tap(ch, Kc - 1);
             }
         }
@@ -669,26 +673,31 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_skinny16_kernel(const voi
     float ss = 0.f;
     struct Operands { bf16x8 a[MT][4]; bf16x8 b[TN][4]; f32x4 x[NORM == NORM_INSIDE ? 4 : 1][2]; };
     Operands o0, o1;
+    // The operands come through buffer loads; an offset beyond the buffer, for rows, columns and k that are not
+    // there, reads as zero and fetches nothing.  With no branch around a load the compiler counts the loads under way and
+    // waits for a chunk's own while the next one's are on their way; with the loads under conditions it waited for all.
+    const buffer_t wbuf = make_buffer(W + tile0 * kb * 512, (int)min((long long)TN, n_tiles16 - tile0) * kb * 1024);
+    const buffer_t xbuf = make_buffer(Xv, NORM == NORM_INSIDE ? 0 : M * K * 2);
+    const int w_at = wlane ? wpiece * 16 : NOWHERE;
     auto load = [&](int c, Operands& o) {
         // instruction j of the wave reads block 4 c + j of its row tile (1 KB) and bytes 64 j .. 64 j + 63 of
         // the chunk of each of the rows of X
-        const int k0 = c * SK_CHUNK + g * 8;
-        const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                o.b[tn][j] = (wlane && tile0 + tn < n_tiles16 && c * 4 + j < kb) ? load_w(W, tile0 + tn, kb, c * 4 + j, wpiece) : z;
+                o.b[tn][j] = load_buffer<true>(wbuf, c * 4 + j < kb ? w_at : NOWHERE, (tn * kb + c * 4 + j) * 1024);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int k = k0 + j * 32;
+            const int kj = c * SK_CHUNK + j * 32 + g * 8;
             if (NORM == NORM_INSIDE) {
-                const bool ok = xrow != nullptr && k < K;
-                o.x[j][0] = ok ? *(const f32x4*)(xrow + k) : f32x4{0.f, 0.f, 0.f, 0.f};
-                o.x[j][1] = ok ? *(const f32x4*)(xrow + k + 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+                const float* xp = xrow + min(kj, K - 8);
+                o.x[j][0] = *(const f32x4*)xp;
+                o.x[j][1] = *(const f32x4*)(xp + 4);
             } else {
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) o.a[mt][j] = load8(X, mt * 16 + r16, M, k, K);
+                for (int mt = 0; mt < MT; ++mt)
+                    o.a[mt][j] = load_buffer<false>(xbuf, kj < K ? ((mt * 16 + r16) * K + g * 8) * 2 : NOWHERE, (c * SK_CHUNK + j * 32) * 2);
             }
         }
     };
@@ -697,11 +706,12 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_skinny16_kernel(const voi
             const int k0 = c * SK_CHUNK + g * 8;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int k = min(k0 + j * 32, K - 8);               // past the end x is zero anyway
+                const int k = min(k0 + j * 32, K - 8);
+                const bool in = xlane && k0 + j * 32 < K;
                 const f32x4 w0 = *(const f32x4*)(&nw_lds[k]), w1 = *(const f32x4*)(&nw_lds[k + 4]);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float x0 = o.x[j][0][e], x1 = o.x[j][1][e];
+                    const float x0 = in ? o.x[j][0][e] : 0.f, x1 = in ? o.x[j][1][e] : 0.f;
                     ss = fmaf(x0, x0, ss);
                     ss = fmaf(x1, x1, ss);
                     o.a[0][j][e] = (bf16_t)(x0 * w0[e]);
@@ -720,38 +730,72 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_skinny16_kernel(const voi
     // the chip reads from all columns of W and not from one.  The order of a tile's additions
     // still depends on N and K only.
     const int rot = (int)((blockIdx.x * 5u) % (unsigned)nchunks);
-    auto chunk_of = [&](int i) { int c = i + rot; return c >= nchunks ? c - nchunks : c; };
-    int i = wave;
-    if (i < nchunks) load(chunk_of(i), o0);
-    if (NORM == NORM_INSIDE) {
-        // the norm weight goes to LDS while the first operands are on their way from HBM
-        for (int k = tid * 4; k < K; k += NW * WAVE * 4) *(f32x4*)(&nw_lds[k]) = *(const f32x4*)(norm_w + k);
-        __syncthreads();
-    }
+    auto chunk_of = [&](int i) { const int c = i + rot; return c >= nchunks ? c - nchunks : c; };
     // NORM_SCALED: 16 parts x ROWS rows; part p adds the tiles p, p + 16, ... of its row.  The first
     // sixteen of them are only asked for here and added after the products, when they have long
     // arrived; a wider matrix adds the rest right away.
     float ss_part[PAIRS][16], ss_rest[PAIRS];
+    const buffer_t sbuf = make_buffer(ss_in, NORM == NORM_SCALED ? n_ss * SSR * 4 : 0);
     if (NORM == NORM_SCALED) {
 #pragma unroll
         for (int q = 0; q < PAIRS; ++q) {
             const int pr = tid + q * NT_;
-            const int row = pr % ROWS, part = pr / ROWS;
             ss_rest[q] = 0.f;
-            if (pr < 16 * ROWS) {
-#pragma unroll
-                for (int u = 0; u < 16; ++u) ss_part[q][u] = (part + 16 * u < n_ss) ? ss_in[(long long)(part + 16 * u) * SSR + row] : 0.f;
-                for (int j = part + 256; j < n_ss; j += 16) ss_rest[q] += ss_in[(long long)j * SSR + row];
-            }
+            if (n_ss > 256 && pr < 16 * ROWS)
+                for (int j = pr / ROWS + 256; j < n_ss; j += 16) ss_rest[q] += ss_in[(long long)j * SSR + pr % ROWS];
         }
     }
-    for (; i < nchunks; i += 2 * NW) {
-        const bool more = i + NW < nchunks;
-        if (more) load(chunk_of(i + NW), o1);
-        multiply(chunk_of(i), o0);
-        if (more) {
-            if (i + 2 * NW < nchunks) load(chunk_of(i + 2 * NW), o0);
-            multiply(chunk_of(i + NW), o1);
+    // What is asked for behind the first operands.
+    auto behind = [&]() {
+        if (NORM == NORM_SCALED) {
+#pragma unroll
+            for (int q = 0; q < PAIRS; ++q) {
+                const int pr = tid + q * NT_;
+#pragma unroll
+                for (int u = 0; u < 16; ++u)
+                    ss_part[q][u] = load_buffer_float(sbuf, pr < 16 * ROWS ? (pr / ROWS * SSR + pr % ROWS) * 4 : NOWHERE, u * 16 * SSR * 4);
+            }
+        }
+        if constexpr (CONV) {
+#pragma unroll
+            for (int i = 0; i < EPI_TILES; ++i) {
+                const int t = tid % 256, l = t / 4, ch = (int)blockIdx.x * 8 + (l % 16), d = N / 3, Kc = cv.taps;
+                const float* st = cv.state + (long long)slot_ahead[i] * (Kc - 1) * d + min(ch, d - 1);
+#pragma unroll
+                for (int k = 0; k < CONV_AHEAD; ++k) st_ahead[i][k] = st[(long long)min(k, Kc - 2) * d];
+            }
+        }
+        if (NORM == NORM_INSIDE) {
+            // the norm weight goes to LDS while the first operands are on their way from HBM
+            for (int k = tid * 4; k < K; k += NW * WAVE * 4) *(f32x4*)(&nw_lds[k]) = *(const f32x4*)(norm_w + k);
+            __syncthreads();
+        }
+    };
+    // The wave's chunks, two sets of operands in turn; every way through has its loads and products in straight order.
+    const int n = (nchunks - wave + NW - 1) / NW;
+    auto nth = [&](int i) { return chunk_of(wave + i * NW); };
+    if (n < 2) {
+        if (n == 1) load(nth(0), o0);
+        behind();
+        if (n == 1) multiply(nth(0), o0);
+    } else {
+        load(nth(0), o0);
+        load(nth(1), o1);
+        behind();
+        int i = 0;
+        for (; i + 3 < n; i += 2) {
+            multiply(nth(i), o0);
+            load(nth(i + 2), o0);
+            multiply(nth(i + 1), o1);
+            load(nth(i + 3), o1);
+        }
+        multiply(nth(i), o0);
+        if (i + 2 < n) {
+            load(nth(i + 2), o0);
+            multiply(nth(i + 1), o1);
+            multiply(nth(i + 2), o0);
+        } else {
+            multiply(nth(i + 1), o1);
         }
     }
 #pragma unroll
@@ -813,7 +857,7 @@ __global__ __launch_bounds__(NW * WAVE) void gemm_bf16_skinny16_kernel(const voi
                 float sv[CONV_MAX_TAPS], wv[CONV_MAX_TAPS];
 #pragma unroll
                 for (int k = 0; k < CONV_MAX_TAPS; ++k) {
-                    if (k < CONV_AHEAD) { sv[k] = st_ahead[ei][k]; wv[k] = tap_ahead[ei][k]; continue; }   // (zero beyond Kc - 1)
+                    if (k < CONV_AHEAD) { sv[k] = st_ahead[ei][k]; wv[k] = tap_ahead[ei][k]; continue; }   // (not used beyond Kc - 1)
                     sv[k] = k < Kc - 1 ? st[(long long)k * d + ch] : 0.f;
                     wv[k] = k < Kc - 1 ? cv.tap(ch, k) : 0.f;
                 }
