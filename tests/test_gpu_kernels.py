@@ -1449,3 +1449,39 @@ def test_repeat_penalty(gpu):
     ops.repeat_penalty(g, recent.to(gpu), torch.tensor([3, 2], dtype=torch.int32, device=gpu),
                        torch.tensor([2.0, 1.0], device=gpu))
     assert g.cpu().tolist() == [[0.5, -4.0, 1.0, 4.0], [2.0, -2.0, 1.0, 4.0]]
+
+
+@pytest.mark.parametrize("H,Hkv,hd,page,window", [(4, 2, 16, 16, 0), (6, 2, 32, 32, 40), (32, 8, 64, 16, 0), (8, 8, 64, 48, 0),
+                                                   (16, 1, 64, 16, 100), (10, 2, 128, 16, 0)])
+def test_attention_f32_gives_the_bits_of_the_general_kernel(gpu, H, Hkv, hd, page, window):
+    """Requests of one token and of portions, at the borders of the tiles of 64 keys; pages nobody wrote, and those a window
+    has passed, hold NaN; one value is infinite."""
+    from tuff_amd.csrc import ops
+    before, new = [0, 63, 64, 130, 5, 200, 0], [1, 1, 1, 1, 64, 37, 131]
+    R, T, total = len(new), sum(new), [b + n for b, n in zip(before, new)]
+    blocks = [-(-t // page) for t in total]
+    g = torch.Generator().manual_seed(hd + H)
+    order = torch.randperm(sum(blocks), generator=g).tolist()
+    table = torch.full((R, max(blocks)), -1, dtype=torch.int32)
+    k = torch.full((sum(blocks), Hkv, page, hd), float("nan"))
+    v = torch.full((sum(blocks), Hkv, hd, page), float("nan"))
+    for r in range(R):
+        for b in range(blocks[r]):
+            n = min(page, total[r] - b * page)
+            if window and (b + 1) * page <= before[r] - window + 1:
+                order.pop()                               # (the window has passed this page)
+                continue
+            table[r, b] = p = order.pop()
+            k[p, :, :n] = torch.randn(Hkv, n, hd, generator=g)
+            v[p, :, :, :n] = torch.randn(Hkv, hd, n, generator=g)
+    v[int(table[6, 40 // page]), 0, 3, 40 % page] = float("inf")
+    starts = np.concatenate([[0], np.cumsum(new)[:-1]])
+    info = torch.tensor([[int(s), n, b, t] for s, n, b, t in zip(starts, new, before, total)], dtype=torch.int32)
+    q = torch.randn(T, H * hd, generator=g) * 3
+    kw = dict(block_table=table.to(gpu), H=H, Hkv=Hkv, hd=hd, page_size=page, window=window)
+    want, got = torch.empty(T, H * hd, device=gpu), torch.full((T, H * hd), float("nan"), device=gpu)
+    ops.attention_general(q.to(gpu), k.to(gpu), v.to(gpu), want, req_of_token=torch.tensor(np.repeat(np.arange(R), new), dtype=torch.int32, device=gpu),
+                          positions=torch.tensor(np.concatenate([np.arange(b, t) for b, t in zip(before, total)]), dtype=torch.int32, device=gpu), **kw)
+    ops.attention_f32(q.to(gpu), k.to(gpu), v.to(gpu), got, req_info=info.to(gpu), max_q_len=max(new), **kw)
+    assert torch.isfinite(want[:int(starts[6]) + 40]).all()
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))

@@ -108,6 +108,8 @@ _SIGNATURES = {
                           _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     },
     "attention": {
+        "tuff_attention_f32": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int,
+                               _c_int, _c_int, _c_int, _c_int, _c_float, _c_void_p],
         "tuff_attention_general": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int,
                                    _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                    _c_float, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p],
@@ -979,6 +981,31 @@ def attention_general(q, k_cache, v_cache, out, *, block_table, req_of_token, po
         None if slopes is None else slopes.data_ptr(), int(v_cache is None),
         None if r1 is None else r1.data_ptr(), None if r2 is None else r2.data_ptr(), int(all_values),
         int(keep_first) if window else 0, int(maps), int(maps > 1 and out.dtype == torch.float32), _stream()), "attention_general")
+
+
+def attention_f32_supported(dtype, H: int, Hkv: int, hd: int, page_size: int) -> bool:
+    """Whether attention_f32 takes these heads (it forms attention_general's sums, bit for bit)."""
+    return dtype == torch.float32 and hd in (16, 32, 64, 128) and H % Hkv == 0 and H // Hkv <= 16 and page_size % 16 == 0
+
+
+def attention_f32(q, k_cache, v_cache, out, *, block_table, req_info, max_q_len, H, Hkv, hd, page_size, window=0, scale=None) -> None:
+    """attention_general on the matrix cores, the same bits: float32, values as wide as keys, no sinks and slopes.
+    req_info int32 [R, 4]: (first token, tokens, position of the first token, length); max_q_len: the most tokens of a request."""
+    T, R, P = q.shape[0], req_info.shape[0], k_cache.shape[0]
+    if not attention_f32_supported(q.dtype, H, Hkv, hd, page_size):
+        raise KernelError(f"attention_f32: {q.dtype}, heads {H}:{Hkv} of {hd}, pages of {page_size} are not supported")
+    _gpu("q", q, shape=(T, H * hd))
+    _gpu("out", out, torch.float32, (T, H * hd))
+    _gpu("k_cache", k_cache, torch.float32, (P, Hkv, page_size, hd))
+    _gpu("v_cache", v_cache, torch.float32, (P, Hkv, hd, page_size))
+    _gpu("block_table", block_table, torch.int32)
+    _gpu("req_info", req_info, torch.int32, (R, 4))
+    if block_table.dim() != 2 or block_table.shape[0] < R:
+        raise KernelError("attention: block_table must be [requests, blocks]")
+    _check(load("attention").tuff_attention_f32(
+        q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(), block_table.data_ptr(), block_table.shape[1],
+        req_info.data_ptr(), R, int(max_q_len), H, Hkv, hd, page_size, int(window or 0),
+        float(1.0 / math.sqrt(hd) if scale is None else scale), _stream()), "attention_f32")
 
 
 def diff_combine(o, out, *, H, vd, combine) -> None:
