@@ -174,9 +174,6 @@ TUFF_EXPORT int tuff_attention_general(const void* q, const void* k_cache, const
 namespace {
 constexpr int F32_COLS = 16;
 
-// A barrier for LDS that lets loads from memory stay under way.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
 template <int HD>
 __global__ __launch_bounds__(256) void attention_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k_cache, const float* __restrict__ v_cache, float* __restrict__ out,

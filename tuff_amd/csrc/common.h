@@ -94,6 +94,9 @@ __device__ __forceinline__ void wait_loads_and_lds() {
     __builtin_amdgcn_s_waitcnt((VM & 15) | ((VM >> 4) << 14) | 0x0070);
 }
 
+// A workgroup's barrier for LDS that lets loads from memory stay under way.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 static inline int launch_status() { return (int)hipGetLastError(); }
 
 static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }

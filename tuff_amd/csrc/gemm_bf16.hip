@@ -926,7 +926,7 @@ __global__ __launch_bounds__(SK_NT) void gemm_bf16_skinny64_kernel(const bf16_t*
     __shared__ __attribute__((aligned(16))) bf16_t xs[2][MT * 16 * XS_STRIDE];
     __shared__ float ss_parts[4][64];
     __shared__ float scale_lds[64];
-    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int r16 = lane % 16, g = lane / 16;
     const int tile = blockIdx.x, slice = blockIdx.y, n_slices = gridDim.y;
     const long long tile16 = (long long)tile * 4 + wave;                 // this wave's row tile of W
@@ -939,16 +939,19 @@ __global__ __launch_bounds__(SK_NT) void gemm_bf16_skinny64_kernel(const bf16_t*
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // X chunk: MT*16 rows x 16 pieces of 16 bytes = MT*256 pieces, MT a thread
-    bf16x8 xr[MT], b0[4], b1[4];
-    auto load_x = [&](int c) {
+    // X chunk: MT*16 rows x 16 pieces of 16 bytes = MT*256 pieces, MT a thread.  Loads through buffers, at an offset beyond them
+    // for what is not there: two chunks' operands are on their way and each is waited for by itself.
+    const buffer_t xbuf = make_buffer(X, M * K * 2);
+    const buffer_t wbuf = make_buffer(W + (tile_ok ? tile16 : 0) * kb * 512, tile_ok ? kb * 1024 : 0);
+    bf16x8 x0[MT], x1[MT], b0[4], b1[4];
+    auto load_x = [&](int c, bf16x8* xr) {
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            const int id = tid + i * SK_NT;
-            xr[i] = load8(X, id / 16, M, c * SK_CHUNK + (id % 16) * 8, K);
+            const int id = tid + i * SK_NT, k = c * SK_CHUNK + (id % 16) * 8;
+            xr[i] = load_buffer<false>(xbuf, c < c_end && k < K ? (id / 16 * K + k) * 2 : NOWHERE, 0);
         }
     };
-    auto store_x = [&](int buf) {
+    auto store_x = [&](int buf, const bf16x8* xr) {
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
             const int id = tid + i * SK_NT;
@@ -956,9 +959,8 @@ __global__ __launch_bounds__(SK_NT) void gemm_bf16_skinny64_kernel(const bf16_t*
         }
     };
     auto load_w4 = [&](int c, bf16x8* b) {
-        const bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = (tile_ok && c * 4 + j < kb) ? load_w(W, tile16, kb, c * 4 + j, lane) : z;
+        for (int j = 0; j < 4; ++j) b[j] = load_buffer<true>(wbuf, c < c_end && c * 4 + j < kb ? lane * 16 : NOWHERE, (c * 4 + j) * 1024);
     };
     auto compute = [&](int buf, const bf16x8* b) {
 #pragma unroll
@@ -971,33 +973,46 @@ __global__ __launch_bounds__(SK_NT) void gemm_bf16_skinny64_kernel(const bf16_t*
     };
 
     if (c_begin < c_end) {
-        load_x(c_begin);
+        load_x(c_begin, x0);
         load_w4(c_begin, b0);
+        load_x(c_begin + 1, x1);
+        load_w4(c_begin + 1, b1);
     }
     if (NORM == NORM_SCALED && !to_ws) {
         // thread -> (row tid % 64, part tid / 64): part p adds the tiles p, p + 4, ... of its row
         float t = 0.f;
         for (int j = tid / 64; j < n_ss; j += 4) t += ss_in[(long long)j * 64 + tid % 64];
         ss_parts[tid / 64][tid % 64] = t;
-    }
-    if (c_begin < c_end) store_x(0);
-    __syncthreads();
-    if (NORM == NORM_SCALED && !to_ws && tid < 64)    // read in the epilogue, behind the barriers of the loop
-        scale_lds[tid] = 1.0f / sqrtf((ss_parts[0][tid] + ss_parts[1][tid] + ss_parts[2][tid] + ss_parts[3][tid]) / (float)K + eps);
-    for (int c = c_begin; c < c_end; c += 2) {
-        // chunk c from buffer 0 / b0, chunk c+1 from buffer 1 / b1
-        const bool more1 = c + 1 < c_end, more2 = c + 2 < c_end;
-        if (more1) { load_x(c + 1); load_w4(c + 1, b1); }
-        compute(0, b0);
-        if (more1) store_x(1);
         __syncthreads();
-        if (more1) {
-            if (more2) { load_x(c + 2); load_w4(c + 2, b0); }
-            compute(1, b1);
-            if (more2) store_x(0);
-            __syncthreads();
-        }
+        if (tid < 64)                                 // read in the epilogue, behind the barriers of the loop
+            scale_lds[tid] = 1.0f / sqrtf((ss_parts[0][tid] + ss_parts[1][tid] + ss_parts[2][tid] + ss_parts[3][tid]) / (float)K + eps);
     }
+    // Chunk c from buffer 0 / b0, chunk c + 1 from buffer 1 / b1.  The barriers wait for LDS only; a buffer is written again
+    // behind the barrier of the chunk after it, which every wave reaches when it has used it.
+    int c = c_begin;
+    for (; c + 2 < c_end; c += 2) {
+        store_x(0, x0);
+        lds_barrier();
+        load_x(c + 2, x0);
+        compute(0, b0);
+        load_w4(c + 2, b0);
+        store_x(1, x1);
+        lds_barrier();
+        load_x(c + 3, x1);
+        compute(1, b1);
+        load_w4(c + 3, b1);
+    }
+    if (c < c_end) {
+        store_x(0, x0);
+        lds_barrier();
+        compute(0, b0);
+    }
+    if (c + 1 < c_end) {
+        store_x(1, x1);
+        lds_barrier();
+        compute(1, b1);
+    }
+    if (NORM == NORM_SCALED && !to_ws) lds_barrier();             // (a slice without a chunk has had no barrier)
 
     const long long col = (long long)tile * 64 + wave * 16 + r16;
     if (to_ws) {
@@ -1221,18 +1236,19 @@ bool rows64_tiled(int M, int N, int K) { return M >= wide64_min_m && M <= 64 && 
 
 // Whether a product of M rows goes through that kernel (else, up to 64 rows: K cut over workgroups and a
 // second kernel that adds the slices).  Up to 16 rows always.  17 to 32 rows: every workgroup reads all M
-// rows of X again, M / (its columns) times the bytes of its share of W, and has half the waves; measured
-// on the shapes of a 1.2B model (against the two kernels of the other way, at 32 rows): 2,048 columns
-// 14.8 us against 11.9, 3,072 columns 8.8 against 10.7, a conv's input projection with the convolution
-// 12.5 against 15.2, 16,384 columns 21.7 against 21.3, 65,536 columns 67.7 against 52.2; at 17 rows
-// it wins everywhere.  So: narrow outputs up to 20 rows, medium ones up to 32, wide ones up to 24 (where the
-// tiled product does not take them, above).
+// rows of X again, M / (its columns) times the bytes of its share of W, and has half the waves.  Measured
+// on the shapes of a 1.2B model (against the two kernels of the other way, at 32 rows): 3,072 columns 8.8 us
+// against 10.7, a conv's input projection with the convolution 12.5 against 15.2, 16,384 columns 21.7 against
+// 21.3, 65,536 columns 67.7 against 52.2, at 17 rows it wins; 2,048 columns of K = 8,192 15.5 against 12.2 at 20
+// rows and 19.8 against 11.5 at 32; of K = 2,048 6.3 against 7.3 at 20 and 7.5 against 7.3 at 32, but it leaves the next
+// norm 256 groups of sums instead of 32, which cost the product after it 1.5 us.  So: narrow outputs never, medium ones up to
+// 32, wide ones up to 24 (where the tiled product does not take them, above).
 bool few_rows_kernel(int M, int N, int K, bool conv = false) {
     if (M <= 16) return true;
     if (M > SKINNY_ROWS) return false;
     if (conv) return true;
     if (rows64_tiled(M, N, K)) return false;
-    return N <= 2048 ? M <= 20 : N <= 8192 ? true : M <= 24;
+    return N <= 2048 ? false : N <= 8192 ? true : M <= 24;
 }
 
 // How a skinny product is cut.  Depends on N and K (and on which of the two kernels M selects).
