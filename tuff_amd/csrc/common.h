@@ -76,7 +76,8 @@ __device__ __forceinline__ void load_to_lds(buffer_t buf, void* lds, int offset,
 #endif
 }
 
-// An offset that lies beyond every buffer, also with a wave's scalar offset added: the lane reads zero.
+// An offset that lies beyond every buffer: the lane reads zero.  (A lane's offset is held against the buffer's size less the
+// wave's scalar offset, so that one must not be larger than the buffer even where no lane reads.)
 constexpr int NOWHERE = (int)0x80000000;
 // 16 bytes, or one float, at `offset` (a lane's) + `scalar` (the wave's) bytes of the buffer.  STREAMING: read once and never again.
 template <bool STREAMING>

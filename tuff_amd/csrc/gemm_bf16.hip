@@ -676,7 +676,8 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
     // The operands come through buffer loads; an offset beyond the buffer, for rows, columns and k that are not
     // there, reads as zero and fetches nothing.  With no branch around a load the compiler counts the loads under way and
     // waits for a chunk's own while the next one's are on their way; with the loads under conditions it waited for all.
-    const buffer_t wbuf = make_buffer(W + tile0 * kb * 512, (int)min((long long)TN, n_tiles16 - tile0) * kb * 1024);
+    const int w_tiles = (int)min((long long)TN, n_tiles16 - tile0);
+    const buffer_t wbuf = make_buffer(W + tile0 * kb * 512, w_tiles * kb * 1024);
     const buffer_t xbuf = make_buffer(Xv, NORM == NORM_INSIDE ? 0 : M * K * 2);
     const int w_at = wlane ? wpiece * 16 : NOWHERE;
     auto load = [&](int c, Operands& o) {
@@ -685,8 +686,10 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                o.b[tn][j] = load_buffer<true>(wbuf, c * 4 + j < kb ? w_at : NOWHERE, (tn * kb + c * 4 + j) * 1024);
+            for (int j = 0; j < 4; ++j) {
+                const bool in = tn < w_tiles && c * 4 + j < kb;
+                o.b[tn][j] = load_buffer<true>(wbuf, in ? w_at : NOWHERE, in ? (tn * kb + c * 4 + j) * 1024 : 0);
+            }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int kj = c * SK_CHUNK + j * 32 + g * 8;
@@ -697,7 +700,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
             } else {
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    o.a[mt][j] = load_buffer<false>(xbuf, kj < K ? ((mt * 16 + r16) * K + g * 8) * 2 : NOWHERE, (c * SK_CHUNK + j * 32) * 2);
+                    o.a[mt][j] = load_buffer<false>(xbuf, kj < K ? ((mt * 16 + r16) * K + g * 8) * 2 : NOWHERE, min(c * SK_CHUNK + j * 32, K - 8) * 2);
             }
         }
     };
@@ -753,7 +756,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
                 const int pr = tid + q * NT_;
 #pragma unroll
                 for (int u = 0; u < 16; ++u)
-                    ss_part[q][u] = load_buffer_float(sbuf, pr < 16 * ROWS ? (pr / ROWS * SSR + pr % ROWS) * 4 : NOWHERE, u * 16 * SSR * 4);
+                    ss_part[q][u] = load_buffer_float(sbuf, pr < 16 * ROWS ? ((pr / ROWS + 16 * u) * SSR + pr % ROWS) * 4 : NOWHERE, 0);
             }
         }
         if constexpr (CONV) {
@@ -960,7 +963,7 @@ __global__ __launch_bounds__(SK_NT) void gemm_bf16_skinny64_kernel(const bf16_t*
     };
     auto load_w4 = [&](int c, bf16x8* b) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = load_buffer<true>(wbuf, c < c_end && c * 4 + j < kb ? lane * 16 : NOWHERE, (c * 4 + j) * 1024);
+        for (int j = 0; j < 4; ++j) b[j] = load_buffer<true>(wbuf, c < c_end && c * 4 + j < kb ? lane * 16 : NOWHERE, c < c_end && c * 4 + j < kb ? (c * 4 + j) * 1024 : 0);
     };
     auto compute = [&](int buf, const bf16x8* b) {
 #pragma unroll
