@@ -922,6 +922,31 @@ def test_attention_long_context(gpu):
         _check_step(case, reqs, out2.cpu().double().reshape(T, H, hd), H, hd, window, ("prefill", window))
 
 
+@pytest.mark.parametrize("hd", [32, 64, 80])
+@pytest.mark.parametrize("window", [0, 3000])
+def test_attention_merge_at_its_edges(gpu, hd, window):
+    """The merge's variants, chosen by the partitions of 256 keys a step has room for: 32 and 33, 64 and 65, and past
+    512, where a wave takes more than one group of 64 partitions.  Each against the plain formula, and with room for
+    156 partitions more to the same bits."""
+    from tuff_amd.csrc import ops
+    H, Hkv, ps = 2, 1, 16
+    for longest in (32 * 256, 33 * 256, 64 * 256, 65 * 256, 512 * 256 + 1, 577 * 256):
+        reqs = [(8000, 1), (longest - 1, 1)]
+        case = _mixed_step_case(gpu, reqs, H, Hkv, hd, ps)
+        out = torch.full((2, H * hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+        blocks = torch.from_numpy(ops.query_blocks(case["q_len"], H // Hkv, 1)).to(gpu)
+        ops.attention_mfma(case["q"].to(gpu), case["kc"], case["vc"], out, block_table=case["table"], blocks=blocks, nb=1,
+                           req_info=case["req_info"], positions=case["positions"], H=H, Hkv=Hkv, hd=hd, page_size=ps,
+                           max_ctx_len=case["max_ctx_len"], window=window)
+        _check_step(case, reqs, out.cpu().double().reshape(2, H, hd), H, hd, window, ("merge", longest, window))
+        more = torch.full_like(out, float("nan"))
+        wide = torch.cat([case["table"], torch.full((2, 40000 // ps), -1, dtype=torch.int32, device=gpu)], dim=1).contiguous()
+        ops.attention_mfma(case["q"].to(gpu), case["kc"], case["vc"], more, block_table=wide, blocks=blocks, nb=1,
+                           req_info=case["req_info"], positions=case["positions"], H=H, Hkv=Hkv, hd=hd, page_size=ps,
+                           max_ctx_len=case["max_ctx_len"] + 40000, window=window)
+        assert torch.equal(out, more), longest
+
+
 @pytest.mark.parametrize("H,Hkv,hd,ps", [(4, 2, 64, 16), (3, 1, 80, 32), (2, 2, 128, 16)])
 @pytest.mark.parametrize("window", [0, 700])
 def test_attention_prefill_key_segments(gpu, H, Hkv, hd, ps, window, monkeypatch):
