@@ -368,6 +368,45 @@ def test_forget_scan_carries_its_state_across_any_cut(gpu):
             assert torch.isnan(state[0]).all() and torch.isnan(state[2]).all()
 
 
+@pytest.mark.parametrize("D", [24, 64, 68, 128, 256])
+def test_scan_gives_the_same_bits_for_any_company_and_alignment(gpu, D):
+    """The recurrence's kernel over nine requests of 0 to 41 tokens (edges of the eight tokens it stages at a time), with
+    heads that do not fill rounds of the chip's eight parts, against each request alone, and with inputs that a wide load
+    cannot fetch: the same bits."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(11)
+    H, lens = 3, [7, 0, 8, 9, 1, 16, 41, 2, 24]
+    T = sum(lens)
+    r, k, v = (torch.randn(T, H * D, generator=gen) for _ in range(3))
+    lw, w0, u = torch.randn(T, H * D, generator=gen), torch.randn(H * D, generator=gen).to(gpu), torch.randn(H, D, generator=gen).to(gpu)
+    state0 = torch.randn(len(lens), H, D, D, generator=gen)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=gpu)
+    starts = [sum(lens[:i]) for i in range(len(lens))]
+
+    def scan(sel, q_start, q_len, slots, shift, dt):
+        def put(t, d):
+            t = t[sel].to(d)
+            room = torch.zeros(t.numel() + shift, dtype=d, device=gpu)
+            room[shift:] = t.flatten().to(gpu)
+            return room[shift:].view(t.shape)
+        state, out = state0.to(gpu), torch.full((len(range(T)[sel]), H * D), float("nan"), device=gpu)
+        ops.wkv_scan(put(r, dt), put(k, dt), put(v, dt), put(lw, torch.float32), w0, u, state, out, q_start=i32(q_start), q_len=i32(q_len),
+                     state_slot=i32(slots), H=H, D=D)
+        return out.cpu(), state.cpu()
+
+    for dt in (torch.bfloat16, torch.float32):
+        out, state = scan(slice(0, T), starts, lens, list(range(len(lens))), 0, dt)
+        assert torch.isfinite(out).all()
+        out1, state1 = scan(slice(0, T), starts, lens, list(range(len(lens))), 1, dt)
+        assert torch.equal(out, out1) and torch.equal(state, state1), "the result depends on the alignment"
+        for i, n in enumerate(lens):
+            if n:
+                alone, s = scan(slice(starts[i], starts[i] + n), [0], [n], [i], 0, dt)
+                assert torch.equal(alone, out[starts[i]:starts[i] + n]) and torch.equal(s[i], state[i]), (dt, i)
+            else:
+                assert torch.equal(state[i], state0[i])
+
+
 # ------------------------------------------------------------------- generation, command line
 def test_greedy_generation_through_the_scheduler(gpu):
     from tuff_amd.engine.llm import LLM

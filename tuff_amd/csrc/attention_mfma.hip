@@ -590,10 +590,6 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
 // both sums over p in ascending order, so the result depends on the token's position only.
 constexpr int COMBINE_MAX_PARTS = 2048;
 
-__device__ __forceinline__ float lane_of(float v, int lane) {
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-
 // Up to 64 partitions: lane p keeps (m_p, l_p) in registers, weights are read out of its lane; no LDS.
 // Same arithmetic as the general kernel below.  PER: channels a lane (head size / 64, rounded up);
 // the partial outputs of BATCH partitions are asked for at once, so that a context of 16,384 positions

@@ -87,6 +87,10 @@ __device__ __forceinline__ bf16x8 load_buffer(buffer_t buf, int offset, int scal
 __device__ __forceinline__ float load_buffer_float(buffer_t buf, int offset, int scalar) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buf, offset, scalar, 0));
 }
+// The value of lane `lane` (the same for the whole wave).
+__device__ __forceinline__ float lane_of(float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
 
 // s_waitcnt vmcnt(VM) lgkmcnt(0)
 template <int VM>

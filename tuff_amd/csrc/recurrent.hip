@@ -456,9 +456,11 @@ struct ScanArgs {
     long long ldv;                  // elements between two tokens' rows of v
     long long lda;                  // elements between two tokens' rows of a and k
     const float* head_bonus;        // ssd: [H], the factor of the token's own value in its output
+    bool by_xcd = false;            // set by the launch
 };
 
-constexpr int SCAN_CH = 8;          // tokens staged at a time
+constexpr int SCAN_CH = 8;          // tokens staged at a time (sixteen: 5 % faster for one long request, but 12 KB of LDS a
+                                    // wave, and 64 single tokens of 32 heads 43 -> 55 us)
 
 // The sum over the SPLIT neighbouring lanes that share a value channel, the same in all of them: exchanges
 // inside a quad (lane ^ 1, then lane ^ 2) and, for 16, rotations by 4 and by 8 within the row of 16 lanes.
@@ -466,38 +468,70 @@ template <int CTRL>
 __device__ __forceinline__ float dpp_of(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
+// group_sums: of several values, step by step side by side.
+template <int SPLIT, int N>
+__device__ __forceinline__ void group_sums(float (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += dpp_of<0xB1>(v[i]);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] += dpp_of<0x4E>(v[i]);
+    if (SPLIT == 16) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] += dpp_of<0x124>(v[i]);
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] += dpp_of<0x128>(v[i]);
+    }
+}
 template <int SPLIT>
 __device__ __forceinline__ float group_sum(float v) {
-    v += dpp_of<0xB1>(v);
-    v += dpp_of<0x4E>(v);
-    if (SPLIT == 16) {
-        v += dpp_of<0x124>(v);
-        v += dpp_of<0x128>(v);
-    }
-    return v;
+    float one[1] = {v};
+    group_sums<SPLIT>(one);
+    return one[0];
 }
 
 // TA: type of a and k (the compute type for wkv's r and k, float for the delta rule's unit vectors); T: type of v.
 // FORGET: a holds silu(q) in float32, the decay is the forget gate f and the key is 1 - f (k and scalar are not used).
 // SSD: S_ij <- w S_ij + (dt k_i) v_j with one decay w for the head, then o_j = sum_i a_i S_ij + bonus_h v_j (the read sees
 // the token's own write); a and k are the convolved rows themselves (C and B of the head's group), of the compute type.
-template <typename TA, typename T, int NI16, int SPLIT, bool DELTA, bool FORGET = false, bool SSD = false>
-__global__ __launch_bounds__(WAVE) void scan_kernel(ScanArgs p) {
+// What bounds it: for one request, the instructions of a wave (a chain over the tokens, a wave a workgroup, two a CU for 16
+// heads of 128 channels).  So: four key channels a load and a staging store; no branch between eight tokens, their rows asked
+// for ahead, their sums over the lanes side by side; and the stores of eight tokens behind the next eight's staging.  One
+// request of 2,048 tokens, 16 heads, 64 key and 128 value channels: 414 -> 217 us.  For many requests, the rows that the
+// blocks of a head all read: by XCD as below, 64 requests of 200 tokens, 16 heads of 128 x 128, 1,281 -> 856 us (forget
+// gate), 2,366 -> 1,053 us (delta rule); without it 1,365 and 2,580.
+template <typename TA, typename T, int NI16, int SPLIT, bool WHOLE, bool DELTA, bool FORGET = false, bool SSD = false>
+__global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_kernel(ScanArgs p) {
     constexpr int RP = NI16 * 4;                       // rows of the state's column a lane keeps
     constexpr int DP = RP * SPLIT;                     // key channels, padded
     constexpr int SCAN_COLS = WAVE / SPLIT;            // value channels a wave
-    constexpr int PER = (DP + WAVE - 1) / WAVE;        // key channels a lane stages
     constexpr int CH = SCAN_CH;
+    constexpr int QUADS = DP / 4;                      // groups of four key channels a token
+    constexpr int PER = (CH * QUADS + WAVE - 1) / WAVE;                  // such groups a lane stages
+    constexpr int PER_V = (CH * SCAN_COLS + WAVE - 1) / WAVE;            // and values
+    typedef TA four __attribute__((ext_vector_type(4)));
     __shared__ __attribute__((aligned(16))) float sa[CH][DP];
     __shared__ __attribute__((aligned(16))) float sk[CH][DP];
-    __shared__ __attribute__((aligned(16))) float sw[CH][DP];
-    const int r = blockIdx.x, head = blockIdx.y, lane = threadIdx.x;
+    __shared__ __attribute__((aligned(16))) float sw[SSD ? 1 : CH][SSD ? 4 : DP];
+    __shared__ __attribute__((aligned(16))) float sv[SCAN_COLS][CH];
+    // The blocks of one (request, head), which all read its rows of a, k and decay, run one after the other on one XCD
+    // (workgroups go round the eight XCDs, each with an L2 of its own): of the pairs that fill rounds of eight, pair i on XCD
+    // i mod 8; the rest in their order.
+    int r = blockIdx.x, head = blockIdx.y, zb = blockIdx.z;
+    const int lane = threadIdx.x;
+    if (p.by_xcd) {
+        const unsigned Z = gridDim.z, id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        const unsigned rounds = gridDim.x * gridDim.y / 8 * 8 * Z;
+        const unsigned pair = id < rounds ? id / 8 / Z * 8 + id % 8 : id / Z;
+        zb = (id < rounds ? id / 8 : id) % Z;
+        r = pair % gridDim.x;
+        head = pair / gridDim.x;
+    }
     const int n = p.q_len[r];
     if (n <= 0) return;
     const int D = p.D, Dv = p.Dv, H = p.H, Ha = p.Ha;
     const int ha = head / (H / Ha);
     const int part = lane % SPLIT;
-    const int j = blockIdx.z * SCAN_COLS + lane / SPLIT;
+    const int j = zb * SCAN_COLS + lane / SPLIT;
     const bool jv = j < Dv;
     const int row0 = part * RP;
     const int t0 = p.q_start[r];
@@ -510,135 +544,176 @@ __global__ __launch_bounds__(WAVE) void scan_kernel(ScanArgs p) {
 #pragma unroll
     for (int i = 0; i < RP; ++i) s[i] = (jv && row0 + i < D) ? S[(long long)(row0 + i) * Dv] : 0.f;
 
-    // what the next eight tokens bring
-    // (kept as they were loaded: a conversion on the spot would wait for the load)
-    TA fa[CH][PER], fk[CH][PER];
-    T fv[CH];
-    float fw[CH][PER], fb[CH];
-    // Every load is issued whatever the lane and token (from a clamped place where there is nothing to fetch);
-    // what does not count is replaced when the values are staged, eight tokens later: a load inside a condition
-    // would be waited for on the spot, and so would a value that is looked at right after its load.
-    // Addresses are a base that is the same for the whole wave (the chunk's first token, this head) plus a small
-    // offset a lane: the rows of a chunk lie less than 2^31 elements apart.
-    const int jc = min(j, Dv - 1);
-    const unsigned strideA = (unsigned)p.lda, strideW = (unsigned)(H * D), strideV = (unsigned)p.ldv, strideS = (unsigned)H;
+    // What the next CH tokens bring (kept as it was loaded: a conversion on the spot would wait for the load).  A lane
+    // fetches groups of four key channels, of any of the tokens, and single values; WHOLE: a group is one load.  What a
+    // token brings once (its scalar, ssd: its decay) comes in one load, lane l that of token l.
+    // Every load is issued whatever the lane and token (from a clamped place where there is nothing to fetch): a load
+    // inside a condition would be waited for on the spot.
+    four fa[PER], fk[PER];
+    f32x4 fw[PER];
+    T fv[PER_V];
+    float fb = 0.f, fd = 0.f;
     const float bonus_h = SSD ? p.head_bonus[head] : 0.f;
-    float fd[CH];                                      // ssd: a token's decay
-    int ic[PER];
+    auto fetch = [&](int c0) {                         // c0: the first token, counted from the request's first of the step
 #pragma unroll
-    for (int e = 0; e < PER; ++e) ic[e] = min(lane + e * WAVE, D - 1);
-    auto fetch = [&](int first, int count) {
-        const TA* ba = pa + (long long)first * p.lda + (long long)ha * D;
-        const TA* bk = pk + (long long)first * p.lda + (long long)ha * D;
-        const float* bw = SSD ? p.decay + (long long)first * H + head : p.decay + ((long long)first * H + head) * D;
-        const T* bv = pv + (long long)first * p.ldv + (long long)head * Dv;
-        const float* bs = p.scalar + (long long)first * H + head;
+        for (int e = 0; e < PER; ++e) {
+            const int id = lane + e * WAVE;
+            const long long t = t0 + min(c0 + id / QUADS, n - 1);
+            const int i = id % QUADS * 4;
+            const TA *ra = pa + t * p.lda + (long long)ha * D, *rk = pk + t * p.lda + (long long)ha * D;
+            const float* rw = SSD ? nullptr : p.decay + (t * H + head) * D;
+            if (WHOLE) {
+                const int ic = min(i, D - 4);
+                fa[e] = *(const four*)(ra + ic);
+                if (!FORGET) fk[e] = *(const four*)(rk + ic);
+                if (!SSD) fw[e] = *(const f32x4*)(rw + ic);
+            } else {
 #pragma unroll
-        for (int tt = 0; tt < CH; ++tt) {
-            const unsigned tc = (unsigned)min(tt, count - 1);
-#pragma unroll
-            for (int e = 0; e < PER; ++e) {
-                fa[tt][e] = ba[tc * strideA + (unsigned)ic[e]];
-                fk[tt][e] = bk[tc * strideA + (unsigned)ic[e]];
-                if (!SSD) fw[tt][e] = bw[tc * strideW + (unsigned)ic[e]];
+                for (int u = 0; u < 4; ++u) {
+                    const int ic = min(i + u, D - 1);
+                    fa[e][u] = ra[ic];
+                    if (!FORGET) fk[e][u] = rk[ic];
+                    if (!SSD) fw[e][u] = rw[ic];
+                }
             }
-            if (SSD) fd[tt] = bw[tc * strideS];
-            fv[tt] = bv[tc * strideV + (unsigned)jc];
-            fb[tt] = bs[tc * strideS];
+        }
+#pragma unroll
+        for (int e = 0; e < PER_V; ++e) {
+            const int id = lane + e * WAVE;
+            const long long t = t0 + min(c0 + id / SCAN_COLS, n - 1);
+            fv[e] = pv[t * p.ldv + (long long)head * Dv + min(zb * SCAN_COLS + id % SCAN_COLS, Dv - 1)];
+        }
+        const long long t = t0 + min(c0 + lane % CH, n - 1);
+        if (!FORGET) fb = p.scalar[t * H + head];
+        if (SSD) fd = p.decay[t * H + head];
+    };
+    // The fetched values to LDS in float32, key channels beyond D as zero (tokens beyond the last are staged and never read).
+    auto stage = [&]() {
+#pragma unroll
+        for (int e = 0; e < PER; ++e) {
+            const int id = lane + e * WAVE, tt = id / QUADS, i = id % QUADS * 4;
+            const float step = SSD ? __shfl(fb, tt, WAVE) : 1.f;
+            f32x4 a, k, w;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool ok = i + u < D;
+                a[u] = ok ? to_f32((TA)fa[e][u]) : 0.f;
+                k[u] = ok ? (FORGET ? 1.0f - fw[e][u] : SSD ? step * to_f32((TA)fk[e][u]) : to_f32((TA)fk[e][u])) : 0.f;
+                w[u] = ok && !SSD ? fw[e][u] : 0.f;
+            }
+            if (CH * QUADS % WAVE == 0 || id < CH * QUADS) {
+                *(f32x4*)&sa[tt][i] = a;
+                *(f32x4*)&sk[tt][i] = k;
+                if (!SSD) *(f32x4*)&sw[tt][i] = w;
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < PER_V; ++e) {
+            const int id = lane + e * WAVE;
+            if (CH * SCAN_COLS % WAVE == 0 || id < CH * SCAN_COLS) sv[id % SCAN_COLS][id / SCAN_COLS] = to_f32(fv[e]);
         }
     };
-    // one token: the state's rows of this lane move on and the token's output leaves.  Four partial sums a
-    // lane (rows 0, 1, 2, 3 of every group of four), added in a fixed order, then the quad's exchange.
-    auto token = [&](int tt, float vt, float sc, float wt, float* orow) {
+    // What a token brings to this lane's rows, out of LDS.
+    struct Rows { f32x4 w[NI16], k[NI16], q[NI16]; };
+    auto rows_of = [&](int tt, Rows& m) {
+#pragma unroll
+        for (int g4 = 0; g4 < NI16; ++g4) {
+            if (!SSD) m.w[g4] = *(const f32x4*)&sw[tt][row0 + g4 * 4];
+            m.k[g4] = *(const f32x4*)&sk[tt][row0 + g4 * 4];
+            m.q[g4] = *(const f32x4*)&sa[tt][row0 + g4 * 4];
+        }
+    };
+    // One token: the state's rows of this lane move on; the lane's share of the token's output.  Four partial sums a
+    // lane (rows 0, 1, 2, 3 of every group of four), added in a fixed order.
+    auto token = [&](const Rows& m, float vt, float sc, float wt) {
         float o4[4] = {0.f, 0.f, 0.f, 0.f};
+        float err = 0.f;
         if (DELTA) {
             float kv4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int g4 = 0; g4 < NI16; ++g4) {
-                const f32x4 w4 = *(const f32x4*)&sw[tt][row0 + g4 * 4];
-                const f32x4 k4 = *(const f32x4*)&sk[tt][row0 + g4 * 4];
+            for (int g4 = 0; g4 < NI16; ++g4)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    s[g4 * 4 + e] *= w4[e];
-                    kv4[e] = fmaf(k4[e], s[g4 * 4 + e], kv4[e]);
+                    s[g4 * 4 + e] *= m.w[g4][e];
+                    kv4[e] = fmaf(m.k[g4][e], s[g4 * 4 + e], kv4[e]);
                 }
-            }
-            const float err = sc * (vt - group_sum<SPLIT>((kv4[0] + kv4[1]) + (kv4[2] + kv4[3])));
-#pragma unroll
-            for (int g4 = 0; g4 < NI16; ++g4) {
-                const f32x4 k4 = *(const f32x4*)&sk[tt][row0 + g4 * 4];
-                const f32x4 q4 = *(const f32x4*)&sa[tt][row0 + g4 * 4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    s[g4 * 4 + e] = fmaf(k4[e], err, s[g4 * 4 + e]);
-                    o4[e] = fmaf(q4[e], s[g4 * 4 + e], o4[e]);
-                }
-            }
-        } else {
-#pragma unroll
-            for (int g4 = 0; g4 < NI16; ++g4) {
-                const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-                const f32x4 w4 = SSD ? zero4 : *(const f32x4*)&sw[tt][row0 + g4 * 4];
-                const f32x4 k4 = *(const f32x4*)&sk[tt][row0 + g4 * 4];
-                const f32x4 r4 = *(const f32x4*)&sa[tt][row0 + g4 * 4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    if (SSD) {
-                        s[g4 * 4 + e] = fmaf(wt, s[g4 * 4 + e], k4[e] * vt);
-                        o4[e] = fmaf(r4[e], s[g4 * 4 + e], o4[e]);
-                    } else if (FORGET) {
-                        s[g4 * 4 + e] = fmaf(w4[e], s[g4 * 4 + e], k4[e] * vt);
-                        o4[e] = fmaf(r4[e], s[g4 * 4 + e], o4[e]);
-                    } else {
-                        o4[e] = fmaf(r4[e], s[g4 * 4 + e], o4[e]);
-                        s[g4 * 4 + e] = fmaf(w4[e], s[g4 * 4 + e], k4[e] * vt);
-                    }
-                }
-            }
+            err = sc * (vt - group_sum<SPLIT>((kv4[0] + kv4[1]) + (kv4[2] + kv4[3])));
         }
-        float o = group_sum<SPLIT>((o4[0] + o4[1]) + (o4[2] + o4[3]));
-        if (SSD) o = fmaf(bonus_h, vt, o);
-        else if (!DELTA && !FORGET) o = fmaf(sc, vt, o);
-        // (the lanes of a group hold the same sum and write it to the same place: no lane is switched off for it)
-        if (jv) orow[(unsigned)tt * (unsigned)(H * Dv)] = o;
+#pragma unroll
+        for (int g4 = 0; g4 < NI16; ++g4)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float& si = s[g4 * 4 + e];
+                const float k = m.k[g4][e], q = m.q[g4][e];
+                if (DELTA) si = fmaf(k, err, si);
+                else if (SSD) si = fmaf(wt, si, k * vt);
+                else if (FORGET) si = fmaf(m.w[g4][e], si, k * vt);
+                o4[e] = fmaf(q, si, o4[e]);
+                if (!DELTA && !SSD && !FORGET) si = fmaf(m.w[g4][e], si, k * vt);
+            }
+        return (o4[0] + o4[1]) + (o4[2] + o4[3]);
     };
+    // With the lanes' shares added: the token's own value, where it counts beside the state.
+    auto own = [&](float o, float vt, float sc) { return SSD ? fmaf(bonus_h, vt, o) : DELTA || FORGET ? o : fmaf(sc, vt, o); };
+    // (the lanes of a group hold the same sum and write it to the same place)
+    float* const out_row = p.out + ((long long)t0 * H + head) * Dv;
+    auto leave = [&](int t, float o) { (out_row + (long long)t * H * Dv)[(unsigned)j] = o; };
 
-    fetch(t0, min(n, CH));
+    // The outputs of CH tokens stay in registers until the next ones have been staged: staging waits for every access to
+    // memory under way, and stores from just before would be waited for too, all the way to memory.
+    float o[CH] = {};
+    fetch(0);
     for (int c0 = 0; c0 < n; c0 += CH) {
         const int count = min(CH, n - c0);
+        stage();
         float v[CH], sc[CH], wd[CH];
 #pragma unroll
         for (int tt = 0; tt < CH; ++tt) {
-            v[tt] = to_f32(fv[tt]);
-            sc[tt] = fb[tt];
-            wd[tt] = SSD ? fd[tt] : 0.f;
-#pragma unroll
-            for (int e = 0; e < PER; ++e) {
-                const int i = lane + e * WAVE;
-                const bool ok = i < D;                 // (tokens beyond the chunk's last are staged and never read)
-                if (i < DP) {
-                    sa[tt][i] = ok ? to_f32(fa[tt][e]) : 0.f;
-                    sk[tt][i] = ok ? (FORGET ? 1.0f - fw[tt][e] : SSD ? fb[tt] * to_f32(fk[tt][e]) : to_f32(fk[tt][e])) : 0.f;
-                    if (!SSD) sw[tt][i] = ok ? fw[tt][e] : 0.f;
-                }
-            }
+            sc[tt] = FORGET ? 0.f : lane_of(fb, tt);
+            wd[tt] = SSD ? lane_of(fd, tt) : 0.f;
         }
-        if (c0 + CH < n) fetch(t0 + c0 + CH, min(CH, n - c0 - CH));
+        if (jv && c0 > 0) {
+#pragma unroll
+            for (int tt = 0; tt < CH; ++tt) leave(c0 - CH + tt, o[tt]);
+        }
+        if (c0 + CH < n) fetch(c0 + CH);
         // The workgroup is one wave and LDS serves a wave's accesses in order: nothing has to be waited for
         // between the writes above and the reads below, only the compiler must keep their order.  (A
         // __syncthreads() would also wait for the loads of the next eight tokens, which are meant to be under
         // way while these are computed.)
         __builtin_amdgcn_wave_barrier();
-        float* orow = p.out + ((long long)(t0 + c0) * H + head) * Dv + j;     // this lane's place in the chunk's first row
-        if (count == CH) {                             // eight whole tokens: no test between them
 #pragma unroll
-            for (int tt = 0; tt < CH; ++tt) token(tt, v[tt], sc[tt], wd[tt], orow);
+        for (int t4 = 0; t4 < CH; t4 += 4) *(f32x4*)&v[t4] = *(const f32x4*)&sv[lane / SPLIT][t4];
+        if (count == CH) {
+            // CH whole tokens, one block of code without a test: the rows of AHEAD tokens are asked for before they are
+            // needed, and the sums over the lanes that share a channel go side by side.
+            constexpr int AHEAD = NI16 == 1 ? 4 : 1;
+            Rows m[AHEAD];
+#pragma unroll
+            for (int tt = 0; tt < AHEAD; ++tt) rows_of(tt, m[tt]);
+#pragma unroll
+            for (int tt = 0; tt < CH; ++tt) {
+                o[tt] = token(m[tt % AHEAD], v[tt], sc[tt], wd[tt]);
+                if (tt + AHEAD < CH) rows_of(tt + AHEAD, m[tt % AHEAD]);
+            }
+            group_sums<SPLIT>(o);
+#pragma unroll
+            for (int tt = 0; tt < CH; ++tt) o[tt] = own(o[tt], v[tt], sc[tt]);
         } else {
 #pragma unroll
             for (int tt = 0; tt < CH; ++tt)
-                if (tt < count) token(tt, v[tt], sc[tt], wd[tt], orow);
+                if (tt < count) {
+                    Rows m;
+                    rows_of(tt, m);
+                    const float ot = own(group_sum<SPLIT>(token(m, v[tt], sc[tt], wd[tt])), v[tt], sc[tt]);
+                    if (jv) leave(c0 + tt, ot);
+                }
         }
         __builtin_amdgcn_wave_barrier();               // the reads stay before the next tokens' writes
+    }
+    if (jv && n % CH == 0) {
+#pragma unroll
+        for (int tt = 0; tt < CH; ++tt) leave(n - CH + tt, o[tt]);
     }
 #pragma unroll
     for (int i = 0; i < RP; ++i)
@@ -678,14 +753,20 @@ __global__ __launch_bounds__(WAVE) void head_norm_gate_kernel(const float* __res
 }
 
 template <typename TA, typename T, bool DELTA, bool FORGET = false, bool SSD = false>
-int launch_scan(const ScanArgs& p, int R, hipStream_t stream) {
+int launch_scan(ScanArgs p, int R, hipStream_t stream) {
     if (p.H > 65535 || p.D > 256) return -2;
     const bool narrow = p.D <= 32;                      // four lanes a value channel; else sixteen
     const int split = narrow ? 4 : 16;
     const int ni = narrow ? (p.D + 15) / 16 : (p.D + 63) / 64;
     dim3 grid(R, p.H, ceil_div(p.Dv, WAVE / split)), block(WAVE);
     if (grid.z > 65535) return -2;
-#define SCAN(NI, SPLIT) hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, DELTA, FORGET, SSD>), grid, block, 0, stream, p)
+    p.by_xcd = (long long)R * p.H * grid.z < (1ll << 32);       // the workgroups' numbers have 32 bits there
+    // four key channels a load, where they lie so that one load can fetch them
+    auto in_fours = [](const void* q, size_t width) { return (uintptr_t)q % (4 * width) == 0; };
+    const bool whole = p.D % 4 == 0 && p.lda % 4 == 0 && in_fours(p.a, sizeof(TA)) && (FORGET || in_fours(p.k, sizeof(TA))) &&
+                       (SSD || in_fours(p.decay, 4));
+#define SCAN(NI, SPLIT) do { if (whole) hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, true, DELTA, FORGET, SSD>), grid, block, 0, stream, p); \
+                             else hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, false, DELTA, FORGET, SSD>), grid, block, 0, stream, p); } while (0)
     if (narrow) { if (ni <= 1) SCAN(1, 4); else SCAN(2, 4); }
     else if (ni <= 1) SCAN(1, 16);
     else if (ni <= 2) SCAN(2, 16);
