@@ -618,7 +618,7 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
     auto rows_of = [&](int tt, Rows& m) {
 #pragma unroll
         for (int g4 = 0; g4 < NI16; ++g4) {
-            if (!SSD) m.w[g4] = *(const f32x4*)&sw[tt][row0 + g4 * 4];
+            m.w[g4] = SSD ? f32x4{0.f, 0.f, 0.f, 0.f} : *(const f32x4*)&sw[tt][row0 + g4 * 4];
             m.k[g4] = *(const f32x4*)&sk[tt][row0 + g4 * 4];
             m.q[g4] = *(const f32x4*)&sa[tt][row0 + g4 * 4];
         }
@@ -627,30 +627,46 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
     // lane (rows 0, 1, 2, 3 of every group of four), added in a fixed order.
     auto token = [&](const Rows& m, float vt, float sc, float wt) {
         float o4[4] = {0.f, 0.f, 0.f, 0.f};
-        float err = 0.f;
         if (DELTA) {
             float kv4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int g4 = 0; g4 < NI16; ++g4)
+            for (int g4 = 0; g4 < NI16; ++g4) {
+                const f32x4 w4 = m.w[g4], k4 = m.k[g4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    s[g4 * 4 + e] *= m.w[g4][e];
-                    kv4[e] = fmaf(m.k[g4][e], s[g4 * 4 + e], kv4[e]);
+                    s[g4 * 4 + e] *= w4[e];
+                    kv4[e] = fmaf(k4[e], s[g4 * 4 + e], kv4[e]);
                 }
-            err = sc * (vt - group_sum<SPLIT>((kv4[0] + kv4[1]) + (kv4[2] + kv4[3])));
-        }
-#pragma unroll
-        for (int g4 = 0; g4 < NI16; ++g4)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                float& si = s[g4 * 4 + e];
-                const float k = m.k[g4][e], q = m.q[g4][e];
-                if (DELTA) si = fmaf(k, err, si);
-                else if (SSD) si = fmaf(wt, si, k * vt);
-                else if (FORGET) si = fmaf(m.w[g4][e], si, k * vt);
-                o4[e] = fmaf(q, si, o4[e]);
-                if (!DELTA && !SSD && !FORGET) si = fmaf(m.w[g4][e], si, k * vt);
             }
+            const float err = sc * (vt - group_sum<SPLIT>((kv4[0] + kv4[1]) + (kv4[2] + kv4[3])));
+#pragma unroll
+            for (int g4 = 0; g4 < NI16; ++g4) {
+                const f32x4 k4 = m.k[g4], q4 = m.q[g4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    s[g4 * 4 + e] = fmaf(k4[e], err, s[g4 * 4 + e]);
+                    o4[e] = fmaf(q4[e], s[g4 * 4 + e], o4[e]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int g4 = 0; g4 < NI16; ++g4) {
+                const f32x4 w4 = m.w[g4], k4 = m.k[g4], r4 = m.q[g4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (SSD) {
+                        s[g4 * 4 + e] = fmaf(wt, s[g4 * 4 + e], k4[e] * vt);
+                        o4[e] = fmaf(r4[e], s[g4 * 4 + e], o4[e]);
+                    } else if (FORGET) {
+                        s[g4 * 4 + e] = fmaf(w4[e], s[g4 * 4 + e], k4[e] * vt);
+                        o4[e] = fmaf(r4[e], s[g4 * 4 + e], o4[e]);
+                    } else {
+                        o4[e] = fmaf(r4[e], s[g4 * 4 + e], o4[e]);
+                        s[g4 * 4 + e] = fmaf(w4[e], s[g4 * 4 + e], k4[e] * vt);
+                    }
+                }
+            }
+        }
         return (o4[0] + o4[1]) + (o4[2] + o4[3]);
     };
     // With the lanes' shares added: the token's own value, where it counts beside the state.
