@@ -368,6 +368,28 @@ def test_forget_scan_carries_its_state_across_any_cut(gpu):
             assert torch.isnan(state[0]).all() and torch.isnan(state[2]).all()
 
 
+@pytest.mark.parametrize("H, Hkv, vd", [(4, 2, 64), (32, 8, 64), (12, 3, 5), (16, 2, 130), (8, 1, 70), (6, 2, 33), (5, 5, 16), (1, 1, 1)])
+def test_mix_of_heads_against_the_sum_in_float64(gpu, H, Hkv, vd):
+    """Two, four and eight heads a kv head (with and without heads left over after eight at a time) and the others: to the
+    rounding of H float32 steps, and of the output's type."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(H + vd)
+    o, talk, gates = (torch.randn(*s, generator=gen) for s in ((7, H * Hkv * vd), (H, H), (7, H + 3)))
+    ov, t64 = o.double().view(7, H, Hkv, vd), talk.double()
+    kv_of = torch.arange(H) // (H // Hkv)
+    picked = ov[:, :, kv_of, :]                                  # [t][summed head][h][vd]
+    want = torch.stack([(t64[h][None, :, None] * picked[:, :, h]).sum(1) for h in range(H)], 1)
+    size = torch.stack([(t64[h].abs()[None, :, None] * picked[:, :, h].abs()).sum(1) for h in range(H)], 1)
+    for gated in (False, True):
+        f = torch.sigmoid(gates[:, :H].double())[:, :, None] if gated else 1.0
+        for dt, unit in ((torch.float32, 2.0 ** -24), (torch.bfloat16, 2.0 ** -8)):
+            out = torch.full((7, H * vd), float("nan"), dtype=dt, device=gpu)
+            ops.head_mix_gate(o.to(gpu), out, H=H, Hkv=Hkv, vd=vd, talk=talk.to(gpu), gates=gates.to(gpu) if gated else None)
+            err = (out.cpu().double().view(7, H, vd) - want * f).abs()
+            # H + 1 roundings of the sum and the gate's few units; then the output's own
+            assert (err <= (H + 8) * 2.0 ** -24 * size * f + unit * (want * f).abs()).all(), (dt, gated)
+
+
 @pytest.mark.parametrize("D", [24, 64, 68, 128, 256])
 def test_scan_gives_the_same_bits_for_any_company_and_alignment(gpu, D):
     """The recurrence's kernel over nine requests of 0 to 41 tokens (edges of the eight tokens it stages at a time), with

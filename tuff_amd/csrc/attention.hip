@@ -400,6 +400,42 @@ __global__ __launch_bounds__(WAVE) void head_mix_gate_kernel(const TI* __restric
         for (int j = threadIdx.x; j < vd; j += WAVE) dst[j] = from_f32<T>(to_f32(src[j]) * g);
     }
 }
+
+// The mix for the G heads of a kv head at once: a wave a (token, kv head), which reads every weighted sum once instead of G
+// times, eight heads' at a time.  Bound by the float32 sums: 2,048 tokens, 32 heads, 8 kv heads of 64:
+// 82 -> 28.5 us.  For 2, 4 and 8 heads a kv head; the kernel above takes the others, and the gates alone.
+template <int G, typename TI, typename T>
+__global__ __launch_bounds__(WAVE) void head_mix_group_kernel(const TI* __restrict__ o, const float* __restrict__ talk,
+                                                              const float* __restrict__ gates, int gate_stride,
+                                                              T* __restrict__ out, int H, int Hkv, int vd) {
+    const long long t = blockIdx.x;
+    const int kvh = blockIdx.y;
+    for (int j = threadIdx.x; j < vd; j += WAVE) {
+        const TI* src = o + (t * H * Hkv + kvh) * vd + j;
+        float acc[G] = {};
+        int q = 0;
+        for (; q + 8 <= H; q += 8) {
+            TI ov[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) ov[u] = src[(long long)(q + u) * Hkv * vd];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int g = 0; g < G; ++g) acc[g] = fmaf(talk[(kvh * G + g) * H + q + u], to_f32(ov[u]), acc[g]);
+        }
+        for (; q < H; ++q) {
+            const float ov = to_f32(src[(long long)q * Hkv * vd]);
+#pragma unroll
+            for (int g = 0; g < G; ++g) acc[g] = fmaf(talk[(kvh * G + g) * H + q], ov, acc[g]);
+        }
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+            const int h = kvh * G + g;
+            const float gate = gates ? 1.0f / (1.0f + expf(-gates[t * gate_stride + h])) : 1.f;
+            out[(t * H + h) * vd + j] = from_f32<T>(acc[g] * gate);
+        }
+    }
+}
 }  // namespace
 
 // in_dt: type of o; dt: type of out.  talk float32 [H][H] or null; gates float32 or null.
@@ -408,12 +444,16 @@ TUFF_EXPORT int tuff_head_mix_gate(const void* o, int in_dt, const float* talk, 
     if (n_tokens <= 0) return 0;
     if (H <= 0 || Hkv <= 0 || H % Hkv || H > 65535 || vd <= 0) return -2;
     dim3 grid(n_tokens, H), block(WAVE);
-#define LAUNCH(TI, T) hipLaunchKernelGGL((head_mix_gate_kernel<TI, T>), grid, block, 0, stream, (const TI*)o, talk, gates, gate_stride, (T*)out, H, Hkv, vd)
+    const int group = talk && Hkv < H ? H / Hkv : 0;                 // heads that read the same sums
+#define GROUP(G, TI, T) hipLaunchKernelGGL((head_mix_group_kernel<G, TI, T>), dim3(n_tokens, Hkv), block, 0, stream, (const TI*)o, talk, gates, gate_stride, (T*)out, H, Hkv, vd)
+#define LAUNCH(TI, T) do { if (group == 2) GROUP(2, TI, T); else if (group == 4) GROUP(4, TI, T); else if (group == 8) GROUP(8, TI, T); \
+                           else hipLaunchKernelGGL((head_mix_gate_kernel<TI, T>), grid, block, 0, stream, (const TI*)o, talk, gates, gate_stride, (T*)out, H, Hkv, vd); } while (0)
     if (in_dt == DT_F32 && dt == DT_F32) LAUNCH(float, float);
     else if (in_dt == DT_F32) LAUNCH(float, bf16_t);
     else if (dt == DT_BF16) LAUNCH(bf16_t, bf16_t);
     else return -2;
 #undef LAUNCH
+#undef GROUP
     return launch_status();
 }
 
