@@ -498,7 +498,8 @@ __device__ __forceinline__ float group_sum(float v) {
 // for ahead, their sums over the lanes side by side; and the stores of eight tokens behind the next eight's staging.  One
 // request of 2,048 tokens, 16 heads, 64 key and 128 value channels: 414 -> 217 us.  For many requests, the rows that the
 // blocks of a head all read: by XCD as below, 64 requests of 200 tokens, 16 heads of 128 x 128, 1,281 -> 856 us (forget
-// gate), 2,366 -> 1,053 us (delta rule); without it 1,365 and 2,580.
+// gate), 2,366 -> 1,053 us (delta rule); without it 1,365 and 2,580.  Four waves a SIMD up to 64 key channels, three up to
+// 128 (with four the registers spill: 64 single tokens, 16 heads of 128, 92 us instead of 80), two beyond.
 template <typename TA, typename T, int NI16, int SPLIT, bool WHOLE, bool DELTA, bool FORGET = false, bool SSD = false>
 __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_kernel(ScanArgs p) {
     constexpr int RP = NI16 * 4;                       // rows of the state's column a lane keeps
