@@ -157,6 +157,13 @@ def test_gemm_with_the_norm_inside(gpu, M, N, K, use_rows):
         assert torch.equal(one[0], out[M - 1])
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1536, 1536), (16, 4608, 1536), (8, 2048, 1280), (5, 48, 640), (3, 40, 896), (16, 64, 256), (2, 80, 128)])
+def test_gemm_with_the_norm_inside_and_waves_of_unequal_shares(gpu, M, N, K):
+    """Inner sizes of which some waves of a workgroup take two pieces of 128 and others one, or one and others none: the norm
+    weight is in LDS before any of them reads it."""
+    test_gemm_with_the_norm_inside(gpu, M, N, K, False)
+
+
 @pytest.mark.parametrize("M,d,K1,N2", [(1, 64, 192, 512), (8, 2048, 8192, 6144), (16, 240, 328, 777 * 2), (5, 96, 96, 40),
                                        (17, 96, 96, 40), (32, 2048, 8192, 6144), (24, 240, 328, 777 * 2), (40, 2048, 8192, 6144), (64, 240, 328, 777 * 2), (33, 64, 192, 512),
                                        (64, 2048, 2048, 65536),

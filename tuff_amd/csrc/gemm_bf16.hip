@@ -582,7 +582,11 @@ constexpr int SS_ROWS_WIDE = 64;
 // workgroups of 16,384 columns run side by side and not in two rounds.
 constexpr int skinny16_waves_a_simd(int NW, int COLS, int MT) { return NW == 8 && COLS == 32 && MT == 1 ? 4 : 1; }
 
-template <int NW, int MODE, int NORM, bool EMIT, int COLS, int MT>
+// How many chunks the waves of a workgroup have: at most one; one or two; two or more.  The norm inside holds a barrier, which
+// has to stand where every wave passes, so there the kernel is built for each.
+enum : int { SHARE_ONE = 0, SHARE_TWO = 1, SHARE_MANY = 2, SHARE_ANY = 3 };
+
+template <int NW, int MODE, int NORM, bool EMIT, int COLS, int MT, int SHARE>
 __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) void gemm_bf16_skinny16_kernel(const void* __restrict__ Xv, const bf16_t* __restrict__ W,
                                                                        void* __restrict__ Y, int M, int N, int K,
                                                                        const float* __restrict__ norm_w, float eps,
@@ -777,11 +781,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
     // The wave's chunks, two sets of operands in turn; every way through has its loads and products in straight order.
     const int n = (nchunks - wave + NW - 1) / NW;
     auto nth = [&](int i) { return chunk_of(wave + i * NW); };
-    if (n < 2) {
-        if (n == 1) load(nth(0), o0);
-        behind();
-        if (n == 1) multiply(nth(0), o0);
-    } else {
+    auto several = [&]() {                             // two chunks or more
         load(nth(0), o0);
         load(nth(1), o1);
         behind();
@@ -800,6 +800,27 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
         } else {
             multiply(nth(i + 1), o1);
         }
+    };
+    auto at_most_one = [&]() {
+        if (n > 0) load(nth(0), o0);
+        behind();
+        if (n > 0) multiply(nth(0), o0);
+    };
+    if constexpr (SHARE == SHARE_ONE) {
+        at_most_one();
+    } else if constexpr (SHARE == SHARE_MANY) {
+        several();
+    } else if constexpr (NORM == NORM_INSIDE) {
+        // one chunk or two; the barrier in behind() stands where every wave passes, whatever it has
+        load(nth(0), o0);
+        if (n > 1) load(nth(1), o1);
+        behind();
+        multiply(nth(0), o0);
+        if (n > 1) multiply(nth(1), o1);
+    } else if (n < 2) {
+        at_most_one();
+    } else {
+        several();
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -1347,10 +1368,16 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
     // the in-kernel norm needs more registers a wave: at most 8 waves a workgroup
     SkinnyPlan p = plan_skinny(M, N, K, NORM == NORM_INSIDE ? 8 : 16, EMIT, MODE == OUT_CONV);
     const size_t lds = NORM == NORM_INSIDE ? (size_t)K * sizeof(float) : 0;
-    const int mt = M > 16 ? 2 : 1;
-#define GO_MT(NW, COLS, MT) hipLaunchKernelGGL((gemm_bf16_skinny16_kernel<NW, MODE, NORM, EMIT, COLS, MT>), grid, dim3(NW * WAVE), lds, stream, \
+    const int mt = M > 16 ? 2 : 1, chunks = ceil_div(K, SK_CHUNK);
+#define GO_SHARE(NW, COLS, MT, SHARE) hipLaunchKernelGGL((gemm_bf16_skinny16_kernel<NW, MODE, NORM, EMIT, COLS, MT, SHARE>), grid, dim3(NW * WAVE), lds, stream, \
                                         X, W, Y, M, N, K, x.norm_w, x.eps, x.rows, x.ldx ? x.ldx : (long long)K, x.ss_in, x.n_ss, x.emit_nw, x.emit_xw, x.emit_ss, \
                                         x.conv)
+#define GO_MT(NW, COLS, MT) do { \
+        if constexpr (NORM != NORM_INSIDE) GO_SHARE(NW, COLS, MT, SHARE_ANY); \
+        else if (chunks <= NW) GO_SHARE(NW, COLS, MT, SHARE_ONE); \
+        else if (chunks <= 2 * NW) GO_SHARE(NW, COLS, MT, SHARE_TWO); \
+        else GO_SHARE(NW, COLS, MT, SHARE_MANY); \
+    } while (0)
 #define GO(NW, COLS) do { \
         if (mt == 1) GO_MT(NW, COLS, 1); \
         else if constexpr (NW <= 8 && COLS <= 32 && NORM != NORM_INSIDE) GO_MT(NW, COLS, 2); \
@@ -1359,9 +1386,9 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
     if constexpr (MODE == OUT_CONV) {
         // eight channels a workgroup (three half tiles); the waves split K as always, at most eight of them:
         // sixteen would leave a wave 128 registers, too few for three tiles' operands of two chunks
-        const int nchunks = ceil_div(K, SK_CHUNK), groups = N / 3 / 8;
+        const int groups = N / 3 / 8;
         int waves = 4;
-        while (waves < 8 && groups * waves < 3072 && nchunks >= 2 * waves) waves *= 2;
+        while (waves < 8 && groups * waves < 3072 && chunks >= 2 * waves) waves *= 2;
         dim3 grid(groups);
         if (waves == 4) GO(4, 8); else GO(8, 8);
     } else {
@@ -1376,6 +1403,7 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
     }
 #undef GO
 #undef GO_MT
+#undef GO_SHARE
     return launch_status();
 }
 
