@@ -164,6 +164,31 @@ def test_gemm_with_the_norm_inside_and_waves_of_unequal_shares(gpu, M, N, K):
     test_gemm_with_the_norm_inside(gpu, M, N, K, False)
 
 
+@pytest.mark.parametrize("N", [40, 2048, 3072, 8200, 16384])
+@pytest.mark.parametrize("K", [8, 128, 136, 384, 640, 1024, 1032, 2048, 2056, 4104])
+def test_gemm_bf16_few_rows_at_the_edges_of_the_waves_shares(gpu, N, K):
+    """Inner sizes of no chunk of 128, one, two and more a wave, whole and ragged, over tiles of 8, 16 and 32 columns: within
+    float32's K roundings of the float64 product; a row of infinities and NaN beside the others, and behind them, stays its own."""
+    from tuff_amd.csrc import ops
+    rows = _r(18, K, seed=K, dtype=torch.bfloat16).to(gpu)
+    rows[2], rows[17] = float("inf"), float("nan")
+    w = _r(N, K, seed=N, dtype=torch.bfloat16).to(gpu)
+    tiled = ops.tile_weight(w)
+    exact = rows[:16].double().nan_to_num(0, 0, 0) @ w.double().T
+    bound = K * 2.0 ** -24 * (rows[:16].double().abs().nan_to_num(0, 0, 0) @ w.double().abs().T)
+    kept = [m for m in range(16) if m != 2]
+    whole = torch.empty(16, N, device=gpu)
+    ops.gemm(rows[:16], tiled, whole)
+    assert ((whole.double() - exact).abs() <= bound)[kept].all() and not torch.isfinite(whole[2]).any()
+    for M in (1, 2, 5):
+        some = torch.empty(M, N, device=gpu)
+        ops.gemm(rows[:M], tiled, some)
+        assert torch.equal(some[:2], whole[:min(M, 2)])
+        acc = torch.ones(M, N, device=gpu)
+        ops.gemm(rows[:M], tiled, acc, accumulate=True)
+        assert torch.equal(acc[:2], 1 + whole[:min(M, 2)])
+
+
 @pytest.mark.parametrize("M,d,K1,N2", [(1, 64, 192, 512), (8, 2048, 8192, 6144), (16, 240, 328, 777 * 2), (5, 96, 96, 40),
                                        (17, 96, 96, 40), (32, 2048, 8192, 6144), (24, 240, 328, 777 * 2), (40, 2048, 8192, 6144), (64, 240, 328, 777 * 2), (33, 64, 192, 512),
                                        (64, 2048, 2048, 65536),

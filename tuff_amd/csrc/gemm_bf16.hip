@@ -544,7 +544,7 @@ constexpr int SK_CHUNK = 128;
 // chunks w, w + NW, w + 2 NW, ... of 128; in a chunk the wave reads four blocks of its row tile of W
 // (1 KB each) and 256 bytes of each of the 16 X rows (four loads of 16 rows x 64 contiguous bytes)
 // and issues four MFMAs.
-// Loads run one chunk ahead.  The wave partials are added in wave order through LDS.  NW is
+// The loads of two chunks are under way.  The wave partials are added in wave order through LDS.  NW is
 // chosen from N and K only.
 //
 // The product may be taken of the RMSNorm of the float32 residual stream x,
@@ -578,16 +578,18 @@ struct ConvTail {
 // in memory (SS_ROWS), as for every product of 17 to 64 rows.
 constexpr int SS_ROWS_WIDE = 64;
 
+// How many chunks the waves of a workgroup have: at most one; one or two; two or more.  Each is a kernel of its own, without
+// the others' code and operands, and with the norm inside its barrier where every wave passes.
+enum : int { SHARE_ONE = 0, SHARE_TWO = 1, SHARE_MANY = 2 };
+
 // Waves a SIMD has to hold.  Eight waves over 32 columns: two workgroups a CU (at most 128 registers a lane), so that the 512
 // workgroups of 16,384 columns run side by side and not in two rounds.
-constexpr int skinny16_waves_a_simd(int NW, int COLS, int MT) { return NW == 8 && COLS == 32 && MT == 1 ? 4 : 1; }
-
-// How many chunks the waves of a workgroup have: at most one; one or two; two or more.  The norm inside holds a barrier, which
-// has to stand where every wave passes, so there the kernel is built for each.
-enum : int { SHARE_ONE = 0, SHARE_TWO = 1, SHARE_MANY = 2, SHARE_ANY = 3 };
+constexpr int skinny16_waves_a_simd(int NW, int COLS, int MT, int MODE, int SHARE) {
+    return NW == 8 && COLS == 32 && MT == 1 && !(MODE == OUT_F32_ACCUM && SHARE == SHARE_MANY) ? 4 : 1;      // (that one would spill)
+}
 
 template <int NW, int MODE, int NORM, bool EMIT, int COLS, int MT, int SHARE>
-__global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) void gemm_bf16_skinny16_kernel(const void* __restrict__ Xv, const bf16_t* __restrict__ W,
+__global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE, SHARE)) void gemm_bf16_skinny16_kernel(const void* __restrict__ Xv, const bf16_t* __restrict__ W,
                                                                        void* __restrict__ Y, int M, int N, int K,
                                                                        const float* __restrict__ norm_w, float eps,
                                                                        const int* __restrict__ rows, long long ldx,
@@ -697,7 +699,12 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int kj = c * SK_CHUNK + j * 32 + g * 8;
-            if (NORM == NORM_INSIDE) {
+            if (COLS == 32 && MT == 1 && NORM != NORM_INSIDE) {
+                // (lanes without a row are switched off: here, where the rows of X are half as many bytes as W, one that reads
+                // nothing still takes its time: 16,384 x 2,048 of 1 row 14.4 us with them on, 13.7 off; narrower tiles no gain)
+                o.a[0][j] = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+                if (r16 < M) o.a[0][j] = load_buffer<false>(xbuf, kj < K ? (r16 * K + g * 8) * 2 : NOWHERE, min(c * SK_CHUNK + j * 32, K - 8) * 2);
+            } else if (NORM == NORM_INSIDE) {
                 const float* xp = xrow + min(kj, K - 8);
                 o.x[j][0] = *(const f32x4*)xp;
                 o.x[j][1] = *(const f32x4*)(xp + 4);
@@ -772,55 +779,83 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
                 for (int k = 0; k < CONV_AHEAD; ++k) st_ahead[i][k] = st[(long long)min(k, Kc - 2) * d];
             }
         }
-        if (NORM == NORM_INSIDE) {
-            // the norm weight goes to LDS while the first operands are on their way from HBM
-            for (int k = tid * 4; k < K; k += NW * WAVE * 4) *(f32x4*)(&nw_lds[k]) = *(const f32x4*)(norm_w + k);
-            __syncthreads();
-        }
+    };
+    // The norm weight goes to LDS while the first operands are on their way from HBM.  (Holds a barrier: it stands where every
+    // wave passes, whatever its number of chunks.)
+    auto norm_weight = [&]() {
+        for (int k = tid * 4; k < K; k += NW * WAVE * 4) *(f32x4*)(&nw_lds[k]) = *(const f32x4*)(norm_w + k);
+        __syncthreads();
     };
     // The wave's chunks, two sets of operands in turn; every way through has its loads and products in straight order.
     const int n = (nchunks - wave + NW - 1) / NW;
     auto nth = [&](int i) { return chunk_of(wave + i * NW); };
-    auto several = [&]() {                             // two chunks or more
+    // Loads are issued where they stand.  Left alone, the instruction scheduler puts off the last ones of a chunk until the first
+    // have arrived and their registers are free again: a second trip to memory (2,048 x 2,048, one chunk a wave, 1 row: 4.64 us,
+    // with this 4.15; 16 rows 5.7 and 5.1).
+    auto issued = [&]() { __builtin_amdgcn_sched_barrier(0); };
+    if constexpr (SHARE == SHARE_ONE) {
+        const int c = n > 0 ? nth(0) : nchunks;        // (a wave without a chunk, K up to 384: the one behind the last is all zeros)
+        load(c, o0);
+        issued();
+        behind();
+        issued();
+        if constexpr (NORM == NORM_INSIDE) norm_weight();
+        multiply(c, o0);
+    } else if constexpr (SHARE == SHARE_TWO && NORM == NORM_INSIDE) {
+        load(nth(0), o0);
+        if (n > 1) load(nth(1), o1);
+        issued();
+        behind();
+        issued();
+        norm_weight();
+        multiply(nth(0), o0);
+        if (n > 1) multiply(nth(1), o1);
+    } else if constexpr (SHARE == SHARE_TWO) {
+        if (n > 1) {
+            load(nth(0), o0);
+            load(nth(1), o1);
+            issued();
+            behind();
+            issued();
+            multiply(nth(0), o0);
+            multiply(nth(1), o1);
+        } else {
+            load(nth(0), o0);
+            issued();
+            behind();
+            issued();
+            multiply(nth(0), o0);
+        }
+    } else {
+        // (two sets of operands over 32 columns and the sums of squares are more than 128 registers: there the sums are asked
+        // for where one of the sets is used up)
+        constexpr bool LATE = NORM == NORM_SCALED && COLS == 32;
         load(nth(0), o0);
         load(nth(1), o1);
-        behind();
+        issued();
+        if (!LATE) behind();
+        issued();
+        if constexpr (NORM == NORM_INSIDE) norm_weight();
         int i = 0;
         for (; i + 3 < n; i += 2) {
             multiply(nth(i), o0);
             load(nth(i + 2), o0);
+            issued();
             multiply(nth(i + 1), o1);
             load(nth(i + 3), o1);
+            issued();
         }
         multiply(nth(i), o0);
         if (i + 2 < n) {
             load(nth(i + 2), o0);
+            issued();
             multiply(nth(i + 1), o1);
+            if (LATE) { issued(); behind(); issued(); }
             multiply(nth(i + 2), o0);
         } else {
+            if (LATE) { issued(); behind(); issued(); }
             multiply(nth(i + 1), o1);
         }
-    };
-    auto at_most_one = [&]() {
-        if (n > 0) load(nth(0), o0);
-        behind();
-        if (n > 0) multiply(nth(0), o0);
-    };
-    if constexpr (SHARE == SHARE_ONE) {
-        at_most_one();
-    } else if constexpr (SHARE == SHARE_MANY) {
-        several();
-    } else if constexpr (NORM == NORM_INSIDE) {
-        // one chunk or two; the barrier in behind() stands where every wave passes, whatever it has
-        load(nth(0), o0);
-        if (n > 1) load(nth(1), o1);
-        behind();
-        multiply(nth(0), o0);
-        if (n > 1) multiply(nth(1), o1);
-    } else if (n < 2) {
-        at_most_one();
-    } else {
-        several();
     }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -877,7 +912,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
             const int row = trow, d = N / 3, Kc = cv.taps;
             const int ch = (int)(blockIdx.x) * 8 + (l % 16);
             if ((l % 16) < 8 && row < M && ch < d) {
-                float* st = cv.state + (long long)cv.state_slot[row] * (Kc - 1) * d;
+                float* st = cv.state + (long long)slot_ahead[ei] * (Kc - 1) * d;
                 float sv[CONV_MAX_TAPS], wv[CONV_MAX_TAPS];
 #pragma unroll
                 for (int k = 0; k < CONV_MAX_TAPS; ++k) {
@@ -934,7 +969,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT)) voi
 
 // 16 < M <= 64.  grid (tiles of 64 columns, K slices).  Wave w owns columns 16w..16w+15 of the
 // tile and all MT row tiles.  The X rows of a K chunk (128 wide) go through LDS once for the
-// four waves, double buffered; W goes from HBM to registers one chunk ahead.  With more than
+// four waves, double buffered; the loads of two chunks are under way.  With more than
 // one K slice, or when the epilogue has to leave the next norm's operand, the partial tiles go to
 // a work space and splitk_finish_kernel adds them in slice order and does the epilogue.
 // NORM_SCALED as above, with the sums of squares per tile of 64 columns: ss_in [n_ss][64].
@@ -1373,8 +1408,7 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
                                         X, W, Y, M, N, K, x.norm_w, x.eps, x.rows, x.ldx ? x.ldx : (long long)K, x.ss_in, x.n_ss, x.emit_nw, x.emit_xw, x.emit_ss, \
                                         x.conv)
 #define GO_MT(NW, COLS, MT) do { \
-        if constexpr (NORM != NORM_INSIDE) GO_SHARE(NW, COLS, MT, SHARE_ANY); \
-        else if (chunks <= NW) GO_SHARE(NW, COLS, MT, SHARE_ONE); \
+        if (chunks <= NW) GO_SHARE(NW, COLS, MT, SHARE_ONE); \
         else if (chunks <= 2 * NW) GO_SHARE(NW, COLS, MT, SHARE_TWO); \
         else GO_SHARE(NW, COLS, MT, SHARE_MANY); \
     } while (0)
@@ -1383,6 +1417,7 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
         else if constexpr (NW <= 8 && COLS <= 32 && NORM != NORM_INSIDE) GO_MT(NW, COLS, 2); \
         else return -3; \
     } while (0)
+#define GO16(COLS) do { if constexpr (NORM != NORM_INSIDE) GO(16, COLS); else return -3; } while (0)
     if constexpr (MODE == OUT_CONV) {
         // eight channels a workgroup (three half tiles); the waves split K as always, at most eight of them:
         // sixteen would leave a wave 128 registers, too few for three tiles' operands of two chunks
@@ -1393,14 +1428,15 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
         if (waves == 4) GO(4, 8); else GO(8, 8);
     } else {
         dim3 grid(p.tiles);
-        if (p.cols == 16) { if (p.waves == 4) GO(4, 16); else if (p.waves == 8) GO(8, 16); else GO(16, 16); }
-        else if (p.cols == 8) { if (p.waves == 4) GO(4, 8); else if (p.waves == 8) GO(8, 8); else GO(16, 8); }
+        if (p.cols == 16) { if (p.waves == 4) GO(4, 16); else if (p.waves == 8) GO(8, 16); else GO16(16); }
+        else if (p.cols == 8) { if (p.waves == 4) GO(4, 8); else if (p.waves == 8) GO(8, 8); else GO16(8); }
         else if constexpr (!EMIT && NORM != NORM_INSIDE) {
             if (p.cols == 32) { if (p.waves == 4) GO(4, 32); else if (p.waves == 8) GO(8, 32); else GO(16, 32); }
-            else if (p.cols == 64) { if (p.waves == 4) GO(4, 64); else if (p.waves == 8) GO(8, 64); else GO(16, 64); }
+            else if (p.cols == 64 && p.waves == 4) GO(4, 64);      // (1,024 tiles or more: four waves)
             else return -3;
         } else return -3;
     }
+#undef GO16
 #undef GO
 #undef GO_MT
 #undef GO_SHARE
