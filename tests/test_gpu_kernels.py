@@ -189,6 +189,28 @@ def test_gemm_bf16_few_rows_at_the_edges_of_the_waves_shares(gpu, N, K):
         assert torch.equal(acc[:2], 1 + whole[:min(M, 2)])
 
 
+@pytest.mark.parametrize("M", [17, 20, 21])
+@pytest.mark.parametrize("N,K", [(256, 64), (1024, 1024), (2048, 1032), (2048, 2048), (2048, 2056)])
+def test_gemm_bf16_narrow_outputs_of_17_to_21_rows(gpu, M, N, K):
+    """On both sides of the rule that sends them to one kernel or to slices of K and a second: within float32's roundings of the
+    float64 product, and the product that leaves the next norm its sums leaves those of what it added."""
+    from tuff_amd.csrc import ops
+    x, w = _r(M, K, seed=1, dtype=torch.bfloat16).to(gpu), _r(N, K, seed=2, dtype=torch.bfloat16).to(gpu)
+    tiled, y0, nw = ops.tile_weight(w), _r(M, N, seed=3).to(gpu), _r(N, seed=4).to(gpu)
+    exact = x.double() @ w.double().T
+    bound = K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    out = torch.empty(M, N, device=gpu)
+    ops.gemm(x, tiled, out)
+    assert ((out.double() - exact).abs() <= bound).all()
+    y, xw = y0.clone(), torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+    ss = torch.full(ops.gemm_emit_layout(M, N, K), float("nan"), device=gpu)
+    ops.gemm_accum_emit(x, tiled, y, nw, xw, ss)
+    assert ((y.double() - exact - y0.double()).abs() <= bound + 2.0 ** -24 * y.double().abs()).all()
+    assert torch.equal(xw, (y * nw).to(torch.bfloat16))
+    want = (y.double() ** 2).sum(1)
+    assert ((ss.double().sum(0)[:M] - want).abs() <= N * 2.0 ** -24 * want).all()
+
+
 @pytest.mark.parametrize("M,d,K1,N2", [(1, 64, 192, 512), (8, 2048, 8192, 6144), (16, 240, 328, 777 * 2), (5, 96, 96, 40),
                                        (17, 96, 96, 40), (32, 2048, 8192, 6144), (24, 240, 328, 777 * 2), (40, 2048, 8192, 6144), (64, 240, 328, 777 * 2), (33, 64, 192, 512),
                                        (64, 2048, 2048, 65536),

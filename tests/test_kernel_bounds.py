@@ -41,3 +41,26 @@ def test_partition_pages_refuses_nonsense(mfma_lib):
     assert mfma_lib.tuff_attention_partition_pages(-1, 16) < 0
     assert mfma_lib.tuff_attention_partition_pages(0, 0) < 0
     assert mfma_lib.tuff_attention_partition_pages(2 ** 31 // 256, 16) < 0
+
+
+@pytest.fixture(scope="module")
+def gemm_lib():
+    from tuff_amd.csrc import ops
+    return ops.load("gemm_bf16")
+
+
+@pytest.mark.parametrize("M,N,K,plain,emit", [
+    (16, 2048, 8192, False, False),                       # up to 16 rows: one kernel, whatever the sizes
+    (17, 2048, 2048, False, True), (20, 1024, 1024, False, False), (20, 2048, 1032, False, True), (17, 256, 64, False, False),
+    (20, 2048, 2056, True, True), (17, 2048, 8192, True, True), (21, 2048, 1024, True, True), (20, 2064, 8192, False, False)])
+def test_narrow_products_of_few_rows_take_slices_only_where_they_are_faster(gemm_lib, M, N, K, plain, emit):
+    """Work space means partial tiles and a second kernel.  Outputs of up to 2,048 columns and 17 to 20 rows go without up to
+    K = 2,048, those that leave the next norm its sums up to K = 1,024."""
+    def floats(e):
+        out = ctypes.c_longlong(-1)
+        assert gemm_lib.tuff_gemm_bf16_workspace(M, N, K, e, ctypes.byref(out)) == 0
+        return out.value
+    assert (floats(0) > 0) == plain and (floats(1) > 0) == emit
+    tiles, rows = ctypes.c_int(), ctypes.c_int()
+    assert gemm_lib.tuff_gemm_bf16_emit_layout(M, N, K, ctypes.byref(tiles), ctypes.byref(rows)) == 0
+    assert tiles.value == -(-N // (64 if emit else 8 if N <= 2048 else 16)) and rows.value == (16 if M <= 16 else 64)

@@ -1298,16 +1298,20 @@ bool rows64_tiled(int M, int N, int K) { return M >= wide64_min_m && M <= 64 && 
 // rows of X again, M / (its columns) times the bytes of its share of W, and has half the waves.  Measured
 // on the shapes of a 1.2B model (against the two kernels of the other way, at 32 rows): 3,072 columns 8.8 us
 // against 10.7, a conv's input projection with the convolution 12.5 against 15.2, 16,384 columns 21.7 against
-// 21.3, 65,536 columns 67.7 against 52.2, at 17 rows it wins; 2,048 columns of K = 8,192 15.5 against 12.2 at 20
-// rows and 19.8 against 11.5 at 32; of K = 2,048 6.3 against 7.3 at 20 and 7.5 against 7.3 at 32, but it leaves the next
-// norm 256 groups of sums instead of 32, which cost the product after it 1.5 us.  So: narrow outputs never, medium ones up to
-// 32, wide ones up to 24 (where the tiled product does not take them, above).
-bool few_rows_kernel(int M, int N, int K, bool conv = false) {
+// 21.3, 65,536 columns 67.7 against 52.2, at 17 rows it wins.  So: medium outputs up to 32 rows, wide ones up to 24 (where
+// the tiled product does not take them, above).  Outputs of up to 2,048 columns: up to 20 rows with a short K, where the
+// second launch costs more than the rows read again (20 rows, this way and the other: 1,024 x 1,024 4.1 us and 5.1, 2,048 x
+// 1,024 4.3 and 5.3, 2,048 x 2,048 5.7 and 6.2, 2,048 x 3,072 8.2 and 7.3, x 8,192 16.2 and 11.4), at 32 rows it
+// loses from K = 1,024 on (2,048 x 2,048 7.5 and 7.3).  One that leaves the next norm its sums leaves a group a workgroup,
+// up to 256 instead of 32, which the product after it adds up: only up to K = 1,024 (1,024 x 1,024 and a product of 3,072
+// columns behind it 9.4 and 11.1, 2,048 x 2,048 14.1 and 13.9).
+constexpr int NARROW_SHORT_K = 2048, NARROW_SHORT_K_EMIT = 1024;
+bool few_rows_kernel(int M, int N, int K, bool conv = false, bool emit = false) {
     if (M <= 16) return true;
     if (M > SKINNY_ROWS) return false;
     if (conv) return true;
     if (rows64_tiled(M, N, K)) return false;
-    return N <= 2048 ? false : N <= 8192 ? true : M <= 24;
+    return N <= 2048 ? M <= 20 && K <= (emit ? NARROW_SHORT_K_EMIT : NARROW_SHORT_K) : N <= 8192 ? true : M <= 24;
 }
 
 // How a skinny product is cut.  Depends on N and K (and on which of the two kernels M selects).
@@ -1316,7 +1320,7 @@ SkinnyPlan plan_skinny(int M, int N, int K, int max_waves = 16, bool emit = fals
     SkinnyPlan p;
     p.slices = 1; p.chunks_per_slice = nchunks; p.ws_floats = 0; p.waves = 4;
     p.cols = 16;
-    if (few_rows_kernel(M, N, K, conv)) {
+    if (few_rows_kernel(M, N, K, conv, emit)) {
         // Narrow outputs: tiles of 8 columns, where 16 would leave CUs without a workgroup (half of
         // each MFMA idles, which costs nothing here: these products wait for memory).  Wide outputs:
         // 32 or 64 columns, whose MFMA tiles share the rows of X: with 16 columns the rows of X
@@ -1640,7 +1644,7 @@ TUFF_EXPORT int tuff_gemm_bf16_scaled_supported(int M, int N, int K) {
 // emit: for tuff_gemm_bf16_accum_emit.
 TUFF_EXPORT int tuff_gemm_bf16_workspace(int M, int N, int K, int emit, long long* ws_floats) {
     *ws_floats = 0;
-    if (N <= 0 || few_rows_kernel(M, N, K)) return 0;
+    if (N <= 0 || few_rows_kernel(M, N, K, false, emit != 0)) return 0;
     // (a wide product of few rows that the tiled kernel takes needs none, but only some of its epilogues go that way)
     *ws_floats = M <= 64 ? plan_skinny(M, N, K, 16, emit != 0).ws_floats : plan_tiled(M, N, K).ws_floats;
     return 0;
@@ -1691,7 +1695,7 @@ TUFF_EXPORT int tuff_gemm_bf16_accum_emit(const void* X, const void* W, float* Y
         t.emit_nw = next_norm_w; t.emit_xw = (bf16_t*)xw; t.emit_ss = ss;
         return launch_mode<OUT_F32_ACCUM, TILED_EMIT>((const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, ws, stream, t);
     }
-    if (few_rows_kernel(M, N, K)) {
+    if (few_rows_kernel(M, N, K, false, true)) {
         Skinny16Extra x;
         x.emit_nw = next_norm_w; x.emit_xw = (bf16_t*)xw; x.emit_ss = ss;
         return launch_skinny16<OUT_F32_ACCUM, NORM_NONE, true>(X, (const bf16_t*)W, Y, M, N, K, x, stream);
