@@ -1001,6 +1001,35 @@ def test_attention_merge_at_its_edges(gpu, hd, window):
         assert torch.equal(out, more), longest
 
 
+@pytest.mark.parametrize("hd", [24, 64, 72])
+@pytest.mark.parametrize("window", [0, 500, 4200, 16500])
+def test_attention_merge_of_short_rows_in_a_long_room(gpu, hd, window):
+    """Rows that see 1, 16, 17, 18, 64 and 65 partitions (whole groups of 64 and parts of two, by length and by window) in a step
+    with room for 80 and for 2,048: the plain formula, and the bits of each request alone in its own room."""
+    from tuff_amd.csrc import ops
+    H, Hkv, ps = 2, 1, 16
+    reqs = [(n, 1) for n in (0, 15 * 256 + 10, 16 * 256 + 1, 17 * 256 + 5, 63 * 256 + 9, 64 * 256 + 3, 79 * 256 + 200)]
+    case = _mixed_step_case(gpu, reqs, H, Hkv, hd, ps)
+    q = case["q"].to(gpu)
+
+    def run(rows, room):
+        wide = torch.full((len(rows), -(-room // ps)), -1, dtype=torch.int32, device=gpu)
+        width = min(wide.shape[1], case["table"].shape[1])
+        wide[:, :width] = case["table"][rows, :width]
+        info = case["req_info"][rows].clone()
+        info[:, 0] = torch.arange(len(rows), device=gpu)
+        out = torch.full((len(rows), H * hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+        ops.attention_mfma(q[rows].contiguous(), case["kc"], case["vc"], out, block_table=wide, blocks=None, nb=1, req_info=info,
+                           positions=case["positions"][rows].contiguous(), H=H, Hkv=Hkv, hd=hd, page_size=ps, max_ctx_len=room, window=window)
+        return out
+    everyone = list(range(len(reqs)))
+    together = run(everyone, case["max_ctx_len"])
+    _check_step(case, reqs, together.cpu().double().reshape(-1, H, hd), H, hd, window, ("short rows", hd, window))
+    assert torch.equal(together, run(everyone, 2048 * 256))
+    for r in everyone:
+        assert torch.equal(together[r], run([r], reqs[r][0] + 1)[0]), r
+
+
 @pytest.mark.parametrize("H,Hkv,hd,ps", [(4, 2, 64, 16), (3, 1, 80, 32), (2, 2, 128, 16)])
 @pytest.mark.parametrize("window", [0, 700])
 def test_attention_prefill_key_segments(gpu, H, Hkv, hd, ps, window, monkeypatch):

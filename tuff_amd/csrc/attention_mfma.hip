@@ -659,16 +659,22 @@ constexpr int COMBINE_WAVES = 8;
 constexpr int COMBINE_GROUP = 64;
 constexpr int COMBINE_MAX_GROUPS = COMBINE_MAX_PARTS / COMBINE_GROUP;
 
-// NARROW: heads of up to 64 channels.  Everything a workgroup may need of up to 512 partitions is asked for before the
-// position is known (a wave: the partial outputs of the group of its own number), one trip to memory instead of six one
-// after the other: 118 partitions of 96 rows 13.8 -> 9.0 us.
+// NARROW: heads of up to 64 channels.  The maxima and sums are asked for with the position; when that is known a wave asks for
+// all partial outputs of the group of its own number at once, as far as the token sees them, and takes the weights meanwhile: two
+// trips to memory instead of six one after the other.  A wave with few of them (a short request beside a long one, a
+// window) fetches them behind the weights, sixteen at a time, in less code.  94 registers: two workgroups a CU (one, with 144,
+// takes half as long again where rows are many).  32 heads, the whole attention: 3 requests of 30,000 keys 51.1 -> 46.6 us, one of
+// 30,000 beside 63 of 256 66.8 -> 60.4, 64 requests with a window of 1,024 and room for 30,000 65.5 -> 61.1 (everything asked for
+// before the position, whatever the row: 46.9, 88.9 and 89.3).
 template <bool NARROW>
 __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml,
                                                                             bf16_t* __restrict__ out, const int* __restrict__ positions,
                                                                             int H, int hd, int window, int n_parts, int part_keys,
                                                                             const float* __restrict__ sinks) {
     constexpr int PER_THREAD = COMBINE_MAX_PARTS / (COMBINE_WAVES * WAVE);
+    constexpr int PER = NARROW ? 1 : 4;                    // channels a lane, at most
     constexpr int AHEAD = NARROW ? COMBINE_GROUP : 1;
+    constexpr int FEW = 16;                                // partitions a trip below
     __shared__ float wts[COMBINE_MAX_PARTS], wls[COMBINE_MAX_PARTS];
     __shared__ float grp_acc[COMBINE_MAX_GROUPS][NARROW ? WAVE : 256], grp_l[COMBINE_MAX_GROUPS];
     __shared__ float red[COMBINE_WAVES];
@@ -683,14 +689,18 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
         m_p[k] = load_buffer_float(mbuf, (tid + k * COMBINE_WAVES * WAVE) * 8, 0);
         l_p[k] = load_buffer_float(mbuf, (tid + k * COMBINE_WAVES * WAVE) * 8 + 4, 0);
     }
-    float first[AHEAD];                                    // the partial outputs of group `wave`
-    if constexpr (NARROW) {
-#pragma unroll
-        for (int u = 0; u < AHEAD; ++u)
-            first[u] = load_buffer_float(obuf, lane < hd ? ((wave * COMBINE_GROUP + u) * hd + lane) * 4 : NOWHERE, 0);
-    }
     const int lo = window > 0 ? max(0, pos - window + 1) : 0;
     const int p_lo = lo / part_keys, p_hi = pos / part_keys;          // the token's partitions, absolute numbers
+    float first[AHEAD];                                    // the partial outputs of group `wave`
+    const int first_lo = max(p_lo, wave * COMBINE_GROUP), first_hi = min(p_hi, wave * COMBINE_GROUP + COMBINE_GROUP - 1);
+    const bool ahead = NARROW && first_hi - first_lo >= FEW;
+    if (ahead) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int p = wave * COMBINE_GROUP + u;
+            first[u] = load_buffer_float(obuf, p >= first_lo && p <= first_hi && lane < hd ? (p * hd + lane) * 4 : NOWHERE, 0);
+        }
+    }
     float M = -INFINITY;
 #pragma unroll
     for (int k = 0; k < PER_THREAD; ++k) {
@@ -719,9 +729,9 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
     for (int grp = wave; grp <= g_hi; grp += COMBINE_WAVES) {
         if (grp < g_lo) continue;
         const int a = max(p_lo, grp * COMBINE_GROUP), b = min(p_hi, grp * COMBINE_GROUP + COMBINE_GROUP - 1);
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+        float acc[PER] = {};
         float L = 0.f;
-        if (NARROW && grp == wave) {
+        if (ahead && grp == wave) {
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u) {
                 const int p = grp * COMBINE_GROUP + u;
@@ -734,11 +744,11 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
         } else {
             // the partial outputs of sixteen partitions are asked for together; the sums run in ascending order
             for (int i0 = a; i0 <= b; i0 += 16) {
-                float ov[16][4];
+                float ov[16][PER];
 #pragma unroll
                 for (int u = 0; u < 16; ++u)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
+                    for (int j = 0; j < PER; ++j) {
                         const int d = lane + j * WAVE;
                         ov[u][j] = (j < per && i0 + u <= b && d < hd) ? o[(long long)(i0 + u) * hd + d] : 0.f;
                     }
@@ -749,13 +759,13 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
                         L += wls[i0 + u];
                         if (w > 0.f) {                     // a partition without weight may hold anything
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) acc[j] = fmaf(w, ov[u][j], acc[j]);
+                            for (int j = 0; j < PER; ++j) acc[j] = fmaf(w, ov[u][j], acc[j]);
                         }
                     }
             }
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < PER; ++j) {
             const int d = lane + j * WAVE;
             if (d < hd) grp_acc[grp][d] = acc[j];
         }
@@ -763,12 +773,12 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
     }
     __syncthreads();
     if (wave == 0) {
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+        float acc[PER] = {};
         float L = 0.f;
         for (int grp = g_lo; grp <= g_hi; ++grp) {
             L += grp_l[grp];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 0; j < PER; ++j) {
                 const int d = lane + j * WAVE;
                 if (d < hd) acc[j] += grp_acc[grp][d];
             }
@@ -776,7 +786,7 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
         if (sinks) L += __expf(sink - M);
         const float inv = 1.0f / L;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < PER; ++j) {
             const int d = lane + j * WAVE;
             if (d < hd) out[row * hd + d] = (bf16_t)(acc[j] * inv);
         }
