@@ -64,3 +64,36 @@ def test_narrow_products_of_few_rows_take_slices_only_where_they_are_faster(gemm
     tiles, rows = ctypes.c_int(), ctypes.c_int()
     assert gemm_lib.tuff_gemm_bf16_emit_layout(M, N, K, ctypes.byref(tiles), ctypes.byref(rows)) == 0
     assert tiles.value == -(-N // (64 if emit else 8 if N <= 2048 else 16)) and rows.value == (16 if M <= 16 else 64)
+
+
+@pytest.mark.parametrize("T,R,q,keys,window,H,Hkv,hd,want", [
+    (1, 1, 1, 1, 0, 32, 8, 64, False), (8, 8, 1, 4, 0, 32, 32, 64, False), (256, 256, 1, 40, 0, 32, 32, 64, False),
+    (128, 128, 1, 20, 0, 8, 8, 128, False), (64, 64, 1, 20000, 4, 32, 32, 64, False),
+    (256, 256, 1, 40, 0, 32, 8, 64, True), (1, 1, 1, 300, 0, 32, 32, 64, True), (4, 4, 1, 1000, 0, 32, 8, 64, True),
+    (500, 1, 500, 500, 0, 32, 8, 64, True), (2000, 1, 2000, 2000, 64, 8, 8, 128, True), (128, 128, 1, 600, 0, 8, 8, 128, True)])
+def test_float32_attention_takes_the_kernel_that_is_faster(T, R, q, keys, window, H, Hkv, hd, want):
+    """Sizes that were measured with both kernels (the same bits): few keys and workgroups of few columns go to the general one."""
+    from tuff_amd.csrc import ops
+    assert ops.attention_f32_pays(T, R, q, keys, window, H, Hkv, hd) is want
+
+
+def test_float32_attention_of_a_mixer_follows_that_rule(monkeypatch):
+    import types
+
+    import torch
+
+    from tuff_amd.csrc import ops
+    from tuff_amd.parts.attention import PagedAttention
+    taken = []
+    for name in ("attention_f32", "attention_general"):
+        monkeypatch.setattr(ops, name, lambda *a, _n=name, **k: taken.append(_n))
+    mixer = PagedAttention.__new__(PagedAttention)
+    mixer.H = mixer.Hkv = 32
+    mixer.hd = mixer.vd = 64
+    mixer.sinks = mixer.slopes = mixer.window = mixer.scale = None
+    cache = types.SimpleNamespace(k=None, v=None, page_size=16)
+    group = types.SimpleNamespace(block_table=None)
+    for keys in (4, 4000):
+        ctx = types.SimpleNamespace(T=8, R=8, max_q_len=1, max_ctx_len=keys, req_info=None, req_of_token=None, positions=None)
+        mixer.attend(torch.zeros(8, 32 * 64), None, ctx, cache, group)
+    assert taken == ["attention_general", "attention_f32"]

@@ -988,6 +988,30 @@ def attention_f32_supported(dtype, H: int, Hkv: int, hd: int, page_size: int) ->
     return dtype == torch.float32 and hd in (16, 32, 64, 128) and H % Hkv == 0 and H // Hkv <= 16 and page_size % 16 == 0
 
 
+# Microseconds of a workgroup of attention_f32 with the chip full of them, by head size: of two columns and one tile of 64 keys.
+_F32_WORKGROUP = {16: 5.6e-3, 32: 7e-3, 64: 10.5e-3, 128: 28e-3}
+
+
+def attention_f32_pays(T: int, R: int, max_q_len: int, max_ctx_len: int, window: int, H: int, Hkv: int, hd: int) -> bool:
+    """Whether attention_f32 is faster than attention_general, which gives the same bits, by what the sizes cost either.  A
+    workgroup of the first takes a tile of 64 keys for up to 16 columns whatever it holds; a wave of the second takes a key
+    after the other for one column.  So few keys, or many requests with few heads to a kv head, go the second way: 256 requests of
+    40 keys, 32 heads and kv heads of 64: 85 us and 61; 8 of 4 keys 7.2 and 6.0; 256 of 40 keys with 8 kv heads 27 and 55;
+    one of 300 keys 18 and 77.  The constants are fitted to 1 to 256 requests of 1 to 4,000 keys and seven arrangements of heads
+    (nowhere is the one taken slower than the other by more than a quarter; over all of them by 0.4 %)."""
+    G = H // Hkv
+    per = 16 // G                                          # tokens a workgroup
+    keys = min(max_ctx_len, window) if window else max_ctx_len
+    tiles = -(-keys // 64)
+    groups = max(R, -(-T // per)) * Hkv
+    columns = min(-(-T // max(R, 1)), per) * G
+    causal = 0.6 if max_q_len * 2 > max_ctx_len and max_q_len > 1 else 1.0
+    general = 4.5 + max(keys * (0.165 + 0.001 * hd), T * H * keys * (0.03 + 0.0022 * hd) * 1e-3 * causal)
+    tiled = 3.5 + max(2.0 + 0.028 * hd + (-(-columns // 4) - 1) * (0.6 + 0.006 * hd) + (tiles - 1) * (1.6 + 0.015 * hd),
+                      groups * _F32_WORKGROUP[hd] * (0.45 + 0.55 * tiles))
+    return tiled < general
+
+
 def attention_f32(q, k_cache, v_cache, out, *, block_table, req_info, max_q_len, H, Hkv, hd, page_size, window=0, scale=None) -> None:
     """attention_general on the matrix cores, the same bits: float32, values as wide as keys, no sinks and slopes.
     req_info int32 [R, 4]: (first token, tokens, position of the first token, length); max_q_len: the most tokens of a request."""

@@ -153,7 +153,8 @@ class PagedAttention:
             ops.attention_mfma(q, cache.k, cache.v, o, blocks=blocks, nb=nb, positions=ctx.positions, **common)
             return
         if (self.vd == self.hd and self.sinks is None and self.slopes is None
-                and ops.attention_f32_supported(q.dtype, self.H, self.Hkv, self.hd, cache.page_size)):
+                and ops.attention_f32_supported(q.dtype, self.H, self.Hkv, self.hd, cache.page_size)
+                and ops.attention_f32_pays(ctx.T, ctx.R, ctx.max_q_len, ctx.max_ctx_len, self.window or 0, self.H, self.Hkv, self.hd)):
             ops.attention_f32(q, cache.k, cache.v, o, block_table=g.block_table, req_info=ctx.req_info, max_q_len=ctx.max_q_len,
                               H=self.H, Hkv=self.Hkv, hd=self.hd, page_size=cache.page_size, window=self.window or 0, scale=self.scale)
             return
