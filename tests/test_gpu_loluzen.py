@@ -390,6 +390,27 @@ def test_mix_of_heads_against_the_sum_in_float64(gpu, H, Hkv, vd):
             assert (err <= (H + 8) * 2.0 ** -24 * size * f + unit * (want * f).abs()).all(), (dt, gated)
 
 
+@pytest.mark.parametrize("H, Hkv, vd", [(32, 2, 64), (24, 2, 130), (12, 2, 65), (20, 2, 33), (8, 1, 256), (4, 2, 512), (6, 1, 70), (3, 1, 64)])
+def test_mix_of_heads_of_few_tokens_and_of_many(gpu, H, Hkv, vd):
+    """Kv heads of 2, 3, 6, 10, 12 and 16 heads: few tokens (a wave for every 64 channels) and many (a wave all of them) to the same
+    bits, and those to H + 1 float32 roundings of the sum in float64."""
+    from tuff_amd.csrc import ops
+    T = 1024 * 4 // H + 5
+    gen = torch.Generator().manual_seed(H * vd)
+    o, talk = (torch.randn(*s, generator=gen) for s in ((T, H * Hkv * vd), (H, H)))
+    od, td = o.to(gpu), talk.to(gpu)
+    out = torch.full((T, H * vd), float("nan"), device=gpu)
+    ops.head_mix_gate(od, out, H=H, Hkv=Hkv, vd=vd, talk=td)
+    for t0, n in ((0, 1), (T - 7, 7)):
+        few = torch.full((n, H * vd), float("nan"), device=gpu)
+        ops.head_mix_gate(od[t0:t0 + n].contiguous(), few, H=H, Hkv=Hkv, vd=vd, talk=td)
+        assert torch.equal(few, out[t0:t0 + n])
+    picked = o.double().view(T, H, Hkv, vd)[:, :, torch.arange(H) // (H // Hkv), :]
+    want = torch.stack([(talk[h].double()[None, :, None] * picked[:, :, h]).sum(1) for h in range(H)], 1)
+    size = torch.stack([(talk[h].double().abs()[None, :, None] * picked[:, :, h].abs()).sum(1) for h in range(H)], 1)
+    assert ((out.cpu().double().view(T, H, vd) - want).abs() <= (H + 1) * 2.0 ** -24 * size).all()
+
+
 @pytest.mark.parametrize("D", [24, 64, 68, 128, 256])
 def test_scan_gives_the_same_bits_for_any_company_and_alignment(gpu, D):
     """The recurrence's kernel over nine requests of 0 to 41 tokens (edges of the eight tokens it stages at a time), with

@@ -401,16 +401,19 @@ __global__ __launch_bounds__(WAVE) void head_mix_gate_kernel(const TI* __restric
     }
 }
 
-// The mix for the G heads of a kv head at once: a wave a (token, kv head), which reads every weighted sum once instead of G
-// times, eight heads' at a time.  Bound by the float32 sums: 2,048 tokens, 32 heads, 8 kv heads of 64:
-// 82 -> 28.5 us.  For 2, 4 and 8 heads a kv head; the kernel above takes the others, and the gates alone.
-template <int G, typename TI, typename T>
+// The mix for G heads of one kv head at once: a wave a (token, G heads, 64 channels), which reads every weighted sum once instead
+// of G times, eight heads' at a time.  Bound by the float32 sums: 2,048 tokens, 32 heads, 8 kv heads of 64:
+// 82 -> 28.5 us.  Two heads, or four where a kv head has a multiple of four (eight keep 64 coefficients under way and take
+// longer: 16 heads, 2 kv heads, one token 6.7 us, in fours 4.0); the kernel above takes odd numbers, and the gates alone.
+template <int G, bool SPLIT, typename TI, typename T>
 __global__ __launch_bounds__(WAVE) void head_mix_group_kernel(const TI* __restrict__ o, const float* __restrict__ talk,
                                                               const float* __restrict__ gates, int gate_stride,
-                                                              T* __restrict__ out, int H, int Hkv, int vd) {
+                                                              T* __restrict__ out, int H, int Hkv, int vd, int parts, int steps) {
     const long long t = blockIdx.x;
-    const int kvh = blockIdx.y;
-    for (int j = threadIdx.x; j < vd; j += WAVE) {
+    // SPLIT: blockIdx.z says which G of the kv head's parts * G heads, and which of `steps` blocks of 64 channels to begin with
+    const int kvh = blockIdx.y, part = SPLIT ? blockIdx.z / steps : 0;
+    const int h0 = (SPLIT ? kvh * parts + part : kvh) * G;
+    for (int j = (SPLIT ? (blockIdx.z - part * steps) * WAVE : 0) + threadIdx.x; j < vd; j += SPLIT ? steps * WAVE : WAVE) {
         const TI* src = o + (t * H * Hkv + kvh) * vd + j;
         float acc[G] = {};
         int q = 0;
@@ -421,16 +424,25 @@ __global__ __launch_bounds__(WAVE) void head_mix_group_kernel(const TI* __restri
 #pragma unroll
             for (int u = 0; u < 8; ++u)
 #pragma unroll
-                for (int g = 0; g < G; ++g) acc[g] = fmaf(talk[(kvh * G + g) * H + q + u], to_f32(ov[u]), acc[g]);
+                for (int g = 0; g < G; ++g) acc[g] = fmaf(talk[(h0 + g) * H + q + u], to_f32(ov[u]), acc[g]);
+        }
+        for (; q + 4 <= H; q += 4) {
+            TI ov[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) ov[u] = src[(long long)(q + u) * Hkv * vd];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int g = 0; g < G; ++g) acc[g] = fmaf(talk[(h0 + g) * H + q + u], to_f32(ov[u]), acc[g]);
         }
         for (; q < H; ++q) {
             const float ov = to_f32(src[(long long)q * Hkv * vd]);
 #pragma unroll
-            for (int g = 0; g < G; ++g) acc[g] = fmaf(talk[(kvh * G + g) * H + q], ov, acc[g]);
+            for (int g = 0; g < G; ++g) acc[g] = fmaf(talk[(h0 + g) * H + q], ov, acc[g]);
         }
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            const int h = kvh * G + g;
+            const int h = h0 + g;
             const float gate = gates ? 1.0f / (1.0f + expf(-gates[t * gate_stride + h])) : 1.f;
             out[(t * H + h) * vd + j] = from_f32<T>(acc[g] * gate);
         }
@@ -444,9 +456,16 @@ TUFF_EXPORT int tuff_head_mix_gate(const void* o, int in_dt, const float* talk, 
     if (n_tokens <= 0) return 0;
     if (H <= 0 || Hkv <= 0 || H % Hkv || H > 65535 || vd <= 0) return -2;
     dim3 grid(n_tokens, H), block(WAVE);
-    const int group = talk && Hkv < H ? H / Hkv : 0;                 // heads that read the same sums
-#define GROUP(G, TI, T) hipLaunchKernelGGL((head_mix_group_kernel<G, TI, T>), dim3(n_tokens, Hkv), block, 0, stream, (const TI*)o, talk, gates, gate_stride, (T*)out, H, Hkv, vd)
-#define LAUNCH(TI, T) do { if (group == 2) GROUP(2, TI, T); else if (group == 4) GROUP(4, TI, T); else if (group == 8) GROUP(8, TI, T); \
+    const int share = talk ? H / Hkv : 1;                            // heads that read the same sums
+    const int group = share % 4 == 0 ? 4 : share % 2 == 0 ? 2 : 1;
+    // Fewer waves than the chip has SIMDs: a wave for every 64 channels.  (4 heads of 512, one token: 7.6 -> 3.4 us; from
+    // 2,000 waves on it is slower, 10.4 us against 8.5.)
+    const int pieces = ceil_div(vd, WAVE);
+    const int steps = (long long)n_tokens * (H / group) < 1024 && (long long)(share / group) * pieces <= 65535 ? pieces : 1;
+#define GROUP_SPLIT(G, SPLIT, TI, T) hipLaunchKernelGGL((head_mix_group_kernel<G, SPLIT, TI, T>), dim3(n_tokens, Hkv, share / G * steps), block, 0, stream, \
+                                     (const TI*)o, talk, gates, gate_stride, (T*)out, H, Hkv, vd, share / G, steps)
+#define GROUP(G, TI, T) do { if (share / G * steps > 1) GROUP_SPLIT(G, true, TI, T); else GROUP_SPLIT(G, false, TI, T); } while (0)
+#define LAUNCH(TI, T) do { if (group == 2) GROUP(2, TI, T); else if (group == 4) GROUP(4, TI, T); \
                            else hipLaunchKernelGGL((head_mix_gate_kernel<TI, T>), grid, block, 0, stream, (const TI*)o, talk, gates, gate_stride, (T*)out, H, Hkv, vd); } while (0)
     if (in_dt == DT_F32 && dt == DT_F32) LAUNCH(float, float);
     else if (in_dt == DT_F32) LAUNCH(float, bf16_t);
@@ -454,6 +473,7 @@ TUFF_EXPORT int tuff_head_mix_gate(const void* o, int in_dt, const float* talk, 
     else return -2;
 #undef LAUNCH
 #undef GROUP
+#undef GROUP_SPLIT
     return launch_status();
 }
 
