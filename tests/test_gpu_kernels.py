@@ -65,6 +65,20 @@ def test_gemm_f32_matrix_cores(gpu, M, N, K):
             assert torch.equal(some, out[M - m:]), m
 
 
+def test_gemm_f32_more_rows_than_small_blocks_count(gpu):
+    """A narrow output of more rows than a grid has blocks of 32 for takes blocks of 64 (it was refused)."""
+    from tuff_amd.csrc import ops
+    M, N, K = 32 * 65535 + 1, 8, 32
+    x, w = torch.randn(M, K, device=gpu, generator=torch.Generator(gpu).manual_seed(5)), _r(N, K, seed=2).to(gpu)
+    out = torch.full((M, N), float("nan"), device=gpu)
+    ops.gemm(x, w, out)
+    bound = K * 2.0 ** -24 * (x.abs() @ w.abs().T).double() * 1.001          # any order of K additions
+    assert ((out.double() - x.double() @ w.double().T).abs() <= bound).all()
+    some = torch.empty(16, N, device=gpu)
+    ops.gemm(x[M - 16:], w, some)
+    assert torch.equal(some, out[M - 16:])
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 8), (5, 1000, 96), (17, 33, 40), (64, 777, 240), (65, 130, 136),
                                    (200, 300, 328), (300, 64, 2048), (128, 128, 64), (2, 2048, 8192),
                                    (72, 2048, 8192), (512, 2050, 2048), (130, 1026, 1000),

@@ -249,6 +249,8 @@ TUFF_EXPORT int tuff_gemm_f32(const float* X, const float* W, float* Y, int M, i
         return launch_status();
     }
     if (M <= 16) return launch_chain<1, 1, 8>(X, W, Y, M, N, K, accumulate, stream);
-    if (block_cycles(M, N, 32) < block_cycles(M, N, 64)) return launch_chain<1, 2, 4>(X, W, Y, M, N, K, accumulate, stream);
+    constexpr int MOST_BLOCKS = 65535;                    // of rows in a grid
+    if (ceil_div(M, 32) <= MOST_BLOCKS && block_cycles(M, N, 32) < block_cycles(M, N, 64))
+        return launch_chain<1, 2, 4>(X, W, Y, M, N, K, accumulate, stream);
     return launch_chain<2, 2, 4>(X, W, Y, M, N, K, accumulate, stream);
 }
