@@ -79,6 +79,24 @@ def test_gemm_f32_more_rows_than_small_blocks_count(gpu):
     assert torch.equal(some, out[M - 16:])
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 16, 2 ** 22), (300, 40, 2 ** 22 + 64), (64, 72, 2 ** 22 + 64)])
+def test_gemm_bf16_very_long_inner_size(gpu, M, N, K):
+    """Where 256 rows have more bytes than 31 bits count, a product of more than 64 rows goes through registers."""
+    from tuff_amd.csrc import ops
+    g = torch.Generator(gpu).manual_seed(3)
+    x = torch.randn(M, K, device=gpu, dtype=torch.bfloat16, generator=g)
+    w = torch.randn(N, K, device=gpu, dtype=torch.bfloat16, generator=g)
+    want, size = torch.zeros(M, N, device=gpu, dtype=torch.float64), 0.0
+    for k in range(0, K, 2 ** 18):
+        a, b = x[:, k:k + 2 ** 18].double(), w[:, k:k + 2 ** 18].double()
+        want += a @ b.T
+        size = size + a.abs() @ b.abs().T
+    out = torch.full((M, N), float("nan"), device=gpu)
+    ops.gemm(x, ops.tile_weight(w), out)
+    # random signs: rounding errors of the K additions add up like their square root; four times that
+    assert ((out.double() - want).abs() <= 4 * K ** 0.5 * 2.0 ** -24 * want.abs().max() + 2.0 ** -24 * size).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 16, 8), (5, 1000, 96), (17, 33, 40), (64, 777, 240), (65, 130, 136),
                                    (200, 300, 328), (300, 64, 2048), (128, 128, 64), (2, 2048, 8192),
                                    (72, 2048, 8192), (512, 2050, 2048), (130, 1026, 1000),

@@ -9,7 +9,7 @@
 //
 // Three kernels, chosen by the sizes on the host:
 //  * tiled     M > 64: 128x128 or 256x256 block tiles staged through LDS (compute bound), in two
-//    forms: operands loaded straight into LDS (K a multiple of 64) or through registers (other K);
+//    forms: operands loaded straight into LDS (K a multiple of 64, up to 2^22) or through registers (other K);
 //  * skinny64  up to 64 rows that skinny16 does not take: a workgroup owns 64 rows of W, one MFMA column
 //    tile a wave; the activations of a K chunk are staged once in LDS for all four waves (bandwidth bound);
 //  * skinny16  M <= 16, and up to 32 rows (two row tiles a wave) where few_rows_kernel() says so:
@@ -1281,6 +1281,12 @@ __global__ __launch_bounds__(FC_ROWS * 16) void splitk_finish_conv_kernel(const 
 
 struct SkinnyPlan { int tiles, waves, slices, chunks_per_slice, cols; long long ws_floats; };
 
+// The kernels count bytes inside a buffer, which is a block's rows of X or of W, in 31 bits: 64 rows at most in those for few rows,
+// 256 in the tiled one that loads straight into LDS.  The one through registers counts elements in 32.
+constexpr int LARGEST_K = (1 << 24) - 64, LARGEST_K_DMA = (1 << 22) - TBK;
+bool inner_ok(int K) { return K % 8 == 0 && K <= LARGEST_K; }
+bool dma_ok(int K) { return K % TBK == 0 && K <= LARGEST_K_DMA; }
+
 constexpr int SKINNY_ROWS = 32;     // the most rows of the kernel whose waves split K inside the workgroup (two row tiles)
 
 // 17 to 64 rows and a wide output with a short K (gate and up of a feed-forward): the tiled product with one
@@ -1366,10 +1372,10 @@ TiledPlan plan_tiled(int M, int N, int K) {
     TiledPlan t;
     t.shape = large >= 160 ? 0 : small > 256 ? 1 : 2;
     t.slices = 1; t.steps_per_slice = nk; t.ws_floats = 0;
-    if (tiled_shape_forced >= 0 && K % TBK == 0) { t.shape = tiled_shape_forced; return t; }
+    if (tiled_shape_forced >= 0 && dma_ok(K)) { t.shape = tiled_shape_forced; return t; }
     // blocks of 256 x 192 where they need fewer rounds of 256 workgroups times columns than 256 x 256
     // (6144 columns and 2048 rows: 256 blocks, one round, instead of 192 blocks that leave a quarter of the CUs idle)
-    if (t.shape == 0 && K % TBK == 0) {
+    if (t.shape == 0 && dma_ok(K)) {
         const long long wide = (long long)ceil_div(N, 192) * ceil_div(M, 256);
         if (ceil_div(wide, 256) * 192 < ceil_div(large, 256) * 256) t.shape = 4;
         return t;
@@ -1377,14 +1383,14 @@ TiledPlan plan_tiled(int M, int N, int K) {
     // A little more than one round of pairs of 128 x 128 blocks (512 of them side by side), where blocks of 256 x 256
     // would be too few for the CUs: the blocks beyond the round run a second one almost alone.  Blocks of 256 x 192
     // in one round instead (4608 columns and 2048 rows, K = 1536: 37.1 us instead of 43.8; 256 x 256: 45.7).
-    if (t.shape == 1 && small > 512 && K % TBK == 0) {
+    if (t.shape == 1 && small > 512 && dma_ok(K)) {
         const long long wide = (long long)ceil_div(N, 192) * ceil_div(M, 256);
         if (wide <= 256) { t.shape = 4; return t; }
     }
     // few blocks and a short K: blocks of 64 x 64 give enough workgroups without slices of K, whose partial
     // tiles cost a second kernel and as much traffic as the product's own (K = 1536 .. 2048, 96 to 512
     // rows: 9 to 14 us instead of 11 to 19); beyond 48 steps the slices win
-    if (t.shape == 2 && small <= 128 && K % TBK == 0 && nk <= 48) { t.shape = 3; return t; }
+    if (t.shape == 2 && small <= 128 && dma_ok(K) && nk <= 48) { t.shape = 3; return t; }
     if (t.shape == 2 && small <= 128) {
         // as many slices as give every CU at most one block, at least eight steps a slice
         int s = max(1, min((int)(256 / small), nk / 8));
@@ -1522,13 +1528,13 @@ int launch_skinny64_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N
 int tiled_emit_group(int M, int N, int K) {
     const TiledPlan t = plan_tiled(M, N, K);
     if (t.slices > 1) return 64;                        // the kernel that adds the slices emits, 64 columns a workgroup
-    if (K % TBK != 0) return 0;
+    if (!dma_ok(K)) return 0;
     const int bn = t.shape == 0 ? 256 : t.shape == 4 ? 192 : t.shape == 3 ? 64 : 128;
     if (N % bn != 0) return 0;
     return bn;                                          // a workgroup's columns
 }
 
-bool tiled_scaled_ok(int M, int N, int K) { return K % TBK == 0 || plan_tiled(M, N, K).slices > 1; }
+bool tiled_scaled_ok(int M, int N, int K) { return dma_ok(K) || plan_tiled(M, N, K).slices > 1; }
 
 template <int MODE, int AROUND = TILED_PLAIN>
 int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, float* ws, hipStream_t stream,
@@ -1569,9 +1575,9 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
                                X, W, Y, M, N, K, t.steps_per_slice, ws, ex); \
         } while (0)
         if constexpr (AROUND != TILED_PLAIN) {
-            if (K % TBK != 0 && t.slices == 1) return -2;            // a product in slices is finished by the kernel that adds them
+            if (!dma_ok(K) && t.slices == 1) return -2;            // a product in slices is finished by the kernel that adds them
         }
-        if (K % TBK == 0) {
+        if (dma_ok(K)) {
             if (t.shape == 3) TILED_DMA(2, 2, 2, 2, 4);
             else if (t.shape == 4) TILED_DMA(8, 3, 2, 4, 2);
             else if (t.shape == 0) TILED_DMA(8, 4, 2, 4, 2);
@@ -1636,7 +1642,7 @@ TUFF_EXPORT int tuff_gemm_bf16_emit_layout(int M, int N, int K, int* tiles, int*
 // 1 if tuff_gemm_bf16_scaled takes a product of these sizes (always for M <= 64; for more rows where the
 // tiled product runs it in one piece), else 0.
 TUFF_EXPORT int tuff_gemm_bf16_scaled_supported(int M, int N, int K) {
-    if (K % 8 != 0 || M <= 0 || N <= 0) return 0;
+    if (!inner_ok(K) || M <= 0 || N <= 0) return 0;
     return M <= 64 || tiled_scaled_ok(M, N, K) ? 1 : 0;
 }
 
@@ -1651,11 +1657,11 @@ TUFF_EXPORT int tuff_gemm_bf16_workspace(int M, int N, int K, int emit, long lon
 }
 
 // W: tile-major, as described at the head of this file (ceil(N/16) * ceil(K/32) blocks of 1 KB).
-// K must be a multiple of 8 (16-byte operand loads); the host wrapper refuses other K.
+// K must be a multiple of 8 (16-byte operand loads), here and below, and at most 2^24 - 64 (else -2); the host wrapper refuses other K.
 TUFF_EXPORT int tuff_gemm_bf16(const void* X, const void* W, void* Y, int M, int N, int K, int mode,
                                float* ws, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (K % 8 != 0) return -2;
+    if (!inner_ok(K)) return -2;
     const bf16_t* x = (const bf16_t*)X;
     const bf16_t* w = (const bf16_t*)W;
     if (mode == OUT_BF16) return launch_mode<OUT_BF16>(x, w, Y, M, N, K, ws, stream);
@@ -1674,7 +1680,7 @@ TUFF_EXPORT int tuff_gemm_bf16(const void* X, const void* W, void* Y, int M, int
 TUFF_EXPORT int tuff_gemm_bf16_normed(const float* X, const int* rows, long long ldx, const float* norm_w, float eps, const void* W,
                                       void* Y, int M, int N, int K, int mode, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (K % 8 != 0 || K > 8192 || M > 16 || ldx < K || ldx % 4 || (uintptr_t)X % 16) return -2;
+    if (!inner_ok(K) || K > 8192 || M > 16 || ldx < K || ldx % 4 || (uintptr_t)X % 16) return -2;
     Skinny16Extra x;
     x.norm_w = norm_w; x.eps = eps; x.rows = rows; x.ldx = ldx;
     return launch_skinny16_mode<NORM_INSIDE>(X, (const bf16_t*)W, Y, M, N, K, mode, x, stream);
@@ -1688,7 +1694,7 @@ TUFF_EXPORT int tuff_gemm_bf16_normed(const float* X, const int* rows, long long
 TUFF_EXPORT int tuff_gemm_bf16_accum_emit(const void* X, const void* W, float* Y, int M, int N, int K,
                                           const float* next_norm_w, void* xw, float* ss, float* ws, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (K % 8 != 0) return -2;
+    if (!inner_ok(K)) return -2;
     if (M > 64) {
         if (!tiled_emit_group(M, N, K)) return -2;
         TiledExtra t;
@@ -1712,7 +1718,7 @@ TUFF_EXPORT int tuff_gemm_bf16_accum_emit(const void* X, const void* W, float* Y
 TUFF_EXPORT int tuff_gemm_bf16_scaled(const void* XW, const float* ss, int n_ss, float eps, const void* W, void* Y,
                                       int M, int N, int K, int mode, float* ws, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
-    if (K % 8 != 0 || n_ss < 1) return -2;
+    if (!inner_ok(K) || n_ss < 1) return -2;
     if (M > 64 || (rows64_tiled(M, N, K) && (mode == OUT_BF16 || mode == OUT_SWIGLU))) {
         // ss [n_ss][M] ([n_ss][64] from a product of at most 64 rows); bfloat16 and SwiGLU outputs (what reads a norm in a layer)
         if (!tiled_scaled_ok(M, N, K)) return -2;
@@ -1752,7 +1758,7 @@ TUFF_EXPORT int tuff_gemm_bf16_conv64(const void* X, const float* ss, int n_ss, 
                                       int M, int d, int K, const void* taps, int taps_dt, int n_taps, float* state,
                                       const int* state_slot, float* ws, hipStream_t stream) {
     if (M <= 0 || d <= 0) return 0;
-    if (K % 8 != 0 || M <= SKINNY_ROWS || M > 64 || d % 16 != 0 || n_taps < 2 || n_taps - 1 > CONV_MAX_TAPS) return -2;
+    if (!inner_ok(K) || M <= SKINNY_ROWS || M > 64 || d % 16 != 0 || n_taps < 2 || n_taps - 1 > CONV_MAX_TAPS) return -2;
     ConvTail cv;
     cv.taps_w = taps; cv.taps_dt = taps_dt; cv.taps = n_taps; cv.state = state; cv.state_slot = state_slot;
     FinishExtra x;
@@ -1769,7 +1775,7 @@ TUFF_EXPORT int tuff_gemm_bf16_conv(const void* X, int norm_kind, const float* n
                                     const void* taps, int taps_dt, int n_taps, float* state, const int* state_slot,
                                     hipStream_t stream) {
     if (M <= 0 || d <= 0) return 0;
-    if (K % 8 != 0 || M > SKINNY_ROWS || d % 16 != 0 || n_taps < 2 || n_taps - 1 > CONV_MAX_TAPS) return -2;
+    if (!inner_ok(K) || M > SKINNY_ROWS || d % 16 != 0 || n_taps < 2 || n_taps - 1 > CONV_MAX_TAPS) return -2;
     if (norm_kind == 1 && M > 16) return -2;
     Skinny16Extra x;
     x.conv.taps_w = taps; x.conv.taps_dt = taps_dt; x.conv.taps = n_taps; x.conv.state = state; x.conv.state_slot = state_slot;
