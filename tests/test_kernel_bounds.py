@@ -68,7 +68,7 @@ def test_narrow_products_of_few_rows_take_slices_only_where_they_are_faster(gemm
 
 @pytest.mark.parametrize("T,R,q,keys,window,H,Hkv,hd,want", [
     (1, 1, 1, 1, 0, 32, 8, 64, False), (8, 8, 1, 4, 0, 32, 32, 64, False), (256, 256, 1, 40, 0, 32, 32, 64, False),
-    (128, 128, 1, 20, 0, 8, 8, 128, False), (64, 64, 1, 20000, 4, 32, 32, 64, False),
+    (128, 128, 1, 20, 0, 8, 8, 128, False), (64, 64, 1, 20000, 4, 32, 32, 64, False), (65536, 65536, 1, 600, 0, 16, 1, 64, False),
     (256, 256, 1, 40, 0, 32, 8, 64, True), (1, 1, 1, 300, 0, 32, 32, 64, True), (4, 4, 1, 1000, 0, 32, 8, 64, True),
     (500, 1, 500, 500, 0, 32, 8, 64, True), (2000, 1, 2000, 2000, 64, 8, 8, 128, True), (128, 128, 1, 600, 0, 8, 8, 128, True)])
 def test_float32_attention_takes_the_kernel_that_is_faster(T, R, q, keys, window, H, Hkv, hd, want):

@@ -999,6 +999,8 @@ def attention_f32_pays(T: int, R: int, max_q_len: int, max_ctx_len: int, window:
     40 keys, 32 heads and kv heads of 64: 85 us and 61; 8 of 4 keys 7.2 and 6.0; 256 of 40 keys with 8 kv heads 27 and 55;
     one of 300 keys 18 and 77.  The constants are fitted to 1 to 256 requests of 1 to 4,000 keys and seven arrangements of heads
     (nowhere is the one taken slower than the other by more than a quarter; over all of them by 0.4 %)."""
+    if R > 65535:                                          # (a grid has no more there)
+        return False
     G = H // Hkv
     per = 16 // G                                          # tokens a workgroup
     keys = min(max_ctx_len, window) if window else max_ctx_len
