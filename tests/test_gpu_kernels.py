@@ -79,6 +79,20 @@ def test_gemm_f32_more_rows_than_small_blocks_count(gpu):
     assert torch.equal(some, out[M - 16:])
 
 
+@pytest.mark.parametrize("M,N,K", [(400, 2570, 320), (1100, 2100, 4224), (160, 2048, 5632), (160, 2056, 1536), (700, 4610, 1536), (1290, 8200, 128)])
+def test_gemm_bf16_blocks_that_reach_beyond_the_matrix(gpu, M, N, K):
+    """Blocks of each shape with rows and columns that are not there, through global loads (more blocks of 64 x 64 than CUs, a long
+    K, blocks of 256 x 192) and through buffers: nothing beyond the operands counts."""
+    from tuff_amd.csrc import ops
+    x = torch.full((M + 300, K), float("nan"), device=gpu, dtype=torch.bfloat16)
+    x[:M] = _r(M, K, seed=1).to(gpu)
+    w = _r(N, K, seed=2, dtype=torch.bfloat16).to(gpu)
+    a, b = x[:M].double(), w.double()
+    out = torch.full((M, N), float("nan"), device=gpu)
+    ops.gemm(x[:M], ops.tile_weight(w), out)
+    assert ((out.double() - a @ b.T).abs() <= K * 2.0 ** -24 * (a.abs() @ b.abs().T)).all()      # any order of K additions
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 16, 2 ** 22), (300, 40, 2 ** 22 + 64), (64, 72, 2 ** 22 + 64)])
 def test_gemm_bf16_very_long_inner_size(gpu, M, N, K):
     """Where 256 rows have more bytes than 31 bits count, a product of more than 64 rows goes through registers."""

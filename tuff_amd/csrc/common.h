@@ -76,6 +76,13 @@ __device__ __forceinline__ void load_to_lds(buffer_t buf, void* lds, int offset,
 #endif
 }
 
+// The same from this lane's address, through a global load.
+__device__ __forceinline__ void load_to_lds(const void* from, void* lds) {
+#ifdef __HIP_DEVICE_COMPILE__
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)from, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+#endif
+}
+
 // An offset that lies beyond every buffer: the lane reads zero.  (A lane's offset is held against the buffer's size less the
 // wave's scalar offset, so that one must not be larger than the buffer even where no lane reads.)
 constexpr int NOWHERE = (int)0x80000000;

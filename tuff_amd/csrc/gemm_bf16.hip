@@ -292,7 +292,12 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_tiled_kernel
 // 35.1 -> 27.4, 2048 x 8192 102.7 -> 81.3, 16384 x 2048 157.6 -> 148.6, 6144 x 2048 69.0 -> 61.2.
 // With all CUs busy and random operands the clock, not the instruction stream, sets the pace: the
 // same loop over constant data runs a quarter faster.
-template <int TM, int TN, int WAVES_M, int WAVES_N, int STAGES, int MODE, int AROUND>
+//
+// BUFFER: the loads go through buffers, which leaves the compiler its count of the LDS reads under way (load_to_lds); else they are
+// global loads, and it waits for more of them.  Buffers win where the whole grid runs side by side, one block a CU, and K is
+// short, and with the blocks of 256 x 256; they lose a little where the operands come slower than the waves could go on:
+// see dma_through_buffer.
+template <int TM, int TN, int WAVES_M, int WAVES_N, int STAGES, bool BUFFER, int MODE, int AROUND>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* __restrict__ Y, int M, int N, int K,
         int steps_per_slice, float* __restrict__ ws, TiledExtra ex) {
@@ -319,26 +324,42 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     const int last_a = (int)min((long long)BM - 1, (long long)M - 1 - m0);
     const int last_tile = (int)min((long long)BN / 16 - 1, (N - 1 - n0) / 16);
     // instruction q of X (q = wave + NW i) fills rows 8 q .. 8 q + 7; instruction q of W fills block q % 2 of row tile q / 2;
-    // offsets in bytes from the block's first row (tile), rows beyond the matrix read its last one
-    int offa[IA], offb[IB];
+    // offsets from the block's first row (tile), in bytes (global loads: in elements).  Rows and tiles beyond the matrix have results
+    // that are never stored.  Through buffers they are not fetched: if they read the last one instead, all blocks ask for the same
+    // line again and again, and 160 rows took longer than 256 (2,048 x 5,632: 20.1 us against 18.1, now 15.9).
+    unsigned offa[IA], offb[IB];
 #pragma unroll
-    for (int i = 0; i < IA; ++i)
-        offa[i] = (min((wave + NW * i) * 8 + lane / 8, last_a) * K + (((lane % 8) ^ (lane / 8)) * 8)) * 2;
+    for (int i = 0; i < IA; ++i) {
+        const int row = (wave + NW * i) * 8 + lane / 8, piece = ((lane % 8) ^ (lane / 8)) * 8;
+        if (BUFFER) offa[i] = row <= last_a ? (unsigned)(row * K + piece) * 2 : (unsigned)NOWHERE;
+        else offa[i] = (unsigned)min(row, last_a) * (unsigned)K + piece;
+    }
 #pragma unroll
     for (int i = 0; i < IB; ++i) {
-        const int q = wave + NW * i;
-        offb[i] = (min(q / 2, last_tile) * kb + q % 2) * 1024 + lane * 16;
+        const int q = wave + NW * i, tile = q / 2;
+        if (BUFFER) offb[i] = tile <= last_tile ? (unsigned)(tile * kb + q % 2) * 1024 + lane * 16 : (unsigned)NOWHERE;
+        else offb[i] = ((unsigned)min(tile, last_tile) * (unsigned)kb + q % 2) * 512 + lane * 8;
     }
     const buffer_t xbuf = make_buffer(X + m0 * K, (last_a + 1) * K * 2);
     const buffer_t wbuf = make_buffer(W + (n0 / 16) * (long long)kb * 512, (last_tile + 1) * kb * 1024);
     const int nk = K / TBK;
     const int kt_begin = blockIdx.z * steps_per_slice, kt_end = min(nk, kt_begin + steps_per_slice);
 
+    const bf16_t* Xb = X + m0 * K;
+    const bf16_t* Wb = W + (n0 / 16) * (long long)kb * 512;
     auto issue = [&](int buf, int kt) {
 #pragma unroll
-        for (int i = 0; i < IA; ++i) load_to_lds(xbuf, As + buf * BM * TBK + (wave + NW * i) * 512, offa[i], kt * (TBK * 2));
+        for (int i = 0; i < IA; ++i) {
+            bf16_t* to = As + buf * BM * TBK + (wave + NW * i) * 512;
+            if constexpr (BUFFER) load_to_lds(xbuf, to, (int)offa[i], kt * (TBK * 2));
+            else load_to_lds(Xb + kt * TBK + offa[i], to);
+        }
 #pragma unroll
-        for (int i = 0; i < IB; ++i) load_to_lds(wbuf, Bs + buf * BN * TBK + (wave + NW * i) * 512, offb[i], kt * 2048);
+        for (int i = 0; i < IB; ++i) {
+            bf16_t* to = Bs + buf * BN * TBK + (wave + NW * i) * 512;
+            if constexpr (BUFFER) load_to_lds(wbuf, to, (int)offb[i], kt * 2048);
+            else load_to_lds(Wb + (unsigned)(kt * 2) * 512u + offb[i], to);
+        }
     };
     const int fa0 = swz(wm + r16, g), fa1 = swz(wm + r16, 4 + g);
     const int fb = (wn / 16) * 1024 + lane * 8;                        // block h of MFMA tile j: + (2 j + h) * 512
@@ -1401,6 +1422,17 @@ TiledPlan plan_tiled(int M, int N, int K) {
     return t;
 }
 
+// Which loads the kernel straight into LDS takes (see there).  Measured through buffers and globally, us: blocks of 64 x 64, up to
+// one a CU 9.7 and 10.0 (300 rows, 2,560 x 2,560), 8.7 and 9.0 (500, 2,048 x 2,048), more 13.6 and 12.8 (400, 2,560 x 2,560), 12.3
+// and 11.8 (512, 2,560 x 2,048); 128 x 128, one a CU, K = 2,048 16.1 and 17.6 (1,024 rows, 2,048 columns), K = 5,632 48.2 and 47.2, K =
+// 6,912 58.4 and 56.2; 256 x 192 45.0 and 43.7 (1,500, 6,144 x 2,048), 35.7 and 34.0 (2,048, 4,608 x 1,536); 256 x 256 111.7 and 114.2 (2,048,
+// 16,384 x 2,048); 128 x 128, two a CU, within 1 %.
+bool dma_through_buffer(const TiledPlan& t, int M, int N) {
+    if (t.shape == 4) return false;
+    if (t.shape == 3) return (long long)ceil_div(M, 64) * ceil_div(N, 64) <= 256;
+    return t.shape != 2 || t.steps_per_slice <= 64;
+}
+
 struct Skinny16Extra {
     const float* norm_w = nullptr; float eps = 0.f; const int* rows = nullptr; long long ldx = 0;       // NORM_INSIDE (ldx: rows of X that far apart)
     const float* ss_in = nullptr; int n_ss = 0;                                      // NORM_SCALED (+ eps)
@@ -1563,8 +1595,8 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
             hipLaunchKernelGGL(kern, dim3(ceil_div(N, bn), ceil_div(M, bm), t.slices), dim3(64 * WM * WN), lds, stream, \
                                X, W, Y, M, N, K, t.steps_per_slice, ws); \
         } while (0)
-#define TILED_DMA(TM, TN, WM, WN, STAGES) do { \
-            auto kern = gemm_bf16_dma_kernel<TM, TN, WM, WN, STAGES, MODE, AROUND>; \
+#define TILED_DMA(TM, TN, WM, WN, STAGES, BUFFER) do { \
+            auto kern = gemm_bf16_dma_kernel<TM, TN, WM, WN, STAGES, BUFFER, MODE, AROUND>; \
             constexpr int bm = 16 * TM * WM, bn = 16 * TN * WN, lds = STAGES * (bm + bn) * TBK * 2; \
             static bool set = false; \
             if (!set) { \
@@ -1578,11 +1610,13 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
             if (!dma_ok(K) && t.slices == 1) return -2;            // a product in slices is finished by the kernel that adds them
         }
         if (dma_ok(K)) {
-            if (t.shape == 3) TILED_DMA(2, 2, 2, 2, 4);
-            else if (t.shape == 4) TILED_DMA(8, 3, 2, 4, 2);
-            else if (t.shape == 0) TILED_DMA(8, 4, 2, 4, 2);
-            else if (t.shape == 1) TILED_DMA(4, 2, 2, 4, 2);
-            else TILED_DMA(4, 2, 2, 4, 4);
+            const bool buffer = dma_through_buffer(t, M, N);
+            if (t.shape == 3) { if (buffer) TILED_DMA(2, 2, 2, 2, 4, true); else TILED_DMA(2, 2, 2, 2, 4, false); }
+            else if (t.shape == 4) TILED_DMA(8, 3, 2, 4, 2, false);
+            else if (t.shape == 0) TILED_DMA(8, 4, 2, 4, 2, true);
+            else if (t.shape == 1) TILED_DMA(4, 2, 2, 4, 2, true);
+            else if (buffer) TILED_DMA(4, 2, 2, 4, 4, true);
+            else TILED_DMA(4, 2, 2, 4, 4, false);
         }
         else if (t.shape == 0) TILED(8, 4, 2, 4, 1);
         else if (t.shape == 1) TILED(4, 2, 2, 4, 1);
