@@ -450,6 +450,39 @@ def test_scan_gives_the_same_bits_for_any_company_and_alignment(gpu, D):
                 assert torch.equal(state[i], state0[i])
 
 
+@pytest.mark.parametrize("D, Dv", [(16, 16), (30, 50), (32, 64), (64, 128), (96, 20), (130, 130), (256, 24)])
+def test_single_tokens_of_a_scan_have_the_bits_of_a_run(gpu, D, Dv):
+    """A request with one token takes no stop in LDS; portions that end inside the tokens staged at a time stage only their own:
+    thirteen tokens in any cut, the same outputs and state."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(D)
+    H, n = 2, 13
+    rnd = lambda *shape: torch.randn(*shape, generator=gen).to(gpu)
+    i32 = lambda x: torch.tensor([x], dtype=torch.int32, device=gpu)
+    state0, hd, h = rnd(1, H, D, Dv), rnd(H * D), [rnd(H) for _ in range(3)]
+    for dt in (torch.bfloat16, torch.float32):
+        x, q, k, v, xbc = (rnd(n, w).to(dt) for w in (2 * H * D + H * Dv, H * D, H * D, H * Dv, H * Dv + 2 * D))
+        a, b = rnd(n, H * D), rnd(n, H)
+        lower = torch.rand(H * D, generator=gen).to(gpu)
+        kinds = {
+            "forget": lambda t, st, o, kw: ops.forget_scan(x[t], hd, lower, st, o, H=H, D=D, Dv=Dv, **kw),
+            "delta": lambda t, st, o, kw: ops.delta_scan(q[t], k[t], v[t], a[t].clone(), hd, h[0], b[t], st, o, H=H, Hk=H, D=D, Dv=Dv, **kw),
+            "state space": lambda t, st, o, kw: ops.ssd_scan(xbc[t], b[t], *h, st, o, H=H, G=1, N=D, P=Dv, **kw)}
+        if D == Dv:
+            kinds["wkv"] = lambda t, st, o, kw: ops.wkv_scan(q[t], k[t], v[t], a[t].clone(), hd, hd.view(H, D), st, o, H=H, D=D, **kw)
+        for name, scan in kinds.items():
+            results = []
+            for cuts in ([n], [1] * n, [1, 2, 3, 7], [4, 1, 8], [5, 6, 1, 1]):
+                state, out, at = state0.clone(), torch.full((n, H * Dv), float("nan"), device=gpu), 0
+                for c in cuts:
+                    scan(slice(at, at + c), state, out[at:at + c], dict(q_start=i32(0), q_len=i32(c), state_slot=i32(0)))
+                    at += c
+                results.append((out, state))
+            assert torch.isfinite(results[0][0]).all(), name
+            for out, state in results[1:]:
+                assert torch.equal(out, results[0][0]) and torch.equal(state, results[0][1]), (name, dt)
+
+
 # ------------------------------------------------------------------- generation, command line
 def test_greedy_generation_through_the_scheduler(gpu):
     from tuff_amd.engine.llm import LLM

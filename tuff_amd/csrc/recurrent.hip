@@ -501,11 +501,11 @@ __device__ __forceinline__ float group_sum(float v) {
 // gate), 2,366 -> 1,053 us (delta rule); without it 1,365 and 2,580.  Four waves a SIMD up to 64 key channels, three up to
 // 128 (with four the registers spill: 64 single tokens, 16 heads of 128, 92 us instead of 80), two beyond.
 template <typename TA, typename T, int NI16, int SPLIT, bool WHOLE, bool DELTA, bool FORGET = false, bool SSD = false>
-__global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_kernel(ScanArgs p) {
+__global__ __launch_bounds__(WAVE, 5 - NI16) void scan_kernel(ScanArgs p) {
     constexpr int RP = NI16 * 4;                       // rows of the state's column a lane keeps
     constexpr int DP = RP * SPLIT;                     // key channels, padded
     constexpr int SCAN_COLS = WAVE / SPLIT;            // value channels a wave
-    constexpr int CH = SCAN_CH;
+    constexpr int CH = NI16 == 4 ? SCAN_CH / 2 : SCAN_CH;
     constexpr int QUADS = DP / 4;                      // groups of four key channels a token
     constexpr int PER = (CH * QUADS + WAVE - 1) / WAVE;                  // such groups a lane stages
     constexpr int PER_V = (CH * SCAN_COLS + WAVE - 1) / WAVE;            // and values
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
         r = pair % gridDim.x;
         head = pair / gridDim.x;
     }
-    const int n = p.q_len[r];
+    const int n = p.q_len[r], t0 = p.q_start[r], slot = p.state_slot[r];        // (asked for together)
     if (n <= 0) return;
     const int D = p.D, Dv = p.Dv, H = p.H, Ha = p.Ha;
     const int ha = head / (H / Ha);
@@ -535,8 +535,7 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
     const int j = zb * SCAN_COLS + lane / SPLIT;
     const bool jv = j < Dv;
     const int row0 = part * RP;
-    const int t0 = p.q_start[r];
-    float* S = p.state + (((long long)p.state_slot[r] * H + head) * D) * Dv + j;
+    float* S = p.state + (((long long)slot * H + head) * D) * Dv + j;
     const TA* pa = (const TA*)p.a;
     const TA* pk = (const TA*)p.k;
     const T* pv = (const T*)p.v;
@@ -555,53 +554,63 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
     T fv[PER_V];
     float fb = 0.f, fd = 0.f;
     const float bonus_h = SSD ? p.head_bonus[head] : 0.f;
+    // Key channels i .. i + 3 of token t + dt.  Addresses are a row that is the same for the whole wave and 32 bits a lane: eight
+    // rows lie less than 2^31 elements apart.
+    const unsigned strideA = (unsigned)p.lda, strideW = (unsigned)(H * D), strideV = (unsigned)p.ldv;
+    auto fetch_four = [&](long long t, unsigned dt, int i, four& a, four& k, f32x4& w) {
+        const TA *ra = pa + t * p.lda + (long long)ha * D, *rk = pk + t * p.lda + (long long)ha * D;
+        const float* rw = SSD ? nullptr : p.decay + (t * H + head) * D;
+        if (WHOLE) {
+            const unsigned ic = min(i, D - 4);
+            a = *(const four*)(ra + (dt * strideA + ic));
+            if (!FORGET) k = *(const four*)(rk + (dt * strideA + ic));
+            if (!SSD) w = *(const f32x4*)(rw + (dt * strideW + ic));
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const unsigned ic = min(i + u, D - 1);
+                a[u] = ra[dt * strideA + ic];
+                if (!FORGET) k[u] = rk[dt * strideA + ic];
+                if (!SSD) w[u] = rw[dt * strideW + ic];
+            }
+        }
+    };
+    // The same in float32, channels beyond D as zero; step: the token's step size (ssd).
+    auto in_float = [&](int i, const four& fa, const four& fk, const f32x4& fw, float step, f32x4& a, f32x4& k, f32x4& w) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const bool ok = i + u < D;
+            a[u] = ok ? to_f32((TA)fa[u]) : 0.f;
+            k[u] = ok ? (FORGET ? 1.0f - fw[u] : SSD ? step * to_f32((TA)fk[u]) : to_f32((TA)fk[u])) : 0.f;
+            w[u] = ok && !SSD ? fw[u] : 0.f;
+        }
+    };
     auto fetch = [&](int c0) {                         // c0: the first token, counted from the request's first of the step
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
             const int id = lane + e * WAVE;
-            const long long t = t0 + min(c0 + id / QUADS, n - 1);
-            const int i = id % QUADS * 4;
-            const TA *ra = pa + t * p.lda + (long long)ha * D, *rk = pk + t * p.lda + (long long)ha * D;
-            const float* rw = SSD ? nullptr : p.decay + (t * H + head) * D;
-            if (WHOLE) {
-                const int ic = min(i, D - 4);
-                fa[e] = *(const four*)(ra + ic);
-                if (!FORGET) fk[e] = *(const four*)(rk + ic);
-                if (!SSD) fw[e] = *(const f32x4*)(rw + ic);
-            } else {
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int ic = min(i + u, D - 1);
-                    fa[e][u] = ra[ic];
-                    if (!FORGET) fk[e][u] = rk[ic];
-                    if (!SSD) fw[e][u] = rw[ic];
-                }
-            }
+            fetch_four(t0 + c0, min(id / QUADS, n - 1 - c0), id % QUADS * 4, fa[e], fk[e], fw[e]);
         }
 #pragma unroll
         for (int e = 0; e < PER_V; ++e) {
             const int id = lane + e * WAVE;
-            const long long t = t0 + min(c0 + id / SCAN_COLS, n - 1);
-            fv[e] = pv[t * p.ldv + (long long)head * Dv + min(zb * SCAN_COLS + id % SCAN_COLS, Dv - 1)];
+            const unsigned dt = min(id / SCAN_COLS, n - 1 - c0);
+            fv[e] = (pv + (long long)(t0 + c0) * p.ldv + (long long)head * Dv)[dt * strideV + (unsigned)min(zb * SCAN_COLS + id % SCAN_COLS, Dv - 1)];
         }
-        const long long t = t0 + min(c0 + lane % CH, n - 1);
-        if (!FORGET) fb = p.scalar[t * H + head];
-        if (SSD) fd = p.decay[t * H + head];
+        const unsigned at = (unsigned)min(lane % CH, n - 1 - c0) * (unsigned)H;
+        const long long first = (long long)(t0 + c0) * H + head;
+        if (!FORGET) fb = (p.scalar + first)[at];
+        if (SSD) fd = (p.decay + first)[at];
     };
     // The fetched values to LDS in float32, key channels beyond D as zero (tokens beyond the last are staged and never read).
-    auto stage = [&]() {
+    auto stage = [&](auto whole, int count) {
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
+            if (!decltype(whole)::value && e * WAVE / QUADS >= count) break;     // (of the last, partial eight: the tokens that are there)
             const int id = lane + e * WAVE, tt = id / QUADS, i = id % QUADS * 4;
             const float step = SSD ? __shfl(fb, tt, WAVE) : 1.f;
             f32x4 a, k, w;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const bool ok = i + u < D;
-                a[u] = ok ? to_f32((TA)fa[e][u]) : 0.f;
-                k[u] = ok ? (FORGET ? 1.0f - fw[e][u] : SSD ? step * to_f32((TA)fk[e][u]) : to_f32((TA)fk[e][u])) : 0.f;
-                w[u] = ok && !SSD ? fw[e][u] : 0.f;
-            }
+            in_float(i, fa[e], fk[e], fw[e], step, a, k, w);
             if (CH * QUADS % WAVE == 0 || id < CH * QUADS) {
                 *(f32x4*)&sa[tt][i] = a;
                 *(f32x4*)&sk[tt][i] = k;
@@ -676,13 +685,37 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
     float* const out_row = p.out + ((long long)t0 * H + head) * Dv;
     auto leave = [&](int t, float o) { (out_row + (long long)t * H * Dv)[(unsigned)j] = o; };
 
+    auto keep = [&]() {
+#pragma unroll
+        for (int i = 0; i < RP; ++i)
+            if (jv && row0 + i < D) S[(long long)(row0 + i) * Dv] = s[i];
+    };
+
+    // A single token: its rows straight from memory, in one trip with the state's, and no stop in LDS, whose eight places and
+    // eight tokens' code cost it 1 us and more.
+    if (n == 1) {
+        Rows m;
+        four a[NI16], k[NI16];
+        f32x4 w[NI16];
+#pragma unroll
+        for (int g4 = 0; g4 < NI16; ++g4) fetch_four(t0, 0, row0 + g4 * 4, a[g4], k[g4], w[g4]);
+        const float vt = to_f32(pv[(long long)t0 * p.ldv + (long long)head * Dv + min(j, Dv - 1)]);
+        const float sc = FORGET ? 0.f : p.scalar[(long long)t0 * H + head], wt = SSD ? p.decay[(long long)t0 * H + head] : 0.f;
+#pragma unroll
+        for (int g4 = 0; g4 < NI16; ++g4) in_float(row0 + g4 * 4, a[g4], k[g4], w[g4], sc, m.q[g4], m.k[g4], m.w[g4]);
+        const float ot = own(group_sum<SPLIT>(token(m, vt, sc, wt)), vt, sc);
+        if (jv) leave(0, ot);
+        keep();
+        return;
+    }
+
     // The outputs of CH tokens stay in registers until the next ones have been staged: staging waits for every access to
     // memory under way, and stores from just before would be waited for too, all the way to memory.
     float o[CH] = {};
     fetch(0);
     for (int c0 = 0; c0 < n; c0 += CH) {
         const int count = min(CH, n - c0);
-        stage();
+        if (count == CH) stage(std::true_type(), CH); else stage(std::false_type(), count);
         float v[CH], sc[CH], wd[CH];
 #pragma unroll
         for (int tt = 0; tt < CH; ++tt) {
@@ -732,9 +765,7 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
 #pragma unroll
         for (int tt = 0; tt < CH; ++tt) leave(n - CH + tt, o[tt]);
     }
-#pragma unroll
-    for (int i = 0; i < RP; ++i)
-        if (jv && row0 + i < D) S[(long long)(row0 + i) * Dv] = s[i];
+    keep();
 }
 
 // ---------------------------------------------------------- per-head unit norm, weight and gate
