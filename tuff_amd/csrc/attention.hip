@@ -168,7 +168,7 @@ TUFF_EXPORT int tuff_attention_general(const void* q, const void* k_cache, const
 //   softmax  a wave four of the columns, lanes are keys: maximum, exponentials and the sum's butterfly as above;
 //   values   wave w the channels 16 w .. + 15 (and + 64): scaled by the column's correction, then a chain over the keys.
 // Keys and values go through LDS, the next tile's on their way to registers meanwhile.  What bounds it: a tile is two chains of
-// sixteen dependent matrix instructions and three exchanges, about 1.5 us, whatever the number of columns.  The general
+// sixteen dependent matrix instructions and three exchanges, about 2.9 us, whatever the number of columns.  The general
 // kernel reads a key's row a lane and a value's column a lane, one wave a (token, head): 4 tokens of 32 heads at 1,000 keys
 // 272 us -> 46, a prompt of 500 tokens 613 us -> 76.
 namespace {

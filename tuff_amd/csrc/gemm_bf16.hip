@@ -61,19 +61,6 @@ __device__ __forceinline__ void store_elem(void* Y, long long row, long long col
     }
 }
 
-// 16-byte load of eight bf16 with a guard; out-of-range pieces read as zero.
-__device__ __forceinline__ bf16x8 load8(const bf16_t* base, long long row, int nrows, int k, int K) {
-    bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (row < nrows && k < K) return *(const bf16x8*)(base + row * (long long)K + k);
-    return z;
-}
-
-// Piece `piece` (0..63) of block (tile, kblock) of a tile-major W with kb blocks a row tile.
-// Weights of a skinny product are read once and never again: a streaming (non-temporal) load.
-__device__ __forceinline__ bf16x8 load_w(const bf16_t* W, long long tile, int kb, int kblock, int piece) {
-    return __builtin_nontemporal_load((const bf16x8*)(W + ((tile * kb + kblock) * 64 + piece) * 8));
-}
-
 // ------------------------------------------------------------------ tiled kernel
 // A workgroup of WAVES_M x WAVES_N waves computes a block of Y; each wave a (16 TM) x (16 TN) part
 // of it as TM x TN MFMA tiles.  K is walked in steps of 64 through two LDS buffers: while a step
