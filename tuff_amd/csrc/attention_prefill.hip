@@ -69,11 +69,15 @@ struct WideArgs {
 
 // Two maps over rows of up to 128 channels: two workgroups a CU (256 registers a wave) with one step's copies under way are
 // faster than one with two (2,048 tokens, 16 heads of two maps of 64 over values of 128, a window of 1,024: 117 -> 67 us).
-constexpr int groups_a_cu(int hdp, int vdp, int maps) { return maps == 2 && hdp <= 128 && vdp <= 128 ? 2 : 1; }
+// The wide form with heads of up to 64 channels: left alone it takes 259 registers, three too many for two workgroups a CU (every
+// head's weights on every kv head's values, 2,048 tokens, 32 heads, 8 kv heads of 64: 870 us, with two 555).
+constexpr int groups_a_cu(int hdp, int vdp, int maps, bool ex) {
+    return (maps == 2 && hdp <= 128 && vdp <= 128) || (maps == 1 && ex && hdp <= 64 && vdp <= 64) ? 2 : 1;
+}
 
 // HDP, VDP: the channels of a key row and of a value in the tiles, multiples of 32 (a map's share of a key row too).
 template <int HDP, int NBW, int AHEAD, bool EX, int VDP, int MAPS>
-__global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS)) void attn_prefill_kernel(
+__global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     bf16_t* __restrict__ out, const int* __restrict__ block_table, int max_blocks,
     const int2* __restrict__ blk, const int4* __restrict__ req_info,
