@@ -500,12 +500,13 @@ __device__ __forceinline__ float group_sum(float v) {
 // blocks of a head all read: by XCD as below, 64 requests of 200 tokens, 16 heads of 128 x 128, 1,281 -> 856 us (forget
 // gate), 2,366 -> 1,053 us (delta rule); without it 1,365 and 2,580.  Four waves a SIMD up to 64 key channels, three up to
 // 128 (with four the registers spill: 64 single tokens, 16 heads of 128, 92 us instead of 80), two beyond.
-template <typename TA, typename T, int NI16, int SPLIT, bool WHOLE, bool DELTA, bool FORGET = false, bool SSD = false>
-__global__ __launch_bounds__(WAVE, 5 - NI16) void scan_kernel(ScanArgs p) {
+// SINGLES: a step in which no request need have more than one token.
+template <typename TA, typename T, int NI16, int SPLIT, bool WHOLE, bool SINGLES, bool DELTA, bool FORGET = false, bool SSD = false>
+__global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_kernel(ScanArgs p) {
     constexpr int RP = NI16 * 4;                       // rows of the state's column a lane keeps
     constexpr int DP = RP * SPLIT;                     // key channels, padded
     constexpr int SCAN_COLS = WAVE / SPLIT;            // value channels a wave
-    constexpr int CH = NI16 == 4 ? SCAN_CH / 2 : SCAN_CH;
+    constexpr int CH = SCAN_CH;
     constexpr int QUADS = DP / 4;                      // groups of four key channels a token
     constexpr int PER = (CH * QUADS + WAVE - 1) / WAVE;                  // such groups a lane stages
     constexpr int PER_V = (CH * SCAN_COLS + WAVE - 1) / WAVE;            // and values
@@ -554,63 +555,53 @@ __global__ __launch_bounds__(WAVE, 5 - NI16) void scan_kernel(ScanArgs p) {
     T fv[PER_V];
     float fb = 0.f, fd = 0.f;
     const float bonus_h = SSD ? p.head_bonus[head] : 0.f;
-    // Key channels i .. i + 3 of token t + dt.  Addresses are a row that is the same for the whole wave and 32 bits a lane: eight
-    // rows lie less than 2^31 elements apart.
-    const unsigned strideA = (unsigned)p.lda, strideW = (unsigned)(H * D), strideV = (unsigned)p.ldv;
-    auto fetch_four = [&](long long t, unsigned dt, int i, four& a, four& k, f32x4& w) {
-        const TA *ra = pa + t * p.lda + (long long)ha * D, *rk = pk + t * p.lda + (long long)ha * D;
-        const float* rw = SSD ? nullptr : p.decay + (t * H + head) * D;
-        if (WHOLE) {
-            const unsigned ic = min(i, D - 4);
-            a = *(const four*)(ra + (dt * strideA + ic));
-            if (!FORGET) k = *(const four*)(rk + (dt * strideA + ic));
-            if (!SSD) w = *(const f32x4*)(rw + (dt * strideW + ic));
-        } else {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const unsigned ic = min(i + u, D - 1);
-                a[u] = ra[dt * strideA + ic];
-                if (!FORGET) k[u] = rk[dt * strideA + ic];
-                if (!SSD) w[u] = rw[dt * strideW + ic];
-            }
-        }
-    };
-    // The same in float32, channels beyond D as zero; step: the token's step size (ssd).
-    auto in_float = [&](int i, const four& fa, const four& fk, const f32x4& fw, float step, f32x4& a, f32x4& k, f32x4& w) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const bool ok = i + u < D;
-            a[u] = ok ? to_f32((TA)fa[u]) : 0.f;
-            k[u] = ok ? (FORGET ? 1.0f - fw[u] : SSD ? step * to_f32((TA)fk[u]) : to_f32((TA)fk[u])) : 0.f;
-            w[u] = ok && !SSD ? fw[u] : 0.f;
-        }
-    };
     auto fetch = [&](int c0) {                         // c0: the first token, counted from the request's first of the step
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
             const int id = lane + e * WAVE;
-            fetch_four(t0 + c0, min(id / QUADS, n - 1 - c0), id % QUADS * 4, fa[e], fk[e], fw[e]);
+            const long long t = t0 + min(c0 + id / QUADS, n - 1);
+            const int i = id % QUADS * 4;
+            const TA *ra = pa + t * p.lda + (long long)ha * D, *rk = pk + t * p.lda + (long long)ha * D;
+            const float* rw = SSD ? nullptr : p.decay + (t * H + head) * D;
+            if (WHOLE) {
+                const int ic = min(i, D - 4);
+                fa[e] = *(const four*)(ra + ic);
+                if (!FORGET) fk[e] = *(const four*)(rk + ic);
+                if (!SSD) fw[e] = *(const f32x4*)(rw + ic);
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int ic = min(i + u, D - 1);
+                    fa[e][u] = ra[ic];
+                    if (!FORGET) fk[e][u] = rk[ic];
+                    if (!SSD) fw[e][u] = rw[ic];
+                }
+            }
         }
 #pragma unroll
         for (int e = 0; e < PER_V; ++e) {
             const int id = lane + e * WAVE;
-            const unsigned dt = min(id / SCAN_COLS, n - 1 - c0);
-            fv[e] = (pv + (long long)(t0 + c0) * p.ldv + (long long)head * Dv)[dt * strideV + (unsigned)min(zb * SCAN_COLS + id % SCAN_COLS, Dv - 1)];
+            const long long t = t0 + min(c0 + id / SCAN_COLS, n - 1);
+            fv[e] = pv[t * p.ldv + (long long)head * Dv + min(zb * SCAN_COLS + id % SCAN_COLS, Dv - 1)];
         }
-        const unsigned at = (unsigned)min(lane % CH, n - 1 - c0) * (unsigned)H;
-        const long long first = (long long)(t0 + c0) * H + head;
-        if (!FORGET) fb = (p.scalar + first)[at];
-        if (SSD) fd = (p.decay + first)[at];
+        const long long t = t0 + min(c0 + lane % CH, n - 1);
+        if (!FORGET) fb = p.scalar[t * H + head];
+        if (SSD) fd = p.decay[t * H + head];
     };
     // The fetched values to LDS in float32, key channels beyond D as zero (tokens beyond the last are staged and never read).
-    auto stage = [&](auto whole, int count) {
+    auto stage = [&]() {
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            if (!decltype(whole)::value && e * WAVE / QUADS >= count) break;     // (of the last, partial eight: the tokens that are there)
             const int id = lane + e * WAVE, tt = id / QUADS, i = id % QUADS * 4;
             const float step = SSD ? __shfl(fb, tt, WAVE) : 1.f;
             f32x4 a, k, w;
-            in_float(i, fa[e], fk[e], fw[e], step, a, k, w);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool ok = i + u < D;
+                a[u] = ok ? to_f32((TA)fa[e][u]) : 0.f;
+                k[u] = ok ? (FORGET ? 1.0f - fw[e][u] : SSD ? step * to_f32((TA)fk[e][u]) : to_f32((TA)fk[e][u])) : 0.f;
+                w[u] = ok && !SSD ? fw[e][u] : 0.f;
+            }
             if (CH * QUADS % WAVE == 0 || id < CH * QUADS) {
                 *(f32x4*)&sa[tt][i] = a;
                 *(f32x4*)&sk[tt][i] = k;
@@ -692,19 +683,45 @@ __global__ __launch_bounds__(WAVE, 5 - NI16) void scan_kernel(ScanArgs p) {
     };
 
     // A single token: its rows straight from memory, in one trip with the state's, and no stop in LDS, whose eight places and
-    // eight tokens' code cost it 1 us and more.
-    if (n == 1) {
-        Rows m;
+    // eight tokens' code cost it up to 1 us more (8 heads of 64 x 128, forget gate, one request 5.8 -> 5.3 us, 64 22.2 -> 20.2).
+    // (Not in the kernel for runs of tokens, which takes 3 % longer with this code beside its own.)
+    if (SINGLES && n == 1) {
+        const TA *ra = pa + (long long)t0 * p.lda + (long long)ha * D, *rk = pk + (long long)t0 * p.lda + (long long)ha * D;
+        const float* rw = SSD ? nullptr : p.decay + ((long long)t0 * H + head) * D;
+        const float vt = to_f32(pv[(long long)t0 * p.ldv + (long long)head * Dv + min(j, Dv - 1)]);
+        const float sc = FORGET ? 0.f : p.scalar[(long long)t0 * H + head], wt = SSD ? p.decay[(long long)t0 * H + head] : 0.f;
         four a[NI16], k[NI16];
         f32x4 w[NI16];
 #pragma unroll
-        for (int g4 = 0; g4 < NI16; ++g4) fetch_four(t0, 0, row0 + g4 * 4, a[g4], k[g4], w[g4]);
-        const float vt = to_f32(pv[(long long)t0 * p.ldv + (long long)head * Dv + min(j, Dv - 1)]);
-        const float sc = FORGET ? 0.f : p.scalar[(long long)t0 * H + head], wt = SSD ? p.decay[(long long)t0 * H + head] : 0.f;
+        for (int g4 = 0; g4 < NI16; ++g4) {
+            const int i = row0 + g4 * 4;
+            if (WHOLE) {
+                const int at = min(i, D - 4);
+                a[g4] = *(const four*)(ra + at);
+                if (!FORGET) k[g4] = *(const four*)(rk + at);
+                if (!SSD) w[g4] = *(const f32x4*)(rw + at);
+            } else {
 #pragma unroll
-        for (int g4 = 0; g4 < NI16; ++g4) in_float(row0 + g4 * 4, a[g4], k[g4], w[g4], sc, m.q[g4], m.k[g4], m.w[g4]);
-        const float ot = own(group_sum<SPLIT>(token(m, vt, sc, wt)), vt, sc);
-        if (jv) leave(0, ot);
+                for (int u = 0; u < 4; ++u) {
+                    const int at = min(i + u, D - 1);
+                    a[g4][u] = ra[at];
+                    if (!FORGET) k[g4][u] = rk[at];
+                    if (!SSD) w[g4][u] = rw[at];
+                }
+            }
+        }
+        Rows m;
+#pragma unroll
+        for (int g4 = 0; g4 < NI16; ++g4)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const bool ok = row0 + g4 * 4 + u < D;
+                m.q[g4][u] = ok ? to_f32((TA)a[g4][u]) : 0.f;
+                m.k[g4][u] = ok ? (FORGET ? 1.0f - w[g4][u] : SSD ? sc * to_f32((TA)k[g4][u]) : to_f32((TA)k[g4][u])) : 0.f;
+                m.w[g4][u] = ok && !SSD ? w[g4][u] : 0.f;
+            }
+        const float o1 = own(group_sum<SPLIT>(token(m, vt, sc, wt)), vt, sc);
+        if (jv) leave(0, o1);
         keep();
         return;
     }
@@ -715,7 +732,7 @@ __global__ __launch_bounds__(WAVE, 5 - NI16) void scan_kernel(ScanArgs p) {
     fetch(0);
     for (int c0 = 0; c0 < n; c0 += CH) {
         const int count = min(CH, n - c0);
-        if (count == CH) stage(std::true_type(), CH); else stage(std::false_type(), count);
+        stage();
         float v[CH], sc[CH], wd[CH];
 #pragma unroll
         for (int tt = 0; tt < CH; ++tt) {
@@ -801,7 +818,7 @@ __global__ __launch_bounds__(WAVE) void head_norm_gate_kernel(const float* __res
 }
 
 template <typename TA, typename T, bool DELTA, bool FORGET = false, bool SSD = false>
-int launch_scan(ScanArgs p, int R, hipStream_t stream) {
+int launch_scan(ScanArgs p, int n_tokens, int R, hipStream_t stream) {
     if (p.H > 65535 || p.D > 256) return -2;
     const bool narrow = p.D <= 32;                      // four lanes a value channel; else sixteen
     const int split = narrow ? 4 : 16;
@@ -813,14 +830,17 @@ int launch_scan(ScanArgs p, int R, hipStream_t stream) {
     auto in_fours = [](const void* q, size_t width) { return (uintptr_t)q % (4 * width) == 0; };
     const bool whole = p.D % 4 == 0 && p.lda % 4 == 0 && in_fours(p.a, sizeof(TA)) && (FORGET || in_fours(p.k, sizeof(TA))) &&
                        (SSD || in_fours(p.decay, 4));
-#define SCAN(NI, SPLIT) do { if (whole) hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, true, DELTA, FORGET, SSD>), grid, block, 0, stream, p); \
-                             else hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, false, DELTA, FORGET, SSD>), grid, block, 0, stream, p); } while (0)
+    const bool singles = n_tokens <= R;
+#define GO(NI, SPLIT, WHOLE, SINGLES) hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, WHOLE, SINGLES, DELTA, FORGET, SSD>), grid, block, 0, stream, p)
+#define SCAN(NI, SPLIT) do { if (whole && singles) GO(NI, SPLIT, true, true); else if (whole) GO(NI, SPLIT, true, false); \
+                             else if (singles) GO(NI, SPLIT, false, true); else GO(NI, SPLIT, false, false); } while (0)
     if (narrow) { if (ni <= 1) SCAN(1, 4); else SCAN(2, 4); }
     else if (ni <= 1) SCAN(1, 16);
     else if (ni <= 2) SCAN(2, 16);
     else if (ni <= 3) SCAN(3, 16);
     else SCAN(4, 16);
 #undef SCAN
+#undef GO
     return launch_status();
 }
 }  // namespace
@@ -878,8 +898,8 @@ TUFF_EXPORT int tuff_wkv_scan(const void* r, const void* k, const void* v, int d
     if (dt == DT_F32) hipLaunchKernelGGL((scan_prep_kernel<float, false>), dim3(n_tokens, H), dim3(WAVE), 0, stream, pp);
     else hipLaunchKernelGGL((scan_prep_kernel<bf16_t, false>), dim3(n_tokens, H), dim3(WAVE), 0, stream, pp);
     ScanArgs p{r, k, v, lw, bonus, state, out, q_start, q_len, state_slot, H, H, D, D, (long long)H * D, (long long)H * D, nullptr};
-    return dt == DT_F32 ? launch_scan<float, float, false>(p, n_requests, stream)
-                        : launch_scan<bf16_t, bf16_t, false>(p, n_requests, stream);
+    return dt == DT_F32 ? launch_scan<float, float, false>(p, n_tokens, n_requests, stream)
+                        : launch_scan<bf16_t, bf16_t, false>(p, n_tokens, n_requests, stream);
 }
 
 // delta: q, k (rows of Hk*D, ld elements apart) and v (rows of H*Dv, ldv apart) of type dt (they
@@ -899,8 +919,8 @@ TUFF_EXPORT int tuff_delta_scan(const void* q, const void* k, const void* v, int
     if (dt == DT_F32) hipLaunchKernelGGL((scan_prep_kernel<float, true>), dim3(n_tokens, H), dim3(WAVE), 0, stream, pp);
     else hipLaunchKernelGGL((scan_prep_kernel<bf16_t, true>), dim3(n_tokens, H), dim3(WAVE), 0, stream, pp);
     ScanArgs p{qn, kn, v, a, beta, state, out, q_start, q_len, state_slot, H, H, D, Dv, ldv, (long long)H * D, nullptr};
-    return dt == DT_F32 ? launch_scan<float, float, true>(p, n_requests, stream)
-                        : launch_scan<float, bf16_t, true>(p, n_requests, stream);
+    return dt == DT_F32 ? launch_scan<float, float, true>(p, n_tokens, n_requests, stream)
+                        : launch_scan<float, bf16_t, true>(p, n_tokens, n_requests, stream);
 }
 
 // gate_dt: type of the gate's rows (float32 sums of a product may come in as they are), gate_ld elements apart; dt:
@@ -936,11 +956,11 @@ TUFF_EXPORT int tuff_ssd_scan(const void* xbc, int dt, long long ld, const float
     if (dt == DT_F32) {
         const float* x = (const float*)xbc;
         ScanArgs p{x + c_off, x + b_off, x, decay, step, state, out, q_start, q_len, state_slot, H, G, N, P, ld, ld, Dh};
-        return launch_scan<float, float, false, false, true>(p, n_requests, stream);
+        return launch_scan<float, float, false, false, true>(p, n_tokens, n_requests, stream);
     }
     const bf16_t* x = (const bf16_t*)xbc;
     ScanArgs p{x + c_off, x + b_off, x, decay, step, state, out, q_start, q_len, state_slot, H, G, N, P, ld, ld, Dh};
-    return launch_scan<bf16_t, bf16_t, false, false, true>(p, n_requests, stream);
+    return launch_scan<bf16_t, bf16_t, false, false, true>(p, n_tokens, n_requests, stream);
 }
 
 // The same recurrence in chunks of 64 tokens on the matrix cores (see above), for bfloat16 rows: N and P multiples of 16,
@@ -984,6 +1004,6 @@ TUFF_EXPORT int tuff_forget_scan(const void* x, int dt, long long ld, const floa
     // (k and the per-token scalar are loaded and not used: they point at arrays of the right reach)
     const void* v = dt == DT_F32 ? (const void*)((const float*)x + 2LL * HD) : (const void*)((const bf16_t*)x + 2LL * HD);
     ScanArgs p{qn, qn, v, f, f, state, out, q_start, q_len, state_slot, H, H, D, Dv, ld, (long long)H * D, nullptr};
-    return dt == DT_F32 ? launch_scan<float, float, false, true>(p, n_requests, stream)
-                        : launch_scan<float, bf16_t, false, true>(p, n_requests, stream);
+    return dt == DT_F32 ? launch_scan<float, float, false, true>(p, n_tokens, n_requests, stream)
+                        : launch_scan<float, bf16_t, false, true>(p, n_tokens, n_requests, stream);
 }
