@@ -52,10 +52,10 @@ def gemm_lib():
 @pytest.mark.parametrize("M,N,K,plain,emit", [
     (16, 2048, 8192, False, False),                       # up to 16 rows: one kernel, whatever the sizes
     (17, 2048, 2048, False, True), (20, 1024, 1024, False, False), (20, 2048, 1032, False, True), (17, 256, 64, False, False),
-    (20, 2048, 2056, True, True), (17, 2048, 8192, True, True), (21, 2048, 1024, True, True), (20, 2064, 8192, False, False)])
+    (20, 2048, 2056, True, True), (20, 512, 2048, True, True), (17, 512, 1024, False, False), (17, 2048, 8192, True, True), (21, 2048, 1024, True, True), (20, 2064, 8192, False, False)])
 def test_narrow_products_of_few_rows_take_slices_only_where_they_are_faster(gemm_lib, M, N, K, plain, emit):
     """Work space means partial tiles and a second kernel.  Outputs of up to 2,048 columns and 17 to 20 rows go without up to
-    K = 2,048, those that leave the next norm its sums up to K = 1,024."""
+    K = 2,048 (of less than 1,024 columns K = 1,024), those that leave the next norm its sums up to K = 1,024."""
     def floats(e):
         out = ctypes.c_longlong(-1)
         assert gemm_lib.tuff_gemm_bf16_workspace(M, N, K, e, ctypes.byref(out)) == 0

@@ -313,7 +313,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     // instruction q of X (q = wave + NW i) fills rows 8 q .. 8 q + 7; instruction q of W fills block q % 2 of row tile q / 2;
     // offsets from the block's first row (tile), in bytes (global loads: in elements).  Rows and tiles beyond the matrix have results
     // that are never stored.  Through buffers they are not fetched: if they read the last one instead, all blocks ask for the same
-    // line again and again, and 160 rows took longer than 256 (2,048 x 5,632: 20.1 us against 18.1, now 15.9).
+    // line again and again, and 160 rows took longer than 256 (2,048 x 5,632: 20.1 us against 18.1, now 15.5).
     unsigned offa[IA], offb[IB];
 #pragma unroll
     for (int i = 0; i < IA; ++i) {
@@ -1319,13 +1319,14 @@ bool rows64_tiled(int M, int N, int K) { return M >= wide64_min_m && M <= 64 && 
 // loses from K = 1,024 on (2,048 x 2,048 7.5 and 7.3).  One that leaves the next norm its sums leaves a group a workgroup,
 // up to 256 instead of 32, which the product after it adds up: only up to K = 1,024 (1,024 x 1,024 and a product of 3,072
 // columns behind it 9.4 and 11.1, 2,048 x 2,048 14.1 and 13.9).
+// Less than 1,024 columns are too few workgroups for K = 2,048 (512 columns 5.5 and 5.2).
 constexpr int NARROW_SHORT_K = 2048, NARROW_SHORT_K_EMIT = 1024;
 bool few_rows_kernel(int M, int N, int K, bool conv = false, bool emit = false) {
     if (M <= 16) return true;
     if (M > SKINNY_ROWS) return false;
     if (conv) return true;
     if (rows64_tiled(M, N, K)) return false;
-    return N <= 2048 ? M <= 20 && K <= (emit ? NARROW_SHORT_K_EMIT : NARROW_SHORT_K) : N <= 8192 ? true : M <= 24;
+    return N <= 2048 ? M <= 20 && K <= (emit || N < 1024 ? NARROW_SHORT_K_EMIT : NARROW_SHORT_K) : N <= 8192 ? true : M <= 24;
 }
 
 // How a skinny product is cut.  Depends on N and K (and on which of the two kernels M selects).
@@ -1411,12 +1412,15 @@ TiledPlan plan_tiled(int M, int N, int K) {
 
 // Which loads the kernel straight into LDS takes (see there).  Measured through buffers and globally, us: blocks of 64 x 64, up to
 // one a CU 9.7 and 10.0 (300 rows, 2,560 x 2,560), 8.7 and 9.0 (500, 2,048 x 2,048), more 13.6 and 12.8 (400, 2,560 x 2,560), 12.3
-// and 11.8 (512, 2,560 x 2,048); 128 x 128, one a CU, K = 2,048 16.1 and 17.6 (1,024 rows, 2,048 columns), K = 5,632 48.2 and 47.2, K =
+// and 11.8 (512, 2,560 x 2,048), but two on every CU 16.7 and 17.2 (512, 4,096 x 2,048); 128 x 128, one a CU, K = 2,048 16.1 and 17.6 (1,024 rows, 2,048 columns), K = 5,632 48.2 and 47.2, K =
 // 6,912 58.4 and 56.2; 256 x 192 45.0 and 43.7 (1,500, 6,144 x 2,048), 35.7 and 34.0 (2,048, 4,608 x 1,536); 256 x 256 111.7 and 114.2 (2,048,
 // 16,384 x 2,048); 128 x 128, two a CU, within 1 %.
 bool dma_through_buffer(const TiledPlan& t, int M, int N) {
     if (t.shape == 4) return false;
-    if (t.shape == 3) return (long long)ceil_div(M, 64) * ceil_div(N, 64) <= 256;
+    if (t.shape == 3) {
+        const long long blocks = (long long)ceil_div(M, 64) * ceil_div(N, 64);
+        return blocks <= 256 || blocks > 448;
+    }
     return t.shape != 2 || t.steps_per_slice <= 64;
 }
 
