@@ -314,6 +314,26 @@ def test_prompt_kernel_in_its_wide_form_against_the_general_kernel(gpu, H, Hkv, 
         assert (got - want).abs().max() <= tol * max(1.0, float(want.abs().max())), opts
 
 
+@pytest.mark.parametrize("ps", [16, 48])
+@pytest.mark.parametrize("H, Hkv, hd, vd", [(8, 8, 64, 64), (10, 5, 64, 24), (9, 9, 16, 32), (12, 3, 40, 64), (4, 4, 32, 32), (6, 6, 8, 8)])
+def test_prompt_kernel_with_the_values_of_several_kv_heads_a_workgroup(gpu, H, Hkv, hd, vd, ps):
+    """Heads of up to 64 channels and more than two kv heads: numbers of kv heads that fill a workgroup's four and that do not, every
+    kind of penalty, page sizes that are and are not a power of two; to float32's rounding, as above."""
+    from tuff_amd.csrc import ops
+    reqs = [(0, 70), (1090, 5), (300, 1), (17, 200)]
+    for opts in [(0, 0, 0, 0, 1, 0), (0, 0, 1, 0, 1, 0), (0, 1, 0, 1, 1, 0), (0, 0, 1, 1, 1, 0), (100, 1, 0, 1, 1, 0)]:
+        c = _paged_case(gpu, H, Hkv, hd, vd, reqs, opts, ps=ps, seed=H + hd)
+        want = _general({**c, "gates": None}, H, Hkv, hd, vd, ps=ps)
+        o = torch.zeros((c["T"], H * Hkv * vd), dtype=torch.float32, device=gpu)
+        blocks = torch.from_numpy(ops.query_blocks(np.array([n for _, n in reqs]), H // Hkv, 8, np.array([a + n for a, n in reqs]))).to(gpu)
+        ops.attention_prefill_wide(c["q"], c["k"], c["v"], o, block_table=c["table"], blocks=blocks, req_info=c["info"], H=H, Hkv=Hkv, hd=hd,
+                                   vd=vd, page_size=ps, max_ctx_len=c["longest"], window=c["window"], scale=0.2, sinks=c["sinks"],
+                                   slopes=c["slopes"], log_distance=c["logd"], all_values=True)
+        got = torch.zeros(c["T"], H * vd, dtype=torch.float32, device=gpu)
+        ops.head_mix_gate(o, got, H=H, Hkv=Hkv, vd=vd, talk=c["talk"], gates=None)
+        assert (got - want).abs().max() <= 3e-5 * max(1.0, float(want.abs().max())), opts
+
+
 @pytest.mark.parametrize("H, Hkv, hd, vd", SHAPES)
 def test_single_token_kernels_with_float32_weights_against_the_general_kernel(gpu, H, Hkv, hd, vd):
     """Single tokens at the first position, on both sides of a part's 256 keys and far behind them."""

@@ -41,10 +41,14 @@
 #include <math.h>
 
 namespace {
+template <int N> using number = std::integral_constant<int, N>;
+
 constexpr int STEP = 64;            // keys a step
-constexpr int NT = 256;             // threads a workgroup
 constexpr float SLACK = 8.f;        // see whole_step
-constexpr int VROW = STEP + 8;      // bf16 a row of V^T in LDS: 64 keys and 16 bytes that keep rows off each other's banks
+// bf16 between rows of the tiles in LDS.  A read of 16 bytes a lane takes eight rows and two pieces of each at a time: rows an odd
+// multiple of 32 bytes apart keep these sixteen pieces on banks of their own (4 cycles a read; 16 bytes of padding: 8).
+constexpr int PAD = 16;
+constexpr int VROW = STEP + PAD;    // bf16 a row of V^T
 
 __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -56,6 +60,22 @@ __device__ __forceinline__ int k_row_of_key(int key) {
     const int sub = key / 32, h = (key / 16) % 2, q = (key / 8) % 2, kb = (key / 4) % 2, m = key % 4;
     return sub * 32 + kb * 16 + h * 8 + q * 4 + m;
 }
+
+// The largest value of the lanes with the same lane % 16, in all of them.  Halves and rows of sixteen lanes change places in
+// registers: through LDS (two shuffles, one after the other, a column block) the wait for them was a fifth of a step.
+__device__ __forceinline__ float max_over_groups(float v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
+    auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
+#endif
+    return v;
+}
+
+// What is taken off the scaled scores: nothing, a slope's part, the logarithmic penalty, both, or what the pointers say when
+// the kernel runs (heads of more than 64 channels in the wide form; narrower ones have a step of which the branches are a part).
+enum { NO_BIAS = 0, SLOPES = 1, LOG_DIST = 2, ANY_BIAS = 4 };
 
 struct WideArgs {
     int vd;                     // channels of a value
@@ -70,14 +90,18 @@ struct WideArgs {
 // Two maps over rows of up to 128 channels: two workgroups a CU (256 registers a wave) with one step's copies under way are
 // faster than one with two (2,048 tokens, 16 heads of two maps of 64 over values of 128, a window of 1,024: 117 -> 67 us).
 // The wide form with heads of up to 64 channels: left alone it takes 259 registers, three too many for two workgroups a CU (every
-// head's weights on every kv head's values, 2,048 tokens, 32 heads, 8 kv heads of 64: 870 us, with two 555).
-constexpr int groups_a_cu(int hdp, int vdp, int maps, bool ex) {
-    return (maps == 2 && hdp <= 128 && vdp <= 128) || (maps == 1 && ex && hdp <= 64 && vdp <= 64) ? 2 : 1;
+// head's weights on every kv head's values, 2,048 tokens, 32 heads, 8 kv heads of 64: 870 us, with two 555, since then by VHS).
+constexpr int groups_a_cu(int hdp, int vdp, int maps, bool ex, int vhs) {
+    return vhs > 1 || (maps == 2 && hdp <= 128 && vdp <= 128) || (maps == 1 && ex && hdp <= 64 && vdp <= 64) ? 2 : 1;
 }
 
-// HDP, VDP: the channels of a key row and of a value in the tiles, multiples of 32 (a map's share of a key row too).
-template <int HDP, int NBW, int AHEAD, bool EX, int VDP, int MAPS>
-__global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_prefill_kernel(
+// HDP, VDP: the channels of a key row and of a value in the tiles, multiples of 32 (a map's share of a key row too).  NW: waves
+// a workgroup.  VHS: with all_v, the kv heads whose values a workgroup reads: what it has computed of a step's weights (scores,
+// penalty, exponentials, their two halves) then serves VHS heads, where a workgroup for each of them would compute it again,
+// most of its time (2,048 tokens, 32 heads, 8 kv heads of 64, logarithmic penalty: 571 us, with four heads 220).  One column
+// block a wave and eight waves, not two and four: the sums of four heads then fit 256 registers, two waves a SIMD.
+template <int HDP, int NBW, int AHEAD, bool EX, int VDP, int MAPS, int BIAS, int VHS, int NW>
+__global__ __launch_bounds__(NW * WAVE, groups_a_cu(HDP, VDP, MAPS, EX, VHS)) void attn_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     bf16_t* __restrict__ out, const int* __restrict__ block_table, int max_blocks,
     const int2* __restrict__ blk, const int4* __restrict__ req_info,
@@ -85,15 +109,17 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
     int seg_keys, float* __restrict__ ws_o, float* __restrict__ ws_ml, const float* __restrict__ sinks,
     const float* __restrict__ slopes, WideArgs wide) {
     static_assert(MAPS == 1 || (MAPS == 2 && EX && NBW == 2), "two maps are the two column blocks of a wave of the wide form");
+    static_assert(VHS == 1 || (EX && MAPS == 1), "several heads' values: the wide form's");
+    constexpr int NT = NW * WAVE;
     constexpr int HM = HDP / MAPS;        // channels of a map's key in the tiles
     constexpr int KC = HM / 32;           // 32-wide chunks of a key
     constexpr int DB = VDP / 16;          // 16-wide blocks of output channels
     constexpr int HC = HDP / 8;           // 16-byte chunks of a K row
-    constexpr int KROW = HDP + 8;         // bf16 a K row in LDS (padded like V^T rows)
-    constexpr int KBUF = STEP * KROW, VBUF = VDP * VROW;
+    constexpr int KROW = HDP + PAD;       // bf16 a K row in LDS
+    constexpr int KBUF = STEP * KROW, VBUF = VHS * VDP * VROW;
     constexpr int KPT = STEP * HC / NT;   // 16-byte pieces of K a thread copies a step
-    constexpr int VPT = VDP * 8 / NT;     // and of V^T
-    constexpr int CB = 4 * NBW * 16 / MAPS;      // columns of a workgroup
+    constexpr int VPT = VHS * VDP * 8 / NT;   // and of V^T
+    constexpr int CB = NW * NBW * 16 / MAPS;      // columns of a workgroup
     extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
     bf16_t* Ks = lds;                     // [2][KBUF]
     bf16_t* Vs = lds + 2 * KBUF;          // [2][VBUF]
@@ -106,8 +132,9 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
     const int kvh = blockIdx.x % Hkv;
     const int G = H / Hkv;
     const int vd = EX ? wide.vd : hd;
-    const int vh = (EX && wide.all_v) ? (int)blockIdx.y : kvh;          // the kv head whose values are read
-    const bool log_dist = EX && wide.log_r1 != nullptr;
+    const int vh = (EX && wide.all_v) ? (int)blockIdx.y * VHS : kvh;    // the (first) kv head whose values are read
+    const bool log_dist = (BIAS & LOG_DIST) || (BIAS == ANY_BIAS && wide.log_r1 != nullptr);
+    const bool slope = (BIAS & SLOPES) || (BIAS == ANY_BIAS && slopes != nullptr);
     int r = qb, col0 = 0;
     if (blk) { const int2 b = blk[qb]; r = b.x; col0 = b.y; }
     const int4 info = req_info[r];         // (first token of the request in the step, tokens, first position, -)
@@ -146,7 +173,7 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
         const bool valid = c < ncols;
         const int tok = t0 + (valid ? c / G : 0);
         const int head = kvh * G + (valid ? c % G : 0);
-        slope_c[nb] = slopes ? slopes[head] * 1.4426950408889634f : 0.f;
+        slope_c[nb] = slope ? slopes[head] * 1.4426950408889634f : 0.f;
         r1_c[nb] = log_dist ? wide.log_r1[head] : 0.f;
         r2_c[nb] = log_dist ? wide.log_r2[head] : 0.f;
         pos_c[nb] = valid ? pos0 + c / G : -1;
@@ -175,13 +202,15 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
     bf16x8 ones;
 #pragma unroll
     for (int e = 0; e < 8; ++e) ones[e] = (bf16_t)(n16 == 0 ? 1.f : 0.f);
-    f32x4 o[DB][NBW];
+    f32x4 o[VHS][DB][NBW];
 #pragma unroll
     for (int nb = 0; nb < NBW; ++nb) {
         m_run[nb] = -INFINITY;
         l_acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int db = 0; db < DB; ++db) o[db][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int vi = 0; vi < VHS; ++vi)
+#pragma unroll
+            for (int db = 0; db < DB; ++db) o[vi][db][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
 
     if (nsteps == 0) {                     // a segment beyond the block's keys: nothing summed
@@ -195,24 +224,35 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
         return;
     }
 
-    // ---- page numbers: lane i holds the page of granule (16 keys) i of sixteen steps, four a step
+    // ---- where keys and values lie: lane i knows it for granule (16 keys, one page) i of sixteen steps, four a step, as the first
+    // element of the granule's rows in either cache, -1: no such page.  Worked out once in sixteen steps: page numbers to
+    // addresses in every step were 200 scalar instructions and their branches, as long as a step's matrix products.
+    auto key_of_granule = [&](int batch) { return key_of_step(batch * 16 + lane / 4) + 16 * (lane % 4); };
     auto pages_of = [&](int batch) {
-        const long long idx = (long long)(key_of_step(batch * 16 + lane / 4) + 16 * (lane % 4)) / page_size;
-        return idx < max_blocks ? table[idx] : -1;
+        const unsigned idx = (unsigned)key_of_granule(batch) / (unsigned)page_size;
+        return idx < (unsigned)max_blocks ? table[idx] : -1;
     };
-    int pages_cur = pages_of(0), pages_next = pages_of(1);
+    long long k_first, v_first;
+    unsigned long long there;                           // granules whose page exists
+    auto places_of = [&](int batch, int page) {
+        const unsigned off = (unsigned)key_of_granule(batch) % (unsigned)page_size;
+        k_first = page >= 0 ? ((long long)page * Hkv + kvh) * page_size * hd + off * (unsigned)hd : -1;
+        v_first = page >= 0 ? ((long long)page * Hkv + (VHS == 1 ? vh : 0)) * page_size * vd + off : -1;
+        there = __ballot(page >= 0);
+    };
+    places_of(0, pages_of(0));
+    int pages_next = pages_of(1);
 
     // ---- copies: what this thread moves each step.  Memory answers later than a step lasts, so
     // the keys and values of AHEAD steps are on their way at any time, each in a register set.
-    // Per piece the thread keeps what does not change from step to step: the granule (16 keys, one
-    // page) it lies in, its offset inside the granule's rows, and where it goes in LDS.  The pieces
-    // are dealt so that the 64 of a wave lie in one granule: where the granule's rows start in the
-    // caches is then scalar arithmetic, once a piece and wave, not a choice among four addresses in
-    // every lane.
+    // Per piece the thread keeps what does not change from step to step: the granule it lies in, its offset
+    // inside the granule's rows, and where it goes in LDS.  The pieces are dealt so that the 64 of a wave lie
+    // in one granule: where the granule's rows start is then read from its lane, once a piece and wave.
     bf16x8 kreg[AHEAD][KPT], vreg[AHEAD][VPT];
     int k_gran[KPT], k_key[KPT], k_off[KPT], k_lds[KPT], v_gran[VPT], v_key[VPT], v_off[VPT], v_lds[VPT];
     bool k_ok[KPT], v_ok[VPT];
-    static_assert((16 * HC) % WAVE == 0 && (2 * VDP) % WAVE == 0 && NT % WAVE == 0, "a wave's pieces lie in one granule");
+    unsigned v_head[VPT];                               // this piece's kv head's share of a page in the value cache
+    static_assert(KPT >= 1 && VPT >= 1 && (16 * HC) % WAVE == 0 && (2 * VDP) % WAVE == 0 && NT % WAVE == 0, "a wave's pieces lie in one granule");
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
         const int id = tid + i * NT, key = id / HC, c = id % HC;
@@ -225,66 +265,37 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-        const int id = tid + i * NT, c8 = id / VDP, dim = id % VDP;      // lanes run over the channels
+        const int id = tid + i * NT, c8 = id / VDP % 8, dim = id % VDP;  // lanes run over the channels
+        const int vi = VHS == 1 ? 0 : __builtin_amdgcn_readfirstlane(id / (VDP * 8));
+        v_head[i] = (unsigned)(min(vh + vi, Hkv - 1) * page_size * vd);  // (heads beyond the last: read again, never written)
         v_gran[i] = __builtin_amdgcn_readfirstlane(c8 / 2);
         v_key[i] = c8 * 8;
         v_off[i] = dim * page_size + (c8 % 2) * 8;
         v_ok[i] = dim < vd;
-        v_lds[i] = dim * VROW + c8 * 8;
+        v_lds[i] = (vi * VDP + dim) * VROW + c8 * 8;
     }
     const bool whole_rows = qd == HM && vd == VDP;
-    const unsigned page_stride = (unsigned)(Hkv * page_size * hd);       // elements of a page in the key cache (the host checks that it fits)
-    const unsigned head_off = (unsigned)(kvh * page_size * hd);          // this kv head's share of it
-    const unsigned page_stride_v = (unsigned)(Hkv * page_size * vd);     // the same of the value cache
-    const unsigned head_off_v = (unsigned)(vh * page_size * vd);
-    const int ps_mask = (page_size & (page_size - 1)) == 0 ? page_size - 1 : 0;   // a power of two: offsets wrap by a mask
-    int ld_off = key_of_step(0) % page_size;            // offset in its page of the first key of the next step to load
-    auto load_step = [&](int set, int s, int pages) {   // step s of the block -> register set; zeros beyond pos_max
+    auto lane_of_64 = [&](long long v, int at) {
+        const unsigned lo = __builtin_amdgcn_readlane((int)(unsigned)v, at), hi = __builtin_amdgcn_readlane((int)(v >> 32), at);
+        return (long long)((unsigned long long)hi << 32 | lo);
+    };
+    auto load_step = [&](int set, int s) {              // step s of the block -> register set; zeros beyond pos_max
         const int key0 = key_of_step(s);
-        if (EX && s == kept_steps && kept_steps > 0) ld_off = key_start % page_size;      // from the first keys to the window's
-        const int gslot0 = (s % 16) * 4;                // granule of the step's first key within `pages`
-        // per piece, the same for the lanes of a wave: where its granule's rows start (-1: no such page)
-        auto granule = [&](int g4, long long& base, int& go, bool values) {
-            const int page = __builtin_amdgcn_readlane(pages, gslot0 + g4);
-            go = ld_off + 16 * g4;
-            if (ps_mask) go &= ps_mask;
-            else {
+        const int slot = (s % 16) * 4;                  // the step's first granule
+        long long bk[KPT], bv[VPT];                     // per piece, the same for the lanes of a wave
+        const bool all_live = key0 + STEP - 1 <= pos_max && ((there >> slot) & 15) == 15;
 #pragma unroll
-                for (int w = 0; w < 3; ++w)
-                    if (go >= page_size) go -= page_size;
-            }
-            if (EX && values) base = page >= 0 ? (long long)((unsigned long long)(unsigned)page * page_stride_v + head_off_v) : -1;
-            else base = page >= 0 ? (long long)((unsigned long long)(unsigned)page * page_stride + head_off) : -1;
-        };
-        long long bk[KPT], bv[VPT];
-        bool all_live = key0 + STEP - 1 <= pos_max;
-#pragma unroll
-        for (int i = 0; i < KPT; ++i) {
-            int go;
-            granule(k_gran[i], bk[i], go, false);
-            all_live = all_live && bk[i] >= 0;
-            bk[i] += (long long)go * hd;                // (-1 stays negative: go * hd < page_stride)
-        }
+        for (int i = 0; i < KPT; ++i) bk[i] = lane_of_64(k_first, slot + k_gran[i]);
 #pragma unroll
         for (int i = 0; i < VPT; ++i) {
-            int go;
-            granule(v_gran[i], bv[i], go, true);
-            all_live = all_live && bv[i] >= 0;
-            bv[i] += go;
-        }
-        if (ps_mask) ld_off = (ld_off + STEP) & ps_mask;
-        else {
-#pragma unroll
-            for (int w = 0; w < 4; ++w) {
-                ld_off += 16;
-                if (ld_off >= page_size) ld_off -= page_size;
-            }
+            bv[i] = lane_of_64(v_first, slot + v_gran[i]);
+            if (VHS > 1 && bv[i] >= 0) bv[i] += v_head[i];
         }
         if (all_live && whole_rows) {
 #pragma unroll
-            for (int i = 0; i < KPT; ++i) kreg[set][i] = *(const bf16x8*)(k_cache + bk[i] + k_off[i]);
+            for (int i = 0; i < KPT; ++i) kreg[set][i] = *(const bf16x8*)((const char*)(k_cache + bk[i]) + 2u * (unsigned)k_off[i]);
 #pragma unroll
-            for (int i = 0; i < VPT; ++i) vreg[set][i] = *(const bf16x8*)(v_cache + bv[i] + v_off[i]);
+            for (int i = 0; i < VPT; ++i) vreg[set][i] = *(const bf16x8*)((const char*)(v_cache + bv[i]) + 2u * (unsigned)v_off[i]);
             return;
         }
         // first steps under a window, the last step, narrow heads: pieces that do not exist read as zero
@@ -358,24 +369,26 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
             // it is the same instruction with and without the mask.
             float mx = -INFINITY;
             bool ok[2][8];
-            if (slopes || log_dist) {
+            if (slope || log_dist) {
                 // Heads with a distance slope: slope * (position - key) is taken off the scaled score (from the
                 // integer distance, so that far positions lose no bits).  The scores become exponents here, the
                 // maximum is theirs, and the scale below is 1.
+                const int far0 = pos_c[nb] - (key0 + 8 * g);
 #pragma unroll
                 for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
                     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            const int key = key0 + 32 * sub + 8 * g + 4 * kb + e;
-                            float z = fmaf(sc[sub].v[kb][nb][e], scale_log2e, slope_c[nb] * (float)(key - pos_c[nb]));
+                            const int far = far0 - (32 * sub + 4 * kb + e);
+                            const float bias = slope ? -slope_c[nb] * (float)far : 0.f;
+                            float z = fmaf(sc[sub].v[kb][nb][e], scale_log2e, bias);
                             // (ln(1 + x) log2(e) = log2(1 + x); keys after the position are masked below)
-                            if (log_dist) z -= r1_c[nb] * __builtin_amdgcn_logf(fmaf(r2_c[nb], (float)max(pos_c[nb] - key, 0), 1.0f));
+                            if (log_dist) z = fmaf(-r1_c[nb], __builtin_amdgcn_logf(fmaf(r2_c[nb], (float)(open ? far : max(far, 0)), 1.0f)), z);
                             sc[sub].v[kb][nb][e] = z;
                         }
             }
-            const float unit = (slopes || log_dist) ? 1.f : scale_log2e;
+            const float unit = (slope || log_dist) ? 1.f : scale_log2e;
 #pragma unroll
             for (int sub = 0; sub < 2; ++sub)
 #pragma unroll
@@ -387,8 +400,7 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
                         ok[sub][kb * 4 + e] = v;
                         mx = fmaxf(mx, v ? sc[sub].v[kb][nb][e] : -INFINITY);
                     }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+            mx = max_over_groups(mx);
             // The reference point of the exponents moves only when a score exceeds it by more than
             // 2^SLACK: until then the weights may reach 2^SLACK instead of 1, which float32 sums and
             // bfloat16 weights hold as well, and the output so far need not be rescaled.
@@ -410,38 +422,59 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
         if (!__all(same)) {                                  // rare; corr is exactly 1 where the reference stayed
             asm volatile("" ::: "memory");                   // a branch, not a select over every accumulator
 #pragma unroll
-            for (int db = 0; db < DB; ++db)
+            for (int vi = 0; vi < VHS; ++vi)
 #pragma unroll
-                for (int nb = 0; nb < NBW; ++nb)
+                for (int db = 0; db < DB; ++db)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) o[db][nb][e] *= corr[nb];
+                    for (int nb = 0; nb < NBW; ++nb)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) o[vi][db][nb][e] *= corr[nb];
 #pragma unroll
             for (int nb = 0; nb < NBW; ++nb) l_acc[nb][0] *= corr[nb];
         }
+        // The products with the values, some blocks of channels at a time: the next blocks' operands are read from LDS while
+        // these are multiplied, and a block's two products (a weight's two halves) stand apart.
+        static_for<2>([&](auto sub_c) {
+            constexpr int sub = decltype(sub_c)::value;
+            if (!(open || (sub ? live1 : live0))) return;
+            constexpr int GB = DB % 4 == 0 ? 4 : DB % 3 == 0 ? 3 : 2, GROUPS = VHS * DB / GB;
+            bf16x8 vf[2][GB];
+            auto read = [&](auto group) {
+                constexpr int gr = decltype(group)::value;
 #pragma unroll
-        for (int sub = 0; sub < 2; ++sub) {
-            if (!(open || (sub ? live1 : live0))) continue;
+                for (int b = 0; b < GB; ++b) vf[gr % 2][b] = *(const bf16x8*)(Vb + (gr * GB + b) * 16 * VROW + sub * 32);
+            };
+            read(number<0>());
+            if constexpr (VHS > 1) __builtin_amdgcn_sched_group_barrier(0x100, GB, 0);           // LDS reads
+            static_for<GROUPS>([&](auto group) {
+                constexpr int gr = decltype(group)::value;
+                if constexpr (gr + 1 < GROUPS) read(number<gr + 1>());
 #pragma unroll
-            for (int db = 0; db < DB; ++db) {
-                const bf16x8 vf = *(const bf16x8*)(Vb + db * 16 * VROW + sub * 32);
+                for (int half = 0; half < (EX ? 2 : 1); ++half)
 #pragma unroll
-                for (int nb = 0; nb < NBW; ++nb) {
-                    o[db][nb] = mfma32(vf, pf[sub][nb], o[db][nb]);
-                    if (EX) o[db][nb] = mfma32(vf, pf_lo[EX ? sub : 0][nb], o[db][nb]);
+                    for (int b = 0; b < GB; ++b)
+#pragma unroll
+                        for (int nb = 0; nb < NBW; ++nb) {
+                            f32x4& to = o[(gr * GB + b) / DB][(gr * GB + b) % DB][nb];
+                            to = mfma32(vf[gr % 2][b], half ? pf_lo[EX ? sub : 0][nb] : pf[sub][nb], to);
+                        }
+                if constexpr (VHS > 1) {
+                    if constexpr (gr + 1 < GROUPS) __builtin_amdgcn_sched_group_barrier(0x100, GB, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, GB * NBW * (EX ? 2 : 1), 0); // matrix products
                 }
-            }
+            });
 #pragma unroll
             for (int nb = 0; nb < NBW; ++nb) {
                 l_acc[nb] = mfma32(ones, pf[sub][nb], l_acc[nb]);
                 if (EX) l_acc[nb] = mfma32(ones, pf_lo[EX ? sub : 0][nb], l_acc[nb]);
             }
-        }
+        });
     };
 
     // set u holds step u, later step u + AHEAD, ...; step s + 1 goes into LDS while step s is computed.
     // (Loops over sets are unrolled, so a set's registers are named at compile time.)
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) load_step(u, u, pages_cur);
+    for (int u = 0; u < AHEAD; ++u) load_step(u, u);
     store_step(0, 0);
     __syncthreads();
     for (int s0 = 0; s0 < nsteps; s0 += AHEAD) {
@@ -452,9 +485,9 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
             const int buf = s & 1;
             const int key0 = key_of_step(s);
             const int ls = s + AHEAD;                   // the step whose loads start now
-            if (ls % 16 == 0) pages_cur = pages_next;
+            if (ls % 16 == 0) places_of(ls / 16, pages_next);
             if (ls % 16 == 1) pages_next = pages_of(ls / 16 + 1);
-            load_step(u, ls, pages_cur);
+            load_step(u, ls);
             const int lo_any = window > 0 ? max(0, wave_pos_min - window + 1) : 0;
             const bool live0 = key0 <= wave_pos_max && (key0 + 31 >= lo_any || (EX && key0 < keep));
             const bool live1 = key0 + 32 <= wave_pos_max && (key0 + 63 >= lo_any || (EX && key0 + 32 < keep));
@@ -474,8 +507,8 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
         for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {                      // (channels beyond vd are zeros in both)
-                const float v = fmaf(-inv1, o[db][1][e], o[db][0][e] * inv0);
-                o[db][0][e] = v;
+                const float v = fmaf(-inv1, o[0][db][1][e], o[0][db][0][e] * inv0);
+                o[0][db][0][e] = v;
                 ss = fmaf(v, v, ss);
             }
         ss += __shfl_xor(ss, 16, WAVE);
@@ -486,7 +519,7 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
         for (int db = 0; db < DB; ++db) {
             const int dim = db * 16 + 4 * g;
             if (dim < vd) {
-                const f32x4 v = o[db][0];
+                const f32x4 v = o[0][db][0];
                 bf16x4 w = {(bf16_t)(v[0] * by), (bf16_t)(v[1] * by), (bf16_t)(v[2] * by), (bf16_t)(v[3] * by)};
                 *(bf16x4*)(out + qrow[0] * vd + dim) = w;
             }
@@ -504,7 +537,7 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
 #pragma unroll
             for (int db = 0; db < DB; ++db) {
                 const int dim = db * 16 + 4 * g;
-                if (dim < hd) *(f32x4*)(ws_o + slot * hd + dim) = o[db][nb];
+                if (dim < hd) *(f32x4*)(ws_o + slot * hd + dim) = o[0][db][nb];
             }
             continue;
         }
@@ -517,13 +550,17 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
             inv = keep / (l * keep + __builtin_amdgcn_exp2f(s2 - m_all));
         }
         if (EX && wide.all_v) {
-            float* dst = wide.out_wide + (qrow[nb] * Hkv + vh) * vd;
 #pragma unroll
-            for (int db = 0; db < DB; ++db) {
-                const int dim = db * 16 + 4 * g;
-                if (dim < vd) {
-                    const f32x4 v = o[db][nb];
-                    *(f32x4*)(dst + dim) = f32x4{v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv};
+            for (int vi = 0; vi < VHS; ++vi) {
+                if (vh + vi >= Hkv) break;
+                float* dst = wide.out_wide + (qrow[nb] * Hkv + vh + vi) * vd;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) {
+                    const int dim = db * 16 + 4 * g;
+                    if (dim < vd) {
+                        const f32x4 v = o[vi][db][nb];
+                        *(f32x4*)(dst + dim) = f32x4{v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv};
+                    }
                 }
             }
             continue;
@@ -532,7 +569,7 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
         for (int db = 0; db < DB; ++db) {
             const int dim = db * 16 + 4 * g;
             if (dim < vd) {
-                const f32x4 v = o[db][nb];
+                const f32x4 v = o[0][db][nb];
                 bf16x4 w = {(bf16_t)(v[0] * inv), (bf16_t)(v[1] * inv), (bf16_t)(v[2] * inv), (bf16_t)(v[3] * inv)};
                 *(bf16x4*)(out + qrow[nb] * vd + dim) = w;
             }
@@ -540,19 +577,19 @@ __global__ __launch_bounds__(NT, groups_a_cu(HDP, VDP, MAPS, EX)) void attn_pref
     }
 }
 
-template <int HDP, int NBW, int AHEAD, bool EX = false, int VDP = HDP, int MAPS = 1>
+template <int HDP, int NBW, int AHEAD, int BIAS, bool EX = false, int VDP = HDP, int MAPS = 1, int VHS = 1, int NW = 4>
 int launch(dim3 grid, hipStream_t stream, const bf16_t* q, const bf16_t* kc, const bf16_t* vc, bf16_t* out,
            const int* bt, int max_blocks, const int2* blk, const int4* req_info,
            int H, int Hkv, int hd, int ps, int window, float scale_log2e, int seg_keys, float* ws_o, float* ws_ml,
            const float* sinks, const float* slopes, WideArgs wide = WideArgs{0, nullptr, nullptr, 0, nullptr, 0, 0.f, 0.f, 0.f}) {
-    auto kern = attn_prefill_kernel<HDP, NBW, AHEAD, EX, VDP, MAPS>;
-    constexpr int lds = 2 * (STEP * (HDP + 8) + VDP * VROW) * 2;
+    auto kern = attn_prefill_kernel<HDP, NBW, AHEAD, EX, VDP, MAPS, BIAS, VHS, NW>;
+    constexpr int lds = 2 * (STEP * (HDP + PAD) + VHS * VDP * VROW) * 2;
     static bool set = false;
     if (!set) {
         if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return -1;
         set = true;
     }
-    hipLaunchKernelGGL(kern, grid, dim3(NT), lds, stream, q, kc, vc, out, bt, max_blocks, blk, req_info,
+    hipLaunchKernelGGL(kern, grid, dim3(NW * WAVE), lds, stream, q, kc, vc, out, bt, max_blocks, blk, req_info,
                        H, Hkv, hd, ps, window, scale_log2e, seg_keys, ws_o, ws_ml, sinks, slopes, wide);
     return launch_status();
 }
@@ -589,14 +626,16 @@ TUFF_EXPORT int tuff_attention_prefill_biased(const void* q, const void* k_cache
     if ((long long)n_qblocks * Hkv > 0x7fffffffll) return -2;
     dim3 grid(n_qblocks * Hkv, 1, n_segs);
     const float sl = scale * 1.4426950408889634f;
-#define GO(HDP, NBW, AHEAD) return launch<HDP, NBW, AHEAD>(grid, stream, Q, K, V, (bf16_t*)out, block_table, max_blocks, (const int2*)blk, \
+#define GO_BIAS(HDP, NBW, AHEAD, BIAS) return launch<HDP, NBW, AHEAD, BIAS>(grid, stream, Q, K, V, (bf16_t*)out, block_table, max_blocks, (const int2*)blk, \
                                              (const int4*)req_info, H, Hkv, hd, page_size, window, sl, seg_keys, ws_o, ws_ml, n_segs > 1 ? nullptr : sinks, slopes)
+#define GO(HDP, NBW, AHEAD) do { if (slopes) GO_BIAS(HDP, NBW, AHEAD, SLOPES); GO_BIAS(HDP, NBW, AHEAD, NO_BIAS); } while (0)
     if (hd <= 32) GO(32, 2, 3);
     else if (hd <= 64) GO(64, 2, 2);
     else if (hd <= 96) GO(96, 2, 2);
     else if (hd <= 128) GO(128, 2, 2);
     else GO(256, 2, 1);
 #undef GO
+#undef GO_BIAS
 }
 
 TUFF_EXPORT int tuff_attention_prefill_sinks(const void* q, const void* k_cache, const void* v_cache, void* out,
@@ -635,12 +674,29 @@ TUFF_EXPORT int tuff_attention_prefill_wide(const void* q, const void* k_cache, 
     const float sl = scale * 1.4426950408889634f;
     const WideArgs wide{vd, log_r1, log_r2, all_v, all_v ? (float*)out : nullptr, window > 0 ? keep_first : 0, 0.f, 0.f, 0.f};
     const int widest = max(hd, vd);
-#define GO(HDP, NBW, AHEAD, VDP) return launch<HDP, NBW, AHEAD, true, VDP>(grid, stream, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, \
+#define GO(HDP, NBW, AHEAD, VDP) return launch<HDP, NBW, AHEAD, ANY_BIAS, true, VDP>(grid, stream, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, \
         (bf16_t*)out, block_table, max_blocks, (const int2*)blk, (const int4*)req_info, H, Hkv, hd, page_size, window, sl, 0, nullptr, \
         nullptr, sinks, slopes, wide)
-    if (widest <= 32) GO(32, 2, 3, 32);
-    else if (widest <= 64) GO(64, 2, 2, 64);
-    else if (widest <= 96) GO(96, 2, 2, 96);
+    auto narrow = [&](auto hdp, auto ahead, auto nbw, auto vhs, auto nw) {
+        auto go = [&](auto bias) {
+            constexpr int HDP = decltype(hdp)::value;
+            return launch<HDP, decltype(nbw)::value, decltype(ahead)::value, decltype(bias)::value, true, HDP, 1, decltype(vhs)::value, decltype(nw)::value>(
+                grid, stream, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, (bf16_t*)out, block_table, max_blocks,
+                (const int2*)blk, (const int4*)req_info, H, Hkv, hd, page_size, window, sl, 0, nullptr, nullptr, sinks, slopes, wide);
+        };
+        if (slopes) return log_r1 ? go(number<SLOPES | LOG_DIST>()) : go(number<SLOPES>());
+        return log_r1 ? go(number<LOG_DIST>()) : go(number<NO_BIAS>());
+    };
+    // Four kv heads' values a workgroup from three kv heads on (from four where heads have at most 32 channels: the tiles are 64
+    // wide; 2,048 tokens, 12 heads on 3 kv heads of 32: 97 us in one-head workgroups, 102 in this; 16 on 4 of 16: 170, 112).
+    constexpr int VHS = 4;
+    if (all_v && widest <= 64 && Hkv > (widest <= 32 ? 3 : 2)) {
+        grid.y = ceil_div(Hkv, VHS);
+        return narrow(number<64>(), number<1>(), number<1>(), number<VHS>(), number<8>());
+    }
+    if (widest <= 32) return narrow(number<32>(), number<3>(), number<2>(), number<1>(), number<4>());
+    if (widest <= 64) return narrow(number<64>(), number<2>(), number<2>(), number<1>(), number<4>());
+    if (widest <= 96) GO(96, 2, 2, 96);
     else if (widest <= 128) GO(128, 2, 2, 128);
     else if (hd <= 192 && vd <= 128) GO(192, 2, 1, 128);       // wide rows: tiles no wider than they need be
     else if (hd <= 192 && vd <= 192) GO(192, 2, 1, 192);
@@ -669,7 +725,7 @@ TUFF_EXPORT int tuff_attention_prefill_diff(const void* q, const void* k_cache, 
     dim3 grid(n_qblocks * Hkv, 1, 1);
     const float sl = scale * 1.4426950408889634f;
     const WideArgs wide{vd, nullptr, nullptr, 0, nullptr, window > 0 ? keep_first : 0, lambda, eps, coef};
-#define GO(HDP, AHEAD, VDP) return launch<HDP, 2, AHEAD, true, VDP, 2>(grid, stream, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, \
+#define GO(HDP, AHEAD, VDP) return launch<HDP, 2, AHEAD, NO_BIAS, true, VDP, 2>(grid, stream, (const bf16_t*)q, (const bf16_t*)k_cache, (const bf16_t*)v_cache, \
         (bf16_t*)out, block_table, max_blocks, (const int2*)blk, (const int4*)req_info, heads, Hkv, hd, page_size, window, sl, 0, nullptr, \
         nullptr, nullptr, nullptr, wide)
     if (dim <= 32) { if (vd <= 64) GO(64, 2, 64); else if (vd <= 128) GO(64, 1, 128); else GO(64, 1, 256); }
