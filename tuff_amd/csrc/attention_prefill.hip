@@ -232,13 +232,19 @@ __global__ __launch_bounds__(NW * WAVE, groups_a_cu(HDP, VDP, MAPS, EX, VHS)) vo
         const unsigned idx = (unsigned)key_of_granule(batch) / (unsigned)page_size;
         return idx < (unsigned)max_blocks ? table[idx] : -1;
     };
+    const unsigned ps_mask = (page_size & (page_size - 1)) == 0 ? page_size - 1 : 0;   // a power of two: offsets wrap by a mask
     long long k_first, v_first;
     unsigned long long there;                           // granules whose page exists
     auto places_of = [&](int batch, int page) {
-        const unsigned off = (unsigned)key_of_granule(batch) % (unsigned)page_size;
-        k_first = page >= 0 ? ((long long)page * Hkv + kvh) * page_size * hd + off * (unsigned)hd : -1;
-        v_first = page >= 0 ? ((long long)page * Hkv + (VHS == 1 ? vh : 0)) * page_size * vd + off : -1;
+        k_first = v_first = -1;
         there = __ballot(page >= 0);
+        if (page >= 0) {
+            unsigned go = (unsigned)key_of_granule(batch);               // becomes the granule's offset in its page
+            if (ps_mask) go &= ps_mask;
+            else go %= (unsigned)page_size;
+            k_first = ((long long)page * Hkv + kvh) * page_size * hd + go * (unsigned)hd;
+            v_first = ((long long)page * Hkv + (VHS == 1 ? vh : 0)) * page_size * vd + go;
+        }
     };
     places_of(0, pages_of(0));
     int pages_next = pages_of(1);
@@ -380,11 +386,16 @@ __global__ __launch_bounds__(NW * WAVE, groups_a_cu(HDP, VDP, MAPS, EX, VHS)) vo
                     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            const int far = far0 - (32 * sub + 4 * kb + e);
+                            const int key = key0 + 32 * sub + 8 * g + 4 * kb + e, far = far0 - (32 * sub + 4 * kb + e);
                             const float bias = slope ? -slope_c[nb] * (float)far : 0.f;
                             float z = fmaf(sc[sub].v[kb][nb][e], scale_log2e, bias);
-                            // (ln(1 + x) log2(e) = log2(1 + x); keys after the position are masked below)
-                            if (log_dist) z = fmaf(-r1_c[nb], __builtin_amdgcn_logf(fmaf(r2_c[nb], (float)(open ? far : max(far, 0)), 1.0f)), z);
+                            if (log_dist) {
+                                // (ln(1 + x) log2(e) = log2(1 + x); keys after the position are masked below)
+                                float grown;
+                                if (open) grown = __builtin_amdgcn_logf(fmaf(r2_c[nb], (float)far, 1.0f));
+                                else grown = __builtin_amdgcn_logf(fmaf(r2_c[nb], (float)max(pos_c[nb] - key, 0), 1.0f));
+                                z = fmaf(-r1_c[nb], grown, z);
+                            }
                             sc[sub].v[kb][nb][e] = z;
                         }
             }
