@@ -65,6 +65,31 @@ def test_gemm_f32_matrix_cores(gpu, M, N, K):
             assert torch.equal(some, out[M - m:]), m
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 64), (4, 17, 128), (3, 250, 704), (4, 4097, 768), (2, 2048, 832), (5, 16, 2112), (13, 2040, 1536),
+                                   (16, 2048, 64), (16, 8200, 320), (9, 4100, 96), (16, 70, 32), (1, 33, 160), (7, 300, 544), (12, 33, 1056)])
+def test_gemm_f32_few_rows(gpu, M, N, K):
+    """Up to 16 rows, on the vector unit in groups of four and on the matrix cores, with steps fewer and more than lie in LDS, odd and
+    even: the bits of the general kernel's chain; rows behind the last, which are not a number, count nowhere."""
+    from tuff_amd.csrc import ops
+    behind = torch.full((M + 16, K), float("nan"), device=gpu)
+    behind[:M] = _r(M, K, seed=1).to(gpu)
+    columns = torch.full((N + 16, K), float("nan"), device=gpu)
+    columns[:N] = _r(N, K, seed=2).to(gpu)
+    x, w, y0 = behind[:M], columns[:N], _r(M, N, seed=3).to(gpu)
+    x[M // 2] *= 1e-20                                # products of denormal size
+    w[N // 2] *= 1e-20
+    out = torch.full((M, N), float("nan"), device=gpu)
+    ops.gemm(x, w, out)
+    off = torch.empty(M * K + 1, device=gpu)[1:].view(M, K)
+    off.copy_(x)
+    general = torch.empty(M, N, device=gpu)
+    ops.gemm(off, w, general)
+    assert torch.equal(out, general)
+    acc = y0.clone()
+    ops.gemm(x, w, acc, accumulate=True)
+    assert torch.equal(acc, y0 + out)
+
+
 def test_gemm_f32_more_rows_than_small_blocks_count(gpu):
     """A narrow output of more rows than a grid has blocks of 32 for takes blocks of 64 (it was refused)."""
     from tuff_amd.csrc import ops

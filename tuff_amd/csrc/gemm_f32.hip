@@ -75,11 +75,9 @@ __global__ __launch_bounds__(NT) void gemm_f32_kernel(const float* __restrict__ 
 // touches spread over the banks.  A wave's load instruction fills 1 KB, eight rows.  For instruction i of a step a lane
 // (row r16 = lane % 16, group g = lane / 16) reads element g of piece i of its row: k = 4 i + g.
 //
-// What bounds it: a matrix instruction takes 32 cycles (157 TFLOP/s), and one that waits for the one before it in its
-// chain 48 or more: with one tile a wave K = 8,192 takes 61 us, whatever the number of rows.  Up to 16 rows: blocks of 16x16,
-// a wave a workgroup (2,048 x 8,192: 61 us; 16,384 x 2,048 of 4 rows: 30 us, 4.4 TB/s; 65,536 x 2,048: 107 us, 5.0 TB/s.  The
-// general kernel: 825, 345 and 432 us).  More rows: blocks of 64x64 or, where those leave CUs idle, of 32x32; see
-// block_cycles (500 rows, 16,384 x 2,048: 283 us, 119 TFLOP/s, the general kernel 577; 2,048 x 8,192: 160 us against 1,480).
+// More than 16 rows: blocks of 64x64 or, where those leave CUs idle, of 32x32; see block_cycles.  What bounds it: a matrix
+// instruction takes 32 cycles (157 TFLOP/s); 500 rows, 16,384 x 2,048: 283 us, 119 TFLOP/s, the general kernel 577; 2,048 x
+// 8,192: 160 us against 1,480.
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
 constexpr int STEP = 32;
@@ -215,6 +213,236 @@ __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(co
     }
 }
 
+// ---------------------------------------------------------------------------------------- few rows
+// Up to 16 rows: a wave a workgroup, 16 columns, the same chain and the same tiles in LDS as above.  With one tile a wave the
+// chain sets the pace, one matrix instruction after the other (33 cycles each with nothing between them): the operands of a
+// whole step (eight instructions) are read from LDS into one of two register sets while the other is multiplied, and all reads
+// are waited for at once, where they have long arrived, so that no product waits for LDS (the kernel above, half a step ahead:
+// 2,048 x 8,192 of 16 rows 58 us, this one 49; 65,536 x 2,048 of 4 rows 107 and 102, 5.3 TB/s).  Rows beyond X are not
+// fetched.  STAGES: steps of 32 k in LDS, 16 where two workgroups fill a CU's share of the launch anyway.
+template <int STAGES>
+__global__ __launch_bounds__(WAVE) void gemm_f32_rows_kernel(const float* __restrict__ X, const float* __restrict__ W,
+                                                             float* __restrict__ Y, int M, int N, int K, int accumulate) {
+    constexpr int TILE = 16 * STEP, PER = 4;              // floats of a tile; load instructions a step
+    static_assert(STAGES % 2 == 0 && PER * (STAGES - 2) < 64, "pairs of steps, and a count that s_waitcnt can hold");
+    extern __shared__ __attribute__((aligned(16))) float tiles[];      // [STAGES][X, W][TILE]
+    const int lane = threadIdx.x, r16 = lane % 16, g = lane / 16;
+    const long long n0 = (long long)blockIdx.x * 16;
+    const int rows_n = (int)min(16ll, (long long)N - n0);
+    const buffer_t xbuf = make_buffer(X, M * K * 4), wbuf = make_buffer(W + n0 * K, rows_n * K * 4);
+    int offx[2], offw[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int row = i * 8 + lane / 8, piece = (lane % 8) ^ (lane / 8);
+        offx[i] = row < M ? (row * K + piece * 4) * 4 : NOWHERE;
+        offw[i] = row < rows_n ? (row * K + piece * 4) * 4 : NOWHERE;
+    }
+    const int steps = K / STEP;
+    auto issue = [&](int s) {
+        float* to = tiles + s % STAGES * (2 * TILE);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) load_to_lds(xbuf, to + i * 256, offx[i], s * (STEP * 4));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) load_to_lds(wbuf, to + TILE + i * 256, offw[i], s * (STEP * 4));
+    };
+    int at[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) at[i] = r16 * STEP + ((i ^ (r16 % 8)) * 4 + g);
+    float x[2][8], w[2][8];
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto read = [&](auto set, int s) {
+        const float* from = tiles + s % STAGES * (2 * TILE);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            w[decltype(set)::value][i] = from[TILE + at[i]];
+            x[decltype(set)::value][i] = from[at[i]];
+        }
+    };
+    auto multiply = [&](auto set) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc = mfma_f32(w[decltype(set)::value][i], x[decltype(set)::value][i], acc);
+    };
+    using Set0 = std::integral_constant<int, 0>;
+    using Set1 = std::integral_constant<int, 1>;
+    // (reads of step s + 1, products of step s)
+    auto turn = [&](auto set, int s) {
+        read(std::integral_constant<int, 1 - decltype(set)::value>(), s + 1);
+        multiply(set);
+        static_for<8>([&](auto) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);         // LDS reads
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);         // a matrix instruction
+        });
+    };
+    for (int st = 0; st < min(STAGES - 1, steps); ++st) issue(st);
+    int s = 0;
+    if (steps < STAGES) wait_loads_and_lds<0>();
+    wait_loads_and_lds<PER * (STAGES - 2)>();
+    read(Set0(), 0);
+    if (steps % 2) {                                      // an odd number of steps: one by itself, then pairs
+        if (STAGES - 1 < steps) issue(STAGES - 1); else wait_loads_and_lds<0>();
+        wait_loads_and_lds<PER * (STAGES - 2)>();
+        if (steps > 1) {
+            turn(Set0(), 0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) { x[0][i] = x[1][i]; w[0][i] = w[1][i]; }
+        } else multiply(Set0());
+        s = 1;
+    }
+    for (; steps - s > STAGES; s += 2) {
+        issue(s + STAGES - 1);
+        wait_loads_and_lds<PER * (STAGES - 2)>();                 // all but those of steps s + 2 and later
+        turn(Set0(), s);
+        issue(s + STAGES);
+        wait_loads_and_lds<PER * (STAGES - 2)>();
+        turn(Set1(), s + 1);
+    }
+    static_for<STAGES>([&](auto i) {                      // the last STAGES steps, fewer if there are fewer; an even number
+        constexpr int later = STAGES - 1 - decltype(i)::value;
+        using Set = std::integral_constant<int, 1 - later % 2>;
+        if (steps - s <= later) return;
+        if constexpr (later == STAGES - 1) issue(s + later);
+        if constexpr (later > 0) {
+            wait_loads_and_lds<PER * (later - 1)>();
+            turn(Set(), s);
+        } else multiply(Set());
+        ++s;
+    });
+    const int row = r16;
+    if (row >= M) return;
+    const long long col = n0 + g * 4;
+    float* y = Y + (long long)row * N + col;
+    if (N % 4 == 0 && col + 3 < N) {
+        if (accumulate) { const f32x4 old = *(const f32x4*)y; acc[0] = old[0] + acc[0]; acc[1] = old[1] + acc[1]; acc[2] = old[2] + acc[2]; acc[3] = old[3] + acc[3]; }
+        *(f32x4*)y = acc;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (col + e < N) y[e] = accumulate ? y[e] + acc[e] : acc[e];
+    }
+}
+
+// ---------------------------------------------------------------------------------------- four rows
+// Four rows by 16 columns a wave, the chain on the vector unit: lane (row g, column r16) has one element, v_fmac_f32 takes its
+// x from lane k % 16 of the row's sixteen lanes (row_newbcast), so sixteen k of X are one register, and its w from the lane's own
+// column.  A fused multiply-add waits 6 cycles for the one before it, four of them 24, where a matrix instruction of four k
+// takes 33 and in a loop with its reads 50: where nothing but the chain's length counts, this is the shorter one.  A lone wave
+// issues an instruction in five cycles, so the loop holds next to nothing but the chain, its reads and loads: places in LDS are
+// constants.  4 rows, 2,048 x 8,192: 35 us (rows kernel 49), 2,048 x 2,048: 10.6 (13.9), 6,144 x 2,048: 12.4 (15.7).
+// K in steps of 64: X rows of 256 bytes, piece p (16 bytes) of row g at p ^ 4 g; W rows of 256 bytes, piece p of column c at p ^ c.
+__device__ __forceinline__ void chain16(float& acc, float x, const f32x4 (&w)[4]) {
+#ifdef __HIP_DEVICE_COMPILE__
+    // (s_nop: two wait states, should the compiler have moved x by a vector instruction just before)
+    asm("s_nop 1\n"
+        "v_fmac_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %3 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %4 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %5 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %6 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %7 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %8 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %9 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %10 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %11 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %12 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %13 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %14 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %15 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %16 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %1, %17 row_newbcast:15 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc)
+        : "v"(x), "v"(w[0][0]), "v"(w[0][1]), "v"(w[0][2]), "v"(w[0][3]), "v"(w[1][0]), "v"(w[1][1]), "v"(w[1][2]), "v"(w[1][3]),
+          "v"(w[2][0]), "v"(w[2][1]), "v"(w[2][2]), "v"(w[2][3]), "v"(w[3][0]), "v"(w[3][1]), "v"(w[3][2]), "v"(w[3][3]));
+#endif
+}
+
+constexpr int LONG_STEP = 64;
+
+// A wave a workgroup; `row_groups` workgroups of one column block on one XCD (numbers eight apart), so that its L2 serves W again.
+template <int STAGES>
+__global__ __launch_bounds__(WAVE) void gemm_f32_quad_kernel(const float* __restrict__ X, const float* __restrict__ W,
+                                                             float* __restrict__ Y, int M, int N, int K, int row_groups, int accumulate) {
+    constexpr int WTILE = 16 * LONG_STEP, XTILE = 4 * LONG_STEP, STAGE = WTILE + XTILE;
+    constexpr int PER = 5;                                // load instructions a step
+    static_assert(PER * (STAGES - 2) < 64, "a count that s_waitcnt can hold");
+    extern __shared__ __attribute__((aligned(16))) float tiles[];      // [STAGES][W, X]
+    const int lane = threadIdx.x, r16 = lane % 16, g = lane / 16;
+    const int id = blockIdx.x, group = id / 8 % row_groups, block = id / (8 * row_groups) * 8 + id % 8;
+    const long long n0 = (long long)block * 16;
+    const int m0 = group * 4;
+    if (n0 >= N) return;
+    const int rows_m = min(4, M - m0), rows_n = (int)min(16ll, (long long)N - n0);
+    const int offx = g < rows_m ? (g * K + (r16 ^ (4 * g)) * 4) * 4 : NOWHERE;
+    int offw[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = i * 4 + g;
+        offw[i] = row < rows_n ? (row * K + (r16 ^ row) * 4) * 4 : NOWHERE;
+    }
+    const int steps = K / LONG_STEP;
+    const float* xrows = X + (long long)m0 * K;
+    const float* wrows = W + n0 * K;
+    // Steps beyond the last are asked for too, of buffers without bytes (zeros, no traffic): the count of loads under way is then
+    // the same in every step, and the places in LDS are constants of a ring of steps.
+    auto issue = [&](auto buf, int s) {
+        const bool there = s < steps;
+        const buffer_t xbuf = make_buffer(xrows, there ? rows_m * K * 4 : 0), wbuf = make_buffer(wrows, there ? rows_n * K * 4 : 0);
+        const int at = there ? s * (LONG_STEP * 4) : 0;
+        float* to = tiles + decltype(buf)::value * STAGE;
+        load_to_lds(xbuf, to + WTILE, offx, at);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) load_to_lds(wbuf, to + i * 256, offw[i], at);
+    };
+    int atw[4][4], atx[4];                                // of every piece of a row: where it lies
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) atw[q][i] = r16 * LONG_STEP + ((4 * q + i) ^ r16) * 4;
+        atx[q] = WTILE + g * LONG_STEP + (q ^ g) * 16 + r16;
+    }
+    struct Half { f32x4 w[2][4]; float x[2]; };
+    auto read = [&](auto buf, auto half) {
+        const float* from = tiles + decltype(buf)::value * STAGE;
+        Half h;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            constexpr int first = 2 * decltype(half)::value;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h.w[q][i] = *(const f32x4*)(from + atw[first + q][i]);
+            h.x[q] = from[atx[first + q]];
+        }
+        return h;
+    };
+    float acc = 0.f;
+    auto multiply = [&](const Half& h) {
+        chain16(acc, h.x[0], h.w[0]);
+        chain16(acc, h.x[1], h.w[1]);
+    };
+    using H0 = std::integral_constant<int, 0>;
+    using H1 = std::integral_constant<int, 1>;
+    static_for<STAGES - 1>([&](auto buf) { issue(buf, decltype(buf)::value); });
+    wait_loads_and_lds<PER * (STAGES - 2)>();
+    Half h0 = read(H0(), H0()), h1;
+    for (int s0 = 0; s0 < steps; s0 += STAGES)
+        static_for<STAGES>([&](auto buf) {
+            constexpr int b = decltype(buf)::value;
+            if (s0 + b >= steps) return;
+            h1 = read(buf, H1());
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(h0);
+            // (the buffer of the step before: its last reads were waited for by the products they went into)
+            issue(std::integral_constant<int, (b + STAGES - 1) % STAGES>(), s0 + b + STAGES - 1);
+            wait_loads_and_lds<PER * (STAGES - 2)>();     // all but those of steps s0 + b + 2 and later
+            h0 = read(std::integral_constant<int, (b + 1) % STAGES>(), H0());
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(h1);
+        });
+    wait_loads_and_lds<0>();                              // nothing may land in LDS that is another workgroup's by then
+    if (g < rows_m && r16 < rows_n) {
+        float* y = Y + (long long)(m0 + g) * N + n0 + r16;
+        *y = accumulate ? *y + acc : acc;
+    }
+}
+
 // What the slowest CU takes for four k, in cycles, as measured over 17 to 2,048 rows and 2,048 to 65,536 columns: a round
 // of 64x64 blocks (four tiles a wave) 170 to 185 whether a CU holds one block or shares its time among several, 32x32 blocks
 // (one tile a wave) 62 to 70 each and 71 at least.  The fewer: 300 rows of 2,048 x 2,048 36 us in 32x32 and 41 in 64x64 blocks, 500
@@ -223,6 +451,24 @@ long long block_cycles(int M, int N, int side) {
     constexpr long long CUS = 256;
     const long long blocks = ceil_div_ll(M, side) * ceil_div_ll(N, side);
     return side == 64 ? ceil_div_ll(blocks, CUS) * 170 : max(71ll, blocks * 62 / CUS);
+}
+
+template <int STAGES>
+int launch_quad(const float* X, const float* W, float* Y, int M, int N, int K, int accumulate, hipStream_t stream) {
+    constexpr int lds = STAGES * 20 * LONG_STEP * (int)sizeof(float);
+    static_assert(lds <= 65536, "without asking for more");
+    const int row_groups = ceil_div(M, 4);
+    hipLaunchKernelGGL((gemm_f32_quad_kernel<STAGES>), dim3(ceil_div(ceil_div(N, 16), 8) * 8 * row_groups), dim3(WAVE), lds, stream,
+                       X, W, Y, M, N, K, row_groups, accumulate);
+    return launch_status();
+}
+
+template <int STAGES>
+int launch_rows(const float* X, const float* W, float* Y, int M, int N, int K, int accumulate, hipStream_t stream) {
+    constexpr int lds = STAGES * 2 * 16 * STEP * (int)sizeof(float);
+    static_assert(lds <= 65536, "without asking for more");
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<STAGES>), dim3(ceil_div(N, 16)), dim3(WAVE), lds, stream, X, W, Y, M, N, K, accumulate);
+    return launch_status();
 }
 
 template <int T, int WAVES, int STAGES>
@@ -248,7 +494,18 @@ TUFF_EXPORT int tuff_gemm_f32(const float* X, const float* W, float* Y, int M, i
         else hipLaunchKernelGGL(gemm_f32_kernel<false>, grid, block, 0, stream, X, W, Y, M, N, K);
         return launch_status();
     }
-    if (M <= 16) return launch_chain<1, 1, 8>(X, W, Y, M, N, K, accumulate, stream);
+    if (M <= 16) {
+        // Four rows a wave as long as one trip over W serves all rows, or the waves are few enough to run side by side, two a CU (16
+        // rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14).  Twelve steps in LDS where
+        // a CU has one wave (8,192 x 1,024, two a CU: 11.7 us, with six 10.3).
+        const long long waves = ceil_div_ll(N, 16) * ceil_div(M, 4);
+        if (K % LONG_STEP == 0 && (M <= 4 || waves <= 512)) {
+            if (waves <= 256) return launch_quad<12>(X, W, Y, M, N, K, accumulate, stream);
+            return launch_quad<6>(X, W, Y, M, N, K, accumulate, stream);
+        }
+        if (N <= 4096) return launch_rows<16>(X, W, Y, M, N, K, accumulate, stream);
+        return launch_rows<8>(X, W, Y, M, N, K, accumulate, stream);
+    }
     constexpr int MOST_BLOCKS = 65535;                    // of rows in a grid
     if (ceil_div(M, 32) <= MOST_BLOCKS && block_cycles(M, N, 32) < block_cycles(M, N, 64))
         return launch_chain<1, 2, 4>(X, W, Y, M, N, K, accumulate, stream);
