@@ -470,6 +470,49 @@ def test_scan_gives_the_same_bits_for_any_company_and_alignment(gpu, D):
                 assert torch.equal(state[i], state0[i])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind, H, D, Dv", [("forget", 3, 40, 33), ("forget", 2, 64, 128), ("forget", 5, 65, 32), ("ssd", 4, 64, 40),
+                                            ("ssd", 2, 128, 64), ("delta", 3, 100, 130), ("delta", 2, 192, 48), ("wkv", 3, 72, 72),
+                                            ("wkv", 1, 128, 128)])
+def test_runs_in_four_waves_have_the_bits_of_short_runs(gpu, kind, H, D, Dv, dtype):
+    """Runs of 32 tokens and more, whose waves bring rows into LDS for each other, in one step with shorter ones; and the same
+    tokens in steps of up to 20, which waves take alone: numbers of tokens around sixteen, channels that fill no tile."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(H + D + Dv)
+    rnd = lambda *shape: torch.randn(*shape, generator=gen)
+    lens = [65, 31, 48, 1, 111]
+    T, R = sum(lens), len(lens)
+    if kind == "forget":
+        rows = [rnd(T, 2 * H * D + H * Dv).to(dtype)]
+        bias, lower = rnd(H * D).to(gpu), torch.rand(H * D, generator=gen).to(gpu)
+        call = lambda x, s, o, **kw: ops.forget_scan(x, bias, lower, s, o, H=H, D=D, Dv=Dv, **kw)
+    elif kind == "ssd":
+        rows = [rnd(T, H * Dv + 2 * D).to(dtype), rnd(T, H)]
+        b, A, skip = (rnd(H).to(gpu) for _ in range(3))
+        call = lambda x, r, s, o, **kw: ops.ssd_scan(x, r, b, A, skip, s, o, H=H, G=1, N=D, P=Dv, **kw)
+    elif kind == "delta":
+        rows = [rnd(T, H * D).to(dtype), rnd(T, H * D).to(dtype), rnd(T, H * Dv).to(dtype), rnd(T, H * D), rnd(T, H)]
+        b, A = rnd(H * D).to(gpu), rnd(H).to(gpu)
+        call = lambda q, k, v, a, beta, s, o, **kw: ops.delta_scan(q, k, v, a, b, A, beta, s, o, H=H, Hk=H, D=D, Dv=Dv, **kw)
+    else:
+        rows = [rnd(T, H * D).to(dtype) for _ in range(3)] + [rnd(T, H * D) * 0.5]
+        w0, u = rnd(H * D).to(gpu), rnd(H, D).to(gpu)
+        call = lambda r, k, v, lw, s, o, **kw: ops.wkv_scan(r, k, v, lw, w0, u, s, o, H=H, D=D, **kw)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)
+    first = [sum(lens[:i]) for i in range(R)]
+    state = rnd(R, H, D, Dv).to(gpu)
+    whole, out = state.clone(), torch.full((T, H * Dv), float("nan"), device=gpu)
+    call(*[t.to(gpu) for t in rows], whole, out, q_start=i32(first), q_len=i32(lens), state_slot=i32(list(range(R))))
+    cut, parts = state.clone(), torch.full((T, H * Dv), float("nan"), device=gpu)
+    for r, n in enumerate(lens):
+        for at in range(first[r], first[r] + n, 20):
+            m = min(20, first[r] + n - at)
+            piece = torch.empty(m, H * Dv, device=gpu)
+            call(*[t[at:at + m].to(gpu) for t in rows], cut, piece, q_start=i32([0]), q_len=i32([m]), state_slot=i32([r]))
+            parts[at:at + m] = piece
+    assert torch.equal(out, parts) and torch.equal(whole, cut)
+
+
 @pytest.mark.parametrize("D, Dv", [(16, 16), (30, 50), (32, 64), (64, 128), (96, 20), (130, 130), (256, 24)])
 def test_single_tokens_of_a_scan_have_the_bits_of_a_run(gpu, D, Dv):
     """A request with one token takes no stop in LDS; portions that end inside the tokens staged at a time stage only their own:

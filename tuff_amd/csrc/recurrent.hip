@@ -462,6 +462,8 @@ struct ScanArgs {
 constexpr int SCAN_CH = 8;          // tokens staged at a time (sixteen: 5 % faster for one long request, but 12 KB of LDS a
                                     // wave, and 64 single tokens of 32 heads 43 -> 55 us)
 
+constexpr int SCAN_CH_WAVES = 16;   // where four waves stage for each other: a lane one group of four channels and one value
+
 // The sum over the SPLIT neighbouring lanes that share a value channel, the same in all of them: exchanges
 // inside a quad (lane ^ 1, then lane ^ 2) and, for 16, rotations by 4 and by 8 within the row of 16 lanes.
 template <int CTRL>
@@ -501,25 +503,30 @@ __device__ __forceinline__ float group_sum(float v) {
 // gate), 2,366 -> 1,053 us (delta rule); without it 1,365 and 2,580.  Four waves a SIMD up to 64 key channels, three up to
 // 128 (with four the registers spill: 64 single tokens, 16 heads of 128, 92 us instead of 80), two beyond.
 // SINGLES: a step in which no request need have more than one token.
-template <typename TA, typename T, int NI16, int SPLIT, bool WHOLE, bool SINGLES, bool DELTA, bool FORGET = false, bool SSD = false>
-__global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_kernel(ScanArgs p) {
+// NW: waves a workgroup.  A lone wave issues an instruction in five cycles, and 22 of the 50 it spends on a token only bring rows
+// into LDS.  Four waves of one head bring them for each other, sixteen tokens at a time into one of two places: forget gate, 16
+// heads, one request of 2,048 tokens, 64 key and 128 value channels 218 -> 181 us, 128 and 128 380 -> 297; 64 requests of 200
+// 454 -> 348 and 888 -> 754 (two waves, or eight tokens: slower for one request).
+template <typename TA, typename T, int NI16, int SPLIT, bool WHOLE, bool SINGLES, int NW, bool DELTA, bool FORGET = false, bool SSD = false>
+__global__ __launch_bounds__(NW * WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_kernel(ScanArgs p) {
     constexpr int RP = NI16 * 4;                       // rows of the state's column a lane keeps
     constexpr int DP = RP * SPLIT;                     // key channels, padded
-    constexpr int SCAN_COLS = WAVE / SPLIT;            // value channels a wave
-    constexpr int CH = SCAN_CH;
+    constexpr int NT = NW * WAVE;
+    constexpr int SCAN_COLS = NT / SPLIT;              // value channels a workgroup
+    constexpr int CH = NW == 1 ? SCAN_CH : SCAN_CH_WAVES, BUFS = NW == 1 ? 1 : 2;
     constexpr int QUADS = DP / 4;                      // groups of four key channels a token
-    constexpr int PER = (CH * QUADS + WAVE - 1) / WAVE;                  // such groups a lane stages
-    constexpr int PER_V = (CH * SCAN_COLS + WAVE - 1) / WAVE;            // and values
+    constexpr int PER = (CH * QUADS + NT - 1) / NT;                      // such groups a lane stages
+    constexpr int PER_V = (CH * SCAN_COLS + NT - 1) / NT;                // and values
     typedef TA four __attribute__((ext_vector_type(4)));
-    __shared__ __attribute__((aligned(16))) float sa[CH][DP];
-    __shared__ __attribute__((aligned(16))) float sk[CH][DP];
-    __shared__ __attribute__((aligned(16))) float sw[SSD ? 1 : CH][SSD ? 4 : DP];
-    __shared__ __attribute__((aligned(16))) float sv[SCAN_COLS][CH];
+    __shared__ __attribute__((aligned(16))) float sa_[BUFS][CH][DP];
+    __shared__ __attribute__((aligned(16))) float sk_[BUFS][CH][DP];
+    __shared__ __attribute__((aligned(16))) float sw_[BUFS][SSD ? 1 : CH][SSD ? 4 : DP];
+    __shared__ __attribute__((aligned(16))) float sv_[BUFS][SCAN_COLS][CH];
     // The blocks of one (request, head), which all read its rows of a, k and decay, run one after the other on one XCD
     // (workgroups go round the eight XCDs, each with an L2 of its own): of the pairs that fill rounds of eight, pair i on XCD
     // i mod 8; the rest in their order.
     int r = blockIdx.x, head = blockIdx.y, zb = blockIdx.z;
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid % WAVE;
     if (p.by_xcd) {
         const unsigned Z = gridDim.z, id = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
         const unsigned rounds = gridDim.x * gridDim.y / 8 * 8 * Z;
@@ -533,7 +540,7 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
     const int D = p.D, Dv = p.Dv, H = p.H, Ha = p.Ha;
     const int ha = head / (H / Ha);
     const int part = lane % SPLIT;
-    const int j = zb * SCAN_COLS + lane / SPLIT;
+    const int j = zb * SCAN_COLS + tid / SPLIT;
     const bool jv = j < Dv;
     const int row0 = part * RP;
     float* S = p.state + (((long long)slot * H + head) * D) * Dv + j;
@@ -558,7 +565,7 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
     auto fetch = [&](int c0) {                         // c0: the first token, counted from the request's first of the step
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            const int id = lane + e * WAVE;
+            const int id = tid + e * NT;
             const long long t = t0 + min(c0 + id / QUADS, n - 1);
             const int i = id % QUADS * 4;
             const TA *ra = pa + t * p.lda + (long long)ha * D, *rk = pk + t * p.lda + (long long)ha * D;
@@ -580,7 +587,7 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
         }
 #pragma unroll
         for (int e = 0; e < PER_V; ++e) {
-            const int id = lane + e * WAVE;
+            const int id = tid + e * NT;
             const long long t = t0 + min(c0 + id / SCAN_COLS, n - 1);
             fv[e] = pv[t * p.ldv + (long long)head * Dv + min(zb * SCAN_COLS + id % SCAN_COLS, Dv - 1)];
         }
@@ -589,10 +596,14 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
         if (SSD) fd = p.decay[t * H + head];
     };
     // The fetched values to LDS in float32, key channels beyond D as zero (tokens beyond the last are staged and never read).
+    int buf = 0;
     auto stage = [&]() {
+        auto &sa = sa_[buf], &sk = sk_[buf];
+        auto& sw = sw_[buf];
+        auto& sv = sv_[buf];
 #pragma unroll
         for (int e = 0; e < PER; ++e) {
-            const int id = lane + e * WAVE, tt = id / QUADS, i = id % QUADS * 4;
+            const int id = tid + e * NT, tt = id / QUADS, i = id % QUADS * 4;
             const float step = SSD ? __shfl(fb, tt, WAVE) : 1.f;
             f32x4 a, k, w;
 #pragma unroll
@@ -602,7 +613,7 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
                 k[u] = ok ? (FORGET ? 1.0f - fw[e][u] : SSD ? step * to_f32((TA)fk[e][u]) : to_f32((TA)fk[e][u])) : 0.f;
                 w[u] = ok && !SSD ? fw[e][u] : 0.f;
             }
-            if (CH * QUADS % WAVE == 0 || id < CH * QUADS) {
+            if (CH * QUADS % NT == 0 || id < CH * QUADS) {
                 *(f32x4*)&sa[tt][i] = a;
                 *(f32x4*)&sk[tt][i] = k;
                 if (!SSD) *(f32x4*)&sw[tt][i] = w;
@@ -610,13 +621,15 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
         }
 #pragma unroll
         for (int e = 0; e < PER_V; ++e) {
-            const int id = lane + e * WAVE;
-            if (CH * SCAN_COLS % WAVE == 0 || id < CH * SCAN_COLS) sv[id % SCAN_COLS][id / SCAN_COLS] = to_f32(fv[e]);
+            const int id = tid + e * NT;
+            if (CH * SCAN_COLS % NT == 0 || id < CH * SCAN_COLS) sv[id % SCAN_COLS][id / SCAN_COLS] = to_f32(fv[e]);
         }
     };
     // What a token brings to this lane's rows, out of LDS.
     struct Rows { f32x4 w[NI16], k[NI16], q[NI16]; };
     auto rows_of = [&](int tt, Rows& m) {
+        const auto &sa = sa_[buf], &sk = sk_[buf];
+        const auto& sw = sw_[buf];
 #pragma unroll
         for (int g4 = 0; g4 < NI16; ++g4) {
             m.w[g4] = SSD ? f32x4{0.f, 0.f, 0.f, 0.f} : *(const f32x4*)&sw[tt][row0 + g4 * 4];
@@ -748,9 +761,11 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
         // between the writes above and the reads below, only the compiler must keep their order.  (A
         // __syncthreads() would also wait for the loads of the next eight tokens, which are meant to be under
         // way while these are computed.)
-        __builtin_amdgcn_wave_barrier();
+        // (Several waves: one barrier; the other tokens' places are free, since who has come this far has read them.)
+        if (NW == 1) __builtin_amdgcn_wave_barrier();
+        else lds_barrier();
 #pragma unroll
-        for (int t4 = 0; t4 < CH; t4 += 4) *(f32x4*)&v[t4] = *(const f32x4*)&sv[lane / SPLIT][t4];
+        for (int t4 = 0; t4 < CH; t4 += 4) *(f32x4*)&v[t4] = *(const f32x4*)&sv_[buf][tid / SPLIT][t4];
         if (count == CH) {
             // CH whole tokens, one block of code without a test: the rows of AHEAD tokens are asked for before they are
             // needed, and the sums over the lanes that share a channel go side by side.
@@ -776,7 +791,8 @@ __global__ __launch_bounds__(WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void scan_
                     if (jv) leave(c0 + tt, ot);
                 }
         }
-        __builtin_amdgcn_wave_barrier();               // the reads stay before the next tokens' writes
+        if (NW == 1) __builtin_amdgcn_wave_barrier();  // the reads stay before the next tokens' writes
+        else buf ^= 1;
     }
     if (jv && n % CH == 0) {
 #pragma unroll
@@ -823,17 +839,25 @@ int launch_scan(ScanArgs p, int n_tokens, int R, hipStream_t stream) {
     const bool narrow = p.D <= 32;                      // four lanes a value channel; else sixteen
     const int split = narrow ? 4 : 16;
     const int ni = narrow ? (p.D + 15) / 16 : (p.D + 63) / 64;
-    dim3 grid(R, p.H, ceil_div(p.Dv, WAVE / split)), block(WAVE);
+    const bool singles = n_tokens <= R;
+    // Four waves a workgroup: up to 192 key channels, up to 64 only the forget gate and the state-space rule (2,048 tokens, 16 heads
+    // of 64: wkv 232 us in single waves, 249 in fours, the delta rule 306 and 310); beyond 192 a SIMD's registers hold too few
+    // waves (wkv, 4 heads of 256: 670, 831).  Runs long enough that the first rows' way into LDS counts little, and values
+    // enough for the waves.
+    auto shared_rows = [](int n16) { return n16 == 1 ? FORGET || SSD : n16 <= 3; };
+    const int waves = !singles && !narrow && shared_rows(ni) && (long long)n_tokens >= 32ll * R && p.Dv >= 32 ? 4 : 1;
+    dim3 grid(R, p.H, ceil_div(p.Dv, waves * WAVE / split)), block(waves * WAVE);
     if (grid.z > 65535) return -2;
     p.by_xcd = (long long)R * p.H * grid.z < (1ll << 32);       // the workgroups' numbers have 32 bits there
     // four key channels a load, where they lie so that one load can fetch them
     auto in_fours = [](const void* q, size_t width) { return (uintptr_t)q % (4 * width) == 0; };
     const bool whole = p.D % 4 == 0 && p.lda % 4 == 0 && in_fours(p.a, sizeof(TA)) && (FORGET || in_fours(p.k, sizeof(TA))) &&
                        (SSD || in_fours(p.decay, 4));
-    const bool singles = n_tokens <= R;
-#define GO(NI, SPLIT, WHOLE, SINGLES) hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, WHOLE, SINGLES, DELTA, FORGET, SSD>), grid, block, 0, stream, p)
-#define SCAN(NI, SPLIT) do { if (whole && singles) GO(NI, SPLIT, true, true); else if (whole) GO(NI, SPLIT, true, false); \
-                             else if (singles) GO(NI, SPLIT, false, true); else GO(NI, SPLIT, false, false); } while (0)
+#define GO(NI, SPLIT, WHOLE, SINGLES, NW) hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, WHOLE, SINGLES, NW, DELTA, FORGET, SSD>), grid, block, 0, stream, p)
+#define SCAN(NI, SPLIT) do { constexpr int MANY = SPLIT == 16 && (NI == 1 ? FORGET || SSD : NI <= 3) ? 4 : 1; \
+                             if (whole && singles) GO(NI, SPLIT, true, true, 1); else if (singles) GO(NI, SPLIT, false, true, 1); \
+                             else if (whole && waves == 1) GO(NI, SPLIT, true, false, 1); else if (whole) GO(NI, SPLIT, true, false, MANY); \
+                             else if (waves == 1) GO(NI, SPLIT, false, false, 1); else GO(NI, SPLIT, false, false, MANY); } while (0)
     if (narrow) { if (ni <= 1) SCAN(1, 4); else SCAN(2, 4); }
     else if (ni <= 1) SCAN(1, 16);
     else if (ni <= 2) SCAN(2, 16);
