@@ -282,6 +282,26 @@ def test_gemm_bf16_narrow_outputs_of_17_to_21_rows(gpu, M, N, K):
     assert ((ss.double().sum(0)[:M] - want).abs() <= N * 2.0 ** -24 * want).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 2048, 8192), (40, 200, 2304), (64, 2048, 2048), (80, 2048, 8192), (33, 2056, 16512)])
+def test_emitting_sum_of_slices_off_a_16_byte_border(gpu, M, N, K):
+    """The kernel that adds slices of K and leaves the next norm's operand, fewer and more than sixteen slices: the same bits
+    whether the residual stream, the norm's weights and the operand lie on borders of 16 bytes or not."""
+    from tuff_amd.csrc import ops
+    x, w = _r(M, K, seed=1, dtype=torch.bfloat16).to(gpu), ops.tile_weight(_r(N, K, seed=2, dtype=torch.bfloat16).to(gpu))
+    res0, nw0 = _r(M, N, seed=3).to(gpu), _r(N, seed=4).to(gpu)
+    outs = []
+    for off in (0, 1):
+        at = lambda n, dtype: torch.empty(n + 1, dtype=dtype, device=gpu)[off:off + n]
+        res, nw, xw = at(M * N, torch.float32).view(M, N), at(N, torch.float32), at(M * N, torch.bfloat16).view(M, N)
+        res.copy_(res0), nw.copy_(nw0)
+        ss = torch.zeros(ops.gemm_emit_layout(M, N, K), device=gpu)
+        ops.gemm_accum_emit(x, w, res, nw, xw, ss)
+        outs.append((res.clone(), xw.clone(), ss))
+    assert all(torch.equal(a, b) for a, b in zip(*outs))
+    a, b = x.double(), _r(N, K, seed=2, dtype=torch.bfloat16).to(gpu).double()
+    assert ((outs[0][0].double() - (res0.double() + a @ b.T)).abs() <= K * 2.0 ** -23 * (a.abs() @ b.abs().T) + 1e-6).all()
+
+
 @pytest.mark.parametrize("M,d,K1,N2", [(1, 64, 192, 512), (8, 2048, 8192, 6144), (16, 240, 328, 777 * 2), (5, 96, 96, 40),
                                        (17, 96, 96, 40), (32, 2048, 8192, 6144), (24, 240, 328, 777 * 2), (40, 2048, 8192, 6144), (64, 240, 328, 777 * 2), (33, 64, 192, 512),
                                        (64, 2048, 2048, 65536),
