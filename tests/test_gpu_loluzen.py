@@ -470,6 +470,58 @@ def test_scan_gives_the_same_bits_for_any_company_and_alignment(gpu, D):
                 assert torch.equal(state[i], state0[i])
 
 
+@pytest.mark.parametrize("C, K, bias, act", [(3072, 4, False, None), (1028, 3, True, "silu"), (516, 2, True, None), (8, 4, False, "silu")])
+@pytest.mark.parametrize("dtype, out", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.bfloat16), (torch.float32, torch.float32)])
+def test_convolution_of_four_channels_a_thread_has_the_bits_of_one(gpu, C, K, bias, act, dtype, out):
+    """Few tokens and many, requests that begin inside a run of four, portions shorter than the taps; rows off a border of four
+    elements take the kernel of one channel a thread."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(C + K)
+    for lens in ([1], [1, 2, 3, 1], [40, 1, 2, 700, 3, 1, 601]):
+        T, R = sum(lens), len(lens)
+        x, taps, state = (torch.randn(*s, generator=gen) for s in ((T, C), (C, K), (R, K - 1, C)))
+        b = torch.randn(C, generator=gen).to(gpu) if bias else None
+        i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)
+        got = []
+        for ld in (C, C + 1):
+            rows = torch.zeros(T, ld, dtype=dtype, device=gpu)
+            rows[:, :C] = x.to(gpu)
+            st, y = state.to(gpu), torch.full((T, C), float("nan"), dtype=out, device=gpu)
+            more = {} if b is None else {"bias": b}
+            ops.conv_act(rows[:, :C], taps.to(gpu), st, y, req_of_token=i32(sum([[r] * n for r, n in enumerate(lens)], [])),
+                         q_start=i32([sum(lens[:r]) for r in range(R)]), q_len=i32(lens), state_slot=i32(list(range(R))), activation=act, **more)
+            got.append((y, st))
+        assert all(torch.equal(a, b_) for a, b_ in zip(*got)), lens
+
+
+@pytest.mark.parametrize("T", [1, 17, 300])
+@pytest.mark.parametrize("H, G, rot, norm, ps", [(32, 8, 32, True, 16), (3, 3, 64, False, 48), (5, 1, 20, True, 32), (4, 2, 0, True, 16), (4, 4, 0, False, 64)])
+def test_heads_of_64_turned_in_pairs_or_not_at_all(gpu, T, H, G, rot, norm, ps):
+    """The kernel of sixteen lanes a head against the one of a wave a head, which rows off a 16-byte border take: the norm's sum in
+    another order, so a last bit of bfloat16 at most; values are the same."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(T + H)
+    width = (H + 2 * G) * 64
+    qkv = torch.randn(T * width, generator=gen).bfloat16().to(gpu)
+    w = [(torch.rand(64, generator=gen) + 0.5).to(gpu) for _ in "qk"] if norm else [None, None]
+    inv = (10000.0 ** (-torch.arange(rot // 2) * 2 / rot)).float().to(gpu) if rot else None
+    pos = torch.arange(5, 5 + T, dtype=torch.int32, device=gpu)
+    got = []
+    for off in (0, 1):
+        at = torch.empty(T * width + 1, dtype=torch.bfloat16, device=gpu)[off:off + T * width]
+        at.copy_(qkv)
+        q = torch.zeros(T, H * 64, dtype=torch.bfloat16, device=gpu)
+        P = -(-(T + 5) // ps) + 1
+        k, v = torch.zeros(P, G, ps, 64, dtype=torch.bfloat16, device=gpu), torch.zeros(P, G, 64, ps, dtype=torch.bfloat16, device=gpu)
+        ops.qkv_post(at.view(T, width), q, H=H, Hkv=G, hd=64, positions=pos, eps=1e-5, q_norm_w=w[0], k_norm_w=w[1], inv_freq=inv,
+                     rotary_dim=rot, interleaved=True, k_cache=k, v_cache=v, slot_mapping=pos + ps, page_size=ps)
+        got.append((q, k, v))
+    for a, b in zip(got[0][:2], got[1][:2]):
+        # the larger of two turned numbers moves by its own last bit, the smaller by that much times the other's cosine or sine
+        assert ((a.float() - b.float()).abs() <= 2.0 ** -7 * a.float().abs() + 2.0 ** -20).all()
+    assert torch.equal(got[0][2], got[1][2])
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("kind, H, D, Dv", [("forget", 3, 40, 33), ("forget", 2, 64, 128), ("forget", 5, 65, 32), ("ssd", 4, 64, 40),
                                             ("ssd", 2, 128, 64), ("delta", 3, 100, 130), ("delta", 2, 192, 48), ("wkv", 3, 72, 72),

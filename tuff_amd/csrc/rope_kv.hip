@@ -148,12 +148,12 @@ __global__ __launch_bounds__(POST_WAVES * WAVE) void qkv_post_kernel(
     }
 }
 
-// The same for heads of 64 channels with the half-split rotation over the whole head, laid out for
-// many tokens.  Two kinds of workgroups in one launch:
+// The same for heads of 64 channels, laid out for many tokens: with the half-split rotation over the whole head, with
+// neighbouring channels turned in pairs (of the first rotary_dim, a multiple of four, channels), or with no rotation.  Two kinds of workgroups in one launch:
 //  * q and k: sixteen lanes take one token and walk a share of its heads; lane l holds the channels
 //    4l .. 4l+3 of a head (one 8-byte load for bfloat16), the norm's sum of squares is a butterfly over
-//    the sixteen lanes, the rotation's partner channel j +- 32 sits in lane l ^ 8, and the token's
-//    cosines and sines are computed once for all its heads.
+//    the sixteen lanes, the rotation's partner channel j +- 32 sits in lane l ^ 8 (a pair's in the same lane), and the
+//    token's cosines and sines are computed once for all its heads.
 //  * v: a workgroup takes sixteen consecutive tokens and one kv head, brings the rows into LDS and
 //    writes, for every channel, the sixteen positions in one run where the tokens fill a run of sixteen
 //    slots from a multiple of sixteen (the usual case in a prompt), else one by one: V is kept with a
@@ -162,13 +162,15 @@ __global__ __launch_bounds__(POST_WAVES * WAVE) void qkv_post_kernel(
 constexpr int P64_GROUPS = 16;                       // sixteen-lane groups a workgroup
 constexpr int P64_TOKENS = 16;                       // tokens a v workgroup
 
-template <typename T, typename TW>
+enum { TURN_NONE, TURN_HALVES, TURN_PAIRS };
+
+template <typename T, typename TW, int TURN>
 __global__ __launch_bounds__(256) void qkv_post64_kernel(
     const T* __restrict__ qkv, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache,
     const TW* __restrict__ q_norm_w, const TW* __restrict__ k_norm_w, float eps, const float* __restrict__ inv_freq,
     const int* __restrict__ positions, const int* __restrict__ slot_mapping,
     int n_tokens, int H, int Hkv, int page_size, int shares, int qk_blocks,
-    const float* __restrict__ angles, int n_angles) {
+    const float* __restrict__ angles, int n_angles, int rotary_dim) {
     constexpr int HD = 64;
     const int tid = threadIdx.x;
     const int row_width = (H + 2 * Hkv) * HD;
@@ -180,20 +182,23 @@ __global__ __launch_bounds__(256) void qkv_post64_kernel(
         const int n_heads = k_cache ? H + Hkv : H;
         const int per = (n_heads + shares - 1) / shares;
         const int head_begin = share * per, head_end = min(n_heads, head_begin + per);
-        const int p = positions[t];
+        const int p = TURN == TURN_NONE ? 0 : positions[t];
         const float pos = (float)p;
-        const bool first = l < 8;
+        const bool first = l < 8, turns = TURN == TURN_HALVES || (TURN == TURN_PAIRS && 4 * l < rotary_dim);
+        const int half = TURN == TURN_HALVES ? 32 : rotary_dim / 2;
         float rc[4], rs[4], wq[4], wk[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const int f = (4 * l + e) & 31;
-            if (p < n_angles) {                          // from the table: the same bits, without the two functions
-                rc[e] = angles[((long long)p * 2) * 32 + f];
-                rs[e] = angles[((long long)p * 2 + 1) * 32 + f];
-            } else {
-                const float a = pos * inv_freq[f];
-                rc[e] = cosf(a);
-                rs[e] = sinf(a);
+            const int f = TURN == TURN_HALVES ? (4 * l + e) & 31 : 2 * l + e / 2;
+            if (turns) {
+                if (p < n_angles) {                      // from the table: the same bits, without the two functions
+                    rc[e] = angles[((long long)p * 2) * half + f];
+                    rs[e] = angles[((long long)p * 2 + 1) * half + f];
+                } else {
+                    const float a = pos * inv_freq[f];
+                    rc[e] = cosf(a);
+                    rs[e] = sinf(a);
+                }
             }
             wq[e] = q_norm_w ? to_f32(q_norm_w[4 * l + e]) : 1.f;
             wk[e] = k_norm_w ? to_f32(k_norm_w[4 * l + e]) : 1.f;
@@ -218,11 +223,20 @@ __global__ __launch_bounds__(256) void qkv_post64_kernel(
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = v[e] * inv * (is_q ? wq[e] : wk[e]);
             }
+            if (TURN == TURN_HALVES) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float other = __shfl_xor(v[e], 8, WAVE);
-                const float x0 = first ? v[e] : other, x1 = first ? other : v[e];
-                v[e] = first ? (x0 * rc[e] - x1 * rs[e]) : (x0 * rs[e] + x1 * rc[e]);
+                for (int e = 0; e < 4; ++e) {
+                    const float other = __shfl_xor(v[e], 8, WAVE);
+                    const float x0 = first ? v[e] : other, x1 = first ? other : v[e];
+                    v[e] = first ? (x0 * rc[e] - x1 * rs[e]) : (x0 * rs[e] + x1 * rc[e]);
+                }
+            } else if (turns) {
+#pragma unroll
+                for (int e = 0; e < 4; e += 2) {
+                    const float x0 = v[e], x1 = v[e + 1];
+                    v[e] = x0 * rc[e] - x1 * rs[e];
+                    v[e + 1] = x0 * rs[e] + x1 * rc[e];
+                }
             }
             if (is_q) store4(q_out + ((long long)t * H + head) * HD + 4 * l, v);
             else if (slot >= 0) {
@@ -447,7 +461,12 @@ TUFF_EXPORT int tuff_qkv_post(const void* qkv, void* q_out, void* k_out, void* k
     // width behind the keys: then nothing is written to the cache here, only q_out and k_out)
     if (row_stride > 0 && (k_cache || row_stride < (H + Hkv) * hd)) return -2;
     if (!angles || !inv_freq) n_angles = 0;              // [n_angles][2][rotary_dim / 2] as tuff_rope_table makes it
-    if (hd == 64 && inv_freq && rotary_dim == 64 && !interleaved && !k_out && page_size % 16 == 0 && row_stride <= 0) {
+    const bool turned = inv_freq && rotary_dim > 0;
+    const int turn = !turned ? TURN_NONE : rotary_dim == 64 && !interleaved ? TURN_HALVES : interleaved && rotary_dim % 4 == 0 ? TURN_PAIRS : -1;
+    // (the other two turns in bfloat16, on borders of 16 bytes: 2,048 tokens, 32 heads and 8 kv heads, 32 channels turned in pairs
+    // 33.6 us in the kernel above, 11.2 in this, no turn 20.9 and 9.7, up to 300 tokens the same)
+    if (hd == 64 && turn >= 0 && !k_out && page_size % 16 == 0 && row_stride <= 0 &&
+        (turn == TURN_HALVES || (dt == DT_BF16 && ((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0))) {
         // shares of a token's heads: enough sixteen-lane groups for the chip, whole heads each
         const int n_heads = k_cache ? H + Hkv : H;
         int shares = 1;
@@ -456,14 +475,17 @@ TUFF_EXPORT int tuff_qkv_post(const void* qkv, void* q_out, void* k_out, void* k
         shares = min(shares, n_heads);
         const int qk_blocks = (int)ceil_div_ll((long long)n_tokens * shares, P64_GROUPS);
         const int v_blocks = k_cache ? ceil_div(n_tokens, P64_TOKENS) * Hkv : 0;
-#define LAUNCH64(T, TW) hipLaunchKernelGGL((qkv_post64_kernel<T, TW>), dim3(qk_blocks + v_blocks), dim3(256), 0, stream, \
+#define GO64(T, TW, TURN) hipLaunchKernelGGL((qkv_post64_kernel<T, TW, TURN>), dim3(qk_blocks + v_blocks), dim3(256), 0, stream, \
         (const T*)qkv, (T*)q_out, (T*)k_cache, (T*)v_cache, (const TW*)q_norm_w, (const TW*)k_norm_w, eps, inv_freq, \
-        positions, slot_mapping, n_tokens, H, Hkv, page_size, shares, qk_blocks, angles, n_angles)
+        positions, slot_mapping, n_tokens, H, Hkv, page_size, shares, qk_blocks, angles, n_angles, rotary_dim)
+#define LAUNCH64(T, TW) do { if (turn == TURN_HALVES) GO64(T, TW, TURN_HALVES); else if (turn == TURN_PAIRS) GO64(T, TW, TURN_PAIRS); \
+                             else GO64(T, TW, TURN_NONE); } while (0)
         if (dt == DT_F32 && norm_dt == DT_F32) LAUNCH64(float, float);
         else if (dt == DT_F32) LAUNCH64(float, bf16_t);
         else if (norm_dt == DT_F32) LAUNCH64(bf16_t, float);
         else LAUNCH64(bf16_t, bf16_t);
 #undef LAUNCH64
+#undef GO64
         return launch_status();
     }
     const int heads = k_cache ? H + 2 * Hkv : (k_out ? H + Hkv : H);
