@@ -200,13 +200,25 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
     auto swizzle = [](int j) { return P >= 16 ? j % 16 : (j * P / 16) % P; };
     const int vpiece = (tid % 16) ^ (tid / 16);           // (the same for all of the thread's value pieces)
     f32x4 kr[KP], vr[KP];
+    // Lane i knows where granule (sixteen keys) i of sixteen tiles lies, four a tile; keys nobody sees lie on a seen one's page.
+    // Worked out once in sixteen tiles, the page numbers asked for sixteen tiles ahead: from the table in every tile they were
+    // a trip to memory that the tile waited for.
+    const int first = lo_first / 64 * 64;
+    auto key_of_granule = [&](int batch) { return (unsigned)max(lo_first, min(first + 1024 * batch + 16 * lane, pos_last)); };
+    auto pages_of = [&](int batch) { return table[key_of_granule(batch) / (unsigned)page_size]; };
+    int pages = pages_of(0), pages_next = pages_of(1), offs = key_of_granule(0) / 16 * 16 % (unsigned)page_size;
     auto load_tile = [&](int t0) {
-        int page[4], off[4];                              // of the tile's groups of sixteen keys; keys nobody sees read a seen one's page
+        const int tile = (t0 - first) / 64;
+        if (tile % 16 == 0 && tile > 0) {
+            pages = pages_next;
+            offs = key_of_granule(tile / 16) / 16 * 16 % (unsigned)page_size;
+            pages_next = pages_of(tile / 16 + 1);
+        }
+        int page[4], off[4];                              // of the tile's groups of sixteen keys
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int key = max(lo_first, min(t0 + 16 * j, pos_last));
-            page[j] = table[key / page_size];
-            off[j] = (key / 16 * 16) % page_size;
+            page[j] = __builtin_amdgcn_readlane(pages, tile % 16 * 4 + j);
+            off[j] = __builtin_amdgcn_readlane(offs, tile % 16 * 4 + j);
         }
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
@@ -243,7 +255,6 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
 #pragma unroll
     for (int c = 0; c < 4; ++c) { m[c] = -INFINITY; l[c] = 0.f; }
 
-    const int first = lo_first / 64 * 64;
     load_tile(first);
     for (int t0 = first; t0 <= pos_last; t0 += 64) {
         lds_barrier();                                    // the last tile's keys, values and weights are used up

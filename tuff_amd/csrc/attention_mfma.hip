@@ -156,10 +156,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
                     ss = fmaf(v[1], v[1], ss);
                     ss = fmaf(v[2], v[2], ss);
                     ss = fmaf(v[3], v[3], ss);
-                    ss += __shfl_xor(ss, 8, WAVE);
-                    ss += __shfl_xor(ss, 4, WAVE);
-                    ss += __shfl_xor(ss, 2, WAVE);
-                    ss += __shfl_xor(ss, 1, WAVE);
+                    ss = row_sum_down(ss);
                     if (fq.k_norm_w != nullptr) {
                         const float inv = 1.0f / sqrtf(ss / 64.0f + fq.eps);
 #pragma unroll
@@ -171,7 +168,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
                     for (int e = 0; e < 4; ++e) {
                         float rc, rs;
                         angle(fq, pos0, (4 * l + e) & 31, rc, rs);
-                        const float other = __shfl_xor(v[e], 8, WAVE);
+                        const float other = lane_xor8(v[e]);
                         const float x0 = first ? v[e] : other, x1 = first ? other : v[e];
                         o4[e] = (bf16_t)(first ? (x0 * rc - x1 * rs) : (x0 * rs + x1 * rc));
                     }
@@ -332,8 +329,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
                 p[0][h] = a; p[1][h] = b;
             }
             float s0 = p[0][0] + p[1][0], s1 = p[0][1] + p[1][1];
-            s0 += __shfl_xor(s0, 32, WAVE); s1 += __shfl_xor(s1, 32, WAVE);
-            s0 += __shfl_xor(s0, 16, WAVE); s1 += __shfl_xor(s1, 16, WAVE);
+            s0 = butterfly_sum<16>(butterfly_sum<32>(s0)); s1 = butterfly_sum<16>(butterfly_sum<32>(s1));
             const float ss = s0 + s1;
             if (fq.q_norm_w != nullptr) {
                 const float inv = 1.0f / sqrtf(ss / 64.0f + fq.eps);
@@ -410,8 +406,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
                     v[kb * 4 + e] = x;
                     mx = fmaxf(mx, x);
                 }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+            mx = butterfly_max<32>(butterfly_max<16>(mx));
             const float m_new = fmaxf(m_run[nb], mx);
             const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
             corr[nb] = __expf(m_run[nb] - m_safe);          // 0 while nothing was seen yet
@@ -458,8 +453,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     auto unit_sums = [&]() {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-            l_run[nb] += __shfl_xor(l_run[nb], 16, WAVE);
-            l_run[nb] += __shfl_xor(l_run[nb], 32, WAVE);
+            l_run[nb] = butterfly_sum<32>(butterfly_sum<16>(l_run[nb]));
         }
     };
 

@@ -61,18 +61,6 @@ __device__ __forceinline__ int k_row_of_key(int key) {
     return sub * 32 + kb * 16 + h * 8 + q * 4 + m;
 }
 
-// The largest value of the lanes with the same lane % 16, in all of them.  Halves and rows of sixteen lanes change places in
-// registers: through LDS (two shuffles, one after the other, a column block) the wait for them was a fifth of a step.
-__device__ __forceinline__ float max_over_groups(float v) {
-#ifdef __HIP_DEVICE_COMPILE__
-    auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1]));
-    auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(rows[0]), __uint_as_float(rows[1]));
-#endif
-    return v;
-}
-
 // What is taken off the scaled scores: nothing, a slope's part, the logarithmic penalty, both, or what the pointers say when
 // the kernel runs (heads of more than 64 channels in the wide form; narrower ones have a step of which the branches are a part).
 enum { NO_BIAS = 0, SLOPES = 1, LOG_DIST = 2, ANY_BIAS = 4 };
@@ -411,7 +399,7 @@ __global__ __launch_bounds__(NW * WAVE, groups_a_cu(HDP, VDP, MAPS, EX, VHS)) vo
                         ok[sub][kb * 4 + e] = v;
                         mx = fmaxf(mx, v ? sc[sub].v[kb][nb][e] : -INFINITY);
                     }
-            mx = max_over_groups(mx);
+            mx = butterfly_max<16>(butterfly_max<32>(mx));
             // The reference point of the exponents moves only when a score exceeds it by more than
             // 2^SLACK: until then the weights may reach 2^SLACK instead of 1, which float32 sums and
             // bfloat16 weights hold as well, and the output so far need not be rescaled.
@@ -522,8 +510,7 @@ __global__ __launch_bounds__(NW * WAVE, groups_a_cu(HDP, VDP, MAPS, EX, VHS)) vo
                 o[0][db][0][e] = v;
                 ss = fmaf(v, v, ss);
             }
-        ss += __shfl_xor(ss, 16, WAVE);
-        ss += __shfl_xor(ss, 32, WAVE);
+        ss = butterfly_sum<32>(butterfly_sum<16>(ss));
         if (qrow[0] < 0) return;
         const float by = wide.coef / sqrtf(ss / (float)vd + wide.eps);
 #pragma unroll

@@ -132,8 +132,7 @@ __global__ __launch_bounds__(NT) void single_part_kernel(const bf16_t* __restric
                 mx = fmaxf(mx, v[h][e]);
             }
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+        mx = butterfly_max<32>(butterfly_max<16>(mx));
         if (g == 0) red[wave][n16] = mx;
         __syncthreads();
         // (a live block holds a visible key, so the maximum is finite)
@@ -181,8 +180,7 @@ __global__ __launch_bounds__(NT) void single_part_kernel(const bf16_t* __restric
         }
     }
 
-    l_run += __shfl_xor(l_run, 16, WAVE);
-    l_run += __shfl_xor(l_run, 32, WAVE);
+    l_run = butterfly_sum<32>(butterfly_sum<16>(l_run));
     __syncthreads();
     if (g == 0) red[wave][n16] = l_run;
     __syncthreads();

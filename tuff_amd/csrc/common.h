@@ -24,17 +24,54 @@ template <typename T> __device__ __forceinline__ T from_f32(float v);
 template <> __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) { return (bf16_t)v; }
 
-// Sum over the 64 lanes of a wave; every lane receives the total.  The order of
+// For a step of a butterfly over the wave, 32 first: this lane's value and that of lane ^ M, in either order.  Through registers: a
+// shuffle goes through LDS, and the steps wait for one another (six of them some 700 cycles, this way 100).  M = 4 takes
+// lane + 4 of the sixteen, which after the step of 8 holds what lane ^ 4 holds.
+struct LanePair { float a, b; };
+template <int M>
+__device__ __forceinline__ LanePair butterfly_pair(float v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const unsigned u = __float_as_uint(v);
+    if constexpr (M == 32) {                               // the halves of two copies change places: (low, low) and (high, high)
+        const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        return {__uint_as_float(p[0]), __uint_as_float(p[1])};
+    } else if constexpr (M == 16) {                        // and rows of sixteen
+        const auto p = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        return {__uint_as_float(p[0]), __uint_as_float(p[1])};
+    } else {
+        constexpr int CTRL = M == 8 ? 0x128 : M == 4 ? 0x124 : M == 2 ? 0x4E : 0xB1;
+        return {v, __uint_as_float((unsigned)__builtin_amdgcn_update_dpp(0, (int)u, CTRL, 0xF, 0xF, true))};
+    }
+#else
+    return {v, v};
+#endif
+}
+template <int M>
+__device__ __forceinline__ float butterfly_sum(float v) { const LanePair p = butterfly_pair<M>(v); return p.a + p.b; }
+template <int M>
+__device__ __forceinline__ float butterfly_max(float v) { const LanePair p = butterfly_pair<M>(v); return fmaxf(p.a, p.b); }
+
+// The value of lane ^ 8, ^ 1, among the sixteen lanes of a row.
+__device__ __forceinline__ float lane_xor8(float v) { return butterfly_pair<8>(v).b; }
+__device__ __forceinline__ float lane_xor1(float v) { return butterfly_pair<1>(v).b; }
+// The sum over the sixteen lanes of a row, steps 8, 4, 2, 1; and in steps 1, 2, 4, 8, where the step of 4 takes a lane of the other
+// four of eight: the two before it have left the same in all four.
+__device__ __forceinline__ float row_sum_down(float v) { return butterfly_sum<1>(butterfly_sum<2>(butterfly_sum<4>(butterfly_sum<8>(v)))); }
+__device__ __forceinline__ float row_sum_up(float v) {
+    v = butterfly_sum<2>(butterfly_sum<1>(v));
+#ifdef __HIP_DEVICE_COMPILE__
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));      // lane 7 - i of eight
+#endif
+    return butterfly_sum<8>(v);
+}
+
+// Sum over the 64 lanes of a wave (all of them active); every lane receives the total.  The order of
 // the butterfly is fixed, so the result does not depend on anything but the inputs.
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int m = WAVE / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, WAVE);
-    return v;
+    return butterfly_sum<1>(butterfly_sum<2>(butterfly_sum<4>(butterfly_sum<8>(butterfly_sum<16>(butterfly_sum<32>(v))))));
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int m = WAVE / 2; m > 0; m >>= 1) v = fmaxf(v, __shfl_xor(v, m, WAVE));
-    return v;
+    return butterfly_max<1>(butterfly_max<2>(butterfly_max<4>(butterfly_max<8>(butterfly_max<16>(butterfly_max<32>(v))))));
 }
 
 // Sum over a workgroup of NWAVES waves; `scratch` holds NWAVES floats of LDS.

@@ -511,8 +511,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
                     for (int e = 0; e < 4; ++e) sq = fmaf(y[e], y[e], sq);
                 }
             }
-            sq += __shfl_xor(sq, 16, WAVE);
-            sq += __shfl_xor(sq, 32, WAVE);
+            sq = butterfly_sum<32>(butterfly_sum<16>(sq));
             wave_sq[i] = sq;
         }
         // the waves that share rows add their sums in the order of their columns, through the LDS the operands
@@ -884,8 +883,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
         }
     }
     if (NORM == NORM_INSIDE) {
-        ss += __shfl_xor(ss, 16, WAVE);
-        ss += __shfl_xor(ss, 32, WAVE);
+        ss = butterfly_sum<32>(butterfly_sum<16>(ss));
         if (g == 0) ssq[wave][r16] = ss;
     }
     __syncthreads();
@@ -961,9 +959,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
                 }
                 float sq = y * y;                       // t256 = (16 q + c) * 4 + e: the 16 columns c are its bits 2..5
                 sq += __shfl_xor(sq, 4, WAVE);
-                sq += __shfl_xor(sq, 8, WAVE);
-                sq += __shfl_xor(sq, 16, WAVE);
-                sq += __shfl_xor(sq, 32, WAVE);
+                sq = butterfly_sum<32>(butterfly_sum<16>(butterfly_sum<8>(sq)));
                 if ((l % 16) == 0 && row < ROWS) emit_ss[(long long)blockIdx.x * SSR + row] = sq;
             } else if (MODE == OUT_F32_ACCUM) {
                 if (row < M && col < N) ((float*)Y)[row * N + col] = y_old[ei][tn] + v;
@@ -1099,7 +1095,7 @@ __global__ __launch_bounds__(SK_NT) void gemm_bf16_skinny64_kernel(const bf16_t*
             const long long row = i * 16 + g * 4 + e;
             float v = acc[i][e];
             if (NORM == NORM_SCALED) v *= scale_lds[row];
-            const float partner = (MODE == OUT_SWIGLU) ? __shfl_xor(v, 1, WAVE) : 0.f;
+            const float partner = (MODE == OUT_SWIGLU) ? lane_xor1(v) : 0.f;
             store_elem<MODE>(Y, row, col, M, N, v, partner);
         }
 }
@@ -1129,10 +1125,7 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const float* __restr
         float t = 0.f;
         if (row < ex.ss_rows)
             for (int j = q; j < ex.n_ss; j += 16) t += ex.ss_in[(long long)j * ex.ss_rows + row];
-        t += __shfl_xor(t, 1, WAVE);
-        t += __shfl_xor(t, 2, WAVE);
-        t += __shfl_xor(t, 4, WAVE);
-        t += __shfl_xor(t, 8, WAVE);
+        t = row_sum_up(t);
         scale = 1.0f / sqrtf(t / (float)ex.K + ex.eps);
     }
     const bool whole = N % 4 == 0 && col + 3 < N;
@@ -1204,10 +1197,7 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const float* __restr
         }
     }
     if (EMIT) {
-        sq += __shfl_xor(sq, 1, WAVE);
-        sq += __shfl_xor(sq, 2, WAVE);
-        sq += __shfl_xor(sq, 4, WAVE);
-        sq += __shfl_xor(sq, 8, WAVE);
+        sq = row_sum_up(sq);
         if (q == 0 && row < ex.ss_rows) ex.emit_ss[(long long)blockIdx.x * ex.ss_rows + row] = sq;   // rows beyond M: zero
     }
 }
@@ -1234,10 +1224,7 @@ __global__ __launch_bounds__(FC_ROWS * 16) void splitk_finish_conv_kernel(const 
         float t = 0.f;
         if (row < ex.ss_rows)
             for (int j = q; j < ex.n_ss; j += 16) t += ex.ss_in[(long long)j * ex.ss_rows + row];
-        t += __shfl_xor(t, 1, WAVE);
-        t += __shfl_xor(t, 2, WAVE);
-        t += __shfl_xor(t, 4, WAVE);
-        t += __shfl_xor(t, 8, WAVE);
+        t = row_sum_up(t);
         scale = 1.0f / sqrtf(t / (float)ex.K + ex.eps);
     }
     if (row >= M || ch0 >= d) return;                      // d is a multiple of 16: four channels or none

@@ -214,10 +214,7 @@ __global__ __launch_bounds__(256) void qkv_post64_kernel(
             ss = fmaf(v[1], v[1], ss);
             ss = fmaf(v[2], v[2], ss);
             ss = fmaf(v[3], v[3], ss);
-            ss += __shfl_xor(ss, 8, WAVE);
-            ss += __shfl_xor(ss, 4, WAVE);
-            ss += __shfl_xor(ss, 2, WAVE);
-            ss += __shfl_xor(ss, 1, WAVE);
+            ss = row_sum_down(ss);
             if (is_q ? q_norm_w != nullptr : k_norm_w != nullptr) {
                 const float inv = 1.0f / sqrtf(ss / (float)HD + eps);
 #pragma unroll
@@ -226,7 +223,7 @@ __global__ __launch_bounds__(256) void qkv_post64_kernel(
             if (TURN == TURN_HALVES) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float other = __shfl_xor(v[e], 8, WAVE);
+                    const float other = lane_xor8(v[e]);
                     const float x0 = first ? v[e] : other, x1 = first ? other : v[e];
                     v[e] = first ? (x0 * rc[e] - x1 * rs[e]) : (x0 * rs[e] + x1 * rc[e]);
                 }
