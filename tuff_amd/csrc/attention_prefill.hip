@@ -79,8 +79,10 @@ struct WideArgs {
 // faster than one with two (2,048 tokens, 16 heads of two maps of 64 over values of 128, a window of 1,024: 117 -> 67 us).
 // The wide form with heads of up to 64 channels: left alone it takes 259 registers, three too many for two workgroups a CU (every
 // head's weights on every kv head's values, 2,048 tokens, 32 heads, 8 kv heads of 64: 870 us, with two 555, since then by VHS).
+// Heads of 96 with one step's copies under way fit two workgroups a CU (2,048 tokens after 16,000, 8 heads: 394 -> 364 us); heads of
+// 128 would not without spilling (16 heads: 509 -> 527).
 constexpr int groups_a_cu(int hdp, int vdp, int maps, bool ex, int vhs) {
-    return vhs > 1 || (maps == 2 && hdp <= 128 && vdp <= 128) || (maps == 1 && ex && hdp <= 64 && vdp <= 64) ? 2 : 1;
+    return vhs > 1 || (!ex && hdp == 96) || (maps == 2 && hdp <= 128 && vdp <= 128) || (maps == 1 && ex && hdp <= 64 && vdp <= 64) ? 2 : 1;
 }
 
 // HDP, VDP: the channels of a key row and of a value in the tiles, multiples of 32 (a map's share of a key row too).  NW: waves
@@ -627,9 +629,12 @@ TUFF_EXPORT int tuff_attention_prefill_biased(const void* q, const void* k_cache
 #define GO_BIAS(HDP, NBW, AHEAD, BIAS) return launch<HDP, NBW, AHEAD, BIAS>(grid, stream, Q, K, V, (bf16_t*)out, block_table, max_blocks, (const int2*)blk, \
                                              (const int4*)req_info, H, Hkv, hd, page_size, window, sl, seg_keys, ws_o, ws_ml, n_segs > 1 ? nullptr : sinks, slopes)
 #define GO(HDP, NBW, AHEAD) do { if (slopes) GO_BIAS(HDP, NBW, AHEAD, SLOPES); GO_BIAS(HDP, NBW, AHEAD, NO_BIAS); } while (0)
-    if (hd <= 32) GO(32, 2, 3);
-    else if (hd <= 64) GO(64, 2, 2);
-    else if (hd <= 96) GO(96, 2, 2);
+    // Steps of copies under way (register sets): one up to 96 channels, where two workgroups a CU cover for each other (2,048 tokens
+    // after 16,000, 32 heads of 64: 414 us with two steps, 396 with one), two for the smallest heads, whose steps are short (16
+    // heads of 32: one 248, two 235, three 261), and where a CU has one workgroup.
+    if (hd <= 32) GO(32, 2, 2);
+    else if (hd <= 64) GO(64, 2, 1);
+    else if (hd <= 96) GO(96, 2, 1);
     else if (hd <= 128) GO(128, 2, 2);
     else GO(256, 2, 1);
 #undef GO
@@ -692,8 +697,8 @@ TUFF_EXPORT int tuff_attention_prefill_wide(const void* q, const void* k_cache, 
         grid.y = ceil_div(Hkv, VHS);
         return narrow(number<64>(), number<1>(), number<1>(), number<VHS>(), number<8>());
     }
-    if (widest <= 32) return narrow(number<32>(), number<3>(), number<2>(), number<1>(), number<4>());
-    if (widest <= 64) return narrow(number<64>(), number<2>(), number<2>(), number<1>(), number<4>());
+    if (widest <= 32) return narrow(number<32>(), number<1>(), number<2>(), number<1>(), number<4>());
+    if (widest <= 64) return narrow(number<64>(), number<1>(), number<2>(), number<1>(), number<4>());
     if (widest <= 96) GO(96, 2, 2, 96);
     else if (widest <= 128) GO(128, 2, 2, 128);
     else if (hd <= 192 && vd <= 128) GO(192, 2, 1, 128);       // wide rows: tiles no wider than they need be
