@@ -494,6 +494,25 @@ def test_convolution_of_four_channels_a_thread_has_the_bits_of_one(gpu, C, K, bi
         assert all(torch.equal(a, b_) for a, b_ in zip(*got)), lens
 
 
+@pytest.mark.parametrize("T, H, vd", [(1, 1, 8), (3, 5, 24), (700, 32, 64), (129, 3, 136)])
+def test_gates_and_biases_of_several_numbers_a_thread_have_the_bits_of_one(gpu, T, H, vd):
+    """Rows off a 16-byte border take the kernels of one number a thread."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(T)
+    o, gates = torch.randn(T * H * vd, generator=gen).bfloat16().to(gpu), torch.randn(T, H, generator=gen).to(gpu)
+    x, bias = torch.randn(T * H * vd, generator=gen).to(gpu), torch.randn(H * vd, generator=gen).to(gpu)
+    got = []
+    for off in (0, 1):
+        at = lambda like: torch.empty(like.numel() + 1, dtype=like.dtype, device=gpu)[off:off + like.numel()].copy_(like)
+        y = torch.empty(T, H * vd, dtype=torch.bfloat16, device=gpu)
+        ops.head_mix_gate(at(o).view(T, H * vd), y, H=H, Hkv=1, vd=vd, gates=gates)
+        casts = [torch.empty(T, H * vd, dtype=dt, device=gpu) for dt in (torch.bfloat16, torch.float32)]
+        for c in casts:
+            ops.cast(at(x).view(T, H * vd), c, bias)
+        got.append([y] + casts)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize("T", [1, 17, 300])
 @pytest.mark.parametrize("H, G, rot, norm, ps", [(32, 8, 32, True, 16), (3, 3, 64, False, 48), (5, 1, 20, True, 32), (4, 2, 0, True, 16), (4, 4, 0, False, 64)])
 def test_heads_of_64_turned_in_pairs_or_not_at_all(gpu, T, H, G, rot, norm, ps):

@@ -412,6 +412,19 @@ __global__ __launch_bounds__(WAVE) void head_mix_gate_kernel(const TI* __restric
     }
 }
 
+// Gates alone, eight bfloat16 channels a thread (2,048 tokens, 32 heads of 64: a wave a head 16.3 us, 5.7 this way).
+__global__ __launch_bounds__(256) void head_gate_eights_kernel(const bf16_t* __restrict__ o, const float* __restrict__ gates, int gate_stride,
+                                                               bf16_t* __restrict__ out, long long n, int H, int vd) {
+    const long long at = ((long long)blockIdx.x * 256 + threadIdx.x) * 8;
+    if (at >= n) return;
+    const long long row = at / vd;
+    const float g = 1.0f / (1.0f + expf(-gates[row / H * gate_stride + row % H]));
+    bf16x8 v = *(const bf16x8*)(o + at);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (bf16_t)((float)v[e] * g);
+    *(bf16x8*)(out + at) = v;
+}
+
 // The mix for G heads of one kv head at once: a wave a (token, G heads, 64 channels), which reads every weighted sum once instead
 // of G times, eight heads' at a time.  Bound by the float32 sums: 2,048 tokens, 32 heads, 8 kv heads of 64:
 // 82 -> 28.5 us.  Two heads, or four where a kv head has a multiple of four (eight keep 64 coefficients under way and take
@@ -466,6 +479,12 @@ TUFF_EXPORT int tuff_head_mix_gate(const void* o, int in_dt, const float* talk, 
                                    int dt, int n_tokens, int H, int Hkv, int vd, hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (H <= 0 || Hkv <= 0 || H % Hkv || H > 65535 || vd <= 0) return -2;
+    const long long n = (long long)n_tokens * H * vd;
+    if (!talk && gates && in_dt == DT_BF16 && dt == DT_BF16 && vd % 8 == 0 && (((uintptr_t)o | (uintptr_t)out) & 15) == 0 && n < (1ll << 40)) {
+        hipLaunchKernelGGL(head_gate_eights_kernel, dim3((unsigned)ceil_div_ll(n, 2048)), dim3(256), 0, stream, (const bf16_t*)o, gates, gate_stride,
+                           (bf16_t*)out, n, H, vd);
+        return launch_status();
+    }
     dim3 grid(n_tokens, H), block(WAVE);
     const int share = talk ? H / Hkv : 1;                            // heads that read the same sums
     const int group = share % 4 == 0 ? 4 : share % 2 == 0 ? 2 : 1;

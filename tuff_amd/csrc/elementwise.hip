@@ -158,9 +158,30 @@ __global__ void cast_bias_kernel(const float* __restrict__ in, const float* __re
     if (i < n) out[i] = from_f32<TO>(in[i] + bias[i % N]);
 }
 
+// Four numbers a thread, a row of N a multiple of four (2,048 rows of 3,072: 12.0 us a number a thread, most of it the remainder of
+// 64-bit numbers, 7.9 this way).
+template <typename TO>
+__global__ void cast_bias_fours_kernel(const float* __restrict__ in, const float* __restrict__ bias, TO* __restrict__ out, unsigned n4, unsigned N4) {
+    typedef TO out4 __attribute__((ext_vector_type(4)));
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const f32x4 v = *(const f32x4*)(in + (long long)i * 4), b = *(const f32x4*)(bias + i % N4 * 4);
+    out4 o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = from_f32<TO>(v[e] + b[e]);
+    *(out4*)(out + (long long)i * 4) = o;
+}
+
 TUFF_EXPORT int tuff_cast_bias(const float* in, const float* bias, void* out, int out_dt, long long n, int N, hipStream_t stream) {
     if (n <= 0) return 0;
     if (N <= 0 || !bias) return -2;
+    if (N % 4 == 0 && n % 4 == 0 && n < (1ll << 32) && (((uintptr_t)in | (uintptr_t)bias | (uintptr_t)out) & 15) == 0) {
+        const unsigned n4 = (unsigned)(n / 4);
+        dim3 grid4(ceil_div_ll(n4, 256)), block4(256);
+        if (out_dt == DT_BF16) hipLaunchKernelGGL((cast_bias_fours_kernel<bf16_t>), grid4, block4, 0, stream, in, bias, (bf16_t*)out, n4, (unsigned)(N / 4));
+        else hipLaunchKernelGGL((cast_bias_fours_kernel<float>), grid4, block4, 0, stream, in, bias, (float*)out, n4, (unsigned)(N / 4));
+        return launch_status();
+    }
     dim3 grid((unsigned)ceil_div_ll(n, 256)), block(256);
     if (out_dt == DT_BF16) hipLaunchKernelGGL((cast_bias_kernel<bf16_t>), grid, block, 0, stream, in, bias, (bf16_t*)out, n, N);
     else hipLaunchKernelGGL((cast_bias_kernel<float>), grid, block, 0, stream, in, bias, (float*)out, n, N);
