@@ -314,13 +314,15 @@ def test_prompt_kernel_in_its_wide_form_against_the_general_kernel(gpu, H, Hkv, 
         assert (got - want).abs().max() <= tol * max(1.0, float(want.abs().max())), opts
 
 
+@pytest.mark.parametrize("many", [False, True])
 @pytest.mark.parametrize("ps", [16, 48])
 @pytest.mark.parametrize("H, Hkv, hd, vd", [(8, 8, 64, 64), (10, 5, 64, 24), (9, 9, 16, 32), (12, 3, 40, 64), (4, 4, 32, 32), (6, 6, 8, 8)])
-def test_prompt_kernel_with_the_values_of_several_kv_heads_a_workgroup(gpu, H, Hkv, hd, vd, ps):
-    """Heads of up to 64 channels and more than two kv heads: numbers of kv heads that fill a workgroup's four and that do not, every
-    kind of penalty, page sizes that are and are not a power of two; to float32's rounding, as above."""
+def test_prompt_kernel_with_the_values_of_several_kv_heads_a_workgroup(gpu, H, Hkv, hd, vd, ps, many):
+    """Heads of up to 64 channels and more than two kv heads: launches of few workgroups, which take two kv heads each, and of many,
+    which take four, numbers of kv heads that fill those and that do not, every kind of penalty, page sizes that are and
+    are not a power of two; to float32's rounding, as above."""
     from tuff_amd.csrc import ops
-    reqs = [(0, 70), (1090, 5), (300, 1), (17, 200)]
+    reqs = [(i % 70, 1 + i % 9) for i in range(64)] if many else [(0, 70), (1090, 5), (300, 1), (17, 200)]
     for opts in [(0, 0, 0, 0, 1, 0), (0, 0, 1, 0, 1, 0), (0, 1, 0, 1, 1, 0), (0, 0, 1, 1, 1, 0), (100, 1, 0, 1, 1, 0)]:
         c = _paged_case(gpu, H, Hkv, hd, vd, reqs, opts, ps=ps, seed=H + hd)
         want = _general({**c, "gates": None}, H, Hkv, hd, vd, ps=ps)

@@ -690,12 +690,18 @@ TUFF_EXPORT int tuff_attention_prefill_wide(const void* q, const void* k_cache, 
         if (slopes) return log_r1 ? go(number<SLOPES | LOG_DIST>()) : go(number<SLOPES>());
         return log_r1 ? go(number<LOG_DIST>()) : go(number<NO_BIAS>());
     };
-    // Four kv heads' values a workgroup from three kv heads on (from four where heads have at most 32 channels: the tiles are 64
-    // wide; 2,048 tokens, 12 heads on 3 kv heads of 32: 97 us in one-head workgroups, 102 in this; 16 on 4 of 16: 170, 112).
-    constexpr int VHS = 4;
+    // Several kv heads' values a workgroup from three kv heads on (from four where heads have at most 32 channels: the tiles are 64
+    // wide; 2,048 tokens, 12 heads on 3 kv heads of 32: 97 us in one-head workgroups, 102 in this; 16 on 4 of 16: 170, 96).  Four,
+    // but two where that gives no CU more than one workgroup: then a block's steps one after the other are all there is (100
+    // tokens, 32 heads on 8 kv heads of 64: one 13.9 us, four 14.6, two 11.6; 400 of 16 on 4: 28.4, 24.7 and 19.9; 400 of 32 on 8,
+    // 416 workgroups of two: 55.7, 27.9 and 32.4).
     if (all_v && widest <= 64 && Hkv > (widest <= 32 ? 3 : 2)) {
-        grid.y = ceil_div(Hkv, VHS);
-        return narrow(number<64>(), number<1>(), number<1>(), number<VHS>(), number<8>());
+        if ((long long)n_qblocks * Hkv * ceil_div(Hkv, 2) <= 256) {
+            grid.y = ceil_div(Hkv, 2);
+            return narrow(number<64>(), number<1>(), number<1>(), number<2>(), number<8>());
+        }
+        grid.y = ceil_div(Hkv, 4);
+        return narrow(number<64>(), number<1>(), number<1>(), number<4>(), number<8>());
     }
     if (widest <= 32) return narrow(number<32>(), number<1>(), number<2>(), number<1>(), number<4>());
     if (widest <= 64) return narrow(number<64>(), number<1>(), number<2>(), number<1>(), number<4>());
