@@ -37,6 +37,15 @@ def test_gemm_f32(gpu, M, N, K):
         assert torch.equal(one[0], out[M - 1])
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1028, 1 << 20])
+@pytest.mark.parametrize("off", [0, 1, 4])
+def test_fill_writes_what_it_is_given_and_nothing_else(gpu, n, off):
+    from tuff_amd.csrc import ops
+    b = torch.full((n + 9,), 7, dtype=torch.int32, device=gpu)
+    ops.fill_u32(b[off:off + n], 5)
+    assert (b[off:off + n] == 5).all() and (b[:off] == 7).all() and (b[off + n:] == 7).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 8, 32), (16, 2048, 96), (17, 2049, 128), (33, 70, 320), (64, 2052, 2080), (65, 64, 2048),
                                    (300, 2050, 2048), (130, 66, 4160), (1030, 4100, 160), (500, 2048, 64)])
 def test_gemm_f32_matrix_cores(gpu, M, N, K):
