@@ -518,8 +518,8 @@ def test_gates_and_biases_of_several_numbers_a_thread_have_the_bits_of_one(gpu, 
 @pytest.mark.parametrize("T", [1, 17, 300])
 @pytest.mark.parametrize("H, G, rot, norm, ps", [(32, 8, 32, True, 16), (3, 3, 64, False, 48), (5, 1, 20, True, 32), (4, 2, 0, True, 16), (4, 4, 0, False, 64)])
 def test_heads_of_64_turned_in_pairs_or_not_at_all(gpu, T, H, G, rot, norm, ps):
-    """The kernel of sixteen lanes a head against the one of a wave a head, which rows off a 16-byte border take: the norm's sum in
-    another order, so a last bit of bfloat16 at most; values are the same."""
+    """The kernel of sixteen lanes a head has the bits of the one of a wave a head, which rows off a 16-byte border take: what
+    comes out does not depend on where a row lies."""
     from tuff_amd.csrc import ops
     gen = torch.Generator().manual_seed(T + H)
     width = (H + 2 * G) * 64
@@ -537,10 +537,7 @@ def test_heads_of_64_turned_in_pairs_or_not_at_all(gpu, T, H, G, rot, norm, ps):
         ops.qkv_post(at.view(T, width), q, H=H, Hkv=G, hd=64, positions=pos, eps=1e-5, q_norm_w=w[0], k_norm_w=w[1], inv_freq=inv,
                      rotary_dim=rot, interleaved=True, k_cache=k, v_cache=v, slot_mapping=pos + ps, page_size=ps)
         got.append((q, k, v))
-    for a, b in zip(got[0][:2], got[1][:2]):
-        # the larger of two turned numbers moves by its own last bit, the smaller by that much times the other's cosine or sine
-        assert ((a.float() - b.float()).abs() <= 2.0 ** -7 * a.float().abs() + 2.0 ** -20).all()
-    assert torch.equal(got[0][2], got[1][2])
+    assert all(torch.equal(a, b) for a, b in zip(*got))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(POST_WAVES * WAVE) void qkv_post_kernel(
                 const float other = vals[partner[i]];
                 const float x0 = first[i] ? v[i] : other;
                 const float x1 = first[i] ? other : v[i];
-                v[i] = first[i] ? (x0 * rc[i] - x1 * rs[i]) : (x0 * rs[i] + x1 * rc[i]);
+                v[i] = first[i] ? fmaf(-rs[i], x1, x0 * rc[i]) : fmaf(rs[i], x0, x1 * rc[i]);
             }
         }
         T* dst = nullptr;
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(POST_WAVES * WAVE) void qkv_post_kernel(
 // neighbouring channels turned in pairs (of the first rotary_dim, a multiple of four, channels), or with no rotation.  Two kinds of workgroups in one launch:
 //  * q and k: sixteen lanes take one token and walk a share of its heads; lane l holds the channels
 //    4l .. 4l+3 of a head (one 8-byte load for bfloat16), the norm's sum of squares is a butterfly over
-//    the sixteen lanes, the rotation's partner channel j +- 32 sits in lane l ^ 8 (a pair's in the same lane), and the
+//    the sixteen lanes (of each of the four channels by itself for the last two turns, see there), the rotation's partner channel j +- 32 sits in lane l ^ 8 (a pair's in the same lane), and the
 //    token's cosines and sines are computed once for all its heads.
 //  * v: a workgroup takes sixteen consecutive tokens and one kv head, brings the rows into LDS and
 //    writes, for every channel, the sixteen positions in one run where the tokens fill a run of sixteen
@@ -210,11 +210,22 @@ __global__ __launch_bounds__(256) void qkv_post64_kernel(
             const bool is_q = head < H;
             float v[4];
             load4(row + (long long)head * HD, v);
-            float ss = v[0] * v[0];
-            ss = fmaf(v[1], v[1], ss);
-            ss = fmaf(v[2], v[2], ss);
-            ss = fmaf(v[3], v[3], ss);
-            ss = row_sum_down(ss);
+            float ss;
+            if (TURN == TURN_HALVES) {
+                ss = v[0] * v[0];
+                ss = fmaf(v[1], v[1], ss);
+                ss = fmaf(v[2], v[2], ss);
+                ss = fmaf(v[3], v[3], ss);
+                ss = row_sum_down(ss);
+            } else {
+                // in the order of the kernel above, which takes these turns where rows lie on no border: channels 32, 16, 8, 4, 2
+                // and 1 apart, the first four in lanes 8, 4, 2 and 1 apart, the last two in this lane (fmaf: the square is
+                // rounded; as a product it could become a part of the first sum)
+                float sq[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sq[e] = row_sum_down(fmaf(v[e], v[e], 0.f));
+                ss = (sq[0] + sq[2]) + (sq[1] + sq[3]);
+            }
             if (is_q ? q_norm_w != nullptr : k_norm_w != nullptr) {
                 const float inv = 1.0f / sqrtf(ss / (float)HD + eps);
 #pragma unroll
@@ -231,8 +242,8 @@ __global__ __launch_bounds__(256) void qkv_post64_kernel(
 #pragma unroll
                 for (int e = 0; e < 4; e += 2) {
                     const float x0 = v[e], x1 = v[e + 1];
-                    v[e] = x0 * rc[e] - x1 * rs[e];
-                    v[e + 1] = x0 * rs[e] + x1 * rc[e];
+                    v[e] = fmaf(-rs[e], x1, x0 * rc[e]);       // (the roundings of the kernel above)
+                    v[e + 1] = fmaf(rs[e], x0, x1 * rc[e]);
                 }
             }
             if (is_q) store4(q_out + ((long long)t * H + head) * HD + 4 * l, v);
@@ -460,8 +471,8 @@ TUFF_EXPORT int tuff_qkv_post(const void* qkv, void* q_out, void* k_out, void* k
     if (!angles || !inv_freq) n_angles = 0;              // [n_angles][2][rotary_dim / 2] as tuff_rope_table makes it
     const bool turned = inv_freq && rotary_dim > 0;
     const int turn = !turned ? TURN_NONE : rotary_dim == 64 && !interleaved ? TURN_HALVES : interleaved && rotary_dim % 4 == 0 ? TURN_PAIRS : -1;
-    // (the other two turns in bfloat16, on borders of 16 bytes: 2,048 tokens, 32 heads and 8 kv heads, 32 channels turned in pairs
-    // 33.6 us in the kernel above, 11.2 in this, no turn 20.9 and 9.7, up to 300 tokens the same)
+    // (the other two turns in bfloat16, on borders of 16 bytes, with the bits of the kernel that takes the rest: 2,048 tokens, 32 heads
+    // and 8 kv heads, 32 channels turned in pairs 33.6 us in that kernel, 10.9 in this, no turn 21.0 and 8.5, up to 300 tokens the same)
     if (hd == 64 && turn >= 0 && !k_out && page_size % 16 == 0 && row_stride <= 0 &&
         (turn == TURN_HALVES || (dt == DT_BF16 && ((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0))) {
         // shares of a token's heads: enough sixteen-lane groups for the chip, whole heads each
