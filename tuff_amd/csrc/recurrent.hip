@@ -891,6 +891,11 @@ __global__ __launch_bounds__(WAVE) void head_norm_gate_kernel(const float* __res
     }
 }
 
+// Waves a workgroup of long runs: four up to 192 key channels, up to 64 only with the forget gate and the state-space rule (2,048
+// tokens, 16 heads of 64: wkv 232 us in single waves, 249 in fours, the delta rule 306 and 310); beyond 192 a SIMD's registers
+// hold too few waves (wkv, 4 heads of 256: 670, 831).
+constexpr int waves_of_runs(int ni, int split, bool forget, bool ssd) { return split == 16 && (ni == 1 ? forget || ssd : ni <= 3) ? 4 : 1; }
+
 template <typename TA, typename T, bool DELTA, bool FORGET = false, bool SSD = false>
 int launch_scan(ScanArgs p, int n_tokens, int R, hipStream_t stream) {
     if (p.H > 65535 || p.D > 256) return -2;
@@ -898,12 +903,15 @@ int launch_scan(ScanArgs p, int n_tokens, int R, hipStream_t stream) {
     const int split = narrow ? 4 : 16;
     const int ni = narrow ? (p.D + 15) / 16 : (p.D + 63) / 64;
     const bool singles = n_tokens <= R;
-    // Four waves a workgroup: up to 192 key channels, up to 64 only the forget gate and the state-space rule (2,048 tokens, 16 heads
-    // of 64: wkv 232 us in single waves, 249 in fours, the delta rule 306 and 310); beyond 192 a SIMD's registers hold too few
-    // waves (wkv, 4 heads of 256: 670, 831).  Runs long enough that the first rows' way into LDS counts little, and values
-    // enough for the waves.
-    auto shared_rows = [](int n16) { return n16 == 1 ? FORGET || SSD : n16 <= 3; };
-    const int waves = !singles && !narrow && shared_rows(ni) && (long long)n_tokens >= 32ll * R && p.Dv >= 32 ? 4 : 1;
+    // Four waves a workgroup, where the shape has them and runs are long enough that the first rows' way into LDS counts little:
+    // from 48 tokens on, or 32 with more than 128 channels or eight single waves a CU (one request of 33 tokens, 16 heads of
+    // 128 x 64, delta rule: 15.2 us in single waves, 15.8 in fours, of 64 21.4 and 21.3; 64 requests of 33 118.4 and 112.9).  The
+    // state-space rule up to 64 channels, whose tokens bring two rows and not three: from 320 on, or 100 with two waves a CU (8 heads
+    // of 64 x 64, one request of 100 tokens: 15.9 us and 17.0, of 300 35.6 and 36.0, of 2,048 207 and 198; 8 of 100 18.8 and 18.0).
+    const long long singly = (long long)R * p.H * ceil_div(p.Dv, WAVE / split);
+    const long long least = SSD && ni == 1 ? (singly >= 512 ? 100 : 320) : ni == 3 || singly >= 2048 ? 32 : 48;
+    const bool long_runs = n_tokens >= least * R;
+    const int waves = !singles && long_runs && p.Dv >= 32 ? waves_of_runs(ni, split, FORGET, SSD) : 1;
     dim3 grid(R, p.H, ceil_div(p.Dv, waves * WAVE / split)), block(waves * WAVE);
     if (grid.z > 65535) return -2;
     p.by_xcd = (long long)R * p.H * grid.z < (1ll << 32);       // the workgroups' numbers have 32 bits there
@@ -912,7 +920,7 @@ int launch_scan(ScanArgs p, int n_tokens, int R, hipStream_t stream) {
     const bool whole = p.D % 4 == 0 && p.lda % 4 == 0 && in_fours(p.a, sizeof(TA)) && (FORGET || in_fours(p.k, sizeof(TA))) &&
                        (SSD || in_fours(p.decay, 4));
 #define GO(NI, SPLIT, WHOLE, SINGLES, NW) hipLaunchKernelGGL((scan_kernel<TA, T, NI, SPLIT, WHOLE, SINGLES, NW, DELTA, FORGET, SSD>), grid, block, 0, stream, p)
-#define SCAN(NI, SPLIT) do { constexpr int MANY = SPLIT == 16 && (NI == 1 ? FORGET || SSD : NI <= 3) ? 4 : 1; \
+#define SCAN(NI, SPLIT) do { constexpr int MANY = waves_of_runs(NI, SPLIT, FORGET, SSD); \
                              if (whole && singles) GO(NI, SPLIT, true, true, 1); else if (singles) GO(NI, SPLIT, false, true, 1); \
                              else if (whole && waves == 1) GO(NI, SPLIT, true, false, 1); else if (whole) GO(NI, SPLIT, true, false, MANY); \
                              else if (waves == 1) GO(NI, SPLIT, false, false, 1); else GO(NI, SPLIT, false, false, MANY); } while (0)
