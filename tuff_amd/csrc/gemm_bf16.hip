@@ -1116,6 +1116,9 @@ template <int MODE, int NORM, bool EMIT>
 __global__ __launch_bounds__(256) void splitk_finish_kernel(const float* __restrict__ ws, void* __restrict__ Y, int M, int N,
                                                             int rows_padded, int n_slices, FinishExtra ex) {
     static_assert(!EMIT || MODE == OUT_F32_ACCUM, "the emitting epilogue adds into the residual stream");
+    // Slices asked for together, sixteen (all of them, as a rule) or, for the plain epilogues, eight (23 rows, 2,048 x 2,048: 7.13 us
+    // with eight, 7.47 with sixteen, product and sum; 64 rows of 3,072 columns behind a norm 10.4 and 10.7)
+    constexpr int TOGETHER = EMIT ? 16 : 8;
     const int tid = threadIdx.x, q = tid % 16;
     const long long row = (long long)blockIdx.y * 16 + tid / 16;
     const long long col = (long long)blockIdx.x * 64 + q * 4;
@@ -1140,16 +1143,16 @@ __global__ __launch_bounds__(256) void splitk_finish_kernel(const float* __restr
     float v[4] = {0.f, 0.f, 0.f, 0.f};
     if (row < M) {
         if (whole) {
-            // the slices of a step of sixteen (all of them, as a rule) are asked for together and added in their order
+            // the slices of a step of TOGETHER are asked for together and added in their order
             const long long stride = (long long)rows_padded * N;
             const float* p0 = ws + row * N + col;
-            for (int s0 = 0; s0 < n_slices; s0 += 16) {
-                f32x4 t[16];
+            for (int s0 = 0; s0 < n_slices; s0 += TOGETHER) {
+                f32x4 t[TOGETHER];
 #pragma unroll
-                for (int u = 0; u < 16; ++u)
+                for (int u = 0; u < TOGETHER; ++u)
                     if (s0 + u < n_slices) t[u] = *(const f32x4*)(p0 + (s0 + u) * stride);
 #pragma unroll
-                for (int u = 0; u < 16; ++u)
+                for (int u = 0; u < TOGETHER; ++u)
                     if (s0 + u < n_slices) {
 #pragma unroll
                         for (int e = 0; e < 4; ++e) v[e] += t[u][e];
