@@ -75,7 +75,8 @@ def test_gemm_f32_matrix_cores(gpu, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 64), (4, 17, 128), (3, 250, 704), (4, 4097, 768), (2, 2048, 832), (5, 16, 2112), (13, 2040, 1536),
-                                   (16, 2048, 64), (16, 8200, 320), (9, 4100, 96), (16, 70, 32), (1, 33, 160), (7, 300, 544), (12, 33, 1056)])
+                                   (16, 2048, 64), (16, 8200, 320), (9, 4100, 96), (16, 70, 32), (1, 33, 160), (7, 300, 544), (12, 33, 1056),
+                                   (4, 17, 192), (2, 5000, 256), (16, 3072, 2048), (13, 4096, 512), (16, 2064, 448), (6, 4112, 512)])
 def test_gemm_f32_few_rows(gpu, M, N, K):
     """Up to 16 rows, on the vector unit in groups of four and on the matrix cores, with steps fewer and more than lie in LDS, odd and
     even: the bits of the general kernel's chain; rows behind the last, which are not a number, count nowhere."""

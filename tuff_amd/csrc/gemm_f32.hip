@@ -496,10 +496,11 @@ TUFF_EXPORT int tuff_gemm_f32(const float* X, const float* W, float* Y, int M, i
     }
     if (M <= 16) {
         // Four rows a wave as long as one trip over W serves all rows, or the waves are few enough to run side by side, two a CU (16
-        // rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14).  Twelve steps in LDS where
-        // a CU has one wave (8,192 x 1,024, two a CU: 11.7 us, with six 10.3).
+        // rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14), and K is not so short that
+        // the empty steps it begins with count (4 rows, 2,048 x 64: 3.2 us and 2.7, x 192 3.6 and 3.5, 32,768 x 192 6.4 and 7.2).
+        // Twelve steps in LDS where a CU has one wave (8,192 x 1,024, two a CU: 11.7 us, with six 10.3).
         const long long waves = ceil_div_ll(N, 16) * ceil_div(M, 4);
-        if (K % LONG_STEP == 0 && (M <= 4 || waves <= 512)) {
+        if (K % LONG_STEP == 0 && K >= 192 && (M <= 4 || waves <= 512)) {
             if (waves <= 256) return launch_quad<12>(X, W, Y, M, N, K, accumulate, stream);
             return launch_quad<6>(X, W, Y, M, N, K, accumulate, stream);
         }
