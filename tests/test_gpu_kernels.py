@@ -1660,13 +1660,10 @@ def test_repeat_penalty(gpu):
     assert g.cpu().tolist() == [[0.5, -4.0, 1.0, 4.0], [2.0, -2.0, 1.0, 4.0]]
 
 
-@pytest.mark.parametrize("H,Hkv,hd,page,window", [(4, 2, 16, 16, 0), (6, 2, 32, 32, 40), (32, 8, 64, 16, 0), (8, 8, 64, 48, 0),
-                                                   (16, 1, 64, 16, 100), (10, 2, 128, 16, 0)])
-def test_attention_f32_gives_the_bits_of_the_general_kernel(gpu, H, Hkv, hd, page, window):
-    """Requests of one token and of portions, at the borders of the tiles of 64 keys; pages nobody wrote, and those a window
-    has passed, hold NaN; one value is infinite."""
+def _attention_f32_beside_the_general_kernel(gpu, H, Hkv, hd, page, window, before, new, infinite):
+    """Requests that hold before[r] tokens and bring new[r]; pages nobody wrote, and those a window has passed, hold NaN; a value
+    of the last request, of position `infinite`, is infinite.  The same bits from both kernels."""
     from tuff_amd.csrc import ops
-    before, new = [0, 63, 64, 130, 5, 200, 0], [1, 1, 1, 1, 64, 37, 131]
     R, T, total = len(new), sum(new), [b + n for b, n in zip(before, new)]
     blocks = [-(-t // page) for t in total]
     g = torch.Generator().manual_seed(hd + H)
@@ -1683,7 +1680,7 @@ def test_attention_f32_gives_the_bits_of_the_general_kernel(gpu, H, Hkv, hd, pag
             table[r, b] = p = order.pop()
             k[p, :, :n] = torch.randn(Hkv, n, hd, generator=g)
             v[p, :, :, :n] = torch.randn(Hkv, hd, n, generator=g)
-    v[int(table[6, 40 // page]), 0, 3, 40 % page] = float("inf")
+    v[int(table[-1, infinite // page]), 0, 3, infinite % page] = float("inf")
     starts = np.concatenate([[0], np.cumsum(new)[:-1]])
     info = torch.tensor([[int(s), n, b, t] for s, n, b, t in zip(starts, new, before, total)], dtype=torch.int32)
     q = torch.randn(T, H * hd, generator=g) * 3
@@ -1692,5 +1689,22 @@ def test_attention_f32_gives_the_bits_of_the_general_kernel(gpu, H, Hkv, hd, pag
     ops.attention_general(q.to(gpu), k.to(gpu), v.to(gpu), want, req_of_token=torch.tensor(np.repeat(np.arange(R), new), dtype=torch.int32, device=gpu),
                           positions=torch.tensor(np.concatenate([np.arange(b, t) for b, t in zip(before, total)]), dtype=torch.int32, device=gpu), **kw)
     ops.attention_f32(q.to(gpu), k.to(gpu), v.to(gpu), got, req_info=info.to(gpu), max_q_len=max(new), **kw)
-    assert torch.isfinite(want[:int(starts[6]) + 40]).all()
+    assert torch.isfinite(want[:int(starts[-1]) + infinite - before[-1]]).all()
     assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.parametrize("H,Hkv,hd,page,window", [(4, 2, 16, 16, 0), (6, 2, 32, 32, 40), (32, 8, 64, 16, 0), (8, 8, 64, 48, 0),
+                                                   (16, 1, 64, 16, 100), (10, 2, 128, 16, 0)])
+def test_attention_f32_gives_the_bits_of_the_general_kernel(gpu, H, Hkv, hd, page, window):
+    """Requests of one token and of portions, at the borders of the tiles of 64 keys; pages nobody wrote, and those a window
+    has passed, hold NaN; one value is infinite."""
+    _attention_f32_beside_the_general_kernel(gpu, H, Hkv, hd, page, window, [0, 63, 64, 130, 5, 200, 0], [1, 1, 1, 1, 64, 37, 131], 40)
+
+
+@pytest.mark.parametrize("H,Hkv,hd,page,window", [(4, 2, 16, 16, 0), (8, 2, 32, 48, 1100), (32, 8, 64, 16, 0), (8, 8, 64, 80, 1000),
+                                                   (16, 1, 64, 16, 1500), (10, 2, 128, 48, 0)])
+def test_attention_f32_gives_the_bits_of_the_general_kernel_beyond_a_thousand_keys(gpu, H, Hkv, hd, page, window):
+    """The places of keys are worked out for 1,024 of them at a time, from the first tile that a window reaches: single tokens and
+    portions whose keys end just before, at and after one and two such stretches, pages that are and are not a power of two."""
+    _attention_f32_beside_the_general_kernel(gpu, H, Hkv, hd, page, window, [1022, 1023, 1024, 1087, 2046, 2047, 2048, 3000, 930, 1000, 2000],
+                                             [1, 1, 1, 1, 1, 1, 1, 1, 200, 24, 100], 2060)
