@@ -336,6 +336,41 @@ def test_prompt_kernel_with_the_values_of_several_kv_heads_a_workgroup(gpu, H, H
         assert (got - want).abs().max() <= 3e-5 * max(1.0, float(want.abs().max())), opts
 
 
+@pytest.mark.parametrize("H, Hkv, hd, vd, ps", [(32, 8, 64, 64, 16), (8, 8, 64, 64, 48), (10, 5, 64, 24, 16), (6, 6, 16, 32, 32), (12, 3, 40, 64, 80)])
+def test_long_requests_of_mixed_heads_have_the_same_bits_alone_and_in_company(gpu, H, Hkv, hd, vd, ps):
+    """A portion alone is a launch of few workgroups, which take two kv heads each; among many short requests the same portion goes
+    through the kernel that takes four.  Whole blocks of 128 columns over more than 1,024 and 2,048 keys (the places of pages are worked
+    out for 1,024 at a time), with windows that reach into the portion and beyond; beside the general kernel to float32's rounding."""
+    from tuff_amd.csrc import ops
+    long = [(1500, 200), (2040, 130), (0, 250)]
+    reqs = [(5 + i % 40, 1) for i in range(40)] + long + [(i, 1) for i in range(24)]
+    small = lambda blocks: blocks.shape[0] * Hkv * -(-Hkv // 2) <= 256
+    for opts in [(0, 0, 0, 1, 1, 0), (100, 1, 0, 1, 1, 0), (1500, 0, 1, 0, 1, 0)]:
+        c = _paged_case(gpu, H, Hkv, hd, vd, reqs, opts, ps=ps, seed=H + hd)
+        want = _general({**c, "gates": None}, H, Hkv, hd, vd, ps=ps)
+
+        def sums(first, which):
+            n = np.array([m for _, m in which])
+            ends = np.array([a + m for a, m in which])
+            starts = np.concatenate([[0], np.cumsum(n)])
+            T, at = int(n.sum()), sum(m for _, m in reqs[:first])
+            info = torch.tensor([[int(s), m, a, 0] for s, (a, m) in zip(starts, which)], dtype=torch.int32, device=gpu)
+            blocks = torch.from_numpy(ops.query_blocks(n, H // Hkv, 8, ends))
+            assert small(blocks) == (len(which) == 1)
+            o = torch.full((T, H * Hkv * vd), float("nan"), device=gpu)
+            ops.attention_prefill_wide(c["q"][at:at + T], c["k"], c["v"], o, block_table=c["table"][first:first + len(which)], blocks=blocks.to(gpu),
+                                       req_info=info, H=H, Hkv=Hkv, hd=hd, vd=vd, page_size=ps, max_ctx_len=int(ends.max()), window=c["window"],
+                                       scale=0.2, sinks=c["sinks"], slopes=c["slopes"], log_distance=c["logd"], all_values=True)
+            return o
+        every = sums(0, reqs)
+        for i, (_, m) in enumerate(long):
+            at = 40 + sum(k for _, k in long[:i])
+            assert torch.equal(sums(40 + i, [long[i]]), every[at:at + m]), (opts, i)
+        got = torch.zeros(c["T"], H * vd, device=gpu)
+        ops.head_mix_gate(every, got, H=H, Hkv=Hkv, vd=vd, talk=c["talk"], gates=None)
+        assert (got - want).abs().max() <= 3e-5 * max(1.0, float(want.abs().max())), opts
+
+
 @pytest.mark.parametrize("H, Hkv, hd, vd", SHAPES)
 def test_single_token_kernels_with_float32_weights_against_the_general_kernel(gpu, H, Hkv, hd, vd):
     """Single tokens at the first position, on both sides of a part's 256 keys and far behind them."""
