@@ -473,10 +473,12 @@ def test_kept_first_tokens_with_one_map_a_head(gpu, H, Hkv, hd, vd, window, keep
 @pytest.mark.parametrize("dim, vd", [(8, 8), (32, 64), (24, 128), (32, 256), (64, 64), (56, 128), (64, 200), (96, 128), (80, 192), (96, 256), (128, 128), (120, 256)])
 def test_prompt_attention_with_maps_of_every_tile_width(gpu, dim, vd, ps):
     """The prompt kernel's tiles come in several widths: a portion far into a request and one from its start, with windows
-    that keep none to hundreds of first tokens (jumps from the kept steps to the window's on and off borders of pages)."""
+    that keep none to a thousand first tokens (jumps from the kept steps to the window's on and off borders of pages), over more than
+    2,048 keys (the places of pages are worked out for 1,024 at a time)."""
     from tuff_amd.csrc import ops
     combine = (0.9, 1e-5, 0.6)
-    for heads, Hkv, window, keep, past, T in ((4, 2, 0, 0, 83, 90), (3, 1, 70, 5, 400, 70), (2, 2, 33, 200, 380, 40), (5, 1, 16, 64, 0, 150), (2, 1, 100, 17, 331, 3)):
+    for heads, Hkv, window, keep, past, T in ((4, 2, 0, 0, 83, 90), (3, 1, 70, 5, 400, 70), (2, 2, 33, 200, 380, 40), (5, 1, 16, 64, 0, 150), (2, 1, 100, 17, 331, 3),
+                                              (2, 1, 1100, 1200, 2500, 40), (3, 3, 0, 0, 2070, 33)):
         positions = list(range(past, past + T))
         n = past + T
         q, kc, vc, want, kw = _kernel_rows(gpu, 2 * heads, Hkv, dim, vd, 2, window, keep, positions, n, dim + vd + T, ps)
