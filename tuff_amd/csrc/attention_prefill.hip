@@ -1,13 +1,14 @@
 // Paged attention for steps that carry prompt portions: bfloat16 cache, matrix cores, keys and
 // values shared by a workgroup through LDS.
 //
-// A workgroup of four waves takes one kv head and one block of 64 * NBW query columns of one
-// request (a column = one query head of one token; NBW * 16 columns a wave) and walks over all
+// A workgroup of NW waves takes one kv head and one block of 16 * NBW * NW query columns of one
+// request (a column = one query head of one token; 16 * NBW columns a wave; 128 columns a block in
+// every form, four waves of 32 or eight of 16, but for two maps, see below) and walks over all
 // keys these columns may see, 64 at a time, from key 0 (or the first 64 the window still
 // reaches).  The K rows and V columns of a step are copied from the pages into LDS once, by all
-// threads, a few steps ahead of their use; every wave reads its MFMA operands from there.  Each
-// column carries a running maximum, sum and output (online softmax) and is written normalised at
-// the end: no work space and no second kernel.
+// threads, AHEAD steps (one or two) before their use; every wave reads its MFMA operands from
+// there.  Each column carries a running maximum, sum and output (online softmax) and is written
+// normalised at the end: no work space and no second kernel (unless the keys are cut into segments).
 //
 // A column's arithmetic depends only on its own position: steps start at multiples of 64, and
 // the columns of a matrix product do not influence each other.  So a token's result does not
@@ -28,7 +29,8 @@
 // logarithmic distance penalty r1_h * ln(1 + r2_h * (position - key)) off the scaled score; weights that keep
 // float32's precision through the matrix cores (a weight p goes in as two bfloat16 numbers, p rounded and
 // what the rounding left, in two products); and every query head's weights applied to the values of every kv
-// head (all_v: the grid's second axis is the kv head whose values are read, the sums are written in float32
+// head (all_v: the grid's second axis is a group of VHS kv heads whose values a workgroup reads, four, two in small
+// launches and one where heads are wider than 64 or kv heads few; the sums are written in float32
 // as [token][head][kv head][vd]), from which a following kernel forms heads whose weights are mixtures of
 // the heads' softmax weights.  A window may keep the sequence's first keys: the steps that hold them and lie before the
 // window's come first, and what a step hides is decided key by key.
@@ -76,7 +78,9 @@ struct WideArgs {
 };
 
 // Two maps over rows of up to 128 channels: two workgroups a CU (256 registers a wave) with one step's copies under way are
-// faster than one with two (2,048 tokens, 16 heads of two maps of 64 over values of 128, a window of 1,024: 117 -> 67 us).
+// faster than one with two (2,048 tokens, 16 heads of two maps of 64 over values of 128, a window of 1,024: 117 -> 67 us; with tiles
+// without bank conflicts, places of pages once in sixteen steps and the values' products in the order they have now 59, though nine
+// registers go to scratch memory where two did).
 // The wide form with heads of up to 64 channels: left alone it takes 259 registers, three too many for two workgroups a CU (every
 // head's weights on every kv head's values, 2,048 tokens, 32 heads, 8 kv heads of 64: 870 us, with two 555, since then by VHS).
 // Heads of 96 with one step's copies under way fit two workgroups a CU (2,048 tokens after 16,000, 8 heads: 394 -> 364 us); heads of

@@ -69,7 +69,7 @@ __global__ __launch_bounds__(NT) void gemm_f32_kernel(const float* __restrict__ 
 }
 
 // -------------------------------------------------------------------------------------------- chain
-// A block of Y of WAVES x WAVES waves, T x T tiles of 16x16 each.  K is walked in steps of 32, which go from memory
+// A block of Y of 2 x 2 waves, T x T tiles of 16x16 each.  K is walked in steps of 32, which go from memory
 // straight into LDS, STAGES buffers: the operands of STAGES - 1 steps are under way.  A step
 // of a row is 128 bytes, eight pieces of 16; piece p of row r lies at position p ^ (r % 8), so the rows a fragment read
 // touches spread over the banks.  A wave's load instruction fills 1 KB, eight rows.  For instruction i of a step a lane
@@ -82,7 +82,9 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __
 
 constexpr int STEP = 32;
 
-template <int T, int WAVES, int STAGES>
+constexpr int WAVES = 2;
+
+template <int T, int STAGES>
 __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(const float* __restrict__ X, const float* __restrict__ W,
                                                                               float* __restrict__ Y, int M, int N, int K, int accumulate) {
     constexpr int SIDE = 16 * T * WAVES;                  // rows and columns of the block
@@ -176,7 +178,7 @@ __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(co
     int buf = 0, s = 0;
     for (; s + STAGES - 1 < steps; ++s) {
         wait_loads_and_lds<2 * IN * (STAGES - 2)>();
-        if (WAVES > 1) __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_s_barrier();
         issue(buf == 0 ? STAGES - 1 : buf - 1, s + STAGES - 1);
         products(buf);
         buf = buf + 1 == STAGES ? 0 : buf + 1;
@@ -185,7 +187,7 @@ __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(co
         constexpr int later = STAGES - 2 - decltype(i)::value;
         if (s < steps - later) {
             wait_loads_and_lds<2 * IN * later>();
-            if (WAVES > 1) __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_s_barrier();
             products(buf);
             buf = buf + 1 == STAGES ? 0 : buf + 1;
             ++s;
@@ -218,7 +220,7 @@ __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(co
 // chain sets the pace, one matrix instruction after the other (33 cycles each with nothing between them): the operands of a
 // whole step (eight instructions) are read from LDS into one of two register sets while the other is multiplied, and all reads
 // are waited for at once, where they have long arrived, so that no product waits for LDS (the kernel above, half a step ahead:
-// 2,048 x 8,192 of 16 rows 58 us, this one 49; 65,536 x 2,048 of 4 rows 107 and 102, 5.3 TB/s).  Rows beyond X are not
+// 2,048 x 8,192 of 16 rows 58 us, this one 49; 65,536 x 2,048 of 8 rows 113 and 109, 4.9 TB/s).  Rows beyond X are not
 // fetched.  STAGES: steps of 32 k in LDS, 16 where two workgroups fill a CU's share of the launch anyway.
 template <int STAGES>
 __global__ __launch_bounds__(WAVE) void gemm_f32_rows_kernel(const float* __restrict__ X, const float* __restrict__ W,
@@ -327,7 +329,9 @@ __global__ __launch_bounds__(WAVE) void gemm_f32_rows_kernel(const float* __rest
 // column.  A fused multiply-add waits 6 cycles for the one before it, four of them 24, where a matrix instruction of four k
 // takes 33 and in a loop with its reads 50: where nothing but the chain's length counts, this is the shorter one.  A lone wave
 // issues an instruction in five cycles, so the loop holds next to nothing but the chain, its reads and loads: places in LDS are
-// constants.  4 rows, 2,048 x 8,192: 35 us (rows kernel 49), 2,048 x 2,048: 10.6 (13.9), 6,144 x 2,048: 12.4 (15.7).
+// constants.  4 rows, 2,048 x 8,192: 35 us (rows kernel 49), 2,048 x 2,048: 10.6 (13.9), 6,144 x 2,048: 12.4 (15.7).  What bounds
+// it: the chain alone would take 6 cycles a k, 21 us of those 35; reads, loads and their counters, issued between by the same
+// wave, are the rest.
 // K in steps of 64: X rows of 256 bytes, piece p (16 bytes) of row g at p ^ 4 g; W rows of 256 bytes, piece p of column c at p ^ c.
 __device__ __forceinline__ void chain16(float& acc, float x, const f32x4 (&w)[4]) {
 #ifdef __HIP_DEVICE_COMPILE__
@@ -471,13 +475,13 @@ int launch_rows(const float* X, const float* W, float* Y, int M, int N, int K, i
     return launch_status();
 }
 
-template <int T, int WAVES, int STAGES>
+template <int T, int STAGES>
 int launch_chain(const float* X, const float* W, float* Y, int M, int N, int K, int accumulate, hipStream_t stream) {
     constexpr int side = 16 * T * WAVES, lds = STAGES * side * STEP * 2 * (int)sizeof(float);
     static_assert(lds <= 65536, "without asking for more");
     dim3 grid(ceil_div(N, side), ceil_div(M, side));
     if (grid.y > 65535) return -2;
-    hipLaunchKernelGGL((gemm_f32_chain_kernel<T, WAVES, STAGES>), grid, dim3(WAVES * WAVES * WAVE), lds, stream, X, W, Y, M, N, K, accumulate);
+    hipLaunchKernelGGL((gemm_f32_chain_kernel<T, STAGES>), grid, dim3(WAVES * WAVES * WAVE), lds, stream, X, W, Y, M, N, K, accumulate);
     return launch_status();
 }
 }  // namespace
@@ -509,6 +513,6 @@ TUFF_EXPORT int tuff_gemm_f32(const float* X, const float* W, float* Y, int M, i
     }
     constexpr int MOST_BLOCKS = 65535;                    // of rows in a grid
     if (ceil_div(M, 32) <= MOST_BLOCKS && block_cycles(M, N, 32) < block_cycles(M, N, 64))
-        return launch_chain<1, 2, 4>(X, W, Y, M, N, K, accumulate, stream);
-    return launch_chain<2, 2, 4>(X, W, Y, M, N, K, accumulate, stream);
+        return launch_chain<1, 4>(X, W, Y, M, N, K, accumulate, stream);
+    return launch_chain<2, 4>(X, W, Y, M, N, K, accumulate, stream);
 }
