@@ -336,11 +336,13 @@ def test_prompt_kernel_with_the_values_of_several_kv_heads_a_workgroup(gpu, H, H
         assert (got - want).abs().max() <= 3e-5 * max(1.0, float(want.abs().max())), opts
 
 
-@pytest.mark.parametrize("H, Hkv, hd, vd, ps", [(32, 8, 64, 64, 16), (8, 8, 64, 64, 48), (10, 5, 64, 24, 16), (6, 6, 16, 32, 32), (12, 3, 40, 64, 80)])
+@pytest.mark.parametrize("H, Hkv, hd, vd, ps", [(32, 8, 64, 64, 16), (8, 8, 64, 64, 48), (10, 5, 64, 24, 16), (6, 6, 16, 32, 32), (12, 3, 40, 64, 80),
+                                                (10, 5, 32, 32, 16)])
 def test_long_requests_of_mixed_heads_have_the_same_bits_alone_and_in_company(gpu, H, Hkv, hd, vd, ps):
     """A portion alone is a launch of few workgroups, which take two kv heads each; among many short requests the same portion goes
     through the kernel that takes four.  Whole blocks of 128 columns over more than 1,024 and 2,048 keys (the places of pages are worked
-    out for 1,024 at a time), with windows that reach into the portion and beyond; beside the general kernel to float32's rounding."""
+    out for 1,024 at a time), with windows that reach into the portion and beyond; beside the general kernel to float32's rounding.
+    (Heads of at most 32 channels stay by themselves in the small launches, and where four would leave places empty.)"""
     from tuff_amd.csrc import ops
     long = [(1500, 200), (2040, 130), (0, 250)]
     reqs = [(5 + i % 40, 1) for i in range(40)] + long + [(i, 1) for i in range(24)]

@@ -694,18 +694,25 @@ TUFF_EXPORT int tuff_attention_prefill_wide(const void* q, const void* k_cache, 
         if (slopes) return log_r1 ? go(number<SLOPES | LOG_DIST>()) : go(number<SLOPES>());
         return log_r1 ? go(number<LOG_DIST>()) : go(number<NO_BIAS>());
     };
-    // Several kv heads' values a workgroup from three kv heads on (from four where heads have at most 32 channels: the tiles are 64
-    // wide; 2,048 tokens, 12 heads on 3 kv heads of 32: 97 us in one-head workgroups, 102 in this; 16 on 4 of 16: 170, 96).  Four,
-    // but two where that gives no CU more than one workgroup: then a block's steps one after the other are all there is (100
-    // tokens, 32 heads on 8 kv heads of 64: one 13.9 us, four 14.6, two 11.6; 400 of 16 on 4: 28.4, 24.7 and 19.9; 400 of 32 on 8,
-    // 416 workgroups of two: 55.7, 27.9 and 32.4).
+    // Several kv heads' values a workgroup from three kv heads on.  Four, but two where that gives no CU more than one workgroup: then a
+    // block's steps one after the other are all there is (100 tokens, 32 heads on 8 kv heads of 64: one 13.9 us, four 14.6, two 11.6;
+    // 400 of 16 on 4: 28.4, 24.7 and 19.9; 400 of 32 on 8, 416 workgroups of two: 55.7, 27.9 and 32.4).
+    // Heads of at most 32 channels have tiles of half the width by themselves, and without the logarithmic penalty little to share.
+    // From four kv heads on, not where a CU has one workgroup anyway (4 on 4, 2,048 tokens after 8,000: one 182 us, two 278), and four
+    // only where their places are less than five quarters of the kv heads, with the logarithmic penalty at most four thirds (32
+    // channels, 2,048 tokens after 8,000 or 1,024 after 3,000, one and four: 32 on 4 814 and 734 us, 20 on 5 696 and 1,078, with the
+    // penalty 1,053 and 1,296; 24 on 6 907 and 1,109, 1,367 and 1,328; 28 on 7 2,048 tokens 193 and 188, 274 and 218).
     if (all_v && widest <= 64 && Hkv > (widest <= 32 ? 3 : 2)) {
-        if ((long long)n_qblocks * Hkv * ceil_div(Hkv, 2) <= 256) {
+        const long long one = (long long)n_qblocks * Hkv * Hkv, two = (long long)n_qblocks * Hkv * ceil_div(Hkv, 2);
+        const int places = ceil_div(Hkv, 4) * 4;
+        if (two <= 256 && (widest > 32 || one > 256)) {
             grid.y = ceil_div(Hkv, 2);
             return narrow(number<64>(), number<1>(), number<1>(), number<2>(), number<8>());
         }
-        grid.y = ceil_div(Hkv, 4);
-        return narrow(number<64>(), number<1>(), number<1>(), number<4>(), number<8>());
+        if (widest > 32 || (one > 256 && (log_r1 ? places * 3 <= Hkv * 4 : places * 4 < Hkv * 5))) {
+            grid.y = ceil_div(Hkv, 4);
+            return narrow(number<64>(), number<1>(), number<1>(), number<4>(), number<8>());
+        }
     }
     if (widest <= 32) return narrow(number<32>(), number<1>(), number<2>(), number<1>(), number<4>());
     if (widest <= 64) return narrow(number<64>(), number<1>(), number<2>(), number<1>(), number<4>());
