@@ -886,6 +886,51 @@ def test_attention_of_single_tokens_is_the_same_with_one_wave_or_four_a_partitio
         assert torch.isfinite(many).all() and torch.equal(few, many[:3]), f"fused={fused}"
 
 
+@pytest.mark.parametrize("H,Hkv,hd,ps", [(32, 8, 64, 16), (24, 8, 64, 16), (64, 8, 64, 48), (128, 8, 64, 16), (16, 8, 40, 16), (24, 8, 56, 64)])
+@pytest.mark.parametrize("window", [0, 300])
+@pytest.mark.parametrize("parts", [4, 8])
+def test_attention_of_single_tokens_by_a_workgroup_a_kv_head(gpu, H, Hkv, hd, ps, window, parts):
+    """Many requests of few partitions: a workgroup takes all keys of its columns and finishes them.  The same bits as from
+    partitions and their merge, which room for more keys than there are asks for; the step's keys and values written as there;
+    stale pages hold NaN, pages that a window has left are -1.  Lengths at the edges of steps, units, turns and partitions."""
+    from tuff_amd.csrc import ops
+    edges = [1, 16, 17, 32, 33, 64, 65, 255, 256, 257, 511, 513, 545, 769, 1000, 1024] + ([1025, 1057, 1537, 1999, 2047, 2048] if parts == 8 else [])
+    lens = (edges * 3)[:8 if parts == 4 else 22] if hd == 64 else (edges[::-1] * 3)[:8 if parts == 4 else 22]
+    lens[0] = parts * 256
+    R = len(lens)
+    assert R * Hkv >= (64 if parts == 4 else 176)
+    hd_args = dict(H=H, Hkv=Hkv, page_size=ps, window=window)
+    sinks, slopes = _r(H, seed=8).float().to(gpu), (2.0 ** -torch.arange(1, H + 1).float() / 8).to(gpu)
+    inv_freq = (1e6 ** (-2 * torch.arange(32, dtype=torch.float64) / 64)).float().to(gpu)
+    qw = (1 + _r(64, seed=5, scale=0.1)).to(gpu)
+    ways = []
+    for room in (parts * 256, 4096):
+        case = _mixed_step_case(gpu, [(n - 1, 1) for n in lens], H, Hkv, hd, ps)
+        width = -(-4096 // ps)
+        table = torch.full((R, width), -1, dtype=torch.int32, device=gpu)
+        table[:, :case["table"].shape[1]] = case["table"]
+        if window:
+            for r, n in enumerate(lens):
+                table[r, :max(0, n - window) // ps] = -1
+        common = dict(block_table=table, req_info=case["req_info"], positions=case["positions"], max_ctx_len=room, **hd_args)
+        got = []
+        for extra in (dict(), dict(sinks=sinks), dict(slopes=slopes)):
+            out = torch.full((R, H * hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+            ops.attention_mfma(case["q"].to(gpu), case["kc"], case["vc"], out, blocks=None, nb=1, hd=hd, **extra, **common)
+            got.append(out.float().cpu())
+        _check_step(case, [(n - 1, 1) for n in lens], got[0].double().reshape(R, H, hd), H, hd, window, room)
+        if hd == 64:
+            slots = torch.tensor([int(table[r, (n - 1) // ps]) * ps + (n - 1) % ps for r, n in enumerate(lens)], dtype=torch.int32, device=gpu)
+            qkv = _r(R, (H + 2 * Hkv) * 64, seed=3, dtype=torch.bfloat16).to(gpu)
+            for angles in (None, ops.rope_table(inv_freq, 600)):
+                out = torch.full((R, H * hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+                ops.attention_decode_fused(qkv, case["kc"], case["vc"], out, inv_freq=inv_freq, slot_mapping=slots, q_norm_w=qw, k_norm_w=qw,
+                                           eps=1e-5, angles=angles, **common)
+                got += [out.float().cpu(), torch.nan_to_num(case["kc"].float(), nan=1e9).cpu(), torch.nan_to_num(case["vc"].float(), nan=1e9).cpu()]
+        ways.append(got)
+    assert all(torch.isfinite(a).all() and torch.equal(a, b) for a, b in zip(*ways))
+
+
 @pytest.mark.parametrize("H,Hkv", [(32, 8), (6, 3), (5, 5), (16, 1)])
 def test_attention_of_single_tokens_does_not_depend_on_the_order_of_its_workgroups(gpu, H, Hkv):
     """Large launches number their workgroups with the kv head changing fastest, small ones with the

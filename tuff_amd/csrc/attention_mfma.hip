@@ -8,7 +8,8 @@
 // where that would leave the chip idle, four waves with a unit each.  Either way a unit starts from
 // a fresh state and the units' results (running maximum m, sum l, unnormalised output o, float32)
 // are merged in ascending order through one chain of operations, so both give the same bits.  A
-// second kernel merges a token's partitions in ascending order.  Since the columns of a matrix product do not influence each
+// second kernel merges a token's partitions in ascending order.  Where column blocks are many and partitions few, a
+// workgroup of eight waves takes all of a block's partitions and does that itself, in the same order.  Since the columns of a matrix product do not influence each
 // other, a token's result does not depend on how the sequence was cut into steps or on what
 // else was in the batch.
 //
@@ -20,7 +21,7 @@
 //    and exp these eight values are, as they lie, the lane's part of the B operand P^T of the
 //    second product (k = 8g + i), and the A operand V^T is one 16-byte load of eight consecutive
 //    positions of a channel from the transposed V page.
-//  * No LDS, no transposes, no barriers; K rows and V columns of the next step are loaded
+//  * No transposes, no barriers, LDS only for K rows on their way; K rows and V columns of the next step are loaded
 //    while the current step computes, with streaming (non-temporal) loads: a step of single tokens
 //    reads every key once.
 //
@@ -74,6 +75,49 @@ __device__ __forceinline__ float norm_weight(const void* w, int dt, int i) {
     return dt == DT_F32 ? ((const float*)w)[i] : (float)((const bf16_t*)w)[i];
 }
 
+// The same for N neighbours from j (i) on, a multiple of N: whole pieces at a time, one branch.
+typedef f32x4 f32x4_any __attribute__((aligned(4)));       // (tables and weights may start anywhere)
+typedef bf16x4 bf16x4_any __attribute__((aligned(2)));
+template <int N>
+__device__ __forceinline__ void angles(const FusedQKV& fq, int pos, int j, float (&rc)[N], float (&rs)[N]) {
+    if (pos < fq.n_angles) {
+        const float* at = fq.angles + (long long)pos * 64 + j;
+#pragma unroll
+        for (int e = 0; e < N; e += 4) {
+            const f32x4 c = *(const f32x4_any*)(at + e), s = *(const f32x4_any*)(at + 32 + e);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { rc[e + i] = c[i]; rs[e + i] = s[i]; }
+        }
+    } else {
+#pragma nounroll
+        for (int e = 0; e < N; ++e) {
+            float c, s;
+            angle(fq, pos, j + e, c, s);
+#pragma unroll
+            for (int i = 0; i < N; ++i) { rc[i] = i == e ? c : rc[i]; rs[i] = i == e ? s : rs[i]; }
+        }
+    }
+}
+
+template <int N>
+__device__ __forceinline__ void norm_weights(const void* w, int dt, int i, float (&out)[N]) {
+    if (dt == DT_F32) {
+#pragma unroll
+        for (int e = 0; e < N; e += 4) {
+            const f32x4 x = *(const f32x4_any*)((const float*)w + i + e);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) out[e + k] = x[k];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < N; e += 4) {
+            const bf16x4 x = *(const bf16x4_any*)((const bf16_t*)w + i + e);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) out[e + k] = (float)x[k];
+        }
+    }
+}
+
 // One partial result (m, l, o) merged into a running one, element by element:
 //   m' = max(m, mu);  l' = l e^(m - m') + lu e^(mu - m');  o' likewise.
 // Both forms of the kernel (one wave or four a partition) merge a partition's four units of 64 keys
@@ -89,6 +133,12 @@ __device__ __forceinline__ void merge_weights(float m, float mu, float& m_new, f
 // instantiations of the kernel may fuse the other product and differ in the last bit
 __device__ __forceinline__ float merged(float a, float ca, float b, float cb) { return fmaf(b, cb, a * ca); }
 
+// a b rounded, whatever is taken from it afterwards
+__device__ __forceinline__ float product(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
+
 constexpr int UNIT = 64;                   // keys a unit: two steps of 32
 constexpr int UNITS = PART / UNIT;
 
@@ -99,82 +149,105 @@ __host__ __device__ inline int partition_pages(int key_begin, int page_size) {
     return (key_begin + PART - 1) / page_size - key_begin / page_size + 1;
 }
 
-// NW: waves a workgroup (1: the wave walks the partition's four units; 4: a unit a wave, merged through LDS).
+// NW: waves a workgroup (1: the wave walks the partition's four units; 4: a unit a wave, merged through LDS; more: the workgroup
+// takes all partitions of its column block, its waves the units in turn, merges them and writes the finished rows, no kernel after it).
 template <int HDP, int NB, int NW, bool FUSED, bool STREAM_V, bool STAGE_K = false>
 __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     const bf16_t* __restrict__ q, bf16_t* __restrict__ k_cache, bf16_t* __restrict__ v_cache,
     float* __restrict__ ws_o, float* __restrict__ ws_ml,
     const int* __restrict__ block_table, int max_blocks,
     const int2* __restrict__ blk, const int4* __restrict__ req_info,
-    int H, int Hkv, int hd, int page_size, int window, float scale, int n_parts, FusedQKV fq, int kv_fast) {
-    static_assert(NW == 1 || NW == UNITS, "one wave a partition or one a unit");
+    int H, int Hkv, int hd, int page_size, int window, float scale, int n_parts, FusedQKV fq, int kv_fast,
+    bf16_t* __restrict__ out, const float* __restrict__ sinks) {
+    constexpr bool WHOLE = NW > UNITS;     // out and sinks are this form's; ws_o and ws_ml the others'
+    static_assert(NW == 1 || NW % UNITS == 0, "one wave a partition, one a unit, or whole partitions side by side");
+    static_assert(!WHOLE || (HDP == 64 && NB == 1), "all partitions a workgroup: heads of up to 64 and one column block");
     static_assert(!FUSED || (HDP == 64 && NB == 1), "the fused form is for heads of 64 and one column block");
     constexpr int KC = HDP / 32;          // 32-wide chunks of the head dimension
     constexpr int DB = HDP / 16;          // 16-wide blocks of output channels
+    const int ps = STREAM_V ? 16 : page_size;              // (STREAM_V: pages of sixteen; what is divided by them is shifted)
+    const int HD = FUSED ? 64 : hd;
     // Workgroups that run side by side read neighbouring memory when the kv head is what changes fastest
     // from one to the next (a page holds its kv heads one after the other): that order for launches of
     // several rounds of waves, partitions first for the others.
-    const int part = kv_fast ? blockIdx.x / Hkv : blockIdx.x, qb = blockIdx.y, kvh = kv_fast ? blockIdx.x % Hkv : blockIdx.z;
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE, n16 = lane % 16, g = lane / 16;
+    const int part = WHOLE ? 0 : kv_fast ? blockIdx.x / Hkv : blockIdx.x, qb = blockIdx.y, kvh = kv_fast ? blockIdx.x % Hkv : blockIdx.z;
+    const int lane = threadIdx.x % WAVE, n16 = lane % 16, g = lane / 16;
+    const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int G = H / Hkv;
-    // Every load that depends on another costs a trip to memory, so the chain is kept short:
-    // block -> request record (start, length, first position: a portion's positions are
-    // consecutive) -> the partition's page numbers, all at once -> keys and values.
+    // Every load that depends on another costs a trip to memory, so the chain is kept short: block -> request record (start,
+    // length, first position: a portion's positions are consecutive), and beside it the page numbers, all at once -> keys and
+    // values.
     int r = qb, col0 = 0;                  // without a block list every request is one block
     if (blk) { const int2 b = blk[qb]; r = b.x; col0 = b.y; }
     const int4 info = req_info[r];         // (first token of the request in the step, tokens, first position, -)
-    const int t0 = info.x, ncols = info.y * G, pos0 = info.z;
     const int* table = block_table + (long long)r * max_blocks;
-    const int key_begin = part * PART;
-    const int first_page = key_begin / page_size;
-    int my_page = -1;                      // lane i: the page of the partition's i-th block of page_size keys
-    if (lane < partition_pages(key_begin, page_size) && first_page + lane < max_blocks) my_page = table[first_page + lane];
-
+    const int t0 = info.x, ncols = info.y * G, pos0 = info.z;
     // the block's range of keys
     const int last_col = min(ncols, col0 + NB * 16) - 1;
     const int pos_max = pos0 + last_col / G;
     const int lo_min = window > 0 ? max(0, pos0 + col0 / G - window + 1) : 0;
-    if (key_begin > pos_max || key_begin + PART <= lo_min) return;
-    const int key_end = min(key_begin + PART, pos_max + 1);
+    const int key_begin = WHOLE ? lo_min / PART * PART : part * PART;
+    const int first_page = key_begin / ps;
+    int my_page = 0;                       // lane i: the page of the partition's i-th block of page_size keys
+    if constexpr (WHOLE) {
+        // lane 8 j + i: the page of the i-th such block of the wave's unit of turn j (a unit touches at most four)
+        const int block = (key_begin + (lane / 8 * NW + wave) * UNIT) / ps + lane % 8;
+        if (block < max_blocks) my_page = table[block];
+    } else {
+        if (lane < partition_pages(key_begin, ps) && first_page + lane < max_blocks) my_page = table[first_page + lane];
+        if (key_begin > pos_max || key_begin + PART <= lo_min) return;
+    }
+    const int key_end = WHOLE ? pos_max + 1 : min(key_begin + PART, pos_max + 1);
 
+    // (of the whole form, the wave that reads the token's key writes it)
+    auto write_token = [&]() {
+        const long long slot = fq.slot_mapping[t0];
+        if (slot >= 0) {
+            const long long page = slot / ps, off = slot % ps;
+            const int row_width = (H + 2 * Hkv) * 64;
+            const bf16_t* row = q + (long long)t0 * row_width;
+            const int l = lane % 16;
+            const bf16_t value = row[(H + Hkv + kvh) * 64 + lane];
+            const bf16x4 raw = *(const bf16x4*)(row + (H + kvh) * 64 + 4 * l);
+            float rc[4], rs[4], nw[4] = {};
+            if (fq.k_norm_w != nullptr) norm_weights<4>(fq.k_norm_w, fq.norm_dt, 4 * l, nw);
+            angles<4>(fq, pos0, (4 * l) & 31, rc, rs);
+            // value: lane = channel, as projected
+            v_cache[((page * Hkv + kvh) * 64 + lane) * ps + off] = value;
+            // key: sixteen lanes hold four channels each (the other lanes do the same work again)
+            float v[4] = {(float)raw[0], (float)raw[1], (float)raw[2], (float)raw[3]};
+            float ss = v[0] * v[0];
+            ss = fmaf(v[1], v[1], ss);
+            ss = fmaf(v[2], v[2], ss);
+            ss = fmaf(v[3], v[3], ss);
+            ss = row_sum_down(ss);
+            if (fq.k_norm_w != nullptr) {
+                const float inv = 1.0f / sqrtf(ss / 64.0f + fq.eps);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = v[e] * inv * nw[e];
+            }
+            const bool first = l < 8;
+            bf16x4 o4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float other = lane_xor8(v[e]);
+                const float x0 = first ? v[e] : other, x1 = first ? other : v[e];
+                o4[e] = (bf16_t)(first ? (x0 * rc[e] - x1 * rs[e]) : (x0 * rs[e] + x1 * rc[e]));
+            }
+            if (lane < 16) *(bf16x4*)(k_cache + ((page * Hkv + kvh) * ps + off) * 64 + 4 * l) = o4;
+        }
+    };
     if constexpr (FUSED) {
         // the token's key and value go into the cache before anybody reads the partition that holds them
-        if (fq.slot_mapping != nullptr && pos0 / PART == part) {
-            if (wave == 0) {
-                const long long slot = fq.slot_mapping[t0];
-                if (slot >= 0) {
-                    const long long page = slot / page_size, off = slot % page_size;
-                    const int row_width = (H + 2 * Hkv) * 64;
-                    const bf16_t* row = q + (long long)t0 * row_width;
-                    // value: lane = channel, as projected
-                    v_cache[((page * Hkv + kvh) * 64 + lane) * page_size + off] = row[(H + Hkv + kvh) * 64 + lane];
-                    // key: sixteen lanes hold four channels each (the other lanes do the same work again)
-                    const int l = lane % 16;
-                    const bf16x4 raw = *(const bf16x4*)(row + (H + kvh) * 64 + 4 * l);
-                    float v[4] = {(float)raw[0], (float)raw[1], (float)raw[2], (float)raw[3]};
-                    float ss = v[0] * v[0];
-                    ss = fmaf(v[1], v[1], ss);
-                    ss = fmaf(v[2], v[2], ss);
-                    ss = fmaf(v[3], v[3], ss);
-                    ss = row_sum_down(ss);
-                    if (fq.k_norm_w != nullptr) {
-                        const float inv = 1.0f / sqrtf(ss / 64.0f + fq.eps);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) v[e] = v[e] * inv * norm_weight(fq.k_norm_w, fq.norm_dt, 4 * l + e);
-                    }
-                    const bool first = l < 8;
-                    bf16x4 o4;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float rc, rs;
-                        angle(fq, pos0, (4 * l + e) & 31, rc, rs);
-                        const float other = lane_xor8(v[e]);
-                        const float x0 = first ? v[e] : other, x1 = first ? other : v[e];
-                        o4[e] = (bf16_t)(first ? (x0 * rc - x1 * rs) : (x0 * rs + x1 * rc));
-                    }
-                    if (lane < 16) *(bf16x4*)(k_cache + ((page * Hkv + kvh) * page_size + off) * 64 + 4 * l) = o4;
-                }
+        if constexpr (WHOLE) {
+            if (fq.slot_mapping != nullptr && wave == (pos0 - key_begin) / UNIT % NW) {
+                write_token();
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");      // for the other lanes of this wave, which reads them
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
             }
+        } else if (fq.slot_mapping != nullptr && pos0 / PART == part) {
+            if (wave == 0) write_token();
             __syncthreads();               // the stores have landed before a wave of this workgroup loads the keys
         }
     }
@@ -198,90 +271,107 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     // the second product's operands hold for k = 8g + i.  A step's K rows and V columns are loaded
     // into registers a step ahead of their use (where the head size leaves room for it); large
     // tiles (head size x columns) load as they go.
+    //
+    // What bounds it: a wave issues an instruction in about five cycles, so with three or four waves a SIMD the instructions
+    // around the loads and products count as much as the bytes.  Hence no branch but those a whole wave takes, every lane loads
+    // from a page that holds keys of the request whatever its own are, only steps at an end of the keys look at single keys,
+    // and pages of sixteen (STREAM_V) are shifted, not divided: a step of 32 keys in some 170 instructions instead of 670.  One
+    // layer's attention, 32 heads on 8: 64 requests of 8,192 keys 201 -> 184 us (5.8 TB/s), 8 of 8,192 29.7 -> 25, one of 256
+    // 8.6 -> 6.4; heads of 128, 32 requests of 4,000 116 -> 95, of 256 (16 on 4) 107 -> 98.
     constexpr bool AHEAD = HDP * NB <= 256;
     // STAGE_K (heads of up to 64 channels): a step's keys are asked for as they lie in memory, 1 KB an instruction (the
     // 16 keys of a half are one run of 16 hd elements), and go through LDS into the order of the matrix operands.  Asked
     // for in that order at once, an instruction touches half of each of sixteen lines and every line is asked for twice:
-    // with several rounds of waves on the chip the memory side is what bounds the kernel, and whole lines are 3 to 7 %
-    // faster (16,384 workgroups; nothing at 6,144); with one round the trip through LDS only adds to each wave's chain
-    // (3 to 7 % slower), so the launch chooses.
-    static_assert(!STAGE_K || (HDP == 64 && HDP * NB <= 256 && NW == 1), "staged keys: heads of up to 64, one wave a partition");
+    // whole lines are 2 to 6 % of a decode step faster wherever waves walk a partition by themselves.
+    static_assert(!STAGE_K || (HDP == 64 && HDP * NB <= 256 && NW != UNITS), "staged keys: heads of up to 64, not with a unit a wave");
     constexpr bool STAGE = STAGE_K;
     __shared__ __attribute__((aligned(16))) bf16_t k_stage[STAGE ? NW : 1][STAGE ? 32 * 64 : 8];
     // where the 16-byte piece `chunk` of key `key` of the step lies in the wave's 4 KB: rows of 128 bytes, the pieces of
     // a row exchanged so that the sixteen rows an operand read takes its pieces from fall into different banks
     auto stage_at = [&](int key, int chunk) { return key * 64 + ((chunk ^ (((key >> 1) & 1) | (((key >> 3) & 3) << 1))) * 8); };
-    const int row_pieces = hd / 8;                                   // 16-byte pieces of a key
+    const int row_pieces = HD / 8;                                   // 16-byte pieces of a key
     int stage_to[2][2];                                              // where this lane's four pieces of a step go (-1: no piece)
+    if constexpr (STAGE) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int piece = 64 * i + lane;
-            stage_to[h][i] = (STAGE && piece < 16 * row_pieces) ? stage_at(16 * h + piece / row_pieces, piece % row_pieces) : -1;
-        }
+            for (int i = 0; i < 2; ++i) {
+                const int piece = 64 * i + lane;
+                stage_to[h][i] = piece < 16 * row_pieces ? stage_at(16 * h + piece / row_pieces, piece % row_pieces) : -1;
+            }
+    }
     struct Tile {
         bf16x8 kf[2][AHEAD ? KC : 1];
         bf16x8 vx[AHEAD ? DB : 1];
-        long long base[2];                 // per half: (page, kv head) start in both caches
-        int off0[2];                       // per half: offset of its first key in the page
-        bool live[2];                      // per half: holds keys some column may see
+        const bf16_t *k_at, *v_at;         // (not AHEAD) where this lane's parts of the keys and values begin
     };
-    const int k_half = n16 / 8;                                    // half of this lane's K rows
-    const int k_off = 8 * ((n16 / 4) % 2) + n16 % 4;               // + 4 kb: offset of the row's key in its half
-    auto k_frag = [&](const Tile& t, int kb, int kc) {
+    const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    const bool narrow = HD < HDP;          // channels beyond the head: its first key channel (the query has zero there), its first
+                                           // value channel (whose result nobody takes)
+    using place_t = std::conditional_t<STREAM_V, unsigned, unsigned long long>;        // (pages of sixteen: 32 bits hold any place in one)
+    const place_t page_elems = (place_t)Hkv * ps * HD;
+    // this lane's place in a half's keys and values: key 8 ((n16 / 4) % 2) + n16 % 4 (+ 4 kb) of half n16 / 8; channel n16
+    // (+ 16 db), positions 8 (g % 2) of half g / 2
+    const bf16_t* const k_mine = k_cache + (long long)kvh * ps * HD + (8 * ((n16 / 4) % 2) + n16 % 4) * HD;
+    const bf16_t* const v_mine = v_cache + (long long)kvh * ps * HD + (g % 2) * 8;
+    auto k_frag = [&](const bf16_t* at, int kb, int kc) {
         const int k = kc * 32 + g * 8;
-        bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-        // selects, not indexing by a lane-dependent value (that would put the arrays in scratch memory)
-        const bool live = k_half ? t.live[1] : t.live[0];
-        const long long base = k_half ? t.base[1] : t.base[0];
-        const int off0 = k_half ? t.off0[1] : t.off0[0];
-        if (!live || k >= hd) return z;
-        return __builtin_nontemporal_load((const bf16x8*)(k_cache + base + (long long)(off0 + k_off + 4 * kb) * hd + k));
+        return __builtin_nontemporal_load((const bf16x8*)(at + 4 * kb * HD + (!narrow || k < HD ? k : 0)));
     };
     // A page's V^T rows are 2 * page_size bytes: with pages of 16 positions a step of 32 keys reads whole rows and
     // never comes back to them; with larger pages it reads a part of each row's cache lines and the steps after it
     // read the rest, so those loads are ordinary ones (a line asked for as streaming does not wait for them):
-    // STREAM_V is page_size <= 16.
-    auto v_frag = [&](const Tile& t, int db) {
+    // STREAM_V is page_size == 16.
+    auto v_frag = [&](const bf16_t* at, int db) {
         const int dim = db * 16 + n16;
-        bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-        const bool live = (g / 2) ? t.live[1] : t.live[0];
-        const long long base = (g / 2) ? t.base[1] : t.base[0];
-        const int off0 = (g / 2) ? t.off0[1] : t.off0[0];
-        if (!live || dim >= hd) return z;
-        const bf16x8* at = (const bf16x8*)(v_cache + base + (long long)dim * page_size + off0 + (g % 2) * 8);
-        if constexpr (STREAM_V) return __builtin_nontemporal_load(at); else return *at;
+        const bf16x8* from = (const bf16x8*)(at + (place_t)(!narrow || dim < HD ? dim : 0) * ps);
+        if constexpr (STREAM_V) return __builtin_nontemporal_load(from); else return *from;
+    };
+    // the page that holds block `block` of page_size keys; key: one of the step's
+    auto page_of = [&](int block, int key) {
+        int holder = block - first_page;
+        if constexpr (WHOLE) {
+            const int unit = (key - key_begin) / UNIT;
+            holder = unit / NW * 8 + block - (key_begin + unit * UNIT) / ps;
+        }
+        return (unsigned)__builtin_amdgcn_readlane(my_page, holder & (WAVE - 1));
     };
     auto load_tile = [&](int key0, Tile& t) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int hs = key0 + h * 16;
-            t.live[h] = hs <= pos_max && hs + 15 >= lo_min;
-            const long long page = t.live[h] ? __shfl(my_page, hs / page_size - first_page, WAVE) : 0;
-            t.off0[h] = hs % page_size;
-            t.base[h] = (page * Hkv + kvh) * (long long)page_size * hd;
-        }
+        // a half without a key that some column may see: the other half's keys in its place (their weights are zero), and
+        // where both are, the first page's (the cache's own first one where that is no longer held)
+        const bool live0 = key0 <= pos_max && key0 + 15 >= lo_min, live1 = key0 + 16 <= pos_max && key0 + 31 >= lo_min;
+        const int h0 = live0 ? key0 : key0 + 16, h1 = live1 ? key0 + 16 : key0;
+        const bool any = live0 || live1;
+        const unsigned at0 = page_of(h0 / ps, key0), at1 = page_of(h1 / ps, key0);
+        const unsigned none = max(__builtin_amdgcn_readlane(my_page, 0), 0);
+        const unsigned p0 = any ? at0 : none, p1 = any ? at1 : none;
+        const int off0 = any ? h0 % ps : 0, off1 = any ? h1 % ps : 0;      // multiples of 16
         if constexpr (STAGE) {
             // kf[h][i]: pieces 64 i + lane of half h, as they lie in memory
+            const bf16_t* const at[2] = {k_cache + ((unsigned long long)p0 * page_elems + ((place_t)kvh * ps + off0) * HD),
+                                         k_cache + ((unsigned long long)p1 * page_elems + ((place_t)kvh * ps + off1) * HD)};
 #pragma unroll
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     const int piece = 64 * i + lane;
-                    bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-                    t.kf[h][i] = (t.live[h] && stage_to[h][i] >= 0)
-                        ? __builtin_nontemporal_load((const bf16x8*)(k_cache + t.base[h] + (long long)t.off0[h] * hd + piece * 8)) : z;
+                    t.kf[h][i] = __builtin_nontemporal_load((const bf16x8*)(at[h] + (!narrow || piece < 16 * row_pieces ? piece : 0) * 8));
                 }
+        }
+        const bf16_t* const v_at = v_mine + ((unsigned long long)(g / 2 ? p1 : p0) * page_elems + (place_t)(g / 2 ? off1 : off0));
+        if constexpr (AHEAD) {
+            if constexpr (!STAGE) {
+                const bf16_t* const k_at = k_mine + ((unsigned long long)(n16 / 8 ? p1 : p0) * page_elems + (place_t)(n16 / 8 ? off1 : off0) * HD);
 #pragma unroll
-            for (int db = 0; db < DB; ++db) t.vx[db] = v_frag(t, db);
-        } else if constexpr (AHEAD) {
+                for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
+                    for (int kc = 0; kc < KC; ++kc) t.kf[kb][kc] = k_frag(k_at, kb, kc);
+            }
 #pragma unroll
-                for (int kc = 0; kc < KC; ++kc) t.kf[kb][kc] = k_frag(t, kb, kc);
-#pragma unroll
-            for (int db = 0; db < DB; ++db) t.vx[db] = v_frag(t, db);
+            for (int db = 0; db < DB; ++db) t.vx[db] = v_frag(v_at, db);
+        } else {
+            t.k_at = k_mine + ((unsigned long long)(n16 / 8 ? p1 : p0) * page_elems + (place_t)(n16 / 8 ? off1 : off0) * HD);
+            t.v_at = v_at;
         }
     };
     // The first keys and values are asked for before the queries are prepared: they depend on the page
@@ -290,31 +380,43 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     Tile ta, tb;
     const int key_first = NW == 1 ? key_begin : key_begin + wave * UNIT;
     if constexpr (AHEAD) {
-        if (key_first < key_end) load_tile(key_first, ta);
-        if (NW > 1 && key_first + 32 < key_end) load_tile(key_first + 32, tb);
+        if (NW == 1 || key_first < key_end) {
+            load_tile(key_first, ta);
+            if (NW > 1 && !WHOLE) load_tile(key_first + 32, tb);
+        }
     }
 
     // this lane's columns
     int pos_c[NB], lo_c[NB];
     float slope_c[NB];
-    const bool has_slopes = fq.slopes != nullptr;
+    const bool has_slopes = !FUSED && fq.slopes != nullptr;
     long long qrow[NB];                    // row of the column in the work space; -1: no column
     bf16x8 qf[NB][KC];
+    // (of the whole form, the wave after the one that writes the token prepares the queries, the others read them from LDS)
+    __shared__ __attribute__((aligned(16))) bf16_t q_stage[WHOLE && FUSED ? KC * WAVE * 8 : 8];
+    const bool prepares = !(WHOLE && FUSED) || wave == ((pos0 - key_begin) / UNIT + 1) % NW;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const int c = col0 + nb * 16 + n16;
         const bool valid = c < ncols;
-        const int tok = t0 + (valid ? c / G : 0);
-        const int head = kvh * G + (valid ? c % G : 0);
+        const int cc = valid ? c : col0;   // no column: another one's query, whose result nobody takes
+        const int tok = t0 + cc / G;
+        const int head = kvh * G + cc % G;
         slope_c[nb] = has_slopes ? fq.slopes[head] : 0.f;
-        pos_c[nb] = valid ? pos0 + c / G : -1;
-        lo_c[nb] = (valid && window > 0) ? max(0, pos_c[nb] - window + 1) : 0;
+        pos_c[nb] = pos0 + cc / G;
+        lo_c[nb] = window > 0 ? max(0, pos_c[nb] - window + 1) : 0;
         qrow[nb] = valid ? (long long)tok * H + head : -1;
         if constexpr (FUSED) {
+            if (!prepares) continue;
             // channels 8g .. 8g+7 and 32 + 8g .. 32 + 8g+7 of the head: partners of the rotation sit in one lane
             const bf16_t* src = q + (long long)tok * ((H + 2 * Hkv) * 64) + head * 64 + g * 8;
-            bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-            const bf16x8 r0 = valid ? *(const bf16x8*)src : z, r1 = valid ? *(const bf16x8*)(src + 32) : z;
+            const bf16x8 r0 = *(const bf16x8*)src, r1 = *(const bf16x8*)(src + 32);
+            float rc[8], rs[8], w0[8], w1[8];
+            if (fq.q_norm_w != nullptr) {
+                norm_weights<8>(fq.q_norm_w, fq.norm_dt, g * 8, w0);
+                norm_weights<8>(fq.q_norm_w, fq.norm_dt, 32 + g * 8, w1);
+            }
+            angles<8>(fq, pos_c[nb], g * 8, rc, rs);
             float v0[8], v1[8];
 #pragma unroll
             for (int e = 0; e < 8; ++e) { v0[e] = (float)r0[e]; v1[e] = (float)r1[e]; }
@@ -335,29 +437,46 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
                 const float inv = 1.0f / sqrtf(ss / 64.0f + fq.eps);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    v0[e] = v0[e] * inv * norm_weight(fq.q_norm_w, fq.norm_dt, g * 8 + e);
-                    v1[e] = v1[e] * inv * norm_weight(fq.q_norm_w, fq.norm_dt, 32 + g * 8 + e);
+                    v0[e] = v0[e] * inv * w0[e];
+                    v1[e] = v1[e] * inv * w1[e];
                 }
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                float rc, rs;
-                angle(fq, max(pos_c[nb], 0), g * 8 + e, rc, rs);
                 const float x0 = v0[e], x1 = v1[e];
-                qf[nb][0][e] = (bf16_t)(x0 * rc - x1 * rs);
-                qf[nb][1][e] = (bf16_t)(x0 * rs + x1 * rc);
+                qf[nb][0][e] = (bf16_t)(x0 * rc[e] - x1 * rs[e]);
+                qf[nb][1][e] = (bf16_t)(x0 * rs[e] + x1 * rc[e]);
             }
         } else {
 #pragma unroll
             for (int kc = 0; kc < KC; ++kc) {
                 const int k = kc * 32 + g * 8;
-                bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-                qf[nb][kc] = (valid && k < hd) ? *(const bf16x8*)(q + qrow[nb] * hd + k) : z;
+                qf[nb][kc] = k < HD ? *(const bf16x8*)(q + ((long long)tok * H + head) * HD + k) : zero8;
             }
         }
     }
+    if constexpr (WHOLE) {
+        if (key_first + 32 < key_end) load_tile(key_first + 32, tb);
+    }
+    if constexpr (WHOLE && FUSED) {
+        if (prepares) {
+#pragma unroll
+            for (int kc = 0; kc < KC; ++kc) *(bf16x8*)(q_stage + (kc * WAVE + lane) * 8) = qf[0][kc];
+        }
+        lds_barrier();
+#pragma unroll
+        for (int kc = 0; kc < KC; ++kc) qf[0][kc] = *(const bf16x8*)(q_stage + (kc * WAVE + lane) * 8);
+    }
 
-    auto compute = [&](int key0, const Tile& t) {
+    // Scores stay as the products leave them, and their scale goes into the base of the exponential: e^(scale (s - max)) is
+    // 2^(log2s s - log2s max).  With distance slopes (or a scale that turns the order round) they are scaled first.
+    const bool scaled = has_slopes || !(scale > 0.f);
+    const float to_m = scaled ? 1.f : scale, log2s = to_m * 1.44269504088896340736f;
+    auto exp2_of = [](float x) { return __builtin_amdgcn_exp2f(x); };
+    // what every column of the block sees: a step within it takes all its keys as they are
+    const int all_lo = window > 0 ? max(0, pos_max - window + 1) : 0, all_hi = pos0 + col0 / G;
+    // FIRST: the unit's first step, which finds nothing to scale
+    auto compute = [&](int key0, Tile& t, auto FIRST) {
         // ---- S^T = K Q^T, twice 16 keys
         f32x4 s[2][NB];
         bf16_t* stage = k_stage[STAGE ? wave : 0];
@@ -366,7 +485,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
             for (int h = 0; h < 2; ++h)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
-                    if (stage_to[h][i] >= 0) *(bf16x8*)(stage + stage_to[h][i]) = t.kf[h][i];
+                    if (!narrow || stage_to[h][i] >= 0) *(bf16x8*)(stage + stage_to[h][i]) = t.kf[h][i];
                 }
             __builtin_amdgcn_wave_barrier();       // the wave's LDS accesses run in the order of the program
         }
@@ -377,69 +496,86 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
 #pragma unroll
             for (int kc = 0; kc < KC; ++kc) {
                 bf16x8 kf;
-                if constexpr (STAGE) {
-                    bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
-                    const int chunk = kc * 4 + g;
-                    kf = chunk < row_pieces ? *(const bf16x8*)(stage + stage_at(8 * (n16 / 4) + 4 * kb + n16 % 4, chunk)) : z;
-                } else if constexpr (AHEAD) kf = t.kf[kb][kc]; else kf = k_frag(t, kb, kc);
+                const int chunk = kc * 4 + g;
+                if constexpr (STAGE) kf = *(const bf16x8*)(stage + stage_at(8 * (n16 / 4) + 4 * kb + n16 % 4, narrow && chunk >= row_pieces ? 0 : chunk));
+                else if constexpr (AHEAD) kf = t.kf[kb][kc];
+                else kf = k_frag(t.k_at, kb, kc);
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) s[kb][nb] = mfma32(kf, qf[nb][kc], s[kb][nb]);
             }
         }
         // ---- mask, running maximum, exp; P^T stays in registers as the next B operand
-        const bool my_live = (g / 2) ? t.live[1] : t.live[0];   // this lane's eight keys lie in half g / 2
+        const bool whole_step = key0 >= all_lo && key0 + 31 <= all_hi;
         bf16x8 pf[NB];
         float corr[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             float v[8];
-            float mx = -INFINITY;
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb)
+            for (int i = 0; i < 8; ++i) v[i] = s[i / 4][nb][i % 4];
+            if (scaled) {
+                // (the distance as an integer first: far positions lose no bits)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int key = key0 + 8 * g + 4 * kb + e;
-                    const bool ok = my_live && key <= pos_c[nb] && key >= lo_c[nb];
-                    // (the distance as an integer first: far positions lose no bits)
-                    const float x = !ok ? -INFINITY : has_slopes ? fmaf(s[kb][nb][e], scale, slope_c[nb] * (float)(key - pos_c[nb]))
-                                                                  : s[kb][nb][e] * scale;
-                    v[kb * 4 + e] = x;
-                    mx = fmaxf(mx, x);
+                for (int i = 0; i < 8; ++i) v[i] = fmaf(v[i], scale, slope_c[nb] * (float)(key0 + 8 * g + i - pos_c[nb]));
+            }
+            if (!whole_step) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int key = key0 + 8 * g + i;
+                    v[i] = key <= pos_c[nb] && key >= lo_c[nb] ? v[i] : -INFINITY;
                 }
+            }
+            float mx = fmaxf(fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])), fmaxf(fmaxf(v[4], v[5]), fmaxf(v[6], v[7])));
             mx = butterfly_max<32>(butterfly_max<16>(mx));
-            const float m_new = fmaxf(m_run[nb], mx);
-            const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
-            corr[nb] = __expf(m_run[nb] - m_safe);          // 0 while nothing was seen yet
-            float sum = 0.f;
+            const float m_new = FIRST ? mx : fmaxf(m_run[nb], mx);
+            const float m_safe = (m_new == -INFINITY) ? 0.f : product(m_new, log2s);
+            if constexpr (!FIRST) corr[nb] = exp2_of(fmaf(m_run[nb], log2s, -m_safe));      // 0 while nothing was seen yet
+            float p[8];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                const float p = __expf(v[i] - m_safe);
-                sum += p;
-                pf[nb][i] = (bf16_t)p;
+                p[i] = exp2_of(fmaf(v[i], log2s, -m_safe));
+                pf[nb][i] = (bf16_t)p[i];
             }
-            l_run[nb] = fmaf(l_run[nb], corr[nb], sum);
+            const float sum = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+            if constexpr (FIRST) l_run[nb] = sum; else l_run[nb] = fmaf(l_run[nb], corr[nb], sum);
             m_run[nb] = m_new;
         }
         // ---- O^T = O^T * corr + V^T P^T
-        const bool tail = key0 + 31 > pos_max;             // keys beyond pos_max were never written
+        // values of keys that no column sees may be anything (beyond pos_max none was written)
+        const bool tail = key0 + 31 > pos_max || key0 < lo_min;
+        auto clear_unseen = [&](bf16x8& vf) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int key = key0 + 8 * g + i;
+                if (key > pos_max || key < lo_min) vf[i] = (bf16_t)0.f;
+            }
+        };
+        if (AHEAD && tail) {
+#pragma unroll
+            for (int db = 0; db < (AHEAD ? DB : 1); ++db) clear_unseen(t.vx[db]);
+        }
 #pragma unroll
         for (int db = 0; db < DB; ++db) {
             bf16x8 vf;
-            if constexpr (AHEAD) vf = t.vx[db]; else vf = v_frag(t, db);
-            if (tail) {
-#pragma unroll
-                for (int i = 0; i < 8; ++i)
-                    if (key0 + 8 * g + i > pos_max) vf[i] = (bf16_t)0.f;
+            if constexpr (AHEAD) vf = t.vx[db];
+            else {
+                vf = v_frag(t.v_at, db);
+                if (tail) clear_unseen(vf);
             }
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
-                f32x4 acc = o[db][nb];
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                if constexpr (!FIRST) {
+                    acc = o[db][nb];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] *= corr[nb];
+                    for (int e = 0; e < 4; ++e) acc[e] *= corr[nb];
+                }
                 o[db][nb] = mfma32(vf, pf[nb], acc);
             }
         }
     };
+    constexpr std::true_type first_step;
+    constexpr std::false_type later_step;
     auto begin_unit = [&]() {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
@@ -449,32 +585,98 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
             for (int db = 0; db < DB; ++db) o[db][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     };
-    // the unit's sum of a column is spread over the four lane groups until here
+    // the unit's sum of a column is spread over the four lane groups until here, and its maximum is one of scores
     auto unit_sums = [&]() {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             l_run[nb] = butterfly_sum<32>(butterfly_sum<16>(l_run[nb]));
+            m_run[nb] = product(m_run[nb], to_m);
         }
     };
 
     // Heads wider than 128 channels have no form of four waves to agree with, and a second set of accumulators does
     // not fit beside the first in a wave's registers: the partition is walked as one unit.
     constexpr bool ONE_UNIT = HDP > 128;
-    if constexpr (NW == 1 && ONE_UNIT) {
+    if constexpr (WHOLE) {
+        // Every wave takes a unit of each turn of NW; a turn's units are merged into partitions through LDS, a wave a column
+        // of a partition at a time, and the partitions at the end, each element through the chains of the other forms and of
+        // their merge.  The next turn's keys are asked for before this one's are merged.
+        extern __shared__ __attribute__((aligned(16))) float whole_lds[];
+        const int cols = FUSED ? G : 16, n_cols = last_col + 1 - col0, n_units = (pos_max - key_begin) / UNIT + 1;
+        float* const u_o = whole_lds;                      // [NW][cols][64]
+        float* const p_o = u_o + NW * cols * 64;           // [n_parts][cols][64]
+        float* const u_ml = p_o + n_parts * cols * 64;     // [NW][cols][2]
+        float* const p_ml = u_ml + NW * cols * 2;          // [n_parts][cols][2]
+        for (int first = 0; first < n_units; first += NW) {
+            const int u = first + wave, key0 = key_begin + u * UNIT, key_next = key0 + NW * UNIT;
+            if (u < n_units) {
+                compute(key0, ta, first_step);
+                if (key_next < key_end) load_tile(key_next, ta);
+                if (key0 + 32 < key_end) compute(key0 + 32, tb, later_step);
+                if (key_next + 32 < key_end) load_tile(key_next + 32, tb);
+                unit_sums();
+            }
+            if (first > 0) lds_barrier();                  // the turn before has been read
+            if (u < n_units && n16 < n_cols) {
+                if (g == 0) { u_ml[(wave * cols + n16) * 2] = m_run[0]; u_ml[(wave * cols + n16) * 2 + 1] = l_run[0]; }
+#pragma unroll
+                for (int db = 0; db < DB; ++db) *(f32x4*)(u_o + (wave * cols + n16) * 64 + db * 16 + 4 * g) = o[db][0];
+            }
+            lds_barrier();
+            const int units = min(NW, n_units - first), jobs = (units + UNITS - 1) / UNITS * n_cols;
+            for (int job = wave; job < jobs; job += NW) {
+                const int p = job / n_cols, c = job % n_cols;
+                float m = -INFINITY, l = 0.f, acc = 0.f;
+#pragma unroll
+                for (int i = 0; i < UNITS; ++i) {
+                    const int v = p * UNITS + i;
+                    if (v < units) {
+                        float m_new, ca, cb;
+                        merge_weights(m, u_ml[(v * cols + c) * 2], m_new, ca, cb);
+                        l = merged(l, ca, u_ml[(v * cols + c) * 2 + 1], cb);
+                        acc = merged(acc, ca, u_o[(v * cols + c) * 64 + lane], cb);
+                        m = m_new;
+                    }
+                }
+                const int at = (first / UNITS + p) * cols + c;
+                if (lane == 0) { p_ml[at * 2] = m; p_ml[at * 2 + 1] = l; }
+                p_o[at * 64 + lane] = acc;
+            }
+        }
+        lds_barrier();
+        const int parts = (n_units + UNITS - 1) / UNITS;
+        for (int c = wave; c < n_cols; c += NW) {
+            const int head = kvh * G + (col0 + c) % G;
+            const float sink = sinks ? sinks[head] : -INFINITY;
+            float m_l = -INFINITY, l_l = 0.f;              // of partition `lane`
+            if (lane < parts) { m_l = p_ml[(lane * cols + c) * 2]; l_l = p_ml[(lane * cols + c) * 2 + 1]; }
+            const float M = fmaxf(wave_max(l_l > 0.f ? m_l : -INFINITY), sink);
+            const float w_l = l_l > 0.f ? __expf(m_l - M) : 0.f, wl_l = w_l * l_l;
+            float L = 0.f, acc = 0.f;
+            for (int p = 0; p < parts; ++p) {
+                const float w = lane_of(w_l, p);
+                L += lane_of(wl_l, p);
+                if (w > 0.f) acc = fmaf(w, p_o[(p * cols + c) * 64 + lane], acc);
+            }
+            if (sinks) L += __expf(sink - M);
+            if (lane < hd) out[((long long)(t0 + (col0 + c) / G) * H + head) * hd + lane] = (bf16_t)(acc * (1.0f / L));
+        }
+        return;
+    } else if constexpr (NW == 1 && ONE_UNIT) {
         begin_unit();
         for (int key0 = key_begin; key0 < key_end; key0 += UNIT) {
             if constexpr (AHEAD) {
                 const bool more = key0 + 32 < key_end;
                 if (more) load_tile(key0 + 32, tb);
-                compute(key0, ta);
+                compute(key0, ta, later_step);
                 if (more) {
                     if (key0 + UNIT < key_end) load_tile(key0 + UNIT, ta);
-                    compute(key0 + 32, tb);
+                    compute(key0 + 32, tb, later_step);
                 }
             } else {
                 for (int k2 = key0; k2 < min(key0 + UNIT, key_end); k2 += 32) {
                     load_tile(k2, ta);
-                    compute(k2, ta);
+                    compute(k2, ta, later_step);
                 }
             }
         }
@@ -487,23 +689,10 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
             for (int db = 0; db < DB; ++db) o_acc[db][nb] = o[db][nb];
         }
     } else if constexpr (NW == 1) {
-        // units in ascending order, each from a fresh state, merged into the partition's result as they end
-        for (int key0 = key_begin; key0 < key_end; key0 += UNIT) {
-            begin_unit();
-            if constexpr (AHEAD) {
-                const bool more = key0 + 32 < key_end;
-                if (more) load_tile(key0 + 32, tb);
-                compute(key0, ta);
-                if (more) {
-                    if (key0 + UNIT < key_end) load_tile(key0 + UNIT, ta);
-                    compute(key0 + 32, tb);
-                }
-            } else {
-                for (int k2 = key0; k2 < min(key0 + UNIT, key_end); k2 += 32) {
-                    load_tile(k2, ta);
-                    compute(k2, ta);
-                }
-            }
+        // units in ascending order, each from a fresh state, merged into the partition's result as they end.  (A step's loads
+        // are never left out, nor is one step's work between two others' loads: where they may be, the compiler no longer
+        // knows how many are under way and waits for all of them.)
+        auto end_unit = [&]() {
             unit_sums();
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
@@ -516,6 +705,30 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
 #pragma unroll
                     for (int e = 0; e < 4; ++e) o_acc[db][nb][e] = merged(o_acc[db][nb][e], ca, o[db][nb][e], cb);
             }
+        };
+        if constexpr (AHEAD) {
+            int key0 = key_begin;
+            for (; key0 + 32 < key_end; key0 += UNIT) {
+                load_tile(key0 + 32, tb);
+                compute(key0, ta, first_step);
+                load_tile(key0 + UNIT, ta);
+                compute(key0 + 32, tb, later_step);
+                end_unit();
+            }
+            if (key0 < key_end) {          // a unit of one step
+                compute(key0, ta, first_step);
+                end_unit();
+            }
+        } else {
+            for (int key0 = key_begin; key0 < key_end; key0 += UNIT) {
+                load_tile(key0, ta);
+                compute(key0, ta, first_step);
+                if (key0 + 32 < key_end) {
+                    load_tile(key0 + 32, ta);
+                    compute(key0 + 32, ta, later_step);
+                }
+                end_unit();
+            }
         }
     } else {
         // a unit a wave; the waves' results go through LDS and every wave merges a share of the elements,
@@ -525,17 +738,15 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
         const int key0 = key_begin + wave * UNIT;
         begin_unit();
         if (key0 < key_end) {
-            if constexpr (AHEAD) {
-                compute(key0, ta);
-                if (key0 + 32 < key_end) compute(key0 + 32, tb);
-            } else {
-                for (int k2 = key0; k2 < min(key0 + UNIT, key_end); k2 += 32) {
-                    load_tile(k2, ta);
-                    compute(k2, ta);
-                }
+            const bool more = key0 + 32 < key_end;
+            if constexpr (!AHEAD) load_tile(key0, ta);
+            compute(key0, ta, first_step);
+            if (more) {
+                if constexpr (!AHEAD) { load_tile(key0 + 32, ta); compute(key0 + 32, ta, later_step); }
+                else compute(key0 + 32, tb, later_step);
             }
+            unit_sums();
         }
-        unit_sums();
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
             if (g == 0) { u_ml[wave][nb][n16][0] = m_run[nb]; u_ml[wave][nb][n16][1] = l_run[nb]; }
@@ -790,12 +1001,43 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
 // Workgroups of four waves where one wave a partition would leave most of the chip idle (a step of a
 // few single tokens); the result is the same bit for bit.
 int few_waves = 2048;
-// From how many workgroups on the kv head is the fastest-changing part of a workgroup's number: with
-// several rounds of waves on the chip (it holds about 3,000 of them) that is 7 to 11 % faster, with one
-// round it is not.
-int kv_fast_waves = 6144;
-// From how many workgroups on the keys of heads of up to 64 channels go through LDS (STAGE_K of the kernel).
-int stage_k_waves = 8192;
+// From how many workgroups on the kv head is the fastest-changing part of a workgroup's number: decode steps with it / without:
+// 8 requests of 20,000 keys 955 / 985 us, 3 of 30,001 838 / 848, one of 20,000 (632 workgroups) 699 / 706; heads of 128, 32 requests
+// of 4,000 95 / 101 us an operation.  With fewer workgroups there is nothing in it.
+int kv_fast_waves = 512;
+// From how many workgroups on the keys of heads of up to 64 channels go through LDS (STAGE_K of the kernel): 3 requests of
+// 30,001 keys (2,832) 870 -> 848 us a step, 12 of 8,000 913 -> 886, 8 of 3,800 (960) 736 -> 722, one of 20,000 (632) 709 -> 706.
+int stage_k_waves = 512;
+
+// Eight waves a workgroup that take all partitions of a column block and write the finished rows, no merge after them: for
+// launches of few partitions with work for the chip all the same.  32 heads on 8, whole decode steps of 16 layers of which 6
+// attend, in partitions / by whole column blocks: room for 1,024 keys, 8 requests of 300 747 / 727 us, 600 746 / 743; 16 of 250
+// 838 / 811, 1,000 844 / 841; 64 of 200 1,118 / 1,083; room for 2,048, 23 requests of 1,111 932 / 910, 64 of 1,900 1,236 / 1,227, but
+// 16 of 1,900 860 / 878; room for 3,072, 48 of 3,000 1,221 / 1,240.  One request of 256 643 / 637, of 1,000 641 / 675: a
+// workgroup's share of a CU is then all there is.
+constexpr int WHOLE_WAVES = 8;
+bool takes_whole(long long blocks, int n_parts) { return n_parts <= 4 ? blocks >= 64 : n_parts <= 8 && blocks >= 176; }
+
+template <bool FUSED, bool STREAM_V = true>
+int launch_whole(dim3 grid, hipStream_t stream, const bf16_t* q, bf16_t* kc, bf16_t* vc, const int* bt, int max_blocks, const int2* blk,
+                 const int4* req_info, int H, int Hkv, int hd, int ps, int window, float scale, int n_parts, const FusedQKV& fq,
+                 bf16_t* out, const float* sinks) {
+    if constexpr (STREAM_V) {
+        if (ps > 16)
+            return launch_whole<FUSED, false>(grid, stream, q, kc, vc, bt, max_blocks, blk, req_info, H, Hkv, hd, ps, window, scale, n_parts,
+                                              fq, out, sinks);
+    }
+    auto kern = attn_partition_kernel<64, 1, WHOLE_WAVES, FUSED, STREAM_V, true>;
+    const int lds = (WHOLE_WAVES + n_parts) * (FUSED ? H / Hkv : 16) * (64 + 2) * 4;       // at most 67,584 bytes
+    static bool set = false;
+    if (!set) {
+        if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * WHOLE_WAVES * 16 * (64 + 2) * 4) != hipSuccess) return -1;
+        set = true;
+    }
+    hipLaunchKernelGGL(kern, grid, dim3(WHOLE_WAVES * WAVE), lds, stream, q, kc, vc, nullptr, nullptr, bt, max_blocks, blk, req_info, H, Hkv,
+                       hd, ps, window, scale, n_parts, fq, 0, out, sinks);
+    return launch_status();
+}
 
 template <int HDP, int NB, bool FUSED, bool STREAM_V = true>
 void launch_partition(dim3 grid, hipStream_t stream, const bf16_t* q, bf16_t* kc, bf16_t* vc, float* ws_o,
@@ -812,22 +1054,23 @@ void launch_partition(dim3 grid, hipStream_t stream, const bf16_t* q, bf16_t* kc
     const int kv_fast = waves >= kv_fast_waves ? 1 : 0;
     if (kv_fast) grid = dim3(grid.x * grid.z, grid.y, 1);
     if constexpr (HDP * NB <= 128) {
-        // the fused form prepares its queries in every wave: four waves pay for that four times
-        if (waves < (FUSED ? few_waves / 2 : few_waves)) {
+        // the fused form prepares its queries in every wave, and four waves pay for that four times: one of 30,000 keys (944
+        // workgroups) 758 us a step with four, 731 with one; one of 8,000 (256) 653 and 662
+        if (waves < (FUSED ? few_waves / 4 : few_waves)) {
             hipLaunchKernelGGL((attn_partition_kernel<HDP, NB, UNITS, FUSED, STREAM_V>), grid, dim3(UNITS * WAVE), 0, stream, q, kc, vc, ws_o,
-                               ws_ml, bt, max_blocks, blk, req_info, H, Hkv, hd, ps, window, scale, n_parts, fq, kv_fast);
+                               ws_ml, bt, max_blocks, blk, req_info, H, Hkv, hd, ps, window, scale, n_parts, fq, kv_fast, nullptr, nullptr);
             return;
         }
     }
     if constexpr (HDP == 64 && HDP * NB <= 256) {
         if (waves >= stage_k_waves) {
             hipLaunchKernelGGL((attn_partition_kernel<HDP, NB, 1, FUSED, STREAM_V, true>), grid, dim3(WAVE), 0, stream, q, kc, vc, ws_o,
-                               ws_ml, bt, max_blocks, blk, req_info, H, Hkv, hd, ps, window, scale, n_parts, fq, kv_fast);
+                               ws_ml, bt, max_blocks, blk, req_info, H, Hkv, hd, ps, window, scale, n_parts, fq, kv_fast, nullptr, nullptr);
             return;
         }
     }
     hipLaunchKernelGGL((attn_partition_kernel<HDP, NB, 1, FUSED, STREAM_V>), grid, dim3(WAVE), 0, stream, q, kc, vc, ws_o, ws_ml, bt,
-                       max_blocks, blk, req_info, H, Hkv, hd, ps, window, scale, n_parts, fq, kv_fast);
+                       max_blocks, blk, req_info, H, Hkv, hd, ps, window, scale, n_parts, fq, kv_fast, nullptr, nullptr);
 }
 }  // namespace
 
@@ -873,6 +1116,9 @@ static int launch_attention(const void* q, const void* k_cache, const void* v_ca
     dim3 grid(n_parts, n_qblocks, Hkv);
     FusedQKV plain_form;
     plain_form.slopes = slopes;
+    if (nb == 1 && hd > 32 && hd <= 64 && takes_whole((long long)n_qblocks * Hkv, n_parts))
+        return launch_whole<false>(dim3(1, n_qblocks, Hkv), stream, Q, K, V, block_table, max_blocks, (const int2*)blk, (const int4*)req_info,
+                                   H, Hkv, hd, page_size, window, scale, n_parts, plain_form, (bf16_t*)out, sinks);
 #define GO(HDP, NB) launch_partition<HDP, NB, false>(grid, stream, Q, K, V, ws_o, ws_ml, block_table, max_blocks, (const int2*)blk, \
                                                      (const int4*)req_info, H, Hkv, hd, page_size, window, scale, n_parts, plain_form)
 #define BY_NB(HDP) do { if (nb == 1) GO(HDP, 1); else if (nb == 2) GO(HDP, 2); else if (nb == 4) GO(HDP, 4); else return -2; } while (0)
@@ -972,6 +1218,10 @@ TUFF_EXPORT int tuff_attention_decode_fused(const void* qkv, void* k_cache, void
     fq.q_norm_w = q_norm_w; fq.k_norm_w = k_norm_w; fq.norm_dt = norm_dt; fq.eps = eps;
     fq.inv_freq = inv_freq; fq.slot_mapping = slot_mapping;
     fq.angles = angles; fq.n_angles = angles ? n_angles : 0;
+    if (takes_whole((long long)n_tokens * Hkv, n_parts))
+        return launch_whole<true>(dim3(1, n_tokens, Hkv), stream, (const bf16_t*)qkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_table,
+                                  max_blocks, nullptr, (const int4*)req_info, H, Hkv, 64, page_size, window, scale, n_parts, fq,
+                                  (bf16_t*)out, nullptr);
     launch_partition<64, 1, true>(dim3(n_parts, n_tokens, Hkv), stream, (const bf16_t*)qkv, (bf16_t*)k_cache, (bf16_t*)v_cache,
                                   ws_o, ws_ml, block_table, max_blocks, nullptr, (const int4*)req_info, H, Hkv, 64, page_size,
                                   window, scale, n_parts, fq);
