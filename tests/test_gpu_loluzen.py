@@ -427,6 +427,45 @@ def test_forget_scan_carries_its_state_across_any_cut(gpu):
             assert torch.isnan(state[0]).all() and torch.isnan(state[2]).all()
 
 
+@pytest.mark.parametrize("H, D, Dv", [(2, 16, 16), (3, 32, 80), (2, 48, 256), (2, 64, 128)])
+@pytest.mark.parametrize("gates", ["spread", "at their bounds"])
+def test_forget_scan_in_chunks_against_the_loop(gpu, H, D, Dv, gates):
+    """The chunked form against the plain loop in float64: requests of 1 to 200 tokens and of none side by side, more of them
+    than a wave has lanes, chunks and blocks that are full, partial and of one token, states in slots between slots of NaN; a second step goes
+    on from the first's states.  Gates of exactly zero and one are among those at their bounds.  A rounding a token and some
+    twenty a sum: 200 + 20 times 2^-24 of the sum of the magnitudes, 1.3e-5."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(H + D + Dv)
+    lens = [200, 1, 0, 64, 65, 16, 17, 129] + [0, 1, 2] * 22
+    R, T = len(lens), sum(lens)
+    x = torch.randn(T, 2 * H * D + H * Dv, generator=gen)
+    fb, lower = torch.randn(H * D, generator=gen), 0.9 * torch.rand(H * D, generator=gen)
+    if gates != "spread":
+        x[:, H * D:2 * H * D] *= 300.0                    # sigmoids of 0 and 1
+        lower[::2] = 0.0
+    q = torch.nn.functional.silu(x[:, :H * D].double()).view(T, H, D)
+    f = (lower.double() + (1 - lower.double()) * torch.sigmoid(x[:, H * D:2 * H * D].double() + fb.double())).view(T, H, D)
+    v = x[:, 2 * H * D:].double().view(T, H, Dv)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)
+    S = [torch.randn(H, D, Dv, generator=gen) * (r % 2) for r in range(R)]
+    state = torch.full((2 * R + 1, H, D, Dv), float("nan"), device=gpu)
+    for r in range(R):
+        state[2 * r + 1] = S[r].to(gpu)
+    S = [s.double() for s in S]
+    starts = [sum(lens[:r]) for r in range(R)]
+    for step in range(2):
+        out = torch.full((T, H * Dv), float("nan"), device=gpu)
+        ops.forget_chunked(x.to(gpu), fb.to(gpu), lower.to(gpu), state, out, q_start=i32(starts), q_len=i32(lens),
+                           state_slot=i32([2 * r + 1 for r in range(R)]), H=H, D=D, Dv=Dv)
+        for r, n in enumerate(lens):
+            for t in range(starts[r], starts[r] + n):
+                S[r] = f[t][:, :, None] * S[r] + (1 - f[t])[:, :, None] * v[t][:, None, :]
+                want, sizes = (S[r] * q[t][:, :, None]).sum(1), (S[r] * q[t][:, :, None]).abs().sum(1)
+                assert ((out[t].double().cpu().view(H, Dv) - want).abs() <= 1.3e-5 * sizes.clamp(min=1.0)).all(), (step, r, t)
+            assert (state[2 * r + 1].double().cpu() - S[r]).abs().max() <= 1.3e-5 * max(1.0, float(S[r].abs().max())), (step, r)
+    assert all(torch.isnan(state[2 * r]).all() for r in range(R + 1))
+
+
 @pytest.mark.parametrize("H, Hkv, vd", [(4, 2, 64), (32, 8, 64), (12, 3, 5), (16, 2, 130), (8, 1, 70), (6, 2, 33), (5, 5, 16), (1, 1, 1)])
 def test_mix_of_heads_against_the_sum_in_float64(gpu, H, Hkv, vd):
     """Two, four and eight heads a kv head (with and without heads left over after eight at a time) and the others: to the

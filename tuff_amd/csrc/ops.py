@@ -64,6 +64,8 @@ _SIGNATURES = {
                              _c_int, _c_int, _c_void_p],
         "tuff_forget_scan": [_c_void_p, _c_int, _c_ll, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                              _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+        "tuff_forget_chunked": [_c_void_p, _c_ll, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p,
+                                _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     },
     "moe": {
         "tuff_moe_route": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p],
@@ -2044,6 +2046,31 @@ def forget_scan(x, bias, lower, state, out, *, q_start, q_len, state_slot, H, D,
         _gpu("state", state, torch.float32, (None, H, D, Dv)), _gpu("out", out, torch.float32, (T, H * Dv)),
         _gpu("q_start", q_start, torch.int32, (R,)), _gpu("q_len", q_len, torch.int32, (R,)),
         _gpu("state_slot", state_slot, torch.int32, (R,)), T, R, H, D, Dv, _stream()), "forget_scan")
+
+
+def forget_chunked_supported(D: int, Dv: int) -> bool:
+    """Whether the chunked form takes these sizes: keys of 16, 32, 48 or 64 channels (what a workgroup's LDS holds twice a
+    CU), values of a multiple of 16 up to 256."""
+    return D % 16 == 0 and 0 < D <= 64 and Dv % 16 == 0 and 0 < Dv <= 256
+
+
+def forget_chunked(x, bias, lower, state, out, *, q_start, q_len, state_slot, H, D, Dv) -> None:
+    """forget_scan's recurrence for prompt portions in chunks of SSD_CHUNK tokens on the matrix cores (float32 matrix
+    instructions; all factors, sums and the state float32): the same function, its sums in another order.  x float32; the other
+    arguments as for forget_scan."""
+    T = x.shape[0]
+    R = q_start.shape[0]
+    if not forget_chunked_supported(D, Dv):
+        raise KernelError(f"forget_chunked: keys of {D} (16, 32, 48 or 64) and values of {Dv} channels (a multiple of 16 up to 256)")
+    chunks = -(-T // SSD_CHUNK) + R
+    U = torch.empty(chunks, H, D, Dv, dtype=torch.float32, device=x.device)
+    cdec = torch.empty(chunks, H, D, dtype=torch.float32, device=x.device)
+    _check(load("recurrent").tuff_forget_chunked(
+        _gpu("x", x, torch.float32, (T, 2 * H * D + H * Dv)), x.shape[1], _opt("bias", bias, torch.float32, (H * D,)),
+        _gpu("lower", lower, torch.float32, (H * D,)), U.data_ptr(), cdec.data_ptr(), chunks,
+        _gpu("state", state, torch.float32, (None, H, D, Dv)), _gpu("out", out, torch.float32, (T, H * Dv)),
+        _gpu("q_start", q_start, torch.int32, (R,)), _gpu("q_len", q_len, torch.int32, (R,)),
+        _gpu("state_slot", state_slot, torch.int32, (R,)), T, R, H, D, Dv, _stream()), "forget_chunked")
 
 
 def head_norm_gate(o, w, gate, out, *, H, Dv, eps, per_head_weight: bool, gate_activation: Optional[str],

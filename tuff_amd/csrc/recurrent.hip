@@ -503,6 +503,306 @@ __global__ __launch_bounds__(256) void ssd_chunk_out_kernel(SsdChunkArgs p) {
     }
 }
 
+// ------------------------------------------------------- the forget-gate recurrence in chunks, on the matrix cores
+// For prompt portions, from float32 projected rows.  Chunks of 64 tokens as above, each of four blocks of 16.  Every decay
+// between two tokens of a block is a product of their gates (no logarithm, no division: gates of zero are as good as any
+// other).  With k = 1 - f and, inside a block, Q_t the product of its gates up to and with t, R_s that of its gates after s,
+// F that of all of them and S the state at its start,
+//     o_t = sum_{s <= t} (sum_i q_t k_s prod_{u in s+1..t} f_u) v_s  +  (q_t Q_t)^T S        S <- F S + sum_s (k_s R_s) v_s^T
+// Three kernels as above: (1) every chunk's own contribution U and the product of its gates, (2) the chunks in order, the
+// state at a chunk's start takes U's place, (3) every chunk's outputs.  All float32, products by float32 matrix instructions
+// (16 x 16 x 4).  A wave keeps the state's columns of 16 value channels as accumulators: element e of tile i of a lane of
+// group q is row 16 i + 4 q + e, and since an inner index may be taken in any order, the accumulators are, as they lie, the
+// second operand of (q_t Q_t)^T S.  What bounds it: float32 matrix instructions (36 a block and wave of the last kernel, 32
+// cycles each) and the way of the rows; token by token it is a chain of 2,048 steps on 512 waves.  One request of 2,048
+// tokens, 16 heads of 64 x 128, with what prepares the rows: 177 -> 59 us (state 19, pass 8, outputs 29).  Outputs are within
+// 8e-8 of 64 bits (token by token 6e-8, the state 9e-8 either way).  The sums of a token are formed in another
+// order than token by token, so a position's result depends on where its portion began, within float32 rounding.
+constexpr int BLOCK = 16;
+
+struct ForgetChunkArgs {
+    const float* x;                 // a token's rows [q (H*D) | z (H*D) | v (H*Dv)], ld apart
+    long long ld;
+    const float *bias, *lower;      // [H*D]; bias or null
+    float* state;                   // [slots][H][D][Dv]
+    float* U;                       // [chunks][H][D][Dv]: a chunk's contribution, then the state at its start
+    float* cdec;                    // [chunks][H][D]: the products of its gates
+    float* out;                     // [T][H][Dv]
+    const int *q_start, *q_len, *state_slot;
+    int R, H, D, Dv;
+};
+
+constexpr int FORGET_LDK = CHUNK + 4;     // floats between two channels' rows of tokens in LDS
+
+// Which request and which of its chunks workgroup `ci` takes, as chunk_of, 64 requests at a time; false: none.
+__device__ __forceinline__ bool chunk_of_wave(const ForgetChunkArgs& p, int ci, int& t0, int& L) {
+    const int lane = threadIdx.x % WAVE;
+    for (int base = 0; base < p.R; base += WAVE) {
+        const int r = base + lane;
+        const int n = r < p.R ? max(p.q_len[r], 0) : 0, start = r < p.R ? p.q_start[r] : 0;
+        int upto = (n + CHUNK - 1) / CHUNK;                // chunks of the requests up to and with this lane's
+#pragma unroll
+        for (int off = 1; off < WAVE; off *= 2) {
+            const int up = __shfl_up(upto, off, WAVE);
+            if (lane >= off) upto += up;
+        }
+        const int all = __builtin_amdgcn_readlane(upto, WAVE - 1);
+        if (ci < all) {
+            const int l = __builtin_ctzll(__ballot(upto > ci));
+            const int nr = __builtin_amdgcn_readlane(n, l), own = (nr + CHUNK - 1) / CHUNK;
+            const int c = ci - (__builtin_amdgcn_readlane(upto, l) - own);
+            t0 = __builtin_amdgcn_readlane(start, l) + c * CHUNK;
+            L = min(CHUNK, nr - c * CHUNK);
+            return true;
+        }
+        ci -= all;
+    }
+    return false;
+}
+
+// Sixteen tokens' elements from element `at` of the chunk's rows on (a token beyond the last: the last one's), in 32 bits.
+__device__ __forceinline__ void column_of_block(const float* rows, unsigned ld, unsigned at, int b, int L, float (&x)[BLOCK]) {
+#pragma unroll
+    for (int u = 0; u < BLOCK; ++u) x[u] = rows[at + (unsigned)min(b * BLOCK + u, L - 1) * ld];
+}
+
+// The gates of a block's tokens from their logits, for channel c (of all heads'), as the kernel that prepares them for the
+// others has them; beyond token L the gate is one and nothing is written.
+__device__ __forceinline__ void gates_of_block(const ForgetChunkArgs& p, int c, int b, int L, float (&f)[BLOCK]) {
+    const float lo = p.lower[c], bias = p.bias ? p.bias[c] : 0.f;
+#pragma unroll
+    for (int u = 0; u < BLOCK; ++u) f[u] = b * BLOCK + u < L ? lo + (1.0f - lo) * sigmoidf_(f[u] + bias) : 1.f;
+}
+
+// P[u] = f[0] .. f[u] in four roundings at most (one after the other they are fifteen); REVERSED: f[15] .. f[u]
+template <bool REVERSED>
+__device__ __forceinline__ void products_of_block(const float (&f)[BLOCK], float (&P)[BLOCK]) {
+#pragma unroll
+    for (int u = 0; u < BLOCK; ++u) P[u] = f[u];
+#pragma unroll
+    for (int d = 1; d < BLOCK; d *= 2)
+#pragma unroll
+        for (int u = 0; u < BLOCK; ++u)
+            if (u & d) {
+                if constexpr (REVERSED) P[BLOCK - 1 - u] *= P[BLOCK - 1 - ((u & ~(2 * d - 1)) + d - 1)];
+                else P[u] *= P[(u & ~(2 * d - 1)) + d - 1];
+            }
+}
+
+// k_s R_s of a block's tokens, and F; sk: the channel's row in LDS
+__device__ __forceinline__ float decayed_keys(const float (&f)[BLOCK], float* sk) {
+    float R[BLOCK], k[BLOCK];
+    products_of_block<true>(f, R);
+#pragma unroll
+    for (int u = 0; u < BLOCK; ++u) k[u] = u + 1 < BLOCK ? (1.0f - f[u]) * R[u + 1] : 1.0f - f[u];
+#pragma unroll
+    for (int u = 0; u < BLOCK; u += 4) *(f32x4*)(sk + u) = f32x4{k[u], k[u + 1], k[u + 2], k[u + 3]};
+    return R[0];
+}
+
+// a lane's values of a block: tokens 4 q .. 4 q + 3, its channel (zero beyond token L)
+__device__ __forceinline__ f32x4 values_of_block(const float* rows, unsigned ld, unsigned at, int b, int q, int L) {
+    f32x4 r;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int t = b * BLOCK + 4 * q + e;
+        const float x = rows[at + (unsigned)min(t, L - 1) * ld];
+        r[e] = t < L ? x : 0.f;
+    }
+    return r;
+}
+
+// S <- F S + sum over the block's tokens; sk [D][FORGET_LDK], sF [D]
+template <int NI>
+__device__ __forceinline__ void state_over_block(f32x4 (&S)[NI], const float* sk, const float* sF, int b, f32x4 v, int l16, int q) {
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const f32x4 F = *(const f32x4*)(sF + i * 16 + 4 * q);
+        const f32x4 k = *(const f32x4*)(sk + (i * 16 + l16) * FORGET_LDK + b * BLOCK + 4 * q);
+        S[i] *= F;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) S[i] = mfma_f32(k[e], v[e], S[i]);
+    }
+}
+
+template <int NI>
+__global__ __launch_bounds__(512, 4) void forget_chunk_state_kernel(ForgetChunkArgs p) {
+    constexpr int D = 16 * NI;
+    __shared__ __attribute__((aligned(16))) float sk[D * FORGET_LDK];
+    __shared__ __attribute__((aligned(16))) float sF[CHUNK / BLOCK][D];
+    const int Dv = p.Dv, head = blockIdx.y, tid = threadIdx.x, lane = tid % WAVE, l16 = lane % 16, q = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), waves = blockDim.x / WAVE;
+    int t0, L;
+    if (!chunk_of_wave(p, blockIdx.x, t0, L)) return;
+    const float* row = p.x + (long long)t0 * p.ld;
+    const unsigned ld = (unsigned)p.ld;
+    for (int job = tid; job < D * (CHUNK / BLOCK); job += blockDim.x) {
+        const int c = job % D, b = job / D;
+        float f[BLOCK];
+        column_of_block(row, ld, (p.H + head) * D + c, b, L, f);
+        gates_of_block(p, head * D + c, b, L, f);
+        sF[b][c] = decayed_keys(f, sk + c * FORGET_LDK + b * BLOCK);
+    }
+    __syncthreads();
+    const long long at = (long long)blockIdx.x * p.H + head;
+    if (tid < D) p.cdec[at * D + tid] = sF[0][tid] * sF[1][tid] * sF[2][tid] * sF[3][tid];
+    float* U = p.U + at * D * Dv;
+    for (int j = wave * 16 + l16; j < Dv; j += waves * 16) {
+        const unsigned v = 2 * p.H * D + head * Dv + j;
+        f32x4 S[NI] = {}, next = values_of_block(row, ld, v, 0, q, L);
+#pragma unroll 1
+        for (int b = 0; b < CHUNK / BLOCK; ++b) {
+            const f32x4 vb = next;
+            next = values_of_block(row, ld, v, min(b + 1, CHUNK / BLOCK - 1), q, L);
+            state_over_block(S, sk, sF[b], b, vb, l16, q);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) U[(long long)(i * 16 + 4 * q + e) * Dv + j] = S[i][e];
+    }
+}
+
+// four neighbouring elements of the state a thread
+__global__ __launch_bounds__(256) void forget_state_pass_kernel(ForgetChunkArgs p) {
+    const int r = blockIdx.x, head = blockIdx.y;
+    const int n = p.q_len[r];
+    if (n <= 0) return;
+    const int DV = p.D * p.Dv, e = (blockIdx.z * 256 + threadIdx.x) * 4;
+    int before = 0;
+    for (int r2 = threadIdx.x % WAVE; r2 < r; r2 += WAVE) before += (max(p.q_len[r2], 0) + CHUNK - 1) / CHUNK;
+#pragma unroll
+    for (int off = 1; off < WAVE; off *= 2) before += __shfl_xor(before, off, WAVE);
+    if (e >= DV) return;
+    const int nc = (n + CHUNK - 1) / CHUNK;
+    float* S = p.state + ((long long)p.state_slot[r] * p.H + head) * DV + e;
+    float* u = p.U + ((long long)before * p.H + head) * DV + e;
+    const float* d = p.cdec + ((long long)before * p.H + head) * p.D + e / p.Dv;
+    const long long next_u = (long long)p.H * DV, next_d = (long long)p.H * p.D;
+    f32x4 s = *(const f32x4*)S;
+    constexpr int AHEAD = 8;             // chunks asked for together: stores in between would hold the loads back
+    for (int c = 0; c < nc; c += AHEAD) {
+        f32x4 own[AHEAD];
+        float dec[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const int ci = min(c + i, nc - 1);
+            own[i] = *(const f32x4*)(u + ci * next_u);
+            dec[i] = d[ci * next_d];
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+            if (c + i < nc) {
+                *(f32x4*)(u + (c + i) * next_u) = s;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) s[k] = fmaf(dec[i], s[k], own[i][k]);
+            }
+    }
+    *(f32x4*)S = s;
+}
+
+template <int NI>
+__global__ __launch_bounds__(512, 4) void forget_chunk_out_kernel(ForgetChunkArgs p) {
+    constexpr int D = 16 * NI, LDQ = D + 4, LDA = BLOCK + 4, BLOCKS = CHUNK / BLOCK;
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    float* const sk = sm;                              // [D][FORGET_LDK]: k_s R_s, a channel's tokens side by side
+    float* const sqd = sk + D * FORGET_LDK;            // [CHUNK][LDQ]: q_t Q_t
+    float* const sq = sqd + CHUNK * LDQ;               // [CHUNK][LDQ]: q
+    float* const sf = sq + CHUNK * LDQ;                // [CHUNK][LDQ]: the gates
+    float* const sF = sf + CHUNK * LDQ;                // [BLOCKS][D]
+    float* const sA = sF + BLOCKS * D;                 // [2][BLOCKS][BLOCK (t)][LDA (s)]: inside a block, by half of the channels
+    const int Dv = p.Dv, head = blockIdx.y, tid = threadIdx.x, lane = tid % WAVE, l16 = lane % 16, q = lane / 16;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), waves = blockDim.x / WAVE;
+    int t0, L;
+    if (!chunk_of_wave(p, blockIdx.x, t0, L)) return;
+    const float* row = p.x + (long long)t0 * p.ld;
+    const unsigned ld = (unsigned)p.ld;
+    for (int job = tid; job < D * BLOCKS; job += blockDim.x) {
+        const int c = job % D, b = job / D;
+        float f[BLOCK], qr[BLOCK];
+        column_of_block(row, ld, (p.H + head) * D + c, b, L, f);
+        column_of_block(row, ld, head * D + c, b, L, qr);
+        gates_of_block(p, head * D + c, b, L, f);
+        sF[b * D + c] = decayed_keys(f, sk + c * FORGET_LDK + b * BLOCK);
+        float Q[BLOCK];
+        products_of_block<false>(f, Q);
+#pragma unroll
+        for (int u = 0; u < BLOCK; ++u) {
+            const float qq = siluf_(qr[u]);
+            sq[(b * BLOCK + u) * LDQ + c] = qq;
+            sf[(b * BLOCK + u) * LDQ + c] = f[u];
+            sqd[(b * BLOCK + u) * LDQ + c] = qq * Q[u];
+        }
+    }
+    __syncthreads();
+    // A[t][s] of a block over half of the channels: a lane takes token s = l16 and a quarter of the half, and carries
+    // k_s prod f from token to token
+    constexpr int PER = D / 8;                         // channels a lane
+    for (int job = wave; job < 2 * BLOCKS; job += waves) {
+        const int b = job % BLOCKS, half = job / BLOCKS, c0 = half * (D / 2) + q * PER;
+        float X[PER] = {};
+        float* to = sA + ((half * BLOCKS + b) * BLOCK + q) * LDA + l16;
+#pragma unroll 1
+        for (int t4 = 0; t4 < BLOCK; t4 += 4) {
+            const float* ft = sf + (b * BLOCK + t4) * LDQ + c0;
+            const float* qt = sq + (b * BLOCK + t4) * LDQ + c0;
+            float A[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                float part[2] = {0.f, 0.f};
+#pragma unroll
+                for (int i = 0; i < PER; ++i) {
+                    X[i] = t4 + t == l16 ? 1.0f - ft[t * LDQ + i] : X[i] * ft[t * LDQ + i];
+                    part[i % 2] = fmaf(qt[t * LDQ + i], X[i], part[i % 2]);
+                }
+                A[t] = butterfly_sum<32>(butterfly_sum<16>(part[0] + part[1]));
+            }
+            to[t4 * LDA] = q == 0 ? A[0] : q == 1 ? A[1] : q == 2 ? A[2] : A[3];
+        }
+    }
+    __syncthreads();
+    const float* Sin = p.U + ((long long)blockIdx.x * p.H + head) * D * Dv;
+    for (int j = wave * 16 + l16; j < Dv; j += waves * 16) {
+        const unsigned v = 2 * p.H * D + head * Dv + j;
+        f32x4 S[NI], next = values_of_block(row, ld, v, 0, q, L);
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S[i][e] = Sin[(long long)(i * 16 + 4 * q + e) * Dv + j];
+#pragma unroll 1
+        for (int b = 0; b < BLOCKS && b * BLOCK < L; ++b) {
+            const f32x4 vb = next;
+            next = values_of_block(row, ld, v, min(b + 1, BLOCKS - 1), q, L);
+            // sums of four products each, added as a tree: as near to the exact sum as token by token
+            const float* a = sA + (b * BLOCK + l16) * LDA + 4 * q;
+            const f32x4 a0 = *(const f32x4*)a, a1 = *(const f32x4*)(a + BLOCKS * BLOCK * LDA), zero = {0.f, 0.f, 0.f, 0.f};
+            f32x4 part[4], o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part[e] = mfma_f32(a0[e] + a1[e], vb[e], zero);
+            o = (part[0] + part[1]) + (part[2] + part[3]);
+            f32x4 sum[NI];
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                const f32x4 qd = *(const f32x4*)(sqd + (b * BLOCK + l16) * LDQ + i * 16 + 4 * q);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part[e] = mfma_f32(qd[e], S[i][e], zero);
+                sum[i] = (part[0] + part[1]) + (part[2] + part[3]);
+            }
+            if constexpr (NI == 4) o += (sum[0] + sum[1]) + (sum[2] + sum[3]);
+            else {
+#pragma unroll
+                for (int i = 0; i < NI; ++i) o += sum[i];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = b * BLOCK + 4 * q + e;
+                if (t < L) p.out[((long long)(t0 + t) * p.H + head) * Dv + j] = o[e];
+            }
+            state_over_block(S, sk, sF + b * D, b, vb, l16, q);
+        }
+    }
+}
+
 struct ScanArgs {
     const void *a, *k, *v;          // per token: a (r, or unit q) and k, rows of Ha*D, lda apart; v: rows of H*Dv, ldv apart   (Ha: heads of a and k)
     const float* decay;             // per token [T][H*D]: w or g; ssd: [T][H], one decay for all of a head's key channels
@@ -1107,4 +1407,32 @@ TUFF_EXPORT int tuff_forget_scan(const void* x, int dt, long long ld, const floa
     ScanArgs p{qn, qn, v, f, f, state, out, q_start, q_len, state_slot, H, H, D, Dv, ld, (long long)H * D, nullptr};
     return dt == DT_F32 ? launch_scan<float, float, false, true>(p, n_tokens, n_requests, stream)
                         : launch_scan<float, bf16_t, false, true>(p, n_tokens, n_requests, stream);
+}
+
+// The same recurrence in chunks of 64 tokens on the matrix cores (see above), from float32 rows: D 16, 32, 48 or 64, Dv a
+// multiple of 16 up to 256.  Work arrays: U float32 [chunks][H][D][Dv] and cdec float32 [chunks][H][D] with chunks >=
+// ceil(T / 64) + requests (what the step's portions can be cut into at most).
+TUFF_EXPORT int tuff_forget_chunked(const float* x, long long ld, const float* bias, const float* lower, float* U, float* cdec, int chunks,
+                                    float* state, float* out, const int* q_start, const int* q_len, const int* state_slot,
+                                    int n_tokens, int n_requests, int H, int D, int Dv, hipStream_t stream) {
+    if (n_requests <= 0 || n_tokens <= 0) return 0;
+    if (H <= 0 || H > 65535 || n_requests > 65535 || ld < 2LL * H * D + (long long)H * Dv || ld > (1 << 24)) return -2;
+    if (D <= 0 || D % 16 || D > 64 || Dv <= 0 || Dv % 16 || Dv > 256 || chunks < ceil_div(n_tokens, CHUNK) + n_requests) return -2;
+    if (((uintptr_t)state | (uintptr_t)U) & 15) return -2;           // read in fours
+    ForgetChunkArgs p{x, ld, bias, lower, state, U, cdec, out, q_start, q_len, state_slot, n_requests, H, D, Dv};
+    const dim3 block(WAVE * min(8, Dv / 16)), grid(chunks, H);
+    const size_t lds = (size_t)(D * FORGET_LDK + 3 * CHUNK * (D + 4) + CHUNK / BLOCK * D + 2 * CHUNK * (BLOCK + 4)) * sizeof(float);
+#define GO(NI) do { \
+        static bool set = false; \
+        if (!set) { \
+            if (hipFuncSetAttribute((const void*)forget_chunk_out_kernel<NI>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) return -1; \
+            set = true; \
+        } \
+        hipLaunchKernelGGL(forget_chunk_state_kernel<NI>, grid, block, 0, stream, p); \
+        hipLaunchKernelGGL(forget_state_pass_kernel, dim3(n_requests, H, ceil_div(D * Dv, 1024)), dim3(256), 0, stream, p); \
+        hipLaunchKernelGGL(forget_chunk_out_kernel<NI>, grid, block, lds, stream, p); \
+    } while (0)
+    if (D == 16) GO(1); else if (D == 32) GO(2); else if (D == 48) GO(3); else GO(4);
+#undef GO
+    return launch_status();
 }
