@@ -270,6 +270,30 @@ def test_gemm_bf16_few_rows_at_the_edges_of_the_waves_shares(gpu, N, K):
         assert torch.equal(acc[:2], 1 + whole[:min(M, 2)])
 
 
+@pytest.mark.parametrize("N,K,most", [(2048, 8192, 8), (520, 4104, 16), (2048, 4480, 15), (72, 16392, 4), (2048, 256, 16)])
+def test_gemm_bf16_few_rows_that_lie_in_lds_in_whole(gpu, N, K, most):
+    """Inner sizes of many chunks a wave, whole and ragged, up to the most rows that fit (one more, where there may be, comes from memory as before):
+    within float32's K roundings of the float64 product, every row with the bits it has alone, one of infinities and NaN too."""
+    from tuff_amd.csrc import ops
+    x, w = _r(most + 1, K, seed=1, dtype=torch.bfloat16).to(gpu), _r(N, K, seed=2, dtype=torch.bfloat16).to(gpu)
+    x[1, ::3], x[1, 1::3] = float("inf"), float("nan")
+    tiled = ops.tile_weight(w)
+    exact = x.double().nan_to_num(0, 0, 0) @ w.double().T
+    bound = K * 2.0 ** -24 * (x.double().abs().nan_to_num(0, 0, 0) @ w.double().abs().T)
+    alone = torch.cat([torch.empty(1, N, device=gpu) for _ in range(most + 1)])
+    for m in range(most + 1):
+        ops.gemm(x[m:m + 1], tiled, alone[m:m + 1])
+    kept = [m for m in range(most + 1) if m != 1]
+    assert ((alone.double() - exact).abs() <= bound)[kept].all() and not torch.isfinite(alone[1]).any()
+    for M in sorted({2, 3, most - 1, most, min(most + 1, 16)}):
+        out, res, nw = torch.empty(M, N, device=gpu), torch.zeros(M, N, device=gpu), torch.ones(N, device=gpu)
+        ops.gemm(x[:M], tiled, out)
+        assert torch.equal(out.nan_to_num(7.0), alone[:M].nan_to_num(7.0)), M
+        xw, ss = torch.empty(M, N, dtype=torch.bfloat16, device=gpu), torch.empty(*ops.gemm_emit_layout(M, N, K), device=gpu)
+        ops.gemm_accum_emit(x[:M], tiled, res, nw, xw, ss)
+        assert torch.equal(res.nan_to_num(7.0), alone[:M].nan_to_num(7.0)), M
+
+
 @pytest.mark.parametrize("M", [17, 20, 21])
 @pytest.mark.parametrize("N,K", [(256, 64), (1024, 1024), (2048, 1032), (2048, 2048), (2048, 2056)])
 def test_gemm_bf16_narrow_outputs_of_17_to_21_rows(gpu, M, N, K):

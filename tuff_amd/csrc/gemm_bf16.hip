@@ -595,7 +595,12 @@ constexpr int skinny16_waves_a_simd(int NW, int COLS, int MT, int MODE, int SHAR
     return NW == 8 && COLS == 32 && MT == 1 && !(MODE == OUT_F32_ACCUM && SHARE == SHARE_MANY) ? 4 : 1;      // (that one would spill)
 }
 
-template <int NW, int MODE, int NORM, bool EMIT, int COLS, int MT, int SHARE>
+// XL: the rows of X lie in LDS, in whole.  A workgroup reads all of them either way; in the order of the operands every load of a
+// wave touches sixteen rows for 64 bytes each, however few rows there are, and there are as many of them as loads of W.  As they
+// lie, one row of 8,192 is one load a wave instead of sixteen.  At most so many pieces of 16 bytes a thread:
+constexpr int skinny16_pieces(int MT) { return MT == 1 ? 9 : 12; }
+
+template <int NW, int MODE, int NORM, bool EMIT, int COLS, int MT, int SHARE, bool XL>
 __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE, SHARE)) void gemm_bf16_skinny16_kernel(const void* __restrict__ Xv, const bf16_t* __restrict__ W,
                                                                        void* __restrict__ Y, int M, int N, int K,
                                                                        const float* __restrict__ norm_w, float eps,
@@ -605,6 +610,10 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
                                                                        bf16_t* __restrict__ emit_xw, float* __restrict__ emit_ss,
                                                                        ConvTail cv) {
     constexpr bool CONV = MODE == OUT_CONV;
+    // Neighbouring columns on one XCD (workgroups go round the eight of them) where all workgroups run side by side: one row,
+    // 16,384 x 2,048 13.4 -> 13.0 us, 2,048 x 8,192 of 8 rows 9.9 -> 9.6, 2,048 x 2,048 4.7 -> 4.5, but 65,536 x 2,048 42.5 -> 42.7; with
+    // two row tiles a decode step of 23 rows is 1 % slower.
+    const unsigned block = MT == 1 && gridDim.x <= 512 && gridDim.x % 8 == 0 ? blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
     static_assert(!CONV || COLS == 8, "the convolution's epilogue takes eight channels a workgroup");
     static_assert(MT == 1 || NORM != NORM_INSIDE, "the norm inside is for at most 16 rows");
     constexpr int TN = CONV ? 3 : (COLS > 16 ? COLS / 16 : 1);           // MFMA tiles side by side: they share the rows of X
@@ -616,10 +625,12 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
     __shared__ float red[MT][TN][NW][WAVE][4];
     __shared__ float ssq[16][ROWS];                                      // [wave or part][row]
     extern __shared__ __attribute__((aligned(16))) float nw_lds[];       // NORM_INSIDE: the norm weight, K floats
+    bf16_t* const x_lds = (bf16_t*)nw_lds;                               // XL: [M][K + 8], eight zeros behind every row
+    static_assert(!XL || NORM != NORM_INSIDE, "rows in LDS are bfloat16");
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int r16 = lane % 16, g = lane / 16;
     // OUT_CONV: workgroup b takes the channels 8 b .. 8 b + 7: half (b % 2) of the three row tiles of group b / 2
-    const long long n0 = CONV ? (long long)(blockIdx.x / 2) * 48 + (blockIdx.x % 2) * 8 : (long long)blockIdx.x * COLS;
+    const long long n0 = CONV ? (long long)(block / 2) * 48 + (block % 2) * 8 : (long long)block * COLS;
     const int nchunks = (K + SK_CHUNK - 1) / SK_CHUNK;
     const long long w_rows = min((long long)N, n0 + COLS);               // this tile's rows of W end here
     // tile-major W: this lane's piece of a block; a workgroup of 8 columns owns half a row tile
@@ -665,7 +676,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
 #pragma unroll
         for (int i = 0; i < EPI_TILES; ++i) {
             const int mt = tid / 256 + i * EPI_GROUPS, t = tid % 256, l = t / 4;
-            const int row = mt * 16 + (l / 16) * 4 + t % 4, ch = (int)blockIdx.x * 8 + (l % 16), d = N / 3, Kc = cv.taps;
+            const int row = mt * 16 + (l / 16) * 4 + t % 4, ch = (int)block * 8 + (l % 16), d = N / 3, Kc = cv.taps;
 #pragma unroll
             for (int k = 0; k <= CONV_AHEAD; ++k) tap_ahead[i][k] = 0.f;
             slot_ahead[i] = cv.state_slot[min(row, M - 1)];
@@ -684,7 +695,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) acc[mt][tn] = f32x4{0.f, 0.f, 0.f, 0.f};
     float ss = 0.f;
-    struct Operands { bf16x8 a[MT][4]; bf16x8 b[TN][4]; f32x4 x[NORM == NORM_INSIDE ? 4 : 1][2]; };
+    struct Operands { bf16x8 a[XL ? 1 : MT][XL ? 1 : 4]; bf16x8 b[TN][4]; f32x4 x[NORM == NORM_INSIDE ? 4 : 1][2]; };
     Operands o0, o1;
     // The operands come through buffer loads; an offset beyond the buffer, for rows, columns and k that are not
     // there, reads as zero and fetches nothing.  With no branch around a load the compiler counts the loads under way and
@@ -704,7 +715,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
                 o.b[tn][j] = load_buffer<true>(wbuf, in ? w_at : NOWHERE, in ? (tn * kb + c * 4 + j) * 1024 : 0);
             }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < (XL ? 0 : 4); ++j) {
             const int kj = c * SK_CHUNK + j * 32 + g * 8;
             if (COLS == 32 && MT == 1 && NORM != NORM_INSIDE) {
                 // (lanes without a row are switched off: here, where the rows of X are half as many bytes as W, one that reads
@@ -722,7 +733,43 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
             }
         }
     };
+    constexpr int PIECES = skinny16_pieces(MT);
+    bf16x8 x_piece[XL ? PIECES : 1];
+    const int n_pieces = XL ? M * K / 8 : 0;
+    auto fetch_x = [&]() {
+        if constexpr (XL) {
+#pragma unroll
+            for (int u = 0; u < PIECES; ++u)
+                if (u * NT_ < n_pieces) x_piece[u] = load_buffer<false>(xbuf, (tid + u * NT_) * 16, 0);
+        }
+    };
+    auto keep_x = [&]() {
+        if constexpr (XL) {
+            const unsigned per_row = (unsigned)K / 8, inverse = 0xFFFFFFFFu / per_row + 1;       // (exact for 2 to 2^16 a row, up to 2^16 pieces)
+#pragma unroll
+            for (int u = 0; u < PIECES; ++u)
+                if (u * NT_ < n_pieces) {
+                    const unsigned i = tid + u * NT_, row = __umulhi(i, inverse);
+                    if (i < (unsigned)n_pieces) *(bf16x8*)(x_lds + 8 * (i + row)) = x_piece[u];
+                }
+            if (tid < M) *(bf16x8*)(x_lds + (tid + 1) * (K + 8) - 8) = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
+            lds_barrier();
+        }
+    };
     auto multiply = [&](int c, Operands& o) {
+        if constexpr (XL) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const bf16_t* row = x_lds + min(mt * 16 + r16, M - 1) * (K + 8);             // (no row: another one's, its result is not taken)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const bf16x8 a = *(const bf16x8*)(row + min(c * SK_CHUNK + j * 32 + g * 8, K));
+#pragma unroll
+                    for (int tn = 0; tn < TN; ++tn) acc[mt][tn] = mfma16(a, o.b[tn][j], acc[mt][tn]);
+                }
+            }
+            return;
+        }
         if (NORM == NORM_INSIDE) {
             const int k0 = c * SK_CHUNK + g * 8;
 #pragma unroll
@@ -741,7 +788,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
             }
         }
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
+        for (int mt = 0; mt < (XL ? 0 : MT); ++mt)
 #pragma unroll
             for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
@@ -750,7 +797,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
     // Workgroups start at different chunks (a rotation by the tile index), so that at any moment
     // the chip reads from all columns of W and not from one.  The order of a tile's additions
     // still depends on N and K only.
-    const int rot = (int)((blockIdx.x * 5u) % (unsigned)nchunks);
+    const int rot = (int)((block * 5u) % (unsigned)nchunks);
     auto chunk_of = [&](int i) { const int c = i + rot; return c >= nchunks ? c - nchunks : c; };
     // NORM_SCALED: 16 parts x ROWS rows; part p adds the tiles p, p + 16, ... of its row.  The first
     // sixteen of them are only asked for here and added after the products, when they have long
@@ -780,7 +827,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
         if constexpr (CONV) {
 #pragma unroll
             for (int i = 0; i < EPI_TILES; ++i) {
-                const int t = tid % 256, l = t / 4, ch = (int)blockIdx.x * 8 + (l % 16), d = N / 3, Kc = cv.taps;
+                const int t = tid % 256, l = t / 4, ch = (int)block * 8 + (l % 16), d = N / 3, Kc = cv.taps;
                 const float* st = cv.state + (long long)slot_ahead[i] * (Kc - 1) * d + min(ch, d - 1);
 #pragma unroll
                 for (int k = 0; k < CONV_AHEAD; ++k) st_ahead[i][k] = st[(long long)min(k, Kc - 2) * d];
@@ -802,11 +849,13 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
     auto issued = [&]() { __builtin_amdgcn_sched_barrier(0); };
     if constexpr (SHARE == SHARE_ONE) {
         const int c = n > 0 ? nth(0) : nchunks;        // (a wave without a chunk, K up to 384: the one behind the last is all zeros)
+        fetch_x();
         load(c, o0);
         issued();
         behind();
         issued();
         if constexpr (NORM == NORM_INSIDE) norm_weight();
+        keep_x();
         multiply(c, o0);
     } else if constexpr (SHARE == SHARE_TWO && NORM == NORM_INSIDE) {
         load(nth(0), o0);
@@ -818,6 +867,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
         multiply(nth(0), o0);
         if (n > 1) multiply(nth(1), o1);
     } else if constexpr (SHARE == SHARE_TWO) {
+        static_assert(!XL, "rows in LDS: one chunk a wave or many");
         if (n > 1) {
             load(nth(0), o0);
             load(nth(1), o1);
@@ -837,12 +887,14 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
         // (two sets of operands over 32 columns and the sums of squares are more than 128 registers: there the sums are asked
         // for where one of the sets is used up)
         constexpr bool LATE = NORM == NORM_SCALED && COLS == 32;
+        fetch_x();
         load(nth(0), o0);
         load(nth(1), o1);
         issued();
         if (!LATE) behind();
         issued();
         if constexpr (NORM == NORM_INSIDE) norm_weight();
+        keep_x();
         int i = 0;
         for (; i + 3 < n; i += 2) {
             multiply(nth(i), o0);
@@ -916,7 +968,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
                 bcx[tn] = (float)(bf16_t)v;
             }
             const int row = trow, d = N / 3, Kc = cv.taps;
-            const int ch = (int)(blockIdx.x) * 8 + (l % 16);
+            const int ch = (int)(block) * 8 + (l % 16);
             if ((l % 16) < 8 && row < M && ch < d) {
                 float* st = cv.state + (long long)slot_ahead[ei] * (Kc - 1) * d;
                 float sv[CONV_MAX_TAPS], wv[CONV_MAX_TAPS];
@@ -960,7 +1012,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
                 float sq = y * y;                       // t256 = (16 q + c) * 4 + e: the 16 columns c are its bits 2..5
                 sq += __shfl_xor(sq, 4, WAVE);
                 sq = butterfly_sum<32>(butterfly_sum<16>(butterfly_sum<8>(sq)));
-                if ((l % 16) == 0 && row < ROWS) emit_ss[(long long)blockIdx.x * SSR + row] = sq;
+                if ((l % 16) == 0 && row < ROWS) emit_ss[(long long)block * SSR + row] = sq;
             } else if (MODE == OUT_F32_ACCUM) {
                 if (row < M && col < N) ((float*)Y)[row * N + col] = y_old[ei][tn] + v;
             } else {
@@ -1440,15 +1492,42 @@ struct Skinny16Extra {
     ConvTail conv;                                                                   // OUT_CONV
 };
 
+// LDS that is left for the rows of X beside the partial sums (up to 16 columns a workgroup).
+constexpr int skinny16_lds_left(int NW, int MT) { return 160 * 1024 - MT * NW * 1024 - 16 * 16 * MT * 4; }
+// Where the waves have many chunks, X goes through LDS as far as it fits; where they have one each, a barrier before its product
+// costs a few rows more than it saves.  Rows from memory / in LDS, us: 2,048 x 8,192 of 1 row 8.9 and 7.8, 4 9.2 and 8.1, 8 9.6 and
+// 8.8; one chunk a wave, 2,048 x 2,048 of 1 row 4.2 and 4.3, 8 4.5 and 4.4, 16 5.2 and 4.7, 3,072 x 2,048 4.8 and 5.2, 5.4 and 5.5, 6.0
+// and 5.7.  (Two chunks a wave lose: 6,144 x 2,048 with the convolution 7.5 and 8.1, 16,384 x 2,048 13.0 and 13.1.)
+bool skinny16_rows_in_lds(int NW, int MT, int SHARE, int M, int K) {
+    if (K < 256 || (SHARE == SHARE_ONE && M <= 8)) return false;
+    return (long long)M * (K + 8) * 2 <= skinny16_lds_left(NW, MT) && (long long)M * K / 8 <= (long long)skinny16_pieces(MT) * NW * WAVE;
+}
+
 template <int MODE, int NORM, bool EMIT>
 int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K, const Skinny16Extra& x, hipStream_t stream) {
     // the in-kernel norm needs more registers a wave: at most 8 waves a workgroup
     SkinnyPlan p = plan_skinny(M, N, K, NORM == NORM_INSIDE ? 8 : 16, EMIT, MODE == OUT_CONV);
-    const size_t lds = NORM == NORM_INSIDE ? (size_t)K * sizeof(float) : 0;
+    size_t lds = NORM == NORM_INSIDE ? (size_t)K * sizeof(float) : 0;
     const int mt = M > 16 ? 2 : 1, chunks = ceil_div(K, SK_CHUNK);
-#define GO_SHARE(NW, COLS, MT, SHARE) hipLaunchKernelGGL((gemm_bf16_skinny16_kernel<NW, MODE, NORM, EMIT, COLS, MT, SHARE>), grid, dim3(NW * WAVE), lds, stream, \
+#define GO_XL(NW, COLS, MT, SHARE, XL) hipLaunchKernelGGL((gemm_bf16_skinny16_kernel<NW, MODE, NORM, EMIT, COLS, MT, SHARE, XL>), grid, dim3(NW * WAVE), lds, stream, \
                                         X, W, Y, M, N, K, x.norm_w, x.eps, x.rows, x.ldx ? x.ldx : (long long)K, x.ss_in, x.n_ss, x.emit_nw, x.emit_xw, x.emit_ss, \
                                         x.conv)
+#define GO_SHARE(NW, COLS, MT, SHARE) do { \
+        if constexpr (NORM != NORM_INSIDE && COLS < 32 && MODE != OUT_CONV && (SHARE == SHARE_MANY || (SHARE == SHARE_ONE && MT == 1))) { \
+            if (skinny16_rows_in_lds(NW, MT, SHARE, M, K)) { \
+                lds = (size_t)M * (K + 8) * sizeof(bf16_t); \
+                static bool set = false; \
+                if (!set) { \
+                    if (hipFuncSetAttribute((const void*)gemm_bf16_skinny16_kernel<NW, MODE, NORM, EMIT, COLS, MT, SHARE, true>, \
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, skinny16_lds_left(NW, MT)) != hipSuccess) return -1; \
+                    set = true; \
+                } \
+                GO_XL(NW, COLS, MT, SHARE, true); \
+                break; \
+            } \
+        } \
+        GO_XL(NW, COLS, MT, SHARE, false); \
+    } while (0)
 #define GO_MT(NW, COLS, MT) do { \
         if (chunks <= NW) GO_SHARE(NW, COLS, MT, SHARE_ONE); \
         else if (chunks <= 2 * NW) GO_SHARE(NW, COLS, MT, SHARE_TWO); \
@@ -1482,6 +1561,7 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
 #undef GO
 #undef GO_MT
 #undef GO_SHARE
+#undef GO_XL
     return launch_status();
 }
 
