@@ -270,6 +270,31 @@ def test_gemm_bf16_few_rows_at_the_edges_of_the_waves_shares(gpu, N, K):
         assert torch.equal(acc[:2], 1 + whole[:min(M, 2)])
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 2048, 2048), (80, 5632, 1024), (300, 2570, 640), (700, 6144, 512), (1500, 4096, 128), (2048, 5632, 192),
+                                   (2048, 136, 64), (4100, 520, 256)])
+@pytest.mark.parametrize("bias", [True, False])
+def test_gemm_bias_and_activation_in_the_products_own_kernel(gpu, M, N, K, bias):
+    """Every shape of block, columns that fill no block and no four: the bits of the product into float32 and the kernel that
+    adds the bias, applies the activation and rounds; an output that is not a whole number of blocks is written nowhere else."""
+    from tuff_amd.csrc import ops
+    if not ops.gemm_bias_supported(M, N, K):
+        pytest.skip("a product in slices of K")
+    x, w = _r(M, K, seed=1, dtype=torch.bfloat16).to(gpu), ops.tile_weight(_r(N, K, seed=2, dtype=torch.bfloat16).to(gpu))
+    b = _r(N, seed=3).to(gpu) if bias else None
+    sums = torch.empty(M, N, device=gpu)
+    ops.gemm(x, w, sums)
+    for activation in (None, "relu2"):
+        room = torch.full((M * N + 512,), 7.0, dtype=torch.bfloat16, device=gpu)
+        out, want = room[:M * N].view(M, N), torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+        ops.gemm_bias(x, w, out, b, activation=activation)
+        if activation:
+            ops.act_rows(sums, want, activation, bias=b)
+        else:
+            ops.cast(sums, want, bias=b)
+        assert torch.equal(out, want), activation
+        assert (room[M * N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("N,K,most", [(2048, 8192, 8), (520, 4104, 16), (2048, 4480, 15), (72, 16392, 4), (2048, 256, 16)])
 def test_gemm_bf16_few_rows_that_lie_in_lds_in_whole(gpu, N, K, most):
     """Inner sizes of many chunks a wave, whole and ragged, up to the most rows that fit (one more, where there may be, comes from memory as before):

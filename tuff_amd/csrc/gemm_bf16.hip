@@ -121,8 +121,11 @@ struct TiledExtra {
     const float* ss_in = nullptr; int n_ss = 0; float eps = 0.f;
     int ss_rows = 0;                      // rows of a group of sums in ss_in (0: M; 64 where a product of at most 64 rows left them)
     const float* emit_nw = nullptr; bf16_t* emit_xw = nullptr; float* emit_ss = nullptr;
+    const float* bias = nullptr;          // TILED_BIAS, TILED_RELU2: [N] or null
 };
-enum : int { TILED_PLAIN = 0, TILED_SCALED = 1, TILED_EMIT = 2 };
+// TILED_BIAS: v + bias[column], rounded to bfloat16; TILED_RELU2: the square of its positive part, rounded.  As a kernel of their
+// own each wrote and read the float32 sums once more (2,048 rows of 5,632 columns: 15 us beside a product of 50).
+enum : int { TILED_PLAIN = 0, TILED_SCALED = 1, TILED_EMIT = 2, TILED_BIAS = 3, TILED_RELU2 = 4 };
 
 template <int TM, int TN, int WAVES_M, int WAVES_N, int AHEAD, int MODE>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_tiled_kernel(
@@ -531,6 +534,16 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         }
         return;
     }
+    f32x4 col_bias[AROUND == TILED_BIAS || AROUND == TILED_RELU2 ? TN : 1];
+    if constexpr (AROUND == TILED_BIAS || AROUND == TILED_RELU2) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const long long col = n0 + wn + j * 16 + g * 4 + e;
+                col_bias[j][e] = ex.bias && col < N ? ex.bias[col] : 0.f;
+            }
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         float sc = 1.f;
@@ -539,6 +552,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         for (int j = 0; j < TN; ++j) {
             f32x4 v = acc[i][j];
             if constexpr (AROUND == TILED_SCALED) { v[0] *= sc; v[1] *= sc; v[2] *= sc; v[3] *= sc; }
+            if constexpr (AROUND == TILED_BIAS || AROUND == TILED_RELU2) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] += col_bias[j][e];
+                    if constexpr (AROUND == TILED_RELU2) { v[e] = fmaxf(v[e], 0.f); v[e] *= v[e]; }
+                }
+            }
             store_quad<MODE>(Y, m0 + wm + i * 16 + r16, n0 + wn + j * 16 + g * 4, M, N, v);
         }
     }
@@ -1646,6 +1666,9 @@ int tiled_emit_group(int M, int N, int K) {
     return bn;                                          // a workgroup's columns
 }
 
+// A product of more than 64 rows in one piece can add a bias to its sums and take the square of their positive part.
+bool tiled_bias_ok(int M, int N, int K) { return M > 64 && dma_ok(K) && plan_tiled(M, N, K).slices <= 1; }
+
 bool tiled_scaled_ok(int M, int N, int K) { return dma_ok(K) || plan_tiled(M, N, K).slices > 1; }
 
 template <int MODE, int AROUND = TILED_PLAIN>
@@ -1686,6 +1709,9 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
             hipLaunchKernelGGL(kern, dim3(ceil_div(N, bn), ceil_div(M, bm), t.slices), dim3(64 * WM * WN), lds, stream, \
                                X, W, Y, M, N, K, t.steps_per_slice, ws, ex); \
         } while (0)
+        if constexpr (AROUND == TILED_BIAS || AROUND == TILED_RELU2) {
+            if (!dma_ok(K) || t.slices > 1) return -2;
+        }
         if constexpr (AROUND != TILED_PLAIN) {
             if (!dma_ok(K) && t.slices == 1) return -2;            // a product in slices is finished by the kernel that adds them
         }
@@ -1703,7 +1729,7 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
         else TILED(4, 2, 2, 4, 4);
 #undef TILED_DMA
 #undef TILED
-        if (t.slices > 1) {
+        if constexpr (AROUND != TILED_BIAS && AROUND != TILED_RELU2) if (t.slices > 1) {
             int rc = launch_status();
             if (rc) return rc;
             FinishExtra fx;
@@ -1772,6 +1798,21 @@ TUFF_EXPORT int tuff_gemm_bf16_workspace(int M, int N, int K, int emit, long lon
 
 // W: tile-major, as described at the head of this file (ceil(N/16) * ceil(K/32) blocks of 1 KB).
 // K must be a multiple of 8 (16-byte operand loads), here and below, and at most 2^24 - 64 (else -2); the host wrapper refuses other K.
+// Y = bf16(X W^T + bias), or with square_positive bf16(max(X W^T + bias, 0)^2), for the products of which
+// tuff_gemm_bf16_bias_supported says so.  bias float32 [N] or null.
+TUFF_EXPORT int tuff_gemm_bf16_bias_supported(int M, int N, int K) {
+    return M > 0 && N > 0 && inner_ok(K) && tiled_bias_ok(M, N, K) ? 1 : 0;
+}
+TUFF_EXPORT int tuff_gemm_bf16_bias(const void* X, const void* W, void* Y, int M, int N, int K, const float* bias, int square_positive,
+                                    hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (!inner_ok(K) || !tiled_bias_ok(M, N, K)) return -2;
+    TiledExtra ex;
+    ex.bias = bias;
+    if (square_positive) return launch_mode<OUT_BF16, TILED_RELU2>((const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, nullptr, stream, ex);
+    return launch_mode<OUT_BF16, TILED_BIAS>((const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, nullptr, stream, ex);
+}
+
 TUFF_EXPORT int tuff_gemm_bf16(const void* X, const void* W, void* Y, int M, int N, int K, int mode,
                                float* ws, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;

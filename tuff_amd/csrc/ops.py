@@ -84,6 +84,8 @@ _SIGNATURES = {
     },
     "gemm_bf16": {
         "tuff_gemm_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p],
+        "tuff_gemm_bf16_bias_supported": [_c_int, _c_int, _c_int],
+        "tuff_gemm_bf16_bias": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_int, _c_void_p],
         "tuff_gemm_bf16_workspace": [_c_int, _c_int, _c_int, _c_int, ctypes.POINTER(_c_ll)],
         "tuff_gemm_bf16_emit_layout": [_c_int, _c_int, _c_int, ctypes.POINTER(_c_int), ctypes.POINTER(_c_int)],
         "tuff_gemm_bf16_scaled_supported": [_c_int, _c_int, _c_int],
@@ -607,6 +609,32 @@ def gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     ws = _gemm_workspace(M, N, K, x.device)
     _check(load("gemm_bf16").tuff_gemm_bf16(x.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, mode,
                                             None if ws is None else ws.data_ptr(), _stream()), "gemm_bf16")
+
+
+_bias_ok: dict = {}
+
+
+def gemm_bias_supported(M: int, N: int, K: int) -> bool:
+    """Whether gemm_bias takes this product: more than 64 rows, in one piece."""
+    if M <= 64 or K % 8:
+        return False
+    key = (M, N, K)
+    if key not in _bias_ok:
+        _bias_ok[key] = bool(load("gemm_bf16").tuff_gemm_bf16_bias_supported(M, N, K))
+    return _bias_ok[key]
+
+
+def gemm_bias(x: torch.Tensor, w, out: torch.Tensor, bias: Optional[torch.Tensor], *, activation: Optional[str] = None) -> None:
+    """out = bf16(x @ w.T + bias), or with activation "relu2" bf16(max(x @ w.T + bias, 0)^2), from the float32 sums in the
+    product's kernel.  x, w, out bfloat16; bias float32 [N] or None."""
+    M, K = x.shape
+    N = w.shape[0]
+    if activation not in (None, "relu2") or not gemm_bias_supported(M, N, K):
+        raise KernelError(f"gemm_bias: a product of {M} rows, {N} outputs, inner size {K} with {activation or 'no activation'} is not supported")
+    w = _tiled(w, N, K)
+    _check(load("gemm_bf16").tuff_gemm_bf16_bias(
+        _gpu("x", x, torch.bfloat16), w.data_ptr(), _gpu("out", out, torch.bfloat16, (M, N)), M, N, K,
+        _opt("bias", bias, torch.float32, (N,)), int(activation == "relu2"), _stream()), "gemm_bias")
 
 
 NORMED_MAX_ROWS, NORMED_MAX_K = 16, 8192      # gemm_normed: the norm inside the product's kernel

@@ -202,9 +202,12 @@ class DenseMLP(FeedForward):
             self.params = torch.log1p(torch.exp(-z.abs())).add(z.clamp_min(0)).float().contiguous()      # softplus, rounded once
 
     def forward(self, h, ctx, residual, next_norm=None, bias_preloaded: bool = False) -> None:
-        u = self.up.forward(h, out_dtype=torch.float32)          # the activation reads the sums as they are, plus the bias
-        act = self.rt.empty(u.shape[0], self.width)
-        ops.act_rows(u, act, self.activation, bias=self.up_bias, params=self.params)
+        # the activation reads the sums as they are, plus the bias
+        act = self.up.forward_activated(h, self.activation, self.up_bias) if self.params is None else None
+        if act is None:
+            u = self.up.forward(h, out_dtype=torch.float32)
+            act = self.rt.empty(u.shape[0], self.width)
+            ops.act_rows(u, act, self.activation, bias=self.up_bias, params=self.params)
         if self.output_bias is None or bias_preloaded:
             self.down.forward(act, accumulate_into=residual, next_norm=next_norm)
             return

@@ -118,6 +118,17 @@ class Linear:
             ops.gemm_conv64(x, self.weight, y, conv_w=conv_w, state=state, state_slot=state_slot, **kw)
         return y
 
+    def forward_activated(self, x, activation: str, bias: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
+        """act(x W^T + bias) [T, out] in bfloat16, from the float32 sums in the product's own kernel, or None where that needs the
+        separate kernels (nothing is launched then).  x [T, in]; for a projection without a bias of its own."""
+        w = self.weight
+        if (activation != "relu2" or not isinstance(x, torch.Tensor) or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16
+                or self.bias is not None or x.shape[1] != self.k_padded or not ops.gemm_bias_supported(x.shape[0], self.out_features, self.k_padded)):
+            return None
+        y = torch.empty(x.shape[0], self.out_features, dtype=torch.bfloat16, device=w.device)
+        ops.gemm_bias(x, w, y, bias, activation=activation)
+        return y
+
     def forward(self, x, *, out_dtype: Optional[torch.dtype] = None,
                 accumulate_into: Optional[torch.Tensor] = None, swiglu: bool = False,
                 next_norm=None) -> Optional[torch.Tensor]:
@@ -193,6 +204,10 @@ class Linear:
             return y
         if self.bias is not None and want != torch.float32:
             # the bias goes onto the float32 sum, which is then rounded once
+            if x.dtype == want == torch.bfloat16 and not swiglu and ops.gemm_bias_supported(T, self.out_features, self.k_padded):
+                y = torch.empty(T, width, dtype=want, device=dev)
+                ops.gemm_bias(x, w, y, self.bias)
+                return y
             y32 = torch.empty(T, width, dtype=torch.float32, device=dev)
             product(y32)
             y = torch.empty(T, width, dtype=want, device=dev)
