@@ -295,6 +295,45 @@ def test_gemm_bias_and_activation_in_the_products_own_kernel(gpu, M, N, K, bias)
         assert (room[M * N:] == 7.0).all()
 
 
+@pytest.mark.parametrize("M,N,K,steps", [
+    (65, 2048, 3136, 9), (300, 2048, 4096, 13), (330, 1536, 3136, 9), (512, 1024, 4160, 9),      # 64 x 64, the slices added inside
+    (321, 4608, 192, 0), (65, 16384, 64, 0), (450, 2560, 128, 0), (512, 3072, 1536, 0),          # 64 x 128
+    (1050, 13824, 128, 0), (3000, 2048, 3136, 0), (2180, 2304, 3200, 0),                         # 128 x 256
+    (1300, 4608, 320, 0), (4100, 2048, 64, 0), (700, 21504, 64, 0), (4200, 5376, 64, 0)])         # blocks in bands
+def test_gemm_bf16_block_shapes_and_orders_give_the_same_bits(gpu, M, N, K, steps):
+    """Blocks that end beyond the matrix, slices and bands that are not whole: the bits of 128 x 128 blocks in the grid's order, or
+    (steps of 64 a slice) of the sums of the slices of K, each by such blocks, added one to the other; into the residual stream too."""
+    from tuff_amd.csrc import ops
+    force = ops.load("gemm_bf16").tuff_gemm_bf16_force_tiled_shape
+    x, w = _r(M, K, seed=1, dtype=torch.bfloat16).to(gpu), _r(N, K, seed=2, dtype=torch.bfloat16).to(gpu)
+    want, part = torch.zeros(M, N, device=gpu), torch.empty(M, N, device=gpu)
+    before = force(1)
+    try:
+        for k in range(0, K, 64 * steps or K):
+            ops.gemm(x[:, k:k + (64 * steps or K)].contiguous(), ops.tile_weight(w[:, k:k + (64 * steps or K)].contiguous()), part)
+            want += part
+    finally:
+        force(before)
+    tiled = ops.tile_weight(w)
+    room = torch.full((M * N + 512,), 7.0, device=gpu)
+    ops.gemm(x, tiled, room[:M * N].view(M, N))
+    assert torch.equal(room[:M * N].view(M, N), want) and (room[M * N:] == 7.0).all()
+    layout = ops.gemm_emit_layout(M, N, K)
+    if layout is not None:
+        y, nw, xw = _r(M, N, seed=3).to(gpu), _r(N, seed=4).to(gpu), torch.empty(M, N, dtype=torch.bfloat16, device=gpu)
+        ss, new = torch.full(layout, 7.0, device=gpu), y + want
+        ops.gemm_accum_emit(x, tiled, y, nw, xw, ss)
+        assert torch.equal(y, new) and torch.equal(xw, (new * nw).bfloat16())
+        exact = new.double().square().sum(1)
+        assert ((ss.double().sum(0) - exact).abs() <= N * 2.0 ** -24 * exact).all()
+    if N % 32 == 0:
+        sums, out, plain = torch.full((20, M), K / 20.0, device=gpu), torch.empty(M, N // 2, dtype=torch.bfloat16, device=gpu), None
+        ops.gemm_scaled(x, sums, 0.0, tiled, out, swiglu=True)                    # every row's scale is 1
+        plain = torch.empty_like(out)
+        ops.gemm(x, tiled, plain, swiglu=True)
+        assert torch.equal(out, plain)
+
+
 @pytest.mark.parametrize("N,K,most", [(2048, 8192, 8), (520, 4104, 16), (2048, 4480, 15), (72, 16392, 4), (2048, 256, 16)])
 def test_gemm_bf16_few_rows_that_lie_in_lds_in_whole(gpu, N, K, most):
     """Inner sizes of many chunks a wave, whole and ragged, up to the most rows that fit (one more, where there may be, comes from memory as before):

@@ -121,6 +121,7 @@ struct TiledExtra {
     const float* ss_in = nullptr; int n_ss = 0; float eps = 0.f;
     int ss_rows = 0;                      // rows of a group of sums in ss_in (0: M; 64 where a product of at most 64 rows left them)
     const float* emit_nw = nullptr; bf16_t* emit_xw = nullptr; float* emit_ss = nullptr;
+    int bands = 0;                        // the order of the blocks (bands_of_rows)
     const float* bias = nullptr;          // TILED_BIAS, TILED_RELU2: [N] or null
 };
 // TILED_BIAS: v + bias[column], rounded to bfloat16; TILED_RELU2: the square of its positive part, rounded.  As a kernel of their
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_tiled_kernel
 // global loads, and it waits for more of them.  Buffers win where the whole grid runs side by side, one block a CU, and K is
 // short, and with the blocks of 256 x 256; they lose a little where the operands come slower than the waves could go on:
 // see dma_through_buffer.
-template <int TM, int TN, int WAVES_M, int WAVES_N, int STAGES, bool BUFFER, int MODE, int AROUND>
+template <int TM, int TN, int WAVES_M, int WAVES_N, int STAGES, bool BUFFER, bool FOLDS, int MODE, int AROUND>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* __restrict__ Y, int M, int N, int K,
         int steps_per_slice, float* __restrict__ ws, TiledExtra ex) {
@@ -302,13 +303,31 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int wm = (wave / WAVES_N) * 16 * TM, wn = (wave % WAVES_N) * 16 * TN;
     const int r16 = lane % 16, g = lane / 16;
-    const long long m0 = (long long)blockIdx.y * BM, n0 = (long long)blockIdx.x * BN;
+    constexpr bool BANDS = BM >= 256 || BN >= 256;
+    // ex.bands (bands_of_rows): an eighth of the blocks, one behind the other, an XCD (block id % 8), bands of eight row blocks,
+    // in a band column by column
+    unsigned bx = blockIdx.x, by = blockIdx.y;
+    if (BANDS && ex.bands) {
+        const unsigned all = gridDim.x * gridDim.y, id = bx + gridDim.x * by, xcd = id % 8;
+        const unsigned at = xcd * (all / 8) + min(xcd, all % 8) + id / 8;
+        const unsigned band = at / (8 * gridDim.x), rest = at - band * (8 * gridDim.x), rows = min(8u, gridDim.y - 8 * band);
+        bx = rest / rows;
+        by = 8 * band + rest % rows;
+    }
+    const long long m0 = (long long)by * BM, n0 = (long long)bx * BN;
 
     f32x4 acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // FOLDS: a block in the place of slices of K adds them itself: a sum each, in the order of the kernel that adds slices, so
+    // the same bits.
+    f32x4 folded[FOLDS ? TM : 1][FOLDS ? TN : 1];
+#pragma unroll
+    for (int i = 0; i < (FOLDS ? TM : 1); ++i)
+#pragma unroll
+        for (int j = 0; j < (FOLDS ? TN : 1); ++j) folded[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const int kb = K / 32;
     const int last_a = (int)min((long long)BM - 1, (long long)M - 1 - m0);
@@ -333,10 +352,25 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     const buffer_t xbuf = make_buffer(X + m0 * K, (last_a + 1) * K * 2);
     const buffer_t wbuf = make_buffer(W + (n0 / 16) * (long long)kb * 512, (last_tile + 1) * kb * 1024);
     const int nk = K / TBK;
-    const int kt_begin = blockIdx.z * steps_per_slice, kt_end = min(nk, kt_begin + steps_per_slice);
+    const int kt_begin = blockIdx.z * steps_per_slice, kt_end = FOLDS ? nk : min(nk, kt_begin + steps_per_slice);
+    int fold_at = kt_begin + steps_per_slice;                          // the step that the next slice begins with (FOLDS)
 
     const bf16_t* Xb = X + m0 * K;
     const bf16_t* Wb = W + (n0 / 16) * (long long)kb * 512;
+    // TILED_EMIT, small blocks: what the epilogue adds to and multiplies with is asked for ahead of the operands (rows beyond
+    // the matrix: the last one's, never used); behind the loop it would be a trip to memory more
+    // (512 rows, 2,048 x 2,048 11.1 and 10.9 us, x 4,096 17.0 and 16.9; 128 x 128 blocks are no faster for it).
+    constexpr bool EARLY = AROUND == TILED_EMIT && BM == 64;
+    f32x4 y_old[EARLY ? TM : 1][EARLY ? TN : 1], next_w[EARLY ? TN : 1];
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            next_w[j] = *(const f32x4*)(ex.emit_nw + n0 + wn + j * 16 + g * 4);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                y_old[i][j] = *(const f32x4*)((const float*)Y + min(m0 + wm + i * 16 + r16, (long long)M - 1) * N + n0 + wn + j * 16 + g * 4);
+        }
+    }
     auto issue = [&](int buf, int kt) {
 #pragma unroll
         for (int i = 0; i < IA; ++i) {
@@ -443,33 +477,64 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         }
         // read in the epilogue, behind the barriers of the loop (every wave waits for its LDS writes before each)
     }
-    auto products = [&](int buf) {
+    auto fold = [&]() {
+        if constexpr (FOLDS) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    folded[i][j] += acc[i][j];
+                    acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            fold_at += steps_per_slice;
+        }
+    };
+    auto products = [&](int buf, auto first_of_slice) {
         read_half(S0(), buf, S0());
         mult(S1());                                            // the second half of the step before (zeros at first)
         spread();
+        if constexpr (decltype(first_of_slice)::value) fold();
         read_half(S1(), buf, S1());
         mult(S0());
         spread();
     };
     int buf = 0, kt = kt_begin;
-    for (; kt + STAGES - 1 < kt_end; ++kt) {
+    auto step = [&](auto first_of_slice) {
         wait_loads_and_lds<(STAGES - 2) * (IA + IB)>();
         __builtin_amdgcn_s_barrier();
         issue(buf == 0 ? STAGES - 1 : buf - 1, kt + STAGES - 1);
-        products(buf);
+        products(buf, first_of_slice);
         buf = buf + 1 == STAGES ? 0 : buf + 1;
+        ++kt;
+    };
+    const int steady = kt_end - (STAGES - 1);                  // the steps before it have loads to issue
+    if constexpr (FOLDS) {
+        while (kt < steady) {
+            if (kt == fold_at) step(std::true_type());
+            const int until = min(steady, fold_at);
+            while (kt < until) step(std::false_type());
+        }
+    } else {
+        while (kt < steady) step(std::false_type());
     }
     static_for<STAGES - 1>([&](auto i) {                       // the last STAGES - 1 steps, fewer if there are fewer
         constexpr int later = STAGES - 2 - decltype(i)::value;
         if (kt < kt_end - later) {
             wait_loads_and_lds<later * (IA + IB)>();
             __builtin_amdgcn_s_barrier();
-            products(buf);
+            if (FOLDS && kt == fold_at) products(buf, std::true_type());
+            else products(buf, std::false_type());
             buf = buf + 1 == STAGES ? 0 : buf + 1;
             ++kt;
         }
     });
     if (kt_begin < kt_end) mult(S1());
+    if constexpr (FOLDS) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] = folded[i][j] + acc[i][j];
+    }
 
     if (gridDim.z > 1) {
         float* mine = ws + (long long)blockIdx.z * M * N;
@@ -503,11 +568,13 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
                 for (int j = 0; j < TN; ++j) {
                     const long long col = n0 + wn + j * 16 + g * 4;
                     f32x4* yp = (f32x4*)((float*)Y + row * N + col);
-                    f32x4 y = *yp;
+                    f32x4 y;
+                    if constexpr (EARLY) y = y_old[i][j]; else y = *yp;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) y[e] += acc[i][j][e];
                     *yp = y;
-                    const f32x4 nw = *(const f32x4*)(ex.emit_nw + col);
+                    f32x4 nw;
+                    if constexpr (EARLY) nw = next_w[j]; else nw = *(const f32x4*)(ex.emit_nw + col);
                     bf16x4 o = {(bf16_t)(y[0] * nw[0]), (bf16_t)(y[1] * nw[1]), (bf16_t)(y[2] * nw[2]), (bf16_t)(y[3] * nw[3])};
                     *(bf16x4*)(ex.emit_xw + row * N + col) = o;
 #pragma unroll
@@ -530,7 +597,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
             float t = red[r];
 #pragma unroll
             for (int w = 1; w < WAVES_N; ++w) t += red[w * BM + r];
-            if (m0 + r < M) ex.emit_ss[(long long)blockIdx.x * M + m0 + r] = t;
+            if (m0 + r < M) ex.emit_ss[(long long)bx * M + m0 + r] = t;
         }
         return;
     }
@@ -1449,8 +1516,8 @@ SkinnyPlan plan_skinny(int M, int N, int K, int max_waves = 16, bool emit = fals
 
 // How a product of more than 64 rows is cut: shape 0: 256 x 256 blocks; 1: 128 x 128 blocks, two a CU;
 // 2: 128 x 128 blocks, one a CU, four steps of operands under way; 3: 64 x 64 blocks of four waves;
-// 4: 256 x 192 blocks.
-// Depends on the sizes only.
+// 4: 256 x 192 blocks; 5: 128 x 256 blocks, three steps under way; 6: 64 x 128 blocks of four waves.
+// Depends on the sizes only.  One slice of fewer steps than K has: the block adds the slices itself (shape 3).
 struct TiledPlan { int shape, slices, steps_per_slice; long long ws_floats; };
 
 int tiled_shape_forced = -1;       // >= 0: every tiled product takes this shape (measurements only)
@@ -1463,29 +1530,49 @@ TiledPlan plan_tiled(int M, int N, int K) {
     t.shape = large >= 160 ? 0 : small > 256 ? 1 : 2;
     t.slices = 1; t.steps_per_slice = nk; t.ws_floats = 0;
     if (tiled_shape_forced >= 0 && dma_ok(K)) { t.shape = tiled_shape_forced; return t; }
-    // blocks of 256 x 192 where they need fewer rounds of 256 workgroups times columns than 256 x 256
-    // (6144 columns and 2048 rows: 256 blocks, one round, instead of 192 blocks that leave a quarter of the CUs idle)
-    if (t.shape == 0 && dma_ok(K)) {
+    if ((t.shape == 0 || (t.shape == 1 && small > 512)) && dma_ok(K)) {
         const long long wide = (long long)ceil_div(N, 192) * ceil_div(M, 256);
-        if (ceil_div(wide, 256) * 192 < ceil_div(large, 256) * 256) t.shape = 4;
+        // blocks of 256 x 192 where they need fewer rounds of 256 workgroups times columns than 256 x 256
+        // (6144 columns and 2048 rows: 256 blocks, one round, instead of 192 blocks that leave a quarter of the CUs idle), and for
+        // a little more than one round of pairs of 128 x 128 blocks (512 of them side by side), where the blocks beyond the round
+        // would run a second one almost alone (4608 columns and 2048 rows, K = 1536: 37.1 us instead of 43.8; 256 x 256: 45.7)
+        if (t.shape == 0 ? ceil_div(wide, 256) * 192 < ceil_div(large, 256) * 256 : wide <= 256) t.shape = 4;
+        // Whole blocks of 128 x 256: the shape whose rounds cost least, of 256 x 256, 256 x 192 and 128 x 256 blocks, as measured a
+        // round and step 1.72, 1.39 and 0.97 us (alike with 1,536 to 8,192 of K; a smaller block reads its operands for
+        // fewer products).  Halves of a round instead of a round almost empty: 1,050 rows 13,824 x 1,536 64.5 -> 48.7 us, 21,504 x 2,048 106 ->
+        // 96, 1,300 rows 16,384 x 2,048 108 -> 90, 1,536 109 -> 94; 256 x 192 instead of 256 x 256, 1,050 rows, 96.5 -> 84.
+        if (N % 256 == 0) {
+            const long long cost0 = 17 * ceil_div(large, 256), cost4 = 14 * ceil_div(wide, 256);
+            const long long cost5 = 10 * ceil_div((long long)(N / 256) * ceil_div(M, 128), 256);
+            t.shape = cost5 < cost0 && cost5 < cost4 ? 5 : cost4 < cost0 ? 4 : 0;
+        }
         return t;
     }
-    // A little more than one round of pairs of 128 x 128 blocks (512 of them side by side), where blocks of 256 x 256
-    // would be too few for the CUs: the blocks beyond the round run a second one almost alone.  Blocks of 256 x 192
-    // in one round instead (4608 columns and 2048 rows, K = 1536: 37.1 us instead of 43.8; 256 x 256: 45.7).
-    if (t.shape == 1 && small > 512 && dma_ok(K)) {
-        const long long wide = (long long)ceil_div(N, 192) * ceil_div(M, 256);
-        if (wide <= 256) { t.shape = 4; return t; }
-    }
+    // One round of 128 x 256 blocks in the place of one of pairs of 128 x 128, where K is long: the pairs read an operand once more and
+    // wait for it (2,048 x 8,192 of 2,560 rows 112 -> 103 us, 3,000 125 -> 101, 4,096 131 -> 110; 2,048 x 2,048 28.6 and 28.5, 29.5 and
+    // 29.3, 34.2 and 33.4, 3,072 x 2,048 of 1,536 rows 27.2 and 28.3).
+    if (t.shape == 1 && dma_ok(K) && N % 256 == 0 && nk > 48) { t.shape = 5; return t; }
     // few blocks and a short K: blocks of 64 x 64 give enough workgroups without slices of K, whose partial
     // tiles cost a second kernel and as much traffic as the product's own (K = 1536 .. 2048, 96 to 512
     // rows: 9 to 14 us instead of 11 to 19); beyond 48 steps the slices win
-    if (t.shape == 2 && small <= 128 && dma_ok(K) && nk <= 48) { t.shape = 3; return t; }
+    const long long least = (long long)ceil_div(N, 64) * ceil_div(M, 64);
+    if (t.shape == 2 && small <= 128 && dma_ok(K) && nk <= 48) {
+        // beyond a round of them one block of 64 x 128 a CU: the second round's few take as long as the first's (400 rows, 4,608 x 1,536:
+        // 14.3 us -> 11.2, 300 rows, 6,144 x 2,048 17.1 -> 13.1, 100 rows, 16,384 x 2,048 21.6 -> 18.9; 280 blocks of 64 x 64 9.7 and 10.3)
+        t.shape = least > 288 && N % 128 == 0 && (long long)(N / 128) * ceil_div(M, 64) <= 256 ? 6 : 3;
+        return t;
+    }
     if (t.shape == 2 && small <= 128) {
         // as many slices as give every CU at most one block, at least eight steps a slice
         int s = max(1, min((int)(256 / small), nk / 8));
         t.steps_per_slice = ceil_div(nk, s);
         t.slices = ceil_div(nk, t.steps_per_slice);
+        // A longer K still in blocks of 64 x 64 that add the slices themselves, where the partial tiles would cost more (their bytes grow
+        // with rows and columns, a block's time with K).  Slices and 64 x 64 into the residual stream, us: 2,048 x 3,584 of 100 rows 13.6 and
+        // 14.0, 200 16.1 and 14.4, 512 19.9 and 15.9; x 4,096 of 100 rows 14.5 and 14.9, 200 16.4 and 15.4, 512 20.4 and 16.9; x 5,632 of 300
+        // rows 19.2 and 20.3, 400 21.4 and 20.9, 512 24.5 and 21.8; 1,536 x 6,912 of 300 rows 21.7 and 22.9, 600 27.0 and 24.6;
+        // 2,048 x 8,192 of 400 rows 25.2 and 28.1, 512 28.6 and 29.2.
+        if (dma_ok(K) && N % 64 == 0 && least <= 256 && 2 * least > 5 * (nk - 24)) { t.shape = 3; t.slices = 1; return t; }
         if (t.slices > 1) t.ws_floats = (long long)t.slices * M * N;
     }
     return t;
@@ -1498,11 +1585,23 @@ TiledPlan plan_tiled(int M, int N, int K) {
 // 16,384 x 2,048); 128 x 128, two a CU, within 1 %.
 bool dma_through_buffer(const TiledPlan& t, int M, int N) {
     if (t.shape == 4) return false;
+    if (t.shape == 5 || t.shape == 6) return true;
     if (t.shape == 3) {
         const long long blocks = (long long)ceil_div(M, 64) * ceil_div(N, 64);
         return blocks <= 256 || blocks > 448;
     }
     return t.shape != 2 || t.steps_per_slice <= 64;
+}
+
+// The order of the blocks of 256 rows or columns.  As the grid counts them an XCD takes every eighth: the same columns again and again
+// where their number is a multiple of eight, else a new mixture a row, and each XCD's L2 reads nearly all of W.  In bands of
+// eight row blocks an XCD has neighbours in both directions.  As counted / in bands, us: 1,050 rows, 16,384 x 2,048 (86 blocks
+// of columns) 96.2 and 84.0; 20,001 rows, 13,824 x 1,536 791 and 741, 6,144 x 2,048 512 and 461, 2,048 x 2,048 171 and 160; 8,192 rows,
+// 2,048 x 8,192 241 and 200.  Few rows and a multiple of eight: 3,000 rows, 6,144 x 2,048 81.0 and 83.9, 520 rows, 16,384 x 2,048 53.4 and
+// 54.6.  The smaller blocks lose (128 x 128 2 to 5 % up to 2,000 rows, 64 x 64 up to 10).
+bool bands_of_rows(const TiledPlan& t, int M, int N) {
+    if (t.shape != 0 && t.shape != 4 && t.shape != 5) return false;
+    return ceil_div(N, t.shape == 4 ? 192 : 256) % 8 != 0 || ceil_div(M, t.shape == 5 ? 128 : 256) >= 16;
 }
 
 struct Skinny16Extra {
@@ -1661,7 +1760,7 @@ int tiled_emit_group(int M, int N, int K) {
     const TiledPlan t = plan_tiled(M, N, K);
     if (t.slices > 1) return 64;                        // the kernel that adds the slices emits, 64 columns a workgroup
     if (!dma_ok(K)) return 0;
-    const int bn = t.shape == 0 ? 256 : t.shape == 4 ? 192 : t.shape == 3 ? 64 : 128;
+    const int bn = t.shape == 0 || t.shape == 5 ? 256 : t.shape == 4 ? 192 : t.shape == 3 ? 64 : 128;
     if (N % bn != 0) return 0;
     return bn;                                          // a workgroup's columns
 }
@@ -1673,7 +1772,7 @@ bool tiled_scaled_ok(int M, int N, int K) { return dma_ok(K) || plan_tiled(M, N,
 
 template <int MODE, int AROUND = TILED_PLAIN>
 int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, float* ws, hipStream_t stream,
-                const TiledExtra& ex = TiledExtra()) {
+                TiledExtra ex = TiledExtra()) {
     if constexpr (AROUND == TILED_PLAIN) {
         if (few_rows_kernel(M, N, K)) return launch_skinny16<MODE, NORM_NONE, false>(X, W, Y, M, N, K, Skinny16Extra(), stream);
         if (M <= 64 && !rows64_tiled(M, N, K)) return launch_skinny64<MODE, NORM_NONE, false>(X, W, Y, M, N, K, ws, FinishExtra(), stream);
@@ -1687,6 +1786,7 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
         TiledPlan t = plan_tiled(M, N, K);
         if (rows64_tiled(M, N, K)) { t.shape = 3; t.slices = 1; t.steps_per_slice = ceil_div(K, TBK); t.ws_floats = 0; }
         if (t.slices > 1 && !ws) return -4;
+        ex.bands = bands_of_rows(t, M, N);
 #define TILED(TM, TN, WM, WN, AHEAD) do { \
             auto kern = gemm_bf16_tiled_kernel<TM, TN, WM, WN, AHEAD, MODE>; \
             constexpr int bm = 16 * TM * WM, bn = 16 * TN * WN, lds = 2 * (bm + bn) * TBK * 2; \
@@ -1698,8 +1798,8 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
             hipLaunchKernelGGL(kern, dim3(ceil_div(N, bn), ceil_div(M, bm), t.slices), dim3(64 * WM * WN), lds, stream, \
                                X, W, Y, M, N, K, t.steps_per_slice, ws); \
         } while (0)
-#define TILED_DMA(TM, TN, WM, WN, STAGES, BUFFER) do { \
-            auto kern = gemm_bf16_dma_kernel<TM, TN, WM, WN, STAGES, BUFFER, MODE, AROUND>; \
+#define TILED_DMA(TM, TN, WM, WN, STAGES, BUFFER, FOLDS) do { \
+            auto kern = gemm_bf16_dma_kernel<TM, TN, WM, WN, STAGES, BUFFER, FOLDS, MODE, AROUND>; \
             constexpr int bm = 16 * TM * WM, bn = 16 * TN * WN, lds = STAGES * (bm + bn) * TBK * 2; \
             static bool set = false; \
             if (!set) { \
@@ -1717,12 +1817,15 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
         }
         if (dma_ok(K)) {
             const bool buffer = dma_through_buffer(t, M, N);
-            if (t.shape == 3) { if (buffer) TILED_DMA(2, 2, 2, 2, 4, true); else TILED_DMA(2, 2, 2, 2, 4, false); }
-            else if (t.shape == 4) TILED_DMA(8, 3, 2, 4, 2, false);
-            else if (t.shape == 0) TILED_DMA(8, 4, 2, 4, 2, true);
-            else if (t.shape == 1) TILED_DMA(4, 2, 2, 4, 2, true);
-            else if (buffer) TILED_DMA(4, 2, 2, 4, 4, true);
-            else TILED_DMA(4, 2, 2, 4, 4, false);
+            if (t.shape == 3 && t.steps_per_slice < ceil_div(K, TBK)) TILED_DMA(2, 2, 2, 2, 4, true, true);
+            else if (t.shape == 3) { if (buffer) TILED_DMA(2, 2, 2, 2, 4, true, false); else TILED_DMA(2, 2, 2, 2, 4, false, false); }
+            else if (t.shape == 4) TILED_DMA(8, 3, 2, 4, 2, false, false);
+            else if (t.shape == 0) TILED_DMA(8, 4, 2, 4, 2, true, false);
+            else if (t.shape == 1) TILED_DMA(4, 2, 2, 4, 2, true, false);
+            else if (t.shape == 5) TILED_DMA(4, 4, 2, 4, 3, true, false);
+            else if (t.shape == 6) TILED_DMA(4, 2, 1, 4, 4, true, false);
+            else if (buffer) TILED_DMA(4, 2, 2, 4, 4, true, false);
+            else TILED_DMA(4, 2, 2, 4, 4, false, false);
         }
         else if (t.shape == 0) TILED(8, 4, 2, 4, 1);
         else if (t.shape == 1) TILED(4, 2, 2, 4, 1);
@@ -1756,7 +1859,7 @@ TUFF_EXPORT int tuff_gemm_bf16_wide64(int min_n, int max_n, int min_m) {
 }
 
 // For measurements: forces the block shape of every product of more than 64 rows whose K is a multiple
-// of 64 (0: 256 x 256, 1: 128 x 128 two a CU, 2: 128 x 128 one a CU, 3: 64 x 64, 4: 256 x 192; -1: by size).
+// of 64 (0: 256 x 256, 1: 128 x 128 two a CU, 2: 128 x 128 one a CU, 3: 64 x 64, 4: 256 x 192, 5: 128 x 256, 6: 64 x 128; -1: by size).
 // Returns the value before.
 TUFF_EXPORT int tuff_gemm_bf16_force_tiled_shape(int shape) {
     const int old = tiled_shape_forced;
