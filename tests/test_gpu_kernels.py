@@ -100,6 +100,26 @@ def test_gemm_f32_few_rows(gpu, M, N, K):
     assert torch.equal(acc, y0 + out)
 
 
+@pytest.mark.parametrize("F,K", [(8192, 192), (1024, 320), (36, 224), (9, 32), (2050, 64)])
+def test_gemm_f32_with_swiglu_inside(gpu, F, K):
+    """Every kernel on whole chains (one wave of few rows, blocks of 32 and 64), columns that fill no block and no eight: the bits of
+    the product and the kernel that applies SwiGLU, infinities and NaN too; nothing beyond the output is written."""
+    from tuff_amd.csrc import ops
+    w = _r(2 * F, K, seed=2).to(gpu)
+    for M in (1, 3, 4, 5, 16, 17, 33, 200, 321):
+        x = _r(M, K, seed=1).to(gpu)
+        x[M // 2, 3], x[M - 1, 5] = float("inf"), float("nan")
+        gu, want = torch.empty(M, 2 * F, device=gpu), torch.empty(M, F, device=gpu)
+        ops.gemm(x, w, gu)
+        ops.swiglu(gu, want)
+        room = torch.full((M * F + 512,), 7.0, device=gpu)
+        ops.gemm_f32_swiglu(x, w, room[:M * F].view(M, F))
+        assert torch.equal(room[:M * F].view(M, F).nan_to_num(3.0), want.nan_to_num(3.0)) and (room[M * F:] == 7.0).all(), M
+    with pytest.raises(ops.KernelError):
+        ops.gemm_f32_swiglu(x[:, :K - 8].contiguous(), w[:, :K - 8].contiguous(), want)
+    assert not ops.gemm_f32_swiglu_supported(x.flatten()[1:1 + 2 * K].view(2, K), w)
+
+
 def test_gemm_f32_more_rows_than_small_blocks_count(gpu):
     """A narrow output of more rows than a grid has blocks of 32 for takes blocks of 64 (it was refused)."""
     from tuff_amd.csrc import ops

@@ -84,7 +84,13 @@ constexpr int STEP = 32;
 
 constexpr int WAVES = 2;
 
-template <int T, int STAGES>
+//
+// SWIGLU, in all three kernels on whole chains: W holds N / 2 gate rows and then as many up rows, a block takes as many of each,
+// and of the two chains of a column, which lie in one lane or in two of one wave, swiglu_value leaves Y [M, N / 2].  As a
+// kernel of its own that wrote and read [M, N] once more: 4 rows, 16,384 x 2,048: product and SwiGLU
+__device__ __forceinline__ float swiglu_value(float gate, float up) { return gate / (1.0f + expf(-gate)) * up; }
+
+template <int T, int STAGES, bool SWIGLU>
 __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(const float* __restrict__ X, const float* __restrict__ W,
                                                                               float* __restrict__ Y, int M, int N, int K, int accumulate) {
     constexpr int SIDE = 16 * T * WAVES;                  // rows and columns of the block
@@ -98,16 +104,21 @@ __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(co
     const int r16 = lane % 16, g = lane / 16;
     const long long m0 = (long long)blockIdx.y * SIDE, n0 = (long long)blockIdx.x * SIDE;
     const int last_m = (int)min((long long)SIDE - 1, (long long)M - 1 - m0);
-    const int last_n = (int)min((long long)SIDE - 1, (long long)N - 1 - n0);
+    // SWIGLU: half the block's rows of W are gate rows, tile by tile (T = 2) or eight by eight, and their up rows follow them
+    constexpr int RUN = T == 2 ? 16 : 8;
+    const long long h0 = n0 / 2;
+    const int last_n = SWIGLU ? (int)min((long long)SIDE / 2 - 1, (long long)N / 2 - 1 - h0) : (int)min((long long)SIDE - 1, (long long)N - 1 - n0);
     // (rows beyond the matrix read its last row instead: their results are never stored)
     int offx[IN], offw[IN];                               // bytes from the block's first row
 #pragma unroll
     for (int i = 0; i < IN; ++i) {
         const int row = (wave * IN + i) * 8 + lane / 8, piece = (lane % 8) ^ (lane / 8);
         offx[i] = (min(row, last_m) * K + piece * 4) * 4;
-        offw[i] = (min(row, last_n) * K + piece * 4) * 4;
+        const int up = SWIGLU && row / RUN % 2 ? N / 2 : 0;
+        offw[i] = ((up + min(SWIGLU ? row / (2 * RUN) * RUN + row % RUN : row, last_n)) * K + piece * 4) * 4;
     }
-    const buffer_t xbuf = make_buffer(X + m0 * K, (last_m + 1) * K * 4), wbuf = make_buffer(W + n0 * K, (last_n + 1) * K * 4);
+    const buffer_t xbuf = make_buffer(X + m0 * K, (last_m + 1) * K * 4);
+    const buffer_t wbuf = make_buffer(W + (SWIGLU ? h0 : n0) * K, ((SWIGLU ? N / 2 : 0) + last_n + 1) * K * 4);
     const int steps = K / STEP;
     auto issue = [&](int buf, int s) {
 #pragma unroll
@@ -194,6 +205,30 @@ __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(co
         }
     });
     multiply(H1());
+    if constexpr (SWIGLU) {
+        const int half_n = N / 2;
+#pragma unroll
+        for (int i = 0; i < T; ++i) {
+            const long long row = m0 + wm + i * 16 + r16;
+            const long long col = h0 + wn / 2 + g * 4;
+            f32x4 gate = acc[i][0], up;
+            if constexpr (T == 2) up = acc[i][T - 1];
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e) up[e] = __shfl_xor(gate[e], 32);      // (lane groups 0 and 1: gate, 2 and 3: up)
+            if (row >= M || (T == 1 && g >= 2)) continue;
+            float* y = Y + row * half_n + col;
+            f32x4 o;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] = swiglu_value(gate[e], up[e]);
+            if (half_n % 4 == 0 && col + 3 < half_n) *(f32x4*)y = o;
+            else
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (col + e < half_n) y[e] = o[e];
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < T; ++i) {
         const long long row = m0 + wm + i * 16 + r16;
@@ -222,7 +257,7 @@ __global__ __launch_bounds__(WAVES * WAVES * WAVE) void gemm_f32_chain_kernel(co
 // are waited for at once, where they have long arrived, so that no product waits for LDS (the kernel above, half a step ahead:
 // 2,048 x 8,192 of 16 rows 58 us, this one 49; 65,536 x 2,048 of 8 rows 113 and 109, 4.9 TB/s).  Rows beyond X are not
 // fetched.  STAGES: steps of 32 k in LDS, 16 where two workgroups fill a CU's share of the launch anyway.
-template <int STAGES>
+template <int STAGES, bool SWIGLU>
 __global__ __launch_bounds__(WAVE) void gemm_f32_rows_kernel(const float* __restrict__ X, const float* __restrict__ W,
                                                              float* __restrict__ Y, int M, int N, int K, int accumulate) {
     constexpr int TILE = 16 * STEP, PER = 4;              // floats of a tile; load instructions a step
@@ -230,14 +265,16 @@ __global__ __launch_bounds__(WAVE) void gemm_f32_rows_kernel(const float* __rest
     extern __shared__ __attribute__((aligned(16))) float tiles[];      // [STAGES][X, W][TILE]
     const int lane = threadIdx.x, r16 = lane % 16, g = lane / 16;
     const long long n0 = (long long)blockIdx.x * 16;
-    const int rows_n = (int)min(16ll, (long long)N - n0);
-    const buffer_t xbuf = make_buffer(X, M * K * 4), wbuf = make_buffer(W + n0 * K, rows_n * K * 4);
+    const long long h0 = n0 / 2;                          // SWIGLU: eight gate rows, then their up rows
+    const int rows_n = SWIGLU ? (int)min(8ll, (long long)N / 2 - h0) : (int)min(16ll, (long long)N - n0);
+    const buffer_t xbuf = make_buffer(X, M * K * 4), wbuf = make_buffer(W + (SWIGLU ? h0 : n0) * K, ((SWIGLU ? N / 2 : 0) + rows_n) * K * 4);
     int offx[2], offw[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const int row = i * 8 + lane / 8, piece = (lane % 8) ^ (lane / 8);
         offx[i] = row < M ? (row * K + piece * 4) * 4 : NOWHERE;
-        offw[i] = row < rows_n ? (row * K + piece * 4) * 4 : NOWHERE;
+        const int wrow = SWIGLU ? row % 8 : row;
+        offw[i] = wrow < rows_n ? (((SWIGLU && row >= 8 ? N / 2 : 0) + wrow) * K + piece * 4) * 4 : NOWHERE;
     }
     const int steps = K / STEP;
     auto issue = [&](int s) {
@@ -310,6 +347,19 @@ __global__ __launch_bounds__(WAVE) void gemm_f32_rows_kernel(const float* __rest
         ++s;
     });
     const int row = r16;
+    if constexpr (SWIGLU) {
+        const int half_n = N / 2;
+        f32x4 up;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) up[e] = __shfl_xor(acc[e], 32);               // (lane groups 0 and 1: gate, 2 and 3: up)
+        if (row >= M || g >= 2) return;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const long long col = h0 + g * 4 + e;
+            if (col < half_n) Y[(long long)row * half_n + col] = swiglu_value(acc[e], up[e]);
+        }
+        return;
+    }
     if (row >= M) return;
     const long long col = n0 + g * 4;
     float* y = Y + (long long)row * N + col;
@@ -362,7 +412,7 @@ __device__ __forceinline__ void chain16(float& acc, float x, const f32x4 (&w)[4]
 constexpr int LONG_STEP = 64;
 
 // A wave a workgroup; `row_groups` workgroups of one column block on one XCD (numbers eight apart), so that its L2 serves W again.
-template <int STAGES>
+template <int STAGES, bool SWIGLU>
 __global__ __launch_bounds__(WAVE) void gemm_f32_quad_kernel(const float* __restrict__ X, const float* __restrict__ W,
                                                              float* __restrict__ Y, int M, int N, int K, int row_groups, int accumulate) {
     constexpr int WTILE = 16 * LONG_STEP, XTILE = 4 * LONG_STEP, STAGE = WTILE + XTILE;
@@ -374,22 +424,24 @@ __global__ __launch_bounds__(WAVE) void gemm_f32_quad_kernel(const float* __rest
     const long long n0 = (long long)block * 16;
     const int m0 = group * 4;
     if (n0 >= N) return;
-    const int rows_m = min(4, M - m0), rows_n = (int)min(16ll, (long long)N - n0);
+    const long long j0 = n0 / 2;                          // SWIGLU: eight gate rows, then their up rows
+    const int rows_m = min(4, M - m0), rows_n = SWIGLU ? (int)min(8ll, (long long)N / 2 - j0) : (int)min(16ll, (long long)N - n0);
     const int offx = g < rows_m ? (g * K + (r16 ^ (4 * g)) * 4) * 4 : NOWHERE;
     int offw[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int row = i * 4 + g;
-        offw[i] = row < rows_n ? (row * K + (r16 ^ row) * 4) * 4 : NOWHERE;
+        const int row = i * 4 + g, wrow = SWIGLU ? row % 8 : row;
+        offw[i] = wrow < rows_n ? (((SWIGLU && row >= 8 ? N / 2 : 0) + wrow) * K + (r16 ^ row) * 4) * 4 : NOWHERE;
     }
     const int steps = K / LONG_STEP;
     const float* xrows = X + (long long)m0 * K;
-    const float* wrows = W + n0 * K;
+    const float* wrows = W + (SWIGLU ? j0 : n0) * K;
+    const int bytes_w = ((SWIGLU ? N / 2 : 0) + rows_n) * K * 4;
     // Steps beyond the last are asked for too, of buffers without bytes (zeros, no traffic): the count of loads under way is then
     // the same in every step, and the places in LDS are constants of a ring of steps.
     auto issue = [&](auto buf, int s) {
         const bool there = s < steps;
-        const buffer_t xbuf = make_buffer(xrows, there ? rows_m * K * 4 : 0), wbuf = make_buffer(wrows, there ? rows_n * K * 4 : 0);
+        const buffer_t xbuf = make_buffer(xrows, there ? rows_m * K * 4 : 0), wbuf = make_buffer(wrows, there ? bytes_w : 0);
         const int at = there ? s * (LONG_STEP * 4) : 0;
         float* to = tiles + decltype(buf)::value * STAGE;
         load_to_lds(xbuf, to + WTILE, offx, at);
@@ -441,6 +493,11 @@ __global__ __launch_bounds__(WAVE) void gemm_f32_quad_kernel(const float* __rest
             multiply(h1);
         });
     wait_loads_and_lds<0>();                              // nothing may land in LDS that is another workgroup's by then
+    if constexpr (SWIGLU) {
+        const float up = __shfl_xor(acc, 8);
+        if (g < rows_m && r16 < rows_n) Y[(long long)(m0 + g) * (N / 2) + j0 + r16] = swiglu_value(acc, up);
+        return;
+    }
     if (g < rows_m && r16 < rows_n) {
         float* y = Y + (long long)(m0 + g) * N + n0 + r16;
         *y = accumulate ? *y + acc : acc;
@@ -457,32 +514,57 @@ long long block_cycles(int M, int N, int side) {
     return side == 64 ? ceil_div_ll(blocks, CUS) * 170 : max(71ll, blocks * 62 / CUS);
 }
 
-template <int STAGES>
+template <bool SWIGLU, int STAGES>
 int launch_quad(const float* X, const float* W, float* Y, int M, int N, int K, int accumulate, hipStream_t stream) {
     constexpr int lds = STAGES * 20 * LONG_STEP * (int)sizeof(float);
     static_assert(lds <= 65536, "without asking for more");
     const int row_groups = ceil_div(M, 4);
-    hipLaunchKernelGGL((gemm_f32_quad_kernel<STAGES>), dim3(ceil_div(ceil_div(N, 16), 8) * 8 * row_groups), dim3(WAVE), lds, stream,
+    hipLaunchKernelGGL((gemm_f32_quad_kernel<STAGES, SWIGLU>), dim3(ceil_div(ceil_div(N, 16), 8) * 8 * row_groups), dim3(WAVE), lds, stream,
                        X, W, Y, M, N, K, row_groups, accumulate);
     return launch_status();
 }
 
-template <int STAGES>
+template <bool SWIGLU, int STAGES>
 int launch_rows(const float* X, const float* W, float* Y, int M, int N, int K, int accumulate, hipStream_t stream) {
     constexpr int lds = STAGES * 2 * 16 * STEP * (int)sizeof(float);
     static_assert(lds <= 65536, "without asking for more");
-    hipLaunchKernelGGL((gemm_f32_rows_kernel<STAGES>), dim3(ceil_div(N, 16)), dim3(WAVE), lds, stream, X, W, Y, M, N, K, accumulate);
+    hipLaunchKernelGGL((gemm_f32_rows_kernel<STAGES, SWIGLU>), dim3(ceil_div(N, 16)), dim3(WAVE), lds, stream, X, W, Y, M, N, K, accumulate);
     return launch_status();
 }
 
-template <int T, int STAGES>
+template <bool SWIGLU, int T, int STAGES>
 int launch_chain(const float* X, const float* W, float* Y, int M, int N, int K, int accumulate, hipStream_t stream) {
     constexpr int side = 16 * T * WAVES, lds = STAGES * side * STEP * 2 * (int)sizeof(float);
     static_assert(lds <= 65536, "without asking for more");
     dim3 grid(ceil_div(N, side), ceil_div(M, side));
     if (grid.y > 65535) return -2;
-    hipLaunchKernelGGL((gemm_f32_chain_kernel<T, STAGES>), grid, dim3(WAVES * WAVES * WAVE), lds, stream, X, W, Y, M, N, K, accumulate);
+    hipLaunchKernelGGL((gemm_f32_chain_kernel<T, STAGES, SWIGLU>), grid, dim3(WAVES * WAVES * WAVE), lds, stream, X, W, Y, M, N, K, accumulate);
     return launch_status();
+}
+constexpr int LARGEST = 1 << 22;                          // K of the chain kernels (they count the bytes of 64 rows in 31 bits)
+
+constexpr long long SWIGLU_LARGEST = 1ll << 28;           // elements of W (the bytes up to an up row are counted in 31 bits)
+
+// Which of the kernels on whole chains (K a multiple of STEP, operands on 16-byte borders).
+template <bool SWIGLU>
+int launch_whole_chain(const float* X, const float* W, float* Y, int M, int N, int K, int accumulate, hipStream_t stream) {
+    if (M <= 16) {
+        // Four rows a wave as long as one trip over W serves all rows, or the waves are few enough to run side by side, two a CU (16
+        // rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14), and K is not so short that
+        // the empty steps it begins with count (4 rows, 2,048 x 64: 3.2 us and 2.7, x 192 3.6 and 3.5, 32,768 x 192 6.4 and 7.2).
+        // Twelve steps in LDS where a CU has one wave (8,192 x 1,024, two a CU: 11.7 us, with six 10.3).
+        const long long waves = ceil_div_ll(N, 16) * ceil_div(M, 4);
+        if (K % LONG_STEP == 0 && K >= 192 && (M <= 4 || waves <= 512)) {
+            if (waves <= 256) return launch_quad<SWIGLU, 12>(X, W, Y, M, N, K, accumulate, stream);
+            return launch_quad<SWIGLU, 6>(X, W, Y, M, N, K, accumulate, stream);
+        }
+        if (N <= 4096) return launch_rows<SWIGLU, 16>(X, W, Y, M, N, K, accumulate, stream);
+        return launch_rows<SWIGLU, 8>(X, W, Y, M, N, K, accumulate, stream);
+    }
+    constexpr int MOST_BLOCKS = 65535;                    // of rows in a grid
+    if (ceil_div(M, 32) <= MOST_BLOCKS && block_cycles(M, N, 32) < block_cycles(M, N, 64))
+        return launch_chain<SWIGLU, 1, 4>(X, W, Y, M, N, K, accumulate, stream);
+    return launch_chain<SWIGLU, 2, 4>(X, W, Y, M, N, K, accumulate, stream);
 }
 }  // namespace
 
@@ -491,28 +573,19 @@ TUFF_EXPORT int tuff_gemm_f32(const float* X, const float* W, float* Y, int M, i
                               int accumulate, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     const bool aligned = (((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) & 15) == 0;
-    constexpr int LARGEST = 1 << 22;                      // (the chain kernel counts the bytes of 64 rows in 31 bits)
     if (K % STEP != 0 || K <= 0 || K > LARGEST || !aligned) {
         dim3 grid(ceil_div(N, BN), ceil_div(M, BM)), block(NT);
         if (accumulate) hipLaunchKernelGGL(gemm_f32_kernel<true>, grid, block, 0, stream, X, W, Y, M, N, K);
         else hipLaunchKernelGGL(gemm_f32_kernel<false>, grid, block, 0, stream, X, W, Y, M, N, K);
         return launch_status();
     }
-    if (M <= 16) {
-        // Four rows a wave as long as one trip over W serves all rows, or the waves are few enough to run side by side, two a CU (16
-        // rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14), and K is not so short that
-        // the empty steps it begins with count (4 rows, 2,048 x 64: 3.2 us and 2.7, x 192 3.6 and 3.5, 32,768 x 192 6.4 and 7.2).
-        // Twelve steps in LDS where a CU has one wave (8,192 x 1,024, two a CU: 11.7 us, with six 10.3).
-        const long long waves = ceil_div_ll(N, 16) * ceil_div(M, 4);
-        if (K % LONG_STEP == 0 && K >= 192 && (M <= 4 || waves <= 512)) {
-            if (waves <= 256) return launch_quad<12>(X, W, Y, M, N, K, accumulate, stream);
-            return launch_quad<6>(X, W, Y, M, N, K, accumulate, stream);
-        }
-        if (N <= 4096) return launch_rows<16>(X, W, Y, M, N, K, accumulate, stream);
-        return launch_rows<8>(X, W, Y, M, N, K, accumulate, stream);
-    }
-    constexpr int MOST_BLOCKS = 65535;                    // of rows in a grid
-    if (ceil_div(M, 32) <= MOST_BLOCKS && block_cycles(M, N, 32) < block_cycles(M, N, 64))
-        return launch_chain<1, 4>(X, W, Y, M, N, K, accumulate, stream);
-    return launch_chain<2, 4>(X, W, Y, M, N, K, accumulate, stream);
+    return launch_whole_chain<false>(X, W, Y, M, N, K, accumulate, stream);
+}
+
+// Y [M, F] = silu(X Wg^T) * (X Wu^T), W [2 F, K]: the gate rows Wg, then the up rows Wu; the bits of tuff_gemm_f32 and the
+// kernel that applies SwiGLU.  -2 where the product is not one of whole chains.
+TUFF_EXPORT int tuff_gemm_f32_swiglu(const float* X, const float* W, float* Y, int M, int F, int K, hipStream_t stream) {
+    if (K % STEP != 0 || K <= 0 || K > LARGEST || (long long)2 * F * K > SWIGLU_LARGEST || (((uintptr_t)X | (uintptr_t)W | (uintptr_t)Y) & 15) != 0) return -2;
+    if (M <= 0 || F <= 0) return 0;
+    return launch_whole_chain<true>(X, W, Y, M, 2 * F, K, 0, stream);
 }

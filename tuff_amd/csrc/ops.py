@@ -81,6 +81,7 @@ _SIGNATURES = {
     },
     "gemm_f32": {
         "tuff_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+        "tuff_gemm_f32_swiglu": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
     },
     "gemm_bf16": {
         "tuff_gemm_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p],
@@ -609,6 +610,25 @@ def gemm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, accumulate: bool =
     ws = _gemm_workspace(M, N, K, x.device)
     _check(load("gemm_bf16").tuff_gemm_bf16(x.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, mode,
                                             None if ws is None else ws.data_ptr(), _stream()), "gemm_bf16")
+
+
+def gemm_f32_swiglu_supported(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether gemm_f32_swiglu takes these: float32 on 16-byte borders, an inner size that is a multiple of 32, w of at most
+    1 GiB."""
+    return (isinstance(w, torch.Tensor) and x.dtype == w.dtype == torch.float32 and x.dim() == 2 and x.is_contiguous() and w.is_contiguous()
+            and x.shape[1] == w.shape[1] and w.shape[0] % 2 == 0 and 0 < w.shape[1] <= 1 << 22 and w.shape[1] % 32 == 0 and w.numel() <= 1 << 28
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+
+
+def gemm_f32_swiglu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
+    """out [M, F] = silu(x Wg^T) * (x Wu^T) in float32, w [2 F, K] the gate rows Wg and then the up rows Wu: the bits of gemm and
+    swiglu."""
+    M, K = x.shape
+    F = w.shape[0] // 2
+    if not gemm_f32_swiglu_supported(x, w):
+        raise KernelError("gemm_f32_swiglu: these operands are not supported (ask gemm_f32_swiglu_supported first)")
+    _check(load("gemm_f32").tuff_gemm_f32_swiglu(_gpu("x", x, torch.float32), _gpu("w", w, torch.float32, (2 * F, K)),
+                                                 _gpu("out", out, torch.float32, (M, F)), M, F, K, _stream()), "gemm_f32_swiglu")
 
 
 _bias_ok: dict = {}

@@ -68,9 +68,13 @@ class SwiGLU(FeedForward):
         if self.gate_up.interleaved:
             act = self.gate_up.forward(h, swiglu=True)          # silu(gate) * up in the product's epilogue
         else:
-            gu = self.gate_up.forward(h)
-            act = self.rt.empty(h.shape[0], self.width, dtype=gu.dtype)
-            ops.swiglu(gu, act)
+            if not isinstance(h, torch.Tensor):
+                h = h.tensor()
+            act = self.gate_up.forward_gated(h)
+            if act is None:
+                gu = self.gate_up.forward(h)
+                act = self.rt.empty(h.shape[0], self.width, dtype=gu.dtype)
+                ops.swiglu(gu, act)
         self.down.forward(act, accumulate_into=residual, next_norm=next_norm)
 
 

@@ -129,6 +129,16 @@ class Linear:
         ops.gemm_bias(x, w, y, bias, activation=activation)
         return y
 
+    def forward_gated(self, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """silu(gate) * up [T, out / 2] of a float32 pair from the product's own kernel, or None where that needs the separate
+        kernels (nothing is launched then).  x [T, in]."""
+        if (not self.swiglu_pair or self.interleaved or self.bias is not None or self.rt.dtype != torch.float32
+                or not ops.gemm_f32_swiglu_supported(x, self.weight)):
+            return None
+        y = torch.empty(x.shape[0], self.out_features // 2, dtype=torch.float32, device=x.device)
+        ops.gemm_f32_swiglu(x, self.weight, y)
+        return y
+
     def forward(self, x, *, out_dtype: Optional[torch.dtype] = None,
                 accumulate_into: Optional[torch.Tensor] = None, swiglu: bool = False,
                 next_norm=None) -> Optional[torch.Tensor]:
