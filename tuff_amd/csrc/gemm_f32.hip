@@ -84,10 +84,11 @@ constexpr int STEP = 32;
 
 constexpr int WAVES = 2;
 
-//
 // SWIGLU, in all three kernels on whole chains: W holds N / 2 gate rows and then as many up rows, a block takes as many of each,
 // and of the two chains of a column, which lie in one lane or in two of one wave, swiglu_value leaves Y [M, N / 2].  As a
-// kernel of its own that wrote and read [M, N] once more: 4 rows, 16,384 x 2,048: product and SwiGLU
+// kernel of its own it wrote and read [M, N] once more.  Two kernels / one, us: 16,384 x 2,048 of 4 rows 31.2 and 29.6, 39 46.7 and
+// 43.9, 500 286.1 and 281.9; 13,824 x 1,536 20.0 and 18.1, 35.8 and 33.8, 193.8 and 186.2; 2,048 x 512 7.0 and 5.1, 8.3 and
+// 6.6, 17.8 and 13.9.
 __device__ __forceinline__ float swiglu_value(float gate, float up) { return gate / (1.0f + expf(-gate)) * up; }
 
 template <int T, int STAGES, bool SWIGLU>
@@ -552,11 +553,13 @@ int launch_whole_chain(const float* X, const float* W, float* Y, int M, int N, i
         // Four rows a wave as long as one trip over W serves all rows, or the waves are few enough to run side by side, two a CU (16
         // rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14), and K is not so short that
         // the empty steps it begins with count (4 rows, 2,048 x 64: 3.2 us and 2.7, x 192 3.6 and 3.5, 32,768 x 192 6.4 and 7.2).
-        // Twelve steps in LDS where a CU has one wave (8,192 x 1,024, two a CU: 11.7 us, with six 10.3).
+        // Twelve steps in LDS where a CU has one wave (8,192 x 1,024, two a CU: 11.7 us, with six 10.3), else five, of which six waves
+        // fit a CU: beyond, the loads under way are more than enough and the waves side by side count (4 rows, six steps / five / four:
+        // 16,384 x 2,048 28.9, 28.5 and 28.2 us, 21,504 x 2,048 41.8, 37.2 and 36.9, 65,536 x 2,048 100, 98 and 101).
         const long long waves = ceil_div_ll(N, 16) * ceil_div(M, 4);
         if (K % LONG_STEP == 0 && K >= 192 && (M <= 4 || waves <= 512)) {
             if (waves <= 256) return launch_quad<SWIGLU, 12>(X, W, Y, M, N, K, accumulate, stream);
-            return launch_quad<SWIGLU, 6>(X, W, Y, M, N, K, accumulate, stream);
+            return launch_quad<SWIGLU, 5>(X, W, Y, M, N, K, accumulate, stream);
         }
         if (N <= 4096) return launch_rows<SWIGLU, 16>(X, W, Y, M, N, K, accumulate, stream);
         return launch_rows<SWIGLU, 8>(X, W, Y, M, N, K, accumulate, stream);
