@@ -168,9 +168,10 @@ TUFF_EXPORT int tuff_attention_general(const void* q, const void* k_cache, const
 //   softmax  a wave four of the columns, lanes are keys: maximum, exponentials and the sum's butterfly as above;
 //   values   wave w the channels 16 w .. + 15 (and + 64): scaled by the column's correction, then a chain over the keys.
 // Keys and values go through LDS, the next tile's on their way to registers meanwhile.  What bounds it: a tile is two chains of
-// sixteen dependent matrix instructions and three exchanges, about 2.9 us, whatever the number of columns.  The general
-// kernel reads a key's row a lane and a value's column a lane, one wave a (token, head): 4 tokens of 32 heads at 1,000 keys
-// 272 us -> 46, a prompt of 500 tokens 613 us -> 76.
+// sixteen dependent matrix instructions, three exchanges and some 400 instructions of a lone wave, about 1.9 us, whatever the
+// number of columns; from the L2 instead of HBM it is 3 % faster.  The general kernel reads a key's row a lane and a value's
+// column a lane, one wave a (token, head): 4 tokens of 32 heads at 1,000 keys 272 us -> 32.7 (with a trip to LDS a value and addresses from
+// page numbers in every tile 37.8), a prompt of 500 tokens 613 us -> 50 (60).
 namespace {
 constexpr int F32_COLS = 16;
 
@@ -201,36 +202,40 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
     const int vpiece = (tid % 16) ^ (tid / 16);           // (the same for all of the thread's value pieces)
     f32x4 kr[KP], vr[KP];
     // Lane i knows where granule (sixteen keys) i of sixteen tiles lies, four a tile; keys nobody sees lie on a seen one's page.
-    // Worked out once in sixteen tiles, the page numbers asked for sixteen tiles ahead: from the table in every tile they were
-    // a trip to memory that the tile waited for.
+    // Worked out once in sixteen tiles, addresses and all, the page numbers asked for sixteen tiles ahead: from the table in every
+    // tile they were a trip to memory that the tile waited for, and addresses from page numbers 150 of a tile's instructions.
     const int first = lo_first / 64 * 64;
     auto key_of_granule = [&](int batch) { return (unsigned)max(lo_first, min(first + 1024 * batch + 16 * lane, pos_last)); };
     auto pages_of = [&](int batch) { return table[key_of_granule(batch) / (unsigned)page_size]; };
-    int pages = pages_of(0), pages_next = pages_of(1), offs = key_of_granule(0) / 16 * 16 % (unsigned)page_size;
+    unsigned long long keys_at, values_at;                // this lane's granule: its first key's row, its first position in channel 0
+    auto locate = [&](int batch, int page) {
+        const int off = key_of_granule(batch) / 16 * 16 % (unsigned)page_size;
+        const long long at = ((long long)page * Hkv + kvh) * page_size * HD;
+        keys_at = (unsigned long long)(k_cache + at + off * HD);
+        values_at = (unsigned long long)(v_cache + at + off);
+    };
+    int pages_next = pages_of(1);
+    locate(0, pages_of(0));
     auto load_tile = [&](int t0) {
         const int tile = (t0 - first) / 64;
         if (tile % 16 == 0 && tile > 0) {
-            pages = pages_next;
-            offs = key_of_granule(tile / 16) / 16 * 16 % (unsigned)page_size;
+            locate(tile / 16, pages_next);
             pages_next = pages_of(tile / 16 + 1);
         }
-        int page[4], off[4];                              // of the tile's groups of sixteen keys
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            page[j] = __builtin_amdgcn_readlane(pages, tile % 16 * 4 + j);
-            off[j] = __builtin_amdgcn_readlane(offs, tile % 16 * 4 + j);
-        }
+        const int granule = tile % 16 * 4;
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
             const int j = (k * 256 + tid) / P, pos = tid % P, piece = pos ^ swizzle(j), jg = __builtin_amdgcn_readfirstlane(j / 16);
-            kr[k] = *(const f32x4*)(k_cache + (((long long)page[jg] * Hkv + kvh) * page_size + off[jg] + j % 16) * HD + piece * 4);
+            const unsigned lo = __builtin_amdgcn_readlane((unsigned)keys_at, granule + jg);
+            const unsigned hi = __builtin_amdgcn_readlane((unsigned)(keys_at >> 32), granule + jg);
+            const char* row = (const char*)((unsigned long long)hi << 32 | lo);
+            kr[k] = *(const f32x4*)(row + (unsigned)((j % 16 * HD + piece * 4) * 4));
         }
-        const int vg = vpiece / 4;
-        const int vpage = vg < 2 ? (vg == 0 ? page[0] : page[1]) : (vg == 2 ? page[2] : page[3]);
-        const int voff = vg < 2 ? (vg == 0 ? off[0] : off[1]) : (vg == 2 ? off[2] : off[3]);
-        const float* vb = v_cache + ((long long)vpage * Hkv + kvh) * HD * page_size + voff + (vpiece % 4) * 4;
+        const int from = granule + vpiece / 4;
+        const unsigned lo = __shfl((unsigned)values_at, from), hi = __shfl((unsigned)(values_at >> 32), from);
+        const float* vb = (const float*)((unsigned long long)hi << 32 | lo) + (vpiece % 4) * 4 + tid / 16 * page_size;
 #pragma unroll
-        for (int k = 0; k < KP; ++k) vr[k] = *(const f32x4*)(vb + (long long)(k * 16 + tid / 16) * page_size);
+        for (int k = 0; k < KP; ++k) vr[k] = *(const f32x4*)(vb + (long long)(k * 16) * page_size);
     };
     auto put_tile = [&]() {
 #pragma unroll
@@ -261,13 +266,42 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
         put_tile();
         if (t0 + 64 <= pos_last) load_tile(t0 + 64);
         lds_barrier();
+        // The wave's values: no branch between the reads, and none that depends on one (sixteen trips to LDS one after the other were a
+        // third of a tile).  In heads of 64 they are read and looked over while one product of the scores waits for the other: 500
+        // tokens 56.8 -> 49.7 us; the others lose (128 channels, two tiles of values held: 55 -> 72, 32 and 16, waves without
+        // values: 4 x 1,000 keys 25.7 -> 27.2, 21.4 -> 24.2).
+        constexpr bool BESIDE = HD == 64;
+        float v[CT][16];
+        bool finite[CT];
+        const bool ragged = t0 < lo_first || t0 + 63 > pos_last;       // some keys were never written, or their pages are gone
+        auto read_values = [&](int c) {
+            const int ch = c * 64 + 16 * wave + r16;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[c][i] = vs[ch * 64 + (i ^ (ch % 16)) * 4 + g];
+        };
+        auto look_over = [&](int c) {
+            float zeros[2] = {0.f, 0.f};                  // NaN if one of the values is infinite or NaN
+            if (ragged) {
+                asm volatile("" :::);                     // (a branch, not sixteen selections in every tile)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int key = t0 + 4 * i + g;
+                    v[c][i] = (key < lo_first) | (key > pos_last) ? 0.f : v[c][i];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) zeros[i % 2] = fmaf(v[c][i], 0.f, zeros[i % 2]);
+            finite[c] = __all(zeros[0] + zeros[1] == 0.f);
+        };
         // scores of the keys 16 wave .. + 15
         {
+            if constexpr (BESIDE) read_values(0);
             const int j = 16 * wave + r16;
             f32x4 s = z;
 #pragma unroll
             for (int i = 0; i < P; ++i)
                 s = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[j * HD + (i ^ swizzle(j)) * 4 + g], qf[i], s, 0, 0, 0);
+            if constexpr (BESIDE) look_over(0);
             *(f32x4*)(sc + r16 * LD + 16 * wave + 4 * g) = s;
         }
         lds_barrier();
@@ -293,25 +327,19 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
         lds_barrier();
         // values: channels 64 c + 16 wave .. + 15
         const float corr = corr_lds[r16];
-        const bool ragged = t0 < lo_first || t0 + 63 > pos_last;       // some keys were never written, or their pages are gone
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
             if (c * 64 + 16 * wave < HD) {
-                const int ch = c * 64 + 16 * wave + r16;
-                float v[16], w[16];
-                bool finite = true;
+                if constexpr (!BESIDE) read_values(c);
+                float w[16];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    v[i] = vs[ch * 64 + (i ^ (ch % 16)) * 4 + g];
-                    w[i] = sc[r16 * LD + 4 * i + g];
-                    if (ragged && (t0 + 4 * i + g < lo_first || t0 + 4 * i + g > pos_last)) v[i] = 0.f;
-                    finite = finite && fabsf(v[i]) <= 3.402823466e38f;
-                }
+                for (int i = 0; i < 16; ++i) w[i] = sc[r16 * LD + 4 * i + g];
+                if constexpr (!BESIDE) look_over(c);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[c][e] *= corr;
-                if (__all(finite)) {
+                if (finite[c]) {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[i], w[i], acc[c], 0, 0, 0);
+                    for (int i = 0; i < 16; ++i) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[c][i], w[i], acc[c], 0, 0, 0);
                 } else {
                     // an infinity or NaN among the values counts only where its weight is not zero
                     for (int j = 0; j < 64; ++j) {
