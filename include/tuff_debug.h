@@ -33,7 +33,8 @@ int tuff_attention_partition_pages(int part, int page_size);
  * leaves its value.  Returns min_n as it was. */
 int tuff_gemm_bf16_wide64(int min_n, int max_n, int min_m);
 /* Forces the block shape of products of more than 64 rows whose K is a multiple of 64
- * (0: 256 x 256, 1: 128 x 128 two a CU, 2: 128 x 128 one a CU, 3: 64 x 64, 4: 256 x 192; -1: by size). */
+ * (0: 256 x 256, 1: 128 x 128 two a CU, 2: 128 x 128 one a CU, 3: 64 x 64, 4: 256 x 192,
+ * 5: 128 x 256, 6: 64 x 128; -1: by size). */
 int tuff_gemm_bf16_force_tiled_shape(int shape);
 
 #ifdef __cplusplus

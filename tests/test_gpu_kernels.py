@@ -346,6 +346,11 @@ def test_gemm_bf16_block_shapes_and_orders_give_the_same_bits(gpu, M, N, K, step
         assert torch.equal(y, new) and torch.equal(xw, (new * nw).bfloat16())
         exact = new.double().square().sum(1)
         assert ((ss.double().sum(0) - exact).abs() <= N * 2.0 ** -24 * exact).all()
+    if ops.gemm_bias_supported(M, N, K):
+        b, out, rounded = _r(N, seed=5).to(gpu), *(torch.empty(M, N, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+        ops.gemm_bias(x, tiled, out, b)
+        ops.cast(want, rounded, bias=b)
+        assert torch.equal(out, rounded)
     if N % 32 == 0:
         sums, out, plain = torch.full((20, M), K / 20.0, device=gpu), torch.empty(M, N // 2, dtype=torch.bfloat16, device=gpu), None
         ops.gemm_scaled(x, sums, 0.0, tiled, out, swiglu=True)                    # every row's scale is 1
