@@ -168,10 +168,10 @@ TUFF_EXPORT int tuff_attention_general(const void* q, const void* k_cache, const
 //   softmax  a wave four of the columns, lanes are keys: maximum, exponentials and the sum's butterfly as above;
 //   values   wave w the channels 16 w .. + 15 (and + 64): scaled by the column's correction, then a chain over the keys.
 // Keys and values go through LDS, the next tile's on their way to registers meanwhile.  What bounds it: a tile is two chains of
-// sixteen dependent matrix instructions, three exchanges and some 400 instructions of a lone wave, about 1.9 us, whatever the
+// sixteen dependent matrix instructions, three exchanges and some 400 instructions of a lone wave, about 1.8 us, whatever the
 // number of columns; from the L2 instead of HBM it is 3 % faster.  The general kernel reads a key's row a lane and a value's
-// column a lane, one wave a (token, head): 4 tokens of 32 heads at 1,000 keys 272 us -> 32.7 (with a trip to LDS a value and addresses from
-// page numbers in every tile 37.8), a prompt of 500 tokens 613 us -> 50 (60).
+// column a lane, one wave a (token, head): 4 tokens of 32 heads at 1,000 keys 272 us -> 30.0 (with a trip to LDS a value and addresses from
+// page numbers in every tile 37.8), a prompt of 500 tokens 613 us -> 47 (60).
 namespace {
 constexpr int F32_COLS = 16;
 
@@ -207,12 +207,14 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
     const int first = lo_first / 64 * 64;
     auto key_of_granule = [&](int batch) { return (unsigned)max(lo_first, min(first + 1024 * batch + 16 * lane, pos_last)); };
     auto pages_of = [&](int batch) { return table[key_of_granule(batch) / (unsigned)page_size]; };
-    unsigned long long keys_at, values_at;                // this lane's granule: its first key's row, its first position in channel 0
+    // this lane's granule, elements from the caches' beginnings (as addresses they would be loaded from through flat instructions, which
+    // the barriers' wait for LDS waits for too): its first key's row, its first position in channel 0
+    unsigned long long keys_at, values_at;
     auto locate = [&](int batch, int page) {
         const int off = key_of_granule(batch) / 16 * 16 % (unsigned)page_size;
         const long long at = ((long long)page * Hkv + kvh) * page_size * HD;
-        keys_at = (unsigned long long)(k_cache + at + off * HD);
-        values_at = (unsigned long long)(v_cache + at + off);
+        keys_at = (unsigned long long)(at + off * HD);
+        values_at = (unsigned long long)(at + off);
     };
     int pages_next = pages_of(1);
     locate(0, pages_of(0));
@@ -225,15 +227,16 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
         const int granule = tile % 16 * 4;
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
-            const int j = (k * 256 + tid) / P, pos = tid % P, piece = pos ^ swizzle(j), jg = __builtin_amdgcn_readfirstlane(j / 16);
+            const int j = (k * 256 + tid) / P, pos = tid % P, piece = pos ^ swizzle(j);
+            const int jg = P >= 16 ? k * 256 / (16 * P) : (unsigned)(k * 256 + wave * 64) / (16 * P);       // j / 16
             const unsigned lo = __builtin_amdgcn_readlane((unsigned)keys_at, granule + jg);
             const unsigned hi = __builtin_amdgcn_readlane((unsigned)(keys_at >> 32), granule + jg);
-            const char* row = (const char*)((unsigned long long)hi << 32 | lo);
-            kr[k] = *(const f32x4*)(row + (unsigned)((j % 16 * HD + piece * 4) * 4));
+            const float* row = k_cache + (long long)((unsigned long long)hi << 32 | lo);
+            kr[k] = *(const f32x4*)(row + (unsigned)(j % 16 * HD + piece * 4));
         }
         const int from = granule + vpiece / 4;
         const unsigned lo = __shfl((unsigned)values_at, from), hi = __shfl((unsigned)(values_at >> 32), from);
-        const float* vb = (const float*)((unsigned long long)hi << 32 | lo) + (vpiece % 4) * 4 + tid / 16 * page_size;
+        const float* vb = v_cache + (long long)((unsigned long long)hi << 32 | lo) + (vpiece % 4) * 4 + tid / 16 * page_size;
 #pragma unroll
         for (int k = 0; k < KP; ++k) vr[k] = *(const f32x4*)(vb + (long long)(k * 16) * page_size);
     };
@@ -260,6 +263,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
 #pragma unroll
     for (int c = 0; c < 4; ++c) { m[c] = -INFINITY; l[c] = 0.f; }
 
+    if (tid < F32_COLS) corr_lds[tid] = 1.f;
     load_tile(first);
     for (int t0 = first; t0 <= pos_last; t0 += 64) {
         lds_barrier();                                    // the last tile's keys, values and weights are used up
@@ -268,7 +272,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
         lds_barrier();
         // The wave's values: no branch between the reads, and none that depends on one (sixteen trips to LDS one after the other were a
         // third of a tile).  In heads of 64 they are read and looked over while one product of the scores waits for the other: 500
-        // tokens 56.8 -> 49.7 us; the others lose (128 channels, two tiles of values held: 55 -> 72, 32 and 16, waves without
+        // tokens 56.8 -> 49.7 us as measured then; the others lose (128 channels, two tiles of values held: 55 -> 72, 32 and 16, waves without
         // values: 4 x 1,000 keys 25.7 -> 27.2, 21.4 -> 24.2).
         constexpr bool BESIDE = HD == 64;
         float v[CT][16];
@@ -319,10 +323,7 @@ __global__ __launch_bounds__(256) void attention_f32_kernel(
                 m[c] = m_new;
                 sc[col * LD + lane] = p;
                 if (lane == 0) corr_lds[col] = corr;
-            } else {
-                sc[col * LD + lane] = 0.f;
-                if (lane == 0) corr_lds[col] = 1.f;
-            }
+            }                                             // (else no column: its sums are nobody's, whatever stands in its row)
         }
         lds_barrier();
         // values: channels 64 c + 16 wave .. + 15
