@@ -1044,6 +1044,46 @@ def test_attention_of_single_tokens_by_a_workgroup_a_kv_head(gpu, H, Hkv, hd, ps
     assert all(torch.isfinite(a).all() and torch.equal(a, b) for a, b in zip(*ways))
 
 
+@pytest.mark.parametrize("H,Hkv,hd,ps", [(4, 2, 16, 16), (4, 2, 40, 16), (8, 8, 56, 48), (6, 3, 72, 16), (4, 2, 112, 32), (2, 1, 136, 16)])
+def test_attention_of_heads_that_fill_no_tile_with_an_infinite_key(gpu, H, Hkv, hd, ps):
+    """A key of minus infinity in one of the head's first channels, whose score is minus infinity for every query: it has no
+    weight, as one whose score is far below all others, bit for bit, in every form of the kernel (a wave a partition, four, keys
+    through LDS or not, whole partitions a workgroup, one column block and two)."""
+    import ctypes
+    from tuff_amd.csrc import ops
+    lib = ops.load("attention_mfma")
+    reqs = [(299, 1), (30, 20), (517, 1)] + [(70 + i, 1) for i in range(29 if Hkv < 8 else 5)]
+    case = _mixed_step_case(gpu, reqs, H, Hkv, hd, ps)
+    q = case["q"].to(gpu)
+    q.view(-1, H, hd)[:, :, 3] = q.view(-1, H, hd)[:, :, 3].abs() + 0.25
+    table = torch.full((len(reqs), 4096 // ps + 1), -1, dtype=torch.int32, device=gpu)
+    table[:, :case["table"].shape[1]] = case["table"]
+    outs = {}
+    few, stage = lib.tuff_attention_few_waves(-1), lib.tuff_attention_stage_k_waves(-1)
+    try:
+        for value in (float("-inf"), -3e38):
+            kc = case["kc"].clone()
+            for r, (past, n) in enumerate(reqs):
+                for key in (0, 17, past - 2):
+                    kc[int(case["table"][r, key // ps]), :, key % ps, 3] = value
+            for nb in (1, 2):
+                blocks = torch.from_numpy(ops.query_blocks(case["q_len"], H // Hkv, nb)).to(gpu)
+                for form in [(0, 0), (0, 1 << 30), (1 << 30, 1 << 30)]:
+                    lib.tuff_attention_few_waves(form[0])
+                    lib.tuff_attention_stage_k_waves(form[1])
+                    for room in (1024, 4096):
+                        out = torch.full((q.shape[0], H * hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+                        ops.attention_mfma(q, kc, case["vc"], out, block_table=table, blocks=blocks, nb=nb, req_info=case["req_info"],
+                                           positions=case["positions"], H=H, Hkv=Hkv, hd=hd, page_size=ps, max_ctx_len=room)
+                        torch.cuda.synchronize()
+                        outs.setdefault((nb, form, room), []).append(out.float().cpu())
+    finally:
+        lib.tuff_attention_few_waves(few)
+        lib.tuff_attention_stage_k_waves(stage)
+    for key, (infinite, far) in outs.items():
+        assert torch.isfinite(far).all() and torch.equal(infinite, far), key
+
+
 @pytest.mark.parametrize("H,Hkv", [(32, 8), (6, 3), (5, 5), (16, 1)])
 def test_attention_of_single_tokens_does_not_depend_on_the_order_of_its_workgroups(gpu, H, Hkv):
     """Large launches number their workgroups with the kv head changing fastest, small ones with the

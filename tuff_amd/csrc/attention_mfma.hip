@@ -306,15 +306,16 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
         const bf16_t *k_at, *v_at;         // (not AHEAD) where this lane's parts of the keys and values begin
     };
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    const bool narrow = HD < HDP;          // channels beyond the head: its first key channel (the query has zero there), its first
-                                           // value channel (whose result nobody takes)
+    // Channels beyond the head are asked for as its first ones.  The keys' are zero before a product reads them, as the query's
+    // are (an infinite key times the query's zero is none); the values' give results that nobody takes.
+    const bool narrow = HD < HDP;
     using place_t = std::conditional_t<STREAM_V, unsigned, unsigned long long>;        // (pages of sixteen: 32 bits hold any place in one)
     const place_t page_elems = (place_t)Hkv * ps * HD;
     // this lane's place in a half's keys and values: key 8 ((n16 / 4) % 2) + n16 % 4 (+ 4 kb) of half n16 / 8; channel n16
     // (+ 16 db), positions 8 (g % 2) of half g / 2
     const bf16_t* const k_mine = k_cache + (long long)kvh * ps * HD + (8 * ((n16 / 4) % 2) + n16 % 4) * HD;
     const bf16_t* const v_mine = v_cache + (long long)kvh * ps * HD + (g % 2) * 8;
-    auto k_frag = [&](const bf16_t* at, int kb, int kc) {
+    auto k_frag = [&](const bf16_t* at, int kb, int kc, bool narrow) {
         const int k = kc * 32 + g * 8;
         return __builtin_nontemporal_load((const bf16x8*)(at + 4 * kb * HD + (!narrow || k < HD ? k : 0)));
     };
@@ -336,6 +337,12 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
         }
         return (unsigned)__builtin_amdgcn_readlane(my_page, holder & (WAVE - 1));
     };
+    if constexpr (STAGE) {
+        // the pieces beyond the head, which no step's keys go to
+        if (narrow)
+            for (int i = lane; i < 32 * 8; i += WAVE)
+                if (i % 8 >= row_pieces) *(bf16x8*)(k_stage[wave] + stage_at(i / 8, i % 8)) = zero8;
+    }
     auto load_tile = [&](int key0, Tile& t) {
         // a half without a key that some column may see: the other half's keys in its place (their weights are zero), and
         // where both are, the first page's (the cache's own first one where that is no longer held)
@@ -365,7 +372,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
 #pragma unroll
                 for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-                    for (int kc = 0; kc < KC; ++kc) t.kf[kb][kc] = k_frag(k_at, kb, kc);
+                    for (int kc = 0; kc < KC; ++kc) t.kf[kb][kc] = k_frag(k_at, kb, kc, narrow);
             }
 #pragma unroll
             for (int db = 0; db < DB; ++db) t.vx[db] = v_frag(v_at, db);
@@ -489,21 +496,36 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
                 }
             __builtin_amdgcn_wave_barrier();       // the wave's LDS accesses run in the order of the program
         }
+        auto scores = [&](auto NARROW) {
 #pragma unroll
-        for (int kb = 0; kb < 2; ++kb) {
+            for (int kb = 0; kb < 2; ++kb) {
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) s[kb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int nb = 0; nb < NB; ++nb) s[kb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int kc = 0; kc < KC; ++kc) {
-                bf16x8 kf;
-                const int chunk = kc * 4 + g;
-                if constexpr (STAGE) kf = *(const bf16x8*)(stage + stage_at(8 * (n16 / 4) + 4 * kb + n16 % 4, narrow && chunk >= row_pieces ? 0 : chunk));
-                else if constexpr (AHEAD) kf = t.kf[kb][kc];
-                else kf = k_frag(t.k_at, kb, kc);
+                for (int kc = 0; kc < KC; ++kc) {
+                    bf16x8 kf;
+                    const int chunk = kc * 4 + g;
+                    if constexpr (STAGE) kf = *(const bf16x8*)(stage + stage_at(8 * (n16 / 4) + 4 * kb + n16 % 4, chunk));
+                    else if constexpr (AHEAD) kf = t.kf[kb][kc];
+                    else kf = k_frag(t.k_at, kb, kc, decltype(NARROW)::value);
+                    if (decltype(NARROW)::value && chunk * 8 >= HD) kf = zero8;
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) s[kb][nb] = mfma32(kf, qf[nb][kc], s[kb][nb]);
+                    for (int nb = 0; nb < NB; ++nb) s[kb][nb] = mfma32(kf, qf[nb][kc], s[kb][nb]);
+                }
             }
-        }
+        };
+        // (staged, the pieces beyond the head lie in LDS as zeros)
+        if constexpr (AHEAD) {
+            if (!STAGE && narrow) {
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int kc = 0; kc < KC; ++kc)
+                        if ((kc * 4 + g) * 8 >= HD) t.kf[kb][kc] = zero8;
+            }
+            scores(std::false_type());
+        } else if (narrow) scores(std::true_type());
+        else scores(std::false_type());
         // ---- mask, running maximum, exp; P^T stays in registers as the next B operand
         const bool whole_step = key0 >= all_lo && key0 + 31 <= all_hi;
         bf16x8 pf[NB];
