@@ -466,6 +466,35 @@ def test_forget_scan_in_chunks_against_the_loop(gpu, H, D, Dv, gates):
     assert all(torch.isnan(state[2 * r]).all() for r in range(R + 1))
 
 
+@pytest.mark.parametrize("H, D, Dv", [(8, 64, 128), (8, 48, 256), (8, 32, 80), (16, 16, 16)])
+@pytest.mark.parametrize("spread, lowest, mean", [(1.0, 0.9, 0.0), (4.0, 0.9, 0.0), (0.3, 0.99, 0.0), (300.0, 0.9, 0.0), (1.0, 0.0, -3.0)])
+def test_forget_scan_in_chunks_is_no_further_from_64_bits(gpu, H, D, Dv, spread, lowest, mean):
+    """Outputs and states of a request of 512 tokens and one of 300, token by token and in chunks, against the loop in float64:
+    the norm of the difference is no larger in chunks, for gates of short and long memories and at their bounds."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(D)
+    lens = [512, 300]
+    T = sum(lens)
+    x = torch.randn(T, 2 * H * D + H * Dv, generator=gen)
+    x[:, H * D:2 * H * D] = x[:, H * D:2 * H * D] * spread + mean
+    x, fb, lower = x.to(gpu), torch.randn(H * D, generator=gen).to(gpu), (lowest * torch.rand(H * D, generator=gen)).to(gpu)
+    q = torch.nn.functional.silu(x[:, :H * D].double()).view(T, H, D)
+    f = (lower.double() + (1 - lower.double()) * torch.sigmoid(x[:, H * D:2 * H * D].double() + fb.double())).view(T, H, D)
+    v = x[:, 2 * H * D:].double().view(T, H, Dv)
+    want, S = torch.empty(T, H, Dv, dtype=torch.float64, device=gpu), torch.zeros(2, H, D, Dv, dtype=torch.float64, device=gpu)
+    for t in range(T):
+        r = int(t >= lens[0])
+        S[r] = f[t][:, :, None] * S[r] + (1 - f[t])[:, :, None] * v[t][:, None, :]
+        want[t] = (S[r] * q[t][:, :, None]).sum(1)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)
+    off = []
+    for fn in (ops.forget_scan, ops.forget_chunked):
+        out, state = torch.empty(T, H * Dv, device=gpu), torch.zeros(2, H, D, Dv, device=gpu)
+        fn(x, fb, lower, state, out, q_start=i32([0, lens[0]]), q_len=i32(lens), state_slot=i32([0, 1]), H=H, D=D, Dv=Dv)
+        off.append((float((out.view_as(want) - want).norm()), float((state - S).norm())))
+    assert off[1][0] <= off[0][0] and off[1][1] <= off[0][1], off
+
+
 @pytest.mark.parametrize("H, Hkv, vd", [(4, 2, 64), (32, 8, 64), (12, 3, 5), (16, 2, 130), (8, 1, 70), (6, 2, 33), (5, 5, 16), (1, 1, 1)])
 def test_mix_of_heads_against_the_sum_in_float64(gpu, H, Hkv, vd):
     """Two, four and eight heads a kv head (with and without heads left over after eight at a time) and the others: to the

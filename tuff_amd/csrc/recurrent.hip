@@ -284,6 +284,8 @@ __global__ void ssd_prep_kernel(const float* __restrict__ dt_raw, long long ld_d
 constexpr int CHUNK = 64;
 
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ f64x4 mfma_f64(double a, double b, f64x4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 
 struct SsdChunkArgs {
     const bf16_t* xbc;              // a token's rows [x (H*P) | B (G*N) | C (G*N)], ld apart
@@ -510,13 +512,17 @@ __global__ __launch_bounds__(256) void ssd_chunk_out_kernel(SsdChunkArgs p) {
 // F that of all of them and S the state at its start,
 //     o_t = sum_{s <= t} (sum_i q_t k_s prod_{u in s+1..t} f_u) v_s  +  (q_t Q_t)^T S        S <- F S + sum_s (k_s R_s) v_s^T
 // Three kernels as above: (1) every chunk's own contribution U and the product of its gates, (2) the chunks in order, the
-// state at a chunk's start takes U's place, (3) every chunk's outputs.  All float32, products by float32 matrix instructions
-// (16 x 16 x 4).  A wave keeps the state's columns of 16 value channels as accumulators: element e of tile i of a lane of
+// state at a chunk's start takes U's place, (3) every chunk's outputs.  Products by float32 matrix instructions (16 x 16 x 4).
+// Token by token a rounding decays with the state it is in; so that the chunks' sums are no further from the exact ones, a
+// block's are formed from its first token to its last, the gates' products and the sums over channels inside a block in 64
+// bits, and the latter meet the values in 64-bit matrix instructions.  A wave keeps the state's columns of 16 value channels as accumulators: element e of tile i of a lane of
 // group q is row 16 i + 4 q + e, and since an inner index may be taken in any order, the accumulators are, as they lie, the
-// second operand of (q_t Q_t)^T S.  What bounds it: float32 matrix instructions (36 a block and wave of the last kernel, 32
-// cycles each) and the way of the rows; token by token it is a chain of 2,048 steps on 512 waves.  One request of 2,048
-// tokens, 16 heads of 64 x 128, with what prepares the rows: 177 -> 59 us (state 19, pass 8, outputs 29).  Outputs are within
-// 8e-8 of 64 bits (token by token 6e-8, the state 9e-8 either way).  The sums of a token are formed in another
+// second operand of (q_t Q_t)^T S.  What bounds it: matrix instructions (32 of float32 and 4 of 64 bits, three times as long, a
+// block and wave of the last kernel) and the way of the rows; token by token it is a chain of 2,048 steps on 512 waves.  One
+// request of 2,048 tokens, 16 heads of 64 x 128, with what prepares the rows: 177 -> 65 us (59 with all sums in float32).
+// Error against 64 bits (norm of the difference over the norm), token by token and in chunks: outputs 6.5e-8 and 5.3e-8, state
+// 1.05e-7 and 1.04e-7; with gates near their lower bounds 7.3e-8 and 6.3e-8, 1.39e-7 and 1.38e-7; with short memories
+// 4.9e-8 and 3.5e-8, 4.2e-8 and 3.4e-8 (all in float32 8.1e-8 and 1.10e-7, 8.7e-8 and 1.42e-7, 6.6e-8 and 3.4e-8).  The sums of a token are formed in another
 // order than token by token, so a position's result depends on where its portion began, within float32 rounding.
 constexpr int BLOCK = 16;
 
@@ -574,38 +580,31 @@ __device__ __forceinline__ void gates_of_block(const ForgetChunkArgs& p, int c, 
     for (int u = 0; u < BLOCK; ++u) f[u] = b * BLOCK + u < L ? lo + (1.0f - lo) * sigmoidf_(f[u] + bias) : 1.f;
 }
 
-// P[u] = f[0] .. f[u] in four roundings at most (one after the other they are fifteen); REVERSED: f[15] .. f[u]
-template <bool REVERSED>
-__device__ __forceinline__ void products_of_block(const float (&f)[BLOCK], float (&P)[BLOCK]) {
-#pragma unroll
-    for (int u = 0; u < BLOCK; ++u) P[u] = f[u];
-#pragma unroll
-    for (int d = 1; d < BLOCK; d *= 2)
-#pragma unroll
-        for (int u = 0; u < BLOCK; ++u)
-            if (u & d) {
-                if constexpr (REVERSED) P[BLOCK - 1 - u] *= P[BLOCK - 1 - ((u & ~(2 * d - 1)) + d - 1)];
-                else P[u] *= P[(u & ~(2 * d - 1)) + d - 1];
-            }
-}
+// Where token u of a block lies in the rows of LDS that the products read, and which row of A^T they read for an output: a lane
+// of group q reads the four at 4 q, tokens 4 e + q for instruction e, so that the chain of a sum goes over the tokens in their
+// order; and the 64-bit instruction leaves row 4 e + q of its operand in element e, where the others leave 4 q + e.
+__device__ __forceinline__ constexpr int place_of(int u) { return 4 * (u % 4) + u / 4; }
 
-// k_s R_s of a block's tokens, and F; sk: the channel's row in LDS
+// k_s R_s of a block's tokens, each rounded once, and F; sk: the channel's row in LDS
 __device__ __forceinline__ float decayed_keys(const float (&f)[BLOCK], float* sk) {
-    float R[BLOCK], k[BLOCK];
-    products_of_block<true>(f, R);
+    double R = 1.0;
+    float k[BLOCK];
 #pragma unroll
-    for (int u = 0; u < BLOCK; ++u) k[u] = u + 1 < BLOCK ? (1.0f - f[u]) * R[u + 1] : 1.0f - f[u];
+    for (int u = BLOCK - 1; u >= 0; --u) {
+        k[u] = (float)((1.0 - (double)f[u]) * R);
+        R *= (double)f[u];
+    }
 #pragma unroll
-    for (int u = 0; u < BLOCK; u += 4) *(f32x4*)(sk + u) = f32x4{k[u], k[u + 1], k[u + 2], k[u + 3]};
-    return R[0];
+    for (int u = 0; u < 4; ++u) *(f32x4*)(sk + 4 * u) = f32x4{k[u], k[4 + u], k[8 + u], k[12 + u]};
+    return (float)R;
 }
 
-// a lane's values of a block: tokens 4 q .. 4 q + 3, its channel (zero beyond token L)
+// a lane's values of a block: tokens 4 e + q, its channel (zero beyond token L)
 __device__ __forceinline__ f32x4 values_of_block(const float* rows, unsigned ld, unsigned at, int b, int q, int L) {
     f32x4 r;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        const int t = b * BLOCK + 4 * q + e;
+        const int t = b * BLOCK + 4 * e + q;
         const float x = rows[at + (unsigned)min(t, L - 1) * ld];
         r[e] = t < L ? x : 0.f;
     }
@@ -645,7 +644,7 @@ __global__ __launch_bounds__(512, 4) void forget_chunk_state_kernel(ForgetChunkA
     }
     __syncthreads();
     const long long at = (long long)blockIdx.x * p.H + head;
-    if (tid < D) p.cdec[at * D + tid] = sF[0][tid] * sF[1][tid] * sF[2][tid] * sF[3][tid];
+    if (tid < D) p.cdec[at * D + tid] = (float)(((double)sF[0][tid] * sF[1][tid]) * ((double)sF[2][tid] * sF[3][tid]));
     float* U = p.U + at * D * Dv;
     for (int j = wave * 16 + l16; j < Dv; j += waves * 16) {
         const unsigned v = 2 * p.H * D + head * Dv + j;
@@ -710,7 +709,7 @@ __global__ __launch_bounds__(512, 4) void forget_chunk_out_kernel(ForgetChunkArg
     float* const sq = sqd + CHUNK * LDQ;               // [CHUNK][LDQ]: q
     float* const sf = sq + CHUNK * LDQ;                // [CHUNK][LDQ]: the gates
     float* const sF = sf + CHUNK * LDQ;                // [BLOCKS][D]
-    float* const sA = sF + BLOCKS * D;                 // [2][BLOCKS][BLOCK (t)][LDA (s)]: inside a block, by half of the channels
+    float* const sA = sF + BLOCKS * D;                 // [2][BLOCKS][BLOCK (t)][LDA (place of s)]: inside a block, by half of the channels
     const int Dv = p.Dv, head = blockIdx.y, tid = threadIdx.x, lane = tid % WAVE, l16 = lane % 16, q = lane / 16;
     const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE), waves = blockDim.x / WAVE;
     int t0, L;
@@ -724,24 +723,24 @@ __global__ __launch_bounds__(512, 4) void forget_chunk_out_kernel(ForgetChunkArg
         column_of_block(row, ld, head * D + c, b, L, qr);
         gates_of_block(p, head * D + c, b, L, f);
         sF[b * D + c] = decayed_keys(f, sk + c * FORGET_LDK + b * BLOCK);
-        float Q[BLOCK];
-        products_of_block<false>(f, Q);
+        double Q = 1.0;
 #pragma unroll
         for (int u = 0; u < BLOCK; ++u) {
             const float qq = siluf_(qr[u]);
+            Q *= (double)f[u];
             sq[(b * BLOCK + u) * LDQ + c] = qq;
             sf[(b * BLOCK + u) * LDQ + c] = f[u];
-            sqd[(b * BLOCK + u) * LDQ + c] = qq * Q[u];
+            sqd[(b * BLOCK + u) * LDQ + c] = (float)(qq * Q);
         }
     }
     __syncthreads();
-    // A[t][s] of a block over half of the channels: a lane takes token s = l16 and a quarter of the half, and carries
-    // k_s prod f from token to token
+    // A[t][s] of a block over half of the channels, in 64 bits up to the half's sum: a lane takes token s = l16 and a quarter
+    // of the half, and carries k_s prod f from token to token
     constexpr int PER = D / 8;                         // channels a lane
     for (int job = wave; job < 2 * BLOCKS; job += waves) {
         const int b = job % BLOCKS, half = job / BLOCKS, c0 = half * (D / 2) + q * PER;
-        float X[PER] = {};
-        float* to = sA + ((half * BLOCKS + b) * BLOCK + q) * LDA + l16;
+        double X[PER] = {};
+        float* to = sA + ((half * BLOCKS + b) * BLOCK + q) * LDA + place_of(l16);
 #pragma unroll 1
         for (int t4 = 0; t4 < BLOCK; t4 += 4) {
             const float* ft = sf + (b * BLOCK + t4) * LDQ + c0;
@@ -749,13 +748,15 @@ __global__ __launch_bounds__(512, 4) void forget_chunk_out_kernel(ForgetChunkArg
             float A[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                float part[2] = {0.f, 0.f};
+                double part = 0.0;
 #pragma unroll
                 for (int i = 0; i < PER; ++i) {
-                    X[i] = t4 + t == l16 ? 1.0f - ft[t * LDQ + i] : X[i] * ft[t * LDQ + i];
-                    part[i % 2] = fmaf(qt[t * LDQ + i], X[i], part[i % 2]);
+                    const double f = ft[t * LDQ + i];
+                    X[i] = t4 + t == l16 ? 1.0 - f : X[i] * f;
+                    part = fma((double)qt[t * LDQ + i], X[i], part);
                 }
-                A[t] = butterfly_sum<32>(butterfly_sum<16>(part[0] + part[1]));
+                part += __shfl_xor(part, 16, WAVE);
+                A[t] = (float)(part + __shfl_xor(part, 32, WAVE));
             }
             to[t4 * LDA] = q == 0 ? A[0] : q == 1 ? A[1] : q == 2 ? A[2] : A[3];
         }
@@ -773,13 +774,13 @@ __global__ __launch_bounds__(512, 4) void forget_chunk_out_kernel(ForgetChunkArg
         for (int b = 0; b < BLOCKS && b * BLOCK < L; ++b) {
             const f32x4 vb = next;
             next = values_of_block(row, ld, v, min(b + 1, BLOCKS - 1), q, L);
-            // sums of four products each, added as a tree: as near to the exact sum as token by token
-            const float* a = sA + (b * BLOCK + l16) * LDA + 4 * q;
+            const float* a = sA + (b * BLOCK + place_of(l16)) * LDA + 4 * q;
             const f32x4 a0 = *(const f32x4*)a, a1 = *(const f32x4*)(a + BLOCKS * BLOCK * LDA), zero = {0.f, 0.f, 0.f, 0.f};
-            f32x4 part[4], o;
+            f64x4 inside = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-            for (int e = 0; e < 4; ++e) part[e] = mfma_f32(a0[e] + a1[e], vb[e], zero);
-            o = (part[0] + part[1]) + (part[2] + part[3]);
+            for (int e = 0; e < 4; ++e) inside = mfma_f64((double)a0[e] + (double)a1[e], (double)vb[e], inside);
+            // from the state: sums of four products each, added as a tree
+            f32x4 part[4], o;
             f32x4 sum[NI];
 #pragma unroll
             for (int i = 0; i < NI; ++i) {
@@ -788,15 +789,16 @@ __global__ __launch_bounds__(512, 4) void forget_chunk_out_kernel(ForgetChunkArg
                 for (int e = 0; e < 4; ++e) part[e] = mfma_f32(qd[e], S[i][e], zero);
                 sum[i] = (part[0] + part[1]) + (part[2] + part[3]);
             }
-            if constexpr (NI == 4) o += (sum[0] + sum[1]) + (sum[2] + sum[3]);
+            if constexpr (NI == 4) o = (sum[0] + sum[1]) + (sum[2] + sum[3]);
             else {
+                o = sum[0];
 #pragma unroll
-                for (int i = 0; i < NI; ++i) o += sum[i];
+                for (int i = 1; i < NI; ++i) o += sum[i];
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int t = b * BLOCK + 4 * q + e;
-                if (t < L) p.out[((long long)(t0 + t) * p.H + head) * Dv + j] = o[e];
+                if (t < L) p.out[((long long)(t0 + t) * p.H + head) * Dv + j] = (float)(inside[e] + (double)o[e]);
             }
             state_over_block(S, sk, sF + b * D, b, vb, l16, q);
         }
