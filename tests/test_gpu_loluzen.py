@@ -495,6 +495,38 @@ def test_forget_scan_in_chunks_is_no_further_from_64_bits(gpu, H, D, Dv, spread,
     assert off[1][0] <= off[0][0] and off[1][1] <= off[0][1], off
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("H, D, Dv", [(2, 64, 128), (3, 32, 48)])
+def test_forget_scan_in_chunks_with_a_value_that_is_not_finite(gpu, H, D, Dv, bad):
+    """One value of one head and channel in the middle of a block: every output before its token is what it is without it, and
+    so is every other channel's; from its token on the channel has none that is finite, as token by token.  The step's
+    other request sees nothing of it."""
+    from tuff_amd.csrc import ops
+    gen = torch.Generator().manual_seed(D)
+    lens, at, head, ch = [100, 20], 73, 1, 5
+    T = sum(lens)
+    x = torch.randn(T, 2 * H * D + H * Dv, generator=gen).to(gpu)
+    fb, lower = torch.randn(H * D, generator=gen).to(gpu), (0.9 * torch.rand(H * D, generator=gen)).to(gpu)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)
+    spoilt = x.clone()
+    spoilt[at, 2 * H * D + head * Dv + ch] = bad
+    got = []
+    for fn, rows in ((ops.forget_chunked, x), (ops.forget_chunked, spoilt), (ops.forget_scan, spoilt)):
+        out, state = torch.empty(T, H * Dv, device=gpu), torch.zeros(2, H, D, Dv, device=gpu)
+        fn(rows, fb, lower, state, out, q_start=i32([0, lens[0]]), q_len=i32(lens), state_slot=i32([0, 1]), H=H, D=D, Dv=Dv)
+        got.append((out.view(T, H, Dv), state))
+    (clean, clean_state), (out, state), (token_by_token, _) = got
+    touched = torch.zeros(T, H, Dv, dtype=torch.bool, device=gpu)
+    touched[at:lens[0], head, ch] = True
+    assert not torch.isfinite(out[touched]).any() and not torch.isfinite(token_by_token[touched]).any()
+    # (the block with the value adds in 64 bits in another order: the last bit of a few of its outputs)
+    assert ((out - clean)[~touched].abs() <= 2.0 ** -23 * clean[~touched].abs()).all() and torch.isfinite(token_by_token[~touched]).all()
+    assert torch.equal(out[:64], clean[:64]) and torch.equal(out[lens[0]:], clean[lens[0]:]) and torch.equal(state[1], clean_state[1])
+    assert not torch.isfinite(state[0, head, :, ch]).any()
+    state[0, head, :, ch] = clean_state[0, head, :, ch]
+    assert torch.equal(state[0], clean_state[0])
+
+
 @pytest.mark.parametrize("H, Hkv, vd", [(4, 2, 64), (32, 8, 64), (12, 3, 5), (16, 2, 130), (8, 1, 70), (6, 2, 33), (5, 5, 16), (1, 1, 1)])
 def test_mix_of_heads_against_the_sum_in_float64(gpu, H, Hkv, vd):
     """Two, four and eight heads a kv head (with and without heads left over after eight at a time) and the others: to the

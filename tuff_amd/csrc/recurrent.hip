@@ -777,8 +777,24 @@ __global__ __launch_bounds__(512, 4) void forget_chunk_out_kernel(ForgetChunkArg
             const float* a = sA + (b * BLOCK + place_of(l16)) * LDA + 4 * q;
             const f32x4 a0 = *(const f32x4*)a, a1 = *(const f32x4*)(a + BLOCKS * BLOCK * LDA), zero = {0.f, 0.f, 0.f, 0.f};
             f64x4 inside = {0.0, 0.0, 0.0, 0.0};
+            float zeros = 0.f;                             // NaN if one of the values is infinite or NaN
 #pragma unroll
-            for (int e = 0; e < 4; ++e) inside = mfma_f64((double)a0[e] + (double)a1[e], (double)vb[e], inside);
+            for (int e = 0; e < 4; ++e) zeros = fmaf(vb[e], 0.f, zeros);
+            if (__all(zeros == 0.f)) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) inside = mfma_f64((double)a0[e] + (double)a1[e], (double)vb[e], inside);
+            } else {
+                // such a value counts for its own token and those after it only
+#pragma unroll 1
+                for (int s = 0; s < BLOCK; ++s) {
+                    const float mine = s < 8 ? (s < 4 ? vb[0] : vb[1]) : s < 12 ? vb[2] : vb[3];
+                    const double v = __shfl(mine, s % 4 * 16 + l16, WAVE);
+                    const float* at = sA + (b * BLOCK + 4 * q) * LDA + place_of(s);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (s <= 4 * q + e) inside[e] = fma((double)at[e * LDA] + (double)at[(BLOCKS * BLOCK + e) * LDA], v, inside[e]);
+                }
+            }
             // from the state: sums of four products each, added as a tree
             f32x4 part[4], o;
             f32x4 sum[NI];
