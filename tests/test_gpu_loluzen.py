@@ -527,6 +527,113 @@ def test_forget_scan_in_chunks_with_a_value_that_is_not_finite(gpu, H, D, Dv, ba
     assert torch.equal(state[0], clean_state[0])
 
 
+@pytest.mark.parametrize("n", [287, 288, 400, 700])
+def test_forget_gate_of_a_request_has_the_same_bits_alone_and_in_company(gpu, n):
+    """The mixer's step for one request alone, and among others with single tokens, short portions and long ones: outputs and
+    state of every request are what the request has alone, whichever form its number of tokens takes."""
+    import types
+    from tuff_amd.engine.batch import StepEntry, build_context
+    from tuff_amd.parts.base import Runtime
+    from tuff_amd.parts.recurrent import ForgetGateMixer
+    H, D, Dv = 4, 64, 32
+    eng = engine("wide", "bfloat16", max_tokens=4096, max_requests=8)
+    gen = torch.Generator().manual_seed(n)
+    m = ForgetGateMixer(96, H, D, Dv, 1e-5, names={k: k for k in ("q", "f", "f.b", "lower", "v", "norm", "o")})
+    m.rt = Runtime(gpu, torch.bfloat16)
+    m.f_bias, m.lower = torch.randn(H * D, generator=gen).to(gpu), (0.9 * torch.rand(H * D, generator=gen)).to(gpu)
+    m.norm_w = torch.ones(Dv, device=gpu)
+    lens = {"a": 1, "b": n, "c": 30, "d": 1, "e": 290, "f": 287, "g": 1}
+    rows = {k: torch.randn(v, H * (2 * D + Dv), generator=gen).to(gpu) for k, v in lens.items()}
+    S0 = torch.randn(8, H, D, Dv, generator=gen).to(gpu)
+
+    def step(ids):
+        for k in ids:
+            eng.begin(k)
+            eng.manager.extend(k, lens[k])
+        ctx = build_context([StepEntry(k, [0] * lens[k], []) for k in ids], eng.manager, gpu, 333)
+        slots = [eng.manager.slot(k) for k in ids]
+        state = torch.full_like(S0, float("nan"))
+        for k, slot in zip(ids, slots):
+            state[slot] = S0[list(lens).index(k)]
+        kept = []
+        m.qfv = types.SimpleNamespace(forward=lambda h, out_dtype: torch.cat([rows[k] for k in ids]))
+        m.out = types.SimpleNamespace(forward=lambda y, **kw: kept.append(y))
+        m.forward(torch.empty(ctx.T, 96, dtype=torch.bfloat16, device=gpu), ctx, types.SimpleNamespace(state=state), None)
+        for k in ids:
+            eng.end(k)
+        return {k: (y.float(), state[slot]) for k, y, slot in zip(ids, kept[0].split([lens[k] for k in ids]), slots)}
+
+    together = step(list(lens))
+    for k in lens:
+        alone = step([k])[k]
+        assert torch.isfinite(alone[0]).all() and torch.isfinite(alone[1]).all()
+        assert torch.equal(alone[0], together[k][0]) and torch.equal(alone[1], together[k][1]), k
+
+
+def _counted(monkeypatch):
+    """How often each form of the forget gate's recurrence was launched."""
+    from tuff_amd.csrc import ops
+    calls = {"forget_scan": 0, "forget_chunked": 0}
+    for name in calls:
+        def wrapped(*a, _name=name, _fn=getattr(ops, name), **kw):
+            calls[_name] += 1
+            return _fn(*a, **kw)
+        monkeypatch.setattr(ops, name, wrapped)
+    return calls
+
+
+@pytest.mark.parametrize("how", ["whole", "then single tokens", "in portions", "beside others"])
+def test_prompts_long_enough_for_the_recurrence_in_chunks(gpu, monkeypatch, how):
+    """Prompts of 288 tokens and more through the engine, whole, decoded on token by token, in portions on both sides of that
+    length, and beside single tokens and short requests: the logits of the plain model every time."""
+    calls = _counted(monkeypatch)
+    reqs = requests("wide", [450, 300] if how == "beside others" else [700, 289], seed=11)
+    if how == "whole":
+        plan = util.plan_whole(reqs)
+    elif how == "then single tokens":
+        plan = util.plan_tail(reqs, tail=33)
+    elif how == "in portions":
+        plan = util.plan_chunks(reqs, sizes=(300, 7, 1, 290, 64, 2))
+    else:
+        reqs.update({"x": util.rand_tokens(24, 333, 7), "y": util.rand_tokens(60, 333, 8)})
+        at = {k: 0 for k in reqs}
+        plan = []
+        for sizes in ({"x": 20}, {"x": 1, "r0": 400, "y": 40}, {"x": 1, "r1": 290, "y": 10, "r0": 20}, {"x": 1, "y": 8, "r1": 10, "r0": 28},
+                      {"x": 1, "y": 2, "r0": 2}):
+            entries = []
+            for k, n in sizes.items():
+                entries.append({"id": k, "tokens": reqs[k][at[k]:at[k] + n], "want": list(range(n))})
+                at[k] += n
+            plan.append({"step": len(plan), "entries": entries, "end": [k for k in sizes if at[k] == len(reqs[k])]})
+    check("wide", "bfloat16", plan, reqs, max_tokens=2048)
+    assert calls["forget_chunked"] > 0 and (how == "whole" or calls["forget_scan"] > 0)
+
+
+def test_recorded_steps_of_long_portions_short_ones_and_both(gpu):
+    """Steps of one number of tokens, as one long portion, as four short ones and as a long one beside short ones, in turn and often
+    enough to be recorded and replayed: every logit is the eager step's, and there is a recording of each kind."""
+    reqs = {k: util.rand_tokens(3000, 333, 20 + i) for i, k in enumerate("abcd")}
+    at, steps = {k: 0 for k in reqs}, []
+    for _ in range(6):
+        for sizes in ({"a": 448}, {k: 112 for k in "abcd"}, {"b": 400, "c": 24, "d": 24}):
+            entries = []
+            for k, n in sizes.items():
+                at[k] = at[k] if at[k] + n <= 3000 else 0
+                entries.append({"id": k, "tokens": reqs[k][at[k]:at[k] + n], "want": [0, n - 1]})
+                at[k] += n
+            steps.append({"step": len(steps), "entries": entries, "end": []})
+        steps.append({"step": len(steps), "entries": [{"id": k, "tokens": reqs[k][:1], "want": [0]} for k in "abcd"], "end": []})
+    steps[-1]["end"] = list("abcd")
+    kw = dict(max_tokens=16384, max_requests=6)
+    want = util.run_plan(engine("wide", "bfloat16", use_graphs=False, **kw), steps)
+    eng = engine("wide", "bfloat16", **kw)
+    got = util.run_plan(eng, steps)
+    assert eng.section_recordings == 3 and eng.section_replays == 3 * 4
+    for k in reqs:
+        wanted = ~torch.isnan(want[k][:, 0])
+        assert wanted.any() and torch.equal(got[k][wanted], want[k][wanted]), k
+
+
 @pytest.mark.parametrize("H, Hkv, vd", [(4, 2, 64), (32, 8, 64), (12, 3, 5), (16, 2, 130), (8, 1, 70), (6, 2, 33), (5, 5, 16), (1, 1, 1)])
 def test_mix_of_heads_against_the_sum_in_float64(gpu, H, Hkv, vd):
     """Two, four and eight heads a kv head (with and without heads left over after eight at a time) and the others: to the

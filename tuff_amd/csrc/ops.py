@@ -63,8 +63,8 @@ _SIGNATURES = {
                              _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                              _c_int, _c_int, _c_void_p],
         "tuff_forget_scan": [_c_void_p, _c_int, _c_ll, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
-                             _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
-        "tuff_forget_chunked": [_c_void_p, _c_ll, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p,
+                             _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+        "tuff_forget_chunked": [_c_void_p, _c_ll, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p,
                                 _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
     },
     "moe": {
@@ -2078,11 +2078,12 @@ def ssd_chunked(xbc, dt_raw, dt_bias, A_log, D_skip, state, out, *, q_start, q_l
         _gpu("state_slot", state_slot, torch.int32, (R,)), T, R, H, G, N, P, _stream()), "ssd_chunked")
 
 
-def forget_scan(x, bias, lower, state, out, *, q_start, q_len, state_slot, H, D, Dv) -> None:
+def forget_scan(x, bias, lower, state, out, *, q_start, q_len, state_slot, H, D, Dv, below: int = 0, own_tokens: int = 0) -> None:
     """The forget-gate recurrence over each request's tokens of the step, from and to state[slot] (float32
     [slots, H, D, Dv]): f = lower + (1 - lower) sigmoid(z + bias); S = diag(f) S + (1 - f) v^T; o = S^T silu(q).
     x [T, 2 H D + H Dv]: a token's projected rows q, z, v side by side; bias (or None) and lower float32 [H * D];
-    out float32 [T, H * Dv]."""
+    out float32 [T, H * Dv].  below > 0: requests of that many tokens of the step and more are left alone; the others have
+    own_tokens of them (the launch is planned by it, the result does not depend on it)."""
     T = x.shape[0]
     R = q_start.shape[0]
     if D > SCAN_MAX_DIM:
@@ -2093,29 +2094,30 @@ def forget_scan(x, bias, lower, state, out, *, q_start, q_len, state_slot, H, D,
         _gpu("lower", lower, torch.float32, (H * D,)), work[0].data_ptr(), work[1].data_ptr(),
         _gpu("state", state, torch.float32, (None, H, D, Dv)), _gpu("out", out, torch.float32, (T, H * Dv)),
         _gpu("q_start", q_start, torch.int32, (R,)), _gpu("q_len", q_len, torch.int32, (R,)),
-        _gpu("state_slot", state_slot, torch.int32, (R,)), T, R, H, D, Dv, _stream()), "forget_scan")
+        _gpu("state_slot", state_slot, torch.int32, (R,)), T, R, H, D, Dv, int(below), int(own_tokens), _stream()), "forget_scan")
 
 
-def forget_chunked_supported(D: int, Dv: int) -> bool:
+def forget_chunked_supported(D: int, Dv: int, state: Optional[torch.Tensor] = None) -> bool:
     """Whether the chunked form takes these sizes: keys of 16, 32, 48 or 64 channels (what a workgroup's LDS holds twice a
-    CU), values of a multiple of 16 up to 256."""
-    return D % 16 == 0 and 0 < D <= 64 and Dv % 16 == 0 and 0 < Dv <= 256
+    CU), values of a multiple of 16 up to 256, and, where it is given, this state (on a 16-byte border)."""
+    return D % 16 == 0 and 0 < D <= 64 and Dv % 16 == 0 and 0 < Dv <= 256 and (state is None or state.data_ptr() % 16 == 0)
 
 
-def forget_chunked(x, bias, lower, state, out, *, q_start, q_len, state_slot, H, D, Dv) -> None:
-    """forget_scan's recurrence for prompt portions in chunks of SSD_CHUNK tokens on the matrix cores (float32 matrix
-    instructions; all factors, sums and the state float32): the same function, its sums in another order.  x float32; the other
-    arguments as for forget_scan."""
+def forget_chunked(x, bias, lower, state, out, *, q_start, q_len, state_slot, H, D, Dv, at_least: int = 1) -> None:
+    """forget_scan's recurrence for prompt portions in chunks of SSD_CHUNK tokens on the matrix cores (factors and the state
+    float32, sums float32 or 64 bits): the same function, its sums in another order.  Requests of fewer than at_least tokens of
+    the step are left alone.  x float32; the other arguments as for forget_scan."""
     T = x.shape[0]
     R = q_start.shape[0]
-    if not forget_chunked_supported(D, Dv):
-        raise KernelError(f"forget_chunked: keys of {D} (16, 32, 48 or 64) and values of {Dv} channels (a multiple of 16 up to 256)")
-    chunks = -(-T // SSD_CHUNK) + R
+    if not forget_chunked_supported(D, Dv, state) or at_least < 1:
+        raise KernelError(f"forget_chunked: keys of {D} (16, 32, 48 or 64) and values of {Dv} channels (a multiple of 16 up to 256), "
+                          f"a state on a 16-byte border, requests of at least {at_least} tokens (1 or more)")
+    chunks = -(-T // SSD_CHUNK) + min(R, T // at_least)
     U = torch.empty(chunks, H, D, Dv, dtype=torch.float32, device=x.device)
     cdec = torch.empty(chunks, H, D, dtype=torch.float32, device=x.device)
     _check(load("recurrent").tuff_forget_chunked(
         _gpu("x", x, torch.float32, (T, 2 * H * D + H * Dv)), x.shape[1], _opt("bias", bias, torch.float32, (H * D,)),
-        _gpu("lower", lower, torch.float32, (H * D,)), U.data_ptr(), cdec.data_ptr(), chunks,
+        _gpu("lower", lower, torch.float32, (H * D,)), U.data_ptr(), cdec.data_ptr(), chunks, int(at_least),
         _gpu("state", state, torch.float32, (None, H, D, Dv)), _gpu("out", out, torch.float32, (T, H * Dv)),
         _gpu("q_start", q_start, torch.int32, (R,)), _gpu("q_len", q_len, torch.int32, (R,)),
         _gpu("state_slot", state_slot, torch.int32, (R,)), T, R, H, D, Dv, _stream()), "forget_chunked")

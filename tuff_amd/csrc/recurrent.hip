@@ -515,15 +515,16 @@ __global__ __launch_bounds__(256) void ssd_chunk_out_kernel(SsdChunkArgs p) {
 // state at a chunk's start takes U's place, (3) every chunk's outputs.  Products by float32 matrix instructions (16 x 16 x 4).
 // Token by token a rounding decays with the state it is in; so that the chunks' sums are no further from the exact ones, a
 // block's are formed from its first token to its last, the gates' products and the sums over channels inside a block in 64
-// bits, and the latter meet the values in 64-bit matrix instructions.  A wave keeps the state's columns of 16 value channels as accumulators: element e of tile i of a lane of
-// group q is row 16 i + 4 q + e, and since an inner index may be taken in any order, the accumulators are, as they lie, the
-// second operand of (q_t Q_t)^T S.  What bounds it: matrix instructions (32 of float32 and 4 of 64 bits, three times as long, a
+// bits, and the latter meet the values in 64-bit matrix instructions.  A wave keeps the state's columns of 16 value channels
+// as accumulators: element e of tile i of a lane of group q is row 16 i + 4 q + e, and since an inner index may be taken in any
+// order, the accumulators are, as they lie, the second operand of (q_t Q_t)^T S.  What bounds it: matrix instructions (32 of float32 and 4 of 64 bits, three times as long, a
 // block and wave of the last kernel) and the way of the rows; token by token it is a chain of 2,048 steps on 512 waves.  One
-// request of 2,048 tokens, 16 heads of 64 x 128, with what prepares the rows: 177 -> 65 us (59 with all sums in float32).
+// request of 2,048 tokens, 16 heads of 64 x 128, with what prepares the rows: 178 -> 66 us (59 with all sums in float32).
 // Error against 64 bits (norm of the difference over the norm), token by token and in chunks: outputs 6.5e-8 and 5.3e-8, state
 // 1.05e-7 and 1.04e-7; with gates near their lower bounds 7.3e-8 and 6.3e-8, 1.39e-7 and 1.38e-7; with short memories
-// 4.9e-8 and 3.5e-8, 4.2e-8 and 3.4e-8 (all in float32 8.1e-8 and 1.10e-7, 8.7e-8 and 1.42e-7, 6.6e-8 and 3.4e-8).  The sums of a token are formed in another
-// order than token by token, so a position's result depends on where its portion began, within float32 rounding.
+// 4.9e-8 and 3.5e-8, 4.2e-8 and 3.4e-8 (all in float32 8.1e-8 and 1.10e-7, 8.7e-8 and 1.42e-7, 6.6e-8 and 3.4e-8).  The sums
+// of a token are formed in another order than token by token, so a position's result depends on how long its portion is and
+// where it began, within float32 rounding, and on nothing else of the step.
 constexpr int BLOCK = 16;
 
 struct ForgetChunkArgs {
@@ -536,6 +537,7 @@ struct ForgetChunkArgs {
     float* out;                     // [T][H][Dv]
     const int *q_start, *q_len, *state_slot;
     int R, H, D, Dv;
+    int at_least;                   // requests of fewer tokens of the step are not looked at
 };
 
 constexpr int FORGET_LDK = CHUNK + 4;     // floats between two channels' rows of tokens in LDS
@@ -545,7 +547,7 @@ __device__ __forceinline__ bool chunk_of_wave(const ForgetChunkArgs& p, int ci, 
     const int lane = threadIdx.x % WAVE;
     for (int base = 0; base < p.R; base += WAVE) {
         const int r = base + lane;
-        const int n = r < p.R ? max(p.q_len[r], 0) : 0, start = r < p.R ? p.q_start[r] : 0;
+        const int len = r < p.R ? p.q_len[r] : 0, n = len >= p.at_least ? len : 0, start = r < p.R ? p.q_start[r] : 0;
         int upto = (n + CHUNK - 1) / CHUNK;                // chunks of the requests up to and with this lane's
 #pragma unroll
         for (int off = 1; off < WAVE; off *= 2) {
@@ -666,10 +668,10 @@ __global__ __launch_bounds__(512, 4) void forget_chunk_state_kernel(ForgetChunkA
 __global__ __launch_bounds__(256) void forget_state_pass_kernel(ForgetChunkArgs p) {
     const int r = blockIdx.x, head = blockIdx.y;
     const int n = p.q_len[r];
-    if (n <= 0) return;
+    if (n < p.at_least) return;
     const int DV = p.D * p.Dv, e = (blockIdx.z * 256 + threadIdx.x) * 4;
     int before = 0;
-    for (int r2 = threadIdx.x % WAVE; r2 < r; r2 += WAVE) before += (max(p.q_len[r2], 0) + CHUNK - 1) / CHUNK;
+    for (int r2 = threadIdx.x % WAVE; r2 < r; r2 += WAVE) before += p.q_len[r2] >= p.at_least ? (p.q_len[r2] + CHUNK - 1) / CHUNK : 0;
 #pragma unroll
     for (int off = 1; off < WAVE; off *= 2) before += __shfl_xor(before, off, WAVE);
     if (e >= DV) return;
@@ -832,6 +834,7 @@ struct ScanArgs {
     long long ldv;                  // elements between two tokens' rows of v
     long long lda;                  // elements between two tokens' rows of a and k
     const float* head_bonus;        // ssd: [H], the factor of the token's own value in its output
+    int below = 0x7FFFFFFF;         // requests of that many tokens of the step and more are not looked at
     bool by_xcd = false;            // set by the launch
 };
 
@@ -912,7 +915,7 @@ __global__ __launch_bounds__(NW * WAVE, NI16 == 1 ? 4 : NI16 == 2 ? 3 : 2) void 
         head = pair / gridDim.x;
     }
     const int n = p.q_len[r], t0 = p.q_start[r], slot = p.state_slot[r];        // (asked for together)
-    if (n <= 0) return;
+    if (n <= 0 || n >= p.below) return;
     const int D = p.D, Dv = p.Dv, H = p.H, Ha = p.Ha;
     const int ha = head / (H / Ha);
     const int part = lane % SPLIT;
@@ -1408,10 +1411,11 @@ TUFF_EXPORT int tuff_ssd_chunked(const void* xbc, long long ld, const float* dt_
 }
 
 // forget: x rows [q (H*D) | z (H*D) | v (H*Dv)] of type dt, ld elements apart, as projected; bias (or null) and lower
-// float32 [H*D]; work arrays qn, f float32 [T][H*D]; state float32 [slots][H][D][Dv]; out float32 [T][H][Dv].
+// float32 [H*D]; work arrays qn, f float32 [T][H*D]; state float32 [slots][H][D][Dv]; out float32 [T][H][Dv].  below > 0:
+// requests of that many tokens and more are left alone, and own_tokens of the step's are the others'.
 TUFF_EXPORT int tuff_forget_scan(const void* x, int dt, long long ld, const float* bias, const float* lower, float* qn, float* f,
                                  float* state, float* out, const int* q_start, const int* q_len, const int* state_slot,
-                                 int n_tokens, int n_requests, int H, int D, int Dv, hipStream_t stream) {
+                                 int n_tokens, int n_requests, int H, int D, int Dv, int below, int own_tokens, hipStream_t stream) {
     if (n_requests <= 0 || n_tokens <= 0) return 0;
     if (H <= 0 || H > 65535 || ld < 2LL * H * D + (long long)H * Dv) return -2;
     const int HD = H * D;
@@ -1423,21 +1427,25 @@ TUFF_EXPORT int tuff_forget_scan(const void* x, int dt, long long ld, const floa
     // (k and the per-token scalar are loaded and not used: they point at arrays of the right reach)
     const void* v = dt == DT_F32 ? (const void*)((const float*)x + 2LL * HD) : (const void*)((const bf16_t*)x + 2LL * HD);
     ScanArgs p{qn, qn, v, f, f, state, out, q_start, q_len, state_slot, H, H, D, Dv, ld, (long long)H * D, nullptr};
-    return dt == DT_F32 ? launch_scan<float, float, false, true>(p, n_tokens, n_requests, stream)
-                        : launch_scan<float, bf16_t, false, true>(p, n_tokens, n_requests, stream);
+    if (below > 0) p.below = below;
+    const int own = below > 0 ? own_tokens : n_tokens;     // (what the launch is planned by; the result is the same for any)
+    return dt == DT_F32 ? launch_scan<float, float, false, true>(p, own, n_requests, stream)
+                        : launch_scan<float, bf16_t, false, true>(p, own, n_requests, stream);
 }
 
 // The same recurrence in chunks of 64 tokens on the matrix cores (see above), from float32 rows: D 16, 32, 48 or 64, Dv a
-// multiple of 16 up to 256.  Work arrays: U float32 [chunks][H][D][Dv] and cdec float32 [chunks][H][D] with chunks >=
-// ceil(T / 64) + requests (what the step's portions can be cut into at most).
+// multiple of 16 up to 256, for the requests of at_least tokens and more (the others are left alone).  Work arrays: U float32
+// [chunks][H][D][Dv] and cdec float32 [chunks][H][D] with chunks >= ceil(T / 64) + the most such requests there can be (what
+// the step's portions can be cut into at most).
 TUFF_EXPORT int tuff_forget_chunked(const float* x, long long ld, const float* bias, const float* lower, float* U, float* cdec, int chunks,
-                                    float* state, float* out, const int* q_start, const int* q_len, const int* state_slot,
+                                    int at_least, float* state, float* out, const int* q_start, const int* q_len, const int* state_slot,
                                     int n_tokens, int n_requests, int H, int D, int Dv, hipStream_t stream) {
     if (n_requests <= 0 || n_tokens <= 0) return 0;
     if (H <= 0 || H > 65535 || n_requests > 65535 || ld < 2LL * H * D + (long long)H * Dv || ld > (1 << 24)) return -2;
-    if (D <= 0 || D % 16 || D > 64 || Dv <= 0 || Dv % 16 || Dv > 256 || chunks < ceil_div(n_tokens, CHUNK) + n_requests) return -2;
+    if (D <= 0 || D % 16 || D > 64 || Dv <= 0 || Dv % 16 || Dv > 256 || at_least < 1) return -2;
+    if (chunks < ceil_div(n_tokens, CHUNK) + min(n_requests, n_tokens / at_least)) return -2;
     if (((uintptr_t)state | (uintptr_t)U) & 15) return -2;           // read in fours
-    ForgetChunkArgs p{x, ld, bias, lower, state, U, cdec, out, q_start, q_len, state_slot, n_requests, H, D, Dv};
+    ForgetChunkArgs p{x, ld, bias, lower, state, U, cdec, out, q_start, q_len, state_slot, n_requests, H, D, Dv, at_least};
     const dim3 block(WAVE * min(8, Dv / 16)), grid(chunks, H);
     const size_t lds = (size_t)(D * FORGET_LDK + 3 * CHUNK * (D + 4) + CHUNK / BLOCK * D + 2 * CHUNK * (BLOCK + 4)) * sizeof(float);
 #define GO(NI) do { \

@@ -13,6 +13,15 @@ import numpy as np
 import torch
 
 
+# From how many tokens of a step on a request's run is a long one: recurrences with a form in chunks take that for it, whatever else
+# is in the step (a request's numbers do not depend on its company).  The line is where the forget gate's two forms cost the same:
+# 16 heads of 64 x 128, token by token / in chunks, us: one run of 256 tokens 29.3 / 32.2, of 288 32.1 / 32.9, 320 35.0 / 32.9,
+# 512 51.9 / 34.9, 2,048 178 / 66; four of 300 50.6 / 56.3, five of 384 71.5 / 63.8, eight of 512 118 / 112; 8 heads of 48 x 256
+# meet at 384, 4 of 32 x 32 below 256.  A step with both kinds runs one form after the other: 1,500 tokens beside 31 single ones
+# 111 us (all token by token 282, all in chunks 119), 400 beside four of 250 96 (63, 58).
+LONG_RUN = 288
+
+
 @dataclasses.dataclass
 class StepEntry:
     """The next tokens of one request, and the places among them whose logits are wanted."""
@@ -47,16 +56,16 @@ class StepContext:
     max_q_len: int = 1
     max_ctx_len: int = 1           # an upper bound of every position + 1 of the step
     host: dict = dataclasses.field(default_factory=dict)     # 'q_len', 'ctx_len' (numpy) and what parts cache
+    long_tokens: int = 0           # tokens of the step that belong to requests with LONG_RUN of them or more
     recorder: object = None        # set while a step is recorded in sections
     inputs: dict = dataclasses.field(default_factory=dict)   # name -> int32 [T, cols]: what parts declared as TokenInput
 
+    LONG_RUN = LONG_RUN
+
     @property
-    def has_long_run(self) -> bool:
-        """Whether a request's tokens of this step are many enough for a recurrence's chunked form.  Token by token a step takes
-        as long as its longest run, in chunks as long as all of them and their number: 16 heads of 64 x 128, runs of 384, 512 and
-        2,048 tokens alone 39 / 30, 50 / 31 and 177 / 59 us, four of 300 and of 512 49 / 49 and 69 / 56, eight of 512 107 / 94,
-        one of 1,500 beside 31 single tokens 282 / 106."""
-        return self.max_q_len >= 384 + 8 * self.R
+    def runs(self) -> tuple[bool, bool]:
+        """Whether the step has requests of LONG_RUN tokens and more, and of fewer."""
+        return self.long_tokens > 0, self.long_tokens < self.T
 
     def run_eagerly(self, fn) -> None:
         """fn(ctx) now; where the step is being recorded in sections, fn is kept instead and runs at
@@ -79,6 +88,7 @@ class PackedStep:
     max_blocks: int
     max_q_len: int
     max_ctx_len: int
+    long_tokens: int
     q_len: np.ndarray
     ctx_len: np.ndarray
     logit_rows_identity: bool = False     # logits are wanted of every token of the step, in order
@@ -165,7 +175,7 @@ def pack_step(entries: Sequence[StepEntry], manager, vocab_size: int,
     tokens, positions, req_of = (buf[offs[i]:offs[i + 1]] for i in range(3))
     q_start, q_len, ctx_len, slot, rows = (buf[offs[i]:offs[i + 1]] for i in range(3, 8))
     info = buf[offs[8 + 2 * n_groups]:offs[9 + 2 * n_groups]].reshape(R, 4)
-    t = li = 0
+    t = li = long_tokens = 0
     max_q = max_ctx = 1
     slot_maps = [buf[offs[8 + 2 * g]:offs[9 + 2 * g]] for g in range(n_groups)]
     block_tables = [buf[offs[9 + 2 * g]:offs[10 + 2 * g]].reshape(R, max_blocks) for g in range(n_groups)]
@@ -210,10 +220,12 @@ def pack_step(entries: Sequence[StepEntry], manager, vocab_size: int,
                 slot_maps[g][t:t + n] = pages * ps + pos % ps
         t += n
         max_q, max_ctx = max(max_q, n), max(max_ctx, total)
+        if n >= LONG_RUN:
+            long_tokens += n
     identity = n_logits == T and bool((rows == np.arange(T)).all())
     check_token_inputs(entries, token_inputs)
     _fill_token_inputs(buf, offs, 9 + 2 * n_groups, token_inputs, entries, manager)
-    return PackedStep(buf, offs, T, R, n_logits, n_groups, max_blocks, max_q, max_ctx, q_len.copy(), ctx_len.copy(),
+    return PackedStep(buf, offs, T, R, n_logits, n_groups, max_blocks, max_q, max_ctx, long_tokens, q_len.copy(), ctx_len.copy(),
                       identity, tuple(token_inputs))
 
 
@@ -226,7 +238,7 @@ def context_on(dev: torch.Tensor, p: PackedStep, max_ctx_len: Optional[int] = No
     return StepContext(T=p.T, R=p.R, n_logits=p.n_logits, tokens=sl(0), positions=sl(1), req_of_token=sl(2),
                        q_start=sl(3), q_len=sl(4), ctx_len=sl(5), state_slot=sl(6), logit_rows=sl(7),
                        req_info=sl(8 + 2 * p.n_groups).view(p.R, 4), groups=groups, max_q_len=p.max_q_len,
-                       max_ctx_len=max_ctx_len if max_ctx_len is not None else p.max_ctx_len,
+                       max_ctx_len=max_ctx_len if max_ctx_len is not None else p.max_ctx_len, long_tokens=p.long_tokens,
                        host={"q_len": p.q_len, "ctx_len": p.ctx_len, "logit_rows_identity": p.logit_rows_identity,
                              "packed": {name: p.buf[int(offs[i]):int(offs[i + 1])] for i, name in
                                         ((0, "tokens"), (2, "req_of_token"), (3, "q_start"), (4, "q_len"), (6, "state_slot"))}},

@@ -379,7 +379,7 @@ class DecoderModel:
         """What forward() reads of a step outside of ctx.run_eagerly and bakes into its launches: a
         recording of a step in sections is valid for steps with the same key."""
         head_fused, all_rows = self._head_fused(ctx)
-        return (ctx.T, bool((head_fused or self.depth_decls is not None) and all_rows), self._recurrent and ctx.has_long_run)
+        return (ctx.T, bool((head_fused or self.depth_decls is not None) and all_rows), ctx.runs if self._recurrent else None)
 
     def _views_of(self, i: int, cache_views: dict):
         """What run i's mixer is handed as `cache`: None, a view, or a tuple of views."""

@@ -132,7 +132,7 @@ class Part:
 
     #: True if a step with prompt portions through this part can be recorded in sections: outside
     #: of ctx.run_eagerly(fn) the part is graph_safe and reads of ctx only T, tokens, req_of_token,
-    #: q_start, q_len, state_slot and, if it launches kernels of "recurrent", has_long_run (they stay in place between replays, with q_len 0 for requests
+    #: q_start, q_len, state_slot and, if it launches kernels of "recurrent", runs (they stay in place between replays, with q_len 0 for requests
     #: beyond the step's own); everything else of the step (positions, tables, wanted rows, host
     #: facts) it reads inside fn(ctx), which runs again at every replay with that step's ctx, on
     #: tensors it was given from outside (they keep their place too).

@@ -385,11 +385,16 @@ class ForgetGateMixer(Mixer):
         T = h.shape[0]
         x = self.qfv.forward(h, out_dtype=torch.float32)
         o = torch.empty(T, self.H * self.Dv, dtype=torch.float32, device=x.device)
-        # a step with a long portion: in chunks on the matrix cores, where the sizes fit; short ones, single tokens and float32
+        # requests with a long portion: in chunks on the matrix cores, where the sizes fit; short ones, single tokens and float32
         # runs: token by token
-        chunked = h.dtype == torch.bfloat16 and ctx.has_long_run and ops.forget_chunked_supported(self.D, self.Dv)
-        (ops.forget_chunked if chunked else ops.forget_scan)(x, self.f_bias, self.lower, cache.state, o, q_start=ctx.q_start,
-                                                             q_len=ctx.q_len, state_slot=ctx.state_slot, H=self.H, D=self.D, Dv=self.Dv)
+        step = dict(q_start=ctx.q_start, q_len=ctx.q_len, state_slot=ctx.state_slot, H=self.H, D=self.D, Dv=self.Dv)
+        have_long, have_short = ctx.runs
+        below = 0
+        if h.dtype == torch.bfloat16 and have_long and ops.forget_chunked_supported(self.D, self.Dv, cache.state):
+            below = ctx.LONG_RUN
+            ops.forget_chunked(x, self.f_bias, self.lower, cache.state, o, at_least=ctx.LONG_RUN, **step)
+        if have_short or not below:
+            ops.forget_scan(x, self.f_bias, self.lower, cache.state, o, below=below, own_tokens=ctx.T - ctx.long_tokens, **step)
         y = self.rt.empty(T, self.H * self.Dv)
         ops.head_norm_gate(o, self.norm_w, None, y, H=self.H, Dv=self.Dv, eps=self.eps, per_head_weight=False,
                            gate_activation=None)
