@@ -634,6 +634,19 @@ def test_recorded_steps_of_long_portions_short_ones_and_both(gpu):
         assert wanted.any() and torch.equal(got[k][wanted], want[k][wanted]), k
 
 
+@pytest.mark.parametrize("name, dtype", [("wide", "float32"), ("mixed", "bfloat16")])
+def test_one_recording_a_number_of_tokens_where_no_part_asks_for_long_runs(gpu, name, dtype):
+    """float32, and sizes that the chunks do not take: a step of one long portion and one of short ones launch the same and
+    share a recording."""
+    reqs = {k: util.rand_tokens(448 * 4, lu.CONFIGS[name]["vocab"], 30 + i) for i, k in enumerate("ab")}
+    steps = [{"step": i, "entries": [{"id": k, "tokens": reqs[k][n * i:n * (i + 1)], "want": [n - 1]} for k, n in sizes], "end": []}
+             for i in range(4) for sizes in ([("a", 448)], [("a", 224), ("b", 224)])]
+    steps[-1]["end"] = ["a", "b"]
+    eng = engine(name, dtype, max_tokens=8192)
+    util.run_plan(eng, steps)
+    assert eng.section_recordings == 1 and eng.section_replays == 6 and len(eng._sectioned) == 1
+
+
 @pytest.mark.parametrize("H, Hkv, vd", [(4, 2, 64), (32, 8, 64), (12, 3, 5), (16, 2, 130), (8, 1, 70), (6, 2, 33), (5, 5, 16), (1, 1, 1)])
 def test_mix_of_heads_against_the_sum_in_float64(gpu, H, Hkv, vd):
     """Two, four and eight heads a kv head (with and without heads left over after eight at a time) and the others: to the

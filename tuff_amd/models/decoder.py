@@ -58,7 +58,6 @@ class DecoderModel:
         entry: a parts.loop.PassEntry; before a run with `enter` = t the stream becomes what the entry makes of it, of the
         embedding and of t (blocks of the kind that hand each other their first input only)."""
         self.pad_hidden = bool(pad_hidden)
-        self._recurrent = any("recurrent" in b.kernel_modules() for b in blocks)
         self.streams = None if streams is None else int(streams)
         if self.streams is not None and (self.streams < 1 or not all(getattr(b, "multi_stream", False) for b in blocks)):
             raise ValueError("a model with several residual streams needs at least one and blocks that take them")
@@ -379,7 +378,7 @@ class DecoderModel:
         """What forward() reads of a step outside of ctx.run_eagerly and bakes into its launches: a
         recording of a step in sections is valid for steps with the same key."""
         head_fused, all_rows = self._head_fused(ctx)
-        return (ctx.T, bool((head_fused or self.depth_decls is not None) and all_rows), ctx.runs if self._recurrent else None)
+        return (ctx.T, bool((head_fused or self.depth_decls is not None) and all_rows), ctx.runs if self.rt.reads_runs else None)
 
     def _views_of(self, i: int, cache_views: dict):
         """What run i's mixer is handed as `cache`: None, a view, or a tuple of views."""

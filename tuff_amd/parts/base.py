@@ -98,6 +98,7 @@ class Runtime:
     """What parts need at bind time: where tensors live and in which type they compute."""
     device: torch.device
     dtype: torch.dtype              # torch.bfloat16 (serving) or torch.float32 (true 32-bit)
+    reads_runs: bool = False        # set by a part, when it is bound, whose launches depend on a step's ctx.runs
 
     def empty(self, *shape, dtype=None) -> torch.Tensor:
         return torch.empty(*shape, dtype=dtype or self.dtype, device=self.device)
@@ -132,8 +133,8 @@ class Part:
 
     #: True if a step with prompt portions through this part can be recorded in sections: outside
     #: of ctx.run_eagerly(fn) the part is graph_safe and reads of ctx only T, tokens, req_of_token,
-    #: q_start, q_len, state_slot and, if it launches kernels of "recurrent", runs (they stay in place between replays, with q_len 0 for requests
-    #: beyond the step's own); everything else of the step (positions, tables, wanted rows, host
+    #: q_start, q_len, state_slot and, if it has set rt.reads_runs, runs (the tensors stay in place between
+    #: replays, with q_len 0 for requests beyond the step's own); everything else of the step (positions, tables, wanted rows, host
     #: facts) it reads inside fn(ctx), which runs again at every replay with that step's ctx, on
     #: tensors it was given from outside (they keep their place too).
     records_portions = False

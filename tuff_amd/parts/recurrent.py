@@ -378,6 +378,8 @@ class ForgetGateMixer(Mixer):
         self.out.bind(weights, rt)
         f32 = lambda name: weights[n[name]].float().contiguous()
         self.f_bias, self.lower, self.norm_w = f32("f.b"), f32("lower"), f32("norm")
+        if rt.dtype == torch.bfloat16 and ops.forget_chunked_supported(self.D, self.Dv):
+            rt.reads_runs = True
 
     def forward(self, h, ctx, cache, residual, write_cache: bool = True, next_norm=None) -> None:
         if not write_cache:
