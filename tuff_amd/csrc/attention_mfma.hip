@@ -71,11 +71,8 @@ __device__ __forceinline__ void angle(const FusedQKV& fq, int pos, int j, float&
     }
 }
 
-__device__ __forceinline__ float norm_weight(const void* w, int dt, int i) {
-    return dt == DT_F32 ? ((const float*)w)[i] : (float)((const bf16_t*)w)[i];
-}
-
-// The same for N neighbours from j (i) on, a multiple of N: whole pieces at a time, one branch.
+// The same of N neighbours from j on, and N norm weights of either type from i on, both multiples of N: whole pieces at a
+// time, one branch.
 typedef f32x4 f32x4_any __attribute__((aligned(4)));       // (tables and weights may start anywhere)
 typedef bf16x4 bf16x4_any __attribute__((aligned(2)));
 template <int N>
