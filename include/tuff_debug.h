@@ -22,6 +22,9 @@ int tuff_attention_few_waves(int n);
 int tuff_attention_kv_fast_waves(int n);
 /* From how many workgroups on keys of heads of up to 64 channels are read in whole lines through LDS. */
 int tuff_attention_stage_k_waves(int n);
+/* Whether a launch of `blocks` column blocks (requests times kv heads) with n_parts partitions of 256 keys, `columns` columns a
+ * block, takes a workgroup a block instead of one a partition and a merge.  Host arithmetic; no knob. */
+int tuff_attention_takes_whole(long long blocks, int n_parts, int columns);
 /* How many lanes fetch page numbers for partition `part` with pages of page_size positions: the pages
  * the partition touches.  Host arithmetic (the kernel's own function); -2 for nonsense. */
 int tuff_attention_partition_pages(int part, int page_size);

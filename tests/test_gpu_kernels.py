@@ -1052,7 +1052,7 @@ def test_attention_of_heads_that_fill_no_tile_with_an_infinite_key(gpu, H, Hkv, 
     import ctypes
     from tuff_amd.csrc import ops
     lib = ops.load("attention_mfma")
-    reqs = [(299, 1), (30, 20), (517, 1)] + [(70 + i, 1) for i in range(29 if Hkv < 8 else 5)]
+    reqs = [(299, 1), (30, 20), (517, 1)] + [(70 + i, 1) for i in range(29 if Hkv < 8 else 7)]
     case = _mixed_step_case(gpu, reqs, H, Hkv, hd, ps)
     q = case["q"].to(gpu)
     q.view(-1, H, hd)[:, :, 3] = q.view(-1, H, hd)[:, :, 3].abs() + 0.25
@@ -1077,6 +1077,12 @@ def test_attention_of_heads_that_fill_no_tile_with_an_infinite_key(gpu, H, Hkv, 
                                            positions=case["positions"], H=H, Hkv=Hkv, hd=hd, page_size=ps, max_ctx_len=room)
                         torch.cuda.synchronize()
                         outs.setdefault((nb, form, room), []).append(out.float().cpu())
+            single = [r for r, (_, n) in enumerate(reqs) if n == 1]                 # (9 of 8 kv heads: whole columns)
+            info = torch.tensor([[i, 1, reqs[r][0], reqs[r][0] + 1] for i, r in enumerate(single)], dtype=torch.int32, device=gpu)
+            out = torch.full((len(single), H * hd), float("nan"), dtype=torch.bfloat16, device=gpu)
+            ops.attention_mfma(q[:len(single)].contiguous(), kc, case["vc"], out, block_table=table[single].contiguous(), blocks=None, nb=1,
+                               req_info=info, positions=info[:, 2].contiguous(), H=H, Hkv=Hkv, hd=hd, page_size=ps, max_ctx_len=1024)
+            outs.setdefault("singles", []).append(out.float().cpu())
     finally:
         lib.tuff_attention_few_waves(few)
         lib.tuff_attention_stage_k_waves(stage)

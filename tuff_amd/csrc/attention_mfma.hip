@@ -1029,13 +1029,25 @@ int kv_fast_waves = 512;
 int stage_k_waves = 512;
 
 // Eight waves a workgroup that take all partitions of a column block and write the finished rows, no merge after them: for
-// launches of few partitions with work for the chip all the same.  32 heads on 8, whole decode steps of 16 layers of which 6
-// attend, in partitions / by whole column blocks: room for 1,024 keys, 8 requests of 300 747 / 727 us, 600 746 / 743; 16 of 250
-// 838 / 811, 1,000 844 / 841; 64 of 200 1,118 / 1,083; room for 2,048, 23 requests of 1,111 932 / 910, 64 of 1,900 1,236 / 1,227, but
-// 16 of 1,900 860 / 878; room for 3,072, 48 of 3,000 1,221 / 1,240.  One request of 256 643 / 637, of 1,000 641 / 675: a
-// workgroup's share of a CU is then all there is.
+// launches of few partitions with work for the chip all the same.  A workgroup's share of a CU must be most of what there is: the
+// blocks have to fill a round of 256 (with four partitions, where the merge is the larger part, a quarter of one), and where they
+// are more, the last round.  And they must have few columns, whose sums all go through LDS.
+// 32 heads on 8, kernel and merge against the one kernel, us, at the least and the most keys of the room:
+//   room for 1,024:  64 blocks 9.8 / 6.5 (200 keys) and 10.6 / 12.1 (1,000), 128 10.8 / 7.0 and 12.5 / 12.8, 256 12.1 / 7.5 and 17.5 / 16.1,
+//                    384 15.0 / 11.9 and 23.2 / 26.9, 512 16.3 / 12.8 and 28.2 / 29.4, 576 19.4 / 16.8 and 32.8 / 37.7
+//   room for 2,048:  128 13.5 / 14.1 (1,100 keys) and 16.7 / 21.3 (2,000), 160 15.9 / 14.5 and 20.4 / 21.4, 192 17.6 / 15.3 and 22.4 / 22.7,
+//                    256 21.2 / 17.3 and 27.4 / 26.1, 384 29.3 / 27.3 and 38.1 / 44.1, 512 32.2 / 31.4 and 49.3 / 48.7,
+//                    576 37.8 / 39.7 and 57.1 / 63.0, 768 46.5 / 45.2 and 72.2 / 71.9
+// and 64 heads on 8: 256 22.5 / 18.7 and 28.2 / 28.5, 512 34.7 / 34.7 and 52.5 / 53.0; 128 on 8: 256 24.2 / 22.1 and 30.8 / 34.0, room for
+// 1,024 192 12.4 / 8.8 and 16.8 / 19.0.  Whole decode steps of 16 layers of which 6 attend: 24 requests of 1,100 919 / 901, 32 of 1,650
+// 995 / 981, 56 of 1,650 1,203 / 1,198, but 48 of 1,650 1,125 / 1,147 and 36 1,076 / 1,119.
 constexpr int WHOLE_WAVES = 8;
-bool takes_whole(long long blocks, int n_parts) { return n_parts <= 4 ? blocks >= 64 : n_parts <= 8 && blocks >= 176; }
+bool takes_whole(long long blocks, int n_parts, int columns) {
+    constexpr int ROUND = 256, MOST_OF_IT = 176;
+    if (n_parts > 8 || columns > 8) return false;
+    if (blocks <= ROUND) return blocks >= (n_parts <= 4 ? ROUND / 4 : MOST_OF_IT);
+    return columns <= 4 && (blocks - 1) % ROUND + 1 >= MOST_OF_IT;
+}
 
 template <bool FUSED, bool STREAM_V = true>
 int launch_whole(dim3 grid, hipStream_t stream, const bf16_t* q, bf16_t* kc, bf16_t* vc, const int* bt, int max_blocks, const int2* blk,
@@ -1135,7 +1147,8 @@ static int launch_attention(const void* q, const void* k_cache, const void* v_ca
     dim3 grid(n_parts, n_qblocks, Hkv);
     FusedQKV plain_form;
     plain_form.slopes = slopes;
-    if (nb == 1 && hd > 32 && hd <= 64 && takes_whole((long long)n_qblocks * Hkv, n_parts))
+    // (as many blocks as tokens: a token a block, of up to eight columns)
+    if (nb == 1 && hd > 32 && hd <= 64 && takes_whole((long long)n_qblocks * Hkv, n_parts, n_qblocks == n_tokens ? H / Hkv : 16))
         return launch_whole<false>(dim3(1, n_qblocks, Hkv), stream, Q, K, V, block_table, max_blocks, (const int2*)blk, (const int4*)req_info,
                                    H, Hkv, hd, page_size, window, scale, n_parts, plain_form, (bf16_t*)out, sinks);
 #define GO(HDP, NB) launch_partition<HDP, NB, false>(grid, stream, Q, K, V, ws_o, ws_ml, block_table, max_blocks, (const int2*)blk, \
@@ -1190,6 +1203,8 @@ TUFF_EXPORT int tuff_attention_stage_k_waves(int n) {
     return old;
 }
 
+TUFF_EXPORT int tuff_attention_takes_whole(long long blocks, int n_parts, int columns) { return takes_whole(blocks, n_parts, columns); }
+
 TUFF_EXPORT int tuff_attention_kv_fast_waves(int n) {
     const int old = kv_fast_waves;
     if (n >= 0) kv_fast_waves = n;
@@ -1237,7 +1252,7 @@ TUFF_EXPORT int tuff_attention_decode_fused(const void* qkv, void* k_cache, void
     fq.q_norm_w = q_norm_w; fq.k_norm_w = k_norm_w; fq.norm_dt = norm_dt; fq.eps = eps;
     fq.inv_freq = inv_freq; fq.slot_mapping = slot_mapping;
     fq.angles = angles; fq.n_angles = angles ? n_angles : 0;
-    if (takes_whole((long long)n_tokens * Hkv, n_parts))
+    if (takes_whole((long long)n_tokens * Hkv, n_parts, H / Hkv))
         return launch_whole<true>(dim3(1, n_tokens, Hkv), stream, (const bf16_t*)qkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_table,
                                   max_blocks, nullptr, (const int4*)req_info, H, Hkv, 64, page_size, window, scale, n_parts, fq,
                                   (bf16_t*)out, nullptr);
