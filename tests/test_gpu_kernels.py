@@ -383,6 +383,34 @@ def test_gemm_bf16_few_rows_that_lie_in_lds_in_whole(gpu, N, K, most):
         assert torch.equal(res.nan_to_num(7.0), alone[:M].nan_to_num(7.0)), M
 
 
+@pytest.mark.parametrize("N,K,most", [(3072, 2560, 19), (4112, 2312, 21), (2064, 2120, 23), (2568, 2888, 17), (8176, 2056, 23)])
+def test_gemm_bf16_two_row_tiles_that_lie_in_lds_in_whole(gpu, N, K, most):
+    """17 to 23 rows of which all that fit lie in LDS, up to the most that do and one more, whole and ragged inner sizes, columns
+    that fill no block: within float32's K roundings of the float64 product, a row's bits whichever rows are beside it, a row of
+    infinities and NaN for itself; nothing beyond the output is written."""
+    from tuff_amd.csrc import ops
+    x, w = _r(most + 1, K, seed=1, dtype=torch.bfloat16).to(gpu), _r(N, K, seed=2, dtype=torch.bfloat16).to(gpu)
+    tiled = ops.tile_weight(w)
+    exact, bound = x.double() @ w.double().T, K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+
+    def product(rows):
+        M = rows.shape[0]
+        room = torch.full((M * N + 512,), 7.0, device=gpu)
+        ops.gemm(rows.contiguous(), tiled, room[:M * N].view(M, N))
+        assert (room[M * N:] == 7.0).all()
+        return room[:M * N].view(M, N)
+
+    whole = product(x)                                    # (one row more than fit: from memory)
+    assert ((whole.double() - exact).abs() <= bound).all()
+    for M in sorted({17, 18, most - 1, most}):
+        if 17 <= M <= most:
+            assert torch.equal(product(x[:M]), whole[:M]), M
+    other = x[:most].clone()
+    other[1, ::3], other[1, 1::3] = float("inf"), float("nan")
+    out, kept = product(other), [m for m in range(most) if m != 1]
+    assert torch.equal(out[kept], whole[kept]) and not torch.isfinite(out[1]).any()
+
+
 @pytest.mark.parametrize("M", [17, 20, 21])
 @pytest.mark.parametrize("N,K", [(256, 64), (1024, 1024), (2048, 1032), (2048, 2048), (2048, 2056)])
 def test_gemm_bf16_narrow_outputs_of_17_to_21_rows(gpu, M, N, K):

@@ -1616,7 +1616,8 @@ constexpr int skinny16_lds_left(int NW, int MT) { return 160 * 1024 - MT * NW * 
 // Where the waves have many chunks, X goes through LDS as far as it fits; where they have one each, a barrier before its product
 // costs a few rows more than it saves.  Rows from memory / in LDS, us: 2,048 x 8,192 of 1 row 8.9 and 7.8, 4 9.2 and 8.1, 8 9.6 and
 // 8.8; one chunk a wave, 2,048 x 2,048 of 1 row 4.2 and 4.3, 8 4.5 and 4.4, 16 5.2 and 4.7, 3,072 x 2,048 4.8 and 5.2, 5.4 and 5.5, 6.0
-// and 5.7.  (Two chunks a wave lose: 6,144 x 2,048 with the convolution 7.5 and 8.1, 16,384 x 2,048 13.0 and 13.1.)
+// and 5.7; two row tiles, 17 rows, 3,072 x 2,560 6.9 and 6.0, 6,144 x 2,560 11.7 and 10.3, 20 rows, 8,176 x 2,304 12.2 and 11.1.  (Two
+// chunks a wave lose: 6,144 x 2,048 with the convolution 7.5 and 8.1, 16,384 x 2,048 13.0 and 13.1.)
 bool skinny16_rows_in_lds(int NW, int MT, int SHARE, int M, int K) {
     if (K < 256 || (SHARE == SHARE_ONE && M <= 8)) return false;
     return (long long)M * (K + 8) * 2 <= skinny16_lds_left(NW, MT) && (long long)M * K / 8 <= (long long)skinny16_pieces(MT) * NW * WAVE;
