@@ -87,6 +87,17 @@ def test_float32_attention_takes_the_kernel_that_is_faster(T, R, q, keys, window
     assert ops.attention_f32_pays(T, R, q, keys, window, H, Hkv, hd) is want
 
 
+@pytest.mark.parametrize("T,R,q,keys,H,Hkv,hd,want", [
+    (256, 256, 1, 64, 32, 32, 128, True), (256, 256, 1, 200, 32, 32, 128, True), (32, 32, 1, 40, 16, 16, 128, True),     # 666 / 119, 2,013 / 371, 19.4 / 9.5 us
+    (4, 4, 1, 40, 8, 8, 128, True), (256, 256, 1, 200, 32, 32, 16, True), (64, 64, 1, 40, 8, 8, 128, True),              # 17.5 / 6.9, 135 / 66, 19.5 / 9.5
+    (256, 256, 1, 16, 32, 32, 32, False), (256, 256, 1, 16, 16, 16, 64, False), (32, 32, 1, 4, 16, 16, 16, False),       # 19.5 / 43.9, 16.5 / 29.1, 4.8 / 5.4
+    (1, 1, 1, 4, 32, 8, 16, False)])                                                                                     # 4.9 / 5.4
+def test_float32_attention_takes_the_faster_kernel_on_both_sides_of_its_line(T, R, q, keys, H, Hkv, hd, want):
+    """Measured points near the line, general kernel / tiles."""
+    from tuff_amd.csrc import ops
+    assert ops.attention_f32_pays(T, R, q, keys, 0, H, Hkv, hd) is want
+
+
 def test_float32_attention_of_a_mixer_follows_that_rule(monkeypatch):
     import types
 

@@ -1039,16 +1039,20 @@ def attention_f32_supported(dtype, H: int, Hkv: int, hd: int, page_size: int) ->
 
 
 # Microseconds of a workgroup of attention_f32 with the chip full of them, by head size: of two columns and one tile of 64 keys.
-_F32_WORKGROUP = {16: 5.6e-3, 32: 7e-3, 64: 10.5e-3, 128: 28e-3}
+# (64: fitted it is 5.1e-3; with that the sum below would be at 0.07 % instead of 0.12, and 256 requests of 40 keys with a kv head a
+# head, 53 us and 83, would change sides.)
+_F32_WORKGROUP = {16: 2.0e-3, 32: 3.9e-3, 64: 7.2e-3, 128: 10.8e-3}
 
 
 def attention_f32_pays(T: int, R: int, max_q_len: int, max_ctx_len: int, window: int, H: int, Hkv: int, hd: int) -> bool:
     """Whether attention_f32 is faster than attention_general, which gives the same bits, by what the sizes cost either.  A
     workgroup of the first takes a tile of 64 keys for up to 16 columns whatever it holds; a wave of the second takes a key
-    after the other for one column.  So few keys, or many requests with few heads to a kv head, go the second way: 256 requests of
-    40 keys, 32 heads and kv heads of 64: 85 us and 61; 8 of 4 keys 7.2 and 6.0; 256 of 40 keys with 8 kv heads 27 and 55;
-    one of 300 keys 18 and 77.  The constants are fitted to 1 to 256 requests of 1 to 4,000 keys and seven arrangements of heads
-    (nowhere is the one taken slower than the other by more than a quarter; over all of them by 0.4 %)."""
+    after the other for one column.  So a few keys go the second way: 8 requests of 4 keys, 32 heads and kv heads of 64, 5.6 us and
+    5.3, 256 of 16 keys with heads of 32 44 and 20; but 256 of 40 keys with 8 kv heads 19 and 55, one of 300 12.0 and 74, 4 of 1,000
+    30.2 and 241, 256 of 64 with heads of 128 119 and 666.  The constants are fitted to 3,302 measured points, 1 to 256 requests
+    of 1 to 4,000 keys, portions of 2 to 500 tokens, seven arrangements of heads: the sum over all of them is 0.12 % above that of
+    the faster ones (fitted to half of the points, 0.13 % over the other half); 12 are more than a tenth slower than the other
+    way, two more than a quarter (that of the note above, and 256 of 16 keys, 32 heads and kv heads of 128, 102 us and 160)."""
     if R > 65535:                                          # (a grid has no more there)
         return False
     G = H // Hkv
@@ -1058,9 +1062,9 @@ def attention_f32_pays(T: int, R: int, max_q_len: int, max_ctx_len: int, window:
     groups = max(R, -(-T // per)) * Hkv
     columns = min(-(-T // max(R, 1)), per) * G
     causal = 0.6 if max_q_len * 2 > max_ctx_len and max_q_len > 1 else 1.0
-    general = 4.5 + max(keys * (0.165 + 0.001 * hd), T * H * keys * (0.03 + 0.0022 * hd) * 1e-3 * causal)
-    tiled = 3.5 + max(2.0 + 0.028 * hd + (-(-columns // 4) - 1) * (0.6 + 0.006 * hd) + (tiles - 1) * (1.6 + 0.015 * hd),
-                      groups * _F32_WORKGROUP[hd] * (0.45 + 0.55 * tiles))
+    general = 3.83 + max(keys * (0.195 + 0.0012 * hd), T * H * keys * (0.0065 + 0.00274 * hd) * 1e-3 * causal)
+    tiled = 5.0 + max(-1.1 + 0.0284 * hd + (-(-columns // 4) - 1) * (0.496 + 0.004 * hd) + (tiles - 1) * (0.872 + 0.0172 * hd),
+                      groups * _F32_WORKGROUP[hd] * (0.07 + 0.93 * tiles))
     return tiled < general
 
 
