@@ -1441,7 +1441,7 @@ TUFF_EXPORT int tuff_forget_chunked(const float* x, long long ld, const float* b
                                     int at_least, float* state, float* out, const int* q_start, const int* q_len, const int* state_slot,
                                     int n_tokens, int n_requests, int H, int D, int Dv, hipStream_t stream) {
     if (n_requests <= 0 || n_tokens <= 0) return 0;
-    if (H <= 0 || H > 65535 || n_requests > 65535 || ld < 2LL * H * D + (long long)H * Dv || ld > (1 << 24)) return -2;
+    if (H <= 0 || H > 65535 || ld < 2LL * H * D + (long long)H * Dv || ld > (1 << 24)) return -2;
     if (D <= 0 || D % 16 || D > 64 || Dv <= 0 || Dv % 16 || Dv > 256 || at_least < 1) return -2;
     if (chunks < ceil_div(n_tokens, CHUNK) + min(n_requests, n_tokens / at_least)) return -2;
     if (((uintptr_t)state | (uintptr_t)U) & 15) return -2;           // read in fours
