@@ -269,8 +269,9 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     // into registers a step ahead of their use (where the head size leaves room for it); large
     // tiles (head size x columns) load as they go.
     //
-    // What bounds it: a wave issues an instruction in about five cycles, so with three or four waves a SIMD the instructions
-    // around the loads and products count as much as the bytes.  Hence no branch but those a whole wave takes, every lane loads
+    // What bounds it: a wave issues an instruction in about five cycles, so with three waves a SIMD the instructions around the loads
+    // and products count as much as the bytes, until they are few: 64 requests of 8,192 keys then move 5.95 TB/s (counters: two
+    // thirds of a wave's time its instructions wait for the memory side to take them), one request is the chain of its trips.  Hence no branch but those a whole wave takes, every lane loads
     // from a page that holds keys of the request whatever its own are, only steps at an end of the keys look at single keys,
     // and pages of sixteen (STREAM_V) are shifted, not divided: a step of 32 keys in some 170 instructions instead of 670.  One
     // layer's attention, 32 heads on 8: 64 requests of 8,192 keys 201 -> 184 us (5.8 TB/s), 8 of 8,192 29.7 -> 25, one of 256
@@ -1029,24 +1030,31 @@ int kv_fast_waves = 512;
 int stage_k_waves = 512;
 
 // Eight waves a workgroup that take all partitions of a column block and write the finished rows, no merge after them: for
-// launches of few partitions with work for the chip all the same.  A workgroup's share of a CU must be most of what there is: the
-// blocks have to fill a round of 256 (with four partitions, where the merge is the larger part, a quarter of one), and where they
-// are more, the last round.  And they must have few columns, whose sums all go through LDS.
-// 32 heads on 8, kernel and merge against the one kernel, us, at the least and the most keys of the room:
-//   room for 1,024:  64 blocks 9.8 / 6.5 (200 keys) and 10.6 / 12.1 (1,000), 128 10.8 / 7.0 and 12.5 / 12.8, 256 12.1 / 7.5 and 17.5 / 16.1,
-//                    384 15.0 / 11.9 and 23.2 / 26.9, 512 16.3 / 12.8 and 28.2 / 29.4, 576 19.4 / 16.8 and 32.8 / 37.7
-//   room for 2,048:  128 13.5 / 14.1 (1,100 keys) and 16.7 / 21.3 (2,000), 160 15.9 / 14.5 and 20.4 / 21.4, 192 17.6 / 15.3 and 22.4 / 22.7,
-//                    256 21.2 / 17.3 and 27.4 / 26.1, 384 29.3 / 27.3 and 38.1 / 44.1, 512 32.2 / 31.4 and 49.3 / 48.7,
-//                    576 37.8 / 39.7 and 57.1 / 63.0, 768 46.5 / 45.2 and 72.2 / 71.9
-// and 64 heads on 8: 256 22.5 / 18.7 and 28.2 / 28.5, 512 34.7 / 34.7 and 52.5 / 53.0; 128 on 8: 256 24.2 / 22.1 and 30.8 / 34.0, room for
-// 1,024 192 12.4 / 8.8 and 16.8 / 19.0.  Whole decode steps of 16 layers of which 6 attend: 24 requests of 1,100 919 / 901, 32 of 1,650
-// 995 / 981, 56 of 1,650 1,203 / 1,198, but 48 of 1,650 1,125 / 1,147 and 36 1,076 / 1,119.
+// launches of few partitions with work for the chip all the same.  A workgroup's share of a CU must be most of what there is: with
+// more than four partitions (a launch knows the room for keys, not the keys) the blocks have to fill a round of 256, and the last
+// round where they are more; with up to four, where the merge is the larger part, a quarter of a round is enough, and a second
+// round that is half empty loses at the most keys of the room what it gains at the least.  And the more columns a block has, whose
+// sums all go through LDS, the less is gained.
+// 32 heads on 8, kernel and merge against the one kernel, us, at 200, 600 and 1,000 keys of room for 1,024:
+//   64 blocks 9.8 / 6.5, 9.6 / 9.2 and 10.6 / 12.1; 128 10.8 / 7.0, 11.2 / 9.6 and 12.5 / 12.8; 256 12.1 / 7.5, 13.7 / 11.5 and 17.5 / 16.1;
+//   384 15.0 / 11.9, 18.0 / 18.6 and 23.2 / 26.9; 512 16.3 / 12.8, 22.6 / 21.2 and 28.2 / 29.4; 576 19.4 / 16.8, 26.3 / 26.8 and 32.8 / 37.7;
+// at 1,100 and 2,000 of room for 2,048:
+//   128 13.5 / 14.1 and 16.7 / 21.3; 160 15.9 / 14.5 and 20.4 / 21.4; 192 17.6 / 15.3 and 22.4 / 22.7; 256 21.2 / 17.3 and 27.4 / 26.1;
+//   384 29.3 / 27.3 and 38.1 / 44.1; 512 32.2 / 31.4 and 49.3 / 48.7; 576 37.8 / 39.7 and 57.1 / 63.0; 768 46.5 / 45.2 and 72.2 / 71.9.
+// 64 heads on 8: room for 1,024, 384 blocks 15.6 / 12.9, 19.8 / 21.2 and 24.6 / 29.9, 512 17.5 / 13.9, 24.2 / 23.4 and 29.7 / 32.6; for 2,048, 256
+// 22.5 / 18.7 and 28.2 / 28.5, 512 34.7 / 34.7 and 52.5 / 53.0.  128 on 8: for 1,024, 128 11.6 / 8.2, 12.3 / 13.1 and 13.5 / 17.8, 256 13.5 / 9.1,
+// 16.2 / 15.1 and 19.8 / 20.9, 512 19.1 / 16.6, 26.6 / 27.9 and 32.7 / 39.2; for 2,048, 256 24.2 / 22.1 and 30.8 / 34.0.  Whole decode steps of 16
+// layers of which 6 attend: 24 requests of 1,100 919 / 901, 32 of 1,650 995 / 981, 56 of 1,650 1,203 / 1,198, 48 of 100 1,007 / 987, but 48 of 1,650
+// 1,125 / 1,147 and 36 1,076 / 1,119.
 constexpr int WHOLE_WAVES = 8;
 bool takes_whole(long long blocks, int n_parts, int columns) {
     constexpr int ROUND = 256, MOST_OF_IT = 176;
-    if (n_parts > 8 || columns > 8) return false;
-    if (blocks <= ROUND) return blocks >= (n_parts <= 4 ? ROUND / 4 : MOST_OF_IT);
-    return columns <= 4 && (blocks - 1) % ROUND + 1 >= MOST_OF_IT;
+    const bool filled = (blocks - 1) % ROUND + 1 >= MOST_OF_IT;
+    if (n_parts > 8) return false;
+    if (n_parts > 4) return filled && (columns <= 4 || (columns <= 8 && blocks <= ROUND));
+    if (columns <= 4) return blocks >= ROUND / 4 && (blocks <= 2 * ROUND || filled);
+    if (columns <= 8) return (blocks >= ROUND / 4 && blocks <= ROUND) || (filled && blocks <= 2 * ROUND);
+    return filled && blocks <= ROUND;
 }
 
 template <bool FUSED, bool STREAM_V = true>
