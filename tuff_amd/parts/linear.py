@@ -19,10 +19,11 @@ class Linear:
         """swiglu_pair: the two stacked tensors are the gate and the up matrix of a SwiGLU; with
         bfloat16 weights their rows are interleaved so that forward(..., swiglu=True) can apply
         silu(gate) * up in the product's epilogue.
-        bias: checkpoint names of a bias vector per stacked tensor ([out] each), y = x W^T + b.  The
-        products' epilogues have no bias: it is added by a kernel of its own after the product, and a
-        projection with one takes none of the fused ways (activation, convolution or the next norm in
-        the product's epilogue); the result is the same function.
+        bias: checkpoint names of a bias vector per stacked tensor ([out] each), y = x W^T + b.  In
+        bfloat16 the product's own kernel adds it to the float32 sums where there are more than 64 rows
+        and K is not in slices, else a kernel of its own after the product does; a projection with one
+        takes none of the fused ways (SwiGLU, convolution or the next norm in the product's epilogue).
+        The result is the same function.
         float32: the weight is kept in float32 and the product runs in true float32 whatever the run's
         type (a router, whose logits decide which experts a token takes).
         An input size that is no multiple of 8 (the bfloat16 kernels read 16 bytes at a time) is filled up
