@@ -634,6 +634,27 @@ def test_recorded_steps_of_long_portions_short_ones_and_both(gpu):
         assert wanted.any() and torch.equal(got[k][wanted], want[k][wanted]), k
 
 
+def test_forget_scan_in_chunks_takes_as_many_requests_as_the_scan(gpu):
+    """More requests than a grid's second axis holds, all but the last without tokens: what the last has alone.  A state that lies on no
+    16-byte border is refused (the mixer then takes the scan)."""
+    from tuff_amd.csrc import ops
+    H, D, Dv, n, R = 1, 16, 16, 70, 70000
+    gen = torch.Generator().manual_seed(1)
+    x, lower = torch.randn(n, 2 * H * D + H * Dv, generator=gen).to(gpu), (0.9 * torch.rand(H * D, generator=gen)).to(gpu)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device=gpu)
+    got = []
+    for many in (1, R):
+        out, state = torch.empty(n, H * Dv, device=gpu), torch.zeros(2, H, D, Dv, device=gpu)
+        ops.forget_chunked(x, None, lower, state, out, q_start=i32([0] * many), q_len=i32([0] * (many - 1) + [n]),
+                           state_slot=i32([0] * (many - 1) + [1]), H=H, D=D, Dv=Dv)
+        got.append((out, state))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1]) and not got[1][1][0].any()
+    off = torch.zeros(2 * H * D * Dv + 1, device=gpu)[1:].view(2, H, D, Dv)
+    assert ops.forget_chunked_supported(D, Dv) and not ops.forget_chunked_supported(D, Dv, off)
+    with pytest.raises(ops.KernelError):
+        ops.forget_chunked(x, None, lower, off, got[0][0], q_start=i32([0]), q_len=i32([n]), state_slot=i32([1]), H=H, D=D, Dv=Dv)
+
+
 @pytest.mark.parametrize("name, dtype", [("wide", "float32"), ("mixed", "bfloat16")])
 def test_one_recording_a_number_of_tokens_where_no_part_asks_for_long_runs(gpu, name, dtype):
     """float32, and sizes that the chunks do not take: a step of one long portion and one of short ones launch the same and

@@ -517,9 +517,9 @@ __global__ __launch_bounds__(256) void ssd_chunk_out_kernel(SsdChunkArgs p) {
 // block's are formed from its first token to its last, the gates' products and the sums over channels inside a block in 64
 // bits, and the latter meet the values in 64-bit matrix instructions.  A wave keeps the state's columns of 16 value channels
 // as accumulators: element e of tile i of a lane of group q is row 16 i + 4 q + e, and since an inner index may be taken in any
-// order, the accumulators are, as they lie, the second operand of (q_t Q_t)^T S.  What bounds it: matrix instructions (32 of float32 and 4 of 64 bits, three times as long, a
-// block and wave of the last kernel) and the way of the rows; token by token it is a chain of 2,048 steps on 512 waves.  One
-// request of 2,048 tokens, 16 heads of 64 x 128, with what prepares the rows: 178 -> 66 us (59 with all sums in float32).
+// order, the accumulators are, as they lie, the second operand of (q_t Q_t)^T S.  What bounds it: matrix instructions (32 of
+// float32 and 4 of 64 bits, three times as long, a block and wave of the last kernel) and the way of the rows; token by token it
+// is a chain of 2,048 steps on 512 waves.  One request of 2,048 tokens, 16 heads of 64 x 128, with what prepares the rows: 178 -> 66 us (59 with all sums in float32).
 // Error against 64 bits (norm of the difference over the norm), token by token and in chunks: outputs 6.5e-8 and 5.3e-8, state
 // 1.05e-7 and 1.04e-7; with gates near their lower bounds 7.3e-8 and 6.3e-8, 1.39e-7 and 1.38e-7; with short memories
 // 4.9e-8 and 3.5e-8, 4.2e-8 and 3.4e-8 (all in float32 8.1e-8 and 1.10e-7, 8.7e-8 and 1.42e-7, 6.6e-8 and 3.4e-8).  The sums
