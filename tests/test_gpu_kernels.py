@@ -100,6 +100,21 @@ def test_gemm_f32_few_rows(gpu, M, N, K):
     assert torch.equal(acc, y0 + out)
 
 
+@pytest.mark.parametrize("M,N,K", [(4, 8209, 192), (1, 8320, 448), (3, 32776, 2048), (2, 32760, 2112), (8, 4096, 320), (16, 2048, 832), (4, 4112, 1024)])
+def test_gemm_f32_four_rows_a_workgroup(gpu, M, N, K):
+    """Rings of four, six and twelve steps in LDS, with as many steps as lie there, one more and fewer, and column blocks that are not
+    whole: the bits of the general kernel's chain; with SwiGLU those of the product and the kernel that applies it."""
+    from tuff_amd.csrc import ops
+    test_gemm_f32_few_rows(gpu, M, N, K)
+    if N % 2 == 0:
+        w, x = _r(N, K, seed=2).to(gpu), _r(M, K, seed=1).to(gpu)
+        gu, want, out = torch.empty(M, N, device=gpu), torch.empty(M, N // 2, device=gpu), torch.full((M * N // 2 + 64,), 7.0, device=gpu)
+        ops.gemm(x, w, gu)
+        ops.swiglu(gu, want)
+        ops.gemm_f32_swiglu(x, w, out[:M * N // 2].view(M, N // 2))
+        assert torch.equal(out[:M * N // 2].view(M, N // 2), want) and (out[M * N // 2:] == 7.0).all()
+
+
 @pytest.mark.parametrize("F,K", [(8192, 192), (1024, 320), (36, 224), (9, 32), (2050, 64)])
 def test_gemm_f32_with_swiglu_inside(gpu, F, K):
     """Every kernel on whole chains (one wave of few rows, blocks of 32 and 64), columns that fill no block and no eight: the bits of

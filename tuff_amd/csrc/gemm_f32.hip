@@ -375,134 +375,144 @@ __global__ __launch_bounds__(WAVE) void gemm_f32_rows_kernel(const float* __rest
 }
 
 // ---------------------------------------------------------------------------------------- four rows
-// Four rows by 16 columns a wave, the chain on the vector unit: lane (row g, column r16) has one element, v_fmac_f32 takes its
-// x from lane k % 16 of the row's sixteen lanes (row_newbcast), so sixteen k of X are one register, and its w from the lane's own
-// column.  A fused multiply-add waits 6 cycles for the one before it, four of them 24, where a matrix instruction of four k
-// takes 33 and in a loop with its reads 50: where nothing but the chain's length counts, this is the shorter one.  A lone wave
-// issues an instruction in five cycles, so the loop holds next to nothing but the chain, its reads and loads: places in LDS are
-// constants.  4 rows, 2,048 x 8,192: 35 us (rows kernel 49), 2,048 x 2,048: 10.6 (13.9), 6,144 x 2,048: 12.4 (15.7).  What bounds
-// it: the chain alone would take 6 cycles a k, 21 us of those 35; reads, loads and their counters, issued between by the same
-// wave, are the rest.
-// K in steps of 64: X rows of 256 bytes, piece p (16 bytes) of row g at p ^ 4 g; W rows of 256 bytes, piece p of column c at p ^ c.
-__device__ __forceinline__ void chain16(float& acc, float x, const f32x4 (&w)[4]) {
+// Four rows by 16 columns a workgroup of two waves, the chain on the vector unit: lane (row g, column r16) of the first wave has one
+// element, v_fmac_f32 takes its x from a lane of the row's sixteen (row_newbcast), so 64 k of X are four registers, and its w from
+// the lane's own column.  A fused multiply-add waits 6 cycles for the one before it, four of them 24, where a matrix instruction of
+// four k takes 33 and in a loop with its reads 50: where nothing but the chain's length counts, this is the shorter one.  A lone wave
+// issues an instruction in four to five cycles, so the first wave's loop holds next to nothing but the chain and, one between
+// four links, its reads of the next step; the second wave, on another SIMD, does the loads into LDS and says by a barrier a step
+// that they have landed.
+// K in steps of 64: X rows of 256 bytes as they lie; W rows of 256 bytes, piece p (16 bytes) of column c at p ^ c.
+// What bounds it: a step of 64 k takes some 530 cycles, of them 64 links of 6 to 6.5 and 17 reads of 4 (measured alone: a dependent link 6 to 7
+// cycles, an instruction between two of them 3 to 4 more).  4 rows, us, one wave that did the loads itself / two: 2,048 x 8,192 35.6 and
+// 31.8 (rows kernel 49), 2,048 x 2,048 11.4 and 10.1 (13.9), 3,072 x 2,048 11.4 and 10.3, 6,144 x 2,048 13.3 and 12.3 (15.7), 1,536 x 6,912 30.2
+// and 26.9; 16 rows of 2,048 x 8,192 40.0 and 34.0; from 16,384 columns on the memory sets the time of both.
+template <int LANE>
+__device__ __forceinline__ void chain4(float& acc, const f32x4& x, const f32x4& w) {
 #ifdef __HIP_DEVICE_COMPILE__
-    // (s_nop: two wait states, should the compiler have moved x by a vector instruction just before)
-    asm("s_nop 1\n"
-        "v_fmac_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %3 row_newbcast:1 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %4 row_newbcast:2 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %5 row_newbcast:3 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %6 row_newbcast:4 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %7 row_newbcast:5 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %8 row_newbcast:6 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %9 row_newbcast:7 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %10 row_newbcast:8 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %11 row_newbcast:9 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %12 row_newbcast:10 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %13 row_newbcast:11 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %14 row_newbcast:12 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %15 row_newbcast:13 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %16 row_newbcast:14 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %1, %17 row_newbcast:15 row_mask:0xf bank_mask:0xf"
+    // k = 4 LANE + e: register e of lane LANE.  (s_nop: two wait states, should the compiler have moved x by a vector instruction
+    // just before)
+    if constexpr (LANE == 0) asm("s_nop 1" : "+v"(acc));
+    asm("v_fmac_f32_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %2, %6 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %3, %7 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
+        "v_fmac_f32_dpp %0, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
         : "+v"(acc)
-        : "v"(x), "v"(w[0][0]), "v"(w[0][1]), "v"(w[0][2]), "v"(w[0][3]), "v"(w[1][0]), "v"(w[1][1]), "v"(w[1][2]), "v"(w[1][3]),
-          "v"(w[2][0]), "v"(w[2][1]), "v"(w[2][2]), "v"(w[2][3]), "v"(w[3][0]), "v"(w[3][1]), "v"(w[3][2]), "v"(w[3][3]));
+        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(LANE));
 #endif
 }
 
 constexpr int LONG_STEP = 64;
 
-// A wave a workgroup; `row_groups` workgroups of one column block on one XCD (numbers eight apart), so that its L2 serves W again.
+// `row_groups` workgroups of one column block on one XCD (numbers eight apart), so that its L2 serves W again.
 template <int STAGES, bool SWIGLU>
-__global__ __launch_bounds__(WAVE) void gemm_f32_quad_kernel(const float* __restrict__ X, const float* __restrict__ W,
-                                                             float* __restrict__ Y, int M, int N, int K, int row_groups, int accumulate) {
+__global__ __launch_bounds__(2 * WAVE) void gemm_f32_quad_kernel(const float* __restrict__ X, const float* __restrict__ W,
+                                                                 float* __restrict__ Y, int M, int N, int K, int row_groups, int accumulate) {
     constexpr int WTILE = 16 * LONG_STEP, XTILE = 4 * LONG_STEP, STAGE = WTILE + XTILE;
     constexpr int PER = 5;                                // load instructions a step
     static_assert(PER * (STAGES - 2) < 64, "a count that s_waitcnt can hold");
+    static_assert(STAGES % 2 == 0, "two sets of registers in turn");
     extern __shared__ __attribute__((aligned(16))) float tiles[];      // [STAGES][W, X]
-    const int lane = threadIdx.x, r16 = lane % 16, g = lane / 16;
+    const int lane = threadIdx.x % WAVE, r16 = lane % 16, g = lane / 16;
+    const bool brings = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE) != 0;
     const int id = blockIdx.x, group = id / 8 % row_groups, block = id / (8 * row_groups) * 8 + id % 8;
     const long long n0 = (long long)block * 16;
     const int m0 = group * 4;
     if (n0 >= N) return;
     const long long j0 = n0 / 2;                          // SWIGLU: eight gate rows, then their up rows
     const int rows_m = min(4, M - m0), rows_n = SWIGLU ? (int)min(8ll, (long long)N / 2 - j0) : (int)min(16ll, (long long)N - n0);
-    const int offx = g < rows_m ? (g * K + (r16 ^ (4 * g)) * 4) * 4 : NOWHERE;
-    int offw[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int row = i * 4 + g, wrow = SWIGLU ? row % 8 : row;
-        offw[i] = wrow < rows_n ? (((SWIGLU && row >= 8 ? N / 2 : 0) + wrow) * K + (r16 ^ row) * 4) * 4 : NOWHERE;
-    }
     const int steps = K / LONG_STEP;
-    const float* xrows = X + (long long)m0 * K;
-    const float* wrows = W + (SWIGLU ? j0 : n0) * K;
-    const int bytes_w = ((SWIGLU ? N / 2 : 0) + rows_n) * K * 4;
-    // Steps beyond the last are asked for too, of buffers without bytes (zeros, no traffic): the count of loads under way is then
-    // the same in every step, and the places in LDS are constants of a ring of steps.
-    auto issue = [&](auto buf, int s) {
-        const bool there = s < steps;
-        const buffer_t xbuf = make_buffer(xrows, there ? rows_m * K * 4 : 0), wbuf = make_buffer(wrows, there ? bytes_w : 0);
-        const int at = there ? s * (LONG_STEP * 4) : 0;
-        float* to = tiles + decltype(buf)::value * STAGE;
-        load_to_lds(xbuf, to + WTILE, offx, at);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) load_to_lds(wbuf, to + i * 256, offw[i], at);
+    auto turn = [&]() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
     };
-    int atw[4][4], atx[4];                                // of every piece of a row: where it lies
+    // Step s lies in buffer s % STAGES.  Behind turn s step s has landed, and the reads of step s - 1 are done: step s - 1 + STAGES
+    // goes into its buffer.
+    if (brings) {
+        const int offx = g < rows_m ? (g * K + r16 * 4) * 4 : NOWHERE;
+        int offw[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) atw[q][i] = r16 * LONG_STEP + ((4 * q + i) ^ r16) * 4;
-        atx[q] = WTILE + g * LONG_STEP + (q ^ g) * 16 + r16;
-    }
-    struct Half { f32x4 w[2][4]; float x[2]; };
-    auto read = [&](auto buf, auto half) {
-        const float* from = tiles + decltype(buf)::value * STAGE;
-        Half h;
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            constexpr int first = 2 * decltype(half)::value;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) h.w[q][i] = *(const f32x4*)(from + atw[first + q][i]);
-            h.x[q] = from[atx[first + q]];
+        for (int i = 0; i < 4; ++i) {
+            const int row = i * 4 + g, wrow = SWIGLU ? row % 8 : row;
+            offw[i] = wrow < rows_n ? (((SWIGLU && row >= 8 ? N / 2 : 0) + wrow) * K + (r16 ^ row) * 4) * 4 : NOWHERE;
         }
-        return h;
-    };
-    float acc = 0.f;
-    auto multiply = [&](const Half& h) {
-        chain16(acc, h.x[0], h.w[0]);
-        chain16(acc, h.x[1], h.w[1]);
-    };
-    using H0 = std::integral_constant<int, 0>;
-    using H1 = std::integral_constant<int, 1>;
-    static_for<STAGES - 1>([&](auto buf) { issue(buf, decltype(buf)::value); });
-    wait_loads_and_lds<PER * (STAGES - 2)>();
-    Half h0 = read(H0(), H0()), h1;
-    for (int s0 = 0; s0 < steps; s0 += STAGES)
-        static_for<STAGES>([&](auto buf) {
-            constexpr int b = decltype(buf)::value;
-            if (s0 + b >= steps) return;
-            h1 = read(buf, H1());
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(h0);
-            // (the buffer of the step before: its last reads were waited for by the products they went into)
-            issue(std::integral_constant<int, (b + STAGES - 1) % STAGES>(), s0 + b + STAGES - 1);
-            wait_loads_and_lds<PER * (STAGES - 2)>();     // all but those of steps s0 + b + 2 and later
-            h0 = read(std::integral_constant<int, (b + 1) % STAGES>(), H0());
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(h1);
-        });
-    wait_loads_and_lds<0>();                              // nothing may land in LDS that is another workgroup's by then
-    if constexpr (SWIGLU) {
-        const float up = __shfl_xor(acc, 8);
-        if (g < rows_m && r16 < rows_n) Y[(long long)(m0 + g) * (N / 2) + j0 + r16] = swiglu_value(acc, up);
+        const float* xrows = X + (long long)m0 * K;
+        const float* wrows = W + (SWIGLU ? j0 : n0) * K;
+        const int bytes_w = ((SWIGLU ? N / 2 : 0) + rows_n) * K * 4;
+        // Steps beyond the last are asked for too, of buffers without bytes (zeros, no traffic): the count of loads under way is then
+        // the same in every step.
+        auto issue = [&](int buf, int s) {
+            const bool there = s < steps;
+            const buffer_t xbuf = make_buffer(xrows, there ? rows_m * K * 4 : 0), wbuf = make_buffer(wrows, there ? bytes_w : 0);
+            const int at = there ? s * (LONG_STEP * 4) : 0;
+            float* to = tiles + buf * STAGE;
+            load_to_lds(xbuf, to + WTILE, offx, at);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) load_to_lds(wbuf, to + i * 256, offw[i], at);
+        };
+        for (int s = 0; s < STAGES; ++s) issue(s, s);
+        int buf = STAGES - 1;
+        for (int s = 0; s < steps; ++s) {
+            wait_loads_and_lds<PER * (STAGES - 2)>();
+            turn();
+            if (s > 0) issue(buf, s - 1 + STAGES);
+            buf = buf + 1 == STAGES ? 0 : buf + 1;
+        }
+        wait_loads_and_lds<0>();                          // nothing may land in LDS that is another workgroup's by then
         return;
     }
-    if (g < rows_m && r16 < rows_n) {
-        float* y = Y + (long long)(m0 + g) * N + n0 + r16;
-        *y = accumulate ? *y + acc : acc;
+    const bool mine = g < rows_m && r16 < rows_n && !(SWIGLU && r16 >= 8);
+    float* const y = Y + (SWIGLU ? (long long)(m0 + g) * (N / 2) + j0 + r16 : (long long)(m0 + g) * N + n0 + r16);
+    float old = 0.f;
+    if (!SWIGLU && accumulate && mine) old = *y;
+    int atw[16];                                          // of every piece of the lane's row of W: where it lies
+#pragma unroll
+    for (int i = 0; i < 16; ++i) atw[i] = r16 * LONG_STEP + (i ^ r16) * 4;
+    const int atx = WTILE + lane * 4;
+    struct Step { f32x4 w[16]; f32x4 x; };
+    Step r0, r1;
+    float acc = 0.f;
+    turn();                                               // step 0
+    r0.x = *(const f32x4*)(tiles + atx);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) r0.w[i] = *(const f32x4*)(tiles + atw[i]);
+    auto step = [&](const Step& now, Step& next, auto buf, bool more) {       // buf: the next step's
+        const float* from = tiles + decltype(buf)::value * STAGE;
+        __builtin_amdgcn_s_waitcnt(0xC07F);               // lgkmcnt(0): this step's reads
+        if (more) {
+            turn();
+            next.x = *(const f32x4*)(from + atx);
+            static_for<16>([&](auto i) {
+                chain4<decltype(i)::value>(acc, now.x, now.w[decltype(i)::value]);
+                __builtin_amdgcn_sched_barrier(0);
+                next.w[decltype(i)::value] = *(const f32x4*)(from + atw[decltype(i)::value]);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        } else static_for<16>([&](auto i) { chain4<decltype(i)::value>(acc, now.x, now.w[decltype(i)::value]); });
+    };
+    // whole turns of the ring with a step to read behind every one of theirs, then what is left
+    auto ring = [&](int s0, auto whole) {
+        static_for<STAGES>([&](auto b) {
+            constexpr int at = decltype(b)::value;
+            if (!decltype(whole)::value && s0 + at >= steps) return;
+            const bool more = decltype(whole)::value || s0 + at + 1 < steps;
+            std::integral_constant<int, (at + 1) % STAGES> next;
+            if constexpr (at % 2 == 0) step(r0, r1, next, more);
+            else step(r1, r0, next, more);
+        });
+    };
+    int s0 = 0;
+    for (; s0 + STAGES < steps; s0 += STAGES) ring(s0, std::true_type());
+    ring(s0, std::false_type());
+    if constexpr (SWIGLU) {
+        const float up = __shfl_xor(acc, 8);
+        if (mine) *y = swiglu_value(acc, up);
+        return;
     }
+    if (mine) *y = accumulate ? old + acc : acc;
 }
 
 // What the slowest CU takes for four k, in cycles, as measured over 17 to 2,048 rows and 2,048 to 65,536 columns: a round
@@ -520,7 +530,7 @@ int launch_quad(const float* X, const float* W, float* Y, int M, int N, int K, i
     constexpr int lds = STAGES * 20 * LONG_STEP * (int)sizeof(float);
     static_assert(lds <= 65536, "without asking for more");
     const int row_groups = ceil_div(M, 4);
-    hipLaunchKernelGGL((gemm_f32_quad_kernel<STAGES, SWIGLU>), dim3(ceil_div(ceil_div(N, 16), 8) * 8 * row_groups), dim3(WAVE), lds, stream,
+    hipLaunchKernelGGL((gemm_f32_quad_kernel<STAGES, SWIGLU>), dim3(ceil_div(ceil_div(N, 16), 8) * 8 * row_groups), dim3(2 * WAVE), lds, stream,
                        X, W, Y, M, N, K, row_groups, accumulate);
     return launch_status();
 }
@@ -553,13 +563,16 @@ int launch_whole_chain(const float* X, const float* W, float* Y, int M, int N, i
         // Four rows a wave as long as one trip over W serves all rows, or the waves are few enough to run side by side, two a CU (16
         // rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14), and K is not so short that
         // the empty steps it begins with count (4 rows, 2,048 x 64: 3.2 us and 2.7, x 192 3.6 and 3.5, 32,768 x 192 6.4 and 7.2).
-        // Twelve steps in LDS where a CU has one wave (8,192 x 1,024, two a CU: 11.7 us, with six 10.3), else five, of which six waves
-        // fit a CU: beyond, the loads under way are more than enough and the waves side by side count (4 rows, six steps / five / four:
-        // 16,384 x 2,048 28.9, 28.5 and 28.2 us, 21,504 x 2,048 41.8, 37.2 and 36.9, 65,536 x 2,048 100, 98 and 101).
+        // Steps in LDS: twelve where a CU has one workgroup, six where it has two (4,608 x 1,536 9.4 us, with four 10.4), and four beyond,
+        // where the loads under way are more than enough and the workgroups side by side count (4 rows, four / six / twelve: 16,384 x
+        // 2,048 with SwiGLU 30.3, 30.9 and 39.4 us, 9,216 x 2,048 17.5, 18.0 and 24.7, 32,768 x 1,024 30.1, 30.3 and 33.2, 65,536 x 1,536 74.4,
+        // 74.9 and 76.8), but twelve again for eight workgroups a CU and more with a K of 2,048 on, whose loads begin and end
+        // at different times (32,768 x 2,048 59.6, 58.0 and 56.1, 65,536 x 2,048 106.7, 105.4 and 102.2).
         const long long waves = ceil_div_ll(N, 16) * ceil_div(M, 4);
         if (K % LONG_STEP == 0 && K >= 192 && (M <= 4 || waves <= 512)) {
-            if (waves <= 256) return launch_quad<SWIGLU, 12>(X, W, Y, M, N, K, accumulate, stream);
-            return launch_quad<SWIGLU, 5>(X, W, Y, M, N, K, accumulate, stream);
+            if (waves <= 256 || (waves >= 2048 && K >= 2048)) return launch_quad<SWIGLU, 12>(X, W, Y, M, N, K, accumulate, stream);
+            if (waves <= 512) return launch_quad<SWIGLU, 6>(X, W, Y, M, N, K, accumulate, stream);
+            return launch_quad<SWIGLU, 4>(X, W, Y, M, N, K, accumulate, stream);
         }
         if (N <= 4096) return launch_rows<SWIGLU, 16>(X, W, Y, M, N, K, accumulate, stream);
         return launch_rows<SWIGLU, 8>(X, W, Y, M, N, K, accumulate, stream);
