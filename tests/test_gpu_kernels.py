@@ -398,6 +398,53 @@ def test_gemm_bf16_few_rows_that_lie_in_lds_in_whole(gpu, N, K, most):
         assert torch.equal(res.nan_to_num(7.0), alone[:M].nan_to_num(7.0)), M
 
 
+@pytest.mark.parametrize("N,K", [(3072, 2048), (2560, 1536), (1024, 1024), (2056, 2176), (16384, 2048), (13824, 1536), (2048, 3072), (2048, 5120),
+                                 (1536, 6912), (2048, 8192), (2056, 10240), (2048, 12288)])
+@pytest.mark.parametrize("M", [1, 3, 8, 9, 16])
+def test_gemm_bf16_few_rows_of_sizes_that_divide_evenly(gpu, M, N, K):
+    """One to six chunks a wave, X from memory and in LDS, columns that fill the XCDs and that do not: behind a norm (with scales that are
+    exact), with SwiGLU, with the convolution and into the stream, the bits that the plain product's kernel for any sizes gives; a
+    row of infinities and NaN for itself; nothing beyond the outputs is written."""
+    from tuff_amd.csrc import ops
+    x, w = _r(M, K, seed=1, dtype=torch.bfloat16).to(gpu), _r(N, K, seed=2, dtype=torch.bfloat16).to(gpu)
+    if M > 3:
+        x[1, ::3], x[1, 1::3] = float("inf"), float("nan")
+    same = lambda a, b: torch.equal(a.nan_to_num(7.0, 8.0, 9.0), b.nan_to_num(7.0, 8.0, 9.0))
+    tiled, plain = ops.tile_weight(w), torch.empty(M, N, device=gpu)
+    ops.gemm(x, tiled, plain)
+    if N < 8192:                                          # (wider ones go into the stream cut otherwise)
+        room = torch.full((M * N + 512,), 7.0, device=gpu)
+        res, nw = room[:M * N].view(M, N), _r(N, seed=4).to(gpu)
+        res.copy_(_r(M, N, seed=3))
+        want = res + plain
+        xw, ss = torch.empty(M, N, dtype=torch.bfloat16, device=gpu), torch.full(ops.gemm_emit_layout(M, N, K), float("nan"), device=gpu)
+        ops.gemm_accum_emit(x, tiled, res, nw, xw, ss)
+        assert same(res, want) and same(xw, (want * nw).bfloat16()) and (room[M * N:] == 7.0).all()
+        kept = [m for m in range(M) if m != 1 or M <= 3]
+        exact = want.double().square().sum(1)
+        assert ((ss.double().sum(0)[:M] - exact).abs() <= N * 2.0 ** -24 * exact)[kept].all()
+    for n_ss in (1, 250, 256, 257):                       # (beyond 256 groups, and off a border of 16 bytes, the other kernel)
+        for off in (0, 1):
+            sums = torch.zeros(n_ss * 16 + 1, device=gpu)[off:off + n_ss * 16].view(n_ss, 16)
+            sums[0, :M], sums[-1, :M] = 3.0 * K, (1.0 if n_ss > 1 else 4.0) * K        # every row's scale is 1 / 2
+            room = torch.full((M * N + 512,), 7.0, dtype=torch.bfloat16, device=gpu)
+            ops.gemm_scaled(x, sums, 0.0, tiled, room[:M * N].view(M, N))
+            assert same(room[:M * N].view(M, N), (plain * 0.5).bfloat16()) and (room[M * N:] == 7.0).all(), (n_ss, off)
+            if N % 32 == 0:
+                out, ref = (torch.full((M * N // 2 + 64,), 7.0, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+                ops.gemm_scaled(x, sums, 0.0, tiled, out[:M * N // 2].view(M, N // 2), swiglu=True)
+                ops.gemm(x * 0.5, tiled, ref[:M * N // 2].view(M, N // 2), swiglu=True)
+                assert same(out, ref) and (out[M * N // 2:] == 7.0).all(), (n_ss, off)
+            if N % 48 == 0 and K <= 2048:
+                d = N // 3
+                taps, state, slots = _r(d, 4, seed=5).to(gpu), _r(M + 3, 3, d, seed=6).to(gpu), torch.arange(M, dtype=torch.int32, device=gpu).flip(0) + 2
+                grouped = ops.tile_weight(ops.conv_group_rows(w))
+                kw, (a, b), (sa, sb) = dict(conv_w=taps, state_slot=slots), torch.empty(2, M, d, dtype=torch.bfloat16, device=gpu), (state.clone(), state.clone())
+                ops.gemm_conv(x, grouped, a, state=sa, ss=sums, eps=0.0, **kw)
+                ops.gemm_conv(x * 0.5, grouped, b, state=sb, **kw)
+                assert same(a, b) and same(sa, sb) and torch.equal(sa[:2], state[:2]), (n_ss, off)
+
+
 @pytest.mark.parametrize("N,K,most", [(3072, 2560, 19), (4112, 2312, 21), (2064, 2120, 23), (2568, 2888, 17), (8176, 2056, 23)])
 def test_gemm_bf16_two_row_tiles_that_lie_in_lds_in_whole(gpu, N, K, most):
     """17 to 23 rows of which all that fit lie in LDS, up to the most that do and one more, whole and ragged inner sizes, columns

@@ -25,7 +25,7 @@ FLAGS = ["-O3", "-std=c++17", f"--offload-arch={ARCH}", "-fPIC", "-shared", "-fv
          # MFMA results in ordinary vector registers: without this the compiler parks accumulators in
          # the accumulation registers and copies them back and forth around every non-matrix use
          "-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-HEADERS = ["common.h"]
+HEADERS = ["common.h", "gemm_bf16_lean.h"]
 
 MODULES = {
     "elementwise": "elementwise.hip",

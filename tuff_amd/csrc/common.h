@@ -54,6 +54,15 @@ __device__ __forceinline__ float butterfly_max(float v) { const LanePair p = but
 // The value of lane ^ 8, ^ 1, among the sixteen lanes of a row.
 __device__ __forceinline__ float lane_xor8(float v) { return butterfly_pair<8>(v).b; }
 __device__ __forceinline__ float lane_xor1(float v) { return butterfly_pair<1>(v).b; }
+// and of lane ^ 4: lane ^ 7 of eight, of which lane ^ 3 of four.
+__device__ __forceinline__ float lane_xor4(float v) {
+#ifdef __HIP_DEVICE_COMPILE__
+    const int u = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true);
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, u, 0x1B, 0xF, 0xF, true));
+#else
+    return v;
+#endif
+}
 // The sum over the sixteen lanes of a row, steps 8, 4, 2, 1; and in steps 1, 2, 4, 8, where the step of 4 takes a lane of the other
 // four of eight: the two before it have left the same in all four.
 __device__ __forceinline__ float row_sum_down(float v) { return butterfly_sum<1>(butterfly_sum<2>(butterfly_sum<4>(butterfly_sum<8>(v)))); }

@@ -697,10 +697,12 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
                                                                        bf16_t* __restrict__ emit_xw, float* __restrict__ emit_ss,
                                                                        ConvTail cv) {
     constexpr bool CONV = MODE == OUT_CONV;
-    // Neighbouring columns on one XCD (workgroups go round the eight of them) where all workgroups run side by side: one row,
-    // 16,384 x 2,048 13.4 -> 13.0 us, 2,048 x 8,192 of 8 rows 9.9 -> 9.6, 2,048 x 2,048 4.7 -> 4.5, but 65,536 x 2,048 42.5 -> 42.7; with
-    // two row tiles a decode step of 23 rows is 1 % slower.
-    const unsigned block = MT == 1 && gridDim.x <= 512 && gridDim.x % 8 == 0 ? blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+    // Neighbouring columns on one XCD (workgroups go round the eight of them) where all workgroups run side by side, of up to 16
+    // columns each: 2,048 x 8,192 of 8 rows 9.9 -> 9.6 us, 2,048 x 2,048 4.7 -> 4.5.  Wider ones read enough of W by themselves and are faster
+    // as the grid counts them (16,384 x 2,048 of 8 rows 13.4 us and 12.9); with two row tiles a decode step of 23 rows is 1 % slower.
+    // All workgroups begin at the first chunk: beginning at chunks of their own was slower whatever the shape (65,536 x 2,048 of 8 rows
+    // 44.9 -> 44.2, 32,768 x 2,048 25.8 -> 23.8, 6,144 x 2,048 of 32 rows 11.5 -> 11.1, 2,048 x 8,192 of 12 12.2 -> 11.7).
+    const unsigned block = MT == 1 && COLS < 32 && gridDim.x <= 512 && gridDim.x % 8 == 0 ? blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
     static_assert(!CONV || COLS == 8, "the convolution's epilogue takes eight channels a workgroup");
     static_assert(MT == 1 || NORM != NORM_INSIDE, "the norm inside is for at most 16 rows");
     constexpr int TN = CONV ? 3 : (COLS > 16 ? COLS / 16 : 1);           // MFMA tiles side by side: they share the rows of X
@@ -881,11 +883,6 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[mt][tn] = mfma16(o.a[mt][j], o.b[tn][j], acc[mt][tn]);
     };
-    // Workgroups start at different chunks (a rotation by the tile index), so that at any moment
-    // the chip reads from all columns of W and not from one.  The order of a tile's additions
-    // still depends on N and K only.
-    const int rot = (int)((block * 5u) % (unsigned)nchunks);
-    auto chunk_of = [&](int i) { const int c = i + rot; return c >= nchunks ? c - nchunks : c; };
     // NORM_SCALED: 16 parts x ROWS rows; part p adds the tiles p, p + 16, ... of its row.  The first
     // sixteen of them are only asked for here and added after the products, when they have long
     // arrived; a wider matrix adds the rest right away.
@@ -929,7 +926,7 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
     };
     // The wave's chunks, two sets of operands in turn; every way through has its loads and products in straight order.
     const int n = (nchunks - wave + NW - 1) / NW;
-    auto nth = [&](int i) { return chunk_of(wave + i * NW); };
+    auto nth = [&](int i) { return wave + i * NW; };
     // Loads are issued where they stand.  Left alone, the instruction scheduler puts off the last ones of a chunk until the first
     // have arrived and their registers are free again: a second trip to memory (2,048 x 2,048, one chunk a wave, 1 row: 4.64 us,
     // with this 4.15; 16 rows 5.7 and 5.1).
@@ -1109,6 +1106,10 @@ __global__ __launch_bounds__(NW * WAVE, skinny16_waves_a_simd(NW, COLS, MT, MODE
         }
     }
 }
+
+}  // namespace
+#include "gemm_bf16_lean.h"
+namespace {
 
 // 16 < M <= 64.  grid (tiles of 64 columns, K slices).  Wave w owns columns 16w..16w+15 of the
 // tile and all MT row tiles.  The X rows of a K chunk (128 wide) go through LDS once for the
@@ -1623,12 +1624,81 @@ bool skinny16_rows_in_lds(int NW, int MT, int SHARE, int M, int K) {
     return (long long)M * (K + 8) * 2 <= skinny16_lds_left(NW, MT) && (long long)M * K / 8 <= (long long)skinny16_pieces(MT) * NW * WAVE;
 }
 
+// The waves of the product with the convolution in its epilogue, eight channels a workgroup (three half tiles); they split K as
+// always, at most eight of them: sixteen would leave a wave 128 registers, too few for three tiles' operands of two chunks.
+int skinny16_conv_waves(int N, int K) {
+    const int groups = N / 3 / 8, chunks = ceil_div(K, SK_CHUNK);
+    int waves = 4;
+    while (waves < 8 && groups * waves < 3072 && chunks >= 2 * waves) waves *= 2;
+    return waves;
+}
+
+// Whether the kernel for sizes that divide evenly takes a product (cut as p says), and launches it: 1 launched, 0 not taken, else an
+// error (negative).
+template <int MODE, int NORM, bool EMIT>
+int launch_lean16(const SkinnyPlan& p, const void* X, const bf16_t* W, void* Y, int M, int N, int K, const Skinny16Extra& x, hipStream_t stream) {
+    constexpr bool CONV = MODE == OUT_CONV, SCALED = NORM == NORM_SCALED;
+    const int chunks = K / SK_CHUNK, share = ceil_div(chunks, p.waves), grid = CONV ? N / 24 : N / p.cols;
+    if (M > 16 || K % SK_CHUNK != 0 || chunks < 8 || (!CONV && N % p.cols != 0) || grid > 8192 || share > 6) return 0;
+    if (SCALED && (x.n_ss > 256 || (uintptr_t)x.ss_in % 16 != 0)) return 0;      // (sums of squares go into LDS in pieces of 16 bytes)
+    // Rows of X in LDS: see skinny16_rows_in_lds.
+    const bool rows_in_lds = share > 2 || (share == 1 && M > 8 && p.cols < 32 && !CONV);
+    constexpr int static_lds = 16 * 1024 + (SCALED ? 17 * 1024 + 512 : 512), lds_left = 160 * 1024 - static_lds;
+    const int lds = rows_in_lds ? M * (K + 8) * (int)sizeof(bf16_t) : 0;
+    if (rows_in_lds && (lds > lds_left || p.cols > 16 || CONV)) return 0;
+    Lean16Args a;
+    a.X = (const bf16_t*)X; a.W = W; a.Y = Y; a.ss_in = x.ss_in; a.emit_nw = x.emit_nw; a.emit_xw = x.emit_xw; a.emit_ss = x.emit_ss;
+    a.M = M; a.N = N; a.K = K; a.n_ss = x.n_ss; a.eps = x.eps;
+    a.per_xcd = (CONV || p.cols < 32) && grid <= 512 && grid % 8 == 0 ? grid / 8 : 0;
+    a.pieces_inverse = 0xFFFFFFFFu / (unsigned)ceil_div(K, 512) + 1;
+    a.cv = x.conv;
+#define LEAN(NW, COLS, CH, XL) do { \
+        auto kern = gemm_bf16_lean16_kernel<NW, MODE, SCALED, EMIT, COLS, CH, XL>; \
+        if constexpr (XL) { \
+            static bool set = false; \
+            if (!set) { \
+                if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_left) != hipSuccess) return -1; \
+                set = true; \
+            } \
+        } \
+        hipLaunchKernelGGL(kern, dim3(grid), dim3(NW * WAVE), lds, stream, a); \
+        return 1; \
+    } while (0)
+    if constexpr (CONV) {
+        if (p.waves != 8) return 0;
+        if (share == 1) LEAN(8, 8, 1, false);
+        if (share == 2) LEAN(8, 8, 2, false);
+    } else if constexpr (MODE == OUT_SWIGLU) {
+        if (p.waves == 8 && p.cols == 32) {
+            if (share == 1) LEAN(8, 32, 1, false);
+            if (share == 2) LEAN(8, 32, 2, false);
+        }
+    } else {
+#define LEAN_COLS(NW, COLS) do { \
+        if (share == 1) { if (rows_in_lds) LEAN(NW, COLS, 1, true); else LEAN(NW, COLS, 1, false); } \
+        else if (share == 2) LEAN(NW, COLS, 2, false); \
+        else if (share <= 4) LEAN(NW, COLS, 4, true); \
+        else LEAN(NW, COLS, 6, true); \
+    } while (0)
+        if (p.cols == 8) { if (p.waves == 8) LEAN_COLS(8, 8); else if (p.waves == 16) LEAN_COLS(16, 8); }
+        else if (p.cols == 16) { if (p.waves == 8) LEAN_COLS(8, 16); else if (p.waves == 16) LEAN_COLS(16, 16); }
+#undef LEAN_COLS
+    }
+#undef LEAN
+    return 0;
+}
+
 template <int MODE, int NORM, bool EMIT>
 int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K, const Skinny16Extra& x, hipStream_t stream) {
     // the in-kernel norm needs more registers a wave: at most 8 waves a workgroup
     SkinnyPlan p = plan_skinny(M, N, K, NORM == NORM_INSIDE ? 8 : 16, EMIT, MODE == OUT_CONV);
     size_t lds = NORM == NORM_INSIDE ? (size_t)K * sizeof(float) : 0;
     const int mt = M > 16 ? 2 : 1, chunks = ceil_div(K, SK_CHUNK);
+    if constexpr (MODE == OUT_CONV) p.waves = skinny16_conv_waves(N, K);
+    if constexpr ((NORM == NORM_SCALED && (MODE == OUT_BF16 || MODE == OUT_SWIGLU || MODE == OUT_CONV)) || EMIT) {
+        const int rc = launch_lean16<MODE, NORM, EMIT>(p, X, W, Y, M, N, K, x, stream);
+        if (rc) return rc < 0 ? rc : launch_status();
+    }
 #define GO_XL(NW, COLS, MT, SHARE, XL) hipLaunchKernelGGL((gemm_bf16_skinny16_kernel<NW, MODE, NORM, EMIT, COLS, MT, SHARE, XL>), grid, dim3(NW * WAVE), lds, stream, \
                                         X, W, Y, M, N, K, x.norm_w, x.eps, x.rows, x.ldx ? x.ldx : (long long)K, x.ss_in, x.n_ss, x.emit_nw, x.emit_xw, x.emit_ss, \
                                         x.conv)
@@ -1660,13 +1730,8 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
     } while (0)
 #define GO16(COLS) do { if constexpr (NORM != NORM_INSIDE) GO(16, COLS); else return -3; } while (0)
     if constexpr (MODE == OUT_CONV) {
-        // eight channels a workgroup (three half tiles); the waves split K as always, at most eight of them:
-        // sixteen would leave a wave 128 registers, too few for three tiles' operands of two chunks
-        const int groups = N / 3 / 8;
-        int waves = 4;
-        while (waves < 8 && groups * waves < 3072 && chunks >= 2 * waves) waves *= 2;
-        dim3 grid(groups);
-        if (waves == 4) GO(4, 8); else GO(8, 8);
+        dim3 grid(N / 3 / 8);
+        if (p.waves == 4) GO(4, 8); else GO(8, 8);
     } else {
         dim3 grid(p.tiles);
         if (p.cols == 16) { if (p.waves == 4) GO(4, 16); else if (p.waves == 8) GO(8, 16); else GO16(16); }
