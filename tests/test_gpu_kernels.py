@@ -374,6 +374,43 @@ def test_gemm_bf16_block_shapes_and_orders_give_the_same_bits(gpu, M, N, K, step
         assert torch.equal(out, plain)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 256, 64), (100, 3072, 128), (130, 4608, 192), (300, 2560, 320), (513, 3072, 256), (400, 4608, 1536), (333, 2052, 256),
+                                   (1100, 1536, 512), (1030, 9216, 128), (2049, 6144, 128), (2500, 2048, 64)])
+def test_gemm_bf16_tiled_scales_and_whole_blocks(gpu, M, N, K):
+    """Every shape of block, with fewer steps than are asked for ahead, columns that are whole blocks and that are not, rows that end inside a
+    block's sixteen: sums of squares of up to 16, 32 and more groups (scales that are exact) and the product into the stream against
+    the plain product's bits; nothing beyond the outputs is written, what lies behind the rows of X counts nowhere."""
+    from tuff_amd.csrc import ops
+    behind = torch.full((M + 64, K), float("nan"), dtype=torch.bfloat16, device=gpu)
+    behind[:M] = _r(M, K, seed=1, dtype=torch.bfloat16)
+    x, tiled, plain = behind[:M], ops.tile_weight(_r(N, K, seed=2, dtype=torch.bfloat16).to(gpu)), torch.empty(M, N, device=gpu)
+    ops.gemm(x, tiled, plain)
+    room = lambda n, dtype: torch.full((n + 8192,), 7.0, dtype=dtype, device=gpu)
+    for n_ss in (1, 16, 17, 32, 33, 70):
+        sums = torch.zeros(n_ss, M, device=gpu)
+        sums[0], sums[-1] = 3.0 * K, (1.0 if n_ss > 1 else 4.0) * K                  # every row's scale is 1 / 2
+        out, sw, ref = room(M * N, torch.bfloat16), room(M * N // 2, torch.bfloat16), torch.empty(M, N // 2, dtype=torch.bfloat16, device=gpu)
+        ops.gemm_scaled(x, sums, 0.0, tiled, out[:M * N].view(M, N))
+        assert torch.equal(out[:M * N].view(M, N), (plain * 0.5).bfloat16()) and (out[M * N:] == 7.0).all(), n_ss
+        ops.gemm_scaled(x, sums, 0.0, tiled, sw[:M * N // 2].view(M, N // 2), swiglu=True)
+        ops.gemm((x * 0.5), tiled, ref, swiglu=True)
+        assert torch.equal(sw[:M * N // 2].view(M, N // 2), ref) and (sw[M * N // 2:] == 7.0).all(), n_ss
+    y, nw, xw, y0 = room(M * N, torch.float32), _r(N, seed=4).to(gpu), room(M * N, torch.bfloat16), _r(M, N, seed=3).to(gpu)
+    want = y0 + plain
+    y[:M * N].view(M, N).copy_(y0)
+    ops.gemm(x, tiled, y[:M * N].view(M, N), accumulate=True)
+    assert torch.equal(y[:M * N].view(M, N), want) and (y[M * N:] == 7.0).all()
+    layout = ops.gemm_emit_layout(M, N, K)
+    if layout is not None:
+        y[:M * N].view(M, N).copy_(y0)
+        ss = torch.full(layout, float("nan"), device=gpu)
+        ops.gemm_accum_emit(x, tiled, y[:M * N].view(M, N), nw, xw[:M * N].view(M, N), ss)
+        assert torch.equal(y[:M * N].view(M, N), want) and (y[M * N:] == 7.0).all()
+        assert torch.equal(xw[:M * N].view(M, N), (want * nw).bfloat16()) and (xw[M * N:] == 7.0).all()
+        exact = want.double().square().sum(1)
+        assert ((ss.double().sum(0) - exact).abs() <= N * 2.0 ** -24 * exact).all()
+
+
 @pytest.mark.parametrize("N,K,most", [(2048, 8192, 8), (520, 4104, 16), (2048, 4480, 15), (72, 16392, 4), (2048, 256, 16)])
 def test_gemm_bf16_few_rows_that_lie_in_lds_in_whole(gpu, N, K, most):
     """Inner sizes of many chunks a wave, whole and ragged, up to the most rows that fit (one more, where there may be, comes from memory as before):

@@ -140,6 +140,19 @@ __device__ __forceinline__ bf16x8 load_buffer(buffer_t buf, int offset, int scal
 __device__ __forceinline__ float load_buffer_float(buffer_t buf, int offset, int scalar) {
     return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(buf, offset, scalar, 0));
 }
+__device__ __forceinline__ f32x4 load_buffer_f32x4(buffer_t buf, int offset, int scalar) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(buf, offset, scalar, 0));
+}
+// 4, 8 or 16 bytes to `offset` (a lane's) + `scalar` (the wave's) bytes of the buffer; nothing beyond it is written.
+template <typename T>
+__device__ __forceinline__ void store_buffer(buffer_t buf, int offset, int scalar, T v) {
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8 || sizeof(T) == 16, "a whole store");
+    typedef unsigned words2 __attribute__((ext_vector_type(2)));
+    typedef unsigned words4 __attribute__((ext_vector_type(4)));
+    if constexpr (sizeof(T) == 4) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), buf, offset, scalar, 0);
+    else if constexpr (sizeof(T) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(words2, v), buf, offset, scalar, 0);
+    else __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(words4, v), buf, offset, scalar, 0);
+}
 // The value of lane `lane` (the same for the whole wave).
 __device__ __forceinline__ float lane_of(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));

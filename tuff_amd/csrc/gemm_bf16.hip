@@ -297,6 +297,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     constexpr int BM = 16 * TM * WAVES_M, BN = 16 * TN * WAVES_N;
     constexpr int IA = BM / 8 / NW, IB = BN / 8 / NW;                  // load instructions of X and of W a wave issues a step
     static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "whole instructions");
+    // all arguments in one trip (left alone they are asked for one by one, where they are first needed)
+    asm volatile("" ::"s"(X), "s"(W), "s"(Y), "s"(M), "s"(N), "s"(K), "s"(steps_per_slice));
+    if constexpr (AROUND == TILED_SCALED) asm volatile("" ::"s"(ex.ss_in), "s"(ex.n_ss), "s"(ex.ss_rows), "s"(ex.eps));
     extern __shared__ __attribute__((aligned(16))) bf16_t tiles[];       // [STAGES][BM * TBK] of X then [STAGES][BN * TBK] of W
     bf16_t* As = tiles;
     bf16_t* Bs = tiles + STAGES * BM * TBK;
@@ -329,9 +332,9 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
 #pragma unroll
         for (int j = 0; j < (FOLDS ? TN : 1); ++j) folded[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    const int kb = K / 32;
-    const int last_a = (int)min((long long)BM - 1, (long long)M - 1 - m0);
-    const int last_tile = (int)min((long long)BN / 16 - 1, (N - 1 - n0) / 16);
+    const int kb = (int)((unsigned)K / 32u);
+    const int last_a = min(BM - 1, M - 1 - (int)m0);
+    const int last_tile = min(BN / 16 - 1, (int)((unsigned)(N - 1 - (int)n0) / 16u));
     // instruction q of X (q = wave + NW i) fills rows 8 q .. 8 q + 7; instruction q of W fills block q % 2 of row tile q / 2;
     // offsets from the block's first row (tile), in bytes (global loads: in elements).  Rows and tiles beyond the matrix have results
     // that are never stored.  Through buffers they are not fetched: if they read the last one instead, all blocks ask for the same
@@ -351,7 +354,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     }
     const buffer_t xbuf = make_buffer(X + m0 * K, (last_a + 1) * K * 2);
     const buffer_t wbuf = make_buffer(W + (n0 / 16) * (long long)kb * 512, (last_tile + 1) * kb * 1024);
-    const int nk = K / TBK;
+    const int nk = (int)((unsigned)K / (unsigned)TBK);
     const int kt_begin = blockIdx.z * steps_per_slice, kt_end = FOLDS ? nk : min(nk, kt_begin + steps_per_slice);
     int fold_at = kt_begin + steps_per_slice;                          // the step that the next slice begins with (FOLDS)
 
@@ -431,33 +434,65 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
     // and of the last ones, with no branch inside: with the loads through buffers (load_to_lds) the compiler then counts the
     // fragment reads under way and waits for the ones it needs, where it waited for all of them, those just issued among
     // them, before every group of MFMAs.
-    static_for<STAGES - 1>([&](auto s) {
-        constexpr int st = decltype(s)::value;
-        if (kt_begin + st < kt_end) issue(st, kt_begin + st);
-    });
-    // TILED_SCALED: the sum of squares of each of the block's rows, in SS_PARTS parts: thread (part, row) adds the groups
-    // part, part + SS_PARTS, ... in that order, sixteen loads at a time (one after the other would be as many trips to
-    // memory: a product of few rows leaves 256 groups for 2,048 columns); behind the loop the parts
-    // of a row are added in their order and the row's scale is left for the epilogue.  (Up to sixteen groups, as the
-    // tiled products of a prompt leave them: one thread a row, the scale at once.)
+    // TILED_SCALED: the scale of each of the block's rows out of its sums of squares over groups of columns.  Up to 32 groups (as products of
+    // 64 and more columns a block leave them): a thread a row asks for all of them ahead of the operands and has the scale before they
+    // are there.  Behind the operands, and one condition a load, the sums came when all that had been asked for was there, and the
+    // loop began 0.3 to 0.5 us later.
     constexpr int SS_PARTS = (64 * NW) / BM >= 4 ? 4 : (64 * NW) / BM >= 2 ? 2 : 1;
+    constexpr int SS_AT_ONCE = 32;
     __shared__ float row_ss[AROUND == TILED_SCALED ? SS_PARTS : 1][AROUND == TILED_SCALED ? BM : 1];
     __shared__ float row_scale[AROUND == TILED_SCALED ? BM : 1];
+    const int ss_rows = ex.ss_rows ? ex.ss_rows : M;
+    const bool at_once = AROUND == TILED_SCALED && ex.n_ss <= SS_AT_ONCE && ss_rows < (1 << 23) && gridDim.z == 1;
+    const bool sums = at_once && wave < BM / 64;
+    float ss_v[AROUND == TILED_SCALED ? SS_AT_ONCE : 1];
     if constexpr (AROUND == TILED_SCALED) {
-        // while the first operands are on their way (a product cut along K leaves the scales to the kernel that adds the slices)
-        const int ss_rows = ex.ss_rows ? ex.ss_rows : M;
-        if (ex.n_ss <= 16) {
-            // one trip to memory a row: the scale at once
-            if (tid < BM && gridDim.z == 1) {
-                const long long row = m0 + tid;
-                float v[16], t = 0.f;
 #pragma unroll
-                for (int u = 0; u < 16; ++u) v[u] = (row < M && u < ex.n_ss) ? ex.ss_in[(long long)u * ss_rows + row] : 0.f;
+        for (int u = 0; u < SS_AT_ONCE; ++u) ss_v[u] = 0.f;
+        if (sums) {
+            // (rows beyond the matrix and groups that are none lie behind the buffer: zeros)
+            const buffer_t sbuf = make_buffer(ex.ss_in + m0, ((ex.n_ss - 1) * ss_rows + last_a + 1) * 4);
+            const int at = tid <= last_a ? tid * 4 : NOWHERE;
 #pragma unroll
-                for (int u = 0; u < 16; ++u) t += v[u];
-                row_scale[tid] = 1.0f / sqrtf(t / (float)K + ex.eps);
+            for (int u = 0; u < SS_AT_ONCE / 2; ++u) ss_v[u] = load_buffer_float(sbuf, u < ex.n_ss ? at : NOWHERE, u < ex.n_ss ? u * ss_rows * 4 : 0);
+            if (ex.n_ss > SS_AT_ONCE / 2) {
+#pragma unroll
+                for (int u = SS_AT_ONCE / 2; u < SS_AT_ONCE; ++u)
+                    ss_v[u] = load_buffer_float(sbuf, u < ex.n_ss ? at : NOWHERE, u < ex.n_ss ? u * ss_rows * 4 : 0);
             }
-        } else if (tid < SS_PARTS * BM && gridDim.z == 1) {
+        }
+    }
+    // (steps that are none: the last one's operands again, so that the count of loads under way is known)
+    static_for<STAGES - 1>([&](auto s) {
+        constexpr int st = decltype(s)::value;
+        issue(st, max(0, min(kt_begin + st, kt_end - 1)));
+    });
+    // (a product cut along K leaves the scales to the kernel that adds the slices)
+    if constexpr (AROUND == TILED_SCALED) {
+        if (sums) {
+            float t;
+            if (ex.n_ss <= 16) {
+                t = ss_v[0];
+#pragma unroll
+                for (int u = 1; u < 16; ++u) t += ss_v[u];
+            } else {
+                // in parts as below, so the same bits
+                float part[SS_PARTS];
+#pragma unroll
+                for (int q = 0; q < SS_PARTS; ++q) {
+                    part[q] = ss_v[q];
+#pragma unroll
+                    for (int u = q + SS_PARTS; u < SS_AT_ONCE; u += SS_PARTS) part[q] += ss_v[u];
+                }
+                t = part[0];
+#pragma unroll
+                for (int q = 1; q < SS_PARTS; ++q) t += part[q];
+            }
+            row_scale[tid] = 1.0f / sqrtf(t / (float)K + ex.eps);      // (read in the epilogue, behind the barriers of the loop)
+        } else if (!at_once && tid < SS_PARTS * BM && gridDim.z == 1) {
+            // More groups: SS_PARTS parts, thread (part, row) adds the groups part, part + SS_PARTS, ... in that order, sixteen loads at a
+            // time (one after the other would be as many trips to memory); behind the loop the parts of a row are added in their
+            // order and the row's scale is left for the epilogue.
             const int r = tid % BM, part = tid / BM;
             const long long row = m0 + r;
             float t = 0.f;
@@ -546,7 +581,7 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         return;
     }
     if constexpr (AROUND == TILED_SCALED) {
-        if (ex.n_ss > 16) {                                    // (the parts were written before the loop's first barrier)
+        if (!at_once) {                                        // (the parts were written before the loop's first barrier)
             if (tid < BM) {
                 float t = row_ss[0][tid];
 #pragma unroll
@@ -557,30 +592,33 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         }
     }
     if constexpr (AROUND == TILED_EMIT) {
-        // whole blocks of columns only (the host sees to it): Y += acc, the next norm's operand, the row's sum of squares
+        // whole blocks of columns only (the host sees to it): Y += acc, the next norm's operand, the row's sum of squares.  Sixteen rows a
+        // buffer: those beyond the matrix lie behind it (nothing is fetched or written), and a lane's place is the same in every one.
+        const int at = r16 * N + (int)n0 + wn + g * 4;
         float wave_sq[TM];
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
-            const long long row = m0 + wm + i * 16 + r16;
             float sq = 0.f;
-            if (row < M) {
+            const int row0 = wm + i * 16, rows = max(0, min(16, last_a + 1 - row0));
+            const long long first = (m0 + (rows > 0 ? row0 : 0)) * N;
+            const buffer_t ybuf = make_buffer((float*)Y + first, rows * N * 4), xwbuf = make_buffer(ex.emit_xw + first, rows * N * 2);
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const long long col = n0 + wn + j * 16 + g * 4;
-                    f32x4* yp = (f32x4*)((float*)Y + row * N + col);
-                    f32x4 y;
-                    if constexpr (EARLY) y = y_old[i][j]; else y = *yp;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] += acc[i][j][e];
-                    *yp = y;
-                    f32x4 nw;
-                    if constexpr (EARLY) nw = next_w[j]; else nw = *(const f32x4*)(ex.emit_nw + col);
-                    bf16x4 o = {(bf16_t)(y[0] * nw[0]), (bf16_t)(y[1] * nw[1]), (bf16_t)(y[2] * nw[2]), (bf16_t)(y[3] * nw[3])};
-                    *(bf16x4*)(ex.emit_xw + row * N + col) = o;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) sq = fmaf(y[e], y[e], sq);
+            for (int j = 0; j < TN; ++j) {
+                f32x4 y, nw;
+                if constexpr (EARLY) { y = y_old[i][j]; nw = next_w[j]; }
+                else {
+                    y = load_buffer_f32x4(ybuf, at * 4 + j * 64, 0);
+                    nw = *(const f32x4*)(ex.emit_nw + n0 + wn + j * 16 + g * 4);
                 }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] += acc[i][j][e];
+                store_buffer(ybuf, at * 4 + j * 64, 0, y);
+                const bf16x4 o = {(bf16_t)(y[0] * nw[0]), (bf16_t)(y[1] * nw[1]), (bf16_t)(y[2] * nw[2]), (bf16_t)(y[3] * nw[3])};
+                store_buffer(xwbuf, at * 2 + j * 32, 0, o);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sq = fmaf(y[e], y[e], sq);
             }
+            sq = r16 < rows ? sq : 0.f;
             sq = butterfly_sum<32>(butterfly_sum<16>(sq));
             wave_sq[i] = sq;
         }
@@ -611,10 +649,16 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
                 col_bias[j][e] = ex.bias && col < N ? ex.bias[col] : 0.f;
             }
     }
+    // whole blocks of columns: through buffers, as above
+    const bool whole = N % BN == 0 && N < (1 << 25);
+    constexpr int SIZE = MODE == OUT_BF16 || MODE == OUT_SWIGLU ? 2 : 4, PER = MODE == OUT_SWIGLU ? 2 : 1;      // bytes an output, columns an output
+    const int at = (r16 * (N / PER) + ((int)n0 + wn + g * 4) / PER) * SIZE;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         float sc = 1.f;
         if constexpr (AROUND == TILED_SCALED) sc = row_scale[wm + i * 16 + r16];
+        const int row0 = wm + i * 16, rows = whole ? max(0, min(16, last_a + 1 - row0)) : 0;
+        const buffer_t ybuf = make_buffer((char*)Y + (m0 + (rows > 0 ? row0 : 0)) * (N / PER) * SIZE, rows * (N / PER) * SIZE);
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             f32x4 v = acc[i][j];
@@ -626,7 +670,15 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
                     if constexpr (AROUND == TILED_RELU2) { v[e] = fmaxf(v[e], 0.f); v[e] *= v[e]; }
                 }
             }
-            store_quad<MODE>(Y, m0 + wm + i * 16 + r16, n0 + wn + j * 16 + g * 4, M, N, v);
+            if (whole) {
+                const int here = at + j * 16 / PER * SIZE;
+                if constexpr (MODE == OUT_SWIGLU) store_buffer(ybuf, here, 0, bf16x2{(bf16_t)silu_mul(v[0], v[1]), (bf16_t)silu_mul(v[2], v[3])});
+                else if constexpr (MODE == OUT_BF16) store_buffer(ybuf, here, 0, bf16x4{(bf16_t)v[0], (bf16_t)v[1], (bf16_t)v[2], (bf16_t)v[3]});
+                else {
+                    if constexpr (MODE == OUT_F32_ACCUM) v += load_buffer_f32x4(ybuf, here, 0);
+                    store_buffer(ybuf, here, 0, v);
+                }
+            } else store_quad<MODE>(Y, m0 + wm + i * 16 + r16, n0 + wn + j * 16 + g * 4, M, N, v);
         }
     }
 }
@@ -1825,7 +1877,7 @@ int launch_skinny64_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N
 int tiled_emit_group(int M, int N, int K) {
     const TiledPlan t = plan_tiled(M, N, K);
     if (t.slices > 1) return 64;                        // the kernel that adds the slices emits, 64 columns a workgroup
-    if (!dma_ok(K)) return 0;
+    if (!dma_ok(K) || N >= (1 << 25)) return 0;         // (it counts the bytes of sixteen rows of Y in 31 bits)
     const int bn = t.shape == 0 || t.shape == 5 ? 256 : t.shape == 4 ? 192 : t.shape == 3 ? 64 : 128;
     if (N % bn != 0) return 0;
     return bn;                                          // a workgroup's columns
@@ -1852,6 +1904,7 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
         TiledPlan t = plan_tiled(M, N, K);
         if (rows64_tiled(M, N, K)) { t.shape = 3; t.slices = 1; t.steps_per_slice = ceil_div(K, TBK); t.ws_floats = 0; }
         if (t.slices > 1 && !ws) return -4;
+        if (K == 0) t.shape = 1;                                       // (nothing to read: loads through buffers of no bytes)
         ex.bands = bands_of_rows(t, M, N);
 #define TILED(TM, TN, WM, WN, AHEAD) do { \
             auto kern = gemm_bf16_tiled_kernel<TM, TN, WM, WN, AHEAD, MODE>; \
