@@ -1601,18 +1601,20 @@ TiledPlan plan_tiled(int M, int N, int K) {
         }
         return t;
     }
-    // One round of 128 x 256 blocks in the place of one of pairs of 128 x 128, where K is long: the pairs read an operand once more and
-    // wait for it (2,048 x 8,192 of 2,560 rows 112 -> 103 us, 3,000 125 -> 101, 4,096 131 -> 110; 2,048 x 2,048 28.6 and 28.5, 29.5 and
-    // 29.3, 34.2 and 33.4, 3,072 x 2,048 of 1,536 rows 27.2 and 28.3).
-    if (t.shape == 1 && dma_ok(K) && N % 256 == 0 && nk > 48) { t.shape = 5; return t; }
+    // One round of 128 x 256 blocks in the place of one of pairs of 128 x 128, which read an operand once more and wait for it: 2,048 x 8,192
+    // of 2,560 rows 112 -> 103 us, 4,096 131 -> 110; 3,072 x 2,048 of 1,536 rows 32.0 -> 30.1, 2,048 33.4 -> 30.9; 2,048 x 2,048 of 2,560
+    // rows into the stream 40.1 -> 37.3; 13,824 x 1,536 with SwiGLU of 512 rows 30.7 -> 28.9, 400 29.4 -> 26.7, 384 27.8 and 28.0.
+    if (t.shape == 1 && dma_ok(K) && N % 256 == 0) { t.shape = 5; return t; }
     // few blocks and a short K: blocks of 64 x 64 give enough workgroups without slices of K, whose partial
     // tiles cost a second kernel and as much traffic as the product's own (K = 1536 .. 2048, 96 to 512
     // rows: 9 to 14 us instead of 11 to 19); beyond 48 steps the slices win
     const long long least = (long long)ceil_div(N, 64) * ceil_div(M, 64);
     if (t.shape == 2 && small <= 128 && dma_ok(K) && nk <= 48) {
-        // beyond a round of them one block of 64 x 128 a CU: the second round's few take as long as the first's (400 rows, 4,608 x 1,536:
-        // 14.3 us -> 11.2, 300 rows, 6,144 x 2,048 17.1 -> 13.1, 100 rows, 16,384 x 2,048 21.6 -> 18.9; 280 blocks of 64 x 64 9.7 and 10.3)
-        t.shape = least > 288 && N % 128 == 0 && (long long)(N / 128) * ceil_div(M, 64) <= 256 ? 6 : 3;
+        // where they are well beyond a round, one block of 64 x 128 a CU: the second round's blocks take as long as the first's (64 x 64 and
+        // 64 x 128, us: 400 rows, 4,608 x 1,536 (504 blocks of 64 x 64) 14.3 and 11.2, 300 rows, 6,144 x 2,048 (480) 17.7 and 16.5, 100 rows,
+        // 16,384 x 2,048 (512) 22.2 and 20.3; 512 rows, 2,560 x 1,536 (320) 11.7 and 13.0, 256 rows, 5,632 x 2,048 (352) 15.2 and 17.5, 512
+        // rows, 3,072 x 2,048 (384) 14.4 and 15.8, 400 rows, 3,584 x 2,048 (392) 14.4 and 14.6)
+        t.shape = least > 400 && N % 128 == 0 && (long long)(N / 128) * ceil_div(M, 64) <= 256 ? 6 : 3;
         return t;
     }
     if (t.shape == 2 && small <= 128) {
