@@ -57,6 +57,7 @@ struct FusedQKV {
     // (not of the fused form, but of every form: it travels here)  A distance slope per head [H], or null:
     // slopes[h] * (position - key) is taken off head h's scaled scores.
     const float* slopes = nullptr;
+    int group = 1;                         // query heads a kv head
 };
 
 // cosine and sine of pos * inv_freq[j]: from the table where it reaches, else computed (the same bits)
@@ -167,10 +168,10 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     // Workgroups that run side by side read neighbouring memory when the kv head is what changes fastest
     // from one to the next (a page holds its kv heads one after the other): that order for launches of
     // several rounds of waves, partitions first for the others.
-    const int part = WHOLE ? 0 : kv_fast ? blockIdx.x / Hkv : blockIdx.x, qb = blockIdx.y, kvh = kv_fast ? blockIdx.x % Hkv : blockIdx.z;
+    const int part = WHOLE ? 0 : kv_fast ? blockIdx.x / (unsigned)Hkv : blockIdx.x, qb = blockIdx.y, kvh = kv_fast ? (int)blockIdx.x - part * Hkv : blockIdx.z;
     const int lane = threadIdx.x % WAVE, n16 = lane % 16, g = lane / 16;
     const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const int G = H / Hkv;
+    const int G = fq.group;
     // Every load that depends on another costs a trip to memory, so the chain is kept short: block -> request record (start,
     // length, first position: a portion's positions are consecutive), and beside it the page numbers, all at once -> keys and
     // values.
@@ -178,11 +179,11 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     if (blk) { const int2 b = blk[qb]; r = b.x; col0 = b.y; }
     const int4 info = req_info[r];         // (first token of the request in the step, tokens, first position, -)
     const int* table = block_table + (long long)r * max_blocks;
-    const int t0 = info.x, ncols = info.y * G, pos0 = info.z;
-    // the block's range of keys
-    const int last_col = min(ncols, col0 + NB * 16) - 1;
-    const int pos_max = pos0 + last_col / G;
-    const int lo_min = window > 0 ? max(0, pos0 + col0 / G - window + 1) : 0;
+    const int t0 = info.x, ncols = FUSED ? G : info.y * G, pos0 = info.z;
+    // the block's range of keys (fused: a block is one token's columns)
+    const int last_col = FUSED ? G - 1 : min(ncols, col0 + NB * 16) - 1;
+    const int pos_max = FUSED ? pos0 : pos0 + last_col / G;
+    const int lo_min = window > 0 ? max(0, pos0 + (FUSED ? 0 : col0 / G) - window + 1) : 0;
     const int key_begin = WHOLE ? lo_min / PART * PART : part * PART;
     const int first_page = key_begin / ps;
     int my_page = 0;                       // lane i: the page of the partition's i-th block of page_size keys
@@ -380,8 +381,29 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
         }
     };
     // The first keys and values are asked for before the queries are prepared: they depend on the page
-    // numbers alone, and the queries' loads (and, in the fused form, their norm and rotation) then run
-    // while the keys are on their way.
+    // numbers alone, and the queries' norm and rotation (in the fused form) then run while the keys are on their way.  What the
+    // queries are made of is asked for ahead of them: loads of a CU come back in the order they were asked for (32 heads on 8, kernel and
+    // merge: one request of 256 keys 7.56 -> 7.15 us, 8 of 256 6.5 -> 6.3, 8 of 3,000 14.3 -> 13.2, one of 30,000 21.3 -> 20.7, with no divisions where
+    // a block is one token; one of 900 7.9 -> 8.0).
+    // (of the whole form, the wave after the one that writes the token prepares the queries, the others read them from LDS)
+    __shared__ __attribute__((aligned(16))) bf16_t q_stage[WHOLE && FUSED ? KC * WAVE * 8 : 8];
+    const bool prepares = !(WHOLE && FUSED) || wave == ((pos0 - key_begin) / UNIT + 1) % NW;
+    struct Raw { bf16x8 r0, r1; float rc[8], rs[8], w0[8], w1[8]; };
+    Raw raw;
+    if constexpr (FUSED) {
+        if (prepares) {
+            // channels 8g .. 8g+7 and 32 + 8g .. 32 + 8g+7 of the head: partners of the rotation sit in one lane
+            const bf16_t* src = q + (long long)t0 * ((H + 2 * Hkv) * 64) + (kvh * G + (n16 < G ? n16 : 0)) * 64 + g * 8;
+            raw.r0 = *(const bf16x8*)src;
+            raw.r1 = *(const bf16x8*)(src + 32);
+            if (fq.q_norm_w != nullptr) {
+                norm_weights<8>(fq.q_norm_w, fq.norm_dt, g * 8, raw.w0);
+                norm_weights<8>(fq.q_norm_w, fq.norm_dt, 32 + g * 8, raw.w1);
+            }
+            angles<8>(fq, pos0, g * 8, raw.rc, raw.rs);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
     Tile ta, tb;
     const int key_first = NW == 1 ? key_begin : key_begin + wave * UNIT;
     if constexpr (AHEAD) {
@@ -397,34 +419,22 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     const bool has_slopes = !FUSED && fq.slopes != nullptr;
     long long qrow[NB];                    // row of the column in the work space; -1: no column
     bf16x8 qf[NB][KC];
-    // (of the whole form, the wave after the one that writes the token prepares the queries, the others read them from LDS)
-    __shared__ __attribute__((aligned(16))) bf16_t q_stage[WHOLE && FUSED ? KC * WAVE * 8 : 8];
-    const bool prepares = !(WHOLE && FUSED) || wave == ((pos0 - key_begin) / UNIT + 1) % NW;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
         const int c = col0 + nb * 16 + n16;
         const bool valid = c < ncols;
         const int cc = valid ? c : col0;   // no column: another one's query, whose result nobody takes
-        const int tok = t0 + cc / G;
-        const int head = kvh * G + cc % G;
+        const int tok = FUSED ? t0 : t0 + cc / G;
+        const int head = kvh * G + (FUSED ? cc : cc % G);
         slope_c[nb] = has_slopes ? fq.slopes[head] : 0.f;
-        pos_c[nb] = pos0 + cc / G;
+        pos_c[nb] = FUSED ? pos0 : pos0 + cc / G;
         lo_c[nb] = window > 0 ? max(0, pos_c[nb] - window + 1) : 0;
         qrow[nb] = valid ? (long long)tok * H + head : -1;
         if constexpr (FUSED) {
             if (!prepares) continue;
-            // channels 8g .. 8g+7 and 32 + 8g .. 32 + 8g+7 of the head: partners of the rotation sit in one lane
-            const bf16_t* src = q + (long long)tok * ((H + 2 * Hkv) * 64) + head * 64 + g * 8;
-            const bf16x8 r0 = *(const bf16x8*)src, r1 = *(const bf16x8*)(src + 32);
-            float rc[8], rs[8], w0[8], w1[8];
-            if (fq.q_norm_w != nullptr) {
-                norm_weights<8>(fq.q_norm_w, fq.norm_dt, g * 8, w0);
-                norm_weights<8>(fq.q_norm_w, fq.norm_dt, 32 + g * 8, w1);
-            }
-            angles<8>(fq, pos_c[nb], g * 8, rc, rs);
             float v0[8], v1[8];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) { v0[e] = (float)r0[e]; v1[e] = (float)r1[e]; }
+            for (int e = 0; e < 8; ++e) { v0[e] = (float)raw.r0[e]; v1[e] = (float)raw.r1[e]; }
             // sums of squares of four channels each, then the butterfly of sixteen such sums in the order
             // of the kernel for portions (partners 32, 16, 8 and 4 channels away)
             float p[2][2];
@@ -442,15 +452,16 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
                 const float inv = 1.0f / sqrtf(ss / 64.0f + fq.eps);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    v0[e] = v0[e] * inv * w0[e];
-                    v1[e] = v1[e] * inv * w1[e];
+                    v0[e] = v0[e] * inv * raw.w0[e];
+                    v1[e] = v1[e] * inv * raw.w1[e];
                 }
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const float x0 = v0[e], x1 = v1[e];
-                qf[nb][0][e] = (bf16_t)(x0 * rc[e] - x1 * rs[e]);
-                qf[nb][1][e] = (bf16_t)(x0 * rs[e] + x1 * rc[e]);
+                // (the fused product spelled out: left to the compiler, the forms of the kernel choose differently)
+                qf[nb][0][e] = (bf16_t)fmaf(x0, raw.rc[e], -product(x1, raw.rs[e]));
+                qf[nb][1][e] = (bf16_t)fmaf(x0, raw.rs[e], product(x1, raw.rc[e]));
             }
         } else {
 #pragma unroll
@@ -479,7 +490,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     const float to_m = scaled ? 1.f : scale, log2s = to_m * 1.44269504088896340736f;
     auto exp2_of = [](float x) { return __builtin_amdgcn_exp2f(x); };
     // what every column of the block sees: a step within it takes all its keys as they are
-    const int all_lo = window > 0 ? max(0, pos_max - window + 1) : 0, all_hi = pos0 + col0 / G;
+    const int all_lo = window > 0 ? max(0, pos_max - window + 1) : 0, all_hi = FUSED ? pos0 : pos0 + col0 / G;
     // FIRST: the unit's first step, which finds nothing to scale
     auto compute = [&](int key0, Tile& t, auto FIRST) {
         // ---- S^T = K Q^T, twice 16 keys
@@ -666,7 +677,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
         lds_barrier();
         const int parts = (n_units + UNITS - 1) / UNITS;
         for (int c = wave; c < n_cols; c += NW) {
-            const int head = kvh * G + (col0 + c) % G;
+            const int head = kvh * G + (FUSED ? c : (col0 + c) % G);
             const float sink = sinks ? sinks[head] : -INFINITY;
             float m_l = -INFINITY, l_l = 0.f;              // of partition `lane`
             if (lane < parts) { m_l = p_ml[(lane * cols + c) * 2]; l_l = p_ml[(lane * cols + c) * 2 + 1]; }
@@ -679,7 +690,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
                 if (w > 0.f) acc = fmaf(w, p_o[(p * cols + c) * 64 + lane], acc);
             }
             if (sinks) L += __expf(sink - M);
-            if (lane < hd) out[((long long)(t0 + (col0 + c) / G) * H + head) * hd + lane] = (bf16_t)(acc * (1.0f / L));
+            if (lane < hd) out[((long long)(FUSED ? t0 : t0 + (col0 + c) / G) * H + head) * hd + lane] = (bf16_t)(acc * (1.0f / L));
         }
         return;
     } else if constexpr (NW == 1 && ONE_UNIT) {
@@ -826,17 +837,18 @@ __global__ __launch_bounds__(WAVE) void attn_combine64_kernel(const float* __res
                                                               const float* __restrict__ sinks) {
     const long long row = blockIdx.x;                      // token * H + head
     const int lane = threadIdx.x;
+    const unsigned token = blockIdx.x / (unsigned)H;
     // a head's sink: a logit without key or value that counts once in the denominator (none: -inf, which adds 0)
-    const float sink = sinks ? sinks[row % H] : -INFINITY;
+    const float sink = sinks ? sinks[blockIdx.x - token * H] : -INFINITY;
     float m_l = -INFINITY, l_l = 0.f;
     if (lane < n_parts) {                                  // read before the position is known: rows exist for all partitions
         const float* ml = ws_ml + (row * n_parts + lane) * 2;
         m_l = ml[0];
         l_l = ml[1];
     }
-    const int pos = positions[row / H];
+    const int pos = positions[token];
     const int lo = window > 0 ? max(0, pos - window + 1) : 0;
-    const int p_lo = lo / part_keys, p_hi = pos / part_keys;
+    const int p_lo = (unsigned)lo / (unsigned)part_keys, p_hi = (unsigned)pos / (unsigned)part_keys;
     const bool valid = lane >= p_lo && lane <= p_hi && l_l > 0.f;
     const float M = fmaxf(wave_max(valid ? m_l : -INFINITY), sink);
     const float w_l = valid ? __expf(m_l - M) : 0.f;
@@ -905,7 +917,8 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
     __shared__ float red[COMBINE_WAVES];
     const long long row = blockIdx.x;                      // token * H + head
     const int tid = threadIdx.x, lane = tid % WAVE, wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-    const int pos = positions[row / H];
+    const unsigned token = blockIdx.x / (unsigned)H;
+    const int pos = positions[token];
     const buffer_t mbuf = make_buffer(ws_ml + row * n_parts * 2, n_parts * 8);
     const buffer_t obuf = make_buffer(ws_o + row * n_parts * hd, n_parts * hd * 4);
     float m_p[PER_THREAD], l_p[PER_THREAD];                // of the partitions tid, tid + 512, ...; beyond the last: zero
@@ -915,7 +928,7 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
         l_p[k] = load_buffer_float(mbuf, (tid + k * COMBINE_WAVES * WAVE) * 8 + 4, 0);
     }
     const int lo = window > 0 ? max(0, pos - window + 1) : 0;
-    const int p_lo = lo / part_keys, p_hi = pos / part_keys;          // the token's partitions, absolute numbers
+    const int p_lo = (unsigned)lo / (unsigned)part_keys, p_hi = (unsigned)pos / (unsigned)part_keys;          // the token's partitions, absolute numbers
     float first[AHEAD];                                    // the partial outputs of group `wave`
     const int first_lo = max(p_lo, wave * COMBINE_GROUP), first_hi = min(p_hi, wave * COMBINE_GROUP + COMBINE_GROUP - 1);
     const bool ahead = NARROW && first_hi - first_lo >= FEW;
@@ -938,7 +951,7 @@ __global__ __launch_bounds__(COMBINE_WAVES * WAVE) void attn_combine_kernel(cons
     lds_barrier();
 #pragma unroll
     for (int w = 0; w < COMBINE_WAVES; ++w) M = fmaxf(M, red[w]);
-    const float sink = sinks ? sinks[row % H] : -INFINITY;
+    const float sink = sinks ? sinks[blockIdx.x - token * H] : -INFINITY;
     M = fmaxf(M, sink);
 #pragma unroll
     for (int k = 0; k < PER_THREAD; ++k) {
@@ -1155,6 +1168,7 @@ static int launch_attention(const void* q, const void* k_cache, const void* v_ca
     dim3 grid(n_parts, n_qblocks, Hkv);
     FusedQKV plain_form;
     plain_form.slopes = slopes;
+    plain_form.group = H / Hkv;
     // (as many blocks as tokens: a token a block, of up to eight columns)
     if (nb == 1 && hd > 32 && hd <= 64 && takes_whole((long long)n_qblocks * Hkv, n_parts, n_qblocks == n_tokens ? H / Hkv : 16))
         return launch_whole<false>(dim3(1, n_qblocks, Hkv), stream, Q, K, V, block_table, max_blocks, (const int2*)blk, (const int4*)req_info,
@@ -1260,6 +1274,7 @@ TUFF_EXPORT int tuff_attention_decode_fused(const void* qkv, void* k_cache, void
     fq.q_norm_w = q_norm_w; fq.k_norm_w = k_norm_w; fq.norm_dt = norm_dt; fq.eps = eps;
     fq.inv_freq = inv_freq; fq.slot_mapping = slot_mapping;
     fq.angles = angles; fq.n_angles = angles ? n_angles : 0;
+    fq.group = H / Hkv;
     if (takes_whole((long long)n_tokens * Hkv, n_parts, H / Hkv))
         return launch_whole<true>(dim3(1, n_tokens, Hkv), stream, (const bf16_t*)qkv, (bf16_t*)k_cache, (bf16_t*)v_cache, block_table,
                                   max_blocks, nullptr, (const int4*)req_info, H, Hkv, 64, page_size, window, scale, n_parts, fq,
