@@ -168,7 +168,7 @@ __global__ __launch_bounds__(NW * WAVE) void attn_partition_kernel(
     // Workgroups that run side by side read neighbouring memory when the kv head is what changes fastest
     // from one to the next (a page holds its kv heads one after the other): that order for launches of
     // several rounds of waves, partitions first for the others.
-    const int part = WHOLE ? 0 : kv_fast ? blockIdx.x / (unsigned)Hkv : blockIdx.x, qb = blockIdx.y, kvh = kv_fast ? (int)blockIdx.x - part * Hkv : blockIdx.z;
+    const int part = WHOLE ? 0 : kv_fast ? blockIdx.x / Hkv : blockIdx.x, qb = blockIdx.y, kvh = kv_fast ? (int)blockIdx.x - part * Hkv : blockIdx.z;
     const int lane = threadIdx.x % WAVE, n16 = lane % 16, g = lane / 16;
     const int wave = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int G = fq.group;
