@@ -677,6 +677,25 @@ def test_rmsnorm(gpu, n, d, out_dtype):
     assert (out.cpu().double() - want).abs().max() <= (1e-5 if out_dtype == torch.float32 else 2 ** -8 * float(want.abs().max()))
 
 
+@pytest.mark.parametrize("d", [4, 1020, 1024, 1028, 2048, 2052, 4096, 4100])
+@pytest.mark.parametrize("w_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])
+def test_rmsnorm_of_rows_in_registers_has_the_bits_of_rows_read_again(gpu, d, w_dtype, out_dtype):
+    """The kernel that keeps rows and weights in registers against the one that reads them again, which a weight off its
+    16-byte border takes; rows of a wider matrix, gathered."""
+    from tuff_amd.csrc import ops
+    x = _r(7, d + 8, seed=7, scale=3.0).to(gpu)[:, 4:4 + d]
+    w = (1 + _r(d, seed=8, scale=0.1)).to(w_dtype).to(gpu)
+    off = torch.empty(d + 1, device=gpu, dtype=w_dtype)[1:]
+    off.copy_(w)
+    rows = torch.tensor([6, 0, 3], dtype=torch.int32, device=gpu)
+    for which in (None, rows):
+        got, want = (torch.empty(7 if which is None else 3, d, device=gpu, dtype=out_dtype) for _ in range(2))
+        ops.rmsnorm(x, w, got, 1e-5, which)
+        ops.rmsnorm(x, off, want, 1e-5, which)
+        assert torch.equal(got, want)
+
+
 def test_embed_and_swiglu(gpu):
     from tuff_amd.csrc import ops
     table = _r(50, 24, seed=9, dtype=torch.bfloat16)

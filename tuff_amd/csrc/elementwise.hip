@@ -103,14 +103,61 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
     }
 }
 
+// The same for rows of a multiple of four elements, up to 1,024 PIECES, whose ends are aligned: row and weight are asked for
+// together and stay in registers, so a row waits for memory once instead of three times (the row, the row again from the cache,
+// the weight).  That wait is what a few rows cost.  The same operations in the same order: the same bits.
+// Rows of 2,048 float32 in a graph, weights in the cache, us, kernel above / this one: 1 row 2.10 / 1.81, 4 2.24 / 1.99, 500
+// 3.63 / 3.26, 2,048 7.0 / 6.3; 4 rows of 4,096 2.78 / 2.12.  In a float32 step of four tokens, weights from memory: 1.1 less a norm.
+template <typename TW, typename TO, int PIECES>
+__global__ __launch_bounds__(256) void rmsnorm_regs_kernel(const float* __restrict__ x, const TW* __restrict__ w, TO* __restrict__ out,
+                                                           const int* __restrict__ rows, int d, long long ldx, float eps) {
+    typedef TW in4 __attribute__((ext_vector_type(4)));
+    typedef TO out4 __attribute__((ext_vector_type(4)));
+    __shared__ float scratch[4];
+    const int r = blockIdx.x;
+    in4 wv[PIECES];
+    f32x4 v[PIECES];
+    auto at = [&](int k) { return (int)threadIdx.x * 4 + k * 1024; };
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) {
+        wv[k] = in4{};
+        if (at(k) < d) wv[k] = *(const in4*)(w + at(k));
+    }
+    const float* xr = x + (long long)(rows ? rows[r] : r) * ldx;
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) {
+        v[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (at(k) < d) v[k] = *(const f32x4*)(xr + at(k));
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) {
+        ss = fmaf(v[k][0], v[k][0], ss); ss = fmaf(v[k][1], v[k][1], ss); ss = fmaf(v[k][2], v[k][2], ss); ss = fmaf(v[k][3], v[k][3], ss);
+    }
+    const float total = block_sum<4>(ss, scratch);
+    const float inv = 1.0f / sqrtf(total / (float)d + eps);
+#pragma unroll
+    for (int k = 0; k < PIECES; ++k) {
+        out4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = from_f32<TO>(v[k][e] * inv * to_f32((TW)wv[k][e]));
+        if (at(k) < d) *(out4*)(out + (long long)r * d + at(k)) = y;
+    }
+}
+
 TUFF_EXPORT int tuff_rmsnorm(const float* x, const void* w, int w_dt, void* out, int out_dt,
                              const int* rows, int n_rows, int d, long long ldx, float eps, hipStream_t stream) {
     if (n_rows <= 0) return 0;
     if (d <= 0 || ldx < d) return -2;
     const bool vec = d % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % 16 == 0;
+    const bool regs = vec && d <= 4096 && (uintptr_t)w % 16 == 0 && (uintptr_t)out % 16 == 0;
     dim3 grid(n_rows), block(256);
+#define REGS(TW, TO, PIECES) hipLaunchKernelGGL((rmsnorm_regs_kernel<TW, TO, PIECES>), grid, block, 0, stream, x, (const TW*)w, (TO*)out, rows, d, ldx, eps)
 #define LAUNCH(TW, TO) do { \
-        if (vec) hipLaunchKernelGGL((rmsnorm_kernel<TW, TO, true>), grid, block, 0, stream, x, (const TW*)w, (TO*)out, rows, d, ldx, eps); \
+        if (regs && d <= 1024) REGS(TW, TO, 1); \
+        else if (regs && d <= 2048) REGS(TW, TO, 2); \
+        else if (regs) REGS(TW, TO, 4); \
+        else if (vec) hipLaunchKernelGGL((rmsnorm_kernel<TW, TO, true>), grid, block, 0, stream, x, (const TW*)w, (TO*)out, rows, d, ldx, eps); \
         else hipLaunchKernelGGL((rmsnorm_kernel<TW, TO, false>), grid, block, 0, stream, x, (const TW*)w, (TO*)out, rows, d, ldx, eps); \
     } while (0)
     if (w_dt == DT_F32 && out_dt == DT_F32) LAUNCH(float, float);
@@ -118,6 +165,7 @@ TUFF_EXPORT int tuff_rmsnorm(const float* x, const void* w, int w_dt, void* out,
     else if (w_dt == DT_BF16 && out_dt == DT_F32) LAUNCH(bf16_t, float);
     else LAUNCH(bf16_t, bf16_t);
 #undef LAUNCH
+#undef REGS
     return launch_status();
 }
 
