@@ -696,6 +696,45 @@ def test_rmsnorm_of_rows_in_registers_has_the_bits_of_rows_read_again(gpu, d, w_
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("d", [4, 260, 1024, 1028, 2047, 2048, 4096, 4100])
+@pytest.mark.parametrize("store", [False, True])
+def test_mean_of_two_normed_rows(gpu, d, store):
+    """Both kernels (16 bytes a load and one number) against float64: sums of d squares in float32 are within d 2^-24 of their
+    value, so a normed row within (d / 2 + 4) 2^-24 of it; stored, what stood in the output does not count."""
+    from tuff_amd.csrc import ops
+    T = 5
+    a, b, out0 = _r(T, d, seed=1, scale=2.0), _r(T, d, seed=2, scale=0.5), _r(T, d, seed=3)
+    wa, wb = 1 + _r(d, seed=4, scale=0.1), 1 + _r(d, seed=5, scale=0.1)
+    parts = [plain.rms_norm(v.double(), w.double(), 1e-5) for v, w in ((a, wa), (b, wb))]
+    want = 0.5 * (parts[0] + parts[1]) + (0 if store else out0.double())
+    bound = (d / 2 + 8) * 2.0 ** -24 * (parts[0].abs() + parts[1].abs() + out0.double().abs())
+    for lead in (0, 1):                                   # (1: off the 16-byte border)
+        def put(v):
+            r = torch.empty(v.numel() + lead, device=gpu)[lead:].view(v.shape)
+            return r.copy_(v)
+        out = put(torch.full_like(out0, float("nan")) if store else out0)
+        ops.normed_mean2(put(a), put(wa), put(b), put(wb), out, eps=1e-5, coef=0.5, store=store)
+        assert ((out.cpu().double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("T", [1, 5, 16, 17, 40, 64, 65, 200, 513])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("bias", [False, True])
+def test_a_stored_output_is_what_is_added_to_zeros(gpu, T, dtype, bias):
+    """Linear.forward(next_norm=STORED) writes its output whatever stood there."""
+    from tuff_amd.parts.base import STORED, Runtime
+    from tuff_amd.parts.linear import Linear
+    K, N = 256, 320
+    lin = Linear("w", K, N, bias="b" if bias else None)
+    lin.bind({"w": _r(N, K, seed=1, scale=K ** -0.5, dtype=dtype).to(gpu), "b": _r(N, seed=2).to(gpu)}, Runtime(gpu, dtype))
+    x = _r(T, K, seed=3, dtype=dtype).to(gpu)
+    added = torch.zeros(T, N, device=gpu)
+    lin.forward(x, accumulate_into=added)
+    stored = torch.full((T, N), float("nan"), device=gpu)
+    lin.forward(x, accumulate_into=stored, next_norm=STORED)
+    assert torch.equal(added, stored)
+
+
 def test_embed_and_swiglu(gpu):
     from tuff_amd.csrc import ops
     table = _r(50, 24, seed=9, dtype=torch.bfloat16)

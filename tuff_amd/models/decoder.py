@@ -299,11 +299,15 @@ class DecoderModel:
         last output into x also adds the embedding where the next run takes it again, and norms x for the next block;
         the final norm runs with the head, on the wanted rows."""
         last = len(self.schedule) - 1
-        y = torch.empty(ctx.T, self.hidden_size, dtype=torch.float32, device=self.rt.device)
-        ops.fill_u32(y, 0)
+        # zeros, for the blocks whose sublayers add into them
+        zeros = None
+        if any(not getattr(self.blocks[run.block], "stores_outputs", False) for run in self.schedule):
+            zeros = torch.empty(ctx.T, self.hidden_size, dtype=torch.float32, device=self.rt.device)
+            ops.fill_u32(zeros, 0)
         carry = z0 = None
         for i, run in enumerate(self.schedule):
             block = self.blocks[run.block]
+            y = None if getattr(block, "stores_outputs", False) else zeros
             nxt = self.schedule[i + 1] if i < last else None
             if run.enter is not None:
                 if z0 is None:                                  # (the first pass of the step)

@@ -187,6 +187,7 @@ class PagedAttention:
 class AttentionMixer(Mixer, PagedAttention):
     accepts_pending_norm = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_kv_heads: int, head_dim: int, *,
                  names: dict[str, str], qk_norm_eps: Optional[float] = None,
@@ -416,6 +417,7 @@ class DifferentialAttentionMixer(Mixer, PagedAttention):
     the biases, rotates and writes."""
     accepts_pending_norm = True
     adds_once_through_linear = True
+    stores_output = True
     records_portions = True
     graph_safe = True
 

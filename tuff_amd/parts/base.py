@@ -149,6 +149,19 @@ class Part:
     #: leave the norm its operand (see Linear.forward).
     adds_once_through_linear = False
 
+    #: True if forward() also takes next_norm=STORED: the residual holds nothing yet, and the output is stored there
+    #: instead of added to what it holds.  (A part that adds an `output_bias` of its own afterwards is not asked.)
+    stores_output = False
+
+
+#: What a part with stores_output is passed for next_norm where nobody has written its residual.
+STORED = object()
+
+
+def stores_output(part: Part) -> bool:
+    """Whether a bound part may be passed next_norm=STORED."""
+    return part.stores_output and getattr(part, "output_bias", None) is None
+
 
 class Norm(Part):
     """forward(x float32 [T, d], rows=None) -> [T or len(rows), d] in the compute dtype."""

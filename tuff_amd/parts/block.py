@@ -27,7 +27,7 @@ from typing import Optional
 import torch
 
 from ..csrc import ops
-from .base import BLOCKS, Block, FeedForward, FixedState, Mixer, Norm, Runtime, WeightDecl
+from .base import BLOCKS, STORED, Block, FeedForward, FixedState, Mixer, Norm, Runtime, WeightDecl, stores_output
 from .norm import LayerNorm, RMSNorm
 
 
@@ -235,6 +235,7 @@ class SandwichBlock(Block):
     side: a parts.side.TokenSide, which adds into x after the last sublayer: x <- x + norm_s(side(x, token))."""
     carries_norm = True
     hands_plain_rows = True            # next_read may be PLAIN_ROWS
+    stores_outputs = False             # set by bind(): every sublayer stores its output, none needs zeros to add into
 
     def __init__(self, before1: Norm, mixer: Mixer, after1: Norm, before2: Optional[Norm] = None,
                  ffn: Optional[FeedForward] = None, after2: Optional[Norm] = None, *, mult: float = 1.0, side=None):
@@ -274,6 +275,7 @@ class SandwichBlock(Block):
         self.rt = rt
         for p in self._parts():
             p.bind(weights, rt)
+        self.stores_outputs = self.side is None and stores_output(self.mixer) and (self.ffn is None or stores_output(self.ffn))
 
     def first_read(self):
         """(norm weight float32 [d], eps): what the block before needs to prepare this block's first input."""
@@ -283,19 +285,32 @@ class SandwichBlock(Block):
         """x float32 [T, d], in place.  carry: before1(x) where the block before left it (None: computed here).
         next_read: (norm weight, eps) of whoever reads x next; that norm of the new x is returned (None: nothing is
         read and None returned; PLAIN_ROWS: x itself in the compute type).  y: float32 [T, d] of zeros that the sublayers add
-        into (left zero again); None: made here.  extra: float32 [T, d] that joins x after everything the block adds,
-        before next_read's norm."""
+        into (left zero again); None: made here, and where all sublayers store their output (stores_outputs) neither
+        cleared nor read by them.  extra: float32 [T, d] that joins x after everything the block adds, before next_read's
+        norm."""
         T, d = x.shape
         if carry is None:
             carry = self.before1.forward(x)
         if y is None:
             y = torch.empty(T, d, dtype=torch.float32, device=x.device)
+            if self.stores_outputs:
+                return self._stored_sublayers(x, y, ctx, cache, write_cache, carry, next_read, extra)
             ops.fill_u32(y, 0)
         if self.side is None:
             return self._sublayers(x, y, ctx, cache, write_cache, carry, next_read, extra)
         rows = self._sublayers(x, y, ctx, cache, write_cache, carry, PLAIN_ROWS, None)
         self.side.forward(rows, ctx, y)
         return self._join(x, y, self.side.norm, next_read, extra, mult=1.0)
+
+    def _stored_sublayers(self, x, y, ctx, cache, write_cache, carry, next_read, extra):
+        """The sublayers where each stores its output: y is written whole by one kernel and read by the next.  Where they add into
+        zeros, each of the two kernels moves the rows once more: for 2,048 tokens of width 2,048 the norm that reads y takes
+        14.9 us with the clearing and 11.7 without, the mean of a pair of mixers 14.7 and 12.1, clearing a pair's outputs 7."""
+        self.mixer.forward(carry, ctx, cache, y, write_cache, next_norm=STORED)
+        if self.ffn is not None:
+            h = self._join(x, y, self.after1, (self.before2.weight_f32, self.before2.eps), None, clear=False)
+            self.ffn.forward(h, ctx, y, next_norm=STORED)
+        return self._join(x, y, self.after1 if self.ffn is None else self.after2, next_read, extra, clear=False)
 
     def _sublayers(self, x, y, ctx, cache, write_cache, carry, next_read, extra):
         kw = {"next_norm": None} if self.mixer.adds_once_through_linear else {}
@@ -315,13 +330,13 @@ class SandwichBlock(Block):
         self.ffn.forward(h, ctx, y, **kw)
         return self._join(x, y, self.after2, next_read, extra)
 
-    def _join(self, x, y, after, read, extra, y_next=None, y_bias=None, mult=None):
+    def _join(self, x, y, after, read, extra, y_next=None, y_bias=None, mult=None, clear=True):
         h = None
         kw = {}
         if read is not None:
             h = self.rt.empty(*x.shape)
             kw = dict(next_w=read[0], next_eps=read[1], h_out=h)
-        ops.post_norm_add(x, y=y, w=after.weight_f32, eps=after.eps, mult=self.mult if mult is None else mult, extra=extra, clear_y=True,
+        ops.post_norm_add(x, y=y, w=after.weight_f32, eps=after.eps, mult=self.mult if mult is None else mult, extra=extra, clear_y=clear,
                           y_next=y_next, y_bias=y_bias, **kw)
         return h
 

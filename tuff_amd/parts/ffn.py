@@ -25,6 +25,7 @@ class SwiGLU(FeedForward):
     records_portions = True
     accepts_pending_norm = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, ffn_dim: int, *, names: dict[str, str],
                  aliases: dict[str, tuple] | None = None):
@@ -87,6 +88,7 @@ class GatedMLP(FeedForward):
     graph_safe = True
     records_portions = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, ffn_dim: int, *, names: dict[str, str], activation: str = "gelu_tanh",
                  bias: bool = False, limit: float = 0.0, alpha: float = 1.0):
@@ -152,6 +154,7 @@ class DenseMLP(FeedForward):
     records_portions = True
     accepts_pending_norm = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, ffn_dim: int, *, names: dict[str, str], activation: str = "relu2", bias: bool = False):
         if activation not in ops.ACTIVATIONS and activation not in ops.PARAM_ACTIVATIONS:

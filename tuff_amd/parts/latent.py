@@ -44,6 +44,7 @@ class LatentAttentionMixer(Mixer, PagedAttention):
     records_portions = True
     accepts_pending_norm = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, num_heads: int, head_dim: int, rot_dim: int, value_dim: int, rank: int, *,
                  names: dict[str, str], norm_eps: float, scale: float, rot_base: float = 1.0, rot_dims: Optional[int] = None,

@@ -9,7 +9,7 @@ from typing import Optional, Sequence
 import torch
 
 from ..csrc import ops
-from .base import Runtime, WeightDecl
+from .base import STORED, Runtime, WeightDecl
 
 
 class Linear:
@@ -147,7 +147,8 @@ class Linear:
         `out_dtype` (default: the compute dtype), or adds into `accumulate_into` (float32) and
         returns None.  swiglu (interleaved pairs only): returns silu(gate) * up, [T, out/2].
         next_norm (with accumulate_into): the norm that reads the sum next; where the kernels can,
-        the product leaves it its operand and row sums (norm.announce_operand)."""
+        the product leaves it its operand and row sums (norm.announce_operand).  STORED in its place:
+        accumulate_into holds nothing yet and is stored into."""
         from .norm import PendingNorm
         w = self.weight
         if swiglu and not self.interleaved:
@@ -160,7 +161,8 @@ class Linear:
             # the row scales left by the product before, or the norm inside this product
             want_out = torch.float32 if accumulate_into is not None else (out_dtype or self.rt.dtype)
             fused = w.dtype == torch.bfloat16 and self.in_features % 8 == 0 and (
-                ops.gemm_scaled_supported(T, self.out_features, self.in_features, want_out, accumulate_into is not None)
+                ops.gemm_scaled_supported(T, self.out_features, self.in_features, want_out,
+                                          accumulate_into is not None and next_norm is not STORED)
                 if pending.pre is not None
                 else T <= ops.NORMED_MAX_ROWS and self.in_features <= ops.NORMED_MAX_K and ops.gemm_normed_rows(pending.x))
             if not fused:
@@ -189,7 +191,8 @@ class Linear:
 
         dev = w.device
         if accumulate_into is not None:
-            nxt = next_norm if self.bias is None else None      # the sum is not final before the bias is in
+            store = next_norm is STORED
+            nxt = next_norm if self.bias is None and not store else None      # the sum is not final before the bias is in
             layout = None
             if (nxt is not None and pending is None and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
                     and self.in_features % 8 == 0):
@@ -201,7 +204,7 @@ class Linear:
                 ops.gemm_accum_emit(x, w, accumulate_into, nxt.weight_f32, xw, ss)
                 nxt.announce_operand(accumulate_into, xw, ss)
                 return None
-            product(accumulate_into, accumulate=True)
+            product(accumulate_into, accumulate=not store)
             if self.bias is not None:
                 ops.add_bias(accumulate_into, self.bias)
             return None

@@ -9,7 +9,7 @@ from __future__ import annotations
 import torch
 
 from ..csrc import ops
-from .base import MIXERS, Mixer, Runtime, WeightDecl, cache_specs_of
+from .base import MIXERS, STORED, Mixer, Runtime, WeightDecl, cache_specs_of, stores_output
 
 
 @MIXERS.register("pair")
@@ -54,15 +54,18 @@ class PairMixer(Mixer):
     def _views(views: tuple, several: bool):
         return views if several else (views[0] if views else None)
 
-    def forward(self, h, ctx, cache, residual, write_cache: bool = True) -> None:
+    def forward(self, h, ctx, cache, residual, write_cache: bool = True, next_norm=None) -> None:
+        """next_norm: None, or STORED where residual holds nothing yet."""
         views = tuple(cache) if cache is not None else ()
         n = len(self._left_specs)
         T = h.shape[0]
-        # what the two add their outputs into, cleared by one kernel
+        # what the two leave their outputs in: cleared for one that adds
         ab = torch.empty(2, T, self.d, dtype=torch.float32, device=residual.device)
-        ops.fill_u32(ab, 0)
         for mixer, out, v, several in ((self.left, ab[0], views[:n], self._left_several),
                                        (self.right, ab[1], views[n:], self._right_several)):
-            kw = {"next_norm": None} if mixer.adds_once_through_linear else {}
+            kw = {"next_norm": STORED} if stores_output(mixer) else {"next_norm": None} if mixer.adds_once_through_linear else {}
+            if not stores_output(mixer):
+                ops.fill_u32(out, 0)
             mixer.forward(h, ctx, self._views(v, several), out, write_cache, **kw)
-        ops.normed_mean2(ab[0], self.w_left, ab[1], self.w_right, residual, eps=self.eps, coef=self.coef)
+        ops.normed_mean2(ab[0], self.w_left, ab[1], self.w_right, residual, eps=self.eps, coef=self.coef,
+                         store=next_norm is STORED)

@@ -104,6 +104,7 @@ class WkvMixer(Mixer):
     graph_safe = True
     records_portions = True
     adds_once_through_linear = True
+    stores_output = True
 
     MIXES = ("r", "k", "v", "g", "w")
 
@@ -173,6 +174,7 @@ class GatedDeltaMixer(Mixer):
     graph_safe = True
     records_portions = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, num_heads: int, num_qk_heads: int, key_dim: int, value_dim: int,
                  conv_taps: int, eps: float, *, names: dict[str, str], gate_activation: str = "sigmoid"):
@@ -275,6 +277,7 @@ class Mamba2Mixer(Mixer):
     graph_safe = True
     records_portions = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, num_heads: int, head_dim: int, state_dim: int, groups: int, norm_groups: int,
                  conv_taps: int, eps: float, *, names: dict[str, str]):
@@ -348,6 +351,7 @@ class ForgetGateMixer(Mixer):
     graph_safe = True
     records_portions = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, num_heads: int, key_dim: int, value_dim: int, eps: float, *, names: dict[str, str]):
         """names: checkpoint names of 'q', 'f' [H*D, d], 'f.b', 'lower' [H*D], 'v' [H*Dv, d], 'norm' [Dv], 'o' [d, H*Dv]."""

@@ -22,6 +22,7 @@ class ShortConvMixer(Mixer):
     records_portions = True
     accepts_pending_norm = True
     adds_once_through_linear = True
+    stores_output = True
 
     def __init__(self, hidden_size: int, kernel_size: int, *, names: dict[str, str],
                  aliases: dict[str, tuple] | None = None):
