@@ -677,6 +677,29 @@ def test_rmsnorm(gpu, n, d, out_dtype):
     assert (out.cpu().double() - want).abs().max() <= (1e-5 if out_dtype == torch.float32 else 2 ** -8 * float(want.abs().max()))
 
 
+@pytest.mark.parametrize("M", [1, 2, 15, 16])
+@pytest.mark.parametrize("N,K", [(24560, 1536), (24561, 1536), (24576, 1544), (65520, 2048), (65521, 2048), (65537, 136), (98304, 264)])
+def test_output_head_behind_a_norm_in_wide_tiles(gpu, M, N, K):
+    """The norm inside a product of many columns, 32 or 64 of them a workgroup: against the sums in float64 of the operands as the
+    kernel rounds them (row times weight to bfloat16), each product's K additions in float32 and the scale's roundings; the row
+    above the first and the row behind the last are not read."""
+    from tuff_amd.csrc import ops
+    x = _r(M + 2, K, seed=1, scale=2.0)
+    rows = torch.randperm(M, generator=torch.Generator().manual_seed(2)).to(torch.int32) + 1
+    x[0] = x[-1] = float("nan")
+    nw = 1 + _r(K, seed=3, scale=0.1)
+    w = _r(N, K, seed=4, scale=K ** -0.5, dtype=torch.bfloat16)
+    out = torch.full((M, N), float("nan"), device=gpu)
+    ops.gemm_normed(x.to(gpu), nw.to(gpu), 1e-5, ops.tile_weight(w.to(gpu)), out, rows=rows.to(gpu))
+    xs = x[rows.long()]
+    operand = (xs * nw).to(torch.bfloat16).to(gpu).double()
+    scale = (1 / (xs.double().pow(2).mean(1, keepdim=True) + 1e-5).sqrt()).to(gpu)
+    wide = w.to(gpu).double()
+    want = operand @ wide.T * scale
+    bound = (operand.abs() @ wide.abs().T) * scale * (K + 8) * 2.0 ** -24
+    assert ((out.double() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("d", [4, 1020, 1024, 1028, 2048, 2052, 4096, 4100])
 @pytest.mark.parametrize("w_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.bfloat16])

@@ -1545,7 +1545,7 @@ SkinnyPlan plan_skinny(int M, int N, int K, int max_waves = 16, bool emit = fals
         if (tiles16 <= 128) p.cols = 8;
         else if (tiles16 >= 4096) p.cols = 64;
         else if (tiles16 >= 512) p.cols = 32;
-        if ((max_waves < 16 || emit) && p.cols > 16) p.cols = 16;       // the norm inside keeps float32 rows in registers;
+        if ((max_waves < 16 || emit) && p.cols > 16) p.cols = 16;       // the norm inside keeps float32 rows in registers (an output head: launch_skinny16);
                                                                         // the emitting epilogue works on one tile
         if (M > 16) {
             // two row tiles: twice the operands of X a wave, so at most two tiles of W side by side and eight waves
@@ -1749,6 +1749,16 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
     size_t lds = NORM == NORM_INSIDE ? (size_t)K * sizeof(float) : 0;
     const int mt = M > 16 ? 2 : 1, chunks = ceil_div(K, SK_CHUNK);
     if constexpr (MODE == OUT_CONV) p.waves = skinny16_conv_waves(N, K);
+    if constexpr (NORM == NORM_INSIDE && MODE == OUT_F32) {
+        // An output head behind the norm, four waves a workgroup: wide tiles, whose workgroups read and norm the rows fewer times, as float32
+        // twice the bytes that the other products read.  16 columns a workgroup / wide ones, us: 65,536 x 2,048 of 1 row 47.7 / 45.2, 8 rows 61.3 /
+        // 47.3, 16 rows 83.2 / 51.7; 32,768 x 2,048 27.1 / 24.5, 33.1 / 26.6 and 43.2 / 31.7.  Up to three rows of a short K have nothing to save
+        // (65,536 x 1,024 of 2 rows 25.0 / 25.3, 16 rows 42.3 / 28.9); 16,384 columns are too few workgroups (1 row 15.9 / 24.0).  The waves cut K as before: the same bits.
+        if (p.cols == 16 && p.waves == 4 && p.tiles >= 1536 && (M > 3 || K >= 1536)) {
+            p.cols = p.tiles >= 4096 ? 64 : 32;
+            p.tiles = ceil_div(N, p.cols);
+        }
+    }
     if constexpr ((NORM == NORM_SCALED && (MODE == OUT_BF16 || MODE == OUT_SWIGLU || MODE == OUT_CONV)) || EMIT) {
         const int rc = launch_lean16<MODE, NORM, EMIT>(p, X, W, Y, M, N, K, x, stream);
         if (rc) return rc < 0 ? rc : launch_status();
@@ -1793,6 +1803,10 @@ int launch_skinny16(const void* X, const bf16_t* W, void* Y, int M, int N, int K
         else if constexpr (!EMIT && NORM != NORM_INSIDE) {
             if (p.cols == 32) { if (p.waves == 4) GO(4, 32); else if (p.waves == 8) GO(8, 32); else GO(16, 32); }
             else if (p.cols == 64 && p.waves == 4) GO(4, 64);      // (1,024 tiles or more: four waves)
+            else return -3;
+        } else if constexpr (NORM == NORM_INSIDE && MODE == OUT_F32) {
+            if (p.cols == 32 && p.waves == 4) GO(4, 32);
+            else if (p.cols == 64 && p.waves == 4) GO(4, 64);
             else return -3;
         } else return -3;
     }
