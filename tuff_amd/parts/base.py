@@ -150,7 +150,8 @@ class Part:
     adds_once_through_linear = False
 
     #: True if forward() also takes next_norm=STORED: the residual holds nothing yet, and the output is stored there
-    #: instead of added to what it holds.  (A part that adds an `output_bias` of its own afterwards is not asked.)
+    #: instead of added to what it holds.  (A part that adds an `output_bias` of its own afterwards is only asked where it is also
+    #: told to leave the bias to the caller.)
     stores_output = False
 
 
@@ -159,7 +160,7 @@ STORED = object()
 
 
 def stores_output(part: Part) -> bool:
-    """Whether a bound part may be passed next_norm=STORED."""
+    """Whether a bound part may be passed next_norm=STORED by itself: it adds no bias of its own."""
     return part.stores_output and getattr(part, "output_bias", None) is None
 
 
