@@ -294,3 +294,31 @@ def test_random_model_folder_round_trip(tmp_path):
     with safe_open(str(tmp_path / "model.safetensors"), "pt") as f:
         lower, talk = f.get_tensor("l1.mix.right.lower").float(), f.get_tensor("l1.mix.left.talk").float()
     assert 0 < lower.min() and lower.max() < 1 and (talk - torch.eye(6)).abs().max() < 0.2
+
+
+def test_only_parts_that_speak_for_their_own_forward_store_their_output():
+    """A block may ask a part to store where it says so in the class its forward() is from, and, unless the block adds it, without
+    a bias of its own."""
+    from tuff_amd.parts.base import Mixer, stores_output
+
+    class Adds(Mixer):
+        def forward(self, h, ctx, cache, residual, write_cache=True):
+            pass
+
+    class Stores(Mixer):
+        stores_output = True
+
+        def forward(self, h, ctx, cache, residual, write_cache=True, next_norm=None):
+            pass
+
+    class Named(Stores):
+        pass
+
+    class AddsAgain(Stores):
+        def forward(self, h, ctx, cache, residual, write_cache=True, next_norm=None):
+            pass
+
+    assert [stores_output(c()) for c in (Adds, Stores, Named, AddsAgain)] == [False, True, True, False]
+    biased = Stores()
+    biased.output_bias = object()
+    assert not stores_output(biased) and stores_output(biased, bias_left=True)

@@ -13,7 +13,8 @@
 //  * skinny64  up to 64 rows that skinny16 does not take: a workgroup owns 64 rows of W, one MFMA column
 //    tile a wave; the activations of a K chunk are staged once in LDS for all four waves (bandwidth bound);
 //  * skinny16  M <= 16, and up to 32 rows (two row tiles a wave) where few_rows_kernel() says so:
-//    a workgroup owns 8 to 64 rows of W; its waves split K (bandwidth bound), no barrier in the loop.
+//    a workgroup owns 8 to 64 rows of W; its waves split K (bandwidth bound), no barrier in the loop.  Sizes
+//    that divide evenly have a kernel of their own with its cut and its bits (gemm_bf16_lean.h).
 // The skinny kernels stream each weight byte once from HBM straight into MFMA operands.  Where
 // N alone gives too little parallelism to fill 256 CUs, skinny16 uses more waves a workgroup
 // (8 or 16, partials added in wave order through LDS) and skinny64 splits K over workgroups

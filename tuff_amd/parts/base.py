@@ -159,9 +159,11 @@ class Part:
 STORED = object()
 
 
-def stores_output(part: Part) -> bool:
-    """Whether a bound part may be passed next_norm=STORED by itself: it adds no bias of its own."""
-    return part.stores_output and getattr(part, "output_bias", None) is None
+def stores_output(part: Part, bias_left: bool = False) -> bool:
+    """Whether a bound part may be passed next_norm=STORED: it says so in the class that its forward() is from (a subclass with a
+    forward() of its own speaks for itself), and it adds no bias of its own or is told to leave it (bias_left)."""
+    owner = next(c for c in type(part).__mro__ if "forward" in vars(c))
+    return part.stores_output and "stores_output" in vars(owner) and (bias_left or getattr(part, "output_bias", None) is None)
 
 
 class Norm(Part):

@@ -27,7 +27,7 @@ from typing import Optional
 import torch
 
 from ..csrc import ops
-from .base import BLOCKS, STORED, Block, FeedForward, FixedState, Mixer, Norm, Runtime, WeightDecl
+from .base import BLOCKS, STORED, Block, FeedForward, FixedState, Mixer, Norm, Runtime, WeightDecl, stores_output
 from .norm import LayerNorm, RMSNorm
 
 
@@ -275,7 +275,7 @@ class SandwichBlock(Block):
         self.rt = rt
         for p in self._parts():
             p.bind(weights, rt)
-        self.stores_outputs = self.side is None and self.mixer.stores_output and (self.ffn is None or self.ffn.stores_output)
+        self.stores_outputs = self.side is None and all(stores_output(p, bias_left=True) for p in (self.mixer, self.ffn) if p is not None)
 
     def first_read(self):
         """(norm weight float32 [d], eps): what the block before needs to prepare this block's first input."""

@@ -14,6 +14,8 @@ from .base import MIXERS, STORED, Mixer, Runtime, WeightDecl, cache_specs_of, st
 
 @MIXERS.register("pair")
 class PairMixer(Mixer):
+    stores_output = True
+
     def __init__(self, hidden_size: int, left: Mixer, right: Mixer, eps: float, *, names: dict[str, str], coef: float = 0.5):
         """names: checkpoint names of 'left_norm' and 'right_norm' [d], the weights of the two outputs' norms."""
         self.d, self.left, self.right, self.eps, self.coef = int(hidden_size), left, right, float(eps), float(coef)
