@@ -411,6 +411,40 @@ def test_gemm_bf16_tiled_scales_and_whole_blocks(gpu, M, N, K):
         assert ((ss.double().sum(0) - exact).abs() <= N * 2.0 ** -24 * exact).all()
 
 
+@pytest.mark.parametrize("M,N", [(4096, 8192), (2000, 2688), (1000, 3200), (100, 192), (100, 256), (400, 3584), (3000, 3072), (2000, 3072), (100, 16384)])
+def test_gemm_bf16_without_an_inner_size(gpu, M, N):
+    """Every shape of block: products of nothing are zero, the stream stays as it is, and its norm's operand and row sums are laid out as
+    asked for, with nothing behind them written."""
+    from tuff_amd.csrc import ops
+    x, w = torch.empty(M, 0, dtype=torch.bfloat16, device=gpu), ops.tile_weight(torch.empty(N, 0, dtype=torch.bfloat16, device=gpu))
+    def room(*shape, dtype=torch.float32):
+        whole = torch.full((math.prod(shape) + 8192,), 7.0, dtype=dtype, device=gpu)
+        return whole[:-8192].view(shape), whole[-8192:]
+    for dtype in (torch.float32, torch.bfloat16):
+        out, behind = room(M, N, dtype=dtype)
+        ops.gemm(x, w, out)
+        assert (out == 0).all() and (behind == 7.0).all()
+    for n_ss in (3, 30, 40):
+        for width, swiglu in ((N, False), (N // 2, True)):
+            out, behind = room(M, width, dtype=torch.bfloat16)
+            ops.gemm_scaled(x, torch.ones(n_ss, M, device=gpu), 1e-5, w, out, swiglu=swiglu)
+            assert (out == 0).all() and (behind == 7.0).all()
+    y, nw = _r(M, N, seed=1).to(gpu), _r(N, seed=2).to(gpu)
+    stream, behind = room(M, N)
+    stream.copy_(y)
+    ops.gemm(x, w, stream, accumulate=True)
+    assert torch.equal(stream, y) and (behind == 7.0).all()
+    layout = ops.gemm_emit_layout(M, N, 0)
+    xw, behind_xw = room(M, N, dtype=torch.bfloat16)
+    ss, behind_ss = room(*layout)
+    ss.fill_(float("nan"))
+    ops.gemm_accum_emit(x, w, stream, nw, xw, ss)
+    assert torch.equal(stream, y) and torch.equal(xw, (y * nw).bfloat16())
+    assert all((b == 7.0).all() for b in (behind, behind_xw, behind_ss))
+    exact = y.double().square().view(M, layout[0], -1).sum(2).T
+    assert ((ss.double() - exact).abs() <= N // layout[0] * 2.0 ** -24 * exact).all()
+
+
 @pytest.mark.parametrize("N,K,most", [(2048, 8192, 8), (520, 4104, 16), (2048, 4480, 15), (72, 16392, 4), (2048, 256, 16)])
 def test_gemm_bf16_few_rows_that_lie_in_lds_in_whole(gpu, N, K, most):
     """Inner sizes of many chunks a wave, whole and ragged, up to the most rows that fit (one more, where there may be, comes from memory as before):

@@ -463,10 +463,11 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
             }
         }
     }
-    // (steps that are none: the last one's operands again, so that the count of loads under way is known)
+    // (steps that are none: the last one's operands again, so that the count of loads under way is known; without an inner size there is
+    // not even that one: buffers of no bytes, and no global loads)
     static_for<STAGES - 1>([&](auto s) {
         constexpr int st = decltype(s)::value;
-        issue(st, max(0, min(kt_begin + st, kt_end - 1)));
+        if (BUFFER || nk > 0) issue(st, max(0, min(kt_begin + st, kt_end - 1)));
     });
     // (a product cut along K leaves the scales to the kernel that adds the slices)
     if constexpr (AROUND == TILED_SCALED) {
@@ -565,6 +566,10 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         }
     });
     if (kt_begin < kt_end) mult(S1());
+    else {                                                     // no step has waited for the loads into LDS and for the rows' scales
+        wait_loads_and_lds<0>();
+        __builtin_amdgcn_s_barrier();
+    }
     if constexpr (FOLDS) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
@@ -1921,7 +1926,6 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
         TiledPlan t = plan_tiled(M, N, K);
         if (rows64_tiled(M, N, K)) { t.shape = 3; t.slices = 1; t.steps_per_slice = ceil_div(K, TBK); t.ws_floats = 0; }
         if (t.slices > 1 && !ws) return -4;
-        if (K == 0) t.shape = 1;                                       // (nothing to read: loads through buffers of no bytes)
         ex.bands = bands_of_rows(t, M, N);
 #define TILED(TM, TN, WM, WN, AHEAD) do { \
             auto kern = gemm_bf16_tiled_kernel<TM, TN, WM, WN, AHEAD, MODE>; \
