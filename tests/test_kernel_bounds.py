@@ -2,6 +2,9 @@
 are the kernels' own (compiled for host and device from one definition) and are called through
 the built library."""
 import ctypes
+import os
+import re
+import subprocess
 
 import pytest
 
@@ -120,3 +123,52 @@ def test_float32_attention_of_a_mixer_follows_that_rule(monkeypatch):
         ctx = types.SimpleNamespace(T=8, R=8, max_q_len=1, max_ctx_len=keys, req_info=None, req_of_token=None, positions=None)
         mixer.attend(torch.zeros(8, 32 * 64), None, ctx, cache, group)
     assert taken == ["attention_general", "attention_f32"]
+
+
+def _early_reads(assembly):
+    """The links (v_fmac_f32_dpp) whose DPP operand a vector instruction writes, or may have written on another way to a label, less
+    than two wait states before: as (line, what stands there).  Also the number of links."""
+    code = [line.split(";")[0].strip() for line in assembly.splitlines()]
+    code = [line for line in code if line and not (line.startswith(".") and not line.endswith(":"))]
+    links, early = 0, []
+    for at, line in enumerate(code):
+        if not line.startswith("v_fmac_f32_dpp"):
+            continue
+        links += 1
+        operand = int(re.match(r"v_fmac_f32_dpp v\d+, v(\d+), v\d+ row_newbcast", line).group(1))
+        states, back = 0, at - 1
+        while states < 2:
+            before = code[back]
+            written = re.match(r"v_\w+ v(?:(\d+)|\[(\d+):(\d+)\])", before)
+            first, last = (int(written.group(1) or written.group(2)), int(written.group(1) or written.group(3))) if written else (0, -1)
+            if before.endswith(":") or first <= operand <= last:
+                early.append((line, before))
+                break
+            nop = re.match(r"s_nop (\d+)", before)
+            states += 1 + int(nop.group(1)) if nop else 1
+            back -= 1
+    return links, early
+
+
+def test_links_of_the_float32_chain_do_not_read_what_was_just_written(tmp_path):
+    """The chain of the float32 product of four rows is inline assembly that the compiler's hazard handling does not look into; a move of
+    an operand that it puts between two links would be read before it is there.  In the kernels' own assembly, and in texts of
+    it with such a move planted."""
+    from tuff_amd.csrc import build
+    out = str(tmp_path / "gemm_f32.s")
+    flags = [f for f in build.FLAGS if f not in ("-shared", "-fPIC")]
+    subprocess.run([build._hipcc()] + flags + ["-I", build.HERE, "--offload-device-only", "-S", "-o", out, os.path.join(build.HERE, build.MODULES["gemm_f32"])],
+                   check=True, capture_output=True, env={**os.environ, "HOME": os.environ.get("HOME", str(tmp_path))})
+    with open(out) as f:
+        assembly = f.read()
+    links, early = _early_reads(assembly)
+    assert links >= 6 * 4 * 64 and not early, early[:4]            # three rings, with and without SwiGLU, of four steps and more
+    lines = assembly.splitlines()
+    first = next(i for i, line in enumerate(lines) if "row_newbcast:0" in line)
+    assert "s_nop 1" in lines[first - 1]
+    for at, between, found in ((first + 1, [], True), (first + 6, [], True), (first + 6, ["s_nop 0"], True), (first + 6, ["s_nop 1"], False), (first - 1, [], False)):
+        while "v_fmac_f32_dpp" not in lines[at] and at >= first:
+            at += 1
+        x = re.search(r"v_fmac_f32_dpp v\d+, (v\d+)", lines[max(at, first)]).group(1)
+        planted = lines[:at] + [f"\tv_mov_b32_e32 {x}, v1"] + between + lines[at:]
+        assert bool(_early_reads("\n".join(planted))[1]) == found, (at - first, between)

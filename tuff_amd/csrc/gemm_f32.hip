@@ -387,18 +387,25 @@ __global__ __launch_bounds__(WAVE) void gemm_f32_rows_kernel(const float* __rest
 // cycles, an instruction between two of them 3 to 4 more).  4 rows, us, one wave that did the loads itself / two: 2,048 x 8,192 35.6 and
 // 31.8 (rows kernel 49), 2,048 x 2,048 11.4 and 10.1 (13.9), 3,072 x 2,048 11.4 and 10.3, 6,144 x 2,048 13.3 and 12.3 (15.7), 1,536 x 6,912 30.2
 // and 26.9; 16 rows of 2,048 x 8,192 40.0 and 34.0; from 16,384 columns on the memory sets the time of both.
+// A DPP operand that a vector instruction has just written is read too early unless two wait states lie between, and the compiler,
+// which keeps that distance for its own instructions, does not look into these.  x comes from LDS, which is waited for; should the
+// compiler move it behind that, then ahead of a step's first link, which stands behind s_nop in one piece with it.  (x as an operand
+// that each link hands on would pin it, and costs four moves a step.)  That no move stands between the links either is looked for
+// in the assembly by tests/test_kernel_bounds.py.
 template <int LANE>
 __device__ __forceinline__ void chain4(float& acc, const f32x4& x, const f32x4& w) {
 #ifdef __HIP_DEVICE_COMPILE__
-    // k = 4 LANE + e: register e of lane LANE.  (s_nop: two wait states, should the compiler have moved x by a vector instruction
-    // just before)
-    if constexpr (LANE == 0) asm("s_nop 1" : "+v"(acc));
-    asm("v_fmac_f32_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %2, %6 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %3, %7 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n"
-        "v_fmac_f32_dpp %0, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
-        : "+v"(acc)
-        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(LANE));
+    // k = 4 LANE + e: register e of lane LANE
+#define TUFF_FOUR_LINKS(FIRST) \
+    asm(FIRST "v_fmac_f32_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n" \
+              "v_fmac_f32_dpp %0, %2, %6 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n" \
+              "v_fmac_f32_dpp %0, %3, %7 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n" \
+              "v_fmac_f32_dpp %0, %4, %8 row_newbcast:%9 row_mask:0xf bank_mask:0xf" \
+        : "+v"(acc) \
+        : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(LANE))
+    if constexpr (LANE == 0) TUFF_FOUR_LINKS("s_nop 1\n");
+    else TUFF_FOUR_LINKS("");
+#undef TUFF_FOUR_LINKS
 #endif
 }
 
