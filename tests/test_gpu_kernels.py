@@ -445,6 +445,29 @@ def test_gemm_bf16_without_an_inner_size(gpu, M, N):
     assert ((ss.double() - exact).abs() <= N // layout[0] * 2.0 ** -24 * exact).all()
 
 
+@pytest.mark.parametrize("M,N,P", [(65, 1 << 25, 4096), (129, 1 << 25, 4096), (65, (1 << 25) + 64, 192)])
+def test_gemm_bf16_into_rows_beyond_31_bits(gpu, M, N, P):
+    """2^25 columns: sixteen rows of the stream are 2^31 bytes (blocks of 128 x 256, 256 x 256 and 256 x 192).  Columns that repeat every
+    P, so that all of them are checked against a product of P columns."""
+    from tuff_amd.csrc import ops
+    K = 64
+    x, w, nw = _r(M, K, seed=1, dtype=torch.bfloat16).to(gpu), _r(P, K, seed=2, dtype=torch.bfloat16).to(gpu), _r(P, seed=4).to(gpu)
+    part = torch.empty(M, P, device=gpu)
+    ops.gemm(x, w, part)
+    part += 0.5
+    layout = ops.gemm_emit_layout(M, N, K)
+    assert layout is not None and N % layout[0] == 0
+    y, xw = torch.full((M * N + 4096,), 0.5, device=gpu), torch.full((M * N + 4096,), 7.0, dtype=torch.bfloat16, device=gpu)
+    ss = torch.full(layout, float("nan"), device=gpu)
+    ops.gemm_accum_emit(x, ops.tile_weight(w.repeat(N // P, 1)), y[:M * N].view(M, N), nw.repeat(N // P), xw[:M * N].view(M, N), ss)
+    assert (y[M * N:] == 0.5).all() and (xw[M * N:] == 7.0).all()
+    group = N // layout[0]
+    exact = part.double().square().view(M, P // group, group).sum(2)
+    for m in range(M):
+        assert (y[m * N:(m + 1) * N].view(-1, P) == part[m]).all() and (xw[m * N:(m + 1) * N].view(-1, P) == (part[m] * nw).bfloat16()).all(), m
+        assert ((ss[:, m].double().view(-1, P // group) - exact[m]).abs() <= group * 2.0 ** -24 * exact[m]).all(), m
+
+
 @pytest.mark.parametrize("N,K,most", [(2048, 8192, 8), (520, 4104, 16), (2048, 4480, 15), (72, 16392, 4), (2048, 256, 16)])
 def test_gemm_bf16_few_rows_that_lie_in_lds_in_whole(gpu, N, K, most):
     """Inner sizes of many chunks a wave, whole and ragged, up to the most rows that fit (one more, where there may be, comes from memory as before):

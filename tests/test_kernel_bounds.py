@@ -64,6 +64,15 @@ def gemm_lib():
     return ops.load("gemm_bf16")
 
 
+@pytest.mark.parametrize("M,N,K,groups", [(65, 1 << 25, 64, 1 << 17), (129, 1 << 25, 64, 1 << 17), (300, 3 << 24, 128, 3 << 16),
+                                         (65, (1 << 25) - 256, 64, (1 << 17) - 1), (65, (1 << 25) + 64, 64, 174763), (65, (1 << 25) + 128, 64, 0)])
+def test_rows_beyond_31_bits_leave_the_next_norm_its_sums(gemm_lib, M, N, K, groups):
+    """Sixteen rows of 2^25 float32 columns are 2^31 bytes; whole blocks of columns emit on both sides of that."""
+    tiles, rows = ctypes.c_int(), ctypes.c_int()
+    assert gemm_lib.tuff_gemm_bf16_emit_layout(M, N, K, ctypes.byref(tiles), ctypes.byref(rows)) == 0
+    assert (tiles.value, rows.value) == (groups, M)
+
+
 @pytest.mark.parametrize("M,N,K,plain,emit", [
     (16, 2048, 8192, False, False),                       # up to 16 rows: one kernel, whatever the sizes
     (17, 2048, 2048, False, True), (20, 1024, 1024, False, False), (20, 2048, 1032, False, True), (17, 256, 64, False, False),

@@ -127,7 +127,9 @@ struct TiledExtra {
 };
 // TILED_BIAS: v + bias[column], rounded to bfloat16; TILED_RELU2: the square of its positive part, rounded.  As a kernel of their
 // own each wrote and read the float32 sums once more (2,048 rows of 5,632 columns: 15 us beside a product of 50).
-enum : int { TILED_PLAIN = 0, TILED_SCALED = 1, TILED_EMIT = 2, TILED_BIAS = 3, TILED_RELU2 = 4 };
+// TILED_EMIT_FAR: TILED_EMIT for rows of 2^25 columns and more, of which sixteen are 2^31 bytes: its epilogue goes by address and not
+// through buffers (both in one kernel cost the others 0.25 us of 10 to 27).
+enum : int { TILED_PLAIN = 0, TILED_SCALED = 1, TILED_EMIT = 2, TILED_BIAS = 3, TILED_RELU2 = 4, TILED_EMIT_FAR = 5 };
 
 template <int TM, int TN, int WAVES_M, int WAVES_N, int AHEAD, int MODE>
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_tiled_kernel(
@@ -293,7 +295,7 @@ template <int TM, int TN, int WAVES_M, int WAVES_N, int STAGES, bool BUFFER, boo
 __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
         const bf16_t* __restrict__ X, const bf16_t* __restrict__ W, void* __restrict__ Y, int M, int N, int K,
         int steps_per_slice, float* __restrict__ ws, TiledExtra ex) {
-    static_assert(AROUND != TILED_EMIT || MODE == OUT_F32_ACCUM, "the emitting epilogue adds into the residual stream");
+    static_assert(!(AROUND == TILED_EMIT || AROUND == TILED_EMIT_FAR) || MODE == OUT_F32_ACCUM, "the emitting epilogue adds into the residual stream");
     constexpr int NW = WAVES_M * WAVES_N;
     constexpr int BM = 16 * TM * WAVES_M, BN = 16 * TN * WAVES_N;
     constexpr int IA = BM / 8 / NW, IB = BN / 8 / NW;                  // load instructions of X and of W a wave issues a step
@@ -597,30 +599,37 @@ __global__ __launch_bounds__(64 * WAVES_M * WAVES_N) void gemm_bf16_dma_kernel(
             __syncthreads();
         }
     }
-    if constexpr (AROUND == TILED_EMIT) {
+    if constexpr (AROUND == TILED_EMIT || AROUND == TILED_EMIT_FAR) {
+        constexpr bool FAR = AROUND == TILED_EMIT_FAR;
         // whole blocks of columns only (the host sees to it): Y += acc, the next norm's operand, the row's sum of squares.  Sixteen rows a
         // buffer: those beyond the matrix lie behind it (nothing is fetched or written), and a lane's place is the same in every one.
-        const int at = r16 * N + (int)n0 + wn + g * 4;
+        const int at = FAR ? 0 : r16 * N + (int)n0 + wn + g * 4;
         float wave_sq[TM];
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             float sq = 0.f;
             const int row0 = wm + i * 16, rows = max(0, min(16, last_a + 1 - row0));
             const long long first = (m0 + (rows > 0 ? row0 : 0)) * N;
-            const buffer_t ybuf = make_buffer((float*)Y + first, rows * N * 4), xwbuf = make_buffer(ex.emit_xw + first, rows * N * 2);
+            const buffer_t ybuf = make_buffer((float*)Y + first, FAR ? 0 : rows * N * 4), xwbuf = make_buffer(ex.emit_xw + first, FAR ? 0 : rows * N * 2);
+            const long long far = first + (long long)r16 * N + n0 + wn + g * 4;
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 f32x4 y, nw;
                 if constexpr (EARLY) { y = y_old[i][j]; nw = next_w[j]; }
                 else {
-                    y = load_buffer_f32x4(ybuf, at * 4 + j * 64, 0);
+                    if constexpr (FAR) y = r16 < rows ? *(const f32x4*)((const float*)Y + far + j * 16) : f32x4{0.f, 0.f, 0.f, 0.f};
+                    else y = load_buffer_f32x4(ybuf, at * 4 + j * 64, 0);
                     nw = *(const f32x4*)(ex.emit_nw + n0 + wn + j * 16 + g * 4);
                 }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) y[e] += acc[i][j][e];
-                store_buffer(ybuf, at * 4 + j * 64, 0, y);
+                if constexpr (!FAR) store_buffer(ybuf, at * 4 + j * 64, 0, y);
                 const bf16x4 o = {(bf16_t)(y[0] * nw[0]), (bf16_t)(y[1] * nw[1]), (bf16_t)(y[2] * nw[2]), (bf16_t)(y[3] * nw[3])};
-                store_buffer(xwbuf, at * 2 + j * 32, 0, o);
+                if constexpr (!FAR) store_buffer(xwbuf, at * 2 + j * 32, 0, o);
+                else if (r16 < rows) {
+                    *(f32x4*)((float*)Y + far + j * 16) = y;
+                    *(bf16x4*)(ex.emit_xw + far + j * 16) = o;
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) sq = fmaf(y[e], y[e], sq);
             }
@@ -1899,7 +1908,7 @@ int launch_skinny64_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N
 int tiled_emit_group(int M, int N, int K) {
     const TiledPlan t = plan_tiled(M, N, K);
     if (t.slices > 1) return 64;                        // the kernel that adds the slices emits, 64 columns a workgroup
-    if (!dma_ok(K) || N >= (1 << 25)) return 0;         // (it counts the bytes of sixteen rows of Y in 31 bits)
+    if (!dma_ok(K)) return 0;
     const int bn = t.shape == 0 || t.shape == 5 ? 256 : t.shape == 4 ? 192 : t.shape == 3 ? 64 : 128;
     if (N % bn != 0) return 0;
     return bn;                                          // a workgroup's columns
@@ -1955,7 +1964,13 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
         if constexpr (AROUND != TILED_PLAIN) {
             if (!dma_ok(K) && t.slices == 1) return -2;            // a product in slices is finished by the kernel that adds them
         }
-        if (dma_ok(K)) {
+        if constexpr (AROUND == TILED_EMIT_FAR) {
+            // (so many columns are many large blocks)
+            if (t.shape == 4) TILED_DMA(8, 3, 2, 4, 2, false, false);
+            else if (t.shape == 0) TILED_DMA(8, 4, 2, 4, 2, true, false);
+            else if (t.shape == 5) TILED_DMA(4, 4, 2, 4, 3, true, false);
+            else return -3;                                            // (a shape forced for a measurement)
+        } else if (dma_ok(K)) {
             const bool buffer = dma_through_buffer(t, M, N);
             if (t.shape == 3 && t.steps_per_slice < ceil_div(K, TBK)) TILED_DMA(2, 2, 2, 2, 4, true, true);
             else if (t.shape == 3) { if (buffer) TILED_DMA(2, 2, 2, 2, 4, true, false); else TILED_DMA(2, 2, 2, 2, 4, false, false); }
@@ -1980,7 +1995,7 @@ int launch_mode(const bf16_t* X, const bf16_t* W, void* Y, int M, int N, int K, 
             fx.ss_in = ex.ss_in; fx.n_ss = ex.n_ss; fx.eps = ex.eps; fx.K = K;
             fx.emit_nw = ex.emit_nw; fx.emit_xw = ex.emit_xw; fx.emit_ss = ex.emit_ss;
             constexpr int FN = AROUND == TILED_SCALED ? NORM_SCALED : NORM_NONE;
-            hipLaunchKernelGGL((splitk_finish_kernel<MODE, FN, AROUND == TILED_EMIT>), dim3(ceil_div(N, 64), ceil_div(M, 16)),
+            hipLaunchKernelGGL((splitk_finish_kernel<MODE, FN, AROUND == TILED_EMIT || AROUND == TILED_EMIT_FAR>), dim3(ceil_div(N, 64), ceil_div(M, 16)),
                                dim3(256), 0, stream, (const float*)ws, Y, M, N, M, t.slices, fx);
         }
     }
@@ -2097,6 +2112,7 @@ TUFF_EXPORT int tuff_gemm_bf16_accum_emit(const void* X, const void* W, float* Y
         if (!tiled_emit_group(M, N, K)) return -2;
         TiledExtra t;
         t.emit_nw = next_norm_w; t.emit_xw = (bf16_t*)xw; t.emit_ss = ss;
+        if (N >= 1 << 25) return launch_mode<OUT_F32_ACCUM, TILED_EMIT_FAR>((const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, ws, stream, t);
         return launch_mode<OUT_F32_ACCUM, TILED_EMIT>((const bf16_t*)X, (const bf16_t*)W, Y, M, N, K, ws, stream, t);
     }
     if (few_rows_kernel(M, N, K, false, true)) {
