@@ -100,10 +100,12 @@ def test_gemm_f32_few_rows(gpu, M, N, K):
     assert torch.equal(acc, y0 + out)
 
 
-@pytest.mark.parametrize("M,N,K", [(4, 8209, 192), (1, 8320, 448), (3, 32776, 2048), (2, 32760, 2112), (8, 4096, 320), (16, 2048, 832), (4, 4112, 1024)])
+@pytest.mark.parametrize("M,N,K", [(4, 8209, 192), (1, 8320, 448), (4, 16384, 256), (2, 8216, 320), (4, 16384, 2048), (3, 32776, 2048), (2, 32760, 2112),
+                                   (8, 4096, 320), (8, 4100, 384), (5, 4112, 448), (4, 4112, 768), (16, 2048, 832), (4, 4112, 1024),
+                                   (4, 2048, 704), (4, 2048, 768), (3, 2056, 832), (4, 2048, 1536), (1, 32768, 3072), (1, 32768, 2304)])
 def test_gemm_f32_four_rows_a_workgroup(gpu, M, N, K):
-    """Rings of four, six and twelve steps in LDS, with as many steps as lie there, one more and fewer, and column blocks that are not
-    whole: the bits of the general kernel's chain; with SwiGLU those of the product and the kernel that applies it."""
+    """Rings of four, six and twelve steps in LDS, with fewer steps than lie there, as many, one more and whole turns, and column blocks
+    that are not whole: the bits of the general kernel's chain; with SwiGLU those of the product and the kernel that applies it."""
     from tuff_amd.csrc import ops
     test_gemm_f32_few_rows(gpu, M, N, K)
     if N % 2 == 0:

@@ -134,6 +134,17 @@ def test_float32_attention_of_a_mixer_follows_that_rule(monkeypatch):
     assert taken == ["attention_general", "attention_f32"]
 
 
+@pytest.mark.parametrize("M,N,K,steps", [
+    (4, 2048, 8192, 12), (4, 4096, 2048, 12), (4, 4112, 1536, 6), (8, 4096, 2048, 6), (4, 8192, 2048, 6), (4, 8208, 2048, 4), (4, 24576, 3072, 4),
+    (4, 32752, 2048, 4), (4, 32768, 2048, 12), (1, 65536, 2048, 12), (4, 65536, 1024, 4), (4, 65536, 1536, 4), (4, 65536, 2304, 4), (4, 40960, 2560, 4),
+    (4, 40960, 2944, 4), (4, 65536, 3072, 12), (4, 65536, 3584, 12), (4, 65536, 4096, 12), (4, 65536, 6144, 12), (1, 65536, 8192, 4), (4, 40960, 8192, 4),
+    (4, 65536, 9216, 12), (4, 65536, 16384, 4), (4, 65536, 24576, 12), (5, 8192, 2048, 0), (16, 2048, 8192, 6), (4, 65536, 96, 0), (4, 65536, 128, 0), (17, 2048, 2048, 0)])
+def test_steps_in_lds_of_the_float32_product_of_four_rows(M, N, K, steps):
+    """Measured points on both sides of each line: twelve steps for products of many columns and a K of 8,192 took 8 to 15 % longer than four."""
+    from tuff_amd.csrc import ops
+    assert ops.load("gemm_f32").tuff_gemm_f32_quad_steps(M, N, K) == steps
+
+
 def _early_reads(assembly):
     """The links (v_fmac_f32_dpp) whose DPP operand a vector instruction writes, or may have written on another way to a label, less
     than two wait states before: as (line, what stands there).  Also the number of links."""

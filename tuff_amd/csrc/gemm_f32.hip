@@ -563,23 +563,35 @@ constexpr int LARGEST = 1 << 22;                          // K of the chain kern
 
 constexpr long long SWIGLU_LARGEST = 1ll << 28;           // elements of W (the bytes up to an up row are counted in 31 bits)
 
+// How many steps of 64 k the four-row kernel keeps in LDS for a product of up to 16 rows; 0: another kernel takes it.
+// Four rows a wave as long as one trip over W serves all rows, or the waves are few enough to run side by side, two a CU (16
+// rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14), and K is not so short that
+// the empty steps it begins with count (4 rows, 2,048 x 64: 3.2 us and 2.7, x 192 3.6 and 3.5, 32,768 x 192 6.4 and 7.2).
+// Steps: twelve where a CU has one workgroup, six where it has two (4,608 x 1,536 9.4 us, with four 10.4), and four beyond, where the
+// loads under way are more than enough and the workgroups side by side count (4 rows, four / six / twelve: 16,384 x 2,048 with
+// SwiGLU 30.3, 30.9 and 39.4 us, 9,216 x 2,048 17.5, 18.0 and 24.7, 24,576 x 3,072 59.1, 69.1 and 63.2, 65,536 x 1,024 52.8, 53.9 and 57.4, x 1,536 75.4,
+// 76.2 and 78.4, x 2,304 110.1, 111.9 and 111.9, 40,960 x 2,560 79.6, 81.3 and 82.2, x 2,944 90.5, 92.8 and 92.5).
+// But twelve again for eight workgroups a CU and more, which begin and end at different times, where K is long: the columns'
+// rows are then so far apart that with few steps under way they are waited for (65,536 x 3,584 169.5, 170.8 and 165.8, x 4,608 216.5, 214.7 and 211.0, x
+// 6,144 297.4, 294.4 and 272.6, x 12,288 566, 574 and 544, 32,768 x 4,608 117.3, 116.5 and 111.8, x 24,576 614, 598 and 550), and earlier where they are whole 4 KB
+// apart (32,768 x 2,048 57.9, 57.4 and 56.0, 65,536 x 2,048 105.5, 105.3 and 100.9, x 3,072 156.0, 155.3 and 147.7).  Rows 32 KB apart or any larger power of two
+// are slow however many steps are under way, and slower with more (65,536 x 8,192 419, 424 and 460, 1 row 415, 426 and 475, 40,960 x 8,192 268,
+// 287 and 291, 65,536 x 16,384 782, 780 and 842).
+int quad_steps(int M, int N, int K) {
+    const long long waves = ceil_div_ll(N, 16) * ceil_div(M, 4);
+    if (M > 16 || K % LONG_STEP != 0 || K < 192 || (M > 4 && waves > 512)) return 0;
+    const bool long_rows = (K % 1024 == 0 ? K >= 2048 : K >= 3072) && !(K >= 8192 && (K & (K - 1)) == 0);
+    return waves <= 256 || (waves >= 2048 && long_rows) ? 12 : waves <= 512 ? 6 : 4;
+}
+
 // Which of the kernels on whole chains (K a multiple of STEP, operands on 16-byte borders).
 template <bool SWIGLU>
 int launch_whole_chain(const float* X, const float* W, float* Y, int M, int N, int K, int accumulate, hipStream_t stream) {
     if (M <= 16) {
-        // Four rows a wave as long as one trip over W serves all rows, or the waves are few enough to run side by side, two a CU (16
-        // rows, 2,048 x 8,192: 42 us, 49 through the rows kernel; 3,072 x 2,048, 768 waves: 23 and 14), and K is not so short that
-        // the empty steps it begins with count (4 rows, 2,048 x 64: 3.2 us and 2.7, x 192 3.6 and 3.5, 32,768 x 192 6.4 and 7.2).
-        // Steps in LDS: twelve where a CU has one workgroup, six where it has two (4,608 x 1,536 9.4 us, with four 10.4), and four beyond,
-        // where the loads under way are more than enough and the workgroups side by side count (4 rows, four / six / twelve: 16,384 x
-        // 2,048 with SwiGLU 30.3, 30.9 and 39.4 us, 9,216 x 2,048 17.5, 18.0 and 24.7, 32,768 x 1,024 30.1, 30.3 and 33.2, 65,536 x 1,536 74.4,
-        // 74.9 and 76.8), but twelve again for eight workgroups a CU and more with a K of 2,048 on, whose loads begin and end
-        // at different times (32,768 x 2,048 59.6, 58.0 and 56.1, 65,536 x 2,048 106.7, 105.4 and 102.2).
-        const long long waves = ceil_div_ll(N, 16) * ceil_div(M, 4);
-        if (K % LONG_STEP == 0 && K >= 192 && (M <= 4 || waves <= 512)) {
-            if (waves <= 256 || (waves >= 2048 && K >= 2048)) return launch_quad<SWIGLU, 12>(X, W, Y, M, N, K, accumulate, stream);
-            if (waves <= 512) return launch_quad<SWIGLU, 6>(X, W, Y, M, N, K, accumulate, stream);
-            return launch_quad<SWIGLU, 4>(X, W, Y, M, N, K, accumulate, stream);
+        switch (quad_steps(M, N, K)) {
+            case 12: return launch_quad<SWIGLU, 12>(X, W, Y, M, N, K, accumulate, stream);
+            case 6: return launch_quad<SWIGLU, 6>(X, W, Y, M, N, K, accumulate, stream);
+            case 4: return launch_quad<SWIGLU, 4>(X, W, Y, M, N, K, accumulate, stream);
         }
         if (N <= 4096) return launch_rows<SWIGLU, 16>(X, W, Y, M, N, K, accumulate, stream);
         return launch_rows<SWIGLU, 8>(X, W, Y, M, N, K, accumulate, stream);
@@ -590,6 +602,9 @@ int launch_whole_chain(const float* X, const float* W, float* Y, int M, int N, i
     return launch_chain<SWIGLU, 2, 4>(X, W, Y, M, N, K, accumulate, stream);
 }
 }  // namespace
+
+// quad_steps, for tests.
+TUFF_EXPORT int tuff_gemm_f32_quad_steps(int M, int N, int K) { return quad_steps(M, N, K); }
 
 // accumulate != 0: Y += X W^T (the residual add of the reference, src/lfm25_gpu.cu:171).
 TUFF_EXPORT int tuff_gemm_f32(const float* X, const float* W, float* Y, int M, int N, int K,
