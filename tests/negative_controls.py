@@ -139,8 +139,11 @@ def _env(scratch: str, control: dict | None) -> dict:
 
 
 def module_of(control: dict) -> str | None:
-    """The kernel module a control's file belongs to, or None for a Python file."""
+    """The kernel module a control's file belongs to (of a header: the one that includes it), or None for a Python file."""
     base = os.path.basename(control["file"])
+    if base.endswith(".h"):
+        folder = os.path.join(ROOT, os.path.dirname(control["file"]))
+        base = next(f for f in sorted(os.listdir(folder)) if f.endswith(".hip") and f'#include "{base}"' in open(os.path.join(folder, f)).read())
     return base[:-4] if base.endswith(".hip") else None
 
 

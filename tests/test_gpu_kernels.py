@@ -413,6 +413,30 @@ def test_gemm_bf16_tiled_scales_and_whole_blocks(gpu, M, N, K):
         assert ((ss.double().sum(0) - exact).abs() <= N * 2.0 ** -24 * exact).all()
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 256, 64), (100, 3072, 128), (400, 4608, 192), (513, 3072, 256), (333, 2052, 256), (1030, 9216, 128),
+                                   (2049, 6144, 128), (2500, 2048, 64)])
+def test_gemm_bf16_tiled_scales_of_sums_that_round(gpu, M, N, K):
+    """Every group of sums counts once: against the sums in float64, and from 17 groups on, which are added in parts, the same bits whether
+    the block asks for all of them at once (up to 32) or in turns (more, here of zeros)."""
+    from tuff_amd.csrc import ops
+    x, tiled, plain = _r(M, K, seed=1, dtype=torch.bfloat16).to(gpu), ops.tile_weight(_r(N, K, seed=2, dtype=torch.bfloat16).to(gpu)), torch.empty(M, N, device=gpu)
+    ops.gemm(x, tiled, plain)
+    def scaled(sums, swiglu=False):
+        out = torch.empty(M, N // 2 if swiglu else N, dtype=torch.bfloat16, device=gpu)
+        ops.gemm_scaled(x, sums.to(gpu), 1e-5, tiled, out, swiglu=swiglu)
+        return out
+    for n_ss in (2, 5, 16, 17, 18, 20, 31, 32):
+        g = torch.Generator().manual_seed(n_ss)
+        sums = torch.rand(n_ss, M, generator=g) * (2.0 * K / n_ss)
+        got = scaled(sums)
+        for behind in (33, 70) if n_ss > 16 else ():
+            more = torch.cat([sums, torch.zeros(behind - n_ss, M)])
+            assert torch.equal(got, scaled(more)) and torch.equal(scaled(sums, True), scaled(more, True)), (n_ss, behind)
+        want = (plain.double() * (1.0 / (sums.double().sum(0) / K + 1e-5).sqrt()).to(gpu)[:, None])
+        # n_ss additions in float32, half of which the square root takes, the roundings of the scale and the product, that of the output
+        assert ((got.double() - want).abs() <= ((n_ss / 2 + 4) * 2.0 ** -24 + 2.0 ** -8) * want.abs()).all(), n_ss
+
+
 @pytest.mark.parametrize("M,N", [(4096, 8192), (2000, 2688), (1000, 3200), (100, 192), (100, 256), (400, 3584), (3000, 3072), (2000, 3072), (100, 16384)])
 def test_gemm_bf16_without_an_inner_size(gpu, M, N):
     """Every shape of block: products of nothing are zero, the stream stays as it is, and its norm's operand and row sums are laid out as
@@ -539,6 +563,29 @@ def test_gemm_bf16_few_rows_of_sizes_that_divide_evenly(gpu, M, N, K):
                 ops.gemm_conv(x, grouped, a, state=sa, ss=sums, eps=0.0, **kw)
                 ops.gemm_conv(x * 0.5, grouped, b, state=sb, **kw)
                 assert same(a, b) and same(sa, sb) and torch.equal(sa[:2], state[:2]), (n_ss, off)
+    # sums that round, another scale a row: the bits of the kernel for any sizes, which takes those off a border of 16 bytes, and of the
+    # one that writes float32
+    for n_ss in (3, 16, 17, 255, 256):
+        g = torch.Generator().manual_seed(n_ss)
+        both = [torch.empty(n_ss * 16 + 1, device=gpu)[off:off + n_ss * 16].view(n_ss, 16) for off in (0, 1)]
+        for sums in both:
+            sums.copy_(torch.rand(n_ss, 16, generator=g.manual_seed(n_ss)) * (2.0 * K / n_ss))
+            sums[:, M:] = float("nan")                    # (rows that are none)
+        wide, out = torch.empty(M, N, device=gpu), torch.empty(2, M, N, dtype=torch.bfloat16, device=gpu)
+        ops.gemm_scaled(x, both[0], 1e-5, tiled, wide)
+        for k in (0, 1):
+            ops.gemm_scaled(x, both[k], 1e-5, tiled, out[k])
+        assert same(out[0], out[1]) and same(out[0], wide.bfloat16()), n_ss
+        if N % 32 == 0:
+            gated = torch.empty(2, M, N // 2, dtype=torch.bfloat16, device=gpu)
+            for k in (0, 1):
+                ops.gemm_scaled(x, both[k], 1e-5, tiled, gated[k], swiglu=True)
+            assert same(gated[0], gated[1]), n_ss
+        if N % 48 == 0 and K <= 2048:
+            states, y = [state.clone(), state.clone()], torch.empty(2, M, d, dtype=torch.bfloat16, device=gpu)
+            for k in (0, 1):
+                ops.gemm_conv(x, grouped, y[k], state=states[k], ss=both[k], eps=1e-5, **kw)
+            assert same(y[0], y[1]) and same(*states), n_ss
 
 
 @pytest.mark.parametrize("N,K,most", [(3072, 2560, 19), (4112, 2312, 21), (2064, 2120, 23), (2568, 2888, 17), (8176, 2056, 23)])

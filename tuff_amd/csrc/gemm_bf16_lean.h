@@ -33,7 +33,7 @@ template <int NW, int MODE, bool SCALED, bool EMIT, int COLS, int CH, bool XL>
 __global__ __launch_bounds__(NW * WAVE, lean16_waves_a_simd(NW, COLS)) void gemm_bf16_lean16_kernel(Lean16Args a) {
     constexpr bool CONV = MODE == OUT_CONV;
     constexpr int TN = CONV ? 3 : COLS > 16 ? COLS / 16 : 1;
-    static_assert(!EMIT || (MODE == OUT_F32_ACCUM && TN == 1), "the emitting epilogue adds into the residual stream, one tile");
+    static_assert(EMIT == (MODE == OUT_F32_ACCUM) && (!EMIT || TN == 1), "into the residual stream with the emitting epilogue, one tile");
     static_assert(!CONV || COLS == 8, "the convolution's epilogue takes eight channels a workgroup");
     static_assert(TN == 1 || CONV || NW * WAVE >= 256 * TN, "256 threads finish a tile");
     __shared__ __attribute__((aligned(16))) float red[TN][NW][WAVE][4];
@@ -59,10 +59,10 @@ __global__ __launch_bounds__(NW * WAVE, lean16_waves_a_simd(NW, COLS)) void gemm
 
     // ---- what is asked for ahead of the operands: sums of squares, what the epilogue adds to, the convolution's slot and taps
     float y_old = 0.f, emit_w = 0.f;
-    if constexpr (MODE == OUT_F32_ACCUM) {
+    if constexpr (EMIT) {
         if (mine) {
             y_old = ((const float*)a.Y)[(long long)trow * N + col];
-            if (EMIT) emit_w = a.emit_nw[col];
+            emit_w = a.emit_nw[col];
         }
     }
     constexpr int CONV_AHEAD = 4;
@@ -234,8 +234,6 @@ __global__ __launch_bounds__(NW * WAVE, lean16_waves_a_simd(NW, COLS)) void gemm
         sq += lane_xor4(sq);
         sq = butterfly_sum<32>(butterfly_sum<16>(butterfly_sum<8>(sq)));
         if (l % 16 == 0) a.emit_ss[(long long)block * 16 + trow] = sq;
-    } else if constexpr (MODE == OUT_F32_ACCUM) {
-        if (mine) ((float*)a.Y)[(long long)trow * N + col] = y_old + v;
     } else if constexpr (MODE == OUT_SWIGLU) {
         const float partner = lane_xor4(v);
         if (mine && (col & 1) == 0) ((bf16_t*)a.Y)[(long long)trow * (N / 2) + col / 2] = (bf16_t)silu_mul(v, partner);
