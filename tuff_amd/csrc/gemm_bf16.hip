@@ -13,8 +13,9 @@
 //  * skinny64  up to 64 rows that skinny16 does not take: a workgroup owns 64 rows of W, one MFMA column
 //    tile a wave; the activations of a K chunk are staged once in LDS for all four waves (bandwidth bound);
 //  * skinny16  M <= 16, and up to 32 rows (two row tiles a wave) where few_rows_kernel() says so:
-//    a workgroup owns 8 to 64 rows of W; its waves split K (bandwidth bound), no barrier in the loop.  Sizes
-//    that divide evenly have a kernel of their own with its cut and its bits (gemm_bf16_lean.h).
+//    a workgroup owns 8 to 64 rows of W; its waves split K (bandwidth bound), no barrier in the loop.  Some products
+//    of up to 16 rows whose sizes divide evenly have a kernel of their own with its cut and its bits (gemm_bf16_lean.h;
+//    launch_lean16() says which).
 // The skinny kernels stream each weight byte once from HBM straight into MFMA operands.  Where
 // N alone gives too little parallelism to fill 256 CUs, skinny16 uses more waves a workgroup
 // (8 or 16, partials added in wave order through LDS) and skinny64 splits K over workgroups
@@ -1703,7 +1704,9 @@ int skinny16_conv_waves(int N, int K) {
 }
 
 // Whether the kernel for sizes that divide evenly takes a product (cut as p says), and launches it: 1 launched, 0 not taken, else an
-// error (negative).
+// error (negative).  Chunks a wave: up to six, whose operands are all under way at once; SwiGLU and the convolution, with two and three
+// tiles of W, two.  From three on X lies in LDS whole or the product is not taken: into the stream up to 8 rows of K = 8,192, 10 of
+// 6,912, 6 of 10,752.
 template <int MODE, int NORM, bool EMIT>
 int launch_lean16(const SkinnyPlan& p, const void* X, const bf16_t* W, void* Y, int M, int N, int K, const Skinny16Extra& x, hipStream_t stream) {
     constexpr bool CONV = MODE == OUT_CONV, SCALED = NORM == NORM_SCALED;
